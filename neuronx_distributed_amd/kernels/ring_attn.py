@@ -86,16 +86,16 @@ def _block_fwd(q, k, v, causal, scale, window=None):
 
         if causal and ops.flash_attn_window_available():
             import ctypes
-            from ..ops import _ptr, _require_lib, _stream
+            from ..ops import _fa_operand, _ptr, _require_lib, _stream
 
             lib = _require_lib()
             B, Hq, S, D = q.shape
             out = torch.empty_like(q)
             lse = torch.empty(B, Hq, S, dtype=torch.float32,
                               device=q.device)
+            qc, kc, vc = (_fa_operand(t.contiguous()) for t in (q, k, v))
             lib.flash_attn_fwd_window(
-                _ptr(q.contiguous()), _ptr(k.contiguous()),
-                _ptr(v.contiguous()), _ptr(out), _ptr(lse),
+                _ptr(qc), _ptr(kc), _ptr(vc), _ptr(out), _ptr(lse),
                 ctypes.c_int(B), ctypes.c_int(Hq),
                 ctypes.c_int(k.shape[1]), ctypes.c_int(S),
                 ctypes.c_float(scale), ctypes.c_int(int(window)),
@@ -107,15 +107,15 @@ def _block_fwd(q, k, v, causal, scale, window=None):
     if q.is_cuda:
         from .. import ops
         import ctypes
-        from ..ops import _ptr, _require_lib, _stream
+        from ..ops import _fa_operand, _ptr, _require_lib, _stream
 
         lib = _require_lib()
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
         out = torch.empty_like(q)
         lse = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
-        lib.flash_attn_fwd(_ptr(q.contiguous()), _ptr(k.contiguous()),
-                           _ptr(v.contiguous()), _ptr(out), _ptr(lse),
+        qc, kc, vc = (_fa_operand(t.contiguous()) for t in (q, k, v))
+        lib.flash_attn_fwd(_ptr(qc), _ptr(kc), _ptr(vc), _ptr(out), _ptr(lse),
                            ctypes.c_int(B), ctypes.c_int(Hq),
                            ctypes.c_int(Hkv), ctypes.c_int(S),
                            ctypes.c_float(scale),
@@ -143,17 +143,17 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
         return _block_bwd_masked(q, k, v, out, dout, lse, scale, 0, window)
     if q.is_cuda:
         import ctypes
-        from ..ops import _fa_strides, _ptr, _require_lib, _stream
+        from ..ops import _fa_operand, _fa_strides, _ptr, _require_lib, _stream
 
         lib = _require_lib()
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
         delta = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
         dq = torch.empty_like(q)
+        qc, kc, vc, oc, doc = (_fa_operand(t.contiguous())
+                               for t in (q, k, v, out, dout))
         dk_pq = torch.empty(B, Hq, S, D, dtype=q.dtype, device=q.device)
         dv_pq = torch.empty(B, Hq, S, D, dtype=q.dtype, device=q.device)
-        qc, kc, vc = q.contiguous(), k.contiguous(), v.contiguous()
-        oc, doc = out.contiguous(), dout.contiguous()
         lib.flash_attn_bwd_strided(
             _ptr(qc), _ptr(kc), _ptr(vc), _ptr(oc), _ptr(doc),
             _ptr(lse.contiguous()), _ptr(delta), _ptr(dq), _ptr(dk_pq),

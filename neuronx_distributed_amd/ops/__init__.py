@@ -411,10 +411,15 @@ def flash_attn_available() -> bool:
     return lib is not None and hasattr(lib, "flash_attn_fwd")
 
 
-def _fa_ok_layout(t) -> bool:
+def _fa_operand(t):
     """The flash kernels take any (batch, head, seq) strides with a DENSE
-    last dim — transpose views of BSHD activations go in with no copy."""
-    return t.stride(3) == 1
+    last dim — transpose views of BSHD activations go in with no copy.  Rows
+    are moved in 16-byte words, so every row has to start at one."""
+    dense = t.stride(3) == 1 and all(
+        st % 8 == 0 for st, n in zip(t.stride()[:3], t.shape) if n > 1)
+    if not dense:
+        t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _fa_strides(*tensors):
@@ -443,12 +448,7 @@ class _FlashAttnFn(torch.autograd.Function):
         Hkv = k.shape[1]
         assert D == 128, "flash kernel supports D=128"
         assert q.dtype == torch.bfloat16
-        if not _fa_ok_layout(q):
-            q = q.contiguous()
-        if not _fa_ok_layout(k):
-            k = k.contiguous()
-        if not _fa_ok_layout(v):
-            v = v.contiguous()
+        q, k, v = _fa_operand(q), _fa_operand(k), _fa_operand(v)
         out = _fa_alloc_like(q)
         lse = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
         lib.flash_attn_fwd_strided(
@@ -471,8 +471,7 @@ class _FlashAttnFn(torch.autograd.Function):
             raise RuntimeError("flash_attn_bwd kernel not built")
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
-        if not _fa_ok_layout(dout):
-            dout = dout.contiguous()
+        dout = _fa_operand(dout)
         delta = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
         # grads are allocated in their producer's LAYOUT so autograd's
         # accumulation into BSHD views stays copy-free
@@ -520,7 +519,7 @@ def flash_attn_windowed(q, k, v, window: int, softmax_scale=None):
     Hkv = k.shape[1]
     assert D == 128 and q.dtype == torch.bfloat16
     scale = softmax_scale or 1.0 / math.sqrt(D)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v = (_fa_operand(t.contiguous()) for t in (q, k, v))
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
     lib.flash_attn_fwd_window(_ptr(q), _ptr(k), _ptr(v), _ptr(out),

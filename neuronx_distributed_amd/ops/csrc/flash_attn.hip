@@ -1,326 +1,282 @@
 // FlashAttention forward for CDNA4 (gfx950) — hand-written MFMA kernel.
 //
-// Replaces the reference's NKI flash kernels K1 (SURVEY.md §2.3,
-// reference kernels/flash_attn.py:18,51-63).  MI355X-first design per
-// cdna_hip_programming.md §B:
-//   * 8 waves/WG, each wave owns 32 q rows (WG = 256 q rows); KV tiles of
-//     64 double-buffered in LDS with the (row&7)<<4 XOR swizzle (G4).
+// Replaces the reference's NKI flash kernel K1 (reference
+// kernels/flash_attn.py:18,51-63).
+//   * 4 waves/WG, each wave owns 32 q rows, two WGs a CU; KV tiles of 64 go
+//     straight from memory into two LDS buffers.
 //   * swapped QK^T — mfma(A=K, B=Q^T) — so each lane's softmax stats are
 //     for ONE q row (l&31): row max / rescale / denom are lane-local
-//     (+ one shfl_xor with the partner half-wave).
-//   * P is repacked to bf16 PV B-fragments with pack_bf16x2 +
-//     v_permlane32_swap (T12/T21 primitive).
+//     (+ one exchange with the partner half-wave).
+//   * P never leaves the registers: the accumulator's order of keys is the
+//     contraction order of P V, and V^T is read from LDS in that order by
+//     transposing reads.
 //   * O is accumulated TRANSPOSED (O^T[d][q], q = lane) so the online
-//     rescale is a per-lane scalar multiply; V is staged transposed (Vt).
+//     rescale is a per-lane scalar multiply.
 //   * GQA: kv head = q head / (Hq/Hkv); causal masking per element on
-//     diagonal tiles, whole-tile skip below the diagonal.
+//     diagonal tiles only, whole-tile skip below the diagonal.
+//
+// Bound by the matrix cores together with the exponentials and the rest of
+// the vector work: at 8192 tokens, 32/8 heads, the matrix pipes are 51 % busy
+// (rocprofv3), LDS 25 %.  845 us before (8 waves, one WG a CU, values turned
+// by scattered writes, masks on every tile), 575 us (956 TFLOP/s) now: 600
+// with the loads into LDS and masks on the boundary alone, 580 with the next
+// tile's scores beside this tile's exponentials, 575 with the order below.
+// 64 q rows a wave (half the LDS reads, one wave a SIMD) took 665.  A running
+// maximum that lags behind by up to 2^8 took 570, but the largest weight of a
+// row is then not exactly one, and the error grows by 5 %.
 //
 // Layouts: q,k,v,out (B, H, S, D) bf16 contiguous, D = 128; lse (B,Hq,S)
 // f32 (natural-log row logsumexp, saved for backward).
 
 #include "common.h"
 #include "mfma.h"
+#include "lds.h"
 
 #define FA_D 128
-#define FA_QW 32       // q rows per wave
-#define FA_WAVES 8
-#define FA_QBLK (FA_QW * FA_WAVES)  // 256 q rows per workgroup
 #define FA_KV 64       // kv tile
 #define LOG2E 1.4426950408889634f
 #define NEG_INF (-1e30f)
+#define FA_QBLK 128    // q rows of a workgroup: 4 waves of 32
+#define FA_TILE_B (FA_KV * FA_D * 2)   // 16 KB: a key or value tile
 
-// LDS: double-buffered K [64][128] bf16 (256B rows, swz16 = conflict-free
-// b128 reads) and Vt [128][72] bf16 (144B padded rows: 16B-aligned, and
-// 36*d = 4*(9d mod 16) banks are distinct within every b128 lane group
-// since 9 is coprime to 16 -> conflict-free, no swizzle needed)
-#define K_TILE_B (FA_KV * FA_D * 2)    // 16 KB
-#define VT_PITCH 72
-#define VT_TILE_B (FA_D * VT_PITCH * 2)  // 18 KB
+struct FwdArgs {
+  const short *q, *k, *v;
+  short* o;
+  float* lse;
+  int Hq, Hkv, S, causal, window;
+  float scale;
+  // element strides of (batch, head, seq); the last dim (d) is dense.
+  // BHSD contiguous: (H*S*128, S*128, 128).  BSHD transpose views (no-copy
+  // model layout): (S*H*128, 128, H*128).
+  long q_bs, q_hs, q_ss, k_bs, k_hs, k_ss, v_bs, v_hs, v_ss, o_bs, o_hs, o_ss;
+};
 
-extern "C" __global__ void __launch_bounds__(512, 2)
-flash_fwd_kernel(const short* __restrict__ qp, const short* __restrict__ kp,
-                 const short* __restrict__ vp, short* __restrict__ op,
-                 float* __restrict__ lsep, int B, int Hq, int Hkv, int S,
-                 float scale, int causal, int window,
-                 long q_bs, long q_hs, long q_ss,
-                 long k_bs, long k_hs, long k_ss,
-                 long v_bs, long v_hs, long v_ss,
-                 long o_bs, long o_hs, long o_ss) {
-  // (*_bs, *_hs, *_ss) = element strides of (batch, head, seq); the last
-  // dim (d) is always dense.  BHSD contiguous: (H*S*128, S*128, 128).
-  // BSHD transpose views (no-copy model layout): (S*H*128, 128, H*128).
-  // window > 0: Mistral-style sliding window — q row i attends kv rows
-  // [i - window + 1, i] (causal implied); whole tiles outside the band
-  // are skipped, boundary tiles masked per element.
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  // THREE rotating K/Vt buffers: tile t is read from buf t%3 while t+1 is
-  // written into (t+1)%3, whose previous readers (tile t-2) finished two
-  // barriers ago -> ONE barrier per tile instead of two.
-  auto kbuf = [&](int i) { return smem + (size_t)i * K_TILE_B; };
-  auto vbuf = [&](int i) {
-    return smem + 3 * K_TILE_B + (size_t)i * VT_TILE_B;
-  };
+// window > 0: Mistral-style sliding window — q row i attends kv rows
+// [i - window + 1, i] (causal implied); whole tiles outside the band are
+// skipped, boundary tiles masked per element.
+__global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FwdArgs a) {
+  // two key and two value tiles; apart by name, so that a read of one need
+  // not wait for the words on their way into the other
+  __shared__ __attribute__((aligned(16))) char k0[FA_TILE_B], k1[FA_TILE_B];
+  __shared__ __attribute__((aligned(16))) char v0[FA_TILE_B], v1[FA_TILE_B];
 
-  const int lane = threadIdx.x & 63;
-  // readfirstlane: provably wave-uniform -> scalar branches for the
-  // per-wave activity guards instead of exec-mask divergence (T20)
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 31;       // q column owned by this lane
-  const int hi = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // readfirstlane: provably wave-uniform -> scalar branches
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hi = lane >> 5;
+  const int S = a.S, window = a.window;
 
   // Dispatch mapping (causal LPT): heads on x, q-blocks on y REVERSED so
-  // the largest-causal-work blocks launch first.  With x = q-block the
-  // hardware pairs CU c with the SAME q-block index every occupancy round
-  // (512 WGs / 256 CUs at 1 WG/CU) -> worst CUs do ~1.9x the mean causal
-  // work while others idle; biggest-first lets early finishers absorb the
-  // small diagonal blocks (greedy LPT, near-ideal pairing).
-  const int qblk = (int)(gridDim.y - 1 - blockIdx.y);
-  const int h = blockIdx.x;
-  const int b = blockIdx.z;
-  const int hkv = h / (Hq / Hkv);
-
-  const long q_base = (long)b * q_bs + (long)h * q_hs;
-  const long kv_base_k = (long)b * k_bs + (long)hkv * k_hs;
-  const long kv_base_v = (long)b * v_bs + (long)hkv * v_hs;
-
-  const int q0 = qblk * FA_QBLK;
-  const int qw0 = q0 + wid * FA_QW;      // this wave's first q row
+  // the largest-causal-work blocks launch first and early finishers absorb
+  // the small diagonal blocks.
+  const int q0 = (int)(gridDim.y - 1 - blockIdx.y) * FA_QBLK;
+  const int h = blockIdx.x, b = blockIdx.z;
+  const int hkv = h / (a.Hq / a.Hkv);
+  const int qw0 = q0 + wid * 32;         // this wave's first q row
   const int my_q = qw0 + col;            // this lane's q row
-  const int q_row_ld = my_q < S ? my_q : S - 1;
 
-  // ---- Q fragments: 8 chunks of (16 d), each lane 8 bf16 --------------
+  // a negative scale turns the sign of the queries, so that the largest
+  // product is the largest score
+  const uint flip = a.scale < 0.f ? 0x80008000u : 0u;
+  const float s2 = fabsf(a.scale) * LOG2E;
   frag_u qf[8];
+  {
+    const short* src = a.q + b * a.q_bs + h * a.q_hs +
+                       (long)min(my_q, S - 1) * a.q_ss + hi * 8;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const short* src = qp + q_base + (long)q_row_ld * q_ss + c * 16 + hi * 8;
-    qf[c].u4 = *(const uint4v*)src;
+    for (int c = 0; c < 8; ++c) {
+      qf[c].u4 = *(const uint4v*)(src + c * 16);
+      qf[c].u4 ^= flip;
+    }
   }
 
-  // ---- accumulators ----------------------------------------------------
-  f32x16 ot[4] = {};          // O^T: d-block nb, rows d_local, col q
-  float m_run = NEG_INF;      // running max (exp2 domain)
-  float l_run = 0.f;
+  f32x16 ot[4] = {};                     // O^T: d-block, rows d, col q
+  float m_run = NEG_INF;                 // running max (exp2 domain)
+  float l_run = 0.f;                     // sum over this half wave's keys
 
-  const int kv_end = causal ? min(S, q0 + FA_QBLK) : S;
+  const int kv_end = a.causal ? min(S, q0 + FA_QBLK) : S;
   const int ntiles = (kv_end + FA_KV - 1) / FA_KV;
-  // this wave can skip tiles fully above its causal row range
-  const int my_kv_end = causal ? min(S, qw0 + FA_QW) : S;
-  // sliding window: tiles fully below ANY of this wave's rows' windows
-  // are skipped; the whole WG starts at the block's earliest window tile
-  const int my_kv_begin = window > 0 ? max(0, qw0 - window + 1) : 0;
+  // the WG starts at its earliest window tile; [w_begin, w_end) are the tiles
+  // that a row of this wave sees
   const int t_begin = window > 0 ? max(0, q0 - window + 1) / FA_KV : 0;
+  const int w_begin = window > 0 ? max(0, qw0 - window + 1) / FA_KV : 0;
+  const int w_end = ((a.causal ? min(S, qw0 + 32) : S) + FA_KV - 1) / FA_KV;
 
-  const float s2 = scale * LOG2E;
-
-  // ---- staging: thread t owns K/V rows {2rp, 2rp+1} at 16B slot c16 ----
-  // (rp = t>>4 in 0..31, c16 = t&15).  K: 2 x ds_write_b128 swizzled;
-  // V: the row PAIR transposes into 8 x b32 writes (two k-columns per
-  // write) instead of 16 scalar b16 scatters.
-  const int tid = threadIdx.x;
-  const int st_rp = tid >> 4;
-  const int st_c16 = tid & 15;
-  const int st_r0 = 2 * st_rp, st_r1 = 2 * st_rp + 1;
-
-  uint4v kreg[2], vreg[2];
-  auto issue_loads = [&](int t) {
-    int kv0 = t * FA_KV;
-    int rr0 = kv0 + st_r0 < S ? kv0 + st_r0 : S - 1;
-    int rr1 = kv0 + st_r1 < S ? kv0 + st_r1 : S - 1;
-    kreg[0] = *(const uint4v*)(kp + kv_base_k + (long)rr0 * k_ss + st_c16 * 8);
-    kreg[1] = *(const uint4v*)(kp + kv_base_k + (long)rr1 * k_ss + st_c16 * 8);
-    vreg[0] = *(const uint4v*)(vp + kv_base_v + (long)rr0 * v_ss + st_c16 * 8);
-    vreg[1] = *(const uint4v*)(vp + kv_base_v + (long)rr1 * v_ss + st_c16 * 8);
-  };
-
-  auto write_tile = [&](int buf) {
-    *(uint4v*)(kbuf(buf) + swz16(st_r0, st_c16 * 16)
-               + st_r0 * (FA_D * 2)) = kreg[0];
-    *(uint4v*)(kbuf(buf) + swz16(st_r1, st_c16 * 16)
-               + st_r1 * (FA_D * 2)) = kreg[1];
-    union { uint4v u; short s[8]; } a, b;
-    a.u = vreg[0];
-    b.u = vreg[1];
+  // Tiles go from memory into LDS as they are, 16 bytes a lane; the rotation
+  // of a row's slots (bank conflicts) is done on the source.  Keys are read
+  // as rows, values by transposing reads.  Both rotations repeat after 16
+  // rows, so the rows st_r + 16 i of a thread have the same.
+  const int st_r = tid >> 4, st_s = tid & 15;
+  const short* kg = a.k + b * a.k_bs + hkv * a.k_hs + (long)st_r * a.k_ss +
+                    (st_s ^ row_turn(st_r)) * 8;
+  const short* vg = a.v + b * a.v_bs + hkv * a.v_hs + (long)st_r * a.v_ss +
+                    (st_s ^ row_turn(st_r)) * 8;
+  auto issue = [&](const short* g, long ss, int t, char* lds) {
+    const int kv0 = t * FA_KV;
+    const short* src = g + kv0 * ss;
+    const long step = 16 * ss;
+    if (kv0 + FA_KV <= S) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      int d = st_c16 * 8 + j;
-      uint pair = ((uint)(unsigned short)a.s[j]) |
-                  (((uint)(unsigned short)b.s[j]) << 16);
-      *(uint*)(vbuf(buf) + d * (VT_PITCH * 2) + st_r0 * 2) = pair;
+      for (int i = 0; i < 4; ++i, src += step)
+        __builtin_amdgcn_global_load_lds(
+            (global_ptr)src, (lds_ptr)(lds + (i * 256 + wid * 64) * 16), 16, 0, 0);
+    } else {                   // rows past the end read the last one
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long back = max(0, kv0 + 16 * i + st_r - (S - 1));
+        __builtin_amdgcn_global_load_lds(
+            (global_ptr)(src + i * step - back * ss),
+            (lds_ptr)(lds + (i * 256 + wid * 64) * 16), 16, 0, 0);
+      }
     }
   };
+  const int kx = row_lane(col, hi), vx = tr_lane(lane);
 
-  issue_loads(t_begin);
-  write_tile(t_begin % 3);
-  __syncthreads();
-
-  for (int t = t_begin; t < ntiles; ++t) {
-    const int kv0 = t * FA_KV;
-    const int cur = t % 3;
-    if (t + 1 < ntiles) issue_loads(t + 1);
-
-    const bool wave_active = kv0 < my_kv_end &&
-        (window <= 0 || kv0 + FA_KV > my_kv_begin);
-    if (wave_active) {
-      // ---- QK^T: S^T[k][q] = sum_d K[k][d] Q^T[d][q] ------------------
-      // All 16 K fragments are prefetched into registers BEFORE the mfma
-      // burst (T3/T4): with ds_reads issued only 1-2 mfmas ahead the
-      // compiler emits lgkmcnt(0) waits before every other mfma and the
-      // ~64-cycle LDS latency stalls the matrix pipe; batching the reads
-      // turns those into counted waits that are already satisfied.
-      f32x16 acc[2] = {};
-      frag_u kfr[2][8];
+  // S^T[k][q] = K Q^T
+  auto scores = [&](f32x16* s, const char* kbuf) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) s[kb] = f32x16{};
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        int row = col + 32 * kb;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          kfr[kb][c].u4 = *(const uint4v*)(kbuf(cur) + row * (FA_D * 2)
-                                           + swz16(row, (c * 16 + hi * 8) * 2));
+        frag_u kf;
+        kf.u4 = *(const uint4v*)(kbuf + (kx ^ (c * 32)) + kb * 8192);
+        s[kb] = mfma_bf16(kf.bf, qf[c].bf, s[kb]);
       }
-      __builtin_amdgcn_s_setprio(1);  // T5: keep the matrix pipe fed
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          acc[kb] = mfma_bf16(kfr[kb][c].bf, qf[c].bf, acc[kb]);
-      __builtin_amdgcn_s_setprio(0);
-
-      // ---- online softmax (exp2 domain), lane-local per q row ---------
-      float sc[2][16];
-      const bool need_mask =
-          (causal && kv0 + FA_KV > qw0) || (kv0 + FA_KV > S) ||
-          (window > 0 && kv0 < qw0 + FA_QW - 1 - window + 1 + FA_KV);
+  };
+  // masks of tile t (only on a boundary) and the running maximum
+  auto level = [&](f32x16* s, int t) {
+    const int kv0 = t * FA_KV;
+    if ((a.causal && kv0 + FA_KV - 1 > qw0) || kv0 + FA_KV > S ||
+        (window > 0 && kv0 <= qw0 + 31 - window)) {
+      asm volatile("");        // a branch: not selects on every tile
+      // key j + 4 hi of the tile is seen if first < j <= last
+      const int i0 = my_q - kv0;
+      const int last = min(a.causal ? i0 : FA_KV, S - 1 - kv0) - 4 * hi;
+      const int first = (window > 0 ? i0 - window : -1) - 4 * hi;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          float v = acc[kb][r] * s2;
-          if (need_mask) {
-            int kg = kv0 + 32 * kb + acc_row(r, hi);
-            if ((causal && kg > my_q) || kg >= S ||
-                (window > 0 && kg <= my_q - window)) v = NEG_INF;
-          }
-          sc[kb][r] = v;
+          const int j = 32 * kb + acc_row(r, 0);
+          s[kb][r] = j > last || j <= first ? -INFINITY : s[kb][r];
         }
-
-      float mt = NEG_INF;
+    }
+    float mt = -INFINITY;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sc[kb][r]);
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));  // combine partner half
-
-      float m_new = fmaxf(m_run, mt);
-      // m_eff floor: when a lane's rows are ALL masked so far, m_new is
-      // -1e30 and exp2(sc - m_new) would be exp2(0)=1 for masked scores;
-      // the floor keeps those at exp2(-9.9e29) = 0.
-      float m_eff = fmaxf(m_new, -1e28f);
-      float alpha = __builtin_amdgcn_exp2f(m_run - m_eff);  // 0 when m_run=-1e30
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[kb][r]);
+    mt = max_halves(mt) * s2;
+    if (__ballot(mt > m_run)) {
+      const float m_new = fmaxf(m_run, mt);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
-
-      float psum = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float p = __builtin_amdgcn_exp2f(sc[kb][r] - m_eff);
-          sc[kb][r] = p;
-          psum += p;
-        }
-      psum += __shfl_xor(psum, 32, 64);
-      l_run = l_run * alpha + psum;
-
+      l_run *= alpha;
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) ot[nb] *= alpha;
-
-      // ---- pack P -> PV B-fragments (4 chunks of 16 k) ----------------
-      frag_u pf[4];
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int cc = 0; cc < 2; ++cc) {
-          uint b0 = pack_bf16x2(sc[kb][8 * cc + 0], sc[kb][8 * cc + 1]);
-          uint b1 = pack_bf16x2(sc[kb][8 * cc + 2], sc[kb][8 * cc + 3]);
-          uint b2 = pack_bf16x2(sc[kb][8 * cc + 4], sc[kb][8 * cc + 5]);
-          uint b3 = pack_bf16x2(sc[kb][8 * cc + 6], sc[kb][8 * cc + 7]);
-          {
-            auto r01 = __builtin_amdgcn_permlane32_swap(b0, b2, false, false);
-            b0 = r01[0]; b2 = r01[1];
-          }
-          {
-            auto r23 = __builtin_amdgcn_permlane32_swap(b1, b3, false, false);
-            b1 = r23[0]; b3 = r23[1];
-          }
-          frag_u& f = pf[2 * kb + cc];
-          f.u[0] = b0; f.u[1] = b1; f.u[2] = b2; f.u[3] = b3;
-        }
-
-      // ---- PV: O^T[d][q] += V^T[d][k] P^T[k][q] -----------------------
-      // Same batched-prefetch structure as QK, two d-blocks at a time
-      // (8 fragments = 32 VGPRs in flight).
-#pragma unroll
-      for (int np = 0; np < 2; ++np) {
-        frag_u vfr[2][4];
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-          int d = 32 * (2 * np + ni) + col;
-#pragma unroll
-          for (int c16 = 0; c16 < 4; ++c16)
-            vfr[ni][c16].u4 = *(const uint4v*)(vbuf(cur) + d * (VT_PITCH * 2)
-                                               + (c16 * 16 + hi * 8) * 2);
-        }
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-          for (int c16 = 0; c16 < 4; ++c16)
-            ot[2 * np + ni] =
-                mfma_bf16(vfr[ni][c16].bf, pf[c16].bf, ot[2 * np + ni]);
-        __builtin_amdgcn_s_setprio(0);
-      }
     }
+  };
+  // weights, as fragments of P^T: the accumulator's order of keys is that in
+  // which the transposing reads give the values
+  auto weigh = [&](f32x16* s, frag_u* pf) {
+    float ps = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] * s2 - m_run);
+        ps += s[kb][r];
+      }
+    l_run += ps;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        pf[c].u[u] = pack_bf16x2(s[c >> 1][8 * (c & 1) + 2 * u],
+                                 s[c >> 1][8 * (c & 1) + 2 * u + 1]);
+  };
+  // O^T[d][q] += V^T P^T
+  auto gather = [&](const frag_u* pf, char* vbuf) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        union { tr4 t[2]; bf16x8 bf; } vf;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_tr4)(vbuf + (vx ^ (nb * 64 + u * 32)) + c * 4096 + u * 2048));
+        ot[nb] = mfma_bf16(vf.bf, pf[c].bf, ot[nb]);
+      }
+  };
+  // Tile t's weights and values, while the next tile's scores are made: the
+  // products of one run beside the exponentials of the other.
+  auto step = [&](int t, f32x16* s, f32x16* next, const char* kbuf, char* vbuf) {
+    const bool now = t >= w_begin && t < w_end;
+    const bool then = t + 1 >= w_begin && t + 1 < w_end;
+    frag_u pf[4];
+    if (now) {
+      level(s, t);
+      scores(next, kbuf);      // past the wave's last tile they are not used
+      weigh(s, pf);
+      gather(pf, vbuf);
+      // four reads ahead; then a product, a read and exponentials in turn;
+      // then the products with the values and what is left
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      }
+    } else if (then) {
+      scores(next, kbuf);
+    }
+  };
 
-    if (t + 1 < ntiles) write_tile((t + 1) % 3);
+  f32x16 sa[2], sb[2];
+  issue(kg, a.k_ss, t_begin, k0);
+  issue(vg, a.v_ss, t_begin, v0);
+  if (t_begin + 1 < ntiles) issue(kg, a.k_ss, t_begin + 1, k1);
+  __syncthreads();             // also waits for the words on their way
+  if (t_begin >= w_begin && t_begin < w_end) scores(sa, k0);
+  __syncthreads();
+  for (int t = t_begin; t < ntiles; t += 2) {
+    // keys of t + 1 and values of t are there
+    if (t + 2 < ntiles) issue(kg, a.k_ss, t + 2, k0);
+    if (t + 1 < ntiles) issue(vg, a.v_ss, t + 1, v1);
+    step(t, sa, sb, k1, v0);
+    __syncthreads();
+    if (t + 1 >= ntiles) break;
+    if (t + 3 < ntiles) issue(kg, a.k_ss, t + 3, k1);
+    if (t + 2 < ntiles) issue(vg, a.v_ss, t + 2, v0);
+    step(t + 1, sb, sa, k0, v1);
     __syncthreads();
   }
 
   // ---- epilogue: normalize, store O (transposed back) and LSE ---------
+  const float l = l_run + __shfl_xor(l_run, 32, 64);
   if (my_q >= S) return;
-  float inv_l = l_run > 0.f ? 1.f / l_run : 0.f;
-  long o_row = (long)b * o_bs + (long)h * o_hs + (long)my_q * o_ss;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  short* dst = a.o + b * a.o_bs + h * a.o_hs + my_q * a.o_ss;
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
+  for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      int d = 32 * nb + 8 * rg + 4 * hi;
-      uint w0 = pack_bf16x2(ot[nb][4 * rg + 0] * inv_l,
-                            ot[nb][4 * rg + 1] * inv_l);
-      uint w1 = pack_bf16x2(ot[nb][4 * rg + 2] * inv_l,
-                            ot[nb][4 * rg + 3] * inv_l);
-      uint2 st = {w0, w1};
-      *(uint2*)(op + o_row + d) = st;
-    }
-  }
-  if (hi == 0 && lsep) {
-    // natural-log LSE: scores were in exp2 domain
-    lsep[(long)(b * Hq + h) * S + my_q] =
-        m_run * 0.6931471805599453f + __logf(l_run);
-  }
-}
-
-extern "C" void flash_attn_fwd(const void* q, const void* k, const void* v,
-                               void* out, void* lse, int B, int Hq, int Hkv,
-                               int S, float scale, int causal,
-                               hipStream_t stream) {
-  dim3 grid(Hq, (S + FA_QBLK - 1) / FA_QBLK, B);
-  size_t lds = 3 * (K_TILE_B + VT_TILE_B);
-  flash_fwd_kernel<<<grid, 512, lds, stream>>>(
-      (const short*)q, (const short*)k, (const short*)v, (short*)out,
-      (float*)lse, B, Hq, Hkv, S, scale, causal, 0,
-      (long)Hq * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hkv * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hkv * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hq * S * FA_D, (long)S * FA_D, FA_D);
+    for (int rg = 0; rg < 4; ++rg)
+      *(uint2*)(dst + 32 * nb + 8 * rg + 4 * hi) =
+          uint2{pack_bf16x2(ot[nb][4 * rg] * inv, ot[nb][4 * rg + 1] * inv),
+                pack_bf16x2(ot[nb][4 * rg + 2] * inv, ot[nb][4 * rg + 3] * inv)};
+  if (hi == 0 && a.lse)        // natural log; scores were in the exp2 domain
+    a.lse[((long)b * a.Hq + h) * S + my_q] =
+        m_run * 0.6931471805599453f + __logf(l);
 }
 
 extern "C" void flash_attn_fwd_strided(
@@ -328,13 +284,30 @@ extern "C" void flash_attn_fwd_strided(
     int B, int Hq, int Hkv, int S, float scale, int causal, int window,
     const long* st, hipStream_t stream) {
   // st = 12 longs: (bs, hs, ss) x (q, k, v, o)
-  dim3 grid(Hq, (S + FA_QBLK - 1) / FA_QBLK, B);
-  size_t lds = 3 * (K_TILE_B + VT_TILE_B);
-  flash_fwd_kernel<<<grid, 512, lds, stream>>>(
-      (const short*)q, (const short*)k, (const short*)v, (short*)out,
-      (float*)lse, B, Hq, Hkv, S, scale, causal, window,
-      st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8],
-      st[9], st[10], st[11]);
+  const FwdArgs a{(const short*)q, (const short*)k, (const short*)v,
+                  (short*)out, (float*)lse, Hq, Hkv, S, causal, window, scale,
+                  st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7],
+                  st[8], st[9], st[10], st[11]};
+  const dim3 grid(Hq, (S + FA_QBLK - 1) / FA_QBLK, B);
+  flash_fwd_kernel<<<grid, 256, 0, stream>>>(a);
+}
+
+static void launch_fwd_dense(const void* q, const void* k, const void* v,
+                             void* out, void* lse, int B, int Hq, int Hkv,
+                             int S, float scale, int causal, int window,
+                             hipStream_t stream) {
+  const long h = (long)S * FA_D;
+  const long st[12] = {Hq * h, h, FA_D, Hkv * h, h, FA_D,
+                       Hkv * h, h, FA_D, Hq * h, h, FA_D};
+  flash_attn_fwd_strided(q, k, v, out, lse, B, Hq, Hkv, S, scale, causal,
+                         window, st, stream);
+}
+
+extern "C" void flash_attn_fwd(const void* q, const void* k, const void* v,
+                               void* out, void* lse, int B, int Hq, int Hkv,
+                               int S, float scale, int causal,
+                               hipStream_t stream) {
+  launch_fwd_dense(q, k, v, out, lse, B, Hq, Hkv, S, scale, causal, 0, stream);
 }
 
 extern "C" void flash_attn_fwd_window(const void* q, const void* k,
@@ -342,13 +315,5 @@ extern "C" void flash_attn_fwd_window(const void* q, const void* k,
                                       int B, int Hq, int Hkv, int S,
                                       float scale, int window,
                                       hipStream_t stream) {
-  dim3 grid(Hq, (S + FA_QBLK - 1) / FA_QBLK, B);
-  size_t lds = 3 * (K_TILE_B + VT_TILE_B);
-  flash_fwd_kernel<<<grid, 512, lds, stream>>>(
-      (const short*)q, (const short*)k, (const short*)v, (short*)out,
-      (float*)lse, B, Hq, Hkv, S, scale, 1, window,
-      (long)Hq * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hkv * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hkv * S * FA_D, (long)S * FA_D, FA_D,
-      (long)Hq * S * FA_D, (long)S * FA_D, FA_D);
+  launch_fwd_dense(q, k, v, out, lse, B, Hq, Hkv, S, scale, 1, window, stream);
 }

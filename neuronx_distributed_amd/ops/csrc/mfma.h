@@ -40,6 +40,15 @@ __device__ __forceinline__ uint pack_bf16x2(float lo, float hi) {
       uint, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 
+// the larger of a lane's value and that of its partner in the other half of
+// the wave (no LDS round trip)
+__device__ __forceinline__ float max_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x),
+                                                  __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // XOR swizzle: spread 16B slots of a row-major LDS tile over banks
 // (cdna_hip_programming.md §6 G4: byte ^= (row&7)<<4)
 __device__ __forceinline__ int swz(int row, int byte_in_row) {

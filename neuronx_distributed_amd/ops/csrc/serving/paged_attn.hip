@@ -591,18 +591,6 @@ struct TilesArgs {
   ScoreArgs mod;            // its gate is one number a head
 };
 
-// The 16-byte slots of a key row are rotated within groups of eight, so that
-// consecutive rows of one column spread over the banks; those of a value row
-// in pieces of four, which a transposing read takes from four rows at once.
-template <int SLOTS>
-__device__ __forceinline__ int key_turn(int row) {
-  return (SLOTS % 16 == 0 ? row : row >> 1) & 7;
-}
-template <int SLOTS>
-__device__ __forceinline__ int value_turn(int row) {
-  return (SLOTS % 16 == 0 ? row & 3 : (row >> 1) & 1) << 2;
-}
-
 // MOD: 0 plain scores, 1 with a distance bias, 2 with a soft cap (and the bias,
 // if there is one); a sink and the gates are handled in all.
 template <int DK, int DE, int NP, bool SHARED, int MOD>

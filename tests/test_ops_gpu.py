@@ -533,6 +533,39 @@ def test_flash_attn_sliding_window(B, Hq, Hkv, S, W):
     _cmp(out, ref, atol=3e-2, rtol=3e-2, name=f"window S={S} W={W}")
 
 
+@pytest.mark.parametrize("S,window,causal", [
+    (1, 0, True), (31, 0, True), (64, 0, True), (65, 0, True),
+    (127, 0, False), (128, 0, True), (129, 0, True), (191, 0, False),
+    (257, 0, True), (300, 33, True), (513, 64, True), (640, 200, True),
+])
+@pytest.mark.parametrize("Hq,Hkv,scale,offset", [
+    (4, 2, None, 0), (2, 2, -0.05, 0), (3, 1, 0.2, 1)])
+def test_flash_attn_tile_edges(S, window, causal, Hq, Hkv, scale, offset):
+    """Forward and backward at the edges of the 32-row waves, 64-key tiles and
+    128-row workgroups; a scale of either sign; rows that start between two
+    16-byte words (``offset`` elements into their storage)."""
+    torch.manual_seed(S + Hq)
+    B, D = 2, 128
+
+    def make(h):
+        n = B * S * h * D
+        t = torch.randn(n + offset, device="cuda").bfloat16()[offset:]
+        return t.view(B, S, h, D).transpose(1, 2).requires_grad_(True)
+
+    q, k, v = make(Hq), make(Hkv), make(Hkv)
+    dy = make(Hq).detach()
+    out = ops.flash_attn(q, k, v, causal, scale, window)
+    got = (out, *torch.autograd.grad(out, (q, k, v), dy))
+    qr, kr, vr = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+    ref = _torch_reference(qr, kr, vr, causal, scale, window or None)
+    want = (ref, *torch.autograd.grad(ref, (qr, kr, vr), dy.float()))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        # weights, their gradients and the result are rounded to bf16, 2^-9
+        # each; gradients that vanish leave the rounding of their summands
+        bound = 3 * 2.0 ** -9 * (b.norm() + 0.05 * b.numel() ** 0.5)
+        assert (a.float() - b).norm() <= bound, name
+
+
 def test_add_rmsnorm_train_matches_unfused_autograd():
     """Training fused add+RMSNorm (fwd + the dpass-folding backward) vs
     the unfused bf16 add -> ops.rmsnorm chain: forward outputs equal and
