@@ -143,7 +143,8 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
         return _block_bwd_masked(q, k, v, out, dout, lse, scale, 0, window)
     if q.is_cuda:
         import ctypes
-        from ..ops import _fa_operand, _fa_strides, _ptr, _require_lib, _stream
+        from ..ops import (_fa_alloc_dkv, _fa_operand, _fa_strides,
+                           _fa_sum_replicas, _ptr, _require_lib, _stream)
 
         lib = _require_lib()
         B, Hq, S, D = q.shape
@@ -152,8 +153,7 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
         dq = torch.empty_like(q)
         qc, kc, vc, oc, doc = (_fa_operand(t.contiguous())
                                for t in (q, k, v, out, dout))
-        dk_pq = torch.empty(B, Hq, S, D, dtype=q.dtype, device=q.device)
-        dv_pq = torch.empty(B, Hq, S, D, dtype=q.dtype, device=q.device)
+        dk_pq, dv_pq = _fa_alloc_dkv(kc, vc, Hq)
         lib.flash_attn_bwd_strided(
             _ptr(qc), _ptr(kc), _ptr(vc), _ptr(oc), _ptr(doc),
             _ptr(lse.contiguous()), _ptr(delta), _ptr(dq), _ptr(dk_pq),
@@ -162,12 +162,7 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
             ctypes.c_int(1 if causal else 0),
             ctypes.c_int(int(window) if window else 0),
             _fa_strides(qc, kc, vc, oc, doc, dq, dk_pq, dv_pq), _stream())
-        rep = Hq // Hkv
-        if rep > 1:
-            dk = dk_pq.view(B, Hkv, rep, S, D).float().sum(2).to(q.dtype)
-            dv = dv_pq.view(B, Hkv, rep, S, D).float().sum(2).to(q.dtype)
-        else:
-            dk, dv = dk_pq, dv_pq
+        dk, dv = _fa_sum_replicas(dk_pq, dv_pq, kc, vc)
         return dq, dk, dv
     B, Hq, S, D = q.shape
     Hkv = k.shape[1]
