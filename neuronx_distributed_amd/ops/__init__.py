@@ -425,16 +425,22 @@ def flash_attn_available() -> bool:
     return lib is not None and hasattr(lib, "flash_attn_fwd")
 
 
-def _fa_operand(t):
+def _fa_ok_layout(t) -> bool:
     """The flash kernels take any (batch, head, seq) strides with a DENSE
     last dim — transpose views of BSHD activations go in with no copy.  Rows
-    are moved in 16-byte words, so every row has to start at one."""
+    are moved in 16-byte words, so the strides are whole numbers of them."""
     b, h, s, d = t.stride()
-    if d == 1 and not (b | h | s) & 7 and not t.data_ptr() & 15:
-        return t
-    if d != 1 or any(st & 7 for st, n in zip((b, h, s), t.shape) if n > 1):
+    if d != 1:
+        return False
+    return not (b | h | s) & 7 or not any(
+        st & 7 for st, n in zip((b, h, s), t.shape) if n > 1)
+
+
+def _fa_operand(t):
+    """``t`` in a layout that the kernels take, at a 16-byte boundary."""
+    if not _fa_ok_layout(t):
         t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+    return t.clone() if t.data_ptr() & 15 else t
 
 
 def _fa_strides(*tensors):
