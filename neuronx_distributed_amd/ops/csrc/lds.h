@@ -10,13 +10,17 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef short tr4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr4* lds_tr4;
 
-// The 16-byte slots of a key row are rotated within groups of eight, so that
-// consecutive rows of one column spread over the banks; those of a value row
-// in pieces of four, which a transposing read takes from four rows at once.
+// The 16-byte slots of a key row are rotated, so that consecutive rows of one
+// column spread over the banks: all 16 of a row of 256 bytes (16 lanes are
+// served at once), else within groups of eight; those of a value row in pieces
+// of four, which a transposing read takes from four rows at once.
 template <int SLOTS>
 __device__ __forceinline__ int key_turn(int row) {
-  return (SLOTS % 16 == 0 ? row : row >> 1) & 7;
+  return SLOTS == 16 ? row & 15 : (SLOTS % 16 == 0 ? row : row >> 1) & 7;
 }
+// after how many fragments of two slots the rotation repeats
+template <int SLOTS> struct KeySlots { static constexpr int steps = 4; };
+template <> struct KeySlots<16> { static constexpr int steps = 8; };
 template <int SLOTS>
 __device__ __forceinline__ int value_turn(int row) {
   return (SLOTS % 16 == 0 ? row & 3 : (row >> 1) & 1) << 2;

@@ -568,6 +568,14 @@ extern "C" int sv_attn_rows(const RowsArgs* a, int vec, int f32,
 // {4 hi + 0..3, 8 + 4 hi + 0..3} of a 16-key chunk is used as the
 // contraction order of P V, and V^T is read from LDS in the same order
 // (transposing loads).
+//
+// Bound by the matrix cores and by the vector work of the splits beside them:
+// four products a tile where plain attention has two, which run at about 1.1
+// PFLOP/s (a large matrix product: 1.3 to 1.5).  6000 tokens of three portions
+// behind up to 4096, 32/8 heads: 621 -> 585 us with the next tile's scores
+// beside this tile's exponentials, page numbers read two tiles ahead, keys
+// rotated over all banks, and a maximum that lags.  An explicit order of
+// products and vector work took 630, splits by v_dot2c_f32_bf16 616.
 // ---------------------------------------------------------------------------
 //
 // A key may end in columns that all heads share (kr): the rotated part of
@@ -590,6 +598,10 @@ struct TilesArgs {
   float scale;
   ScoreArgs mod;            // its gate is one number a head
 };
+
+// The running maximum may lag behind by this much (in log 2): O is rescaled only
+// when a row outgrows it.  The weights are 32-bit either way.
+#define TILES_LAG 8.f
 
 // MOD: 0 plain scores, 1 with a distance bias, 2 with a soft cap (and the bias,
 // if there is one); a sink and the gates are handled in all.
@@ -617,6 +629,18 @@ attn_tiles_kernel(TilesArgs a) {
   const int my_pos = p0 + my;
   const int D = a.D, E = a.E;
 
+  // A factor below zero turns the sign of the queries, so that the largest
+  // product is the largest score; one of zero is as good as a tiny one, which
+  // leaves a masked score at minus infinity.
+  const float factor = a.scale * SV_LOG2E *
+      (a.mod.temp ? bits2f(((const short*)a.mod.temp)[h]) : 1.f);
+  const uint flip = MOD == 0 && factor < 0.f ? 0x80008000u : 0u;
+  const float s2 = MOD == 0 ? fmaxf(fabsf(factor), 1e-37f) : factor;
+  const float slope = MOD && a.mod.slope ? a.mod.slope[h] * SV_LOG2E : 0.f;
+  // tanh(x) = 1 - 2 / (1 + e^2x), with x in units of log 2 / cap
+  const float cap2 = MOD == 2 ? a.mod.cap * SV_LOG2E : 0.f;
+  const float in_cap = MOD == 2 ? 2.f / a.mod.cap : 0.f;
+
   frag_u qf[NC];
   {
     const short* src =
@@ -625,17 +649,13 @@ attn_tiles_kernel(TilesArgs a) {
     for (int c = 0; c < NC; ++c) {
       const int d = c * 16 + hi * 8;
       qf[c].u4 = d < D ? *(const uint4v*)(src + d) : uint4v{0, 0, 0, 0};
+      qf[c].u4 ^= flip;
     }
   }
 
   f32x16 ot[NB] = {};
-  float m_run = NEG_BIG, l_run = 0.f;
-  const float s2 = a.scale * SV_LOG2E *
-      (a.mod.temp ? bits2f(((const short*)a.mod.temp)[h]) : 1.f);
-  const float slope = MOD && a.mod.slope ? a.mod.slope[h] * SV_LOG2E : 0.f;
-  // tanh(x) = 1 - 2 / (1 + e^2x), with x in units of log 2 / cap
-  const float cap2 = MOD == 2 ? a.mod.cap * SV_LOG2E : 0.f;
-  const float in_cap = MOD == 2 ? 2.f / a.mod.cap : 0.f;
+  float m_run = NEG_BIG;
+  float l_run = 0.f;                 // over this half wave's keys
 
   const int q_hi = p0 + nrow - 1;
   const int t_hi = q_hi / SV_PAGE;
@@ -649,12 +669,11 @@ attn_tiles_kernel(TilesArgs a) {
   // 32-bit within a page
   const int krow = (int)a.krow, vrow = (int)a.vrow, rrow = (int)a.rrow;
   auto tile_of = [&](int n) { return n < nk ? n : t_lo + n - nk; };
-  // Ask for the rows of a tile: a wave's 64 slots of 16 bytes follow each
+  auto page_of = [&](int n) { return bt[tile_of(min(n, ntiles - 1))]; };
+  // Ask for the rows of a page: a wave's 64 slots of 16 bytes follow each
   // other in LDS, so the rotation of a row's slots is done on the source.
-  auto issue = [&](int n, char* kd, char* vd) {
-    const long page = bt[tile_of(n)];
+  auto issue_k = [&](long page, char* kd) {
     const short* kb = a.kc + page * a.kpage + g * a.khead;
-    const short* vb = a.vc + page * a.vpage + g * a.vhead;
     const short* rb = SHARED ? a.kr + page * SV_PAGE * rrow - a.DS : nullptr;
 #pragma unroll
     for (int p = 0; p < CK / 4; ++p) {
@@ -666,6 +685,9 @@ attn_tiles_kernel(TilesArgs a) {
                                            : kb + (r * krow + c)),
           (lds_ptr)(kd + (p * 256 + wid * 64) * 16), 16, 0, 0);
     }
+  };
+  auto issue_v = [&](long page, char* vd) {
+    const short* vb = a.vc + page * a.vpage + g * a.vhead;
 #pragma unroll
     for (int p = 0; p < CV / 4; ++p) {
       const int it = p * 256 + tid, r = it / CV;
@@ -678,130 +700,139 @@ attn_tiles_kernel(TilesArgs a) {
   };
   // this lane's part of the addresses in a tile (bytes): slot 2 c + hi of key
   // row col; a transposing read, where 16 lanes turn 4 keys by 16 columns
-  int kx[4];
+  int kx[KeySlots<CK>::steps];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < KeySlots<CK>::steps; ++c)
     kx[c] = col * KP + ((2 * c + hi) ^ key_turn<CK>(col)) * 16;
   const int tr_key = 4 * hi + ((lane & 15) >> 2);
   const int vx = (tr_key * DE + ((lane >> 4) & 1) * 16 + (lane & 3) * 4 +
                   value_turn<CV>(tr_key) * 8) * 2;
 
-  auto attend = [&](int n, const char* kbuf, char* vbuf) {
-    const int kv0 = tile_of(n) * SV_PAGE;
-    const bool active = wid * 32 < nrow && kv0 <= w_hi &&
-        (a.window <= 0 || kv0 < a.keep || kv0 + SV_PAGE - 1 > w_lo - a.window);
-    if (!active) return;
-
-    f32x16 acc[2] = {};
+  // S^T = K Q^T
+  auto scores = [&](f32x16* s, const char* kbuf) __attribute__((always_inline)) {
+    s[0] = s[1] = f32x16{};
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
+        constexpr int M = KeySlots<CK>::steps;
         frag_u kf;
-        kf.u4 = *(const uint4v*)(kbuf + kx[c & 3] + (c >> 2) * 128 +
+        kf.u4 = *(const uint4v*)(kbuf + kx[c % M] + (c / M) * M * 32 +
                                  kb * 32 * KP);
-        acc[kb] = mfma_bf16(kf.bf, qf[c].bf, acc[kb]);
+        s[kb] = mfma_bf16(kf.bf, qf[c].bf, s[kb]);
       }
-    // the reads run two chunks ahead
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+  };
+  // scores of tile n as they enter the softmax, and the running maximum
+  auto level = [&](int n, f32x16* s) __attribute__((always_inline)) {
+    const int kv0 = tile_of(n) * SV_PAGE;
+    const int i0 = my_pos - kv0 - 4 * hi;      // of this lane's key 0
+    if (MOD) {
 #pragma unroll
-    for (int c = 0; c < NC - 2; ++c) {
-      __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      for (int kb = 0; kb < 2; ++kb) s[kb] *= s2;
+      if (MOD == 2)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[kb][r] = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(
+                1.f + __builtin_amdgcn_exp2f(s[kb][r] * in_cap));
+      if (MOD == 1 || slope != 0.f)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[kb][r] -= slope * (float)(i0 - 32 * kb - acc_row(r, 0));
     }
-    __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
-
-    const bool masked = kv0 + SV_PAGE - 1 > w_lo ||
-        (a.window > 0 && w_hi - kv0 >= a.window &&
-         kv0 + SV_PAGE > a.keep);
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) acc[kb] *= s2;
-    const int i0 = my_pos - kv0;               // keys up to i0 are not ahead
-    if (MOD == 2)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[kb][r] = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(
-              1.f + __builtin_amdgcn_exp2f(acc[kb][r] * in_cap));
-    if (MOD == 1 || (MOD == 2 && slope != 0.f))
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[kb][r] -= slope * (float)(i0 - 32 * kb - acc_row(r, hi));
-    if (masked) {
+    if (kv0 + SV_PAGE - 1 > w_lo ||
+        (a.window > 0 && w_hi - kv0 >= a.window && kv0 + SV_PAGE > a.keep)) {
+      asm volatile("");          // a branch: not selects on every tile
+      // key j is seen if j <= i0 and (j > first or j < kept)
+      const int first = a.window > 0 ? i0 - a.window : -1 - 4 * hi;
+      const int kept = a.window > 0 ? a.keep - kv0 - 4 * hi : 0;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int j = 32 * kb + acc_row(r, hi);
-          const bool gone = j > i0 || (a.window > 0 && i0 - j >= a.window &&
-                                       kv0 + j >= a.keep);
-          acc[kb][r] = gone ? NEG_BIG : acc[kb][r];
+          const int j = 32 * kb + acc_row(r, 0);
+          const bool gone = j > i0 || (j <= first && j >= kept);
+          s[kb][r] = gone ? -INFINITY : s[kb][r];
         }
     }
-    float mt = NEG_BIG;
+    float mt = -INFINITY;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, acc[kb][r]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float m_new = fmaxf(m_run, mt);
-    const float m_eff = fmaxf(m_new, -1e28f);  // an all-masked row stays 0
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_eff);
-    m_run = m_new;
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[kb][r]);
+    mt = max_halves(mt);
+    if (MOD == 0) mt *= s2;
+    if (__ballot(mt > m_run + TILES_LAG)) {
+      const float m_new = fmaxf(m_run, mt);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) ot[nb] *= alpha;
+    }
+  };
+  auto weigh = [&](f32x16* s) __attribute__((always_inline)) {
     float ps = 0.f;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        acc[kb][r] = __builtin_amdgcn_exp2f(acc[kb][r] - m_eff);
-        ps += acc[kb][r];
+        s[kb][r] = __builtin_amdgcn_exp2f(MOD == 0 ? s[kb][r] * s2 - m_run
+                                                   : s[kb][r] - m_run);
+        ps += s[kb][r];
       }
-    ps += __shfl_xor(ps, 32, 64);
-    l_run = l_run * alpha + ps;
-    if (__ballot(alpha != 1.f)) {
+    l_run += ps;
+  };
+  // O^T += V^T P, 16 keys after 16; the next ones' planes are made beside the
+  // products
+  auto gather = [&](const f32x16* s, char* vbuf) __attribute__((always_inline)) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) ot[nb] *= alpha;
+    for (int c = 0; c < 4; ++c) {
+      frag_u pf[NP];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float x = s[c >> 1][8 * (c & 1) + 2 * u];
+        float y = s[c >> 1][8 * (c & 1) + 2 * u + 1];
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+          const uint w = pack_bf16x2(x, y);
+          pf[z].u[u] = w;
+          x -= __uint_as_float(w << 16);
+          y -= __uint_as_float(w & 0xffff0000u);
+        }
+      }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        union { tr4 t[2]; bf16x8 bf; } vf;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_tr4)(vbuf + (vx ^ (nb * 64)) + (16 * c + 8 * u) * DE * 2));
+#pragma unroll
+        for (int z = 0; z < NP; ++z)
+          ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
+      }
     }
-
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc) {
-        frag_u pf[NP];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          float x = acc[kb][8 * cc + 2 * u], y = acc[kb][8 * cc + 2 * u + 1];
-#pragma unroll
-          for (int z = 0; z < NP; ++z) {
-            const uint w = pack_bf16x2(x, y);
-            pf[z].u[u] = w;
-            x -= __uint_as_float(w << 16);
-            y -= __uint_as_float(w & 0xffff0000u);
-          }
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          union { tr4 t[2]; bf16x8 bf; } vf;
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_tr4)(vbuf + (vx ^ (nb * 64)) +
-                          (32 * kb + 16 * cc + 8 * u) * DE * 2));
-#pragma unroll
-          for (int z = 0; z < NP; ++z)
-            ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int nb = 0; nb < NB - 2; ++nb) {
-          __builtin_amdgcn_sched_group_barrier(0x8, NP, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x8, 2 * NP, 0);
-      }
+  };
+  auto active = [&](int n) {
+    const int kv0 = tile_of(n) * SV_PAGE;
+    return n < ntiles && wid * 32 < nrow && kv0 <= w_hi &&
+        (a.window <= 0 || kv0 < a.keep || kv0 + SV_PAGE - 1 > w_lo - a.window);
+  };
+  // Tile n's weights and values, while the next tile's scores are made: the
+  // products of one run beside the exponentials of the other.
+  auto step = [&](int n, f32x16* s, f32x16* next, const char* kbuf, char* vbuf)
+      __attribute__((always_inline)) {
+    const bool now = active(n);
+    if (now) level(n, s);
+    if (now || active(n + 1)) scores(next, kbuf);
+    if (now) {
+      weigh(s);
+      gather(s, vbuf);
+    }
   };
 
   if (D < DK) {                // columns that no tile writes
@@ -811,19 +842,32 @@ attn_tiles_kernel(TilesArgs a) {
     }
     __syncthreads();
   }
-  issue(0, k0, v0);
+  f32x16 sa[2], sb[2];
+  int pa = page_of(0), pb = page_of(1), pc = page_of(2);
+  issue_k(pa, k0);
+  issue_v(pa, v0);
+  if (ntiles > 1) issue_k(pb, k1);
   __syncthreads();             // also waits for the words on their way
+  if (active(0)) scores(sa, k0);
+  __syncthreads();
   for (int n = 0; n < ntiles; n += 2) {
-    const bool more = n + 1 < ntiles;
-    if (more) issue(n + 1, k1, v1);
-    attend(n, k0, v0);
+    // keys of n + 1 and values of n are there; pb, pc: pages of n + 1, n + 2
+    const int pd = page_of(n + 3);
+    if (n + 2 < ntiles) issue_k(pc, k0);
+    if (n + 1 < ntiles) issue_v(pb, v1);
+    step(n, sa, sb, k1, v0);
     __syncthreads();
-    if (!more) break;
-    if (n + 2 < ntiles) issue(n + 2, k0, v0);
-    attend(n + 1, k1, v1);
+    if (n + 1 >= ntiles) break;
+    const int pe = page_of(n + 4);
+    if (n + 3 < ntiles) issue_k(pd, k1);
+    if (n + 2 < ntiles) issue_v(pc, v0);
+    step(n + 1, sb, sa, k0, v1);
     __syncthreads();
+    pb = pd;
+    pc = pe;
   }
 
+  l_run += __shfl_xor(l_run, 32, 64);
   if (my >= nrow) return;
   float inv = 1.f / l_run;
   if (a.mod.sink) {

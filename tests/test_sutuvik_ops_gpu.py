@@ -310,6 +310,44 @@ def test_modified_scores(dtype, kind, H, G, D, E):
     _near(got, want[r], dtype, "append")
 
 
+@pytest.mark.parametrize("T,cuts", [(64, (64,)), (65, (1, 64)),
+                                    (449, (129, 320)), (700, (31, 33, 636))])
+@pytest.mark.parametrize("window,keep", [(0, 0), (70, 0), (130, 64)])
+@pytest.mark.parametrize("G,D,E", [(2, 128, 128), (1, 64, 40), (4, 192, 128)])
+def test_tiles_at_their_edges(T, cuts, window, keep, G, D, E):
+    """Prompt tiles whose pages, windows and rows end at borders; factors of
+    the scores below, at and above zero, rising scores."""
+    H = 4
+    q, k, v = (_rand(T, n, m, seed=n + m, dtype=BF16) for n, m in
+               ((H, D), (G, D), (G, E)))
+    k = (k * torch.linspace(0.2, 3, T)[:, None, None]).to(BF16)
+    temp = torch.tensor([1.0, -0.75, 0.0, 2.0]).to(BF16)
+    scale, i = D ** -0.5, torch.arange(T)
+    seen = i[None] <= i[:, None]
+    if window:
+        seen &= (i[:, None] - i[None] < window) | (i[None] < keep)
+    want = []
+    for h in range(H):
+        s = q[:, h].double() @ k[:, h // (H // G)].double().T
+        s = s * scale * temp[h].double()
+        s = s.masked_fill(~seen, -float("inf")).softmax(1)
+        want.append(s @ v[:, h // (H // G)].double())
+    kc, vc, bt = _pages([T], G, D, E, BF16)
+    q, k, v = (x.reshape(T, -1).cuda() for x in (q, k, v))
+    pos = torch.arange(T, dtype=torch.int32, device="cuda")
+    zero, at, got = torch.zeros_like(pos), 0, []
+    for n in cuts:
+        r = slice(at, at + n)
+        tiles = _i32([(0, s, min(128, n - s), at + s)
+                      for s in range(0, n, 128)])
+        got.append(sv.attn_portions(
+            q[r], k[r], v[r], kc, vc, pos[r], zero[r], bt, tiles, H, scale,
+            window, keep, mod=sv.ScoreMod(temp=temp.cuda())))
+        at += n
+    # the result's rounding, 2^-9 of its largest number
+    _near(torch.cat(got), torch.cat(want, 1), BF16, tol=2.0 ** -8)
+
+
 def test_a_far_biased_key_is_not_lost():
     """A key thousands of positions back wins against its distance bias, in a
     prompt tile and when decoding."""
