@@ -19,6 +19,9 @@
 #include "serving.h"
 
 #define NEG_BIG (-1e30f)
+// The running maximum may lag behind by this much (in log 2): O is rescaled only
+// when a row outgrows it.  The weights are 32-bit either way.
+#define TILES_LAG 8.f
 
 // ---------------------------------------------------------------------------
 // append
@@ -451,6 +454,261 @@ attn_rows_kernel(RowsArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same on MFMA, for bf16 heads of 64 or 128.  One workgroup = 4 waves, one
+// query row, up to 16 heads that share their keys, a range of the keys in tiles
+// of 32 (half a page); every wave takes every fourth tile with buffers of its
+// own, so that waves never wait for each other.  Keys go straight into
+// registers as fragments (a lane's 16 bytes of a row), values into LDS, from
+// where transposing reads turn them.  S^T has its keys in the accumulator's
+// rows, which is the order in which the values come; the weights stay 32-bit, in
+// three planes that add up to them.
+//
+// Bound by memory: 8 waves a CU have 16 KB each on their way.  The kernel above
+// spends its time on vector work (a key costs 140 cycles of a wave; here 30).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// the larger of the four lanes 16 apart
+__device__ __forceinline__ float max_quarters(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x),
+                                                  __float_as_uint(x), false,
+                                                  false);
+  return max_halves(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+
+template <bool MOD, int DE>
+__global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
+  constexpr int NC = DE / 32;            // chunks of a key
+  constexpr int NB = DE / 16;            // 16-row blocks of O^T
+  constexpr int CV = DE / 8;             // 16-byte slots of a value row
+  constexpr int VB = 32 * DE * 2;        // bytes of a value tile
+  // a tile a wave each; apart by name, so that a read of one need not wait for
+  // the words on their way into the other
+  __shared__ __attribute__((aligned(16))) char v0[4 * VB], v1[4 * VB];
+  __shared__ float sml[4][16][2];
+
+  const int rep = a.H / a.G, nrc = (rep + 15) / 16;
+  const int split = blockIdx.x % a.splits;
+  const int unit = blockIdx.x / a.splits;
+  const int rc = unit % nrc, g = unit / nrc % a.G, row = unit / nrc / a.G;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, grp = lane >> 4;
+  const int h = g * rep + min(rc * 16 + c16, rep - 1);
+
+  const int i_pos = a.pos[row];
+  const int* bt = a.bt + (long)a.seq[row] * a.MB;
+  const short* kn = (const short*)a.k + row * a.kst + (long)g * DE;
+  const short* vn = (const short*)a.v + row * a.vst + (long)g * DE;
+  if (a.append && split == 0 && rc == 0) {
+    const long page = bt[i_pos / SV_PAGE];
+    const long base = (page * a.G + g) * SV_PAGE + i_pos % SV_PAGE;
+    for (int i = tid; i < DE; i += 256) {
+      ((short*)a.kc)[base * a.kcs + i] = kn[i];
+      ((short*)a.vc)[base * a.vcs + i] = vn[i];
+    }
+  }
+
+  frag_u qf[NC];
+  {
+    const short* src = (const short*)a.q + row * a.qst + (long)h * DE + grp * 8;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) qf[c].u4 = *(const uint4v*)(src + c * 32);
+  }
+  // scores in units of log 2; of the cap, if there is one
+  const float cap = MOD ? a.mod.cap : 0.f;
+  float s2 = cap > 0.f ? a.scale / cap : a.scale * SV_LOG2E;
+  if (MOD && a.mod.temp) s2 *= bits2f(((const short*)a.mod.temp)[h]);
+  const float slope = MOD && a.mod.slope ? a.mod.slope[h] * SV_LOG2E : 0.f;
+
+  // visible tiles as one list: those of the kept first keys, then the window's
+  const int lo = a.window > 0 ? max(0, i_pos - a.window + 1) : 0;
+  const int t_hi = i_pos / 32;
+  const int nk = a.window > 0 ? min((a.keep + 31) / 32, t_hi + 1) : 0;
+  const int t_lo = max(nk, lo / 32);
+  const int total = nk + max(0, t_hi - t_lo + 1);
+  const int per = (total + a.splits - 1) / a.splits;
+  const int n1 = min(total, (split + 1) * per);
+  auto tile_of = [&](int n) { return n < nk ? n : t_lo + n - nk; };
+
+  // Ask for a tile.  Keys past the newest read its row again, and the row's own
+  // key and value come from the projection, also where they are not written
+  // yet.
+  auto issue = [&](int n, frag_u (*kf)[NC], char* vd) __attribute__((always_inline)) {
+    const int t = tile_of(n);
+    const int newest = i_pos - t * 32;   // row of the tile
+    const long base = ((long)bt[t / 2] * a.G + g) * SV_PAGE + (t & 1) * 32;
+    const short* kb = (const short*)a.kc + base * a.kcs;
+    const short* vb = (const short*)a.vc + base * a.vcs;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = i * 16 + c16;
+      const short* src = a.append && r >= newest
+                             ? kn : kb + (long)min(r, newest) * a.kcs;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        kf[i][c].u4 = *(const uint4v*)(src + c * 32 + grp * 8);
+    }
+#pragma unroll
+    for (int p = 0; p < CV / 2; ++p) {
+      const int it = p * 64 + lane, r = it / CV;
+      // pairs of slots are rotated, so that 8 rows of a pair use every bank
+      const int c = (it % CV ^ ((CV == 16 ? r : r >> 1) % (CV / 2)) * 2) * 8;
+      const short* src = a.append && r >= newest
+                             ? vn : vb + (long)min(r, newest) * a.vcs;
+      __builtin_amdgcn_global_load_lds(
+          (global_ptr)(src + c), (lds_ptr)(vd + wid * VB + p * 1024), 16, 0, 0);
+    }
+  };
+  // a transposing read: 16 lanes turn 4 keys by 16 columns
+  const int tr_row = 4 * grp + (c16 >> 2);
+  const int tr_turn = (CV == 16 ? tr_row : tr_row >> 1) % (CV / 2);
+  const int vx = wid * VB + tr_row * DE * 2 + tr_turn * 32 + (c16 & 3) * 8;
+
+  f32x4 o[NB] = {};                      // O^T: rows d, col head
+  float m = NEG_BIG, l = 0.f;            // l: of this lane's keys
+
+  auto attend = [&](int n, const frag_u (*kf)[NC], char* vbuf) __attribute__((always_inline)) {
+    const int t = tile_of(n);
+    f32x4 s[2] = {};
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) s[i] = mfma16(kf[i][c].bf, qf[c].bf, s[i]);
+    const int i0 = i_pos - t * 32 - 4 * grp;   // of this lane's key 0
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      s[i] *= s2;
+      if (MOD) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (cap > 0.f) s[i][r] = cap * SV_LOG2E * tanh_t(s[i][r], short());
+          s[i][r] -= slope * (float)(i0 - 16 * i - r);
+        }
+      }
+    }
+    if (t == t_hi || (a.window > 0 && t * 32 <= i_pos - a.window)) {
+      asm volatile("");
+      const int first = a.window > 0 ? i0 - a.window : -1 - 4 * grp;
+      const int kept = a.window > 0 ? a.keep - t * 32 - 4 * grp : 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * i + r;
+          s[i][r] = j > i0 || (j <= first && j >= kept) ? -INFINITY : s[i][r];
+        }
+    }
+    float mt = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mt = fmaxf(mt, s[i][r]);
+    mt = max_quarters(mt);
+    if (__ballot(mt > m + TILES_LAG)) {
+      const float mn = fmaxf(m, mt);
+      const float al = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= al;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] *= al;
+    }
+    frag_u pf[3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float x = __builtin_amdgcn_exp2f(s[u >> 1][2 * (u & 1)] - m);
+      float y = __builtin_amdgcn_exp2f(s[u >> 1][2 * (u & 1) + 1] - m);
+      l += x + y;
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        const uint w = pack_bf16x2(x, y);
+        pf[z].u[u] = w;
+        x -= __uint_as_float(w << 16);
+        y -= __uint_as_float(w & 0xffff0000u);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      union { tr4 t[2]; bf16x8 bf; } vf;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        vf.t[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_tr4)(vbuf + (vx ^ (b * 32)) + i * 16 * DE * 2));
+#pragma unroll
+      for (int z = 0; z < 3; ++z) o[b] = mfma16(vf.bf, pf[z].bf, o[b]);
+    }
+  };
+  // all words that this wave has asked for are there, and its reads are done
+  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); };
+
+  frag_u ka[2][NC], kb[2][NC];
+  int n = split * per + wid;
+  if (n < n1) issue(n, ka, v0);
+  for (; n < n1; n += 8) {
+    arrived();
+    if (n + 4 < n1) issue(n + 4, kb, v1);
+    attend(n, ka, v0);
+    if (n + 4 >= n1) break;
+    arrived();
+    if (n + 8 < n1) issue(n + 8, ka, v0);
+    attend(n + 4, kb, v1);
+  }
+
+  // the four waves
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (grp == 0) {
+    sml[wid][c16][0] = m;
+    sml[wid][c16][1] = l;
+  }
+  __syncthreads();                       // the tiles have been read
+  float* so = (float*)(wid < 2 ? v0 : v1) + (wid & 1) * 16 * DE;  // [head][DE]
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    *(f32x4*)(so + c16 * DE + ((b * 16 + 4 * grp) ^ (c16 & 7) * 4)) = o[b];
+  __syncthreads();
+  for (int it = tid; it < min(16, rep - rc * 16) * DE; it += 256) {
+    const int r = it / DE, e = it % DE;
+    float mm = NEG_BIG;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sml[w][r][0]);
+    float ll = 0.f, oo = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float c = __builtin_amdgcn_exp2f(sml[w][r][0] - mm);
+      ll += sml[w][r][1] * c;
+      oo += ((const float*)(w < 2 ? v0 : v1))[((w & 1) * 16 + r) * DE +
+                                              (e ^ (r & 7) * 4)] * c;
+    }
+    const int hh = g * rep + rc * 16 + r;
+    if (MOD && a.mod.sink && split == 0) {   // once for all splits
+      const float sink = bits2f(((const short*)a.mod.sink)[hh]) * SV_LOG2E;
+      const float mn = fmaxf(mm, sink);
+      const float c = __builtin_amdgcn_exp2f(mm - mn);
+      ll = ll * c + __builtin_amdgcn_exp2f(sink - mn);
+      oo *= c;
+      mm = mn;
+    }
+    if (MOD && a.mod.gate)
+      oo *= sigmoid_f(bits2f(
+          ((const short*)a.mod.gate)[row * a.mod.gst + hh]));
+    const long rh = (long)row * a.H + hh;
+    if (a.splits == 1) {
+      ((short*)a.out)[rh * DE + e] = f2bits(oo / ll);
+    } else {
+      float* p = a.part + (rh * a.splits + split) * (DE + 2);
+      p[e] = oo;
+      if (e == 0) {
+        p[DE] = mm;
+        p[DE + 1] = ll;
+      }
+    }
+  }
+}
+
 // One workgroup = one query row and head, 64 V columns; its four waves take
 // every fourth split.  At most 64 splits.
 template <typename T, int V>
@@ -512,14 +770,25 @@ extern "C" int sv_attn_merge(const float* part, void* out, long rows,
   return (int)hipGetLastError();
 }
 
+// vec: 1 D, E, strides and bases in 8 elements; 2 on MFMA (bf16, D = E = 64 or
+// 128)
 template <bool MOD, typename T>
 static int launch_rows(const RowsArgs& a, int vec, hipStream_t stream) {
   const int rep = a.H / a.G;
   const int big = a.D > a.E ? a.D : a.E;
   const int rcn = big > 512 ? (rep > 1 ? 2 : 1)
                             : rep >= 8 ? 8 : rep > 2 ? 4 : rep;
-  const int nrc = (rep + rcn - 1) / rcn;
+  const int nrc = vec == 2 ? (rep + 15) / 16 : (rep + rcn - 1) / rcn;
   const long grid = (long)a.rows * a.G * nrc * a.splits;
+  if (vec == 2) {
+    if (sizeof(T) != 2 || a.D != a.E || (a.D != 64 && a.D != 128)) return 1;
+    if (a.D == 64) attn_rows_mfma_kernel<MOD, 64><<<grid, 256, 0, stream>>>(a);
+    else attn_rows_mfma_kernel<MOD, 128><<<grid, 256, 0, stream>>>(a);
+    if (a.splits > 1)
+      return sv_attn_merge(a.part, a.out, (long)a.rows * a.H, a.splits, a.E, 0,
+                           stream);
+    return (int)hipGetLastError();
+  }
 #define AR(L, ...) \
   attn_rows_kernel<MOD, T, L, __VA_ARGS__><<<grid, 256, 0, stream>>>(a)
 #define ARV(L, R) do { if (vec) AR(L, R, true); else AR(L, R, false); } while (0)
@@ -598,10 +867,6 @@ struct TilesArgs {
   float scale;
   ScoreArgs mod;            // its gate is one number a head
 };
-
-// The running maximum may lag behind by this much (in log 2): O is rescaled only
-// when a row outgrows it.  The weights are 32-bit either way.
-#define TILES_LAG 8.f
 
 // MOD: 0 plain scores, 1 with a distance bias, 2 with a soft cap (and the bias,
 // if there is one); a sink and the gates are handled in all.

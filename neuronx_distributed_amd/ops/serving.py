@@ -651,7 +651,10 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
     assert pos.shape[0] == rows and seq.shape[0] == rows
     if window > 0:
         max_keys = min(max_keys, window + keep) if max_keys else window + keep
-    splits = _row_splits(1024, rows * G, max_keys, 128)
+    vec = int(_aligned((D, E), q, k, v))
+    if vec and q.dtype == torch.bfloat16 and D == E and D in (64, 128):
+        vec = 2
+    splits = _row_splits(2048 if vec == 2 else 1024, rows * G, max_keys, 128)
     out = _out(out, rows, heads * E, q)
     part = torch.empty(rows * heads * splits * (E + 2), dtype=torch.float32,
                        device=q.device) if splits > 1 else None
@@ -663,9 +666,8 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
                   rows=rows, H=heads, G=G, D=D, E=E, splits=splits,
                   append=int(append), window=window, keep=keep, scale=scale,
                   mod=_score_args(mod, q, heads))
-    _check(library().sv_attn_rows(ctypes.byref(a),
-                                  int(_aligned((D, E), q, k, v)), _f32(q),
-                                  _stream()), "attn_rows")
+    _check(library().sv_attn_rows(ctypes.byref(a), vec, _f32(q), _stream()),
+           "attn_rows")
     return out
 
 

@@ -348,6 +348,67 @@ def test_tiles_at_their_edges(T, cuts, window, keep, G, D, E):
     _near(torch.cat(got), torch.cat(want, 1), BF16, tol=2.0 ** -8)
 
 
+@pytest.mark.parametrize("window,keep", [(0, 0), (1, 0), (33, 64), (300, 65)])
+@pytest.mark.parametrize("kind", [None, "bias", "cap", "all"])
+@pytest.mark.parametrize("H,G,D", [(2, 2, 128), (6, 2, 64), (20, 1, 128),
+                                   (8, 1, 64)])
+def test_rows_of_common_heads_at_their_edges(H, G, D, kind, window, keep):
+    """Decoding with heads of 64 and 128: contexts that end at the borders of
+    tiles and pages, few and many workgroups a row, the newest key cached
+    already or not; stale numbers that are no numbers behind the newest."""
+    on = MODS.get(kind, {})
+    lens = [1, 32, 33, 64, 65, 127, 400, 1030]
+    B, scale = len(lens), 2.0 * D ** -0.5
+    q = _rand(B, H * D, seed=1, dtype=BF16)
+    ks = [_rand(n, G, D, seed=n, dtype=BF16) for n in lens]
+    vs = [_rand(n, G, D, seed=n + 1, dtype=BF16) for n in lens]
+    temp = (1.0 - _rand(H, seed=2)).to(BF16) if on.get("temp") else None
+    sink = _rand(H, seed=3, dtype=BF16) if on.get("sink") else None
+    gate = _rand(B, H, seed=4, dtype=BF16) if on.get("gate") else None
+    slope = torch.tensor([so.slope(h, H) for h in range(H)]) \
+        if on.get("slope") else None
+    cap, want = on.get("cap", 0.0), torch.zeros(B, H, D, dtype=torch.float64)
+    for b, n in enumerate(lens):
+        away = n - 1 - torch.arange(n)
+        seen = torch.ones(n, dtype=torch.bool)
+        if window:
+            seen = (away < window) | (torch.arange(n) < keep)
+        for h in range(H):
+            g = h // (H // G)
+            s = ks[b][:, g].double() @ q[b, h * D:(h + 1) * D].double() * scale
+            s = s * temp[h].double() if temp is not None else s
+            s = cap * torch.tanh(s / cap) if cap else s
+            s = s - slope[h].double() * away if slope is not None else s
+            s = s.masked_fill(~seen, -float("inf"))
+            if sink is not None:
+                s = torch.cat([s, sink[h:h + 1].double()])
+            o = s.softmax(0)[:n] @ vs[b][:, g].double()
+            want[b, h] = o * so.sigmoid(gate[b, h].double()) \
+                if gate is not None else o
+    mod = sv.ScoreMod(*(t.cuda() if t is not None else None for t in (temp,)),
+                      cap=cap, slope=None if slope is None else
+                      slope.float().cuda(),
+                      sink=None if sink is None else sink.cuda(),
+                      gate=None if gate is None else gate.cuda()) \
+        if kind else None
+    kc, vc, bt = _pages(lens, G, D, D, BF16)
+    kc.fill_(float("nan"))
+    vc.fill_(float("nan"))
+    for b, n in enumerate(lens):
+        for p in range(n - 1):
+            kc[bt[b, p // 64], :, p % 64] = ks[b][p].cuda()
+            vc[bt[b, p // 64], :, p % 64] = vs[b][p].cuda()
+    pos, seq = _i32([n - 1 for n in lens]), _i32(range(B))
+    k, v = (torch.stack([x[-1] for x in t]).reshape(B, G * D).cuda()
+            for t in (ks, vs))
+    for append, max_keys in ((True, 64), (True, 4000), (False, 500)):
+        got = sv.attn_rows(q.cuda(), k, v, kc, vc, pos, seq, bt, H, scale,
+                           window, keep, append=append, max_keys=max_keys,
+                           mod=mod)
+        # the result's rounding, 2^-9 of its largest number
+        _near(got, want.view(B, -1), BF16, (append, max_keys), tol=2.0 ** -8)
+
+
 def test_a_far_biased_key_is_not_lost():
     """A key thousands of positions back wins against its distance bias, in a
     prompt tile and when decoding."""
