@@ -340,7 +340,23 @@ class LlamaMLP(nn.Module):
             init_method=_init_method(config.initializer_range))
 
     def forward(self, x):
-        return self.down_proj(ops.swiglu(self.gate_up_proj(x)))
+        act = None
+        if not torch.is_grad_enabled() and self._glu_in_one():
+            act = ops.skinny_or_none(x, self.gate_up_proj.weight, glu=True)
+        if act is None:
+            act = ops.swiglu(self.gate_up_proj(x))
+        return self.down_proj(act)
+
+    def _glu_in_one(self) -> bool:
+        """May a few rows skip the call of gate_up_proj: it is the layer made
+        here, and nobody watches it?"""
+        p = self.gate_up_proj
+        return (type(p) is ColumnParallelLinear and "forward" not in p.__dict__
+                and not (p._forward_hooks or p._forward_pre_hooks)
+                and not (nn.modules.module._global_forward_hooks
+                         or nn.modules.module._global_forward_pre_hooks)
+                and p.bias is None and not p.skip_bias_add
+                and not (p.gather_output or p.sequence_parallel_enabled))
 
 
 def fused_norm_train_ok(config, hidden, training=True) -> bool:

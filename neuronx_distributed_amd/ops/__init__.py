@@ -657,40 +657,36 @@ def moe_decode_glu(hidden: torch.Tensor, gate_up_w: torch.Tensor,
 
 
 # ---------------------------------------------------------------------------
-# Skinny-M decode GEMM (csrc/skinny_gemm.hip)
+# Skinny-M decode GEMM (csrc/serving/stream_linear.hip)
 # ---------------------------------------------------------------------------
 
 def skinny_gemm_available() -> bool:
-    lib = _load()
-    return lib is not None and hasattr(lib, "skinny_gemm")
+    from . import serving as sv
+
+    return sv.available()
 
 
 def skinny_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x2 (M<=32, K) bf16 @ w (N, K)^T -> (M, N) bf16 via the split-K
-    weight-streaming kernel (decode shapes run ~10x hipBLASLt's skinny
-    kernels; see profiles/README.md)."""
-    lib = _require_lib()
-    M, K = x2.shape
-    N = w.shape[0]
-    out = torch.zeros(M, N, dtype=torch.float32, device=x2.device)
-    lib.skinny_gemm(_ptr(x2), _ptr(w), _ptr(out), M, N, K, _stream())
-    return out.to(torch.bfloat16)
+    """x2 (M<=32, K) bf16 @ w (N, K)^T -> (M, N) bf16 via the
+    weight-streaming kernel."""
+    from . import serving as sv
+
+    return sv.stream_linear(x2, w)
 
 
-def use_skinny_linear(inp: torch.Tensor, weight: torch.Tensor,
-                      sequence_parallel_enabled: bool = False) -> bool:
-    """Gate for the decode GEMM fast path (opt-in via NXDA_SKINNY_GEMM=1):
-    measured on MI355X, hipBLASLt's skinny kernels already run the decode
-    shapes at 1.8-6.6 TB/s — this kernel is kept for shapes/layouts where
-    the library falls over, not as the default."""
-    if os.environ.get("NXDA_SKINNY_GEMM", "0") != "1":
-        return False
-    return (not torch.is_grad_enabled() and not sequence_parallel_enabled
-            and inp.is_cuda and inp.dtype == torch.bfloat16
-            and weight.dtype == torch.bfloat16
-            and inp.numel() // inp.shape[-1] <= 32
-            and weight.shape[-1] % 8 == 0 and inp.shape[-1] == weight.shape[-1]
-            and skinny_gemm_available())
+def skinny_or_none(inp: torch.Tensor, weight: torch.Tensor,
+                   sequence_parallel_enabled: bool = False,
+                   glu: bool = False):
+    """inp (.., K) @ weight (N, K)^T, or with ``glu`` silu(gate) * up of
+    weight = [gate; up], by the weight-streaming kernels where they beat the
+    library (a few rows; ``serving.stream_rule``), else None.
+    NXDA_SKINNY_GEMM=0 keeps everything on the library."""
+    if torch.is_grad_enabled() or sequence_parallel_enabled or \
+            os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
+        return None
+    from . import serving as sv
+
+    return sv.streamed(inp, weight, glu=glu)
 
 
 # ---------------------------------------------------------------------------

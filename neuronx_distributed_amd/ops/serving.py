@@ -39,6 +39,13 @@ def library():
     return _LIB
 
 
+def available() -> bool:
+    """Is the library there to be loaded?"""
+    from .build import SERVING_LIB
+
+    return _LIB is not None or os.path.exists(SERVING_LIB)
+
+
 def ensure_built():
     """Compile the serving library if it is missing or out of date (and
     nothing else)."""
@@ -88,6 +95,13 @@ class _ResidualNormArgs(ctypes.Structure):
                 + _fields("eps scale w_base p_base h_scale", ctypes.c_float)
                 + _fields("branches", ctypes.c_int)
                 + [("br", _BranchArgs * 2)])
+
+
+class _StreamArgs(ctypes.Structure):
+    _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
+                + _fields("w", ctypes.c_void_p) + _fields("wst", ctypes.c_long)
+                + _fields("out", ctypes.c_void_p)
+                + _fields("T N K", ctypes.c_int))
 
 
 class _ConvArgs(ctypes.Structure):
@@ -208,12 +222,104 @@ class _ChunkArgs(ctypes.Structure):
 # matrix products with a 32-bit result
 # ---------------------------------------------------------------------------
 
+def stream_rule(T: int, N: int, K: int, f32: bool = False,
+                glu: bool = False) -> Optional[int]:
+    """How T rows x (T, K) meet a large weight (N, K): 0 every workgroup
+    streams its weight rows and all of x, 1 workgroups stay with x in registers,
+    None the library's product is as fast.  All measured over N 512..128256,
+    K 512..28672 (``stream_linear.hip``):
+
+    - up to 4 rows stream, unless a part of the CUs gets one workgroup more
+      than the others (5120 x 5120: 17 us, library 14) or x is large itself;
+      up to 16 where the weight is small (4096 x 4096: 9..12 us, library 15)
+      but not too small to share x (64 x 4096, 16 rows: 9.3 us, library 8.1);
+    - staying takes two and more tiles a CU.  With 32-bit results of
+      K = 8192 the library is 2% faster; with 17..32 rows it is where 5 or 6 of
+      the 8 waves have columns (K = 3072: 35.5 us, library 34)."""
+    tiles = N // (32 if glu else 16)
+    stay = N % (32 if glu else 16) == 0 and K <= (4096 if f32 else 8192)
+    if glu:
+        return 1 if stay and tiles >= 640 and (
+            T <= 16 or T <= 32 and (K <= 2048 or 3584 < K <= 4096)) else None
+    tiles = -(-N // 16)
+    even = tiles <= 256 or 384 <= tiles <= 512 or \
+        tiles > 512 and tiles >= 384 * -(-tiles // 512)
+    if T <= 4 and even and T * K <= 4 * 14336:
+        return 0
+    if stay and tiles >= 1024 and T <= 16:
+        return 1
+    small = K <= 4096 and N * K <= 4096 * 4096
+    return 0 if small and T <= (16 if N >= 512 else 8) else None
+
+
+def stream_linear(x: torch.Tensor, w: torch.Tensor, stay: int = 0,
+                  f32: bool = False, glu: bool = False) -> torch.Tensor:
+    """x (T, K) @ w (N, K)^T, bfloat16, with the sums rounded once or not at
+    all (``f32``); ``glu``: silu(gate) * up of w = [gate; up]."""
+    T, K = x.shape
+    N = w.shape[0]
+    assert x.dtype == w.dtype == torch.bfloat16 and w.shape[1] == K
+    assert x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
+    assert _words(x) and _words(w) and not (f32 and glu)
+    out = torch.empty(T, N // 2 if glu else N, device=x.device,
+                      dtype=torch.float32 if f32 else torch.bfloat16)
+    a = _StreamArgs(x=x.data_ptr(), xst=x.stride(0), w=w.data_ptr(),
+                    wst=w.stride(0), out=out.data_ptr(), T=T, N=N, K=K)
+    _check(library().sv_stream_linear(
+        ctypes.byref(a), 2 if glu else int(f32), stay, _stream()),
+        "stream_linear")
+    return out
+
+
+def _words(t: torch.Tensor) -> bool:
+    """Does every row start at a 16-byte word and hold a whole number?"""
+    return not (t.stride(0) | t.shape[1]) & 7 and not t.data_ptr() & 15
+
+
+def _plain(t) -> bool:
+    return type(t) in (torch.Tensor, torch.nn.Parameter)
+
+
+def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
+             glu: bool = False) -> Optional[torch.Tensor]:
+    """``stream_linear`` of the rows of x (..., K), where it is the faster one;
+    None elsewhere, under autograd, and where somebody else watches the
+    operations (tracing, dispatch modes, autocast)."""
+    if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
+            not x.is_cuda or x.dim() < 2 or w.dim() != 2:
+        return None
+    K = x.shape[-1]
+    T = x.numel() // K if K else 0
+    if not 0 < T <= 32 or x.dtype != torch.bfloat16 or \
+            w.dtype != torch.bfloat16 or w.shape[1] != K or \
+            w.stride(1) != 1 or w.device != x.device or \
+            x.device.index != torch.cuda.current_device():
+        return None
+    how = stream_rule(T, w.shape[0], K, f32, glu)
+    if how is None or not available() or not _unwatched():
+        return None
+    rows = x.reshape(T, K)
+    if rows.stride(1) != 1 or not (_words(rows) and _words(w)):
+        return None
+    return stream_linear(rows, w, how, f32, glu).view(*x.shape[:-1], -1)
+
+
+def _unwatched() -> bool:
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch.is_autocast_enabled("cuda")
+                or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x (T, K) @ w (N, K)^T with a float32 result (no rounding to the
     activation type): gate logits, vocabulary logits, residual projections."""
     if x.dtype == torch.float32:
         return torch.mm(x, w.t())
-    return torch.mm(x, w.t(), out_dtype=torch.float32)
+    out = streamed(x, w, f32=True)
+    return torch.mm(x, w.t(), out_dtype=torch.float32) if out is None else out
 
 
 # ---------------------------------------------------------------------------

@@ -350,14 +350,12 @@ def linear_with_async_allreduce(input_, weight, bias=None,
                                 sequence_parallel_enabled=False):
     from .. import ops as _ops
 
-    if _ops.use_skinny_linear(input_, weight, sequence_parallel_enabled):
-        # decode fast path: M <= 32 tokens, inference — the split-K
-        # weight-streaming HIP kernel instead of hipBLASLt skinny kernels
-        flat = input_.reshape(-1, input_.shape[-1]).contiguous()
-        out = _ops.skinny_linear(flat, weight)
-        if bias is not None:
-            out = out + bias
-        return out.reshape(*input_.shape[:-1], weight.shape[0])
+    # decode fast path: the weight-streaming HIP kernels instead of
+    # hipBLASLt's skinny ones
+    if bias is None:
+        out = _ops.skinny_or_none(input_, weight, sequence_parallel_enabled)
+        if out is not None:
+            return out
     args = cast_if_autocast_enabled(input_, weight, bias)
     with torch.amp.autocast("cuda", enabled=False):
         return LinearWithAsyncCommunication.apply(

@@ -317,23 +317,15 @@ class GQAQKVColumnParallelLinear(BaseParallelLinear):
             # inference: ONE fused GEMM, then split (reference
             # qkv_linear.py:164-176 fused-QKV)
             wcat, bcat = self._fused_qkv_weight()
-            out = F.linear(input_, wcat, bcat)
+            out = _ops.skinny_or_none(input_, wcat) if bcat is None else None
+            if out is None:
+                out = F.linear(input_, wcat, bcat)
             nq = self.q_output_size_per_partition
             nkv = self.kv_output_size_per_partition
             q = out[..., :nq]
             k = out[..., nq:nq + nkv]
             v = out[..., nq + nkv:]
             return q, k, v
-        if _ops.use_skinny_linear(input_, self.weight_q,
-                                  self.sequence_parallel_enabled) and \
-                self.bias_q is None:
-            flat = input_.reshape(-1, input_.shape[-1]).contiguous()
-            lead = input_.shape[:-1]
-            q = _ops.skinny_linear(flat, self.weight_q)
-            k = _ops.skinny_linear(flat, self.weight_k)
-            v = _ops.skinny_linear(flat, self.weight_v)
-            return (q.reshape(*lead, -1), k.reshape(*lead, -1),
-                    v.reshape(*lead, -1))
         q, k, v = _QKVLinearWithAsyncCommunication.apply(
             input_, self.weight_q, self.weight_k, self.weight_v,
             self.bias_q, self.bias_k, self.bias_v,

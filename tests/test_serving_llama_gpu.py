@@ -73,3 +73,34 @@ def test_bf16_and_table_limit():
                        for t in x[0, 100:].tolist()]).double()
     err = (out - want).pow(2).mean(1).sqrt() / want.pow(2).mean().sqrt()
     assert err.max() < 0.05, err.max().item()
+
+
+def test_mlp_of_few_rows_calls_a_watched_layer():
+    """Gates and projections in one kernel, unless a hook sits on the layer
+    that it passes by."""
+    from neuronx_distributed_amd.models import LlamaConfig
+    from neuronx_distributed_amd.models.llama import LlamaMLP
+
+    torch.manual_seed(0)
+    mlp = LlamaMLP(LlamaConfig(hidden_size=1024, intermediate_size=10240,
+                               num_attention_heads=8, num_key_value_heads=8))
+    mlp = mlp.to("cuda", torch.bfloat16)
+    x = torch.randn(3, 1, 1024, device="cuda").bfloat16()
+    seen = []
+    with torch.no_grad():
+        gu = x.double() @ mlp.gate_up_proj.weight.double().t()
+        ref = torch.nn.functional.silu(gu[..., :10240]) * gu[..., 10240:]
+        ref = ref @ mlp.down_proj.weight.double().t()
+        few = mlp(x)
+        handle = mlp.gate_up_proj.register_forward_hook(
+            lambda m, i, o: seen.append(o.shape))
+        watched = mlp(x)
+        handle.remove()
+    assert seen == [(3, 1, 20480)]
+
+    def error(out):
+        return ((out.double() - ref).norm() / ref.norm()).item()
+
+    # one rounding of 8 bits to the activations, one to the result
+    assert error(few) < 2 * 2.0 ** -9
+    assert error(few) <= error(watched)

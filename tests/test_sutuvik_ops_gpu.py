@@ -628,3 +628,63 @@ def test_bad_arguments_are_refused():
     with pytest.raises(RuntimeError):
         sv.gelu_rows_(torch.zeros(2, 4), torch.zeros(3, 8),
                       torch.zeros(2, dtype=torch.int32), 0)
+
+
+@pytest.mark.parametrize("T,N,K,how", [
+    (1, 16, 8, 0), (4, 4112, 4104, 0), (16, 1001, 520, 0), (17, 48, 1032, 0),
+    (1, 32, 8, 1), (16, 8224, 4096, 1), (5, 96, 4104, 1), (16, 64, 8192, 1),
+    (17, 32, 4088, 1), (32, 8224, 520, 1)])
+def test_products_of_few_rows(T, N, K, how):
+    """Rounded, 32-bit and gated results against 64-bit products; the last
+    tiles, columns and rows ragged.  Weights and rows lie in wider ones."""
+    torch.manual_seed(T + N + K)
+    x = torch.randn(T, K + 8, device="cuda").bfloat16()[:, :K]
+    w = torch.randn(N, K + 24, device="cuda").div(K ** 0.5).bfloat16()[:, :K]
+    ref = x.double() @ w.double().t()
+    # K products of 32 bits summed in 32 bits: K ** 0.5 roundings of the
+    # partial sums (about 1) on average, 16 of them at the outside
+    tol = 16 * K ** 0.5 * 2.0 ** -24
+    out = sv.stream_linear(x, w, how, f32=True)
+    assert out.dtype == torch.float32
+    torch.testing.assert_close(out.double(), ref, rtol=0, atol=tol)
+    torch.testing.assert_close(sv.stream_linear(x, w, how).double(), ref,
+                               rtol=2.0 ** -8, atol=tol)
+    if how:
+        gate, up = ref[:, :N // 2], ref[:, N // 2:]
+        torch.testing.assert_close(
+            sv.stream_linear(x, w, how, glu=True).double(),
+            torch.nn.functional.silu(gate) * up, rtol=2.0 ** -8,
+            atol=tol * 16)
+
+
+@pytest.mark.parametrize("glu", [False, True])
+def test_few_rows_are_streamed_where_nobody_watches(glu):
+    x = torch.randn(2, 3, 4096, device="cuda").bfloat16()
+    w = torch.randn(28672, 4096, device="cuda").div(64).bfloat16()
+    assert sv.streamed(x, w, glu=glu) is None          # under autograd
+    with torch.no_grad():
+        out = sv.streamed(x, w, glu=glu)
+        ref = x.double() @ w.double().t()
+        if glu:
+            ref = torch.nn.functional.silu(ref[..., :14336]) * ref[..., 14336:]
+        # K products, rounded to 8 bits at the end; gates and projections of
+        # about 1 with the error of 64 32-bit roundings each
+        torch.testing.assert_close(out.double(), ref, rtol=2.0 ** -8,
+                                   atol=64 * 16 * 2.0 ** -24)
+        for other in (x.float(), x[..., :4090], x.cpu(), x[0, 0]):
+            assert sv.streamed(other, w, glu=glu) is None
+        assert sv.streamed(x, w[:, 1:], glu=glu) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert sv.streamed(x, w, glu=glu) is None
+        with torch.autograd.forward_ad.dual_level():
+            assert sv.streamed(x, w, glu=glu) is None
+        seen = []
+
+        class Watch(torch.utils._python_dispatch.TorchDispatchMode):
+            def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+                seen.append(f)
+                return f(*args, **(kwargs or {}))
+
+        with Watch():
+            assert sv.streamed(x, w, glu=glu) is None
+        assert not any("empty" in str(f) for f in seen)
