@@ -83,6 +83,8 @@ residual_norm_kernel(ResidualNormArgs a) {
   const T* d1 = (const T*)a.delta + r * W;
   const float* d1f = (const float*)a.delta + r * W;
   const T* d2 = (const T*)a.delta2 + r * W;
+  float w_first[VEC];              // on its way while the sums are made
+  if (a.h && a.w && tid * VEC < W) ld<T, VEC>((const T*)a.w + tid * VEC, w_first);
 
   // the pending result when it is one tensor or a weighted sum of rows
   auto single = [&](int i, float* v) {
@@ -256,7 +258,12 @@ residual_norm_kernel(ResidualNormArgs a) {
   for (int i = tid * VEC; i < W; i += NT * VEC) {
     float v[VEC], u[VEC];
     ld<float, VEC>(row + i, v);  // written by this same thread
-    ld<T, VEC>((const T*)a.w + i, u);
+    if (i == tid * VEC) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) u[j] = w_first[j];
+    } else {
+      ld<T, VEC>((const T*)a.w + i, u);
+    }
     if (a.groups > 1) rstd = part_rstd[i / size];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) v[j] *= rstd * (a.w_base + u[j]) * a.h_scale;
@@ -308,7 +315,8 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
                   (a->br[b].gst % 4 == 0 &&
                    (size_t)a->br[b].gate % (f32 ? 16 : 8) == 0));
   if (a->branches < 0 || a->branches > 2 || (a->branches && a->delta)) return 1;
-  // few rows: a longer workgroup hides the way to memory
+  // few rows: a longer workgroup waits for fewer words one after the other
+  // (1 row of 4096: 8.2 -> 5.2 us, 32 rows 8.1 -> 5.3)
   const bool wide = a->rows_out <= 512 && a->W >= 2048;
 #define RNB(T, V, B, N)                                                    \
   residual_norm_kernel<T, V, B, N><<<a->rows_out, N, lds, stream>>>(*a)
@@ -316,6 +324,7 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
   do {                                                                     \
     if (a->branches && wide) RNB(T, V, true, 1024);                        \
     else if (a->branches) RNB(T, V, true, 256);                            \
+    else if (wide) RNB(T, V, false, 1024);                                 \
     else RNB(T, V, false, 256);                                            \
   } while (0)
   if (f32) { if (vec) RN(float, 4); else RN(float, 1); }

@@ -418,3 +418,51 @@ def test_pointwise(sv, dtype):
 def test_cpu_tensors_are_refused(sv):
     with pytest.raises(RuntimeError):
         sv.relu_squared_(torch.zeros(4, 4))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,W", [(1, 2049), (1, 4096), (512, 2052),
+                                    (513, 2052), (3, 9004)])
+def test_residual_norm_of_wide_rows(sv, rows, W, dtype):
+    """Long and ordinary workgroups; the last words of a row ragged."""
+    eps = 0.03
+    x = _rand(rows, W, dtype=torch.float32)
+    a, w1, w = (_rand(*n, dtype=dtype, seed=s, scale=3.0)
+                for s, n in ((1, (rows, W)), (2, (W,)), (3, (W,))))
+    for pend, want in (
+            (sv.Pending(a.cuda()), x.double() + a.double()),
+            (sv.Pending(a.cuda(), w1=w1.cuda()),
+             x.double() + vo.rms_norm(a.double(), w1.double(), eps))):
+        nx, h, _ = sv.residual_norm(x.cuda(), pend, eps, w.cuda())
+        _close(nx, want, torch.float32)
+        _close(h, vo.rms_norm(want, w.double(), eps), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,shift", [(1, 0, 2, 0), (3, 1, 24, 0),
+                                         (5, 2, 36, 0), (32, 8, 128, 0),
+                                         (32, 8, 128, 1), (7, 7, 64, 4)])
+@pytest.mark.parametrize("T", [1, 33])
+def test_rope_rows(sv, T, H, G, D, shift, dtype):
+    """Every pair of every head is turned once: words and single pairs, heads
+    that start between words, the last workgroup ragged."""
+    half = D // 2
+    qkv = _rand(T, (H + G) * D + shift + 8 * (shift == 4), dtype=dtype).cuda()
+    q, k = qkv[:, shift:shift + H * D], qkv[:, shift + H * D:][:, :G * D]
+    angle = torch.arange(64)[:, None] * torch.rand(half)[None]
+    cos, sin = angle.cos().cuda(), angle.sin().cuda()
+    pos = torch.randint(0, 64, (T,), dtype=torch.int32)
+    before = qkv.clone()
+    sv.rope_rows_(q, k, cos, sin, pos.cuda(), D, 64)
+    n = (H + G) * D
+    x, y = before[:, shift:shift + n].double().view(T, -1, 2, half).unbind(2)
+    c, s = (t[pos.cuda()].double()[:, None] for t in (cos, sin))
+    want = torch.stack((x * c - y * s, y * c + x * s), 2).view(T, n)
+    got = qkv[:, shift:shift + n].double()
+    # two products and a sum in 32 bits of factors that reach 4 and 1, and
+    # half a unit of the type's 8 or 24 bits: 2 ** -8 or 2 ** -24 of the value
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    assert ((got - want).abs() <= want.abs() * unit * 1.01
+            + (x.abs() + y.abs()).max() * 2.0 ** -23).all()
+    assert torch.equal(qkv[:, :shift], before[:, :shift])
+    assert torch.equal(qkv[:, shift + n:], before[:, shift + n:])
