@@ -25,7 +25,8 @@ struct MoePlanArgs {
   int* idx;                 // [T * top] chosen experts
   float* coef;              // [T * top] their weights
   int* order;               // [T * top] slot -> pair
-  int* tiles;               // [max_tiles][4]: expert, first slot, slots, 0
+  int* tiles;               // [max_tiles][4]: expert, first slot, slots, number
+                            //   of tiles; no slots past it
   int T, E, top, tile_rows, max_tiles;
   int kind;                 // 0: weights are a softmax over the chosen;
                             // 1: scores sigmoid(z), chosen by score + bias;
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(1024) moe_plan_kernel(MoePlanArgs a) {
       t[0] = tid;
       t[1] = s0 + i * a.tile_rows;
       t[2] = min(a.tile_rows, n - i * a.tile_rows);
-      t[3] = 0;
+      t[3] = total;
     }
     count[tid] = s0;
   }
@@ -415,63 +416,204 @@ moe_tiles_kernel(MoeGemmArgs a) {
 }
 
 // -- a few rows per expert: stream the weights --------------------------------
-// One workgroup = 32 weight rows (16 gate and their 16 up rows) by up to 32
-// slots; its four waves take every fourth 64-column block of K and meet in
-// LDS.  Weights go straight from memory to registers, once per tile.
+// Weights go from memory straight into registers as fragments, a lane's 16
+// bytes of a row, and meet up to 32 slots of x (16 and less leave the second
+// half out).  A unit is 16 weight rows (16 gates and their 16 up rows) of one
+// slot tile.  Bound by reading the weights.  Plan and two products, us (4 waves
+// that share 32 weight rows, nothing read ahead | now; 32-slot tiles):
+//   64 experts 2048 x 1408, top 6   1 row  46 |  42    8: 156 | 127   32: 279 | 216
+//   64 and 192 rows, on tiles              252 | 236         286 | 236
+//   8 experts 4096 x 14336, top 2   1 row 187 | 140    8: 613 | 464
+//   32 and 64 rows, on tiles               613 | 542         635 | 608
+// 32 rows read 1.07 GB of 64 experts at 5.3 TB/s.
+
+// acc rows 4 grp + 0..3 are the unit's weight rows, columns slots
 template <bool GLU>
-__global__ void __launch_bounds__(256) moe_stream_kernel(MoeGemmArgs a) {
-  constexpr int NOUT = GLU ? 16 : 32;
-  __shared__ float part[4][16][64];
+__device__ __forceinline__ void store_unit(const MoeGemmArgs& a, int slot0,
+                                           int rows, int r, int c, f32x4 v,
+                                           f32x4 u) {
+  if (r >= rows || c >= a.N) return;
+  if (GLU)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = glu(a, v[j], u[j]);
+  short* dst = (short*)a.out +
+      (long)(a.top ? slot0 + r : a.order[slot0 + r]) * a.N + c;
+  *(uint2*)dst = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+__device__ __forceinline__ const short* unit_x(const MoeGemmArgs& a, int slot) {
+  return (const short*)a.x + (long)(a.top ? a.order[slot] / a.top : slot) * a.xst;
+}
+
+template <int N> struct Count { static constexpr int value = N; };
+
+// K up to 512 NW: a workgroup stays.  It takes the same share of all units as
+// the others, one after the other, with the columns of its slots in registers:
+// wave w those of 64-column blocks w, w + NW, ...  Four blocks of a weight row
+// are read at a time, one such part ahead, past the units' borders.
+template <int NW, bool GLU>
+__global__ void __launch_bounds__(NW * 64, 2) moe_stay_kernel(MoeGemmArgs a) {
+  constexpr int RT = GLU ? 2 : 1, PARTS = 2, UNITS = RT * PARTS;
+  __shared__ f32x4 part[2][NW][RT * 2][64];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, grp = lane >> 4;
+  const int K = a.K, N = a.N, ntn = (N + 15) / 16;
+  const long units = (long)a.tiles[3] * ntn;      // all tiles that have rows
+  const long first = units * blockIdx.x / gridDim.x;
+  int left = (int)(units * (blockIdx.x + 1) / gridDim.x - first);
+  if (left == 0) return;
+  const uint4v zero = {0, 0, 0, 0};
+  const int k0 = wid * 64 + grp * 8;
+  // the lane's columns of its chunk c start at k0 + at(c)
+  auto at = [](int c) { return (c >> 1) * NW * 64 + (c & 1) * 32; };
+
+  // the unit that is read next
+  int tn = (int)(first % ntn);
+  const int* tl = a.tiles + 4 * (first / ntn);
+  const short* w = (const short*)a.w + (long)tl[0] * RT * N * K;
+  auto load = [&](int u, frag_u* fw) __attribute__((always_inline)) {
+    const int n = min(tn * 16 + c16, N - 1) + (u / PARTS ? N : 0);
+    const short* src = w + (long)n * K + (k0 + at(u % PARTS * 8));
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      fw[c].u4 = k0 + at(u % PARTS * 8 + c) < K ? *(const uint4v*)(src + at(c))
+                                                : zero;
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
+    if (left == 1) return;         // past the last one that one again, unused
+    if (++tn == ntn) {
+      tn = 0;
+      tl += 4;
+      w = (const short*)a.w + (long)tl[0] * RT * N * K;
+    }
+  };
+
+  frag_u wa[8], wb[8];
+  int buf = 0;
+  // the units of one slot tile, MT times 16 slots
+  auto run = [&](auto tiles_of_16) __attribute__((always_inline)) {
+    constexpr int MT = decltype(tiles_of_16)::value;
+    const int slot0 = tl[1], rows = tl[2];
+    frag_u fx[PARTS * 8][MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const short* x = unit_x(a, slot0 + min(j * 16 + c16, rows - 1)) + k0;
+#pragma unroll
+      for (int c = 0; c < PARTS * 8; ++c)
+        fx[c][j].u4 = k0 + at(c) < K ? *(const uint4v*)(x + at(c)) : zero;
+    }
+    f32x4 acc[MT];
+    auto multiply = [&](int u, const frag_u* fw) __attribute__((always_inline)) {
+      const int p = u % PARTS;
+      if (p == 0)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[j] = f32x4{};
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[j] = mfma16(fw[c].bf, fx[p * 8 + c][j].bf, acc[j]);
+      if (p == PARTS - 1)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          part[buf][wid][u / PARTS * 2 + j][lane] = acc[j];
+    };
+    for (int n = min(left, ntn - tn); n > 0; --n, --left, buf ^= 1) {
+      const int n0 = tn * 16;
+#pragma unroll
+      for (int u = 0; u < UNITS; u += 2) {
+        const bool last = u + 2 == UNITS;
+        if (last) advance();
+        multiply(u, wa);
+        load(last ? 0 : u + 2, wa);
+        multiply(u + 1, wb);
+        load(last ? 1 : u + 3, wb);
+      }
+      // the first waves add up the sums of all; the others go on
+      __syncthreads();
+      if (wid >= MT) continue;
+      f32x4 v = {}, u = {};
+#pragma unroll 2
+      for (int s = 0; s < NW; ++s) {
+        v += part[buf][s][wid][lane];
+        if (GLU) u += part[buf][s][2 + wid][lane];
+      }
+      store_unit<GLU>(a, slot0, rows, wid * 16 + c16, n0 + 4 * grp, v, u);
+    }
+  };
+  load(0, wa);
+  load(1, wb);
+  while (left > 0) {
+    if (tl[2] > 16) run(Count<2>());
+    else run(Count<1>());
+  }
+}
+
+// Longer rows: a workgroup a unit; its 16 waves take turns of 64 columns of
+// the weight rows and of x, a turn ahead.
+template <bool GLU>
+__global__ void __launch_bounds__(1024) moe_stream_kernel(MoeGemmArgs a) {
+  constexpr int RT = GLU ? 2 : 1, U = 2, STEP = 16 / RT * U * 32;
+  __shared__ f32x4 part[16][2][64];
   const int* tl = a.tiles + 4L * blockIdx.y;
   const int rows = tl[2];
   if (rows == 0) return;
-  const int e = tl[0], slot0 = tl[1];
+  const int slot0 = tl[1];
+  const bool two = rows > 16;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 31, hi = lane >> 5;
-  const int K = a.K, N = a.N, n0 = blockIdx.x * NOUT;
-  const int n = min(n0 + (GLU ? col & 15 : col), N - 1);
-  const bool live = col < rows;
-  const int slot = slot0 + (live ? col : 0);
-  const int pair = a.order[slot];
-  const short* w = (const short*)a.w +
-      ((long)e * (GLU ? 2 * N : N) + n + (GLU && col >= 16 ? N : 0)) * K + 32 * hi;
-  const short* x = (const short*)a.x +
-      (long)(a.top ? pair / a.top : slot) * a.xst + 32 * hi;
+  const int c16 = lane & 15, grp = lane >> 4;
+  const int K = a.K, N = a.N, n0 = blockIdx.x * 16;
+  const short* w = (const short*)a.w + grp * 8 +
+      ((long)tl[0] * RT * N + min(n0 + c16, N - 1) + (wid % RT ? N : 0)) * K;
+  const short* x[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    x[j] = unit_x(a, slot0 + min(j * 16 + c16, rows - 1)) + grp * 8;
 
-  f32x16 acc = {};
+  f32x4 acc[2] = {};
   const uint4v zero = {0, 0, 0, 0};
-  for (int k0 = wid * 64; k0 < K; k0 += 512) {
-    frag_u fw[8], fx[8];
+  auto load = [&](int k0, frag_u* fw, frag_u (*fx)[2])
+      __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int k = k0 + (c >> 2) * 256 + (c & 3) * 8;  // this lane's order
-      const bool in = k + 32 * hi < K;
-      fw[c].u4 = in ? *(const uint4v*)(w + k) : zero;
-      fx[c].u4 = in && live ? *(const uint4v*)(x + k) : zero;
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * 32;
+      const bool in = k + grp * 8 < K;
+      fw[u].u4 = in ? *(const uint4v*)(w + k) : zero;
+      fx[u][0].u4 = in ? *(const uint4v*)(x[0] + k) : zero;
+      fx[u][1].u4 = in && two ? *(const uint4v*)(x[1] + k) : zero;
     }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc = mfma_bf16(fw[c].bf, fx[c].bf, acc);
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) part[wid][r][lane] = acc[r];
-  __syncthreads();
-  auto total = [&](int r) {
-    return part[0][r][lane] + part[1][r][lane] + part[2][r][lane] +
-           part[3][r][lane];
   };
-  if (!live || (GLU && wid >= 2)) return;
-  // accumulator rows 4 w .. 4 w + 3 are weight rows 8 w + 4 hi + 0..3
-  const int c = n0 + 8 * wid + 4 * hi;
-  if (c >= N) return;
-  float v[4];
+  auto multiply = [&](const frag_u* fw, const frag_u (*fx)[2])
+      __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[j] = total(4 * wid + j);
-    if (GLU) v[j] = glu(a, v[j], total(8 + 4 * wid + j));
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[j] = mfma16(fw[u].bf, fx[u][j].bf, acc[j]);
+  };
+  frag_u wa[U], xa[U][2], wb[U], xb[U][2];
+  int k = wid / RT * U * 32;
+  if (k < K) load(k, wa, xa);
+  for (; k < K; k += 2 * STEP) {
+    if (k + STEP < K) load(k + STEP, wb, xb);
+    multiply(wa, xa);
+    if (k + STEP >= K) break;
+    if (k + 2 * STEP < K) load(k + 2 * STEP, wa, xa);
+    multiply(wb, xb);
   }
-  short* dst = (short*)a.out + (long)(a.top ? slot : pair) * N + c;
-  *(uint2*)dst = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) part[wid][j][lane] = acc[j];
+  __syncthreads();
+  if (wid >= 2 || (wid == 1 && !two)) return;
+  f32x4 v = {}, u = {};
+#pragma unroll
+  for (int s = 0; s < 16; s += RT) {
+    v += part[s][wid][lane];
+    if (GLU) u += part[s + 1][wid][lane];
+  }
+  store_unit<GLU>(a, slot0, rows, wid * 16 + c16, n0 + 4 * grp, v, u);
 }
 
 // -- any size and type -------------------------------------------------------
@@ -539,6 +681,22 @@ static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
     moe_tiles_kernel<BM, BN, WM, WN, GLU, false><<<grid, NT, 0, stream>>>(a);
 }
 
+template <bool GLU>
+static void launch_stream(const MoeGemmArgs& a, hipStream_t stream) {
+  const int units = (a.N + 15) / 16;
+  const long all = (long)units * a.max_tiles;
+  // as many workgroups as are resident: with twice as many, 2% to 30% longer.
+  // They share whole units, so they need a few (6 tiles of 2048 x 1408: a
+  // workgroup a unit 42 us, two products and the plan; staying 47).
+  const int grid = a.K <= 2048 ? 512 : 256;
+  if (a.K > 4096 || all < 2 * grid)
+    moe_stream_kernel<GLU><<<dim3(units, a.max_tiles), 1024, 0, stream>>>(a);
+  else if (a.K <= 2048)
+    moe_stay_kernel<4, GLU><<<grid, 256, 0, stream>>>(a);
+  else
+    moe_stay_kernel<8, GLU><<<grid, 512, 0, stream>>>(a);
+}
+
 // how: 0 any size and type, 1 stream, 2 to 5 tiles (1 to 5: bf16, N, K, xst
 // and bases in 8 elements).  The plan's tile_rows: 32, 32, 32, 64, 128, 256.
 extern "C" int sv_moe_gemm(const MoeGemmArgs* a, int how, int gated, int f32,
@@ -557,9 +715,8 @@ extern "C" int sv_moe_gemm(const MoeGemmArgs* a, int how, int gated, int f32,
     if (gated) launch_tiles<32, 256, 32, 64, true>(*a, stream);
     else launch_tiles<32, 128, 32, 32, false>(*a, stream);
   } else if (how == 1) {
-    const dim3 grid((a->N + (gated ? 15 : 31)) / (gated ? 16 : 32), a->max_tiles);
-    if (gated) moe_stream_kernel<true><<<grid, 256, 0, stream>>>(*a);
-    else moe_stream_kernel<false><<<grid, 256, 0, stream>>>(*a);
+    if (gated) launch_stream<true>(*a, stream);
+    else launch_stream<false>(*a, stream);
   } else {
     const dim3 grid((a->N + 31) / 32, a->max_tiles);
 #define PK(T, G) moe_plain_kernel<T, G><<<grid, 256, 0, stream>>>(*a)

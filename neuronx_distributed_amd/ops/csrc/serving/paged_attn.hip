@@ -467,10 +467,6 @@ attn_rows_kernel(RowsArgs a) {
 // Bound by memory: 8 waves a CU have 16 KB each on their way.  The kernel above
 // spends its time on vector work (a key costs 140 cycles of a wave; here 30).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 // the larger of the four lanes 16 apart
 __device__ __forceinline__ float max_quarters(float x) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x),

@@ -14,6 +14,10 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s4v __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 __device__ __forceinline__ float to_f(short v) { return bits2f(v); }
 __device__ __forceinline__ float to_f(float v) { return v; }
 __device__ __forceinline__ void from_f(short& o, float v) { o = f2bits(v); }

@@ -26,10 +26,6 @@ struct StreamArgs {
   int T, N, K;
 };
 
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 enum Epilogue { PLAIN = 0, F32 = 1, GLU = 2 };
 
 // Accumulator rows are weight rows 4 grp + 0..3, columns rows of x: the results

@@ -456,3 +456,34 @@ def test_kernels_refuse_the_cpu(sv):
         sv.head_linear(x, 8, torch.randn(1, 8, 8), torch.empty(4, 8), 8)
     with pytest.raises(ValueError):
         sv.moe_plan(torch.randn(4, 8).cuda(), None, 9, 0)
+
+
+@pytest.mark.parametrize("E,top,T,W,ff,one", [
+    (3, 1, 40, 136, 72, True), (5, 2, 33, 2048, 88, False),
+    (70, 4, 9, 1040, 2056, False), (40, 2, 70, 2056, 1000, False),
+    (2, 2, 17, 4096, 8, False), (9, 3, 31, 4104, 520, True),
+    (64, 6, 16, 64, 4096, False)])
+def test_streamed_experts_at_their_edges(sv, E, top, T, W, ff, one):
+    """Workgroups that stay and workgroups of one unit: units that end in the
+    middle of a tile of slots, 16 and 17 slots, rows and columns ragged;
+    ``one``: every row to the same experts."""
+    h = _rand(T, W, dtype=torch.bfloat16)
+    z = _rand(T, E, dtype=torch.float32, seed=1)
+    if one:
+        z[:, 1:1 + top] += 9.0
+    gu = _rand(E, 2 * ff, W, dtype=torch.bfloat16, seed=3, scale=W ** -0.5)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, seed=5, scale=ff ** -0.5)
+    p = sv.moe_plan(z.cuda(), None, top, sv.MOE_STREAM)
+    act = sv.moe_gemm(h.cuda(), gu.cuda(), p, True)
+    y = sv.moe_gemm(act, down.cuda(), p, False)
+    order, idx = p.order.cpu().long(), p.idx.cpu().reshape(-1).long()
+    got = act.double().cpu()
+    for e in range(E):
+        slots = (idx[order] == e).nonzero()[:, 0]
+        if not len(slots):
+            continue
+        pairs = order[slots]
+        g, u = (h[pairs // top].double() @ gu[e].double().T).chunk(2, 1)
+        _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
+        _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
+               torch.bfloat16)
