@@ -79,26 +79,39 @@ __device__ __forceinline__ void best_groups(const MoePlanArgs& a, float* v,
   }
 }
 
+// the largest value of the wave
+__device__ __forceinline__ float wave_max(float x) {
+#define TURN(n)                                                              \
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(                      \
+                   __float_as_int(x), 0x120 + n, 0xf, 0xf, true)))
+  TURN(8); TURN(4); TURN(2); TURN(1);       // of the 16 lanes of a row
+#undef TURN
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x),
+                                                  __float_as_uint(x), false,
+                                                  false);
+  return max_halves(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+
 // One wave, one row: the largest choice scores in descending order, the lower
 // index first among equals.  Choice scores are the logits with their bias, the
 // weights a softmax over the chosen, or over all (then they are not scaled to
 // a sum of one); or sigmoids with a bias, the weights the chosen sigmoids over
-// their sum.
-template <typename T>
+// their sum.  `chosen`: the experts once more, or null.
+template <int NV, typename T>
 __device__ __forceinline__ void route_row(const MoePlanArgs& a, int t,
-                                          float* mem) {
+                                          float* mem, int* chosen) {
   const int lane = threadIdx.x & 63;
-  constexpr int NV = MOE_MAX_EXPERTS / 64;
   const T* bias = (const T*)a.bias;
-  float v[NV];
+  float v[NV], own[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int e = i * 64 + lane;
     v[i] = -INFINITY;
+    own[i] = 0.f;
     if (e < a.E) {
       const float z = a.z[(long)t * a.E + e];
-      v[i] = (a.kind == 1 ? 1.f / (1.f + expf(-z)) : z) +
-             (bias ? to_f(bias[e]) : 0.f);
+      own[i] = a.kind == 1 ? 1.f / (1.f + expf(-z)) : z;
+      v[i] = own[i] + (bias ? to_f(bias[e]) : 0.f);
     }
   }
   float first = 0.f, sum = 0.f;
@@ -106,7 +119,7 @@ __device__ __forceinline__ void route_row(const MoePlanArgs& a, int t,
     first = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NV; ++i) first = fmaxf(first, v[i]);
-    first = wave_reduce(first, MaxOp());
+    first = wave_max(first);
 #pragma unroll
     for (int i = 0; i < NV; ++i) sum += expf(v[i] - first);
     sum = wave_reduce(sum, SumOp());
@@ -123,23 +136,28 @@ __device__ __forceinline__ void route_row(const MoePlanArgs& a, int t,
         best = v[i];
         at = i * 64 + lane;
       }
+    const float most = wave_max(best);
+    const unsigned long long have = __ballot(best == most);
+    if (__popcll(have) == 1) {
+      at = __builtin_amdgcn_readlane(at, __ffsll(have) - 1);
+    } else {                     // equals: the lowest index
+      if (best != most) at = MOE_MAX_EXPERTS;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oa = __shfl_xor(at, off, 64);
-      if (ob > best || (ob == best && oa < at)) {
-        best = ob;
-        at = oa;
-      }
+      for (int off = 32; off > 0; off >>= 1) at = min(at, __shfl_xor(at, off, 64));
+      at = __builtin_amdgcn_readfirstlane(at);
     }
+    best = most;
     at = min(at, a.E - 1);       // logits that are no numbers stay in bounds
+    float score = 0.f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
+    for (int i = 0; i < NV; ++i) {
+      if (at >> 6 == i) score = own[i];
       if (at == i * 64 + lane) v[i] = -INFINITY;
+    }
     if (k == 0 && a.kind != 2) first = best;
-    const float w =
-        a.kind == 1 ? 1.f / (1.f + expf(-a.z[(long)t * a.E + at]))
-                       : expf(best - first);
+    const float w = a.kind == 1
+        ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(score), at & 63))
+        : expf(best - first);
     if (a.kind != 2) sum += w;
     if (lane == k) {
       mine = w;
@@ -150,57 +168,94 @@ __device__ __forceinline__ void route_row(const MoePlanArgs& a, int t,
   if (lane < a.top) {
     a.idx[(long)t * a.top + lane] = mine_e;
     a.coef[(long)t * a.top + lane] = mine / sum;
+    if (chosen) chosen[t * a.top + lane] = mine_e;
   }
+}
+
+template <typename T>
+__device__ __forceinline__ void route(const MoePlanArgs& a, int t, float* mem,
+                                      int* chosen) {
+  if (a.E <= 64) route_row<1, T>(a, t, mem, chosen);
+  else if (a.E <= 256) route_row<4, T>(a, t, mem, chosen);
+  else route_row<MOE_MAX_EXPERTS / 64, T>(a, t, mem, chosen);
 }
 
 template <typename T>
 __global__ void __launch_bounds__(256) moe_route_kernel(MoePlanArgs a) {
   __shared__ float mem[4][MOE_MAX_EXPERTS];
   const int wid = threadIdx.x >> 6, t = blockIdx.x * 4 + wid;
-  if (t < a.T) route_row<T>(a, t, mem[wid]);
+  if (t < a.T) route<T>(a, t, mem[wid], nullptr);
 }
 
-// One workgroup.  ROUTE: it also routes the (few) rows first.
+#define MOE_FUSED_ROWS 16   // a wave each (32 in one kernel 9.4 us, in two 6.6)
+
+// One workgroup; a chain of short steps.  ROUTE: it also routes the (few) rows
+// first and keeps their experts in LDS.  Rows to 6 of 64 experts with the routing,
+// against maxima and sums by exchanges over LDS, row after row: 64 rows 28 -> 6.5
+// us, 8: 9.3 -> 5.6, 4096: 28 -> 21.
 template <typename T, bool ROUTE>
 __global__ void __launch_bounds__(1024) moe_plan_kernel(MoePlanArgs a) {
-  __shared__ int count[MOE_MAX_EXPERTS], slots[1024], tile_at[1024];
-  const int tid = threadIdx.x, E = a.E, pairs = a.T * a.top;
+  __shared__ int count[MOE_MAX_EXPERTS], wave_slots[8], wave_tiles[8];
   __shared__ float mem[ROUTE ? 16 : 1][MOE_MAX_EXPERTS];
-  if (ROUTE)
-    for (int t = tid >> 6; t < a.T; t += 16) route_row<T>(a, t, mem[tid >> 6]);
+  __shared__ int chosen[ROUTE ? MOE_FUSED_ROWS * 64 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, E = a.E, pairs = a.T * a.top;
   for (int e = tid; e < E; e += 1024) count[e] = 0;
-  __syncthreads();               // orders the block's own global writes too
-  for (int p = tid; p < pairs; p += 1024) atomicAdd(&count[a.idx[p]], 1);
+  if (ROUTE)
+    for (int t = tid >> 6; t < a.T; t += 16)
+      route<T>(a, t, mem[tid >> 6], chosen);
   __syncthreads();
+  // four experts on their way at a time
+  auto each = [&](auto f) __attribute__((always_inline)) {
+    for (int p = tid; p < pairs; p += 4096) {
+      int e[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (p + j * 1024 < pairs)
+          e[j] = ROUTE ? chosen[p + j * 1024] : a.idx[p + j * 1024];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (p + j * 1024 < pairs) f(p + j * 1024, e[j]);
+    }
+  };
+  each([&](int, int e) { atomicAdd(&count[e], 1); });
+  __syncthreads();
+  // sums of slots and tiles up to each expert: in its wave, then of the waves
   const int n = tid < E ? count[tid] : 0;
   const int nt = (n + a.tile_rows - 1) / a.tile_rows;
-  slots[tid] = n;
-  tile_at[tid] = nt;
-  __syncthreads();
-  for (int off = 1; off < E; off <<= 1) {   // inclusive sums
-    const int x = tid >= off ? slots[tid - off] : 0;
-    const int y = tid >= off ? tile_at[tid - off] : 0;
-    __syncthreads();
-    slots[tid] += x;
-    tile_at[tid] += y;
-    __syncthreads();
-  }
-  const int total = tile_at[E - 1];
-  const int s0 = slots[tid] - n, t0 = tile_at[tid] - nt;
-  if (tid < E) {
-    for (int i = 0; i < nt; ++i) {
-      int* t = a.tiles + 4L * (t0 + i);
-      t[0] = tid;
-      t[1] = s0 + i * a.tile_rows;
-      t[2] = min(a.tile_rows, n - i * a.tile_rows);
-      t[3] = total;
+  int slots = n, tile_at = nt;
+  if (tid < MOE_MAX_EXPERTS) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int x = __shfl_up(slots, off, 64), y = __shfl_up(tile_at, off, 64);
+      if (lane >= off) {
+        slots += x;
+        tile_at += y;
+      }
     }
+    if (lane == 63) {
+      wave_slots[tid >> 6] = slots;
+      wave_tiles[tid >> 6] = tile_at;
+    }
+  }
+  __syncthreads();
+  int total = 0, s0 = slots - n, t0 = tile_at - nt;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (i < tid >> 6) {
+      s0 += wave_slots[i];
+      t0 += wave_tiles[i];
+    }
+    total += wave_tiles[i];
+  }
+  if (tid < E) {
+    for (int i = 0; i < nt; ++i)
+      *(int4*)(a.tiles + 4L * (t0 + i)) = int4{
+          tid, s0 + i * a.tile_rows, min(a.tile_rows, n - i * a.tile_rows), total};
     count[tid] = s0;
   }
   for (int i = total + tid; i < a.max_tiles; i += 1024) a.tiles[4L * i + 2] = 0;
   __syncthreads();
-  for (int p = tid; p < pairs; p += 1024)
-    a.order[atomicAdd(&count[a.idx[p]], 1)] = p;
+  each([&](int p, int e) { a.order[atomicAdd(&count[e], 1)] = p; });
 }
 
 extern "C" int sv_moe_plan(const MoePlanArgs* a, int f32,
@@ -211,7 +266,7 @@ extern "C" int sv_moe_plan(const MoePlanArgs* a, int f32,
       a->keep > a->groups || a->keep * (a->E / a->groups) < a->top ||
       a->best < 1 || a->best > 2)
     return 1;
-  const bool fused = a->T <= 64;
+  const bool fused = a->T <= MOE_FUSED_ROWS;
   if (!fused) {
     const int grid = (a->T + 3) / 4;
     if (f32) moe_route_kernel<float><<<grid, 256, 0, stream>>>(*a);

@@ -487,3 +487,21 @@ def test_streamed_experts_at_their_edges(sv, E, top, T, W, ff, one):
         _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
         _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
                torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind", ["plain", "sigmoid", "softmax"])
+@pytest.mark.parametrize("T,E,top", [(16, 64, 64), (17, 64, 6), (16, 65, 9),
+                                     (17, 256, 40), (3, 257, 7), (64, 512, 64)])
+def test_equal_scores_are_chosen_by_index(sv, T, E, top, kind):
+    """Many equal scores, in one lane and over lanes; one kernel and two."""
+    z = _rand(T, E, dtype=torch.float32).mul(2).round().div(2)
+    p = sv.moe_plan(z.cuda(), None, sv.Routing(top, sigmoid=kind == "sigmoid",
+                                               softmax=kind == "softmax"), 0)
+    d = z.double()
+    want = d.sort(dim=1, descending=True, stable=True)[1][:, :top]
+    assert torch.equal(p.idx.cpu().long(), want)
+    s = torch.sigmoid(d) if kind == "sigmoid" else d.exp()
+    w = s.gather(1, want)
+    w = w / (s if kind == "softmax" else w).sum(1, keepdim=True)
+    _close(p.coef, w, torch.float32)
+    assert sorted(p.order.tolist()) == list(range(T * top))
