@@ -308,41 +308,21 @@ __device__ __forceinline__ float glu(const MoeGemmArgs& a, float g, float u) {
 // (DMA, K a multiple of 64) or through registers.  With a gated activation
 // the weight rows of a tile alternate 32 gate, 32 up, so a lane holds both of
 // a column.
+// slot0, rows: the tile's; tn: its columns
 template <int BM, int BN, int WM, int WN, bool GLU, bool DMA>
-__global__ void __launch_bounds__(BM / WM * BN / WN * 64)
-moe_tiles_kernel(MoeGemmArgs a) {
+__device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
+                                         int rows, int tn, short* xs0,
+                                         short* xs1, short* ws0, short* ws1) {
   constexpr int NT = BM / WM * BN / WN * 64;
   constexpr int CM = WM / 32, CN = WN / 32;
   constexpr int LX = BM * 8 / NT, LW = BN * 8 / NT;
-  constexpr int GROUP = 8;
   constexpr int NOUT = GLU ? BN / 2 : BN;    // columns of a tile's result
-  // apart by name, so that a read of one buffer need not wait for the words
-  // on their way into the other
-  __shared__ __attribute__((aligned(16))) short xs0[BM * 64], xs1[BM * 64];
-  __shared__ __attribute__((aligned(16))) short ws0[BN * 64], ws1[BN * 64];
-
-  // neighbours in the list of tiles run on one XCD: groups of GROUP slot
-  // tiles by all column tiles, slot tiles fastest
-  const int total = gridDim.x;
-  int id = blockIdx.x;
-  {
-    const int per = total / 8, rest = total % 8, xcd = id % 8;
-    id = xcd * per + min(xcd, rest) + id / 8;
-  }
-  const int ntn = (a.N + NOUT - 1) / NOUT;
-  const int g0 = id / (GROUP * ntn) * GROUP;
-  const int gm = min(GROUP, a.max_tiles - g0);
-  const int in = id - g0 * ntn;
-  const int tn = in / gm;
-  const int* tl = a.tiles + 4L * (g0 + in % gm);
-  const int rows = tl[2];
-  if (rows == 0) return;
-  const int e = tl[0], slot0 = tl[1];
-
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, hi = lane >> 5;
-  const int wm = wid % (BM / WM) * WM, wn = wid / (BM / WM) * WN;
+  // a SIMD has waves of all slots, so that it gains where some have no rows
+  const int wm = wid / (BN / WN) * WM, wn = wid % (BN / WN) * WN;
+  const bool idle = DMA && wm >= rows;
   const int K = a.K, N = a.N;
   // 16-byte slot (r, s) of a tile lies at place s ^ (r >> 1); thread tid
   // fills places tid, tid + NT, ... of a buffer, NT / 8 rows apart
@@ -409,6 +389,7 @@ moe_tiles_kernel(MoeGemmArgs a) {
         acc[n][m] = mfma_bf16(fw[c & 1][n].bf, fx[c & 1][m].bf, acc[n][m]);
   };
   auto step = [&](const short* xs, const short* ws) {
+    if (idle) return;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -443,6 +424,7 @@ moe_tiles_kernel(MoeGemmArgs a) {
     __syncthreads();
   }
   if (steps & 1) step(xs0, ws0);
+  if (idle) return;
   multiply(3);
 
 #pragma unroll
@@ -467,6 +449,61 @@ moe_tiles_kernel(MoeGemmArgs a) {
         *(uint2*)(dst + c) = uint2{pack_bf16x2(v[0], v[1]),
                                    pack_bf16x2(v[2], v[3])};
       }
+  }
+}
+
+// One workgroup a tile.  TAIL: the last tiles, if they leave half of the CUs
+// without one, are computed in halves of the slots, or quarters, by all of them
+// (36 tiles of 4096 x 14336, 576 workgroups on 256 CUs: 966 us, in whole tiles
+// 1128).
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL>
+__global__ void __launch_bounds__(BM / WM * BN / WN * 64)
+moe_tiles_kernel(MoeGemmArgs a) {
+  constexpr int GROUP = 8;
+  constexpr int NOUT = GLU ? BN / 2 : BN;
+  // apart by name, so that a read of one buffer need not wait for the words
+  // on their way into the other
+  __shared__ __attribute__((aligned(16))) short xs0[BM * 64], xs1[BM * 64];
+  __shared__ __attribute__((aligned(16))) short ws0[BN * 64], ws1[BN * 64];
+
+  // neighbours in the list of tiles run on one XCD: groups of GROUP slot
+  // tiles by all column tiles, slot tiles fastest.  The XCDs share the tiles
+  // that have rows (all places in the list, the last ones empty: gates of 36
+  // tiles of 28672 x 4096 2222 us, now 1789)
+  const int ntn = (a.N + NOUT - 1) / NOUT;
+  const int live = a.tiles[3], total = live * ntn;
+  const int tail = total % 256;
+  const int split = !TAIL || tail == 0 || tail > 128 ? 1 : tail > 64 ? 2 : 4;
+  const int whole = split > 1 ? total - tail : total;
+  int id = blockIdx.x, piece = 0;
+  if (id < whole) {
+    const int per = whole / 8, rest = whole % 8, xcd = id % 8;
+    id = xcd * per + min(xcd, rest) + id / 8;
+  } else {
+    piece = (id - whole) % split;
+    id = whole + (id - whole) / split;
+    if (id >= total) return;
+  }
+  const int g0 = id / (GROUP * ntn) * GROUP;
+  const int gm = min(GROUP, live - g0);
+  const int in = id - g0 * ntn;
+  const int tn = in / gm;
+  const int* tl = a.tiles + 4L * (g0 + in % gm);
+  const int e = tl[0], slot0 = tl[1], rows = tl[2];
+  if (!TAIL || id < whole) {
+    moe_tile<BM, BN, WM, WN, GLU, DMA>(a, e, slot0, rows, tn, xs0, xs1, ws0, ws1);
+    return;
+  }
+  if constexpr (TAIL) {
+    const int s = piece % 2 * (BM / 2);
+    if (s >= rows) return;
+    if (split == 2)
+      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn, xs0, xs1, ws0, ws1);
+    else if ((tn * 2 + piece / 2) * (NOUT / 2) < a.N)
+      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, xs0, xs1,
+          ws0, ws1);
   }
 }
 
@@ -729,11 +766,14 @@ template <int BM, int BN, int WM, int WN, bool GLU>
 static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
   constexpr int NOUT = GLU ? BN / 2 : BN;
   constexpr int NT = BM / WM * BN / WN * 64;
+  constexpr bool TAIL = BM == 256;
   const long grid = (long)a.max_tiles * ((a.N + NOUT - 1) / NOUT);
-  if (a.K % 64 == 0)
-    moe_tiles_kernel<BM, BN, WM, WN, GLU, true><<<grid, NT, 0, stream>>>(a);
+  if (a.K % 64 == 0)                     // at most 3 * 64 or 128 pieces more
+    moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL>
+        <<<grid + (TAIL ? 192 : 0), NT, 0, stream>>>(a);
   else
-    moe_tiles_kernel<BM, BN, WM, WN, GLU, false><<<grid, NT, 0, stream>>>(a);
+    moe_tiles_kernel<BM, BN, WM, WN, GLU, false, false>
+        <<<grid, NT, 0, stream>>>(a);
 }
 
 template <bool GLU>

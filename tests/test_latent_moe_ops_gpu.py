@@ -505,3 +505,28 @@ def test_equal_scores_are_chosen_by_index(sv, T, E, top, kind):
     w = w / (s if kind == "softmax" else w).sum(1, keepdim=True)
     _close(p.coef, w, torch.float32)
     assert sorted(p.order.tolist()) == list(range(T * top))
+
+
+@pytest.mark.parametrize("E,top,T,W,ff", [(2, 2, 700, 64, 1856),
+                                          (2, 2, 700, 128, 5824),
+                                          (1, 1, 300, 2304, 64),
+                                          (3, 1, 513, 192, 8192)])
+def test_last_tiles_in_halves_and_quarters(sv, E, top, T, W, ff):
+    """90, 6, 276 and 276, 12, 18, 2, ... workgroups of whole tiles: halves,
+    quarters, both after 256 whole ones; pieces without rows or columns."""
+    h = _rand(T, W, dtype=torch.bfloat16)
+    z = _rand(T, E, dtype=torch.float32, seed=1)
+    gu = _rand(E, 2 * ff, W, dtype=torch.bfloat16, seed=3, scale=W ** -0.5)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, seed=5, scale=ff ** -0.5)
+    p = sv.moe_plan(z.cuda(), None, top, 5)
+    act = sv.moe_gemm(h.cuda(), gu.cuda(), p, True)
+    y = sv.moe_gemm(act, down.cuda(), p, False)
+    order, idx = p.order.cpu().long(), p.idx.cpu().reshape(-1).long()
+    got = act.double().cpu()
+    for e in range(E):
+        slots = (idx[order] == e).nonzero()[:, 0]
+        pairs = order[slots]
+        g, u = (h[pairs // top].double() @ gu[e].double().T).chunk(2, 1)
+        _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
+        _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
+               torch.bfloat16)
