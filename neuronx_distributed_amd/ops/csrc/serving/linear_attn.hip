@@ -368,7 +368,8 @@ struct ChunkArgs {
   float* N;                 // [n_chunks][H][D] (gated): N, then n before
   short* P;                 // [n_chunks][H][3][E][D] state before the chunk
   float* mst;               // [n_chunks][H] m before the chunk (gated)
-  short* VT;                // [n_chunks][H][E][256] V^T, activated
+  short* VT;                // [n_chunks][H][E][256] V^T, activated; or null
+                            //   (timed, D 64 or 128, E a multiple of 64)
   short* KA;                // [T][H][D] activated K (decay); two planes of
                             //   rotated K (turned)
   short* QA;                // two planes of rotated Q (turned)
@@ -641,7 +642,7 @@ memory_states_kernel(ChunkArgs x) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int e = (i * 256 + tid) >> 3, sl = tid & 7;
-      if (e0 + e < E)
+      if (x.VT && e0 + e < E)
         *(uint4v*)(x.VT + (ci * E + e0 + e) * MC_L + c0 + 8 * sl) =
             *(const uint4v*)(vu + tslot(e, 8 * sl));
     }
@@ -1116,6 +1117,240 @@ memory_outputs_kernel(ChunkArgs x) {
     }
 }
 
+// ---- timed outputs of D = 64 or 128, 64 columns per workgroup ---------------
+// The same 128 queries, but all tiles come straight into LDS (DMA), one ahead:
+// the carried state's planes, 32 columns a tile, then keys and values, 64 tokens
+// a tile; values are turned by transposing reads.  Without tiles in registers
+// three workgroups share a CU: two wait half of the time for memory and barriers
+// (2 x 2048 tokens, 128 heads of 128 x 64: 207 -> 121 us, 300 MB of which are
+// 60).
+// The weights of an earlier group's keys are products: what is left at the end
+// of their group, and from there to the query.
+template <int DP>
+__global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
+  constexpr int NC = DP / 16, SL = DP / 8, KP = DP * 2;
+  constexpr int STATE = 3 * 32 * KP, KEYS = 64 * KP;
+  constexpr int OP = 68;                 // pitch of two waves' results
+  constexpr int SIZE = STATE > KEYS + 64 * 128 ? STATE : KEYS + 64 * 128;
+  constexpr int OUTS = 2 * 32 * OP * sizeof(float);
+  __shared__ __attribute__((aligned(16))) char b0[SIZE > OUTS ? SIZE : OUTS],
+      b1[SIZE > OUTS ? SIZE : OUTS];
+  __shared__ float s_col[MC_L], s_step[MC_L], s_far[MC_L];
+  const MemoryArgs& a = x.a;
+  const int E = a.E, nt = E / 64;
+  // the halves and the heads that share keys follow each other on one XCD
+  int id = blockIdx.x;
+  {
+    const int total = gridDim.x, per = total / 8, rest = total % 8, xcd = id % 8;
+    id = xcd * per + min(xcd, rest) + id / 8;
+  }
+  const int half = id & 1, et = id / 2 % nt;
+  const int h = id / 2 / nt % a.H, ch = id / 2 / nt / a.H;
+  const int row0 = x.chunks[4 * ch + 1], nrow = x.chunks[4 * ch + 2];
+  const bool carried = x.chunks[4 * ch + 3];
+  if (half * 128 >= nrow) return;        // the whole workgroup
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hi = lane >> 5;
+  const int e0 = et * 64;
+  const long ci = (long)ch * a.H + h;
+  const int t = half * 128 + wid * 32 + col;   // place in the chunk
+  const int tt = half * 4 + wid, jt = tt >> 1; // its 32 and 64 tokens
+  const int hk = h / (a.H / a.G);
+
+  // thread tid fills 16-byte places tid, tid + 256, ... of a tile
+  auto turn = [](int r) { return SL == 16 ? row_turn(r) : key_turn<SL>(r); };
+  const short* P = x.P + (ci * 3 * E + e0) * DP;
+  auto issue_state = [&](int nb, char* buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < STATE / 4096; ++p) {
+      const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
+      __builtin_amdgcn_global_load_lds(
+          (global_ptr)(P + ((long)(r >> 5) * E + 32 * nb + (r & 31)) * DP + s * 8),
+          (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16, 0, 0);
+    }
+  };
+  const short* kp = (const short*)a.k + (long)row0 * a.kst + hk * DP;
+  const short* vp = (const short*)a.v + (long)row0 * a.vst + (long)h * E + e0;
+  auto issue = [&](int J, char* buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < KEYS / 4096; ++p) {
+      const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
+      __builtin_amdgcn_global_load_lds(
+          (global_ptr)(kp + min(64 * J + r, nrow - 1) * a.kst + s * 8),
+          (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int r = (p * 256 + tid) >> 3, s = (tid & 7) ^ value_turn<8>(r);
+      __builtin_amdgcn_global_load_lds(
+          (global_ptr)(vp + min(64 * J + r, nrow - 1) * a.vst + s * 8),
+          (lds_ptr)(buf + KEYS + (p * 256 + wid * 64) * 16), 16, 0, 0);
+    }
+  };
+  const int J1 = min(half * 2 + 1, (nrow - 1) / 64);
+  if (carried) issue_state(0, b0);
+  else issue(J1, b0);
+
+  frag_u qf[NC];
+  const short* q = (const short*)a.q + (row0 + min(t, nrow - 1)) * a.qst + hk * DP;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) qf[c].u4 = *(const uint4v*)(q + c * 16 + hi * 8);
+  float tot[4], before = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    tot[j] = x.tot[ci * 4 + j];
+    if (j < jt) before += tot[j];
+  }
+  const long ho = (long)h * x.T + row0;
+  const float bt = x.b[ho + min(t, nrow - 1)];
+  {
+    float c = -INFINITY, s = 0.f;
+    if (tid < nrow) {
+      c = -x.b[ho + tid];
+      s = x.i[ho + tid];
+    }
+    s_col[tid] = c;
+    s_step[tid] = s;
+    s_far[tid] = __expf(tot[0] * (wid == 0) + tot[1] * (wid == 1) +
+                        tot[2] * (wid == 2) + tot[3] * (wid == 3) + c) * s;
+  }
+  const float inter = __expf(bt + before);
+
+  // this lane's part of the addresses: slot 2 c + hi of row col; a transposing
+  // read, where 16 lanes turn 4 keys by 16 columns
+  const int kx = SL == 16 ? row_lane(col, hi)
+                          : col * KP + (hi ^ key_turn<SL>(col)) * 16;
+  const int tr_key = 4 * hi + ((lane & 15) >> 2);
+  const int vx = (tr_key * 64 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4 +
+                  value_turn<8>(tr_key) * 8) * 2;
+  f32x16 ot[2] = {};
+  auto state = [&](int nb, const char* buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int z = 0; z < 3; ++z)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        frag_u sf;
+        sf.u4 = *(const uint4v*)(buf + z * 32 * KP + (kx ^ (32 * c)));
+        ot[nb] = mfma_bf16(sf.bf, qf[c].bf, ot[nb]);
+      }
+    ot[nb] *= inter;
+  };
+  const bool rows = half * 128 + wid * 32 < nrow;
+  auto keys = [&](int J, const char* buf) __attribute__((always_inline)) {
+    if (J > jt || !rows) return;         // wave-uniform
+    float from = bt;                     // from the end of the group
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j > J && j < jt) from += tot[j];
+    from = __expf(from);
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2) {
+      if (2 * J + k2 > tt) break;        // later keys
+      f32x16 acc = {};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        frag_u kf;
+        kf.u4 = *(const uint4v*)(buf + k2 * 32 * KP + (kx ^ (32 * c)));
+        acc = mfma_bf16(kf.bf, qf[c].bf, acc);
+      }
+      const int s0 = 64 * J + 32 * k2;
+      if (J < jt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[r] *= s_far[s0 + acc_row(r, hi)] * from;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int s = s0 + acc_row(r, hi);
+          const float w = __expf(bt + s_col[s]) * s_step[s];
+          acc[r] *= s > t ? 0.f : w;
+        }
+      }
+#pragma unroll
+      for (int cc = 0; cc < 2; ++cc) {
+        frag_u pf[3];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          uint w[3];
+          split3(acc[8 * cc + 2 * u], acc[8 * cc + 2 * u + 1], w);
+#pragma unroll
+          for (int z = 0; z < 3; ++z) pf[z].u[u] = w[z];
+        }
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+          union { tr4 t[2]; bf16x8 bf; } vf;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_tr4)(buf + KEYS + (vx ^ (nb * 64)) +
+                          (32 * k2 + 16 * cc + 8 * u) * 128));
+#pragma unroll
+          for (int z = 0; z < 3; ++z) ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
+        }
+      }
+    }
+  };
+  if (carried) {
+    __syncthreads();                     // also waits for the words on their way
+    issue_state(1, b1);
+    state(0, b0);
+    __syncthreads();
+    issue(J1, b0);
+    state(1, b1);
+  }
+  for (int J = J1;; J -= 2) {            // from the newest keys back
+    __syncthreads();
+    if (J > 0) issue(J - 1, b1);
+    keys(J, b0);
+    if (J == 0) break;
+    __syncthreads();
+    if (J > 1) issue(J - 2, b0);
+    keys(J - 1, b1);
+    if (J == 1) break;
+  }
+
+  // through LDS, so that every row is read and written as a whole (8 bytes a
+  // lane, each of another row: 163 us in place of 121)
+  float* o = (float*)(wid < 2 ? b0 : b1) + (wid & 1) * 32 * OP;
+  const float skip = bits2f(((const short*)a.skip)[h]);
+  const int r0 = half * 128 + wid * 32 + (lane >> 3), c0 = (lane & 7) * 8;
+  const long at = (long)h * E + e0 + c0;
+  uint4v vv[4], zz[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const long r = row0 + min(r0 + 8 * i, nrow - 1);
+    vv[i] = *(const uint4v*)((const short*)a.v + r * a.vst + at);
+    zz[i] = *(const uint4v*)((const short*)a.z + r * a.zst + at);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg)
+      *(f32x4*)(o + col * OP + 32 * nb + 8 * rg + 4 * hi) =
+          f32x4{ot[nb][4 * rg], ot[nb][4 * rg + 1], ot[nb][4 * rg + 2],
+                ot[nb][4 * rg + 3]};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (r0 + 8 * i >= nrow) break;
+    const float* src = o + ((lane >> 3) + 8 * i) * OP + c0;
+    float y[8], v[8], z[8];
+    load4(src, y);
+    load4(src + 4, y + 4);
+    unpack8(vv[i], v);
+    unpack8(zz[i], z);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[j] = (y[j] + skip * v[j]) * silu_f(z[j]);
+    uint4v w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(y[2 * j], y[2 * j + 1]);
+    *(uint4v*)((short*)a.out + (long)(row0 + r0 + 8 * i) * a.H * E + at) = w;
+  }
+}
+
 // wider column tiles read the keys less often, as long as the accumulators
 // leave registers for two workgroups per CU
 template <int DP, int GATE>
@@ -1133,6 +1368,11 @@ static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
       <<<ch * ((a.E + 63) / 64), 256, 0, stream>>>(x);
   memory_scan_kernel<GATE><<<(long)x.n_seg * a.H * ((a.D + 63) / 64) *
                                  ((a.E + 15) / 16), 256, 0, stream>>>(x);
+  if constexpr (GATE == TIMED && DP <= 128)
+    if (!x.VT) {
+      memory_timed_kernel<DP><<<ch * 2 * (a.E / 64), 256, 0, stream>>>(x);
+      return;
+    }
   if (a.E <= 64 || DP > 128)
     memory_outputs_kernel<DP, 64, GATE>
         <<<ch * 2 * ((a.E + 63) / 64), 256, 0, stream>>>(x);
@@ -1148,6 +1388,9 @@ extern "C" int sv_memory_chunks(const ChunkArgs* x, int gating,
   if (gating == TURNED &&
       (x->a.rot % 2 || x->a.rot > x->a.D ||
        (x->a.z && (x->a.E > 128 || (x->a.E > 64 && x->a.D > 128)))))
+    return 1;
+  if (!x->VT && (gating != TIMED || x->a.E % 64 ||
+                 (x->a.D != 64 && x->a.D != 128)))
     return 1;
 #define MC(P)                                                     \
   do {                                                            \

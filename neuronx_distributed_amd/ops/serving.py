@@ -1006,8 +1006,9 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         U = torch.empty(nc, heads, E, D, **f32)
         P = torch.empty(nc, heads, 3, E, D, dtype=torch.bfloat16,
                         device=q.device)
-        VT = torch.empty(nc, heads, E, CHUNK, dtype=torch.bfloat16,
-                         device=q.device)
+        VT = None if timed and D in (64, 128) and E % 64 == 0 else \
+            torch.empty(nc, heads, E, CHUNK, dtype=torch.bfloat16,
+                        device=q.device)
         KA = torch.empty(T, heads * D, dtype=q.dtype, device=q.device) \
             if isinstance(gate, DecayGate) else None
         if turned:

@@ -688,3 +688,35 @@ def test_few_rows_are_streamed_where_nobody_watches(glu):
         with Watch():
             assert sv.streamed(x, w, glu=glu) is None
         assert not any("empty" in str(f) for f in seen)
+
+
+@pytest.mark.parametrize("H,G,N,P", [(2, 1, 64, 64), (6, 3, 128, 128),
+                                     (3, 1, 64, 192), (16, 2, 128, 64)])
+def test_timed_memory_in_tiles(H, G, N, P):
+    """Sizes whose tiles come straight into LDS: portions that end around 32,
+    64, 128 and 256 tokens, from zero and from a carried state, rows that lie
+    in wider ones."""
+    lens = [257, 33, 90, 512, 31, 129, 65, 192]
+    firsts = [0, 1, 32, 256, 30, 64, 0, 191]
+    cases = [_ssm(n, H, G, N, P, 20 * i, BF16) for i, n in enumerate(lens)]
+    params = _ssm_params(H, BF16)
+    want = [_ssm_want(c, params, H, G, N, P) for c in cases]
+    S = torch.zeros(len(lens), H, N, P, device="cuda")
+    got = [[] for _ in lens]
+    for begin in (True, False):
+        part = [(i, 0 if begin else f, f if begin else n)
+                for i, (f, n) in enumerate(zip(firsts, lens))]
+        part = [p for p in part if p[2] > p[1]]
+        x, B, C, z, raw = (torch.cat([cases[i][j][a:b] for i, a, b in part])
+                           for j in range(5))
+        wide = torch.cat([z, x, B, C], 1).cuda()       # rows of a projection
+        z, x, B, C = wide.split([H * P, H * P, G * N, G * N], 1)
+        seg, chunks, first = _segments([(i, b - a, a) for i, a, b in part])
+        out = sv.memory_mix(C, B, x, sv.TimeGate(
+            raw.cuda(), *[t.cuda() for t in params], z), S, None, None, seg,
+            H, chunks, first)
+        for (i, a, b), o in zip(part, out.split([b - a for _, a, b in part])):
+            got[i].append(o)
+    for i, w in enumerate(want):
+        _near(torch.cat(got[i]), w[0], BF16, i)
+        _near(S[i], w[1], F32, i, 2e-5)
