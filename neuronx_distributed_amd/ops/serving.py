@@ -55,7 +55,9 @@ def ensure_built():
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the current stream's handle alone (0.3 us, with the object around it 2.9)
+    return ctypes.c_void_p(
+        torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -607,15 +609,20 @@ def softcap_(x: torch.Tensor, cap: float) -> torch.Tensor:
 
 def _aligned(sizes, *tensors) -> bool:
     """Can rows be read in 16-byte pieces of 8 bf16 (or 2 x 4 f32)?"""
-    return all(s % 8 == 0 for s in sizes) and all(
-        t.stride(0) % 8 == 0 and t.storage_offset() % 8 == 0
-        for t in tensors)
+    return not _low_bits(sizes, tensors) & 7
 
 
 def _vec4(sizes, *tensors) -> int:
-    return int(all(s % 4 == 0 for s in sizes) and all(
-        t.stride(0) % 4 == 0 and t.storage_offset() % 4 == 0
-        for t in tensors))
+    return int(not _low_bits(sizes, tensors) & 3)
+
+
+def _low_bits(sizes, tensors) -> int:
+    bits = 0
+    for s in sizes:
+        bits |= s
+    for t in tensors:
+        bits |= t.stride(0) | t.storage_offset()
+    return bits
 
 
 def _check_cache(q, k, v, kc, vc, H):
