@@ -14,7 +14,8 @@ from ..parallel.layers import (
     ParallelEmbedding,
 )
 from ..parallel.layer_norm import LayerNorm
-from ..parallel.loss_functions import parallel_cross_entropy
+from ..parallel.loss_functions import (
+    next_token_cross_entropy, parallel_cross_entropy)
 
 # fx.wrap patches name lookups in THIS module's globals (the defining
 # module's wrap does not cover imported references) so the pipeline tracer
@@ -148,5 +149,8 @@ class GPT2LMHeadModel(nn.Module):
         if labels is None:
             return logits
         shift = labels[:, 1:].contiguous()
-        loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(), shift)
+        loss = next_token_cross_entropy(logits, labels)
+        if loss is None:
+            loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(),
+                                          shift)
         return loss.sum() / (shift != -100).sum().clamp(min=1)

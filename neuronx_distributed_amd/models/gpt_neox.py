@@ -19,7 +19,8 @@ from ..parallel.layers import (
     ParallelEmbedding,
     RowParallelLinear,
 )
-from ..parallel.loss_functions import parallel_cross_entropy
+from ..parallel.loss_functions import (
+    next_token_cross_entropy, parallel_cross_entropy)
 
 torch.fx.wrap("parallel_cross_entropy")
 
@@ -200,5 +201,8 @@ class GPTNeoXForCausalLM(nn.Module):
         if labels is None:
             return logits
         shift = labels[:, 1:].contiguous()
-        loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(), shift)
+        loss = next_token_cross_entropy(logits, labels)
+        if loss is None:
+            loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(),
+                                          shift)
         return loss.sum() / (shift != -100).sum().clamp(min=1)

@@ -29,7 +29,8 @@ from ..parallel.layers import (
     ParallelEmbedding,
 )
 from ..parallel.qkv_linear import GQAQKVColumnParallelLinear
-from ..parallel.loss_functions import parallel_cross_entropy
+from ..parallel.loss_functions import (
+    next_token_cross_entropy, parallel_cross_entropy)
 
 # fx.wrap patches name lookups in THIS module's globals (the defining
 # module's wrap does not cover imported references) so the pipeline tracer
@@ -571,6 +572,9 @@ class LlamaForCausalLM(nn.Module):
         if labels is None:
             return logits
         shift = labels[:, 1:].contiguous()
-        loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(), shift)
+        loss = next_token_cross_entropy(logits, labels)
+        if loss is None:
+            loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(),
+                                          shift)
         valid = (shift != -100).sum().clamp(min=1)
         return loss.sum() / valid

@@ -30,7 +30,8 @@ from ..moe.model import MoE
 from ..moe.routing import (GroupLimitedRouter, RouterSinkhorn, RouterTopK)
 from ..moe.shared_experts import SharedExperts
 from ..parallel.layers import ColumnParallelLinear, ParallelEmbedding
-from ..parallel.loss_functions import parallel_cross_entropy
+from ..parallel.loss_functions import (
+    next_token_cross_entropy, parallel_cross_entropy)
 from ..parallel.mappings import (
     gather_from_sequence_parallel_region,
     scatter_to_sequence_parallel_region,
@@ -267,9 +268,11 @@ class MixtralForCausalLM(nn.Module):
         if labels is None:
             return logits
         shift = labels[:, 1:].contiguous()
-        loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(),
-                                      shift).sum() / \
-            (shift != -100).sum().clamp(min=1)
+        loss = next_token_cross_entropy(logits, labels)
+        if loss is None:
+            loss = parallel_cross_entropy(logits[:, :-1, :].contiguous(),
+                                          shift)
+        loss = loss.sum() / (shift != -100).sum().clamp(min=1)
         if router_logits and self.config.router_aux_loss_coef > 0:
             aux = load_balancing_loss_func(
                 torch.cat(router_logits, dim=0),

@@ -20,6 +20,13 @@ from . import comm
 from . import parallel_state as ps
 
 
+def _over(rowmax, own, sumexp, predicted, owned):
+    """A shard's sum and predicted logit over the max of all shards."""
+    less = own - rowmax
+    return torch.stack((sumexp * less.exp(),
+                        torch.where(owned, predicted + less, 0.0)))
+
+
 class _FusedParallelCrossEntropy(torch.autograd.Function):
     """HIP-fused path (ops/csrc/cross_entropy.hip): bf16 logits shard, no
     fp32/softmax materialization; backward recomputes exp."""
@@ -37,18 +44,22 @@ class _FusedParallelCrossEntropy(torch.autograd.Function):
         dev = logits.device
         t64 = target.reshape(-1).to(torch.int64).contiguous()
 
-        rowmax = torch.empty(N, dtype=torch.float32, device=dev)
-        lib.ce_rowmax(ops._ptr(logits), ops._ptr(rowmax), ctypes.c_long(N),
-                      ctypes.c_int(V), ops._stream())
-        comm.all_reduce(rowmax, op=dist.ReduceOp.MAX, group=tp)
-
-        se_pred = torch.empty(2, N, dtype=torch.float32, device=dev)
-        lib.ce_sumexp(ops._ptr(logits), ops._ptr(rowmax), ops._ptr(t64),
-                      ops._ptr(se_pred[0]), ops._ptr(se_pred[1]),
-                      ctypes.c_long(N), ctypes.c_int(V),
-                      ctypes.c_long(tp_rank * V), ops._stream())
-        comm.all_reduce(se_pred, group=tp)
-        sumexp, predicted = se_pred[0], se_pred[1]
+        stats = torch.empty(3, N, dtype=torch.float32, device=dev)
+        lib.ce_stats(ops._ptr(logits), ops._ptr(t64), ops._ptr(stats[0]),
+                     ops._ptr(stats[1]), ops._ptr(stats[2]),
+                     ctypes.c_long(N), ctypes.c_int(V),
+                     ctypes.c_long(tp_rank * V), ops._stream())
+        rowmax, sumexp, predicted = stats
+        if comm.group_size(tp) > 1:
+            # from the shard's own max to that of all shards
+            own = rowmax
+            rowmax = own.clone()
+            comm.all_reduce(rowmax, op=dist.ReduceOp.MAX, group=tp)
+            at = t64 - tp_rank * V
+            se_pred = _over(rowmax, own, sumexp, predicted,
+                            (at >= 0) & (at < V))
+            comm.all_reduce(se_pred, group=tp)
+            sumexp, predicted = se_pred
         loss = (sumexp.log() - predicted).reshape(target.shape)
         ctx.save_for_backward(logits, rowmax, sumexp, t64)
         ctx.vocab_start = tp_rank * V
@@ -131,26 +142,38 @@ class _ParallelCrossEntropy(torch.autograd.Function):
         return grad_input, None, None
 
 
+def _fused(logits) -> bool:
+    if (isinstance(logits, torch.fx.Proxy) or not logits.is_cuda
+            or logits.dtype != torch.bfloat16 or logits.shape[-1] % 8):
+        return False
+    from .. import ops
+
+    return ops.is_available()
+
+
+def next_token_cross_entropy(logits, labels):
+    """Loss of every position's logits (B, S, V/tp) against the label after it
+    by the fused kernels; None where they do not apply.  The last position is
+    ignored like a padded one, so the logits are neither copied without it nor
+    their gradients filled up with zeros (8192 x 32000: 470 us of passes)."""
+    if not _fused(logits):
+        return None
+    return parallel_cross_entropy(
+        logits, torch.nn.functional.pad(labels[:, 1:], (0, 1), value=-100))
+
+
 def parallel_cross_entropy(vocab_parallel_logits, target, label_smoothing=0.0,
                            ignore_index=-100):
     """Per-token loss on vocab-sharded logits (reference loss_functions.py:217).
     GPU bf16 + no smoothing dispatches to the fused HIP kernels.
 
     Targets equal to ``ignore_index`` (HF padding convention) contribute
-    ZERO loss and zero gradient (the mask multiply below routes a zero
+    ZERO loss and zero gradient (the mask below routes a zero
     grad_output into the CE backward); callers wanting mean-over-valid
     divide by the valid count (see the model zoo loss heads)."""
-    if (not isinstance(vocab_parallel_logits, torch.fx.Proxy)
-            and vocab_parallel_logits.is_cuda
-            and vocab_parallel_logits.dtype == torch.bfloat16
-            and label_smoothing == 0.0
-            and vocab_parallel_logits.shape[-1] % 8 == 0):
-        from .. import ops
-
-        if ops.is_available():
-            raw = _FusedParallelCrossEntropy.apply(vocab_parallel_logits,
-                                                   target)
-            return raw * (target != ignore_index).to(raw.dtype)
+    if label_smoothing == 0.0 and _fused(vocab_parallel_logits):
+        raw = _FusedParallelCrossEntropy.apply(vocab_parallel_logits, target)
+        return raw.masked_fill(target == ignore_index, 0.0)
     if not isinstance(vocab_parallel_logits, torch.fx.Proxy) and \
             vocab_parallel_logits.dtype in (torch.bfloat16, torch.float16):
         vocab_parallel_logits = vocab_parallel_logits.float()

@@ -1,7 +1,9 @@
 """GPU numerics: every HIP kernel vs the plain-torch fp32 reference
 (the CPU fallback implementations in ops/__init__.py and kernels/)."""
 
+import ctypes
 import math
+import os
 
 import pytest
 import torch
@@ -651,3 +653,99 @@ def test_flash_attn_windowed_bwd(B, Hq, Hkv, S, W):
     _cmp(q.grad, ref_in[0].grad * 0.5, atol=5e-2, rtol=5e-2, name="win dq")
     _cmp(k.grad, ref_in[1].grad * 0.5, atol=5e-2, rtol=5e-2, name="win dk")
     _cmp(v.grad, ref_in[2].grad * 0.5, atol=5e-2, rtol=5e-2, name="win dv")
+
+
+def _one_rank():
+    import torch.distributed as dist
+    from neuronx_distributed_amd.parallel import parallel_state as ps
+
+    if not dist.is_initialized():
+        os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
+        os.environ.setdefault("MASTER_PORT", "29553")
+        dist.init_process_group("nccl", rank=0, world_size=1)
+    if not ps.model_parallel_is_initialized():
+        ps.initialize_model_parallel(tensor_model_parallel_size=1)
+
+
+@pytest.mark.parametrize("N,V", [(1, 8), (3, 2040), (5, 2048), (2, 8200),
+                                 (2100, 16376)])
+def test_fused_ce_in_one_pass(N, V):
+    """Loss and gradient against 64 bits; rows that rise, that hold -inf and
+    that are far out; an ignored row of NaN stays out of both."""
+    from neuronx_distributed_amd.parallel.loss_functions import (
+        parallel_cross_entropy)
+
+    _one_rank()
+    torch.manual_seed(0)
+    x = torch.randn(N, V, device="cuda")
+    tgt = torch.randint(0, V, (N,), device="cuda")
+    if N > 2:
+        x[0] = torch.linspace(-30, 30, V)
+        x[1] -= 3e4
+        x[2, 1::2] = float("-inf")
+        tgt[2] = 4
+    if N > 4:
+        x[3] = float("nan")
+        tgt[3] = -100
+    x = x.bfloat16().requires_grad_()
+    loss = parallel_cross_entropy(x, tgt)
+    (loss * torch.arange(1, N + 1, device="cuda")).sum().backward()
+    keep = tgt != -100
+    d = x.detach().double()[keep].requires_grad_()
+    ref = torch.nn.functional.cross_entropy(d, tgt[keep], reduction="none")
+    (ref * torch.arange(1, N + 1, device="cuda")[keep]).sum().backward()
+    # V exponentials of 2 ulp summed in 32 bits, each thread V / 256 of them
+    torch.testing.assert_close(loss[keep].double(), ref.detach(), rtol=1e-5,
+                               atol=2.0 ** -23 * (8 + V / 256))
+    torch.testing.assert_close(x.grad[keep].double(), d.grad, rtol=2.0 ** -7,
+                               atol=1e-6 * N)
+    assert (loss[~keep] == 0).all() and (x.grad[~keep] == 0).all()
+
+
+def test_next_token_loss_ignores_the_last_position():
+    from neuronx_distributed_amd.parallel.loss_functions import (
+        next_token_cross_entropy, parallel_cross_entropy)
+
+    _one_rank()
+    torch.manual_seed(1)
+    x = torch.randn(2, 37, 512, device="cuda").bfloat16()
+    labels = torch.randint(0, 512, (2, 37), device="cuda")
+    labels[0, 5:9] = -100
+    a, b = (x.clone().requires_grad_() for _ in range(2))
+    want = parallel_cross_entropy(a[:, :-1].contiguous(),
+                                  labels[:, 1:].contiguous())
+    got = next_token_cross_entropy(b, labels)
+    assert torch.equal(got[:, :-1], want) and (got[:, -1] == 0).all()
+    want.sum().backward()
+    got.sum().backward()
+    assert torch.equal(a.grad, b.grad)
+    assert next_token_cross_entropy(x.float(), labels) is None
+    assert next_token_cross_entropy(x.cpu(), labels.cpu()) is None
+
+
+def test_ce_shards_meet_at_the_common_max():
+    """What ranks all-reduce, for two halves of the vocabulary in one process;
+    one half all -inf in a row."""
+    from neuronx_distributed_amd.parallel import loss_functions as lf
+
+    torch.manual_seed(2)
+    x = torch.randn(6, 512, device="cuda").mul(4).bfloat16()
+    x[2, :256] = float("-inf")
+    tgt = torch.tensor([0, 255, 300, 511, -100, 256], device="cuda")
+    parts = []
+    for i in range(2):
+        half = x[:, i * 256:(i + 1) * 256].contiguous()
+        st = torch.empty(3, 6, device="cuda")
+        ops._require_lib().ce_stats(
+            ops._ptr(half), ops._ptr(tgt), ops._ptr(st[0]), ops._ptr(st[1]),
+            ops._ptr(st[2]), ctypes.c_long(6), ctypes.c_int(256),
+            ctypes.c_long(256 * i), ops._stream())
+        parts.append(st)
+    top = torch.maximum(parts[0][0], parts[1][0])
+    both = sum(lf._over(top, *p, (tgt >= 256 * i) & (tgt < 256 * i + 256))
+               for i, p in enumerate(parts))
+    loss = (both[0].log() - both[1]).double()
+    ref = torch.nn.functional.cross_entropy(x.double(), tgt.clamp(min=0),
+                                            reduction="none")
+    keep = tgt >= 0
+    torch.testing.assert_close(loss[keep], ref[keep], rtol=1e-5, atol=1e-5)
