@@ -79,6 +79,26 @@ def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
 # RMSNorm
 # ---------------------------------------------------------------------------
 
+def _rmsnorm_bwd(x, weight, dy, rstd, dpass=None):
+    """dx (+ dpass) and dw of contiguous bf16 rows x."""
+    lib = _require_lib()
+    H = x.shape[-1]
+    rows = x.numel() // H
+    # named, so that copies live until the launch
+    w, dy = weight.contiguous(), dy.contiguous()
+    dpass = None if dpass is None else dpass.contiguous()
+    dx = torch.empty_like(x)
+    short = weight.dtype == torch.bfloat16
+    dw = torch.empty(H, dtype=weight.dtype if short else torch.float32,
+                     device=x.device)
+    part = torch.empty(lib.rmsnorm_bwd_parts(rows), H, dtype=torch.float32,
+                       device=x.device)
+    lib.rmsnorm_bwd(_ptr(x), _ptr(w), _ptr(dy), _ptr(rstd),
+                    None if dpass is None else _ptr(dpass), _ptr(dx),
+                    _ptr(part), _ptr(dw), int(not short), rows, H, _stream())
+    return dx, dw.to(weight.dtype)
+
+
 class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps):
@@ -106,15 +126,7 @@ class _RMSNormFn(torch.autograd.Function):
         x, weight, rstd = ctx.saved_tensors
         H = x.shape[-1]
         if x.is_cuda and x.dtype == torch.bfloat16 and H % 8 == 0:
-            lib = _require_lib()
-            dy2 = dy.contiguous()
-            rows = x.numel() // H
-            dx = torch.empty_like(x)
-            dw32 = torch.zeros(H, dtype=torch.float32, device=x.device)
-            lib.rmsnorm_bwd(_ptr(x), _ptr(weight.contiguous()), _ptr(dy2),
-                            _ptr(rstd), _ptr(dx), _ptr(dw32),
-                            ctypes.c_int(rows), ctypes.c_int(H), _stream())
-            return dx, dw32.to(weight.dtype), None
+            return (*_rmsnorm_bwd(x, weight, dy, rstd), None)
         xf = x.float()
         dyf = dy.float()
         wf = weight.float()
@@ -155,7 +167,7 @@ class _AddRMSNormFn(torch.autograd.Function):
     """Training fused residual-add + RMSNorm: (delta, res) -> (h, normed)
     with h = bf16(delta + res), normed = rmsnorm(h) * w.  The backward
     folds the residual fork's pass-through gradient dh into the RMSNorm
-    backward pass (``rmsnorm_bwd_add``), so the fused site costs one
+    backward pass, so the fused site costs one
     kernel in each direction instead of norm + a 3-pass eager add
     (CUDAFunctor_add was ~2%% of the training step)."""
 
@@ -195,21 +207,8 @@ class _AddRMSNormFn(torch.autograd.Function):
             # grads pass straight through, no weight grad
             return dh, dh, None, None
         if h.is_cuda and h.dtype == torch.bfloat16 and H % 8 == 0:
-            lib = _require_lib()
-            rows = h.numel() // H
-            dy = dnormed.contiguous()
-            dx = torch.empty_like(h)
-            dw32 = torch.zeros(H, dtype=torch.float32, device=h.device)
-            if dh is None:
-                lib.rmsnorm_bwd(_ptr(h), _ptr(weight.contiguous()),
-                                _ptr(dy), _ptr(rstd), _ptr(dx), _ptr(dw32),
-                                rows, H, _stream())
-            else:
-                lib.rmsnorm_bwd_add(_ptr(h), _ptr(weight.contiguous()),
-                                    _ptr(dy), _ptr(rstd),
-                                    _ptr(dh.contiguous()), _ptr(dx),
-                                    _ptr(dw32), rows, H, _stream())
-            return dx, dx, dw32.to(weight.dtype), None
+            dx, dw = _rmsnorm_bwd(h, weight, dnormed, rstd, dh)
+            return dx, dx, dw, None
         hf = h.float()
         dyf = dnormed.float()
         wf = weight.float()

@@ -749,3 +749,36 @@ def test_ce_shards_meet_at_the_common_max():
                                             reduction="none")
     keep = tgt >= 0
     torch.testing.assert_close(loss[keep], ref[keep], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("rows,H", [(1, 8), (2, 2048), (511, 2056),
+                                    (513, 4096), (1025, 4104), (3, 6152),
+                                    (1030, 8192), (515, 8200), (0, 64)])
+@pytest.mark.parametrize("forked", [False, True])
+def test_rmsnorm_rows_and_widths(rows, H, forked):
+    """Forward and backward against 64 bits around the rows of a round of
+    workgroups and the columns of a thread."""
+    torch.manual_seed(rows + H)
+    x, r = (torch.randn(rows, H, device="cuda").bfloat16().requires_grad_()
+            for _ in range(2))
+    w = torch.randn(H, device="cuda").bfloat16().requires_grad_()
+    gy, gh = (torch.randn(rows, H, device="cuda").bfloat16()
+              for _ in range(2))
+    if forked:
+        h, y = ops.add_rmsnorm_train(x, r, w, 1e-5)
+        torch.autograd.backward([h, y], [gh, gy])
+    else:
+        y = ops.rmsnorm(x, w, 1e-5)
+        y.backward(gy)
+    d = (x + r if forked else x).detach().double().requires_grad_()
+    wd = w.detach().double().requires_grad_()
+    ref = d * torch.rsqrt(d.pow(2).mean(-1, keepdim=True) + 1e-5) * wd
+    ref.backward(gy.double())
+    # rounded once to 8 bits; 32-bit sums of H columns or of the rows
+    for got, want in ((y, ref), (x.grad, d.grad + (gh if forked else 0))):
+        torch.testing.assert_close(got.double(), want, rtol=2.0 ** -7,
+                                   atol=1e-4)
+    torch.testing.assert_close(w.grad.double(), wd.grad, rtol=2.0 ** -7,
+                               atol=1e-4 * max(rows, 1) ** 0.5)
+    if forked:
+        assert torch.equal(x.grad, r.grad)
