@@ -1334,11 +1334,20 @@ def moe_kernel(pairs: int, experts: int, width: int = 0, ff: int = 0) -> int:
     (measured): streaming up to 24 rows an expert where workgroups can stay with
     their rows (width and ff up to 4096), 16 where only the gates' can; else the
     rows are read again and again, and tiles are faster from 4 on (256 experts
-    7168 x 2048, 4 rows: 3.64 ms, streamed 4.21)."""
+    7168 x 2048, 4 rows: 3.64 ms, streamed 4.21).  Tiles of 128 and 256 slots
+    read weights two steps ahead where width and ff are multiples of 64, and are
+    the faster ones from 24 (64 experts 2048 x 1408, 72 rows: 64 slots 305 us,
+    128 262) and 112 rows on (128 rows: 128 slots 341, 256 322); long rows of few
+    slots are read faster by two workgroups a CU (8 experts 4096 x 14336, 32
+    rows: 64 slots 577, 128 603, from 48 rows on 608)."""
     rows = pairs / experts
     stay = 0 < width <= 4096
     if rows < ((24 if ff <= 4096 else 16) if stay else 4):
         return MOE_STREAM
+    if rows >= 24 and width and not (width | ff) & 63:
+        if rows < 48 and max(width, ff) > 4096:
+            return MOE_TILES[1]
+        return MOE_TILES[2 if rows < 112 else 3]
     return MOE_TILES[sum(rows >= r for r in (24, 112, 160))]
 
 

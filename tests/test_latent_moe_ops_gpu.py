@@ -530,3 +530,27 @@ def test_last_tiles_in_halves_and_quarters(sv, E, top, T, W, ff):
         _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
         _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
                torch.bfloat16)
+
+
+@pytest.mark.parametrize("how", [4, 5])
+@pytest.mark.parametrize("W,ff", [(64, 128), (192, 64), (320, 384), (448, 704)])
+def test_tiles_read_weights_ahead(sv, how, W, ff):
+    """1 to 11 steps of 64 columns: fewer than are read ahead, and every rest
+    of a round of six."""
+    T, E, top = 150, 3, 2
+    h = _rand(T, W, dtype=torch.bfloat16)
+    z = _rand(T, E, dtype=torch.float32, seed=1)
+    gu = _rand(E, 2 * ff, W, dtype=torch.bfloat16, seed=3, scale=W ** -0.5)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, seed=5, scale=ff ** -0.5)
+    p = sv.moe_plan(z.cuda(), None, top, how)
+    act = sv.moe_gemm(h.cuda(), gu.cuda(), p, True)
+    y = sv.moe_gemm(act, down.cuda(), p, False)
+    order, idx = p.order.cpu().long(), p.idx.cpu().reshape(-1).long()
+    got = act.double().cpu()
+    for e in range(E):
+        slots = (idx[order] == e).nonzero()[:, 0]
+        pairs = order[slots]
+        g, u = (h[pairs // top].double() @ gu[e].double().T).chunk(2, 1)
+        _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
+        _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
+               torch.bfloat16)
