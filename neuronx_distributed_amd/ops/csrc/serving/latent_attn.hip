@@ -41,7 +41,8 @@ struct LatentAppendArgs {
   int pairs;                // columns 2i and 2i + 1 turn, not i and i + rot / 2
 };
 
-template <typename T, int NT>
+// VEC: words of four elements
+template <typename T, int NT, bool VEC>
 __global__ void __launch_bounds__(NT)
 latent_append_kernel(LatentAppendArgs a) {
   extern __shared__ float cs[];          // cos [rot / 2], sin [rot / 2]
@@ -52,9 +53,17 @@ latent_append_kernel(LatentAppendArgs a) {
   const T* kv = (const T*)a.kv + t * a.kvst;
   const long page = a.bt[(long)a.seq[t] * a.MB + p / SV_PAGE];
   float sq = 0.f;
-  for (int i = tid; i < R; i += NT) {
-    const float v = to_f(kv[i]);
-    sq += v * v;
+  if (VEC) {
+    for (int i = tid * 4; i < R; i += NT * 4) {
+      float v[4];
+      load4(kv + i, v);
+      sq += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+    }
+  } else {
+    for (int i = tid; i < R; i += NT) {
+      const float v = to_f(kv[i]);
+      sq += v * v;
+    }
   }
   for (int i = NT - 1 - tid; i < half; i += NT) {      // by the last threads
     float c, s;
@@ -65,23 +74,76 @@ latent_append_kernel(LatentAppendArgs a) {
   sq = block_reduce_sum(sq, red);        // its barriers publish cs as well
   const float rstd = 1.f / sqrtf(sq / R + a.eps);
   T* row = (T*)a.cache + (page * SV_PAGE + p % SV_PAGE) * (R + P);
-  for (int i = tid; i < R; i += NT)
-    from_f(row[i], to_f(kv[i]) * rstd * to_f(((const T*)a.w)[i]));
+  const T* w = (const T*)a.w;
+  if (VEC) {
+    for (int i = tid * 4; i < R; i += NT * 4) {
+      float v[4], u[4];
+      load4(kv + i, v);
+      load4(w + i, u);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] *= rstd * u[j];
+      store4(row + i, v);
+    }
+  } else {
+    for (int i = tid; i < R; i += NT)
+      from_f(row[i], to_f(kv[i]) * rstd * to_f(w[i]));
+  }
 
-  auto rotate = [&](const T* src, T* dst, int i) {   // i in [0, P - half)
-    if (i < half) {
-      const float c = cs[i], s = cs[half + i];
-      const int u = a.pairs ? 2 * i : i, w = a.pairs ? u + 1 : i + half;
-      const float x = to_f(src[u]), y = to_f(src[w]);
-      from_f(dst[u], x * c - y * s);
-      from_f(dst[w], y * c + x * s);
+  // V pairs, or elements past them, from i in [0, P - half) on
+  constexpr int V = VEC ? 4 : 1;
+  auto rotate = [&](const T* src, T* dst, int i) {
+    if (i >= half) {
+      if (VEC) {
+        float v[4];
+        load4(src + i + half, v);
+        store4(dst + i + half, v);
+      } else {
+        dst[i + half] = src[i + half];
+      }
+      return;
+    }
+    float x[V], y[V];
+    const int u = a.pairs ? 2 * i : i, z = a.pairs ? u + V : i + half;
+    if (VEC) {
+      load4(src + u, x);
+      load4(src + z, y);
     } else {
-      dst[i + half] = src[i + half];
+      x[0] = to_f(src[u]);
+      y[0] = to_f(src[z]);
+    }
+    if (VEC && a.pairs) {                // neighbours: x0 y0 x1 y1 | x2 y2 ...
+      const float t[4] = {x[1], x[3], y[1], y[3]};
+      x[1] = x[2];
+      x[2] = y[0];
+      x[3] = y[2];
+#pragma unroll
+      for (int j = 0; j < V; ++j) y[j] = t[j];
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const float c = cs[i + j], s = cs[half + i + j], v = x[j];
+      x[j] = v * c - y[j] * s;
+      y[j] = y[j] * c + v * s;
+    }
+    if (VEC && a.pairs) {
+      const float t[4] = {x[2], y[2], x[3], y[3]};
+      x[2] = x[1];
+      x[3] = y[1];
+      x[1] = y[0];
+#pragma unroll
+      for (int j = 0; j < V; ++j) y[j] = t[j];
+    }
+    if (VEC) {
+      store4(dst + u, x);
+      store4(dst + z, y);
+    } else {
+      from_f(dst[u], x[0]);
+      from_f(dst[z], y[0]);
     }
   };
-  const int items = P - half;
+  const int items = (P - half) / V;
   for (int i = tid; i < (a.H + 1) * items; i += NT) {
-    const int h = i / items, j = i % items;
+    const int h = i / items, j = i % items * V;
     if (h == a.H)
       rotate(kv + R, row + R, j);
     else
@@ -94,14 +156,23 @@ extern "C" int sv_latent_append(const LatentAppendArgs* a, int T, int f32,
                                 hipStream_t stream) {
   if (T <= 0) return 0;
   const size_t lds = a->rot * sizeof(float);
+  const size_t size = f32 ? 4 : 2;
+  const bool vec = ((a->rot / 2 | a->R | a->P | a->qst | a->qh | a->qrst |
+                     a->qrh | a->kvst) & 3) == 0 &&
+      (((size_t)a->q | (size_t)a->qr | (size_t)a->kv | (size_t)a->w |
+        (size_t)a->cache) & (4 * size - 1)) == 0;
   // few rows: a longer workgroup waits for fewer words one after the other
-  // (32 rows of 512 + 64, 32 heads: 7.1 -> 4.3 us)
-#define LA(T_)                                                               \
-  do {                                                                       \
-    if (T <= 512) latent_append_kernel<T_, 1024><<<T, 1024, lds, stream>>>(*a); \
-    else latent_append_kernel<T_, 256><<<T, 256, lds, stream>>>(*a);         \
+  // (32 rows of 512 + 64, 32 heads: 7.1 -> 4.3 us; 4096 rows, element after
+  // element 21, in words 15)
+#define LAV(T_, NT, V)                                                        \
+  latent_append_kernel<T_, NT, V><<<T, NT, lds, stream>>>(*a)
+#define LA(T_)                                                                \
+  do {                                                                        \
+    if (T <= 512) { if (vec) LAV(T_, 1024, true); else LAV(T_, 1024, false); } \
+    else { if (vec) LAV(T_, 256, true); else LAV(T_, 256, false); }           \
   } while (0)
   if (f32) LA(float); else LA(short);
+#undef LAV
 #undef LA
   return (int)hipGetLastError();
 }

@@ -554,3 +554,51 @@ def test_tiles_read_weights_ahead(sv, how, W, ff):
         _close(act[slots.cuda()], g * torch.sigmoid(g) * u, torch.bfloat16)
         _close(y[pairs.cuda()], got[slots] @ down[e].double().T,
                torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("pairs", [False, True])
+@pytest.mark.parametrize("T,H,D,P,R,rot,shift", [
+    (5, 2, 8, 64, 512, 64, 0), (5, 3, 128, 64, 512, 64, 2),
+    (513, 1, 4, 16, 20, 8, 0), (3, 40, 4, 24, 1000, 24, 0),
+    (520, 2, 6, 10, 22, 4, 0)])
+def test_appended_in_words_and_elements(sv, T, H, D, P, R, rot, shift, pairs,
+                                        dtype):
+    """Words of four elements and single ones, long and short workgroups,
+    halves and neighbours, columns that pass; rows that start between words."""
+    kv = _rand(T, R + P + 4, dtype=dtype, seed=3).cuda()[:, shift:shift + R + P]
+    q = _rand(T, H * (D + P) + 4, dtype=dtype).cuda()
+    before = q.clone()
+    qv = q[:, shift:shift + H * (D + P)]
+    norm = _rand(R, dtype=dtype, seed=4).cuda()
+    cache = torch.zeros(-(-T // 64), 64, R + P, dtype=dtype).cuda()
+    bt = torch.arange(cache.shape[0], dtype=torch.int32)[None].cuda()
+    w = sv.LatentWeights(norm, None, None, sv.rotary_frequencies(
+        100.0, rot, "cuda"), pairs=pairs)
+    pos = torch.randperm(T, dtype=torch.int32)
+    sv.latent_append(qv, D, D + P, qv, D, D + P, kv, w, cache, pos.cuda(),
+                     torch.zeros(T, dtype=torch.int32).cuda(), bt, H, 1e-3)
+    f = 100.0 ** (-2.0 * torch.arange(rot // 2, dtype=torch.float64) / rot)
+    angle = pos.double()[:, None] * f
+
+    def turned(x):
+        x = x.double().cpu()
+        a = angle.view(T, *(1,) * (x.dim() - 2), rot // 2)
+        c, s = a.cos(), a.sin()
+        if pairs:
+            u, v = x[..., 0:rot:2], x[..., 1:rot:2]
+            out = torch.stack((u * c - v * s, v * c + u * s), -1).flatten(-2)
+        else:
+            u, v = x[..., :rot // 2], x[..., rot // 2:rot]
+            out = torch.cat((u * c - v * s, v * c + u * s), -1)
+        return torch.cat((out, x[..., rot:]), -1)
+
+    was = before[:, shift:shift + H * (D + P)].view(T, H, D + P)
+    got = qv.reshape(T, H, D + P)
+    _close(got[..., D:], turned(was[..., D:]), dtype)
+    assert torch.equal(got[..., :D], was[..., :D])
+    assert torch.equal(q[:, :shift], before[:, :shift])
+    rows = cache.view(-1, R + P)[pos.long().cuda()]
+    _close(rows[:, R:], turned(kv[:, R:]), dtype)
+    _close(rows[:, :R], no.plain_norm(kv[:, :R].double().cpu(),
+                                      norm.double().cpu(), 1e-3), dtype)
