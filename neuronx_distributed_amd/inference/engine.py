@@ -90,6 +90,29 @@ class _Layout:
                            max_keys=max_keys, spans=spans, **v)
 
 
+class _Staging:
+    """Pinned inputs of a step.  Two take turns, so that the host prepares a
+    step while the device is at the one before (from pageable memory it waited
+    for that: 45 us a step without work on the device)."""
+
+    def __init__(self, size):
+        self.turns = [(torch.zeros(size, dtype=torch.int32, pin_memory=True),
+                       torch.cuda.Event()) for _ in range(2)]
+
+    def open(self) -> np.ndarray:
+        """The inputs whose turn it is, once the device has read what they
+        last held."""
+        self.turns.reverse()
+        host, read = self.turns[0]
+        read.synchronize()
+        return host.numpy()
+
+    def send(self, buf):
+        host, read = self.turns[0]
+        buf.copy_(host, non_blocking=True)
+        read.record()
+
+
 class InferenceEngine:
     def __init__(self, model, max_tokens: int, max_seqs: int,
                  max_context: Optional[int] = None, use_graphs: bool = True):
@@ -257,9 +280,10 @@ class InferenceEngine:
         padding rows only."""
         lay = _Layout(bucket, 0, bucket, 0, 0, 0, bucket, bucket,
                       self.cache.table_width)
-        host = np.zeros(lay.size, dtype=np.int32)
-        self._fill_singles(lay.views(host), [], [], bucket)
-        buf = torch.from_numpy(host).to(self.device)
+        inputs = _Staging(lay.size)
+        buf = torch.empty(lay.size, dtype=torch.int32, device=self.device)
+        self._fill_singles(lay.views(inputs.open()), [], [], bucket)
+        inputs.send(buf)
         batch = lay.batch(buf, self.cache.max_context)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -273,15 +297,15 @@ class InferenceEngine:
             logits = self.model.forward_ragged(batch, self.cache.pools)
         if self._pool is None:
             self._pool = g.pool()
-        self._graphs[bucket] = (g, lay, host, buf, logits)
+        self._graphs[bucket] = (g, lay, inputs, buf, logits)
         return self._graphs[bucket]
 
     def _replay(self, entries, states):
         bucket = self._bucket(len(entries))
-        g, lay, host, buf, logits = (self._graphs.get(bucket)
-                                     or self._capture(bucket))
-        self._fill_singles(lay.views(host), entries, states, bucket)
-        buf.copy_(torch.from_numpy(host))
+        g, lay, inputs, buf, logits = (self._graphs.get(bucket)
+                                       or self._capture(bucket))
+        self._fill_singles(lay.views(inputs.open()), entries, states, bucket)
+        inputs.send(buf)
         g.replay()
         rows = [s for s, e in enumerate(entries) for _ in e.want]
         if not rows:

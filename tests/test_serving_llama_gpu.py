@@ -104,3 +104,31 @@ def test_mlp_of_few_rows_calls_a_watched_layer():
     # one rounding of 8 bits to the activations, one to the result
     assert error(few) < 2 * 2.0 ** -9
     assert error(few) <= error(watched)
+
+
+def test_steps_ahead_of_the_device_read_their_own_inputs():
+    """Decoding steps that the host sends without waiting give what steps one
+    at a time give, over two buckets that share the device."""
+    from neuronx_distributed_amd.inference import InferenceEngine, StepEntry
+
+    m = _model()
+    toks = torch.randint(0, m.config.vocab_size, (3, 40)).tolist()
+
+    def run(wait):
+        eng, out = InferenceEngine(m, 1024, 3), []
+        for i in range(3):
+            eng.step([StepEntry(i, toks[i][:20], [19])])
+        for t in range(20, 40):
+            some = range(3) if t % 3 else range(1, 2)
+            out.append(eng.step([StepEntry(i, [toks[i][t]], [0])
+                                 for i in some]))
+            if wait:
+                torch.cuda.synchronize()
+        return out
+
+    want = run(True)
+    big = torch.randn(4096, 4096, device="cuda")
+    for _ in range(20):                # the device is behind from the start
+        big = big @ big
+    for a, b in zip(run(False), want):
+        assert torch.equal(a, b)
