@@ -1065,17 +1065,21 @@ attn_tiles_kernel(TilesArgs a) {
           y -= __uint_as_float(w & 0xffff0000u);
         }
       }
+      // a plane of all columns after the other: a product that adds to the one
+      // before it waits for it (6000 prompt tokens: 590 -> 582 us, latent 395 ->
+      // 381)
+      union { tr4 t[2]; bf16x8 bf; } vf[NB];
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        union { tr4 t[2]; bf16x8 bf; } vf;
+      for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
-          vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          vf[nb].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
               (lds_tr4)(vbuf + (vx ^ (nb * 64)) + (16 * c + 8 * u) * DE * 2));
 #pragma unroll
-        for (int z = 0; z < NP; ++z)
-          ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
-      }
+      for (int z = 0; z < NP; ++z)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          ot[nb] = mfma_bf16(vf[nb].bf, pf[z].bf, ot[nb]);
     }
   };
   auto active = [&](int n) {
