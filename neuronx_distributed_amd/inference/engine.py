@@ -110,7 +110,7 @@ class _Staging:
     def send(self, buf):
         host, read = self.turns[0]
         buf.copy_(host, non_blocking=True)
-        read.record()
+        read.record(torch.cuda.current_stream(buf.device))
 
 
 class InferenceEngine:
