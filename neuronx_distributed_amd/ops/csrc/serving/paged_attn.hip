@@ -839,8 +839,9 @@ extern "C" int sv_attn_rows(const RowsArgs* a, int vec, int f32,
 // PFLOP/s (a large matrix product: 1.3 to 1.5).  6000 tokens of three portions
 // behind up to 4096, 32/8 heads: 621 -> 585 us with the next tile's scores
 // beside this tile's exponentials, page numbers read two tiles ahead, keys
-// rotated over all banks, and a maximum that lags.  An explicit order of
-// products and vector work took 630, splits by v_dot2c_f32_bf16 616.
+// rotated over all banks, and a maximum that lags; 577 with the order of the
+// planes below.  An explicit order of products and vector work took 630, splits
+// by v_dot2c_f32_bf16 616.
 // ---------------------------------------------------------------------------
 //
 // A key may end in columns that all heads share (kr): the rotated part of
