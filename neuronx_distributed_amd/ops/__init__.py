@@ -79,6 +79,14 @@ def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
 # RMSNorm
 # ---------------------------------------------------------------------------
 
+def _bf16_rows(x, *beside) -> bool:
+    """May the norm kernels run: everything that they read is bf16, in rows of
+    whole 16-byte words.  (A 32-bit weight beside bf16 rows takes the composed
+    form, which reads it as it is.)"""
+    return x.is_cuda and x.shape[-1] % 8 == 0 and \
+        x.dtype == torch.bfloat16 and all(t.dtype == x.dtype for t in beside)
+
+
 def _rmsnorm_bwd(x, weight, dy, rstd, dpass=None):
     """dx (+ dpass) and dw of contiguous bf16 rows x."""
     lib = _require_lib()
@@ -88,22 +96,20 @@ def _rmsnorm_bwd(x, weight, dy, rstd, dpass=None):
     w, dy = weight.contiguous(), dy.contiguous()
     dpass = None if dpass is None else dpass.contiguous()
     dx = torch.empty_like(x)
-    short = weight.dtype == torch.bfloat16
-    dw = torch.empty(H, dtype=weight.dtype if short else torch.float32,
-                     device=x.device)
+    dw = torch.empty(H, dtype=weight.dtype, device=x.device)
     part = torch.empty(lib.rmsnorm_bwd_parts(rows), H, dtype=torch.float32,
                        device=x.device)
     lib.rmsnorm_bwd(_ptr(x), _ptr(w), _ptr(dy), _ptr(rstd),
                     None if dpass is None else _ptr(dpass), _ptr(dx),
-                    _ptr(part), _ptr(dw), int(not short), rows, H, _stream())
-    return dx, dw.to(weight.dtype)
+                    _ptr(part), _ptr(dw), rows, H, _stream())
+    return dx, dw
 
 
 class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps):
         ctx.eps = eps
-        if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0:
+        if _bf16_rows(x, weight):
             lib = _require_lib()
             x2 = x.contiguous()
             rows = x2.numel() // x2.shape[-1]
@@ -115,7 +121,7 @@ class _RMSNormFn(torch.autograd.Function):
                             _stream())
             ctx.save_for_backward(x2, weight, rstd)
             return out
-        # CPU reference (fp32 math like the kernel)
+        # composed form (fp32 math like the kernel)
         xf = x.float()
         rstd = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
         ctx.save_for_backward(x, weight, rstd.squeeze(-1).reshape(-1))
@@ -125,7 +131,7 @@ class _RMSNormFn(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, rstd = ctx.saved_tensors
         H = x.shape[-1]
-        if x.is_cuda and x.dtype == torch.bfloat16 and H % 8 == 0:
+        if _bf16_rows(x, weight):
             return (*_rmsnorm_bwd(x, weight, dy, rstd), None)
         xf = x.float()
         dyf = dy.float()
@@ -149,8 +155,11 @@ def add_rmsnorm_available() -> bool:
 def add_rmsnorm(residual: torch.Tensor, delta: torch.Tensor,
                 weight: torch.Tensor, eps: float = 1e-6):
     """Fused ``res_out = residual + delta; normed = rmsnorm(res_out)*w``
-    (inference only, no autograd).  bf16 GPU rows; H % 8 == 0."""
+    (inference only, no autograd).  GPU rows; the kernel takes bf16 rows and
+    weight of H % 8 == 0."""
     lib = _require_lib()
+    if not _bf16_rows(residual, delta, weight):
+        return _add_rmsnorm_composed(residual, delta, weight, eps)[:2]
     H = residual.shape[-1]
     rows = residual.numel() // H
     r = residual.contiguous()
@@ -161,6 +170,15 @@ def add_rmsnorm(residual: torch.Tensor, delta: torch.Tensor,
                         _ptr(res_out), _ptr(normed), rows, H,
                         ctypes.c_float(eps), _stream())
     return res_out, normed
+
+
+def _add_rmsnorm_composed(res, delta, weight, eps):
+    """(h, normed, rstd) in fp32 math, norm stats on the rounded sum: matches
+    the kernel and an unfused bf16 add -> rmsnorm chain."""
+    h = (delta.float() + res.float()).to(delta.dtype)
+    hf = h.float()
+    rstd = torch.rsqrt(hf.pow(2).mean(-1, keepdim=True) + eps)
+    return h, (hf * rstd * weight.float()).to(delta.dtype), rstd
 
 
 class _AddRMSNormFn(torch.autograd.Function):
@@ -174,8 +192,7 @@ class _AddRMSNormFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, delta, res, weight, eps):
         ctx.eps = eps
-        if delta.is_cuda and delta.dtype == torch.bfloat16 \
-                and delta.shape[-1] % 8 == 0:
+        if _bf16_rows(delta, res, weight):
             lib = _require_lib()
             H = delta.shape[-1]
             rows = delta.numel() // H
@@ -190,13 +207,9 @@ class _AddRMSNormFn(torch.autograd.Function):
                                       ctypes.c_float(eps), _stream())
             ctx.save_for_backward(h, weight, rstd)
             return h, normed
-        # composed reference (fp32 math, norm stats on the rounded sum —
-        # matches the kernel and an unfused bf16 add -> rmsnorm chain)
-        h = (delta.float() + res.float()).to(delta.dtype)
-        hf = h.float()
-        rstd = torch.rsqrt(hf.pow(2).mean(-1, keepdim=True) + eps)
+        h, normed, rstd = _add_rmsnorm_composed(res, delta, weight, eps)
         ctx.save_for_backward(h, weight, rstd.squeeze(-1).reshape(-1))
-        return h, (hf * rstd * weight.float()).to(delta.dtype)
+        return h, normed
 
     @staticmethod
     def backward(ctx, dh, dnormed):
@@ -206,7 +219,7 @@ class _AddRMSNormFn(torch.autograd.Function):
             # normed output unused: the op reduces to the residual add —
             # grads pass straight through, no weight grad
             return dh, dh, None, None
-        if h.is_cuda and h.dtype == torch.bfloat16 and H % 8 == 0:
+        if _bf16_rows(h, weight):
             dx, dw = _rmsnorm_bwd(h, weight, dnormed, rstd, dh)
             return dx, dx, dw, None
         hf = h.float()

@@ -215,9 +215,8 @@ rmsnorm_bwd_long_kernel(const short* __restrict__ x, const short* __restrict__ w
 
 // dw = the sum of the workgroups' parts: 32 columns a workgroup, every eighth
 // part a row of threads
-template <typename T>
 __global__ void __launch_bounds__(256)
-rmsnorm_dw_kernel(const float* __restrict__ part, T* __restrict__ dw, int H,
+rmsnorm_dw_kernel(const float* __restrict__ part, short* __restrict__ dw, int H,
                   int parts) {
   __shared__ float sum[8][32];
   const int c = blockIdx.x * 32 + (threadIdx.x & 31), g = threadIdx.x >> 5;
@@ -231,7 +230,7 @@ rmsnorm_dw_kernel(const float* __restrict__ part, T* __restrict__ dw, int H,
   if (g || c >= H) return;
 #pragma unroll
   for (int i = 1; i < 8; ++i) s += sum[i][threadIdx.x];
-  if constexpr (sizeof(T) == 2) dw[c] = f2bits(s); else dw[c] = s;
+  dw[c] = f2bits(s);
 }
 
 // ---------------------------------------------------------------------------
@@ -339,10 +338,10 @@ extern "C" int rmsnorm_bwd_parts(int rows) {
   return rows < BWD_BLOCKS ? rows : BWD_BLOCKS;
 }
 
-// dx and dw (bf16, or f32) of rows of H % 8 == 0; dpass or null is added to dx
+// dx and dw of rows of H % 8 == 0; dpass or null is added to dx
 extern "C" void rmsnorm_bwd(const void* x, const void* w, const void* dy,
                             const void* rstd, const void* dpass, void* dx,
-                            void* part, void* dw, int dw_f32, int rows, int H,
+                            void* part, void* dw, int rows, int H,
                             hipStream_t stream) {
   const int blocks = rmsnorm_bwd_parts(rows);
 #define BWD(KERNEL, LDS)                                                     \
@@ -358,10 +357,6 @@ extern "C" void rmsnorm_bwd(const void* x, const void* w, const void* dy,
     else BWD(rmsnorm_bwd_long_kernel, (size_t)(H + 16) * sizeof(float));
   }
 #undef BWD
-  if (dw_f32)
-    rmsnorm_dw_kernel<float><<<(H + 31) / 32, 256, 0, stream>>>(
-        (const float*)part, (float*)dw, H, blocks);
-  else
-    rmsnorm_dw_kernel<short><<<(H + 31) / 32, 256, 0, stream>>>(
-        (const float*)part, (short*)dw, H, blocks);
+  rmsnorm_dw_kernel<<<(H + 31) / 32, 256, 0, stream>>>(
+      (const float*)part, (short*)dw, H, blocks);
 }

@@ -782,3 +782,37 @@ def test_rmsnorm_rows_and_widths(rows, H, forked):
                                atol=1e-4 * max(rows, 1) ** 0.5)
     if forked:
         assert torch.equal(x.grad, r.grad)
+
+
+@pytest.mark.parametrize("form", ["plain", "forked", "inference"])
+def test_norms_read_a_32_bit_weight_as_it_is(form):
+    """bf16 rows beside a float32 weight, against 64 bits."""
+    torch.manual_seed(3)
+    x, r, gy, gh = (torch.randn(5, 512, device="cuda").bfloat16()
+                    for _ in range(4))
+    w = torch.randn(512, device="cuda")
+    wd = w.double().requires_grad_()
+    xd = (x if form == "plain" else x + r).double().requires_grad_()
+    ref = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5) * wd
+    if form == "inference":
+        h, y = ops.add_rmsnorm(r, x, w, 1e-5)
+        assert torch.equal(h, x + r)
+    else:
+        x.requires_grad_()
+        w.requires_grad_()
+        if form == "plain":
+            y = ops.rmsnorm(x, w, 1e-5)
+            y.backward(gy)
+        else:
+            h, y = ops.add_rmsnorm_train(x, r, w, 1e-5)
+            torch.autograd.backward([h, y], [gh, gy])
+        ref.backward(gy.double())
+        # rounded once to 8 bits; sums of 512 columns, of 5 rows in 32 bits
+        torch.testing.assert_close(
+            x.grad.double(), xd.grad + (gh if form == "forked" else 0),
+            rtol=2.0 ** -7, atol=1e-4)
+        assert w.grad.dtype == torch.float32
+        torch.testing.assert_close(w.grad.double(), wd.grad, rtol=1e-5,
+                                   atol=1e-5)
+    assert y.dtype == torch.bfloat16
+    torch.testing.assert_close(y.double(), ref, rtol=2.0 ** -8, atol=1e-5)
