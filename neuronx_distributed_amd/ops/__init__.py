@@ -693,10 +693,8 @@ def skinny_or_none(inp: torch.Tensor, weight: torch.Tensor,
                    glu: bool = False):
     """inp (.., K) @ weight (N, K)^T, or with ``glu`` silu(gate) * up of
     weight = [gate; up], by the weight-streaming kernels where they beat the
-    library (a few rows; ``serving.stream_rule``), else None.
-    NXDA_SKINNY_GEMM=0 keeps everything on the library."""
-    if torch.is_grad_enabled() or sequence_parallel_enabled or \
-            os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
+    library (a few rows; ``serving.stream_rule``), else None."""
+    if torch.is_grad_enabled() or sequence_parallel_enabled:
         return None
     from . import serving as sv
 

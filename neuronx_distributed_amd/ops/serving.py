@@ -286,9 +286,11 @@ def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
              glu: bool = False) -> Optional[torch.Tensor]:
     """``stream_linear`` of the rows of x (..., K), where it is the faster one;
     None elsewhere, under autograd, and where somebody else watches the
-    operations (tracing, dispatch modes, autocast)."""
+    operations (tracing, dispatch modes, autocast).  NXDA_SKINNY_GEMM=0 keeps
+    every product on the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
-            not x.is_cuda or x.dim() < 2 or w.dim() != 2:
+            not x.is_cuda or x.dim() < 2 or w.dim() != 2 or \
+            os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
         return None
     K = x.shape[-1]
     T = x.numel() // K if K else 0

@@ -690,6 +690,21 @@ def test_few_rows_are_streamed_where_nobody_watches(glu):
         assert not any("empty" in str(f) for f in seen)
 
 
+def test_the_switch_keeps_32_bit_products_on_the_library(monkeypatch):
+    x = torch.randn(2, 4096, device="cuda").bfloat16()
+    w = torch.randn(6144, 4096, device="cuda").bfloat16()
+    taken, stream = [], sv.stream_linear
+    monkeypatch.setattr(sv, "stream_linear",
+                        lambda *a: taken.append(a) or stream(*a))
+    with torch.no_grad():
+        sv.linear_f32(x, w)
+        assert len(taken) == 1
+        monkeypatch.setenv("NXDA_SKINNY_GEMM", "0")
+        out = sv.linear_f32(x, w)
+    assert len(taken) == 1
+    assert torch.equal(out, torch.mm(x, w.t(), out_dtype=torch.float32))
+
+
 @pytest.mark.parametrize("H,G,N,P", [(2, 1, 64, 64), (6, 3, 128, 128),
                                      (3, 1, 64, 192), (16, 2, 128, 64)])
 def test_timed_memory_in_tiles(H, G, N, P):
