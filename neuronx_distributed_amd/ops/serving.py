@@ -40,10 +40,12 @@ def library():
 
 
 def available() -> bool:
-    """Is the library there to be loaded?"""
+    """Is the library there, with the products of few rows (one that was built
+    before they came has none, and layers then use torch's)?"""
     from .build import SERVING_LIB
 
-    return _LIB is not None or os.path.exists(SERVING_LIB)
+    return (_LIB is not None or os.path.exists(SERVING_LIB)) and \
+        hasattr(library(), "sv_stream_linear")
 
 
 def ensure_built():
