@@ -682,10 +682,27 @@ def skinny_gemm_available() -> bool:
 
 def skinny_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x2 (M<=32, K) bf16 @ w (N, K)^T -> (M, N) bf16 via the
-    weight-streaming kernel."""
+    weight-streaming kernel, which reads words of 16 bytes: of a K that is no
+    multiple of 8, or rows that start elsewhere, it reads a copy."""
     from . import serving as sv
 
-    return sv.stream_linear(x2, w)
+    def words(t):
+        t = torch.nn.functional.pad(t, (0, -t.shape[1] % 8))
+        if t.stride(1) != 1 or t.stride(0) & 7:
+            t = t.contiguous()
+        return t.clone() if t.data_ptr() & 15 else t
+
+    return sv.stream_linear(words(x2), words(w))
+
+
+def use_skinny_linear(inp: torch.Tensor, weight: torch.Tensor,
+                      sequence_parallel_enabled: bool = False) -> bool:
+    """Is ``skinny_linear`` faster than the library for the rows of ``inp``, and
+    nobody in its way (autograd, tracing, modes, NXDA_SKINNY_GEMM=0)?"""
+    from . import serving as sv
+
+    return not sequence_parallel_enabled and \
+        sv.stream_how(inp, weight) is not None
 
 
 def skinny_or_none(inp: torch.Tensor, weight: torch.Tensor,

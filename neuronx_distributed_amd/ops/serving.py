@@ -284,10 +284,10 @@ def _plain(t) -> bool:
     return type(t) in (torch.Tensor, torch.nn.Parameter)
 
 
-def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
-             glu: bool = False) -> Optional[torch.Tensor]:
-    """``stream_linear`` of the rows of x (..., K), where it is the faster one;
-    None elsewhere, under autograd, and where somebody else watches the
+def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
+               glu: bool = False) -> Optional[int]:
+    """How ``stream_linear`` takes the rows of x (..., K) where it is the faster
+    one; None elsewhere, under autograd, and where somebody else watches the
     operations (tracing, dispatch modes, autocast).  NXDA_SKINNY_GEMM=0 keeps
     every product on the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
@@ -307,7 +307,17 @@ def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
     rows = x.reshape(T, K)
     if rows.stride(1) != 1 or not (_words(rows) and _words(w)):
         return None
-    return stream_linear(rows, w, how, f32, glu).view(*x.shape[:-1], -1)
+    return how
+
+
+def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
+             glu: bool = False) -> Optional[torch.Tensor]:
+    """``stream_linear`` of the rows of x (..., K) by ``stream_how``, or None."""
+    how = stream_how(x, w, f32, glu)
+    if how is None:
+        return None
+    return stream_linear(x.reshape(-1, x.shape[-1]), w, how, f32,
+                         glu).view(*x.shape[:-1], -1)
 
 
 def _unwatched() -> bool:

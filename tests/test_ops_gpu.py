@@ -448,7 +448,7 @@ def test_moe_decode_imbalanced_routing():
 
 
 def test_skinny_gemm_matches_matmul():
-    """Split-K skinny-M decode GEMM vs torch matmul (fp32 reference)."""
+    """Products of few rows vs torch matmul (fp32 reference)."""
     torch.manual_seed(0)
     for M, N, K in [(32, 4096, 4096), (8, 1024, 11008), (1, 512, 256),
                     (32, 1000, 4096)]:
@@ -458,6 +458,45 @@ def test_skinny_gemm_matches_matmul():
         ref = (x.float() @ w.float().t())
         _cmp(out, ref.to(torch.bfloat16), atol=2e-2,
              name=f"skinny_{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("K,at,pitch", [(256, 1, 256), (256, 0, 257),
+                                        (250, 0, 250), (7, 3, 9)])
+def test_skinny_linear_of_rows_off_the_words(K, at, pitch):
+    torch.manual_seed(K + at)
+
+    def rows(n):
+        return torch.randn(n * pitch + 8, device="cuda").bfloat16()[
+            at:at + n * pitch].view(n, pitch)[:, :K]
+
+    x, w = rows(5), rows(33)
+    ref = x.double() @ w.double().t()
+    # rounded once to 8 bits; K products of 32 bits
+    torch.testing.assert_close(ops.skinny_linear(x, w).double(), ref,
+                               rtol=2.0 ** -8, atol=K * 2.0 ** -22)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_layers_of_few_rows_match_64_bits(bias):
+    """What the layers dispatch: own products of few rows, the library's of
+    more rows, under autograd and with a bias."""
+    from neuronx_distributed_amd.parallel.layers import \
+        linear_with_async_allreduce
+
+    torch.manual_seed(1)
+    x = torch.randn(40, 1, 4096, device="cuda").bfloat16()
+    w = torch.randn(6144, 4096, device="cuda").div(64).bfloat16()
+    b = torch.randn(6144, device="cuda").bfloat16() if bias else None
+    for rows in (1, 4, 5, 32, 40):
+        with torch.no_grad():
+            assert ops.use_skinny_linear(x[:rows], w) == (rows <= 4)
+            out = linear_with_async_allreduce(x[:rows], w, b)
+        ref = x[:rows].double() @ w.double().t()
+        ref = ref + b.double() if bias else ref
+        # sums of about 1 rounded once to 8 bits, with a bias twice
+        torch.testing.assert_close(out.double(), ref, rtol=2.0 ** -7,
+                                   atol=4096 * 2.0 ** -22)
+    assert not ops.use_skinny_linear(x[:1], w)         # under autograd
 
 
 def test_ring_block_primitives_gpu():
