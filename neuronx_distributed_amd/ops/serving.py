@@ -230,30 +230,68 @@ def stream_rule(T: int, N: int, K: int, f32: bool = False,
                 glu: bool = False) -> Optional[int]:
     """How T rows x (T, K) meet a large weight (N, K): 0 every workgroup
     streams its weight rows and all of x, 1 workgroups stay with x in registers,
-    None the library's product is as fast.  All measured over N 512..128256,
-    K 512..28672 (``stream_linear.hip``):
+    None the library's product is as fast.  The library reads weights at 2.5 to
+    6 TB/s, by their sizes; the lines were drawn where it was not the faster one
+    in 220 sizes (N 8..201088, K 512..28672, 1..32 rows, both results; two are
+    left where it is, by 4 and 7%).  Below, us here and the library's.  512
+    streaming workgroups, of 16 weight rows each, run at a time:
 
-    - up to 4 rows stream, unless a part of the CUs gets one workgroup more
-      than the others (5120 x 5120: 17 us, library 14) or x is large itself;
-      up to 16 where the weight is small (4096 x 4096: 9..12 us, library 15)
-      but not too small to share x (64 x 4096, 16 rows: 9.3 us, library 8.1);
-    - staying takes two and more tiles a CU.  With 32-bit results of
-      K = 8192 the library is 2% faster; with 17..32 rows it is where 5 or 6 of
-      the 8 waves have columns (K = 3072: 35.5 us, library 34)."""
-    tiles = N // (32 if glu else 16)
-    stay = N % (32 if glu else 16) == 0 and K <= (4096 if f32 else 8192)
+    - more than one such round: the last must not be nearly empty (13824 x 5120
+      of 32 bits, 1 row: 30, 27) and K long enough to be worth a workgroup's
+      start (151936 x 896, 1 row: 64, 53).  All of them read x, so streaming
+      ends at 4 rows (at 3 of a large weight: 61344 x 3200, 4 rows: 75, 70; at
+      one of a long K: 64000 x 7168, 4 rows: 171, 152).  Then staying, for a K
+      that gives all 8 waves columns and leaves them registers (54784 x 1536, 8
+      rows: 40, 34; 64000 x 7168, 16 rows: 168, 153);
+    - one round in which some CUs have a second workgroup: the shorter K, the
+      more rows before that shows (5632 x 2048, 12 rows: 9.7, 11.8; 4608 x 3584,
+      8 rows: 14.3, 12.2);
+    - a workgroup a CU or fewer: of a long K the library takes pieces, which few
+      workgroups do not keep up with (1152 x 7168, 1 row: 10, 8.4), and of a
+      multiple of 1024 those of one on nearly every CU (3136 x 10240, 4 rows:
+      18, 16.7; 4096 x 14336: 24.6, 25.3; 4096 x 11008: 22, 37);
+      a gate's weight is too small to share x (64 x 4096 of 32 bits, 4 rows:
+      6.7, 5.9), and 16 rows are as much to read as the weight (2048 x 4096 of
+      32 bits, 16 rows: 9.4, 8.5);
+    - gates: staying takes two and more tiles a CU; with 17..32 rows the library
+      is as fast where 5 or 6 of the 8 waves have columns (K = 3072: 35.5, 34).
+      Two of 37 sizes are left where it is 5% faster (K = 5120, 25600 gates, 12
+      rows on; K = 640, 32 rows)."""
     if glu:
-        return 1 if stay and tiles >= 640 and (
+        stay = N % 32 == 0 and K <= 8192 and N // 32 >= 640
+        return 1 if stay and (
             T <= 16 or T <= 32 and (K <= 2048 or 3584 < K <= 4096)) else None
-    tiles = -(-N // 16)
-    even = tiles <= 256 or 384 <= tiles <= 512 or \
-        tiles > 512 and tiles >= 384 * -(-tiles // 512)
-    if T <= 4 and even and T * K <= 4 * 14336:
-        return 0
-    if stay and tiles >= 1024 and T <= 16:
-        return 1
-    small = K <= 4096 and N * K <= 4096 * 4096
-    return 0 if small and T <= (16 if N >= 512 else 8) else None
+    tiles, long = -(-N // 16), K > 4096
+    if tiles > 512:
+        uneven = f32 or long and tiles <= 1024
+        if K < 1536:
+            return None
+        if tiles >= (441 if uneven else 384) * -(-tiles // 512) and \
+                T <= (1 if long else 4 if tiles < 2048 else 3) and \
+                not (f32 and long and tiles < 1024):
+            return 0
+        return 1 if N % 16 == 0 and tiles >= 1024 and 2048 <= K <= 6144 and \
+            T <= (4 if f32 and long else 16) else None
+    if tiles > 256:
+        if tiles < 384:
+            most = 12 if K <= 2048 else 4 if K <= 3072 else 0
+        elif N * K <= 4096 * 4096:
+            most = 16
+        else:
+            most = 4 if not long else 0 if f32 else 1
+    elif N < 512:
+        most = 8 if K <= (2048 if f32 else 3072) else \
+            4 if not (f32 or long) else 0
+    elif long:
+        if tiles <= 120:
+            most = 4 if K <= 4864 else 0
+        elif K % 1024 == 0 and tiles <= 224:
+            most = 1
+        else:
+            most = min(2 if tiles <= 160 and K > 4864 else 4, 4 * 14336 // K)
+    else:
+        most = 8 if f32 and K > 2048 and N < 2560 else 16
+    return 0 if T <= most else None
 
 
 def stream_linear(x: torch.Tensor, w: torch.Tensor, stay: int = 0,

@@ -2,6 +2,8 @@
 
 import types
 
+import pytest
+
 from neuronx_distributed_amd.ops import serving as sv
 
 
@@ -12,3 +14,50 @@ def test_a_library_without_the_products_is_not_used(monkeypatch):
     monkeypatch.setattr(sv, "_LIB",
                         types.SimpleNamespace(sv_stream_linear=None))
     assert sv.available()
+
+
+SIZES = (8, 16, 24, 64, 248, 512, 576, 896, 1000, 1408, 2048, 2880, 3072,
+         3584, 4096, 4104, 4864, 5120, 6144, 8192, 8200, 14336, 28672, 32000,
+         50000, 50257, 151936)
+
+
+@pytest.mark.parametrize("f32,glu", [(False, False), (True, False),
+                                     (False, True)])
+def test_every_choice_is_one_that_the_launcher_takes(f32, glu):
+    """Streaming is for plain products; staying takes whole tiles of weight
+    rows, and 8192 columns of 16 rows or 4096 of 32 in registers."""
+    taken = set()
+    for T in range(1, 34):
+        for N in SIZES:
+            for K in SIZES:
+                how = sv.stream_rule(T, N, K, f32, glu)
+                taken.add(how)
+                assert how in (None, 0, 1)
+                if how == 0:
+                    assert not glu
+                if how == 1:
+                    assert N % (32 if glu else 16) == 0
+                    assert K <= (8192 if T <= 16 else 4096 if T <= 32 else 0)
+    assert taken == ({None, 1} if glu else {None, 0, 1})
+
+
+@pytest.mark.parametrize("T,N,K,f32,how", [
+    # where the library is faster, and the neighbours where it is not
+    (1, 151936, 896, False, None), (1, 33792, 1792, False, 0),
+    (8, 54784, 1536, False, None), (8, 32000, 2048, False, 1),
+    (4, 61344, 3200, False, 1), (4, 32000, 4096, True, 0),
+    (1, 13824, 5120, True, None), (1, 27648, 5120, False, 0),
+    (4, 64000, 7168, False, None), (1, 64000, 7168, False, 0),
+    (4, 27648, 5120, False, 1), (4, 28672, 4096, True, 0),
+    (5, 28672, 4096, True, 1), (17, 28672, 4096, False, None),
+    (8, 4608, 3584, False, None), (8, 5632, 2048, False, 0),
+    (16, 5504, 2560, False, None), (2, 7680, 5120, False, None),
+    (4, 6144, 4096, False, 0), (5, 6144, 4096, False, None),
+    (1, 1152, 7168, False, None), (4, 4096, 11008, False, 0),
+    (5, 4096, 11008, False, None), (4, 4096, 14336, False, 0),
+    (4, 64, 4096, True, None), (4, 64, 4096, False, 0),
+    (8, 256, 2048, True, 0), (9, 256, 2048, True, None),
+    (16, 2048, 4096, True, None), (16, 2048, 4096, False, 0),
+    (16, 4096, 4096, True, 0), (17, 4096, 4096, False, None)])
+def test_lines_of_the_rule(T, N, K, f32, how):
+    assert sv.stream_rule(T, N, K, f32) == how
