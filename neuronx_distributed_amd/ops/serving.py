@@ -802,6 +802,35 @@ def _row_splits(target: int, units: int, max_keys: int, per: int) -> int:
     return max(1, min(target // max(1, units), -(-max_keys // per), 64))
 
 
+def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
+                modified: bool = False):
+    """Form (2 on matrix cores, 1 on vectors) and workgroups a row of
+    ``attn_rows``, for bf16 heads of D = 64 or 128.  Of the first form 512
+    workgroups run at a time, each for one key head of a row, and each takes 4
+    to 7 us: with more of them, heads to themselves or in pairs, and short
+    contexts the second is the faster one (64 rows of 32/32 heads of 128, 64
+    keys: 18 and 12 us, 200: 26 and 23; 128 of 32/16, 64: 18.5 and 16.6; 128 of
+    32/32 of 64, 20: 14.2 and 12.6; 32 of 32/32 with modified scores, 100: 12.4
+    and 11.5).  Sharing a row costs a merge, 5 us and more, which up to 700 keys
+    pays only while CUs have no workgroup (32 rows of 32/32 heads, 300 keys: 25,
+    in two 31; 8 of 32/32, 600 keys: 15.5, in five 20).  Over 2300 sizes 0.65 of
+    the second form's time; up to 8% over it are left with modified scores of
+    heads to themselves (96 rows of 16/16 of 64, 300 keys: 16.6 and 15.8)."""
+    units, rep = rows * groups, heads // groups
+    if D == 64:
+        short = 64 if rep == 1 and units > (1024 if modified else 2048) else 0
+    elif rep == 1:
+        short = 200 if modified or units > 1024 else 64
+    else:
+        short = 0 if rep > 2 else \
+            100 if units > (1024 if modified else 2048) else 64
+    if units > 512 and 0 < max_keys <= short:
+        return 1, _row_splits(1024, units, max_keys, 128)
+    target = 2048 if max_keys > 700 or units <= 32 else \
+        512 if units <= 128 else 256
+    return 2, _row_splits(target, units, max_keys, 128)
+
+
 def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
               scale: float, window: int = 0, keep: int = 0,
               append: bool = True, max_keys: int = 0,
@@ -809,8 +838,8 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
               mod: Optional[ScoreMod] = None) -> torch.Tensor:
     """One query row per request row: decoding.  ``append`` also writes the
     row's own k/v into the cache (without it they must be there already).
-    ``max_keys`` bounds the visible keys of any row (it only sets how many
-    workgroups share a row)."""
+    ``max_keys`` bounds the visible keys of any row (it only chooses the kernel
+    and how many workgroups share a row)."""
     G, D, E = _check_cache(q, k, v, kc, vc, heads)
     rows = q.shape[0]
     assert pos.shape[0] == rows and seq.shape[0] == rows
@@ -818,8 +847,10 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
         max_keys = min(max_keys, window + keep) if max_keys else window + keep
     vec = int(_aligned((D, E), q, k, v))
     if vec and q.dtype == torch.bfloat16 and D == E and D in (64, 128):
-        vec = 2
-    splits = _row_splits(2048 if vec == 2 else 1024, rows * G, max_keys, 128)
+        vec, splits = rows_kernel(rows, heads, G, D, max_keys,
+                                  mod is not None)
+    else:
+        splits = _row_splits(1024, rows * G, max_keys, 128)
     out = _out(out, rows, heads * E, q)
     part = torch.empty(rows * heads * splits * (E + 2), dtype=torch.float32,
                        device=q.device) if splits > 1 else None

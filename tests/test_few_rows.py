@@ -1,4 +1,5 @@
-"""Products of a few rows: which of them the weight-streaming kernels take."""
+"""Decoding: which kernels take products of a few rows, attention of single
+rows and experts of few rows."""
 
 import types
 
@@ -61,3 +62,21 @@ def test_every_choice_is_one_that_the_launcher_takes(f32, glu):
     (16, 4096, 4096, True, 0), (17, 4096, 4096, False, None)])
 def test_lines_of_the_rule(T, N, K, f32, how):
     assert sv.stream_rule(T, N, K, f32) == how
+
+
+@pytest.mark.parametrize("rows,heads,groups,D,keys,modified,want", [
+    (32, 32, 8, 128, 4097, False, (2, 8)), (32, 32, 8, 64, 300, False, (2, 1)),
+    (1, 32, 8, 128, 4097, False, (2, 33)), (1, 32, 8, 128, 300, False, (2, 3)),
+    (16, 32, 8, 128, 300, False, (2, 3)), (17, 32, 8, 128, 300, False, (2, 1)),
+    # many workgroups of short rows
+    (16, 32, 32, 128, 64, False, (2, 1)), (17, 32, 32, 128, 64, False, (1, 1)),
+    (17, 32, 32, 128, 65, False, (2, 1)), (33, 32, 32, 128, 200, False, (1, 1)),
+    (33, 32, 32, 128, 201, False, (2, 1)), (17, 32, 32, 128, 200, True, (1, 1)),
+    (33, 32, 16, 128, 64, False, (1, 1)), (33, 32, 16, 128, 65, False, (2, 1)),
+    (129, 32, 16, 128, 100, False, (1, 1)), (129, 24, 8, 128, 20, False, (2, 1)),
+    (64, 32, 32, 64, 64, False, (2, 1)), (65, 32, 32, 64, 64, False, (1, 1)),
+    (33, 32, 32, 64, 64, True, (1, 1)), (65, 64, 32, 64, 64, False, (2, 1)),
+    # a bound that nobody gave
+    (65, 32, 32, 128, 0, False, (2, 1))])
+def test_kernel_of_single_rows(rows, heads, groups, D, keys, modified, want):
+    assert sv.rows_kernel(rows, heads, groups, D, keys, modified) == want

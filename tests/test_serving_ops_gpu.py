@@ -179,6 +179,28 @@ def test_attention_batch_of_unequal_requests(sv, dtype):
     _close(got, torch.cat([d[3][-1:] for d in data]), dtype)
 
 
+@pytest.mark.parametrize("H,G,D,n", [(8, 8, 128, 64), (8, 8, 128, 201),
+                                     (16, 8, 128, 64), (16, 8, 128, 65),
+                                     (24, 8, 128, 20), (8, 8, 64, 64)])
+def test_decoding_of_many_short_requests(sv, H, G, D, n):
+    """More rows and heads than run at a time, around the lengths at which
+    another kernel takes them."""
+    B, dtype = 300, torch.bfloat16
+    q, k, v, want = _attn_case(H, G, D, D, 0, 0, n, dtype)
+    lens = [n - i % 5 for i in range(B)]
+    c = Paged(lens, G, D, D, dtype)
+    at = [(r, p) for r, m in enumerate(lens) for p in range(m - 1)]
+    seq, pos = (torch.tensor(x, dtype=torch.int32).cuda() for x in zip(*at))
+    sv.kv_append(k.cuda()[pos.long()], v.cuda()[pos.long()], c.kc, c.vc, pos,
+                 seq, c.bt)
+    last = torch.tensor(lens) - 1
+    rows = torch.arange(B, dtype=torch.int32).cuda()
+    got = sv.attn_rows(q[last].cuda(), k[last].cuda(), v[last].cuda(), c.kc,
+                       c.vc, last.int().cuda(), rows, c.bt, H, 0.11,
+                       max_keys=n)
+    _close(got, want[last], dtype)
+
+
 def test_attention_weights_keep_32_bits(sv):
     """Two far apart values under nearly equal weights: bf16 weights would
     lose the small one's contribution to the sum of many."""
