@@ -83,8 +83,12 @@ residual_norm_kernel(ResidualNormArgs a) {
   const T* d1 = (const T*)a.delta + r * W;
   const float* d1f = (const float*)a.delta + r * W;
   const T* d2 = (const T*)a.delta2 + r * W;
-  float w_first[VEC];              // on its way while the sums are made
-  if (a.h && a.w && tid * VEC < W) ld<T, VEC>((const T*)a.w + tid * VEC, w_first);
+  // of few rows the weight is on its way while the sums are made (not beside
+  // branches, where it sent 68 bytes of a thread to scratch memory)
+  constexpr bool EARLY = NT == 1024 && !BRANCHES;
+  float w_first[VEC];
+  if (EARLY && a.h && a.w && tid * VEC < W)
+    ld<T, VEC>((const T*)a.w + tid * VEC, w_first);
 
   // the pending result when it is one tensor or a weighted sum of rows
   auto single = [&](int i, float* v) {
@@ -258,7 +262,7 @@ residual_norm_kernel(ResidualNormArgs a) {
   for (int i = tid * VEC; i < W; i += NT * VEC) {
     float v[VEC], u[VEC];
     ld<float, VEC>(row + i, v);  // written by this same thread
-    if (i == tid * VEC) {
+    if (EARLY && i == tid * VEC) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) u[j] = w_first[j];
     } else {
@@ -316,8 +320,11 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
                    (size_t)a->br[b].gate % (f32 ? 16 : 8) == 0));
   if (a->branches < 0 || a->branches > 2 || (a->branches && a->delta)) return 1;
   // few rows: a longer workgroup waits for fewer words one after the other
-  // (1 row of 4096: 8.2 -> 5.2 us, 32 rows 8.1 -> 5.3)
-  const bool wide = a->rows_out <= 512 && a->W >= 2048;
+  // (1 row of 4096: 8.2 -> 5.2 us, 32 rows 8.1 -> 5.3); without branches while
+  // there is one a CU, and up to two of rows of several words a thread (320
+  // rows of 2048: 4.5 us, long 6.0; of 4096: 6.8, 7.9; of 8192: 50, 49)
+  const bool wide = a->W >= 2048 &&
+      a->rows_out <= (a->branches || a->W > 4096 ? 512 : 256);
 #define RNB(T, V, B, N)                                                    \
   residual_norm_kernel<T, V, B, N><<<a->rows_out, N, lds, stream>>>(*a)
 #define RN(T, V)                                                           \

@@ -444,7 +444,8 @@ def test_cpu_tensors_are_refused(sv):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,W", [(1, 2049), (1, 4096), (512, 2052),
-                                    (513, 2052), (3, 9004)])
+                                    (513, 2052), (3, 9004), (256, 2052),
+                                    (257, 2052), (512, 4100), (513, 4100)])
 def test_residual_norm_of_wide_rows(sv, rows, W, dtype):
     """Long and ordinary workgroups; the last words of a row ragged."""
     eps = 0.03
