@@ -1412,7 +1412,7 @@ MOE_TILES = (2, 3, 4, 5)
 MOE_TILE_ROWS = (32, 32, 32, 64, 128, 256)
 
 
-def moe_kernel(pairs: int, experts: int, width: int = 0, ff: int = 0) -> int:
+def moe_kernel(pairs: int, experts: int, width: int, ff: int) -> int:
     """The fastest kernel for ``pairs`` spread over ``experts`` of ff x width
     (measured): streaming up to 24 rows an expert where workgroups can stay with
     their rows (width and ff up to 4096), 16 where only the gates' can; else the
@@ -1422,12 +1422,16 @@ def moe_kernel(pairs: int, experts: int, width: int = 0, ff: int = 0) -> int:
     the faster ones from 24 (64 experts 2048 x 1408, 72 rows: 64 slots 305 us,
     128 262) and 112 rows on (128 rows: 128 slots 341, 256 322); long rows of few
     slots are read faster by two workgroups a CU (8 experts 4096 x 14336, 32
-    rows: 64 slots 577, 128 603, from 48 rows on 608)."""
+    rows: 64 slots 577, 128 603, from 48 rows on 608).  The mean rows are all
+    that the host knows: where 32 rows go to the same 6 of 64 experts, staying
+    takes 66 us, a workgroup for every 16 weight rows would take 62; and 64
+    experts 4096 x 2048, whose tiles all start at one place of a power of two,
+    took 732 with 24 rows before the XCDs shared the tiles, and 777 now."""
     rows = pairs / experts
-    stay = 0 < width <= 4096
+    stay = width <= 4096
     if rows < ((24 if ff <= 4096 else 16) if stay else 4):
         return MOE_STREAM
-    if rows >= 24 and width and not (width | ff) & 63:
+    if rows >= 24 and not (width | ff) & 63:
         if rows < 48 and max(width, ff) > 4096:
             return MOE_TILES[1]
         return MOE_TILES[2 if rows < 112 else 3]

@@ -70,13 +70,37 @@ def test_lines_of_the_rule(T, N, K, f32, how):
     (16, 32, 8, 128, 300, False, (2, 3)), (17, 32, 8, 128, 300, False, (2, 1)),
     # many workgroups of short rows
     (16, 32, 32, 128, 64, False, (2, 1)), (17, 32, 32, 128, 64, False, (1, 1)),
-    (17, 32, 32, 128, 65, False, (2, 1)), (33, 32, 32, 128, 200, False, (1, 1)),
-    (33, 32, 32, 128, 201, False, (2, 1)), (17, 32, 32, 128, 200, True, (1, 1)),
+    (17, 32, 32, 128, 65, False, (2, 1)),
+    (33, 32, 32, 128, 200, False, (1, 1)),
+    (33, 32, 32, 128, 201, False, (2, 1)),
+    (17, 32, 32, 128, 200, True, (1, 1)),
     (33, 32, 16, 128, 64, False, (1, 1)), (33, 32, 16, 128, 65, False, (2, 1)),
-    (129, 32, 16, 128, 100, False, (1, 1)), (129, 24, 8, 128, 20, False, (2, 1)),
+    (129, 32, 16, 128, 100, False, (1, 1)),
+    (129, 24, 8, 128, 20, False, (2, 1)),
     (64, 32, 32, 64, 64, False, (2, 1)), (65, 32, 32, 64, 64, False, (1, 1)),
     (33, 32, 32, 64, 64, True, (1, 1)), (65, 64, 32, 64, 64, False, (2, 1)),
     # a bound that nobody gave
     (65, 32, 32, 128, 0, False, (2, 1))])
 def test_kernel_of_single_rows(rows, heads, groups, D, keys, modified, want):
     assert sv.rows_kernel(rows, heads, groups, D, keys, modified) == want
+
+
+@pytest.mark.parametrize("rows,width,ff,want", [
+    # streaming, to the line of each size and past it
+    (1, 2048, 1408, 1), (23, 2048, 1408, 1), (24, 2048, 1408, 4),
+    (23, 4096, 4096, 1), (15, 4096, 4104, 1), (16, 4096, 4104, 2),
+    (3, 4104, 2048, 1), (4, 4104, 2048, 2), (23, 1000, 2760, 1),
+    (23, 4104, 2048, 2), (24, 4104, 2048, 3), (23, 4096, 896, 1),
+    # tiles of sizes that are read two steps ahead
+    (24, 4096, 14336, 3), (47, 4096, 14336, 3), (48, 4096, 14336, 4),
+    (111, 2048, 1408, 4), (112, 2048, 1408, 5), (24, 5120, 2048, 3),
+    # and of others
+    (24, 1000, 2760, 3), (111, 2048, 1416, 3), (112, 2048, 1416, 4),
+    (159, 2048, 1416, 4), (160, 2048, 1416, 5)])
+def test_kernel_of_the_experts(rows, width, ff, want):
+    assert sv.moe_kernel(rows * 8, 8, width, ff) == want
+
+
+def test_a_choice_without_the_sizes_is_refused():
+    with pytest.raises(TypeError):
+        sv.moe_kernel(64, 8)

@@ -314,7 +314,11 @@ def test_plan_routes_and_groups(sv, T, E, top, how):
 def test_kernel_of_the_grouped_products_fits_the_load():
     from neuronx_distributed_amd.ops import serving as sv
 
-    rows = [sv.MOE_TILE_ROWS[sv.moe_kernel(n, 8)]
+    rows = [sv.MOE_TILE_ROWS[sv.moe_kernel(n, 8, 4096, 14336)]
+            for n in (1, 40, 64, 300, 1000, 5000)]
+    assert rows == [32, 32, 32, 64, 256, 256]
+    # off the sizes whose weights are read two steps ahead
+    rows = [sv.MOE_TILE_ROWS[sv.moe_kernel(n, 8, 4104, 14336)]
             for n in (1, 40, 64, 300, 1000, 5000)]
     assert rows == [32, 32, 32, 64, 128, 256]
 
