@@ -1417,7 +1417,10 @@ def moe_kernel(pairs: int, experts: int, width: int, ff: int) -> int:
     (measured): streaming up to 24 rows an expert where workgroups can stay with
     their rows (width and ff up to 4096), 16 where only the gates' can; else the
     rows are read again and again, and tiles are faster from 4 on (256 experts
-    7168 x 2048, 4 rows: 3.64 ms, streamed 4.21).  Tiles of 128 and 256 slots
+    7168 x 2048, 4 rows: 3.64 ms, streamed 4.21), as where less than half of the
+    columns that a staying workgroup covers are there and the tiles of 256 gates
+    and projections fill the CUs (8 rows of 128 experts 2048 x 768: 238 us,
+    streamed 254; of 64 of 2048 x 512: 104, 96).  Tiles of 128 and 256 slots
     read weights two steps ahead where width and ff are multiples of 64, and are
     the faster ones from 24 (64 experts 2048 x 1408, 72 rows: 64 slots 305 us,
     128 262) and 112 rows on (128 rows: 128 slots 341, 256 322); long rows of few
@@ -1428,7 +1431,8 @@ def moe_kernel(pairs: int, experts: int, width: int, ff: int) -> int:
     experts 4096 x 2048, whose tiles all start at one place of a power of two,
     took 732 with 24 rows before the XCDs shared the tiles, and 777 now."""
     rows = pairs / experts
-    stay = width <= 4096
+    stay = width <= 4096 and (min(width, ff) > 960 or
+                              experts * ff <= 256 * 128)
     if rows < ((24 if ff <= 4096 else 16) if stay else 4):
         return MOE_STREAM
     if rows >= 24 and not (width | ff) & 63:

@@ -101,6 +101,13 @@ def test_kernel_of_the_experts(rows, width, ff, want):
     assert sv.moe_kernel(rows * 8, 8, width, ff) == want
 
 
+@pytest.mark.parametrize("rows,experts,width,ff,want", [
+    (3, 128, 2048, 768, 1), (4, 128, 2048, 768, 2), (4, 64, 768, 2048, 2),
+    (4, 64, 2048, 520, 2), (4, 64, 2048, 512, 1), (4, 64, 2048, 968, 1)])
+def test_kernel_of_many_small_experts(rows, experts, width, ff, want):
+    assert sv.moe_kernel(rows * experts, experts, width, ff) == want
+
+
 def test_a_choice_without_the_sizes_is_refused():
     with pytest.raises(TypeError):
         sv.moe_kernel(64, 8)
