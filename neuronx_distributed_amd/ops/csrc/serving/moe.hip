@@ -420,20 +420,28 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   if (AHEAD) {
     // step i: its words are here, in all waves, and the weights of i + 1 may be
     // on their way; the step before is read.  Past the last step that one
-    // again, so that the words on their way keep their number
+    // again, so that the words on their way keep their number.
+    // The wait counts: it is right only if the LW loads of the weights of i + 1
+    // are the last that were asked for, behind the rows and the weights of i.
+    // Nothing else tells the compiler so (they go to different arrays).
+    auto in_order = []() __attribute__((always_inline)) {
+      asm volatile("" ::: "memory");
+    };
     auto turn = [&](int i, short* xs, short* ws, short* xn, short* wn)
         __attribute__((always_inline)) {
       static_assert(LW < 16, "");
       __builtin_amdgcn_s_waitcnt(0x70 | LW);       // vmcnt(LW) lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      in_order();
       issue_x(min(i + 1, steps - 1) * 64, xn);
+      in_order();
       issue_w(min(i + 2, steps - 1) * 64, wn);
       step(xs, ws);
     };
     short *const xr[2] = {xs0, xs1}, *const wr[3] = {ws0, ws1, ws2};
     issue_x(0, xs0);
     issue_w(0, ws0);
+    in_order();
     issue_w(min(1, steps - 1) * 64, ws1);
     int i = 0;
     for (; i + 6 <= steps; i += 6)
