@@ -465,7 +465,7 @@ def test_residual_norm_of_wide_rows(sv, rows, W, dtype):
 @pytest.mark.parametrize("H,G,D,shift", [(1, 0, 2, 0), (3, 1, 24, 0),
                                          (5, 2, 36, 0), (32, 8, 128, 0),
                                          (32, 8, 128, 1), (7, 7, 64, 4)])
-@pytest.mark.parametrize("T", [1, 33])
+@pytest.mark.parametrize("T", [1, 33, 257])
 def test_rope_rows(sv, T, H, G, D, shift, dtype):
     """Every pair of every head is turned once: words and single pairs, heads
     that start between words, the last workgroup ragged."""
