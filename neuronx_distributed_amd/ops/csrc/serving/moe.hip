@@ -832,7 +832,8 @@ static void launch_stream(const MoeGemmArgs& a, hipStream_t stream) {
   const long all = (long)units * a.max_tiles;
   // as many workgroups as are resident: with twice as many, 2% to 30% longer.
   // They share whole units, so they need a few (6 tiles of 2048 x 1408: a
-  // workgroup a unit 42 us, two products and the plan; staying 47).
+  // workgroup a unit 42 us, two products and the plan; staying 47).  The host
+  // knows the most tiles there can be: rows that share few experts stay as well.
   const int grid = a.K <= 2048 ? 512 : 256;
   if (a.K > 4096 || all < 2 * grid)
     moe_stream_kernel<GLU><<<dim3(units, a.max_tiles), 1024, 0, stream>>>(a);

@@ -1426,10 +1426,11 @@ def moe_kernel(pairs: int, experts: int, width: int, ff: int) -> int:
     128 262) and 112 rows on (128 rows: 128 slots 341, 256 322); long rows of few
     slots are read faster by two workgroups a CU (8 experts 4096 x 14336, 32
     rows: 64 slots 577, 128 603, from 48 rows on 608).  The mean rows are all
-    that the host knows: where 32 rows go to the same 6 of 64 experts, staying
-    takes 66 us, a workgroup for every 16 weight rows would take 62; and 64
-    experts 4096 x 2048, whose tiles all start at one place of a power of two,
-    took 732 with 24 rows before the XCDs shared the tiles, and 777 now."""
+    that the host knows: 32 rows that go to the same 6 of 64 experts stay as well,
+    528 units on 512 workgroups (58 us; 71 before staying came).  One size is
+    slower than it was: 64 experts 4096 x 2048 of 24 to 32 rows, 777 to 796 us
+    where tiles of 64 took 732 to 760 before the XCDs shared the tiles that have
+    rows."""
     rows = pairs / experts
     stay = width <= 4096 and (min(width, ff) > 960 or
                               experts * ff <= 256 * 128)
