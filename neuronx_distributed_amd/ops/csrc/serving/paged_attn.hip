@@ -465,7 +465,10 @@ attn_rows_kernel(RowsArgs a) {
 // three planes that add up to them.
 //
 // Bound by memory: 8 waves a CU have 16 KB each on their way.  The kernel above
-// spends its time on vector work (a key costs 140 cycles of a wave; here 30).
+// spends its time on vector work (a key costs 140 cycles of a wave; here 30), but
+// has more workgroups on a CU and less to start with: of many short rows whose
+// heads have keys of their own it is the faster one (rows_kernel in
+// ops/serving.py).
 // ---------------------------------------------------------------------------
 // the larger of the four lanes 16 apart
 __device__ __forceinline__ float max_quarters(float x) {

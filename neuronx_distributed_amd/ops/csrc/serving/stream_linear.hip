@@ -206,7 +206,8 @@ static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
   if (stay) {
     if (a.N % rows) return 1;
     const int grid = min(tiles, 256);
-    // at most 128 registers of x beside the weights
+    // at most 128 registers of x beside the weights (plain products of 17 to
+    // 32 rows by a direct call alone, here and below: the library is faster)
     if (a.T <= 16 && a.K <= 4096)
       stay_linear_kernel<8, 2, 1, EPI><<<grid, 512, 0, stream>>>(a);
     else if (a.T <= 16 && a.K <= 8192)
