@@ -21,9 +21,11 @@
 // 8192 tokens, 32/8 heads: dK/dV 2680 -> 1123 us (979 TFLOP/s), dQ 1404 -> 739
 // us (1116 TFLOP/s); before, tiles were turned by scattered writes, the halves
 // of dK/dV exchanged P and dS through LDS behind a third barrier, and every
-// element was masked.  Scores and their gradients by turns took the pair of
-// directions from 2610 to 2487 us.  Both are bound by the matrix cores (40 to 45 % of their
-// nominal rate) with the exponentials and reads beside them.
+// element was masked.  The vector work then stood between the products, beside
+// those of another wave at best; cut into pieces, one beside each product of the
+// same wave, both directions took 1823 us instead of 1874 (2 x 4096, 32 heads: 986
+// for 1021).  Bound by the matrix cores, 45 to 57 % busy at the 1.8 GHz that the
+// card holds under such work.
 
 #include "common.h"
 #include "mfma.h"
@@ -181,7 +183,9 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   const float* delta = a.delta + ((long)b * a.Hq + h) * S;
 
   f32x16 dv[4] = {}, dk[4] = {};         // [d][kv]
-  const float s2 = a.scale * LOG2E;
+  // a masked score has no weight, whatever the sign of the scale
+  const float s2 = a.scale == 0.f ? 1e-37f : a.scale * LOG2E;
+  const float gone = s2 > 0.f ? -INFINITY : INFINITY;
   // this lane in the wave's rows of a q tile, of the kv tile
   const int rq = row_lane(col, hi) + half * 8192, tq = tr_lane(lane) + half * 8192;
   const int rk = row_lane(col, hi) + g * 8192;
@@ -206,32 +210,26 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
         (window > 0 && q0 >= kw0 + 31 + window))
       return;
     const float* ld = ld_t + half * 32;
-    // S^T and dP^T: q in the accumulators' rows, kv in the lanes
+    // S^T and dP^T: q in the accumulators' rows, kv in the lanes.  Every product
+    // has its own piece of the vector work beside it and reads two ahead.
     f32x16 s = {}, dp = {};
-    // both by turns, so that no product waits for the one before it; the next
-    // columns are on their way (8192 rows of 32 heads: 2 to 7% of the kernel)
-    frag_u f[2][4];
-    auto read = [&](int c) __attribute__((always_inline)) {
-      f[c & 1][0] = read_row(qb, rq, c);
-      f[c & 1][1] = read_row(kb, rk, c);
-      f[c & 1][2] = read_row(db, rq, c);
-      f[c & 1][3] = read_row(vb, rk, c);
+    frag_u f[3][2];
+    auto rows_s = [&](int c) __attribute__((always_inline)) {
+      f[c % 3][0] = read_row(qb, rq, c);
+      f[c % 3][1] = read_row(kb, rk, c);
     };
-    read(0);
+    auto rows_dp = [&](int c) __attribute__((always_inline)) {
+      f[(c + 2) % 3][0] = read_row(db, rq, c);
+      f[(c + 2) % 3][1] = read_row(vb, rk, c);
+    };
+    rows_s(0);
+    rows_s(1);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      if (c < 7) read(c + 1);
+      if (c < 6) rows_s(c + 2); else rows_dp(c - 6);
       __builtin_amdgcn_sched_barrier(0);
-      s = mfma_bf16(f[c & 1][0].bf, f[c & 1][1].bf, s);
-      dp = mfma_bf16(f[c & 1][2].bf, f[c & 1][3].bf, dp);
+      s = mfma_bf16(f[c % 3][0].bf, f[c % 3][1].bf, s);
       __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const f4v l = *(const f4v*)(ld + 8 * r4 + 4 * hi);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        s[4 * r4 + j] = __builtin_amdgcn_exp2f(s[4 * r4 + j] * s2 - l[j]);
     }
     if ((a.causal && q0 < kw0 + 31) || q0 + 32 > S ||
         (window > 0 && q0 + 31 >= kw0 + window)) {
@@ -242,28 +240,46 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int j = acc_row(r, 0);
-        s[r] = j < first || j >= last ? 0.f : s[r];
+        s[r] = j < first || j >= last ? gone : s[r];
       }
     }
     frag_u pf[2], df[2];
-    to_frags(s, pf);
+    bf16x8 t[3];
+    f4v l[2];
+    l[0] = *(const f4v*)(ld + 4 * hi);
 #pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const f4v l = *(const f4v*)(ld + 64 + 8 * r4 + 4 * hi);
+    for (int c = 0; c < 8; ++c) {
+      if (c < 6) rows_dp(c + 2); else t[c - 6] = read_turned(db, tq, 0, c - 6);
+      if (c % 2 == 0)            // then delta
+        l[(c / 2 + 1) % 2] = *(const f4v*)(
+            ld + (c < 6 ? 8 * (c / 2 + 1) : 64) + 4 * hi);
+      __builtin_amdgcn_sched_barrier(0);
+      dp = mfma_bf16(f[(c + 2) % 3][0].bf, f[(c + 2) % 3][1].bf, dp);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[4 * r4 + j] *= dp[4 * r4 + j] - l[j];
+      for (int i = 0; i < 2; ++i) {
+        const int r = 2 * c + i;
+        s[r] = __builtin_amdgcn_exp2f(s[r] * s2 - l[c / 2 % 2][r % 4]);
+      }
+      pf[c / 4].u[c % 4] = pack_bf16x2(s[2 * c], s[2 * c + 1]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    to_frags(s, df);
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int i = 0; i < 16; ++i) {
+      const int n = i + 2;       // fragments of dO, then of Q
+      if (n < 16) t[n % 3] = read_turned(n < 8 ? db : qb, tq, n / 4 % 2, n % 4);
+      if (i < 6 && i % 2 == 0)
+        l[(i / 2 + 1) % 2] = *(const f4v*)(ld + 64 + 8 * (i / 2 + 1) + 4 * hi);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16& to = i < 8 ? dv[i % 4] : dk[i % 4];
+      to = mfma_bf16(t[i % 3], (i < 8 ? pf : df)[i / 4 % 2].bf, to);
+      if (i < 8) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        dv[nb] = mfma_bf16(read_turned(db, tq, c, nb), pf[c].bf, dv[nb]);
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        dk[nb] = mfma_bf16(read_turned(qb, tq, c, nb), df[c].bf, dk[nb]);
+        for (int j = 0; j < 2; ++j)
+          s[2 * i + j] *= dp[2 * i + j] - l[i / 2 % 2][(2 * i + j) % 4];
+        df[i / 4].u[i % 4] = pack_bf16x2(s[2 * i], s[2 * i + 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
 
   fill_rows<128, 512>(a.k + b * a.k_bs + hkv * a.k_hs + st_r * a.k_ss + st_c,
@@ -344,7 +360,8 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
   }
   const long at = ((long)b * a.Hq + h) * S + q_ld;
   const float lse2 = a.lse[at] * LOG2E, dlt = a.delta[at];
-  const float s2 = a.scale * LOG2E;
+  const float s2 = a.scale == 0.f ? 1e-37f : a.scale * LOG2E;
+  const float gone = s2 > 0.f ? -INFINITY : INFINITY;
 
   f32x16 dq[4] = {};                     // [d][q]
   const int rx = row_lane(col, hi), tx = tr_lane(lane);
@@ -365,29 +382,19 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
     if ((a.causal && k0 > qw0 + 31) || k0 >= S ||
         (window > 0 && k0 + 31 + window <= qw0))
       return;
-    // S^T and dP^T: keys in the accumulators' rows, q in the lanes
+    // S^T and dP^T: keys in the accumulators' rows, q in the lanes.  As above,
+    // every product has vector work beside it and reads two ahead.
     f32x16 s = {}, dp = {};
-    // both by turns, two columns of the fragments on their way (one after the
-    // other, every product waited for its read and the one before: 2 x 4096 rows
-    // of 32 heads 400 us, now 384)
-    frag_u f[3][2];
-    auto read = [&](int c) __attribute__((always_inline)) {
-      f[c % 3][0] = read_row(kb, rx, c);
-      f[c % 3][1] = read_row(vb, rx, c);
-    };
-    read(0);
-    read(1);
+    frag_u f[3];
+    f[0] = read_row(kb, rx, 0);
+    f[1] = read_row(kb, rx, 1);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      if (c < 6) read(c + 2);
+      f[(c + 2) % 3] = c < 6 ? read_row(kb, rx, c + 2) : read_row(vb, rx, c - 6);
       __builtin_amdgcn_sched_barrier(0);
-      s = mfma_bf16(f[c % 3][0].bf, qf[c].bf, s);
-      dp = mfma_bf16(f[c % 3][1].bf, dof[c].bf, dp);
+      s = mfma_bf16(f[c % 3].bf, qf[c].bf, s);
       __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      s[r] = __builtin_amdgcn_exp2f(s[r] * s2 - lse2);
     if ((a.causal && k0 + 31 > qw0) || k0 + 32 > S ||
         (window > 0 && k0 <= qw0 + 31 - window)) {
       asm volatile("");        // a branch: not selects on every tile
@@ -398,19 +405,39 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int j = acc_row(r, 0);
-        s[r] = j > last || j <= first ? 0.f : s[r];
+        s[r] = j > last || j <= first ? gone : s[r];
       }
     }
+    bf16x8 t[3];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] *= dp[r] - dlt;
+    for (int c = 0; c < 8; ++c) {
+      if (c < 6) f[(c + 4) % 3] = read_row(vb, rx, c + 2);
+      else t[c - 6] = read_turned(kb, tx, 0, c - 6);
+      __builtin_amdgcn_sched_barrier(0);
+      dp = mfma_bf16(f[(c + 2) % 3].bf, dof[c].bf, dp);
+#pragma unroll
+      for (int r = 2 * c; r < 2 * c + 2; ++r)
+        s[r] = __builtin_amdgcn_exp2f(s[r] * s2 - lse2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     frag_u df[2];
-    to_frags(s, df);
+    auto weigh = [&](int u) __attribute__((always_inline)) {
+      s[2 * u] *= dp[2 * u] - dlt;
+      s[2 * u + 1] *= dp[2 * u + 1] - dlt;
+      df[u / 4].u[u % 4] = pack_bf16x2(s[2 * u], s[2 * u + 1]);
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) weigh(u);
     // dQ^T[d][q] += K^T dS^T
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        dq[nb] = mfma_bf16(read_turned(kb, tx, c, nb), df[c].bf, dq[nb]);
+    for (int i = 0; i < 8; ++i) {
+      const int n = i + 2;
+      if (n < 8) t[n % 3] = read_turned(kb, tx, n / 4, n % 4);
+      __builtin_amdgcn_sched_barrier(0);
+      dq[i % 4] = mfma_bf16(t[i % 3], df[i / 4].bf, dq[i % 4]);
+      if (i < 4) weigh(4 + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
   auto tile = [&](int k0, char* kb, const char* vb) __attribute__((always_inline)) {
     step(k0, kb, vb);
