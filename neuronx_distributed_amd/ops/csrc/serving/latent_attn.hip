@@ -41,13 +41,14 @@ struct LatentAppendArgs {
   int pairs;                // columns 2i and 2i + 1 turn, not i and i + rot / 2
 };
 
-// VEC: words of four elements
+extern __shared__ float dynamic_lds[];
+
+// row t; VEC: words of four elements
 template <typename T, int NT, bool VEC>
-__global__ void __launch_bounds__(NT)
-latent_append_kernel(LatentAppendArgs a) {
-  extern __shared__ float cs[];          // cos [rot / 2], sin [rot / 2]
+__device__ __forceinline__ void latent_append(const LatentAppendArgs& a, int t) {
+  float* cs = dynamic_lds;               // cos [rot / 2], sin [rot / 2]
   __shared__ float red[16];
-  const int t = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const int half = a.rot / 2, R = a.R, P = a.P;
   const int p = a.pos[t];
   const T* kv = (const T*)a.kv + t * a.kvst;
@@ -152,15 +153,24 @@ latent_append_kernel(LatentAppendArgs a) {
   }
 }
 
+template <typename T, int NT, bool VEC>
+__global__ void __launch_bounds__(NT)
+latent_append_kernel(LatentAppendArgs a) {
+  latent_append<T, NT, VEC>(a, blockIdx.x);
+}
+
+static bool append_in_words(const LatentAppendArgs* a, size_t size) {
+  return ((a->rot / 2 | a->R | a->P | a->qst | a->qh | a->qrst | a->qrh |
+           a->kvst) & 3) == 0 &&
+      (((size_t)a->q | (size_t)a->qr | (size_t)a->kv | (size_t)a->w |
+        (size_t)a->cache) & (4 * size - 1)) == 0;
+}
+
 extern "C" int sv_latent_append(const LatentAppendArgs* a, int T, int f32,
                                 hipStream_t stream) {
   if (T <= 0) return 0;
   const size_t lds = a->rot * sizeof(float);
-  const size_t size = f32 ? 4 : 2;
-  const bool vec = ((a->rot / 2 | a->R | a->P | a->qst | a->qh | a->qrst |
-                     a->qrh | a->kvst) & 3) == 0 &&
-      (((size_t)a->q | (size_t)a->qr | (size_t)a->kv | (size_t)a->w |
-        (size_t)a->cache) & (4 * size - 1)) == 0;
+  const bool vec = append_in_words(a, f32 ? 4 : 2);
   // few rows: a longer workgroup waits for fewer words one after the other
   // (32 rows of 512 + 64, 32 heads: 7.1 -> 4.3 us; 4096 rows, element after
   // element 21, in words 15)
@@ -213,31 +223,36 @@ struct HeadLinearArgs {
   int T, H, N, K;
 };
 
+// 8 elements at p + k, zero from n on: a word is read in either case, since a
+// branch a word costs more than the word
+__device__ __forceinline__ uint4v word_or_zero(const short* p, int k, int n) {
+  const uint4v w = *(const uint4v*)(p + (k < n ? k : 0));
+  return k < n ? w : uint4v{0, 0, 0, 0};
+}
+
 // One wave of a workgroup's four takes every fourth 64-column block of K for
 // 32 outputs and 32 rows; the partial sums meet in LDS.  With SPLIT off each
 // wave has 32 outputs of its own.  K, strides and bases in 8 elements.
 template <bool SPLIT>
-__global__ void __launch_bounds__(256)
-head_linear_mfma_kernel(HeadLinearArgs a) {
+__device__ __forceinline__ void head_linear_mfma(const HeadLinearArgs& a, int nb,
+                                                 int h, int t0) {
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, hi = lane >> 5;
-  const int h = blockIdx.y, t0 = blockIdx.z * 32;
-  const int n0 = (SPLIT ? blockIdx.x : blockIdx.x * 4 + wid) * 32;
+  const int n0 = (SPLIT ? nb : nb * 4 + wid) * 32;
   const int K = a.K;
   const bool vn = n0 + col < a.N, vt = t0 + col < a.T;
   const short* w = (const short*)a.w + ((long)h * a.N + (vn ? n0 + col : 0)) * K;
   const short* x = (const short*)a.x + (long)(vt ? t0 + col : 0) * a.xst + h * a.xh;
   f32x16 acc = {};
-  const uint4v zero = {0, 0, 0, 0};
   if (n0 < a.N)
     for (int k0 = SPLIT ? wid * 64 : 0; k0 < K; k0 += SPLIT ? 256 : 64) {
       frag_u fw[4], fx[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const int k = k0 + 32 * hi + 8 * c;   // any order, the same for both
-        fw[c].u4 = vn && k < K ? *(const uint4v*)(w + k) : zero;
-        fx[c].u4 = vt && k < K ? *(const uint4v*)(x + k) : zero;
+        const int k = k0 + 16 * c + 8 * hi;
+        fw[c].u4 = word_or_zero(w, k, K);
+        fx[c].u4 = word_or_zero(x, k, K);
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc = mfma_bf16(fw[c].bf, fx[c].bf, acc);
@@ -274,6 +289,27 @@ head_linear_mfma_kernel(HeadLinearArgs a) {
       store4((short*)a.out + t * a.ost + h * a.oh + n, v);
     }
   }
+}
+
+template <bool SPLIT>
+__global__ void __launch_bounds__(256)
+head_linear_mfma_kernel(HeadLinearArgs a) {
+  head_linear_mfma<SPLIT>(a, blockIdx.x, blockIdx.y, blockIdx.z * 32);
+}
+
+// What a decoding step does before its attention, in one launch: rows are
+// appended by the first `rows` workgroups, the others take the queries into the
+// latent space (32 rows, 32 heads of 128 + 64, rank 512: 6 us for 10.5 of two
+// launches).
+template <bool VEC, bool SPLIT>
+__global__ void __launch_bounds__(256)
+latent_absorb_kernel(LatentAppendArgs a, HeadLinearArgs l, int rows, int nb) {
+  if ((int)blockIdx.x < rows) {
+    latent_append<short, 256, VEC>(a, blockIdx.x);
+    return;
+  }
+  const int id = blockIdx.x - rows;
+  head_linear_mfma<SPLIT>(l, id % nb, id / nb % l.H, id / nb / l.H * 32);
 }
 
 // any size and type: one output a thread
@@ -320,19 +356,101 @@ extern "C" int sv_head_linear(const HeadLinearArgs* a, int mfma, int f32,
 //   3. O^T += V^T P^T, each wave a quarter of the latent columns; V^T is the
 //      same tile, read through the transposing LDS load
 // The columns are padded to EP latents and 64 rotated ones, with zeros.
+//
+// Several splits: rows * splits workgroups share all rows' tiles, about as many
+// each, so that long rows are not waited for (32 rows of 512 to 4096 keys: 33 us
+// with as many workgroups for every row, 27 with as many tiles).  A workgroup
+// finds its share from the positions.
 // ---------------------------------------------------------------------------
 struct LatentRowsArgs {
   const short* q;           // [rows][H][R + P]
   const short* cache;
   const int *pos, *seq, *bt;
-  float* part;              // [rows][H][splits][R + 2] or null (1 split)
+  float* part;              // sums [rows * splits][H][R], their maxima and
+                            //   totals [rows * splits][H][2], of every row its
+                            //   first share and their number; null: 1 split
   short* out;               // [rows][H][R]
   int MB, rows, H, R, P, splits, window;
   float scale;
   const short* sink;        // [H] or null
 };
 
-template <int EP>
+__device__ __forceinline__ float2* share_totals(const LatentRowsArgs& a) {
+  return (float2*)(a.part + (long)a.rows * a.splits * a.H * a.R);
+}
+__device__ __forceinline__ int2* row_shares(const LatentRowsArgs& a) {
+  return (int2*)(share_totals(a) + (long)a.rows * a.splits * a.H);
+}
+
+// Sums and maxima over lanes without a way through LDS.
+template <int CTRL, int ROWS = 0xf, typename T>
+__device__ __forceinline__ T lanes_by(T x) {  // zero where no lane is
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(
+      0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xf, false));
+}
+// over the 8 lanes that share lane / 8
+template <typename Op>
+__device__ __forceinline__ float fold8(float x, Op op) {
+  x = op(x, lanes_by<0xB1>(x));          // neighbours
+  x = op(x, lanes_by<0x4E>(x));          // pairs of them
+  return op(x, lanes_by<0x141>(x));      // mirrored
+}
+template <typename Op>
+__device__ __forceinline__ float fold64(float x, Op op) {
+  x = fold8(x, op);
+  x = op(x, lanes_by<0x140>(x));         // 16 lanes mirrored
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x),
+                                            false, false);
+  x = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
+                                       false, false);
+  return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// the sum up to a lane
+__device__ __forceinline__ int scan64(int x) {
+  x += lanes_by<0x111>(x);
+  x += lanes_by<0x112>(x);
+  x += lanes_by<0x114>(x);
+  x += lanes_by<0x118>(x);
+  x += lanes_by<0x142, 0xa>(x);          // the rows before, 16 lanes each
+  x += lanes_by<0x143, 0xc>(x);
+  return x;
+}
+
+struct Share { int row, i, n; };         // the i-th of n of a row
+
+// The share of workgroup `item`; row is -1 if there is none.  Shares are of at
+// most `per` tiles, so there are no more than total / per + rows of them.
+__device__ __forceinline__ Share share_of(const LatentRowsArgs& a, int item) {
+  const int lane = threadIdx.x & 63;
+  const int items = a.rows * a.splits;
+  auto tiles = [&](int b) {
+    if (b + lane >= a.rows) return 0;
+    const int p = a.pos[b + lane];
+    return p / 32 - (a.window > 0 ? max(0, p - a.window + 1) / 32 : 0) + 1;
+  };
+  int n = tiles(0), total = __builtin_amdgcn_readlane(scan64(n), 63);
+  for (int b = 64; b < a.rows; b += 64)
+    total += __builtin_amdgcn_readlane(scan64(tiles(b)), 63);
+  const int per = (total + items - a.rows - 1) / (items - a.rows);
+  for (int b = 0;;) {
+    const int mine = (n + per - 1) / per;
+    const int last = scan64(mine);       // of the shares up to this lane's row
+    const int sum = __builtin_amdgcn_readlane(last, 63);
+    if (item < sum) {
+      const int l = __ffsll((unsigned long long)__ballot(last > item)) - 1;
+      const int k = __builtin_amdgcn_readlane(mine, l);
+      return {b + l, item - __builtin_amdgcn_readlane(last, l) + k, k};
+    }
+    item -= sum;
+    b += 64;
+    if (b >= a.rows) return {-1, 0, 0};
+    n = tiles(b);
+  }
+}
+
+// FULL: R = EP and P = 64, no padding
+template <int EP, bool FULL>
 __global__ void __launch_bounds__(256, 2)
 latent_rows_kernel(LatentRowsArgs a) {
   constexpr int KP = EP + 64;            // columns of a tile row
@@ -346,20 +464,32 @@ latent_rows_kernel(LatentRowsArgs a) {
   __shared__ __attribute__((aligned(16))) short pp[3][32 * PP];
   __shared__ float corr[32], lsum[32], mrow[32];
 
-  const int split = blockIdx.x % a.splits;
-  const int unit = blockIdx.x / a.splits;
-  const int nhg = (a.H + 31) / 32;
-  const int h0 = unit % nhg * 32, row = unit / nhg;
+  const int items = a.rows * a.splits, item = blockIdx.x % items;
+  const int h0 = blockIdx.x / items * 32;
+  Share my = {item, 0, 1};
+  if (a.splits > 1) {
+    my = share_of(a, item);
+    if (my.row < 0) return;
+    if (my.i == 0 && h0 == 0 && threadIdx.x == 0)
+      row_shares(a)[my.row] = int2{item, my.n};
+  }
+  my.i = __builtin_amdgcn_readfirstlane(my.i);
+  my.n = __builtin_amdgcn_readfirstlane(my.n);
+  const int row = __builtin_amdgcn_readfirstlane(my.row);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, hi = lane >> 5;
-  const int R = a.R, P = a.P, RP = R + P;
-  const uint4v zero = {0, 0, 0, 0};
+  const int R = FULL ? EP : a.R, P = FULL ? 64 : a.P, RP = R + P;
 
   // column of a slot in a cached row, -1 for padding
   auto column = [&](int slot) {
     const int c = slot * 8;
+    if (FULL) return c;
     return c < EP ? (c < R ? c : -1) : (c - EP < P ? R + c - EP : -1);
+  };
+  auto word = [&](const short* src, int k) {
+    const uint4v w = *(const uint4v*)(src + max(k, 0));
+    return k < 0 ? uint4v{0, 0, 0, 0} : w;
   };
   auto swz_slot = [](int r, int slot) {
     return slot ^ (CPR % 16 == 0 ? r & 15 : (r >> 1) & 7);
@@ -367,37 +497,39 @@ latent_rows_kernel(LatentRowsArgs a) {
 
   frag_u qf[NCW];
   {
-    const bool live = h0 + col < a.H;
-    const short* src = a.q + ((long)row * a.H + (live ? h0 + col : 0)) * RP;
+    // heads that are none repeat the last one
+    const short* src = a.q + ((long)row * a.H + min(h0 + col, a.H - 1)) * RP;
 #pragma unroll
-    for (int c = 0; c < NCW; ++c) {
-      const int k = column((wid * NCW + c) * 2 + hi);
-      qf[c].u4 = live && k >= 0 ? *(const uint4v*)(src + k) : zero;
-    }
+    for (int c = 0; c < NCW; ++c)
+      qf[c].u4 = word(src, column((wid * NCW + c) * 2 + hi));
   }
 
   const int i_pos = a.pos[row];
   const int* bt = a.bt + (long)a.seq[row] * a.MB;
   const int lo = a.window > 0 ? max(0, i_pos - a.window + 1) : 0;
   const int t_lo = lo / 32, total = i_pos / 32 - t_lo + 1;
-  const int per = (total + a.splits - 1) / a.splits;
-  const int t0 = t_lo + split * per, t1 = min(t_lo + total, t0 + per);
+  const int per = (total + my.n - 1) / my.n;   // all of them have some
+  const int t0 = t_lo + my.i * per, t1 = min(t_lo + total, t0 + per);
 
   uint4v reg[NL];
+  int page = bt[t0 / 2];                 // of the tile that is asked for next
   auto issue = [&](int t) {
-    const short* src = a.cache + ((long)bt[t / 2] * SV_PAGE + (t & 1) * 32) * RP;
+    const short* src = a.cache + ((long)page * SV_PAGE + (t & 1) * 32) * RP;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int it = i * 256 + tid;
-      const int k = column(it % CPR);
-      reg[i] = k >= 0 ? *(const uint4v*)(src + it / CPR * RP + k) : zero;
+      if (FULL)                          // a tile is one piece
+        reg[i] = *(const uint4v*)(src + it * 8u);
+      else
+        reg[i] = word(src + (uint)(it / CPR * RP), column(it % CPR));
     }
+    page = bt[min(t + 1, t1 - 1) / 2];
   };
 
   f32x16 o[NB] = {};
   const int sh = tid >> 3, sk = tid & 7;   // softmax: head, 4-key group
   float m_run = NEG_BIG, l_run = 0.f;
-  if (a.sink && split == 0 && h0 + sh < a.H) {   // once for all splits
+  if (a.sink && my.i == 0 && h0 + sh < a.H) {    // once for all splits
     m_run = bits2f(a.sink[h0 + sh]) * SV_LOG2E;
     l_run = 1.f;
   }
@@ -441,8 +573,7 @@ latent_rows_kernel(LatentRowsArgs a) {
         s[j] = key >= lo && key <= i_pos ? s[j] * s2 : NEG_BIG;
         mt = fmaxf(mt, s[j]);
       }
-#pragma unroll
-      for (int off = 1; off < 8; off <<= 1) mt = fmaxf(mt, __shfl_xor(mt, off, 64));
+      mt = fold8(mt, MaxOp());
       const float mn = fmaxf(m_run, mt);   // every tile holds a visible key
       const float al = __builtin_amdgcn_exp2f(m_run - mn);
       m_run = mn;
@@ -452,8 +583,7 @@ latent_rows_kernel(LatentRowsArgs a) {
         s[j] = __builtin_amdgcn_exp2f(s[j] - mn);
         ps += s[j];
       }
-#pragma unroll
-      for (int off = 1; off < 8; off <<= 1) ps += __shfl_xor(ps, off, 64);
+      ps = fold8(ps, SumOp());
       l_run = l_run * al + ps;
       float x[4] = {s[0], s[1], s[2], s[3]};
 #pragma unroll
@@ -483,7 +613,7 @@ latent_rows_kernel(LatentRowsArgs a) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
         const int e = (wid * NB + nb) * 32;
-        if (e >= EP) continue;
+        if (EP < 128 && e >= EP) continue;
         union { tr4 h[2]; bf16x8 bf; } vf;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -503,49 +633,240 @@ latent_rows_kernel(LatentRowsArgs a) {
   }
   __syncthreads();
   if (h0 + col >= a.H) return;
-  const long rh = (long)row * a.H + h0 + col;
   const float inv = 1.f / lsum[col];
+  short* out = a.out + ((long)row * a.H + h0 + col) * R;
+  float* part = a.part + ((long)item * a.H + h0 + col) * R;
+  auto put = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      const int e = (wid * NB + nb) * 32 + 8 * rg + 4 * hi;
-      if (e >= R) continue;
-      if (a.splits == 1) {
-        const uint2 w = {pack_bf16x2(o[nb][4 * rg] * inv, o[nb][4 * rg + 1] * inv),
-                         pack_bf16x2(o[nb][4 * rg + 2] * inv,
-                                     o[nb][4 * rg + 3] * inv)};
-        *(uint2*)(a.out + rh * R + e) = w;
-      } else {
-        float* p = a.part + (rh * a.splits + split) * (R + 2) + e;
-        *(float2*)p = make_float2(o[nb][4 * rg], o[nb][4 * rg + 1]);
-        *(float2*)(p + 2) = make_float2(o[nb][4 * rg + 2], o[nb][4 * rg + 3]);
+      for (int rg = 0; rg < 4; ++rg) {
+        const int e = (wid * NB + nb) * 32 + 8 * rg + 4 * hi;
+        if ((!FULL || EP < 128) && e >= R) continue;
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = o[nb][4 * rg + j];
+        if (whole) {
+          v *= inv;
+          *(uint2*)(out + e) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        } else {
+          *(f32x4*)(part + e) = v;
+        }
+      }
+  };
+  if (a.splits == 1) put(std::true_type()); else put(std::false_type());
+  if (a.splits > 1 && wid == 0 && hi == 0)
+    share_totals(a)[(long)item * a.H + h0 + col] = float2{mrow[col], lsum[col]};
+}
+
+// ---------------------------------------------------------------------------
+// merge: the shares of RB rows of a head, every row by two waves; LINEAR: then
+// the head's values of them (and their gate), whose weights are asked for first.
+// Two launches with the merged rows in memory took 13.4 us for 32 rows, 32 heads,
+// rank 512, this 11.5.
+// ---------------------------------------------------------------------------
+template <int RB, bool LINEAR>
+__global__ void __launch_bounds__(512)
+latent_merge_kernel(LatentRowsArgs a, HeadLinearArgs l) {
+  constexpr int XP = 512 + 8;            // pitch of merged rows
+  __shared__ __attribute__((aligned(16))) float other[4][512];
+  __shared__ __attribute__((aligned(16))) short xs[LINEAR ? 16 * XP : 8];
+  __shared__ __attribute__((aligned(16))) float ys[LINEAR ? 4 : 1][2][256];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wid >> 2;             // of the shares, of the columns
+  const int c16 = lane & 15, grp = lane >> 4;
+  const int h = blockIdx.x, r0 = blockIdx.y * RB, t = r0 + c16;
+  const int R = a.R;
+  // 32 outputs a wave, every other 32 columns.  16 rows of 64 bytes a load: as
+  // 32 rows of two words each (32 x 32 products) the loads alone took 4 us.
+  frag_u fw[2][8];
+  s4v gate[2];
+  auto weights = [&](int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const short* w = (const short*)l.w +
+                       ((long)h * l.N + min(n + 16 * i + c16, l.N - 1)) * R;
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+        fw[i][b].u4 = word_or_zero(w, 32 * (2 * b + part) + 8 * grp, R);
+      if (l.gate)
+        gate[i] = *(const s4v*)((const short*)l.gate + min(t, a.rows - 1) * l.gst +
+                                h * l.gh + min(n + 16 * i + 4 * grp, l.N - 4));
+    }
+  };
+  int n0 = (wid & 3) * 32;
+  if (LINEAR) {
+    weights(n0);
+    if (RB < 16)                         // rows that are none
+      for (int i = threadIdx.x * 8; i < (16 - RB) * XP; i += 512 * 8)
+        *(uint4v*)(xs + RB * XP + i) = uint4v{0, 0, 0, 0};
+  }
+  const int e = lane * 8;
+  const long step = (long)a.H * R;
+#pragma unroll
+  for (int rr = wid & 3; rr < RB; rr += 4) {
+    const int row = r0 + rr;
+    f32x4 acc[2] = {};
+    float inv = 0.f;
+    if (row < a.rows) {
+      const int2 sh = row_shares(a)[row];
+      const float2* ml = share_totals(a) + (long)sh.x * a.H + h;
+      const float* p = a.part + ((long)sh.x * a.H + h) * R + (e < R ? e : 0);
+      auto total = [&](int s) {
+        const float2 v = ml[(long)min(s + lane, sh.y - 1) * a.H];
+        return s + lane < sh.y ? v : float2{NEG_BIG, 0.f};
+      };
+      float2 mine = total(0);
+      float mm = mine.x, sum = 0.f;
+      for (int s = 64; s < sh.y; s += 64) mm = fmaxf(mm, total(s).x);
+      mm = fold64(mm, MaxOp());
+      for (int b = 0; b < sh.y; b += 64) {
+        if (b > 0) mine = total(b);
+        const float w = __builtin_amdgcn_exp2f(mine.x - mm);
+        sum += w * mine.y;
+        const int end = min(64, sh.y - b);
+        // eight of this wave's on their way at a time, also the last ones
+        for (int s = part; s < end; s += 16) {
+          f32x4 v[8][2];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const f32x4* src = (const f32x4*)(p + (b + min(s + 2 * i, end - 1)) * step);
+            v[i][0] = src[0];
+            v[i][1] = src[1];
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {  // those past the end weigh nothing
+            const float c = __uint_as_float(
+                __builtin_amdgcn_readlane(__float_as_uint(w), (s + 2 * i) & 63));
+            acc[0] += c * v[i][0];
+            acc[1] += c * v[i][1];
+          }
+        }
+      }
+      sum = fold64(sum, SumOp());        // by all lanes
+      inv = e < R ? 1.f / sum : 0.f;
+    }
+    f32x4* meet = (f32x4*)(other[wid & 3] + e);
+    if (part) {
+      meet[0] = acc[0];
+      meet[1] = acc[1];
+    }
+    __syncthreads();
+    if (!part) {
+      acc[0] = (acc[0] + meet[0]) * inv;
+      acc[1] = (acc[1] + meet[1]) * inv;
+      const uint4v w = {pack_bf16x2(acc[0][0], acc[0][1]),
+                        pack_bf16x2(acc[0][2], acc[0][3]),
+                        pack_bf16x2(acc[1][0], acc[1][1]),
+                        pack_bf16x2(acc[1][2], acc[1][3])};
+      if (LINEAR) {
+        *(uint4v*)(xs + rr * XP + e) = w;  // zeros past R and past the last row
+      } else if (row < a.rows && e < R) {
+        *(uint4v*)(a.out + ((long)row * a.H + h) * R + e) = w;
       }
     }
-  if (a.splits > 1 && wid == 0 && hi == 0) {
-    float* p = a.part + (rh * a.splits + split) * (R + 2) + R;
-    p[0] = mrow[col];
-    p[1] = lsum[col];
+    if (LINEAR || RB > 4) __syncthreads();
+  }
+  if (!LINEAR) return;
+  for (int n1 = 0; n1 < l.N; n1 += 128, n0 += 128) {
+    if (n1 > 0) {
+      __syncthreads();                   // ys has been read
+      weights(n0);
+    }
+    f32x4 acc[2] = {};
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      frag_u fx;                         // zeros from R on
+      fx.u4 = *(const uint4v*)(xs + c16 * XP + 32 * (2 * b + part) + 8 * grp);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = mfma16(fw[i][b].bf, fx.bf, acc[i]);
+    }
+    if (part)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *(f32x4*)(ys[wid & 3][i] + lane * 4) = acc[i];
+    __syncthreads();
+    if (part || c16 >= RB || t >= a.rows) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int n = n0 + 16 * i + 4 * grp;
+      if (n + 3 >= l.N) continue;
+      acc[i] += *(const f32x4*)(ys[wid & 3][i] + lane * 4);
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[j] = l.gate ? acc[i][j] * sigmoid_f(bits2f(gate[i][j])) : acc[i][j];
+      store4((short*)l.out + t * l.ost + h * l.oh + n, v);
+    }
   }
 }
 
-extern "C" int sv_attn_merge(const float* part, void* out, long rows,
-                             int splits, int E, int f32, hipStream_t stream);
+#define LATENT_SHARES 512                // most of a group of 32 heads
 
-// R and P multiples of 8, R <= 512, P <= 64, rows 16-byte aligned
-extern "C" int sv_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
-  if (a->rows <= 0) return 0;
+static int launch_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
   const long grid = (long)a->rows * ((a->H + 31) / 32) * a->splits;
-#define LR(E) latent_rows_kernel<E><<<grid, 256, 0, stream>>>(*a)
-  if (a->P > 64) return 1;
+  const bool full = a->P == 64 && (a->R == 64 || a->R == 128 || a->R == 256 ||
+                                   a->R == 512);
+#define LR(E)                                                       \
+  do {                                                              \
+    if (full) latent_rows_kernel<E, true><<<grid, 256, 0, stream>>>(*a); \
+    else latent_rows_kernel<E, false><<<grid, 256, 0, stream>>>(*a);     \
+  } while (0)
+  if (a->P > 64 ||
+      (a->splits > 1 && (long)a->rows * a->splits > LATENT_SHARES))
+    return 1;
   if (a->R <= 64) LR(64);
   else if (a->R <= 128) LR(128);
   else if (a->R <= 256) LR(256);
   else if (a->R <= 512) LR(512);
   else return 1;
 #undef LR
+  return 0;
+}
+
+// R and P multiples of 8, R <= 512, P <= 64, rows 16-byte aligned; with several
+// splits at most LATENT_SHARES workgroups for a group of 32 heads
+extern "C" int sv_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
+  if (a->rows <= 0) return 0;
+  if (launch_latent_rows(a, stream)) return 1;
   if (a->splits > 1)
-    return sv_attn_merge(a->part, a->out, (long)a->rows * a->H, a->splits,
-                         a->R, 0, stream);
+    latent_merge_kernel<4, false>
+        <<<dim3(a->H, (a->rows + 3) / 4), 512, 0, stream>>>(*a, HeadLinearArgs{});
+  return (int)hipGetLastError();
+}
+
+struct LatentStepArgs {
+  LatentAppendArgs append;
+  HeadLinearArgs absorb;
+  LatentRowsArgs rows;
+  HeadLinearArgs values;    // of rows.out
+};
+
+// A decoding step: append and absorb, attend, values.  As sv_latent_rows and the
+// form on matrix cores of sv_head_linear.
+extern "C" int sv_latent_step(const LatentStepArgs* a, hipStream_t stream) {
+  const HeadLinearArgs& l = a->absorb;
+  const int T = a->rows.rows;
+  if (T <= 0) return 0;
+  {
+    const bool split = l.K >= 256;
+    const int nt = (l.N + 31) / 32, nb = split ? nt : (nt + 3) / 4;
+    const long grid = T + (long)nb * l.H * ((T + 31) / 32);
+    const size_t lds = a->append.rot * sizeof(float);
+#define LA(V, S) \
+  latent_absorb_kernel<V, S><<<grid, 256, lds, stream>>>(a->append, l, T, nb)
+    if (append_in_words(&a->append, 2)) { if (split) LA(true, true); else LA(true, false); }
+    else { if (split) LA(false, true); else LA(false, false); }
+#undef LA
+  }
+  if (launch_latent_rows(&a->rows, stream)) return 1;
+  if (a->rows.splits == 1) return sv_head_linear(&a->values, 1, 0, stream);
+#define LM(RB)                                                           \
+  latent_merge_kernel<RB, true>                                          \
+      <<<dim3(a->rows.H, (T + RB - 1) / RB), 512, 0, stream>>>(a->rows, a->values)
+  if (T <= 32) LM(4);
+  else if (T <= 64) LM(8);
+  else LM(16);
+#undef LM
   return (int)hipGetLastError();
 }

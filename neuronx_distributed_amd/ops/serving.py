@@ -185,6 +185,11 @@ class _LatentRowsArgs(ctypes.Structure):
                 + _fields("sink", ctypes.c_void_p))
 
 
+class _LatentStepArgs(ctypes.Structure):
+    _fields_ = [("append", _LatentAppendArgs), ("absorb", _HeadLinearArgs),
+                ("rows", _LatentRowsArgs), ("values", _HeadLinearArgs)]
+
+
 class _MoePlanArgs(ctypes.Structure):
     _fields_ = (_fields("z bias idx coef order tiles", ctypes.c_void_p)
                 + _fields("T E top tile_rows max_tiles kind groups keep best",
@@ -1210,12 +1215,8 @@ class LatentWeights:
     sink: Optional[torch.Tensor] = None   # (H,) joins the denominator
 
 
-def latent_append(q, rot_at: int, q_step: int, qr, qr_at: int, qr_step: int,
-                  kv, w: LatentWeights, cache, pos, seq, block_table,
-                  heads: int, eps: float):
-    """Norm the latents of kv (T, rank + P), rotate the shared key, write
-    both into the cache (pages, 64, rank + P); rotate columns [rot_at, + P) of
-    every head of q (heads ``q_step`` apart) into those at ``qr_at`` of qr."""
+def _append_args(q, rot_at, q_step, qr, qr_at, qr_step, kv, w, cache, pos, seq,
+                 block_table, heads, eps):
     T, R = q.shape[0], w.norm.shape[0]
     P = cache.shape[2] - R
     half = w.freq.shape[0]
@@ -1228,21 +1229,29 @@ def latent_append(q, rot_at: int, q_step: int, qr, qr_at: int, qr_step: int,
     assert (heads - 1) * qr_step + qr_at + P <= qr.shape[1]
     assert pos.shape[0] == seq.shape[0] == T == qr.shape[0]
     size = q.element_size()
-    a = _LatentAppendArgs(
+    return _LatentAppendArgs(
         q=_p(q) + rot_at * size, qst=q.stride(0), qh=q_step,
         qr=_p(qr) + qr_at * size, qrst=qr.stride(0), qrh=qr_step, kv=_p(kv),
         kvst=kv.stride(0), w=_p(w.norm), freq=_p(w.freq), cache=_p(cache),
         pos=_p(pos), seq=_p(seq), bt=_p(block_table),
         MB=block_table.shape[1], H=heads, R=R, P=P, rot=2 * half, eps=eps,
         amp=w.amplitude, pairs=int(w.pairs))
-    _check(library().sv_latent_append(ctypes.byref(a), T, _f32(q),
+
+
+def latent_append(q, rot_at: int, q_step: int, qr, qr_at: int, qr_step: int,
+                  kv, w: LatentWeights, cache, pos, seq, block_table,
+                  heads: int, eps: float):
+    """Norm the latents of kv (T, rank + P), rotate the shared key, write
+    both into the cache (pages, 64, rank + P); rotate columns [rot_at, + P) of
+    every head of q (heads ``q_step`` apart) into those at ``qr_at`` of qr."""
+    a = _append_args(q, rot_at, q_step, qr, qr_at, qr_step, kv, w, cache, pos,
+                     seq, block_table, heads, eps)
+    _check(library().sv_latent_append(ctypes.byref(a), q.shape[0], _f32(q),
                                       _stream()), "latent_append")
 
 
-def head_linear(x, x_step: int, w, out, out_step: int,
-                gate: Optional[torch.Tensor] = None):
-    """out[t, h * out_step + n] = sum_k x[t, h * x_step + k] w[h, n, k], times
-    sigmoid(gate[t, h * N + n])."""
+def _linear_args(x, x_step, w, out, out_step, gate):
+    """Arguments, and whether the form on matrix cores takes them."""
     H, N, K = w.shape
     T = x.shape[0]
     assert w.is_contiguous() and x.stride(1) == out.stride(1) == 1
@@ -1259,6 +1268,14 @@ def head_linear(x, x_step: int, w, out, out_step: int,
         assert gate.dtype == x.dtype
         a.gate, a.gst, a.gh = _p(gate), gate.stride(0), N
         mfma = mfma and _aligned((), gate)
+    return a, mfma
+
+
+def head_linear(x, x_step: int, w, out, out_step: int,
+                gate: Optional[torch.Tensor] = None):
+    """out[t, h * out_step + n] = sum_k x[t, h * x_step + k] w[h, n, k], times
+    sigmoid(gate[t, h * N + n])."""
+    a, mfma = _linear_args(x, x_step, w, out, out_step, gate)
     _check(library().sv_head_linear(ctypes.byref(a), int(mfma), _f32(x),
                                     _stream()), "head_linear")
     return out
@@ -1267,6 +1284,28 @@ def head_linear(x, x_step: int, w, out, out_step: int,
 def latent_rows_supported(dtype, rank: int, shared: int) -> bool:
     return (dtype == torch.bfloat16 and rank % 8 == 0 and shared % 8 == 0
             and rank <= 512 and shared <= 64)
+
+
+def _latent_rows_args(q, cache, rank, pos, seq, block_table, heads, scale,
+                      window, max_keys, sink, out):
+    """Arguments and the workspace that they point to.  Workgroups of 64 keys
+    while CUs have none (1 row of 1000 keys: the whole step 28.1 us with 128,
+    24.9 with 64), then of 128 (8 of 4096: 32.5, with 64 35.7), and no merge for
+    up to 128 (43 rows of 82: 23.6, in two 28.7)."""
+    rows, D = q.shape[0], cache.shape[2]
+    units = rows * -(-heads // 32)
+    splits = 1 if max_keys <= 128 else max(
+        _row_splits(512, units, max_keys, 128),
+        _row_splits(256, units, max_keys, 64))
+    # sums, maxima and totals of every share; of every row, its shares
+    part = torch.empty(rows * heads * splits * (rank + 2) + 2 * rows,
+                       dtype=torch.float32, device=q.device) \
+        if splits > 1 else None
+    return _LatentRowsArgs(
+        q=_p(q), cache=_p(cache), pos=_p(pos), seq=_p(seq),
+        bt=_p(block_table), part=_p(part), out=_p(out),
+        MB=block_table.shape[1], rows=rows, H=heads, R=rank, P=D - rank,
+        splits=splits, window=window, scale=scale, sink=sink), part
 
 
 def latent_rows(q, cache, rank: int, pos, seq, block_table, heads: int,
@@ -1286,20 +1325,17 @@ def latent_rows(q, cache, rank: int, pos, seq, block_table, heads: int,
         max_keys = min(max_keys, window) if max_keys else window
     out = torch.empty(rows, heads * rank, dtype=q.dtype, device=q.device)
     fast = latent_rows_supported(q.dtype, rank, D - rank)
-    splits = _row_splits(512, rows * -(-heads // 32), max_keys, 128) if fast \
-        else _row_splits(1024, rows, max_keys, 128)
-    part = torch.empty(rows * heads * splits * (rank + 2),
-                       dtype=torch.float32, device=q.device) \
-        if splits > 1 else None
     if fast:
-        a = _LatentRowsArgs(
-            q=_p(q), cache=_p(cache), pos=_p(pos), seq=_p(seq),
-            bt=_p(block_table), part=_p(part), out=_p(out),
-            MB=block_table.shape[1], rows=rows, H=heads, R=rank, P=D - rank,
-            splits=splits, window=window, scale=scale, sink=mod.sink)
+        a, part = _latent_rows_args(q, cache, rank, pos, seq, block_table,
+                                    heads, scale, window, max_keys, mod.sink,
+                                    out)
         _check(library().sv_latent_rows(ctypes.byref(a), _stream()),
                "latent_rows")
         return out
+    splits = _row_splits(1024, rows, max_keys, 128)
+    part = torch.empty(rows * heads * splits * (rank + 2),
+                       dtype=torch.float32, device=q.device) \
+        if splits > 1 else None
     # one key/value head whose value is the front of its key
     a = _RowsArgs(q=_p(q), k=_p(q), v=_p(q), qst=q.stride(0),
                   kst=q.stride(0), vst=q.stride(0), kc=_p(cache),
@@ -1390,15 +1426,37 @@ def latent_attention(q, kv, gate, batch, cache, w: LatentWeights, heads: int,
         latent_portions(q[:n], g, cache, w, batch, spans, heads, dim, vdim,
                         scale, window, out[:n])
     if n < T:
-        at = (batch.pos[n:], batch.seq[n:], batch.block_table)
+        one = (batch.pos, batch.seq)
+        if n:
+            q, kv, gate = (t if t is None else t[n:] for t in (q, kv, gate))
+            one = [t[n:] for t in one]
+        at = (*one, batch.block_table)
         ql = torch.empty(T - n, heads * D, dtype=q.dtype, device=q.device)
-        latent_append(q[n:], dim, dim + P, ql, R, D, kv[n:], w, cache, *at,
-                      heads, eps)
-        head_linear(q[n:], dim + P, w.absorb, ql, D)
+        lat = torch.empty(T - n, heads * R, dtype=q.dtype, device=q.device)
+        up, fast = _linear_args(q, dim + P, w.absorb, ql, D, None)
+        down, ok = _linear_args(
+            lat, R, w.expand[heads * dim:].view(heads, vdim, R),
+            out[n:] if n else out, vdim, gate)
+        if fast and ok and latent_rows_supported(q.dtype, R, P):
+            keys = batch.max_keys
+            if window > 0:
+                keys = min(keys, window) if keys else window
+            sink = _score_args(ScoreMod(sink=w.sink), ql, heads).sink
+            rows, part = _latent_rows_args(ql, cache, R, *at, heads, scale,
+                                           window, keys, sink, lat)
+            a = _LatentStepArgs(
+                append=_append_args(q, dim, dim + P, ql, R, D, kv, w, cache,
+                                    *at, heads, eps),
+                absorb=up, rows=rows, values=down)
+            _check(library().sv_latent_step(ctypes.byref(a), _stream()),
+                   "latent_step")
+            return out
+        latent_append(q, dim, dim + P, ql, R, D, kv, w, cache, *at, heads, eps)
+        head_linear(q, dim + P, w.absorb, ql, D)
         lat = latent_rows(ql, cache, R, *at, heads, scale, window,
                           batch.max_keys, w.sink)
         head_linear(lat, R, w.expand[heads * dim:].view(heads, vdim, R),
-                    out[n:], vdim, None if gate is None else gate[n:])
+                    out[n:] if n else out, vdim, gate)
     return out
 
 

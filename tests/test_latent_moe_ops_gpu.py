@@ -162,6 +162,53 @@ def test_latent_mixed_batch(sv, dtype):
                dtype, 4.0, expand)
 
 
+@pytest.mark.parametrize("H,R,P", [(3, 64, 64), (33, 72, 16), (2, 512, 64),
+                                   (5, 256, 40)])
+@pytest.mark.parametrize("rows", [1, 2, 9, 65, 130, 255, 300])
+@pytest.mark.parametrize("window", [0, 45])
+def test_rows_of_all_lengths_share_workgroups(sv, rows, H, R, P, window):
+    """Short and long rows in one call: every key once, in whatever share."""
+    dtype, T = torch.bfloat16, 900
+    cache, bt = _cache([T], R + P, dtype, seed=rows)
+    keys = _rand(T, R + P, dtype=dtype, seed=1)
+    for p in range(-(-T // 64)):
+        part = keys[64 * p:64 * p + 64].cuda()
+        cache[int(bt[0, p]), :len(part)] = part
+    pos = [(0, 31, 899, 64, 32, 450)[i % 6] * 997 // (997 + i // 6)
+           for i in range(rows)]
+    q = _rand(rows, H * (R + P), dtype=dtype, seed=2, scale=0.3)
+    got = sv.latent_rows(q.cuda(), cache, R, _ints(pos), _ints([0] * rows), bt,
+                         H, 0.21, window, max(pos) + 1).view(rows, H, R)
+    qd, kd = q.double().view(rows, H, R + P), keys.double()
+    want = torch.empty(rows, H, R, dtype=torch.float64)
+    for i, p in enumerate(pos):
+        seen = slice(max(0, p - window + 1) if window else 0, p + 1)
+        want[i] = (qd[i] @ kd[seen].T * 0.21).softmax(-1) @ kd[seen, :R]
+    _close(got, want, dtype, what=(rows, H, R, P, window))
+
+
+@pytest.mark.parametrize("T", [3, 40, 70, 130])
+@pytest.mark.parametrize("H,D,P,E,R", [(2, 16, 64, 136, 320), (3, 40, 8, 12, 40),
+                                       (2, 264, 64, 260, 512)])
+def test_decoding_step_of_many_requests(sv, T, H, D, P, E, R):
+    """Single tokens of T requests behind 150 others each, in one step."""
+    dtype, ctx, window = torch.bfloat16, 150, 0
+    cases = [_latent_case(sv, H, D, P, E, R, window, ctx + 1, dtype, seed=9 * i)
+             for i in range(3)]
+    w, cfg = cases[0][3:5]
+    cache, bt = _cache([ctx + 1] * T, R + P, dtype)
+    for i in range(T):
+        q, kv, g = (t[:ctx] for t in cases[i % 3][:3])
+        _run(sv, Batch(sv, [(i, 0, ctx)], bt, window, False), q, kv, g, cache,
+             w, cfg)
+    b = Batch(sv, [(i, ctx, 1) for i in range(T)], bt, window, False)
+    q, kv, g = (torch.cat([cases[i % 3][k][ctx:] for i in range(T)])
+                for k in range(3))
+    got = _run(sv, b, q, kv, g, cache, w, cfg)
+    want = torch.cat([cases[i % 3][5][ctx:] for i in range(T)])
+    _close(got, want, dtype, 4.0, (T, H, D, P, E, R))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [64, 70, 33, 128, 1, 65])
 def test_latent_window_edges_show(sv, window, dtype):
