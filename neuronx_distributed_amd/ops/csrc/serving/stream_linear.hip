@@ -8,12 +8,14 @@
 //
 // Measured cold, us (library product, with the activation behind it | stream |
 // stay), which the rule of ops/serving.py follows:
-//   28672 x 4096 gated   1 row 66 | 46 | 45   16 rows 68 | 71 | 48   32: 60 | - | 53
-//   28672 x 4096         1 row 63 | 41 | 46    4 rows 64 | 45 | 46   16: 65 | 66 | 50
-//   32000 x 4096, 32 bit 1 row 59 | 45 | 50    4 rows 60 | 49 | 51   16: 60 | 72 | 53
-//   4096 x 14336         1 row 27 | 25 | -     4 rows 27 | 27 | -
-//   4096 x 4096          1 row 15 |  9 | 12   16 rows 15 | 12 | 14   32: 13 | 16 | 18
-// One row reads 5.2 to 5.7 TB/s of weights, a copy 5.2.
+//   28672 x 4096 gated   1 row 66 | 46 | 44   16 rows 68 | 71 | 47   32: 60 | - | 51
+//   28672 x 4096         1 row 63 | 40 | 46    4 rows 64 | 43 | 46   16: 65 | 60 | 49
+//   32000 x 4096, 32 bit 1 row 59 | 42 | 48    4 rows 60 | 45 | 48   16: 60 | 64 | 51
+//   4096 x 14336         1 row 27 | 22 | -     4 rows 27 | 23 | -
+//   4096 x 4096          1 row 14 | 7.5 | 12  16 rows 14 | 10 | 14   32: 13 | 14 | 17
+// One row reads 4.5 to 5.7 TB/s of weights, a copy 5.1.  With a branch a load every
+// product waited for all loads on their way: 8.5, 23 and 45 us where one row of
+// 4096 x 4096, 4096 x 14336 and 28672 gated columns now take 7.5, 22 and 43.5.
 
 #include "serving.h"
 
@@ -54,11 +56,23 @@ __device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n,
         uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
 }
 
+// Words past a row are read as its first ones, and become zeros where they are
+// multiplied: a branch a load, or a select behind it, would make every product
+// wait for the loads of the next turn.
+__device__ __forceinline__ uint4v word_at(const short* p, bool in, int k) {
+  return *(const uint4v*)(p + (in ? k : 0));
+}
+__device__ __forceinline__ bf16x8 if_there(bool in, frag_u f) {
+  if (!in) f.u4 = uint4v{0, 0, 0, 0};
+  return f.bf;
+}
+
 // One workgroup = 16 weight rows by MT tiles of 16 rows of x; its 16 waves take
 // K in turns of 64 columns and meet in LDS.  Weights go from memory straight into registers as fragments (a lane's
 // 16 bytes of a row, 64 bytes of 16 rows a load), a turn ahead.  Every workgroup
 // reads all of x, as much as its weights at 16 rows.
-template <int MT, int EPI>
+// FULL: K is a multiple of 64.
+template <int MT, int EPI, bool FULL>
 __global__ void __launch_bounds__(1024) stream_linear_kernel(StreamArgs a) {
   constexpr int U = 2, STEP = 16 * U * 32;
   __shared__ f32x4 part[16][MT][64];
@@ -75,44 +89,58 @@ __global__ void __launch_bounds__(1024) stream_linear_kernel(StreamArgs a) {
     x[i] = a.x + (long)min(t0 + i * 16 + c16, a.T - 1) * a.xst + grp * 8;
 
   f32x4 acc[MT] = {};
-  const uint4v zero = {0, 0, 0, 0};
   auto load = [&](int k0, frag_u* fw, frag_u (*fx)[MT])
       __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = k0 + u * 32;
-      const bool in = k + grp * 8 < K;
-      fw[u].u4 = in ? *(const uint4v*)(w + k) : zero;
+      const bool in = FULL || k + grp * 8 < K;
+      fw[u].u4 = word_at(w, in, k);
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-        fx[u][i].u4 = in ? *(const uint4v*)(x[i] + k) : zero;
+      for (int i = 0; i < MT; ++i) fx[u][i].u4 = word_at(x[i], in, k);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&](const frag_u* fw, const frag_u (*fx)[MT])
+  auto multiply = [&](int k0, const frag_u* fw, const frag_u (*fx)[MT])
       __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      const bool in = FULL || k0 + u * 32 + grp * 8 < K;
 #pragma unroll
       for (int j = 0; j < MT; ++j)
-        acc[j] = mfma16(fw[u].bf, fx[u][j].bf, acc[j]);
+        acc[j] = mfma16(if_there(in, fw[u]), if_there(in, fx[u][j]), acc[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   frag_u wa[U], xa[U][MT], wb[U], xb[U][MT];
   int k = wid * U * 32;
-  if (k < K) load(k, wa, xa);
-  for (; k < K; k += 2 * STEP) {
-    if (k + STEP < K) load(k + STEP, wb, xb);
-    multiply(wa, xa);
-    if (k + STEP >= K) break;
-    if (k + 2 * STEP < K) load(k + 2 * STEP, wa, xa);
-    multiply(wb, xb);
+  if (k < K) {
+    load(k, wa, xa);
+    // The last turns have no load behind them, in code of their own: where both
+    // ways join, a product would wait as for the shorter one.
+    for (; k + 2 * STEP < K; k += 2 * STEP) {
+      load(k + STEP, wb, xb);
+      multiply(k, wa, xa);
+      load(k + 2 * STEP, wa, xa);
+      multiply(k + STEP, wb, xb);
+    }
+    if (k + STEP < K) {
+      load(k + STEP, wb, xb);
+      multiply(k, wa, xa);
+      multiply(k + STEP, wb, xb);
+    } else {
+      multiply(k, wa, xa);
+    }
   }
 #pragma unroll
   for (int j = 0; j < MT; ++j) part[wid][j][lane] = acc[j];
   __syncthreads();
   if (wid >= MT) return;
-  f32x4 v = {};
+  f32x4 v = {}, y[16];
 #pragma unroll
-  for (int s = 0; s < 16; ++s) v += part[s][wid][lane];
+  for (int s = 0; s < 16; ++s) y[s] = part[s][wid][lane];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) v += y[s];
   store_rows<EPI>(a, t0 + wid * 16 + c16, n0 + 4 * grp, v, v);
 }
 
@@ -120,7 +148,10 @@ __global__ void __launch_bounds__(1024) stream_linear_kernel(StreamArgs a) {
 // 16 weight rows (or 16 gates and their projections).  Each of its NW waves
 // keeps its 256 PARTS columns of x in registers and reads the same columns of
 // one tile after the other, 256 at a time, one such part ahead.
-template <int NW, int PARTS, int MT, int EPI>
+// FULL: K is what they hold.  Otherwise words past it are zeros behind a branch
+// each, and a product waits for all loads on their way (zeros made of words that
+// are read in any case do not fit the registers).
+template <int NW, int PARTS, int MT, int EPI, bool FULL>
 __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   constexpr int RT = EPI == GLU ? 2 : 1;
   constexpr int UNITS = RT * PARTS;      // parts of a tile
@@ -130,27 +161,27 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   const int c16 = lane & 15, grp = lane >> 4;
   const int tiles = a.N / (16 * RT), step = gridDim.x;
   const int k0 = wid * PARTS * 256 + grp * 8;
-  const uint4v zero = {0, 0, 0, 0};
+  auto word = [&](const short* row, int k) __attribute__((always_inline)) {
+    return FULL || k0 + k < a.K ? *(const uint4v*)(row + k0 + k)
+                                : uint4v{0, 0, 0, 0};
+  };
 
   frag_u fx[PARTS * 8][MT];
 #pragma unroll
   for (int c = 0; c < PARTS * 8; ++c)
 #pragma unroll
     for (int j = 0; j < MT; ++j)
-      fx[c][j].u4 = k0 + c * 32 < a.K
-          ? *(const uint4v*)(a.x + (long)min(j * 16 + c16, a.T - 1) * a.xst +
-                             k0 + c * 32)
-          : zero;
-  const short* w = a.w + (long)c16 * a.wst + k0;
+      fx[c][j].u4 = word(a.x + (long)min(j * 16 + c16, a.T - 1) * a.xst, c * 32);
+  const short* w = a.w + (long)c16 * a.wst;
   // unit u of a tile; past the last tile that one again, and not used
   auto load = [&](int tile, int u, frag_u* fw) __attribute__((always_inline)) {
     const int p = u % PARTS;
-    const short* src = w + p * 256 +
+    const short* src = w +
         (long)(min(tile, tiles - 1) * 16 + (u / PARTS ? a.N / 2 : 0)) * a.wst;
 #pragma unroll
     for (int c = 0; c < 8; ++c)
-      fw[c].u4 = k0 + p * 256 + c * 32 < a.K ? *(const uint4v*)(src + c * 32)
-                                             : zero;
+      fw[c].u4 = word(src, p * 256 + c * 32);
+    __builtin_amdgcn_sched_barrier(0);
   };
   f32x4 acc[MT];
   auto multiply = [&](int u, const frag_u* fw, int buf)
@@ -164,6 +195,7 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         acc[j] = mfma16(fw[c].bf, fx[p * 8 + c][j].bf, acc[j]);
+    __builtin_amdgcn_sched_barrier(0);
     if (p == PARTS - 1)
 #pragma unroll
       for (int j = 0; j < MT; ++j)
@@ -174,11 +206,15 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
     __syncthreads();
     if (wid >= MT) return;
     f32x4 v = {}, u = {};
+    auto sum = [&](int row, f32x4& to) __attribute__((always_inline)) {
+      f32x4 y[NW];
 #pragma unroll
-    for (int s = 0; s < NW; ++s) {
-      v += part[buf][s][wid][lane];
-      if (EPI == GLU) u += part[buf][s][MT + wid][lane];
-    }
+      for (int s = 0; s < NW; ++s) y[s] = part[buf][s][row][lane];
+#pragma unroll
+      for (int s = 0; s < NW; ++s) to += y[s];
+    };
+    sum(wid, v);
+    if (EPI == GLU) sum(MT + wid, u);
     store_rows<EPI>(a, wid * 16 + c16, tile * 16 + 4 * grp, v, u);
   };
 
@@ -208,21 +244,28 @@ static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
     const int grid = min(tiles, 256);
     // at most 128 registers of x beside the weights (plain products of 17 to
     // 32 rows by a direct call alone, here and below: the library is faster)
-    if (a.T <= 16 && a.K <= 4096)
-      stay_linear_kernel<8, 2, 1, EPI><<<grid, 512, 0, stream>>>(a);
-    else if (a.T <= 16 && a.K <= 8192)
-      stay_linear_kernel<8, 4, 1, EPI><<<grid, 512, 0, stream>>>(a);
-    else if (a.T <= 32 && a.K <= 4096)
-      stay_linear_kernel<8, 2, 2, EPI><<<grid, 512, 0, stream>>>(a);
-    else
-      return 1;
+#define STAY(P, M)                                                          \
+  do {                                                                      \
+    if (a.K == 2048 * P)                                                    \
+      stay_linear_kernel<8, P, M, EPI, true><<<grid, 512, 0, stream>>>(a);  \
+    else                                                                    \
+      stay_linear_kernel<8, P, M, EPI, false><<<grid, 512, 0, stream>>>(a); \
+  } while (0)
+    if (a.T <= 16 && a.K <= 4096) STAY(2, 1);
+    else if (a.T <= 16 && a.K <= 8192) STAY(4, 1);
+    else if (a.T <= 32 && a.K <= 4096) STAY(2, 2);
+    else return 1;
+#undef STAY
   } else {
     if constexpr (EPI == GLU) return 1;
-    else if (a.T <= 16)
-      stream_linear_kernel<1, EPI><<<tiles, 1024, 0, stream>>>(a);
-    else
-      stream_linear_kernel<2, EPI>
-          <<<dim3(tiles, (a.T + 31) / 32), 1024, 0, stream>>>(a);
+    else {
+      const bool full = a.K % 64 == 0;
+      const dim3 grid(tiles, a.T <= 16 ? 1 : (a.T + 31) / 32);
+#define STREAM(M, F) stream_linear_kernel<M, EPI, F><<<grid, 1024, 0, stream>>>(a)
+      if (a.T <= 16) { if (full) STREAM(1, true); else STREAM(1, false); }
+      else { if (full) STREAM(2, true); else STREAM(2, false); }
+#undef STREAM
+    }
   }
   return (int)hipGetLastError();
 }
