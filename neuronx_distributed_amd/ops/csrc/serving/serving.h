@@ -73,6 +73,41 @@ __device__ __forceinline__ void load8<true, short>(const short* p, int n,
   for (int j = 0; j < 8; ++j) v[j] = bits2f(a[j]);
 }
 
+// Sums and maxima over lanes without a way through LDS.
+template <int CTRL, int ROWS = 0xf, typename T>
+__device__ __forceinline__ T lanes_by(T x) {  // zero where no lane is
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(
+      0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xf, false));
+}
+// over the 8 lanes that share lane / 8
+template <typename Op>
+__device__ __forceinline__ float fold8(float x, Op op) {
+  x = op(x, lanes_by<0xB1>(x));          // neighbours
+  x = op(x, lanes_by<0x4E>(x));          // pairs of them
+  return op(x, lanes_by<0x141>(x));      // mirrored
+}
+template <typename Op>
+__device__ __forceinline__ float fold64(float x, Op op) {
+  x = fold8(x, op);
+  x = op(x, lanes_by<0x140>(x));         // 16 lanes mirrored
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x),
+                                            false, false);
+  x = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
+                                       false, false);
+  return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// the sum up to a lane
+__device__ __forceinline__ int scan64(int x) {
+  x += lanes_by<0x111>(x);
+  x += lanes_by<0x112>(x);
+  x += lanes_by<0x114>(x);
+  x += lanes_by<0x118>(x);
+  x += lanes_by<0x142, 0xa>(x);          // the rows before, 16 lanes each
+  x += lanes_by<0x143, 0xc>(x);
+  return x;
+}
+
 // v_rcp_f32 and v_exp_f32 are good to one unit in the last place
 __device__ __forceinline__ float sigmoid_f(float x) {
   return __builtin_amdgcn_rcpf(1.f +

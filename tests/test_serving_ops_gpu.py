@@ -380,6 +380,45 @@ def test_memory_batch_and_slots(sv, dtype, gated):
 # norms and pointwise steps
 # ---------------------------------------------------------------------------
 
+@pytest.mark.parametrize("W", [2048, 2052, 4096, 4100, 8192, 8196, 16384, 16388])
+@pytest.mark.parametrize("pending,parts", [
+    ("rows", 0), ("rows", 1), ("rows", 6), ("rows", 8), ("rows", 9),
+    ("rows32", 0), (None, 0)])
+def test_residual_norm_of_few_rows(sv, W, parts, pending):
+    """A row a workgroup, one word after the other or a sum of rows; with and
+    without a residual, some rows only."""
+    T, eps, bf = 7, 0.03, torch.bfloat16
+    x = _rand(T, W, dtype=torch.float32)
+    d = _rand(T * max(1, parts), W, dtype=bf, seed=1, scale=3.0)
+    w = _rand(W, dtype=bf, seed=2)
+    coef = _rand(T, parts, dtype=torch.float32, seed=3) if parts else None
+    if pending == "rows32":
+        d = d.float() * 1.01
+    index = torch.tensor([5, 0, 5, 2], dtype=torch.int32)
+    y = d.double().view(T, -1, W)
+    y = (y * coef.double()[:, :, None] if parts else y).sum(1)
+    for res in (True, False):
+        if pending is None and not res:
+            continue
+        p = None if pending is None else sv.Pending(
+            d.cuda(), scale=0.7,
+            coef=coef.cuda() if parts else None)
+        base = x.double() if res else 0.0
+        want = base + 0.7 * y if p is not None else base
+        normed = want * (want.pow(2).mean(-1, keepdim=True) + eps).rsqrt() * \
+            (1.0 + w.double()) * 1.3
+        for ix in (None, index):
+            got, h, _ = sv.residual_norm(
+                x.cuda() if res else None, p, eps, w.cuda(), centred=True,
+                scale=1.3, index=None if ix is None else ix.cuda())
+            rows = slice(None) if ix is None else ix.long()
+            # 32-bit sums of up to 10 terms, then one rounding to bf16
+            torch.testing.assert_close(got.cpu().double(), want[rows],
+                                       rtol=2e-6, atol=2e-5)
+            torch.testing.assert_close(h.cpu().double(), normed[rows],
+                                       rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("W", [64, 100, 97, 1000, 4096])
 def test_residual_norm(sv, W, dtype):
