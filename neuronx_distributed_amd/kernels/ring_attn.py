@@ -143,8 +143,9 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
         return _block_bwd_masked(q, k, v, out, dout, lse, scale, 0, window)
     if q.is_cuda:
         import ctypes
-        from ..ops import (_fa_alloc_dkv, _fa_operand, _fa_strides,
-                           _fa_sum_replicas, _ptr, _require_lib, _stream)
+        from ..ops import (_fa_alloc_dkv, _fa_dkv_heads, _fa_operand,
+                           _fa_strides, _fa_sum_replicas, _ptr, _require_lib,
+                           _stream)
 
         lib = _require_lib()
         B, Hq, S, D = q.shape
@@ -153,13 +154,14 @@ def _block_bwd(q, k, v, out, dout, lse, causal, scale, window=None):
         dq = torch.empty_like(q)
         qc, kc, vc, oc, doc = (_fa_operand(t.contiguous())
                                for t in (q, k, v, out, dout))
-        dk_pq, dv_pq = _fa_alloc_dkv(kc, vc, Hq)
+        heads = _fa_dkv_heads(B, Hq, Hkv, S, causal, int(window or 0))
+        dk_pq, dv_pq = _fa_alloc_dkv(kc, vc, heads)
         lib.flash_attn_bwd_strided(
             _ptr(qc), _ptr(kc), _ptr(vc), _ptr(oc), _ptr(doc),
             _ptr(lse.contiguous()), _ptr(delta), _ptr(dq), _ptr(dk_pq),
             _ptr(dv_pq), ctypes.c_int(B), ctypes.c_int(Hq),
-            ctypes.c_int(Hkv), ctypes.c_int(S), ctypes.c_float(scale),
-            ctypes.c_int(1 if causal else 0),
+            ctypes.c_int(Hkv), ctypes.c_int(heads), ctypes.c_int(S),
+            ctypes.c_float(scale), ctypes.c_int(1 if causal else 0),
             ctypes.c_int(int(window) if window else 0),
             _fa_strides(qc, kc, vc, oc, doc, dq, dk_pq, dv_pq), _stream())
         dk, dv = _fa_sum_replicas(dk_pq, dv_pq, kc, vc)

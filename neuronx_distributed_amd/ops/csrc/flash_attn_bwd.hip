@@ -2,13 +2,13 @@
 //
 // Replaces the reference's NKI flash_attn_bwd (K2; reference
 // kernels/flash_attn.py:18,76-88):
-//   * fa_bwd_delta: delta[q] = sum_d dO*O (rowwise fp32)
+//   * fa_bwd_dq:    128-row Q blocks (4 waves x 32 q rows); delta[q] = sum_d
+//       dO*O (32-bit) of its rows; sequential kv loop, dQ accumulated in
+//       registers.
 //   * fa_bwd_dkdv:  128-row KV blocks; a sequential q loop recomputes P^T from
 //       (Q,K,lse), forms dS^T = P^T*(dP^T - delta), accumulates dK/dV in
-//       registers, for every Q HEAD.
-//   * fa_bwd_reduce: their sum over the q heads of a kv head (GQA).
-//   * fa_bwd_dq:    128-row Q blocks (4 waves x 32 q rows); sequential kv loop,
-//       dQ accumulated in registers.
+//       registers, for one or several q heads of a kv head.
+//   * fa_bwd_reduce: the sum of what is left of them (GQA).
 // No atomics anywhere: every output region is written by exactly one
 // workgroup.
 //
@@ -24,7 +24,9 @@
 // element was masked.  The vector work then stood between the products, beside
 // those of another wave at best; cut into pieces, one beside each product of the
 // same wave, both directions took 1823 us instead of 1874 (2 x 4096, 32 heads: 986
-// for 1021).  Bound by the matrix cores, 45 to 57 % busy at the 1.8 GHz that the
+// for 1021); delta beside the dQ kernel's fragments of dO and the q heads of a kv
+// head in one workgroup 1790 (a kernel for delta 22, the sum over heads 31).
+// Bound by the matrix cores, 45 to 57 % busy at the 1.8 GHz that the
 // card holds under such work.
 
 #include "common.h"
@@ -35,51 +37,20 @@
 #define LOG2E 1.4426950408889634f
 
 // ---------------------------------------------------------------------------
-// delta = rowsum(dO * O)
-// ---------------------------------------------------------------------------
-extern "C" __global__ void __launch_bounds__(256)
-fa_bwd_delta_kernel(const short* __restrict__ dout,
-                    const short* __restrict__ out, float* __restrict__ delta,
-                    long rows, int Hq, int S,
-                    long do_bs, long do_hs, long do_ss,
-                    long o_bs, long o_hs, long o_ss) {
-  // row enumerates (b, h, s).  16 lanes own one 128-elem row (8 bf16 per
-  // lane via b128 loads, coalesced 256 B per row segment); 4 shfl_xor
-  // steps fold the 16 partials — no LDS, no block barrier.  This is a
-  // pure streaming op (read 2 x B*Hq*S*128 bf16) and runs at HBM rate;
-  // the previous one-block-per-row form was ~14x off the read floor.
-  const int sub = threadIdx.x & 15;
-  const long row0 = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-  const long row_step = ((long)gridDim.x * blockDim.x) >> 4;
-  for (long row = row0; row < rows; row += row_step) {
-    const long b = row / ((long)Hq * S);
-    const long h = (row / S) % Hq;
-    const long sq = row % S;
-    s8v dv = *(const s8v*)(dout + b * do_bs + h * do_hs + sq * do_ss
-                           + sub * 8);
-    s8v ov = *(const s8v*)(out + b * o_bs + h * o_hs + sq * o_ss + sub * 8);
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s += bits2f(dv[j]) * bits2f(ov[j]);
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (sub == 0) delta[row] = s;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // dK/dV and dQ.  Tiles go from memory into two LDS buffers as they are and are
 // read both as rows and by transposing reads (lds.h).  Masks are applied only
 // on tiles that a boundary crosses.
 // ---------------------------------------------------------------------------
 struct BwdArgs {
-  const short *q, *k, *v, *dout;
-  const float *lse, *delta;
-  short *dq, *dk, *dv;      // dk, dv: one for every q head
-  int Hq, Hkv, S, causal, window;
+  const short *q, *k, *v, *out, *dout;
+  const float* lse;
+  float* delta;             // [B][Hq][S], written by the dQ kernel
+  short *dq, *dk, *dv;      // dk, dv: Hdk heads, each the sum of Hq / Hdk q heads
+  int Hq, Hkv, Hdk, S, causal, window;
   float scale;
   // element strides of (batch, head, seq)
   long q_bs, q_hs, q_ss, k_bs, k_hs, k_ss, v_bs, v_hs, v_ss;
+  long o_bs, o_hs, o_ss;
   long do_bs, do_hs, do_ss, dq_bs, dq_hs, dq_ss;
   long dk_bs, dk_hs, dk_ss, dv_bs, dv_hs, dv_ss;
 };
@@ -170,7 +141,8 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
 
   // heads on x, kv-blocks on y: causal work DEcreases with kv-block index,
   // so ascending y already dispatches biggest-first
-  const int k0 = blockIdx.y * 128, h = blockIdx.x, b = blockIdx.z;
+  const int k0 = blockIdx.y * 128, hd = blockIdx.x, b = blockIdx.z;
+  const int heads = a.Hq / a.Hdk, h = hd * heads;
   const int hkv = h / (a.Hq / a.Hkv);
   const int g = wid >> 1, half = wid & 1;
   const int kw0 = k0 + g * 32;           // this wave's first kv row
@@ -194,13 +166,23 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   // sliding window: q attends k iff k <= q < k + window
   const int q_end = window > 0 ? min(S, k0 + 127 + window) : S;
 
-  auto issue = [&](int q0, char* qb, char* db) __attribute__((always_inline)) {
-    fill_rows<64, 512>(qg, a.q_ss, q0, S, qb);
-    fill_rows<64, 512>(dg, a.do_ss, q0, S, db);
+  // Tiles of the first q head, then of the next ones: what is asked for next
+  int next = q_start;
+  auto issue = [&](char* qb, char* db) __attribute__((always_inline)) {
+    fill_rows<64, 512>(qg, a.q_ss, next, S, qb);
+    fill_rows<64, 512>(dg, a.do_ss, next, S, db);
   };
-  auto row_numbers = [&](int q0) __attribute__((always_inline)) {
-    const int q = min(q0 + (tid & 63), S - 1);
+  auto row_numbers = [&]() __attribute__((always_inline)) {
+    const int q = min(next + (tid & 63), S - 1);
     return tid < 64 ? lse[q] * LOG2E : tid < 128 ? delta[q] : 0.f;
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
+    if ((next += 64) < q_end) return;
+    next = q_start;
+    qg += a.q_hs;
+    dg += a.do_hs;
+    lse += S;
+    delta += S;
   };
 
   auto step = [&](int qt, char* qb, char* db, const float* ld_t)
@@ -286,22 +268,30 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
                       a.k_ss, k0, S, kb);
   fill_rows<128, 512>(a.v + b * a.v_bs + hkv * a.v_hs + st_r * a.v_ss + st_c,
                       a.v_ss, k0, S, vb);
-  float nl = row_numbers(q_start);
-  issue(q_start, q0b, d0b);
+  const int steps = heads * ((q_end - q_start + 63) / 64);
+  float nl = row_numbers();
+  issue(q0b, d0b);
   if (tid < 128) ld0[tid] = nl;
   __syncthreads();             // also waits for the words on their way
-  for (int q0 = q_start; q0 < q_end; q0 += 128) {
-    const int q1 = q0 + 64, q2 = q0 + 128;
-    nl = row_numbers(q1);
-    if (q1 < q_end) issue(q1, q1b, d1b);
-    if (tid < 128) ld1[tid] = nl;
+  for (int i = 0; i < steps; i += 2) {
+    int q0 = next;
+    advance();
+    if (i + 1 < steps) {
+      nl = row_numbers();
+      issue(q1b, d1b);
+      if (tid < 128) ld1[tid] = nl;
+    }
     step(q0, q0b, d0b, ld0);
     __syncthreads();
-    if (q1 >= q_end) break;
-    nl = row_numbers(q2);
-    if (q2 < q_end) issue(q2, q0b, d0b);
-    if (tid < 128) ld0[tid] = nl;
-    step(q1, q1b, d1b, ld1);
+    if (i + 1 >= steps) break;
+    q0 = next;
+    advance();
+    if (i + 2 < steps) {
+      nl = row_numbers();
+      issue(q0b, d0b);
+      if (tid < 128) ld0[tid] = nl;
+    }
+    step(q0, q1b, d1b, ld1);
     __syncthreads();
   }
 
@@ -326,8 +316,8 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   __syncthreads();
   meet(dk, room);
   if (half || my_k >= S) return;
-  store_turned(dv, 1.f, a.dv + b * a.dv_bs + h * a.dv_hs + my_k * a.dv_ss, hi);
-  store_turned(dk, a.scale, a.dk + b * a.dk_bs + h * a.dk_hs + my_k * a.dk_ss, hi);
+  store_turned(dv, 1.f, a.dv + b * a.dv_bs + hd * a.dv_hs + my_k * a.dv_ss, hi);
+  store_turned(dk, a.scale, a.dk + b * a.dk_bs + hd * a.dk_hs + my_k * a.dk_ss, hi);
 }
 
 __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
@@ -359,7 +349,23 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
     }
   }
   const long at = ((long)b * a.Hq + h) * S + q_ld;
-  const float lse2 = a.lse[at] * LOG2E, dlt = a.delta[at];
+  const float lse2 = a.lse[at] * LOG2E;
+  // delta = sum of dO O over the row, half of it in this lane
+  float dlt = 0.f;
+  {
+    const short* os = a.out + b * a.o_bs + h * a.o_hs + q_ld * a.o_ss + hi * 8;
+    s8v o[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) o[c] = *(const s8v*)(os + c * 16);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        dlt += __uint_as_float(dof[c].u[j] << 16) * bits2f(o[c][2 * j]) +
+               __uint_as_float(dof[c].u[j] & 0xffff0000u) * bits2f(o[c][2 * j + 1]);
+    dlt += __shfl_xor(dlt, 32, 64);
+    if (hi == 0 && my_q < S) a.delta[at] = dlt;
+  }
   const float s2 = a.scale == 0.f ? 1e-37f : a.scale * LOG2E;
   const float gone = s2 > 0.f ? -INFINITY : INFINITY;
 
@@ -507,27 +513,20 @@ extern "C" void flash_attn_bwd_reduce(const void* kq, const void* vq, void* dk,
 extern "C" void flash_attn_bwd_strided(
     const void* q, const void* k, const void* v, const void* out,
     const void* dout, const void* lse, void* delta, void* dq, void* dk,
-    void* dv, int B, int Hq, int Hkv, int S, float scale, int causal,
+    void* dv, int B, int Hq, int Hkv, int Hdk, int S, float scale, int causal,
     int window, const long* st, hipStream_t stream) {
-  // st = 24 longs: (bs, hs, ss) x (q, k, v, o, dout, dq, dk, dv)
-  long rows = (long)B * Hq * S;
-  // 16 lanes per row -> 16 rows per 256-thread block; cap well above the
-  // 256-CU fill point and grid-stride the rest
-  long blocks = (rows + 15) / 16;
-  int nb = blocks < 8192 ? (int)blocks : 8192;
-  fa_bwd_delta_kernel<<<nb, 256, 0, stream>>>(
-      (const short*)dout, (const short*)out, (float*)delta, rows, Hq, S,
-      st[12], st[13], st[14], st[9], st[10], st[11]);
+  // st = 24 longs: (bs, hs, ss) x (q, k, v, o, dout, dq, dk, dv); dk and dv of
+  // Hdk heads, Hkv <= Hdk <= Hq, each dividing the next
   const BwdArgs a{(const short*)q, (const short*)k, (const short*)v,
-                  (const short*)dout, (const float*)lse, (const float*)delta,
-                  (short*)dq, (short*)dk, (short*)dv, Hq, Hkv, S, causal,
-                  window, scale,
+                  (const short*)out, (const short*)dout, (const float*)lse,
+                  (float*)delta, (short*)dq, (short*)dk, (short*)dv, Hq, Hkv,
+                  Hdk, S, causal, window, scale,
                   st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8],
-                  st[12], st[13], st[14], st[15], st[16], st[17],
-                  st[18], st[19], st[20], st[21], st[22], st[23]};
-  const dim3 grid(Hq, (S + 127) / 128, B);
-  fa_bwd_dkdv_kernel<<<grid, 512, 0, stream>>>(a);
-  fa_bwd_dq_kernel<<<grid, 256, 0, stream>>>(a);
+                  st[9], st[10], st[11], st[12], st[13], st[14], st[15], st[16],
+                  st[17], st[18], st[19], st[20], st[21], st[22], st[23]};
+  const int blocks = (S + 127) / 128;
+  fa_bwd_dq_kernel<<<dim3(Hq, blocks, B), 256, 0, stream>>>(a);
+  fa_bwd_dkdv_kernel<<<dim3(Hdk, blocks, B), 512, 0, stream>>>(a);
 }
 
 extern "C" void flash_attn_bwd(const void* q, const void* k, const void* v,
@@ -550,5 +549,5 @@ extern "C" void flash_attn_bwd(const void* q, const void* k, const void* v,
     st[21 + i] = qd[i];           // dv
   }
   flash_attn_bwd_strided(q, k, v, out, dout, lse, delta, dq, dk, dv, B, Hq,
-                         Hkv, S, scale, causal, 0, st, stream);
+                         Hkv, Hq, S, scale, causal, 0, st, stream);
 }

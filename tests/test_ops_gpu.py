@@ -173,6 +173,42 @@ def test_flash_attn_bwd(B, Hq, Hkv, S, causal):
     _cmp(v.grad, vr.grad * 0.5, atol=5e-2, rtol=5e-2, name="dv")
 
 
+@pytest.mark.parametrize("Hq,Hkv,heads", [(4, 1, 1), (4, 1, 2), (4, 1, 4),
+                                          (6, 2, 2), (6, 2, 6)])
+@pytest.mark.parametrize("S,causal,window,scale", [
+    (1, True, 0, 0.09), (64, True, 0, -0.09), (129, True, 0, 0.09),
+    (333, True, 70, 0.09), (700, True, 130, -0.09), (290, False, 0, 0.09)])
+def test_flash_attn_bwd_sums_heads_in_a_workgroup(monkeypatch, Hq, Hkv, heads,
+                                                  S, causal, window, scale):
+    """dK and dV of one, some or all q heads of a kv head from a workgroup."""
+    monkeypatch.setattr(ops, "_fa_dkv_heads", lambda *a: heads)
+    torch.manual_seed(S)
+    B, D = 2, 128
+    leaves = [torch.randn(B, S, h, D, device="cuda").bfloat16().requires_grad_()
+              for h in (Hq, Hkv, Hkv)]
+    dy = torch.randn(B, S, Hq, D, device="cuda").bfloat16().transpose(1, 2)
+    out = ops.flash_attn(*(t.transpose(1, 2) for t in leaves), causal, scale,
+                         window)
+    got = torch.autograd.grad(out, leaves, dy)
+    exact = [t.detach().double().cpu().requires_grad_() for t in leaves]
+    ref = _torch_reference(*(t.transpose(1, 2) for t in exact), causal, scale,
+                           window or None)
+    want = torch.autograd.grad(ref, exact, dy.double().cpu())
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        # P, dS and the results are rounded to bf16 once each, 2^-9 relative
+        err = (a.double().cpu() - b).norm() / b.norm().clamp(min=1e-3)
+        assert err < 3 * 2 ** -8, (name, err)
+
+
+def test_flash_attn_bwd_heads_of_a_workgroup():
+    """They divide the group, and no CU is left idle for them."""
+    for B, Hq, Hkv, S, causal, window, n in (
+            (2, 32, 8, 3001, True, 1024, 2), (1, 32, 8, 8192, True, 0, 4),
+            (1, 32, 8, 4096, True, 0, 2), (1, 28, 4, 300, True, 0, 1),
+            (1, 40, 40, 5000, True, 0, 1), (2, 32, 8, 2000, False, 0, 4)):
+        assert ops._fa_dkv_heads(B, Hq, Hkv, S, causal, window) * n == Hq
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S", [
     (2, 8, 2, 512),
     (1, 32, 8, 2048),   # production GQA shape
