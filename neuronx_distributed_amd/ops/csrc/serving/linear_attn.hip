@@ -364,9 +364,12 @@ struct ChunkArgs {
   float *b, *i, *c;         // [H][T] (gated; timed: i is the step, no c)
   float *tot, *cend;        // [n_chunks][H][4], [n_chunks][H] (gated; timed:
                             //   no cend)
-  float* U;                 // [n_chunks][H][E][D]
+  float* U;                 // [n_chunks][H][E][D]; or null (no VT): a state is
+                            //   carried from chunk to chunk
   float* N;                 // [n_chunks][H][D] (gated): N, then n before
-  short* P;                 // [n_chunks][H][3][E][D] state before the chunk
+  short* P;                 // [n_chunks][H][3][E][D] state before the chunk; if
+                            //   there is no U [n_chunks][H][E / 32][3][D / 16]
+                            //   [64][8]: keys 16 c + 8 hi + 0..7 of column col
   float* mst;               // [n_chunks][H] m before the chunk (gated)
   short* VT;                // [n_chunks][H][E][256] V^T, activated; or null
                             //   (timed, D 64 or 128, E a multiple of 64)
@@ -1117,24 +1120,278 @@ memory_outputs_kernel(ChunkArgs x) {
     }
 }
 
+// ---- timed states of D = 64 or 128 by a multiple of 64, chunk after chunk ---
+// One workgroup carries DP keys x ET columns of a head's state through its
+// segment: the state stays in the accumulators, is scaled by what a chunk
+// forgets, and the chunk's weighted keys and values are added to it, 64 tokens a
+// piece.  Before a chunk its three planes go out as the outputs' fragments, 16
+// bytes a lane.  Keys come straight into LDS, two pieces ahead, and are turned by
+// transposing reads; values come through registers, two ahead as well, where
+// they are weighted and split.  One barrier a piece, which waits by count.
+//
+// The states of all chunks at once and a scan over them moved 70 MB of 32 bits
+// out and back and took two launches (2 x 2048 tokens, 128 heads of 128 x 64: 49 +
+// 30 us, now 55).  The planes' 107 MB and the values' 67 are what is left.
+template <int DP>
+__global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
+  constexpr int MT = DP / 32, ET = 128 / MT;   // tiles of keys; columns
+  constexpr int NC = DP / 16, SL = DP / 8, VS = ET / 8;
+  constexpr int LK = DP / 32, LV = ET / 32;    // words of a thread and piece
+  constexpr int PLANE = 64 * ET * 2, VA = 6;   // pieces that values are ahead
+  // apart by name, so that a read of one need not wait for the words on their
+  // way into another
+  __shared__ __attribute__((aligned(16))) char k0[64 * DP * 2], k1[64 * DP * 2],
+      k2[64 * DP * 2];
+  __shared__ __attribute__((aligned(16))) char v0[3 * PLANE], v1[3 * PLANE];
+  __shared__ float s_w[2][MC_L];
+  const MemoryArgs& a = x.a;
+  const int E = a.E;
+  // an XCD has the same heads of all segments: heads that share keys, and long
+  // segments beside short ones
+  const int units = a.H * (E / ET), per = (units + 7) / 8;
+  const int unit = blockIdx.x % 8 * per + blockIdx.x / 8 % per;
+  const int sg = blockIdx.x / 8 / per;
+  if (unit >= units) return;
+  const int h = unit / (E / ET), e0 = unit % (E / ET) * ET;
+  const int row0 = a.seg[4 * sg + 1], rows = a.seg[4 * sg + 2];
+  const int ctx = a.seg[4 * sg + 3];
+  const int ch0 = x.first[sg], ch1 = x.first[sg + 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hi = lane >> 5;
+  const int m = wid % MT, n = wid / MT;
+
+  auto turn = [](int r) { return SL == 16 ? row_turn(r) : value_turn<SL>(r); };
+  const short* kp = (const short*)a.k + row0 * a.kst + h / (a.H / a.G) * DP;
+  const short* vp = (const short*)a.v + row0 * a.vst + (long)h * E + e0;
+  // Pieces past the last are that one again, so that the words on their way keep
+  // their number.  As buffer loads: behind other loads into LDS the compiler
+  // waits for all of them where it needs a value.
+  const int last = max(0, rows - 1) / 64;
+  const int kst = (int)a.kst * 2, vst = (int)a.vst * 2;
+  auto issue_k = [&](int i, char* buf) __attribute__((always_inline)) {
+    i = min(i, last);
+    const auto src = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(kp + 64L * i * a.kst), 0, 0x7fffffff, 0x00027000);
+#pragma unroll
+    for (int p = 0; p < LK; ++p) {
+      const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src, (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16,
+          min(r, rows - 1 - 64 * i) * kst + s * 16, 0, 0, 0);
+    }
+  };
+  auto load_v = [&](int i, uint4v* v) __attribute__((always_inline)) {
+    i = min(i, last);
+    const char* src = (const char*)(vp + 64L * i * a.vst);
+#pragma unroll
+    for (int p = 0; p < LV; ++p) {
+      const int r = (p * 256 + tid) / VS;
+      v[p] = *(const uint4v*)(src + (uint)(min(r, rows - 1 - 64 * i) * vst +
+                                           tid % VS * 16));
+    }
+  };
+  // the weight of this thread's token of a chunk, at its end; what the chunk
+  // leaves of the state before it
+  float wb, wi, keep = 0.f;
+  f32x4 wt;
+  auto load_w = [&](int ch) __attribute__((always_inline)) {
+    const long o = (long)h * x.T + row0 + min((ch - ch0) * MC_L + tid, rows - 1);
+    wb = x.b[o];
+    wi = x.i[o];
+    wt = *(const f32x4*)(x.tot + ((long)ch * a.H + h) * 4);
+  };
+  auto weight = [&](int ch, float& keep) __attribute__((always_inline)) {
+    float d = wt[3] * (wid < 3);
+    d += wt[2] * (wid < 2);
+    d += wt[1] * (wid < 1);
+    d += wt[wid] - wb;
+    keep = expf(wt[0] + wt[1] + wt[2] + wt[3]);
+    return (ch - ch0) * MC_L + tid < rows ? expf(d) * wi : 0.f;
+  };
+  // the compiler knows nothing of the order that the wait below counts on
+  auto in_order = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+  };
+
+  f32x16 acc = {};
+  float* Sp = a.S + ((long)a.seg[4 * sg] * a.H + h) * DP * E + e0 + 32 * n + col;
+  if (ctx > 0)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[r] = Sp[(long)(32 * m + acc_row(r, hi)) * E];
+
+  // this lane's part of the addresses of transposing reads (bytes)
+  const int tr_key = 4 * hi + ((lane & 15) >> 2);
+  const int tr_col = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  const int kx = SL == 16 ? tr_lane(lane)
+                          : tr_key * DP * 2 + tr_col + value_turn<SL>(tr_key) * 16;
+  const int vx = tr_key * ET * 2 + tr_col + (VS == 8 ? value_turn<8>(tr_key) : 0) * 16;
+  // the weighted values of a piece, split
+  auto convert = [&](int i, const float* w, char* vb, const uint4v* v)
+      __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < LV; ++p) {
+      const int r = (p * 256 + tid) / VS;
+      const int s = tid % VS ^ (VS == 8 ? value_turn<8>(r) : 0);
+      float f[8];
+      uint4v u[3];
+      unpack8(64 * i + r < rows ? v[p] : uint4v{0, 0, 0, 0}, f);
+      const float wr = w[r];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint t[3];
+        split3(f[2 * j] * wr, f[2 * j + 1] * wr, t);
+#pragma unroll
+        for (int z = 0; z < 3; ++z) u[z][j] = t[z];
+      }
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+        *(uint4v*)(vb + z * PLANE + r * ET * 2 + s * 16) = u[z];
+    }
+  };
+  // piece i; w: of the piece behind it, whose values are made ready
+  auto piece = [&](int i, bool fresh, const float* w, char* kb, char* kn, char* vb, char* vn,
+                   uint4v* v) __attribute__((always_inline)) {
+    // The keys of this piece are here: behind them only those of the next were
+    // asked for, twice values, and the planes of the chunk's state if it is the
+    // first or second of a chunk (of the first chunk, these keys are here).
+    if (64 * i + 64 > rows) {
+      __builtin_amdgcn_s_waitcnt(0xf70);           // vmcnt(0)
+      in_order();
+#pragma unroll
+      for (int p = 0; p < LK; ++p)
+        if (64 * i + (p * 256 + tid) / SL >= rows)
+          *(uint4v*)(kb + (p * 256 + tid) * 16) = uint4v{0, 0, 0, 0};
+    }
+    in_order();
+    static_assert(LK + 2 * LV + 6 < 16, "");
+    if (fresh) __builtin_amdgcn_s_waitcnt(0x70 | (LK + 2 * LV + 6));
+    else __builtin_amdgcn_s_waitcnt(0x70 | (LK + 2 * LV));   // and lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    in_order();
+    issue_k(i + 2, kn);
+    in_order();
+    __builtin_amdgcn_sched_barrier(0);
+    union { tr4 t[2]; bf16x8 bf; } kf[4], vf[4][3];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        kf[c].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr4)(
+            kb + (SL == 16 ? (kx ^ (64 * m) ^ (32 * u)) : (kx ^ (64 * m))) +
+            (16 * c + 8 * u) * DP * 2));
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+          vf[c][z].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr4)(
+              vb + z * PLANE + (vx ^ (64 * n)) + (16 * c + 8 * u) * ET * 2));
+      }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int z = 0; z < 3; ++z) acc = mfma_bf16(kf[c].bf, vf[c][z].bf, acc);
+    convert(i + 1, w, vn, v);
+    __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
+#pragma unroll
+    for (int y = 0; y < 12; ++y) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, 7 * LV, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    in_order();
+    load_v(i + 1 + VA, v);
+    in_order();
+  };
+  // the planes as fragments of the outputs' products: lane (col, hi) has keys 16 c
+  // + 8 hi ... of column col
+  auto leave = [&](int ch) __attribute__((always_inline)) {
+    short* P = x.P + ((((long)ch * a.H + h) * (E / 32) + e0 / 32 + n) * 3 * NC +
+                      2 * m) * 512 + lane * 8;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      uint w[4][3];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        split3(acc[8 * c + 2 * u], acc[8 * c + 2 * u + 1], w[u]);
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        const auto r0 = __builtin_amdgcn_permlane32_swap(w[0][z], w[2][z], false,
+                                                         false);
+        const auto r1 = __builtin_amdgcn_permlane32_swap(w[1][z], w[3][z], false,
+                                                         false);
+        *(uint4v*)(P + (z * NC + c) * 512) = uint4v{r0[0], r1[0], r0[1], r1[1]};
+      }
+    }
+  };
+
+  if (rows > 0) {
+    uint4v v[VA][LV];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) load_v(i, v[i]);
+    load_w(ch0);
+    in_order();
+    issue_k(0, k0);
+    in_order();
+    issue_k(1, k1);
+    s_w[0][tid] = weight(ch0, keep);
+    __syncthreads();
+    convert(0, s_w[0], v0, v[0]);
+    in_order();
+    load_v(VA, v[0]);
+    char *const kr[3] = {k0, k1, k2}, *const vr[2] = {v0, v1};
+    const int pieces = last + 1;
+    if (ctx > 0) leave(ch0);
+    for (int cb = ch0; cb < ch1; cb += 3) {
+#pragma unroll
+      for (int y = 0; y < 3; ++y) {
+        const int ch = cb + y;
+        if (ch >= ch1) break;
+        acc *= keep;
+        const int i = 4 * (ch - ch0), now = (ch - ch0) & 1;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          if (i + p >= pieces) break;
+          if (p == 2) s_w[now ^ 1][tid] = weight(min(ch + 1, ch1 - 1), keep);
+          piece(i + p, p < 2, p < 3 ? s_w[now] + 64 * p + 64 : s_w[now ^ 1],
+                kr[(4 * y + p) % 3], kr[(4 * y + p + 2) % 3], vr[p % 2],
+                vr[(p + 1) % 2], v[(4 * y + p + 1) % VA]);
+          if (p == 0) load_w(min(ch + 1, ch1 - 1));
+        }
+        if (ch + 1 < ch1) leave(ch + 1);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xf70);             // vmcnt(0): LDS is given back
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    Sp[(long)(32 * m + acc_row(r, hi)) * E] = acc[r];
+}
+
 // ---- timed outputs of D = 64 or 128, 64 columns per workgroup ---------------
-// The same 128 queries, but all tiles come straight into LDS (DMA), one ahead:
-// the carried state's planes, 32 columns a tile, then keys and values, 64 tokens
-// a tile; values are turned by transposing reads.  Without tiles in registers
-// three workgroups share a CU: two wait half of the time for memory and barriers
-// (2 x 2048 tokens, 128 heads of 128 x 64: 207 -> 121 us, 300 MB of which are
-// 60).
+// The same 128 queries, but all tiles come straight into LDS (DMA), up to three
+// ahead of the one that is multiplied, in a ring of four: the carried state's
+// planes, as fragments, then keys and values, 32 tokens a tile, the oldest first;
+// values are turned by transposing reads.  One barrier a tile, which waits by
+// count.  Bound by latency: three workgroups share a CU, vector work fills 40 % of
+// the time, products 25 %.  2 x 2048 tokens, 128 heads of 128 x 64: tiles of 64
+// tokens, one ahead, with all words waited for at every barrier 129 us, now 117
+// (200 MB: 40).
 // The weights of an earlier group's keys are products: what is left at the end
-// of their group, and from there to the query.
+// of their group, and from there to the query.  The skip is part of a token's
+// weight on itself.
 template <int DP>
 __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   constexpr int NC = DP / 16, SL = DP / 8, KP = DP * 2;
-  constexpr int STATE = 3 * 32 * KP, KEYS = 64 * KP;
-  constexpr int OP = 68;                 // pitch of two waves' results
-  constexpr int SIZE = STATE > KEYS + 64 * 128 ? STATE : KEYS + 64 * 128;
-  constexpr int OUTS = 2 * 32 * OP * sizeof(float);
-  __shared__ __attribute__((aligned(16))) char b0[SIZE > OUTS ? SIZE : OUTS],
-      b1[SIZE > OUTS ? SIZE : OUTS];
+  constexpr int TILE = 12288, KEYS = 32 * KP;
+  constexpr int NS = DP / 32;            // tiles of the state: 8 NC / NS fragments
+  constexpr int LS = 3, LK = DP / 64, LT = LK + 1;   // words of a thread and tile
+  constexpr int OP = 68;                 // pitch of a wave's results
+  static_assert(32 * OP * 4 <= TILE && KEYS + 32 * 128 <= TILE &&
+                2 * 3 * NC * 1024 == NS * TILE, "");
+  // apart by name, so that a read of one need not wait for the words on their
+  // way into another
+  __shared__ __attribute__((aligned(16))) char b0[TILE], b1[TILE], b2[TILE], b3[TILE];
   __shared__ float s_col[MC_L], s_step[MC_L], s_far[MC_L];
   const MemoryArgs& a = x.a;
   const int E = a.E, nt = E / 64;
@@ -1158,64 +1415,93 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   const int tt = half * 4 + wid, jt = tt >> 1; // its 32 and 64 tokens
   const int hk = h / (a.H / a.G);
 
-  // thread tid fills 16-byte places tid, tid + 256, ... of a tile
-  auto turn = [](int r) { return SL == 16 ? row_turn(r) : key_turn<SL>(r); };
-  const short* P = x.P + (ci * 3 * E + e0) * DP;
-  auto issue_state = [&](int nb, char* buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int p = 0; p < STATE / 4096; ++p) {
-      const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(P + ((long)(r >> 5) * E + 32 * nb + (r & 31)) * DP + s * 8),
-          (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16, 0, 0);
-    }
-  };
-  const short* kp = (const short*)a.k + (long)row0 * a.kst + hk * DP;
-  const short* vp = (const short*)a.v + (long)row0 * a.vst + (long)h * E + e0;
-  auto issue = [&](int J, char* buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int p = 0; p < KEYS / 4096; ++p) {
-      const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(kp + min(64 * J + r, nrow - 1) * a.kst + s * 8),
-          (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16, 0, 0);
-    }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int r = (p * 256 + tid) >> 3, s = (tid & 7) ^ value_turn<8>(r);
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(vp + min(64 * J + r, nrow - 1) * a.vst + s * 8),
-          (lds_ptr)(buf + KEYS + (p * 256 + wid * 64) * 16), 16, 0, 0);
-    }
-  };
-  const int J1 = min(half * 2 + 1, (nrow - 1) / 64);
-  if (carried) issue_state(0, b0);
-  else issue(J1, b0);
-
   frag_u qf[NC];
   const short* q = (const short*)a.q + (row0 + min(t, nrow - 1)) * a.qst + hk * DP;
 #pragma unroll
   for (int c = 0; c < NC; ++c) qf[c].u4 = *(const uint4v*)(q + c * 16 + hi * 8);
-  float tot[4], before = 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    tot[j] = x.tot[ci * 4 + j];
-    if (j < jt) before += tot[j];
-  }
   const long ho = (long)h * x.T + row0;
   const float bt = x.b[ho + min(t, nrow - 1)];
-  {
-    float c = -INFINITY, s = 0.f;
-    if (tid < nrow) {
-      c = -x.b[ho + tid];
-      s = x.i[ho + tid];
+  const float b_tok = x.b[ho + min(tid, nrow - 1)];
+  const float i_tok = x.i[ho + min(tid, nrow - 1)];
+  const f32x4 tot = *(const f32x4*)(x.tot + ci * 4);
+  const float skip = bits2f(((const short*)a.skip)[h]);
+  // the loads below are counted, these are not
+  auto in_order = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+  };
+  in_order();
+
+  // Thread tid fills 16-byte places tid, tid + 256, ... of a tile.  Buffer loads:
+  // behind other loads into LDS the compiler waits for all of them where it needs
+  // a value.  Tiles 4 - NS to 3: the state, then keys and values.
+  auto turn = [](int r) { return SL == 16 ? row_turn(r) : key_turn<SL>(r); };
+  const auto state_src = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(x.P + ci * 3 * E * DP + (x.U ? e0 : 3 * e0) * DP), 0, 0x7fffffff,
+      0x00027000);
+  const auto key_src = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const short*)a.k + (long)row0 * a.kst + hk * DP), 0, 0x7fffffff,
+      0x00027000);
+  const auto value_src = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const short*)a.v + (long)row0 * a.vst + (long)h * E + e0), 0,
+      0x7fffffff, 0x00027000);
+  const int kst = (int)a.kst * 2, vst = (int)a.vst * 2;
+  auto issue = [&](int i, char* buf) __attribute__((always_inline)) {
+    in_order();
+    if (i < 4) {
+#pragma unroll
+      for (int p = 0; p < LS; ++p) {
+        // fragments, or from rows of planes
+        const int f = 12 * (i - (4 - NS)) + 4 * p + wid;
+        const int row = f % (3 * NC) / NC * E + f / (3 * NC) * 32 + col;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            state_src, (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16,
+            x.U ? row * DP * 2 + f % NC * 32 + hi * 16 : f * 1024 + lane * 16, 0,
+            0, 0);
+      }
+    } else {
+      const int s0 = (i - 4) * 32;
+#pragma unroll
+      for (int p = 0; p < LK; ++p) {
+        const int r = (p * 256 + tid) / SL, s = tid % SL ^ turn(r);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            key_src, (lds_ptr)(buf + (p * 256 + wid * 64) * 16), 16,
+            min(s0 + r, nrow - 1) * kst + s * 16, 0, 0, 0);
+      }
+      const int r = tid >> 3, s = (tid & 7) ^ value_turn<8>(r);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          value_src, (lds_ptr)(buf + KEYS + wid * 1024), 16,
+          min(s0 + r, nrow - 1) * vst + s * 16, 0, 0, 0);
     }
+    in_order();
+  };
+  // A tile is here, in all waves, and the one before is read; `behind` words of this
+  // thread were asked for after it.  Full halves have 4 or 8 tiles of keys; others
+  // too, with their last row for those that they do not have.
+  auto arrive = [&](int behind) __attribute__((always_inline)) {
+    in_order();
+    // a constant, but the builtin wants a literal
+    if (behind == 6) __builtin_amdgcn_s_waitcnt(0x76);
+    else if (behind == 5) __builtin_amdgcn_s_waitcnt(0x75);
+    else if (behind == 7) __builtin_amdgcn_s_waitcnt(0x77);
+    else __builtin_amdgcn_s_waitcnt(0x74);   // 4 is right for all: no less
+    __builtin_amdgcn_s_barrier();
+    in_order();
+  };
+  char *const ring[4] = {b0, b1, b2, b3};
+  float inter;
+  auto weights = [&]() __attribute__((always_inline)) {
+    float before = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < jt) before += tot[j];
+    const float c = tid < nrow ? -b_tok : -INFINITY;
+    const float s = tid < nrow ? i_tok : 0.f;
     s_col[tid] = c;
     s_step[tid] = s;
     s_far[tid] = __expf(tot[0] * (wid == 0) + tot[1] * (wid == 1) +
                         tot[2] * (wid == 2) + tot[3] * (wid == 3) + c) * s;
-  }
-  const float inter = __expf(bt + before);
+    inter = __expf(bt + before);
+  };
 
   // this lane's part of the addresses: slot 2 c + hi of row col; a transposing
   // read, where 16 lanes turn 4 keys by 16 columns
@@ -1225,104 +1511,110 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   const int vx = (tr_key * 64 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4 +
                   value_turn<8>(tr_key) * 8) * 2;
   f32x16 ot[2] = {};
-  auto state = [&](int nb, const char* buf) __attribute__((always_inline)) {
+  // part y of the state: fragments c of plane z of 32 columns nb, c fastest
+  auto state = [&](int y, const char* buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int z = 0; z < 3; ++z)
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        frag_u sf;
-        sf.u4 = *(const uint4v*)(buf + z * 32 * KP + (kx ^ (32 * c)));
-        ot[nb] = mfma_bf16(sf.bf, qf[c].bf, ot[nb]);
-      }
-    ot[nb] *= inter;
+    for (int f = 0; f < 12; ++f) {
+      const int at = 12 * y + f, nb = at / (3 * NC), c = at % NC;
+      frag_u sf;
+      sf.u4 = *(const uint4v*)(buf + f * 1024 + lane * 16);
+      ot[nb] = mfma_bf16(sf.bf, qf[c].bf, ot[nb]);
+    }
   };
   const bool rows = half * 128 + wid * 32 < nrow;
-  auto keys = [&](int J, const char* buf) __attribute__((always_inline)) {
-    if (J > jt || !rows) return;         // wave-uniform
-    float from = bt;                     // from the end of the group
+  auto keys = [&](int i, const char* buf) __attribute__((always_inline)) {
+    if (i > tt || !rows) return;         // later keys; wave-uniform
+    const int J = i >> 1, s0 = i * 32;
+    f32x16 acc = {};
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j > J && j < jt) from += tot[j];
-    from = __expf(from);
+    for (int c = 0; c < NC; ++c) {
+      frag_u kf;
+      kf.u4 = *(const uint4v*)(buf + (kx ^ (32 * c)));
+      acc = mfma_bf16(kf.bf, qf[c].bf, acc);
+    }
+    if (J < jt) {
+      float from = bt;                   // from the end of the group
 #pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
-      if (2 * J + k2 > tt) break;        // later keys
-      f32x16 acc = {};
+      for (int j = 0; j < 4; ++j)
+        if (j > J && j < jt) from += tot[j];
+      from = __expf(from);
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        frag_u kf;
-        kf.u4 = *(const uint4v*)(buf + k2 * 32 * KP + (kx ^ (32 * c)));
-        acc = mfma_bf16(kf.bf, qf[c].bf, acc);
+      for (int r = 0; r < 16; ++r)
+        acc[r] *= s_far[s0 + acc_row(r, hi)] * from;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int s = s0 + acc_row(r, hi);
+        const float w = __expf(bt + s_col[s]) * s_step[s];
+        acc[r] *= s > t ? 0.f : w;
+        acc[r] += s == t ? skip : 0.f;
       }
-      const int s0 = 64 * J + 32 * k2;
-      if (J < jt) {
+    }
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[r] *= s_far[s0 + acc_row(r, hi)] * from;
-      } else {
+    for (int cc = 0; cc < 2; ++cc) {
+      frag_u pf[3];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int s = s0 + acc_row(r, hi);
-          const float w = __expf(bt + s_col[s]) * s_step[s];
-          acc[r] *= s > t ? 0.f : w;
-        }
+      for (int u = 0; u < 4; ++u) {
+        uint w[3];
+        split3(acc[8 * cc + 2 * u], acc[8 * cc + 2 * u + 1], w);
+#pragma unroll
+        for (int z = 0; z < 3; ++z) pf[z].u[u] = w[z];
       }
 #pragma unroll
-      for (int cc = 0; cc < 2; ++cc) {
-        frag_u pf[3];
+      for (int nb = 0; nb < 2; ++nb) {
+        union { tr4 t[2]; bf16x8 bf; } vf;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          uint w[3];
-          split3(acc[8 * cc + 2 * u], acc[8 * cc + 2 * u + 1], w);
+        for (int u = 0; u < 2; ++u)
+          vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_tr4)(buf + KEYS + (vx ^ (nb * 64)) + (16 * cc + 8 * u) * 128));
 #pragma unroll
-          for (int z = 0; z < 3; ++z) pf[z].u[u] = w[z];
-        }
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          union { tr4 t[2]; bf16x8 bf; } vf;
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            vf.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_tr4)(buf + KEYS + (vx ^ (nb * 64)) +
-                          (32 * k2 + 16 * cc + 8 * u) * 128));
-#pragma unroll
-          for (int z = 0; z < 3; ++z) ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
-        }
+        for (int z = 0; z < 3; ++z) ot[nb] = mfma_bf16(vf.bf, pf[z].bf, ot[nb]);
       }
     }
   };
+  // (weights in both branches, where the compiler knows what was asked for)
   if (carried) {
-    __syncthreads();                     // also waits for the words on their way
-    issue_state(1, b1);
-    state(0, b0);
-    __syncthreads();
-    issue(J1, b0);
-    state(1, b1);
+#pragma unroll
+    for (int i = 4 - NS; i < 7 - NS; ++i) issue(i, ring[i % 4]);
+    weights();
+#pragma unroll
+    for (int i = 4 - NS; i < 4; ++i) {
+      arrive((i + 1 < 4 ? LS : LT) + (i + 2 < 4 ? LS : LT));
+      issue(i + 3, ring[(i + 3) % 4]);
+      state(i - (4 - NS), ring[i % 4]);
+    }
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) ot[nb] *= inter;
+  } else {
+#pragma unroll
+    for (int i = 4; i < 7; ++i) issue(i, ring[i % 4]);
+    weights();
   }
-  for (int J = J1;; J -= 2) {            // from the newest keys back
-    __syncthreads();
-    if (J > 0) issue(J - 1, b1);
-    keys(J, b0);
-    if (J == 0) break;
-    __syncthreads();
-    if (J > 1) issue(J - 2, b0);
-    keys(J - 1, b1);
-    if (J == 1) break;
-  }
-
   // through LDS, so that every row is read and written as a whole (8 bytes a
   // lane, each of another row: 163 us in place of 121)
-  float* o = (float*)(wid < 2 ? b0 : b1) + (wid & 1) * 32 * OP;
-  const float skip = bits2f(((const short*)a.skip)[h]);
   const int r0 = half * 128 + wid * 32 + (lane >> 3), c0 = (lane & 7) * 8;
   const long at = (long)h * E + e0 + c0;
-  uint4v vv[4], zz[4];
+  uint4v zz[4];
+  if (half)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      arrive(LT + LT);
+      issue(i + 7, ring[(i + 3) % 4]);
+      keys(i, ring[i]);
+    }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const long r = row0 + min(r0 + 8 * i, nrow - 1);
-    vv[i] = *(const uint4v*)((const short*)a.v + r * a.vst + at);
-    zz[i] = *(const uint4v*)((const short*)a.z + r * a.zst + at);
+    arrive(i < 2 ? LT + LT : i == 2 ? LT + 4 : 4);
+    if (i == 0) issue(half * 4 + 7, b3);
+    if (i == 1)
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+        zz[y] = *(const uint4v*)((const short*)a.z +
+                                 (row0 + min(r0 + 8 * y, nrow - 1)) * a.zst + at);
+    keys(half * 4 + i, ring[i]);
   }
+
+  float* o = (float*)(wid == 0 ? b0 : wid == 1 ? b1 : wid == 2 ? b2 : b3);
   __syncthreads();
 #pragma unroll
   for (int nb = 0; nb < 2; ++nb)
@@ -1337,16 +1629,15 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   for (int i = 0; i < 4; ++i) {
     if (r0 + 8 * i >= nrow) break;
     const float* src = o + ((lane >> 3) + 8 * i) * OP + c0;
-    float y[8], v[8], z[8];
+    float y[8], z[8];
     load4(src, y);
     load4(src + 4, y + 4);
-    unpack8(vv[i], v);
     unpack8(zz[i], z);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = (y[j] + skip * v[j]) * silu_f(z[j]);
     uint4v w;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(y[2 * j], y[2 * j + 1]);
+    for (int j = 0; j < 4; ++j)
+      w[j] = pack_bf16x2(y[2 * j] * silu_f(z[2 * j]),
+                         y[2 * j + 1] * silu_f(z[2 * j + 1]));
     *(uint4v*)((short*)a.out + (long)(row0 + r0 + 8 * i) * a.H * E + at) = w;
   }
 }
@@ -1364,15 +1655,24 @@ static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
     if (a.rot % 16 == 0) memory_turn_kernel<true><<<rows, 256, lds, stream>>>(x);
     else memory_turn_kernel<false><<<rows, 256, lds, stream>>>(x);
   }
+  if constexpr (GATE == TIMED && DP <= 128)
+    if (!x.VT) {
+      if (x.U) {
+        memory_states_kernel<DP, GATE><<<ch * (a.E / 64), 256, 0, stream>>>(x);
+        memory_scan_kernel<GATE><<<(long)x.n_seg * a.H * (DP / 64) * (a.E / 16),
+                                   256, 0, stream>>>(x);
+      } else {
+        const int units = a.H * (a.E * DP / 4096);
+        memory_carry_kernel<DP>
+            <<<(long)x.n_seg * 8 * ((units + 7) / 8), 256, 0, stream>>>(x);
+      }
+      memory_timed_kernel<DP><<<ch * 2 * (a.E / 64), 256, 0, stream>>>(x);
+      return;
+    }
   memory_states_kernel<DP, GATE>
       <<<ch * ((a.E + 63) / 64), 256, 0, stream>>>(x);
   memory_scan_kernel<GATE><<<(long)x.n_seg * a.H * ((a.D + 63) / 64) *
                                  ((a.E + 15) / 16), 256, 0, stream>>>(x);
-  if constexpr (GATE == TIMED && DP <= 128)
-    if (!x.VT) {
-      memory_timed_kernel<DP><<<ch * 2 * (a.E / 64), 256, 0, stream>>>(x);
-      return;
-    }
   if (a.E <= 64 || DP > 128)
     memory_outputs_kernel<DP, 64, GATE>
         <<<ch * 2 * ((a.E + 63) / 64), 256, 0, stream>>>(x);
@@ -1392,6 +1692,9 @@ extern "C" int sv_memory_chunks(const ChunkArgs* x, int gating,
   if (!x->VT && (gating != TIMED || x->a.E % 64 ||
                  (x->a.D != 64 && x->a.D != 128)))
     return 1;
+  if (!x->U && x->VT) return 1;
+  // offsets of a chunk's rows are of 32 bits
+  if (!x->VT && (x->a.kst >= 1 << 22 || x->a.vst >= 1 << 22)) return 1;
 #define MC(P)                                                     \
   do {                                                            \
     if (gating == GATED) launch_chunks<P, GATED>(*x, stream);     \

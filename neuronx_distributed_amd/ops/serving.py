@@ -1017,6 +1017,18 @@ def chunk_table(segments):
     return rows, first
 
 
+def memory_carries(chunks: int, segments: int, state: int) -> bool:
+    """Are the states of a timed memory (``state`` elements a segment) carried
+    from chunk to chunk, not made for all chunks at once and scanned?  A chunk
+    of the longest segment takes a workgroup 4 us; at once, 4096 elements of a
+    chunk's state take 0.018 us of the device, and two launches more.  The
+    longest segment is at most as long as all but one chunk a segment.
+    Whole calls, at once and carried: 2 x 2048 tokens, 128 heads of 128 x 64
+    222 and 184 us; 1000 tokens of 64 heads 46 and 46; 16384 tokens of 64 heads
+    419 and 424, of 16 heads of 64 x 64 105 and 286."""
+    return chunks - segments + 1 <= chunks * (state // 4096) / 217 + 2
+
+
 def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
                chunks: Optional[torch.Tensor] = None,
                chunk_first: Optional[torch.Tensor] = None,
@@ -1098,10 +1110,13 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         nc = chunks.shape[0]
         assert chunk_first.shape[0] == seg.shape[0] + 1
         f32 = dict(dtype=torch.float32, device=q.device)
-        U = torch.empty(nc, heads, E, D, **f32)
+        tiled = timed and D in (64, 128) and E % 64 == 0 and \
+            max(t.stride(0) for t in strided) < 1 << 22
+        U = None if tiled and memory_carries(nc, seg.shape[0], heads * D * E) \
+            else torch.empty(nc, heads, E, D, **f32)
         P = torch.empty(nc, heads, 3, E, D, dtype=torch.bfloat16,
                         device=q.device)
-        VT = None if timed and D in (64, 128) and E % 64 == 0 else \
+        VT = None if tiled else \
             torch.empty(nc, heads, E, CHUNK, dtype=torch.bfloat16,
                         device=q.device)
         KA = torch.empty(T, heads * D, dtype=q.dtype, device=q.device) \

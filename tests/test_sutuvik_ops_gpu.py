@@ -517,6 +517,42 @@ def test_timed_memory_in_batches(dtype):
         _near(S[s], w[1], F32, s, 2e-5 if dtype == BF16 else 2e-6)
 
 
+@pytest.mark.parametrize("carried", [True, False])
+@pytest.mark.parametrize("N,P", [(64, 64), (128, 64), (64, 192), (128, 128)])
+def test_timed_memory_states_carried_and_scanned(monkeypatch, N, P, carried):
+    """Portions that end at, before and behind pieces of 64 and chunks of 256
+    tokens, whose states are carried or made at once, then portions behind
+    them."""
+    monkeypatch.setattr(sv, "memory_carries", lambda *a: carried)
+    H, G = 6, 2
+    lens, more = [1, 63, 64, 130, 256, 257, 800, 1025], [70, 1, 300, 64, 2, 511,
+                                                         256, 33]
+    cases = [_ssm(a + b, H, G, N, P, 30 * i, BF16)
+             for i, (a, b) in enumerate(zip(lens, more))]
+    params = _ssm_params(H, BF16)
+    S = torch.full((8, H, N, P), 7.0, device="cuda")
+    got = []
+    for at, n in (([0] * 8, lens), (lens, more)):
+        x, B, C, z, raw = (torch.cat(t).cuda() for t in zip(*(
+            [t[a:a + k] for t in c] for c, a, k in zip(cases, at, n))))
+        seg, chunks, first = _segments([(7 - i, k, a) for i, (a, k) in
+                                        enumerate(zip(at, n))])
+        got.append(sv.memory_mix(
+            C, B, x, sv.TimeGate(raw, *[t.cuda() for t in params], z), S, None,
+            None, seg, H, chunks, first).split(n))
+    for i, c in enumerate(cases):
+        want, S_want = _ssm_want(c, params, H, G, N, P)
+        _near(torch.cat([g[i] for g in got]), want, BF16, i)
+        _near(S[7 - i], S_want, F32, i, 2e-5)
+
+
+def test_states_are_carried_where_that_is_faster():
+    assert sv.memory_carries(17, 2, 128 * 128 * 64)      # 2 x 2048 tokens
+    assert sv.memory_carries(4, 1, 64 * 128 * 64)        # 1000 tokens
+    assert not sv.memory_carries(64, 1, 64 * 128 * 64)   # 16384 tokens
+    assert not sv.memory_carries(64, 1, 16 * 64 * 64)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_an_old_input_is_still_in_the_state(dtype):
     """Decays near one: an input 2000 tokens back decides the output."""
