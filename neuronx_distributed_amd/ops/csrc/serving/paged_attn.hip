@@ -842,9 +842,12 @@ extern "C" int sv_attn_rows(const RowsArgs* a, int vec, int f32,
 // PFLOP/s (a large matrix product: 1.3 to 1.5).  6000 tokens of three portions
 // behind up to 4096, 32/8 heads: 621 -> 585 us with the next tile's scores
 // beside this tile's exponentials, page numbers read two tiles ahead, keys
-// rotated over all banks, and a maximum that lags; 577 with the order of the
-// planes below.  An explicit order of products and vector work took 630, splits
-// by v_dot2c_f32_bf16 616.
+// rotated over all banks, and a maximum that lags; 568 with the order of the
+// planes below, 556 with keys read ahead of their products, page numbers that
+// nobody waits for and no branch a word on its way into LDS (latent attention of 2
+// x 2048 tokens 355 -> 345, of 3 x 230 with 16 heads 196 -> 168).  An explicit order
+// of products and vector work took 630, scores in one block with the weights of the
+// tile before them spill 300 registers, splits by v_dot2c_f32_bf16 616.
 // ---------------------------------------------------------------------------
 //
 // A key may end in columns that all heads share (kr): the rotated part of
@@ -934,33 +937,53 @@ attn_tiles_kernel(TilesArgs a) {
   // 32-bit within a page
   const int krow = (int)a.krow, vrow = (int)a.vrow, rrow = (int)a.rrow;
   auto tile_of = [&](int n) { return n < nk ? n : t_lo + n - nk; };
+  // A page number is a vector load, which the compiler waits for, with all words on
+  // their way into LDS, as soon as it has it: `settle` keeps that behind a barrier
+  // that waits for them anyway.
   auto page_of = [&](int n) { return bt[tile_of(min(n, ntiles - 1))]; };
+  auto settle = [](int page) {
+    asm volatile("" : "+v"(page));
+    return __builtin_amdgcn_readfirstlane(page);
+  };
   // Ask for the rows of a page: a wave's 64 slots of 16 bytes follow each
   // other in LDS, so the rotation of a row's slots is done on the source.
+  // Rows that fill the tile need no branch a word.
   auto issue_k = [&](long page, char* kd) {
     const short* kb = a.kc + page * a.kpage + g * a.khead;
     const short* rb = SHARED ? a.kr + page * SV_PAGE * rrow - a.DS : nullptr;
-#pragma unroll
-    for (int p = 0; p < CK / 4; ++p) {
+    auto word = [&](int p, bool all) __attribute__((always_inline)) {
       const int it = p * 256 + tid, r = it / CK;
       const int c = (it % CK ^ key_turn<CK>(r)) * 8;
-      if (c >= D) continue;
+      if (!all && c >= D) return;
       __builtin_amdgcn_global_load_lds(
           (global_ptr)(SHARED && c >= a.DS ? rb + (r * rrow + c)
                                            : kb + (r * krow + c)),
           (lds_ptr)(kd + (p * 256 + wid * 64) * 16), 16, 0, 0);
+    };
+    if (D == DK) {
+#pragma unroll
+      for (int p = 0; p < CK / 4; ++p) word(p, true);
+    } else {
+#pragma unroll
+      for (int p = 0; p < CK / 4; ++p) word(p, false);
     }
   };
   auto issue_v = [&](long page, char* vd) {
     const short* vb = a.vc + page * a.vpage + g * a.vhead;
-#pragma unroll
-    for (int p = 0; p < CV / 4; ++p) {
+    auto word = [&](int p, bool all) __attribute__((always_inline)) {
       const int it = p * 256 + tid, r = it / CV;
       const int c = (it % CV ^ value_turn<CV>(r)) * 8;
-      if (c >= E) continue;
+      if (!all && c >= E) return;
       __builtin_amdgcn_global_load_lds(
           (global_ptr)(vb + (r * vrow + c)),
           (lds_ptr)(vd + (p * 256 + wid * 64) * 16), 16, 0, 0);
+    };
+    if (E == DE) {
+#pragma unroll
+      for (int p = 0; p < CV / 4; ++p) word(p, true);
+    } else {
+#pragma unroll
+      for (int p = 0; p < CV / 4; ++p) word(p, false);
     }
   };
   // this lane's part of the addresses in a tile (bytes): slot 2 c + hi of key
@@ -973,19 +996,29 @@ attn_tiles_kernel(TilesArgs a) {
   const int vx = (tr_key * DE + ((lane >> 4) & 1) * 16 + (lane & 3) * 4 +
                   value_turn<CV>(tr_key) * 8) * 2;
 
-  // S^T = K Q^T
+  // S^T = K Q^T, the keys of two products AHEAD of them
   auto scores = [&](f32x16* s, const char* kbuf) __attribute__((always_inline)) {
+    constexpr int AHEAD = 2;
+    frag_u kf[AHEAD + 1][2];
+    auto read = [&](int c) __attribute__((always_inline)) {
+      constexpr int M = KeySlots<CK>::steps;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        kf[c % (AHEAD + 1)][kb].u4 = *(const uint4v*)(
+            kbuf + kx[c % M] + (c / M) * M * 32 + kb * 32 * KP);
+    };
     s[0] = s[1] = f32x16{};
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < AHEAD; ++c) read(c);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        constexpr int M = KeySlots<CK>::steps;
-        frag_u kf;
-        kf.u4 = *(const uint4v*)(kbuf + kx[c % M] + (c / M) * M * 32 +
-                                 kb * 32 * KP);
-        s[kb] = mfma_bf16(kf.bf, qf[c].bf, s[kb]);
-      }
+    for (int c = 0; c < NC; ++c) {
+      if (c + AHEAD < NC) read(c + AHEAD);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        s[kb] = mfma_bf16(kf[c % (AHEAD + 1)][kb].bf, qf[c].bf, s[kb]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
   // scores of tile n as they enter the softmax, and the running maximum
   auto level = [&](int n, f32x16* s) __attribute__((always_inline)) {
@@ -1121,19 +1154,19 @@ attn_tiles_kernel(TilesArgs a) {
   __syncthreads();
   for (int n = 0; n < ntiles; n += 2) {
     // keys of n + 1 and values of n are there; pb, pc: pages of n + 1, n + 2
-    const int pd = page_of(n + 3);
+    const int vd = page_of(n + 3);
     if (n + 2 < ntiles) issue_k(pc, k0);
     if (n + 1 < ntiles) issue_v(pb, v1);
     step(n, sa, sb, k1, v0);
     __syncthreads();
     if (n + 1 >= ntiles) break;
-    const int pe = page_of(n + 4);
-    if (n + 3 < ntiles) issue_k(pd, k1);
+    pb = settle(vd);
+    const int ve = page_of(n + 4);
+    if (n + 3 < ntiles) issue_k(pb, k1);
     if (n + 2 < ntiles) issue_v(pc, v0);
     step(n + 1, sb, sa, k0, v1);
     __syncthreads();
-    pb = pd;
-    pc = pe;
+    pc = settle(ve);
   }
 
   l_run += __shfl_xor(l_run, 32, 64);
