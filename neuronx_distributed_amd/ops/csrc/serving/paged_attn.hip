@@ -533,13 +533,21 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   const int n1 = min(total, (split + 1) * per);
   auto tile_of = [&](int n) { return n < nk ? n : t_lo + n - nk; };
 
+  // The page of a tile, asked for a turn before: a vector load, which the compiler
+  // would wait for as soon as it has it.
+  auto page_of = [&](int n) { return bt[tile_of(min(n, n1 - 1)) / 2]; };
+  auto settle = [](int page) {
+    asm volatile("" : "+v"(page));
+    return __builtin_amdgcn_readfirstlane(page);
+  };
   // Ask for a tile.  Keys past the newest read its row again, and the row's own
   // key and value come from the projection, also where they are not written
   // yet.
-  auto issue = [&](int n, frag_u (*kf)[NC], char* vd) __attribute__((always_inline)) {
+  auto issue = [&](int n, int page, frag_u (*kf)[NC], char* vd)
+      __attribute__((always_inline)) {
     const int t = tile_of(n);
     const int newest = i_pos - t * 32;   // row of the tile
-    const long base = ((long)bt[t / 2] * a.G + g) * SV_PAGE + (t & 1) * 32;
+    const long base = ((long)settle(page) * a.G + g) * SV_PAGE + (t & 1) * 32;
     const short* kb = (const short*)a.kc + base * a.kcs;
     const short* vb = (const short*)a.vc + base * a.vcs;
 #pragma unroll
@@ -640,19 +648,32 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
       for (int z = 0; z < 3; ++z) o[b] = mfma16(vf.bf, pf[z].bf, o[b]);
     }
   };
-  // all words that this wave has asked for are there, and its reads are done
-  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); };
+  // All words that this wave has asked for are there, and its reads are done.  The
+  // compiler has to know: behind a wait in asm it waits for the next tile's words
+  // before it multiplies this one's keys.
+  auto arrived = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x70);              // vmcnt(0) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  };
 
   frag_u ka[2][NC], kb[2][NC];
   int n = split * per + wid;
-  if (n < n1) issue(n, ka, v0);
+  int page = 0;
+  if (n < n1) {
+    const int first = page_of(n);
+    page = page_of(n + 4);
+    issue(n, first, ka, v0);
+  }
   for (; n < n1; n += 8) {
     arrived();
-    if (n + 4 < n1) issue(n + 4, kb, v1);
+    if (n + 4 < n1) issue(n + 4, page, kb, v1);
+    page = page_of(n + 8);
     attend(n, ka, v0);
     if (n + 4 >= n1) break;
     arrived();
-    if (n + 8 < n1) issue(n + 8, ka, v0);
+    if (n + 8 < n1) issue(n + 8, page, ka, v0);
+    page = page_of(n + 12);
     attend(n + 4, kb, v1);
   }
 

@@ -7,6 +7,7 @@ library raises.  Activations and weights are bfloat16, or float32 in the
 gates and recurrent state are 32-bit in both.
 """
 
+import bisect
 import ctypes
 import math
 import os
@@ -807,6 +808,24 @@ def _row_splits(target: int, units: int, max_keys: int, per: int) -> int:
     return max(1, min(target // max(1, units), -(-max_keys // per), 64))
 
 
+# Workgroups of the first form of ``rows_kernel`` to aim at, where up to so many
+# (row, key head) meet keys up to 256, 700, 1200, 2500, 5000 and more; 0 shares no
+# row.  One a CU (256) or less while rows are short: more meet on one CU and read
+# no faster.  Longer rows fill all 512 places, and of many rows there are several
+# rounds, so that unequal ones end together.  Over 740 sizes of 1 to 128 rows of
+# 32/32, 32/8 and 28/4 heads of 128, up to 12000 keys, equal and unequal, 1.8% over
+# the best number, where 1024 to 2048 above 700 keys were 8.6% (us then and now: 8
+# rows of 32/8 heads, 4000 keys 26.4, 21.3; 32, 1000: 26.6, 18.8; 64, 2000: 54.0,
+# 52.8; 128 rows of 28/4, 1000: 37.5, 28.4), up to 5% over it in 5 of them (45 rows of
+# 32/8, 2000 equal keys: 75.8, 77.7).
+_SHARED_KEYS = (256, 700, 1200, 2500, 5000)
+_SHARED_ROWS = ((64, (0, 256, 256, 256, 512, 512)),
+                (128, (0, 512, 512, 512, 512, 768)),
+                (255, (0, 0, 0, 512, 1024, 1536)),
+                (512, (0, 0, 0, 640, 2048, 2048)),
+                (math.inf, (0, 0, 0, 1024, 2048, 2048)))
+
+
 def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
                 modified: bool = False):
     """Form (2 on matrix cores, 1 on vectors) and workgroups a row of
@@ -816,11 +835,11 @@ def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
     contexts the second is the faster one (64 rows of 32/32 heads of 128, 64
     keys: 18 and 12 us, 200: 26 and 23; 128 of 32/16, 64: 18.5 and 16.6; 128 of
     32/32 of 64, 20: 14.2 and 12.6; 32 of 32/32 with modified scores, 100: 12.4
-    and 11.5).  Sharing a row costs a merge, 5 us and more, which up to 700 keys
-    pays only while CUs have no workgroup (32 rows of 32/32 heads, 300 keys: 25,
-    in two 31; 8 of 32/32, 600 keys: 15.5, in five 20).  Over 2300 sizes 0.65 of
-    the second form's time; up to 8% over it are left with modified scores of
-    heads to themselves (96 rows of 16/16 of 64, 300 keys: 16.6 and 15.8)."""
+    and 11.5).  Over 2300 sizes 0.65 of the second form's time; up to 8% over it
+    are left with modified scores of heads to themselves (96 rows of 16/16 of 64,
+    300 keys: 16.6 and 15.8).
+
+    Sharing a row costs a merge, and partial results: ``_SHARED_ROWS``."""
     units, rep = rows * groups, heads // groups
     if D == 64:
         short = 64 if rep == 1 and units > (1024 if modified else 2048) else 0
@@ -831,8 +850,8 @@ def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
             100 if units > (1024 if modified else 2048) else 64
     if units > 512 and 0 < max_keys <= short:
         return 1, _row_splits(1024, units, max_keys, 128)
-    target = 2048 if max_keys > 700 or units <= 32 else \
-        512 if units <= 128 else 256
+    target = next(t for most, t in _SHARED_ROWS if units <= most)
+    target = target[bisect.bisect_left(_SHARED_KEYS, max_keys)]
     return 2, _row_splits(target, units, max_keys, 128)
 
 

@@ -85,6 +85,17 @@ def test_kernel_of_single_rows(rows, heads, groups, D, keys, modified, want):
     assert sv.rows_kernel(rows, heads, groups, D, keys, modified) == want
 
 
+@pytest.mark.parametrize("rows,groups,keys,want", [
+    # each line of the table, and past it
+    (8, 8, 256, 1), (8, 8, 257, 3), (8, 8, 2500, 4), (8, 8, 2501, 8),
+    (9, 8, 700, 6), (16, 8, 2501, 4), (16, 8, 5001, 6), (17, 8, 700, 1),
+    (17, 8, 701, 1), (17, 8, 1201, 3), (17, 8, 2501, 7), (32, 8, 1200, 1),
+    (32, 8, 1201, 2), (32, 8, 2501, 8), (65, 8, 1200, 1), (65, 8, 1201, 1),
+    (65, 8, 2501, 3), (512, 8, 9000, 1), (1, 8, 100000, 64)])
+def test_workgroups_that_share_a_row(rows, groups, keys, want):
+    assert sv.rows_kernel(rows, 4 * groups, groups, 128, keys) == (2, want)
+
+
 @pytest.mark.parametrize("rows,width,ff,want", [
     # streaming, to the line of each size and past it
     (1, 2048, 1408, 1), (23, 2048, 1408, 1), (24, 2048, 1408, 4),
