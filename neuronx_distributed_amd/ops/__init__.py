@@ -442,9 +442,10 @@ def flash_attn_available() -> bool:
 def _fa_ok_layout(t) -> bool:
     """The flash kernels take any (batch, head, seq) strides with a DENSE
     last dim — transpose views of BSHD activations go in with no copy.  Rows
-    are moved in 16-byte words, so the strides are whole numbers of them."""
+    are moved in 16-byte words, so the strides are whole numbers of them; 31
+    rows are less than 2 GB."""
     b, h, s, d = t.stride()
-    if d != 1:
+    if d != 1 or s >= 1 << 25:
         return False
     return not (b | h | s) & 7 or not any(
         st & 7 for st, n in zip((b, h, s), t.shape) if n > 1)

@@ -107,26 +107,23 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FwdArgs a) {
   // as rows, values by transposing reads.  Both rotations repeat after 16
   // rows, so the rows st_r + 16 i of a thread have the same.
   const int st_r = tid >> 4, st_s = tid & 15;
-  const short* kg = a.k + b * a.k_bs + hkv * a.k_hs + (long)st_r * a.k_ss +
-                    (st_s ^ row_turn(st_r)) * 8;
-  const short* vg = a.v + b * a.v_bs + hkv * a.v_hs + (long)st_r * a.v_ss +
-                    (st_s ^ row_turn(st_r)) * 8;
+  const int st_c = (st_s ^ row_turn(st_r)) * 16;
+  const short* kg = a.k + b * a.k_bs + hkv * a.k_hs;
+  const short* vg = a.v + b * a.v_bs + hkv * a.v_hs;
   auto issue = [&](const short* g, long ss, int t, char* lds) {
     const int kv0 = t * FA_KV;
-    const short* src = g + kv0 * ss;
-    const long step = 16 * ss;
+    const int pitch = (int)ss * 2;
     if (kv0 + FA_KV <= S) {
+      const int off = st_r * pitch + st_c;
 #pragma unroll
-      for (int i = 0; i < 4; ++i, src += step)
-        __builtin_amdgcn_global_load_lds(
-            (global_ptr)src, (lds_ptr)(lds + (i * 256 + wid * 64) * 16), 16, 0, 0);
+      for (int i = 0; i < 4; ++i)
+        words_to_lds(g + (kv0 + 16 * i) * ss, off, lds + (i * 256 + wid * 64) * 16);
     } else {                   // rows past the end read the last one
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const long back = max(0, kv0 + 16 * i + st_r - (S - 1));
-        __builtin_amdgcn_global_load_lds(
-            (global_ptr)(src + i * step - back * ss),
-            (lds_ptr)(lds + (i * 256 + wid * 64) * 16), 16, 0, 0);
+        const int r = min(kv0 + 16 * i, S - 1);
+        words_to_lds(g + r * ss, min(st_r, S - 1 - r) * pitch + st_c,
+                     lds + (i * 256 + wid * 64) * 16);
       }
     }
   };

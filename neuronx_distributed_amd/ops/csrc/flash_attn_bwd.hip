@@ -55,28 +55,27 @@ struct BwdArgs {
   long dk_bs, dk_hs, dk_ss, dv_bs, dv_hs, dv_ss;
 };
 
-// N rows of `g` (this thread's slot of the first row it fills) from row r0
-// on, by NT threads; rows past the last one read that again.
+// N rows of `g` from row r0 on, by NT threads; rows past the last one read that
+// again.
 template <int N, int NT>
 __device__ __forceinline__ void fill_rows(const short* g, long ss, int r0,
                                           int rows, char* lds) {
   constexpr int PASS = NT / 16;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const short* src = g + r0 * ss;
-  const long step = PASS * ss;
+  const int st_r = threadIdx.x >> 4;
+  const int st_c = ((threadIdx.x & 15) ^ row_turn(st_r)) * 16;
+  const int pitch = (int)ss * 2;
   if (r0 + N <= rows) {
+    const int off = st_r * pitch + st_c;
 #pragma unroll
-    for (int i = 0; i < N / PASS; ++i, src += step)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)src, (lds_ptr)(lds + (i * NT + wid * 64) * 16), 16, 0, 0);
+    for (int i = 0; i < N / PASS; ++i)
+      words_to_lds(g + (r0 + PASS * i) * ss, off, lds + (i * NT + wid * 64) * 16);
   } else {
 #pragma unroll
     for (int i = 0; i < N / PASS; ++i) {
-      const long back =
-          max(0, r0 + PASS * i + (int)(threadIdx.x >> 4) - (rows - 1));
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(src + i * step - back * ss),
-          (lds_ptr)(lds + (i * NT + wid * 64) * 16), 16, 0, 0);
+      const int r = min(r0 + PASS * i, rows - 1);
+      words_to_lds(g + r * ss, min(st_r, rows - 1 - r) * pitch + st_c,
+                   lds + (i * NT + wid * 64) * 16);
     }
   }
 }
@@ -147,10 +146,8 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   const int g = wid >> 1, half = wid & 1;
   const int kw0 = k0 + g * 32;           // this wave's first kv row
   const int my_k = kw0 + col;
-  const int st_r = tid >> 4;             // rows st_r + 32 i of a tile
-  const int st_c = ((tid & 15) ^ row_turn(st_r)) * 8;
-  const short* qg = a.q + b * a.q_bs + h * a.q_hs + st_r * a.q_ss + st_c;
-  const short* dg = a.dout + b * a.do_bs + h * a.do_hs + st_r * a.do_ss + st_c;
+  const short* qg = a.q + b * a.q_bs + h * a.q_hs;
+  const short* dg = a.dout + b * a.do_bs + h * a.do_hs;
   const float* lse = a.lse + ((long)b * a.Hq + h) * S;
   const float* delta = a.delta + ((long)b * a.Hq + h) * S;
 
@@ -168,13 +165,16 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
 
   // Tiles of the first q head, then of the next ones: what is asked for next
   int next = q_start;
+  // (two waves' numbers go into LDS only behind the step: where they are asked for,
+  // those two would wait for them, and all others for these two)
+  float nl = 0.f;
   auto issue = [&](char* qb, char* db) __attribute__((always_inline)) {
+    if (wid < 2) nl = (wid ? delta : lse)[min(next + lane, S - 1)];
     fill_rows<64, 512>(qg, a.q_ss, next, S, qb);
     fill_rows<64, 512>(dg, a.do_ss, next, S, db);
   };
-  auto row_numbers = [&]() __attribute__((always_inline)) {
-    const int q = min(next + (tid & 63), S - 1);
-    return tid < 64 ? lse[q] * LOG2E : tid < 128 ? delta[q] : 0.f;
+  auto leave = [&](float* ld) __attribute__((always_inline)) {
+    if (wid < 2) ld[tid] = wid ? nl : nl * LOG2E;
   };
   auto advance = [&]() __attribute__((always_inline)) {
     if ((next += 64) < q_end) return;
@@ -264,34 +264,25 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
     }
   };
 
-  fill_rows<128, 512>(a.k + b * a.k_bs + hkv * a.k_hs + st_r * a.k_ss + st_c,
-                      a.k_ss, k0, S, kb);
-  fill_rows<128, 512>(a.v + b * a.v_bs + hkv * a.v_hs + st_r * a.v_ss + st_c,
-                      a.v_ss, k0, S, vb);
+  fill_rows<128, 512>(a.k + b * a.k_bs + hkv * a.k_hs, a.k_ss, k0, S, kb);
+  fill_rows<128, 512>(a.v + b * a.v_bs + hkv * a.v_hs, a.v_ss, k0, S, vb);
   const int steps = heads * ((q_end - q_start + 63) / 64);
-  float nl = row_numbers();
   issue(q0b, d0b);
-  if (tid < 128) ld0[tid] = nl;
+  leave(ld0);
   __syncthreads();             // also waits for the words on their way
   for (int i = 0; i < steps; i += 2) {
     int q0 = next;
     advance();
-    if (i + 1 < steps) {
-      nl = row_numbers();
-      issue(q1b, d1b);
-      if (tid < 128) ld1[tid] = nl;
-    }
+    if (i + 1 < steps) issue(q1b, d1b);
     step(q0, q0b, d0b, ld0);
+    leave(ld1);
     __syncthreads();
     if (i + 1 >= steps) break;
     q0 = next;
     advance();
-    if (i + 2 < steps) {
-      nl = row_numbers();
-      issue(q0b, d0b);
-      if (tid < 128) ld0[tid] = nl;
-    }
+    if (i + 2 < steps) issue(q0b, d0b);
     step(q0, q1b, d1b, ld1);
+    leave(ld0);
     __syncthreads();
   }
 
@@ -371,9 +362,8 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
 
   f32x16 dq[4] = {};                     // [d][q]
   const int rx = row_lane(col, hi), tx = tr_lane(lane);
-  const int st_r = tid >> 4, st_c = ((tid & 15) ^ row_turn(st_r)) * 8;
-  const short* kg = a.k + b * a.k_bs + hkv * a.k_hs + st_r * a.k_ss + st_c;
-  const short* vg = a.v + b * a.v_bs + hkv * a.v_hs + st_r * a.v_ss + st_c;
+  const short* kg = a.k + b * a.k_bs + hkv * a.k_hs;
+  const short* vg = a.v + b * a.v_bs + hkv * a.v_hs;
 
   const int kv_end = a.causal ? min(S, q0 + 128) : S;
   // sliding window: this q block's earliest active kv row (tile-aligned)

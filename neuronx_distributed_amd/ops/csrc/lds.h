@@ -10,6 +10,17 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef short tr4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr4* lds_tr4;
 
+// 16 bytes a lane from `off` bytes (less than 2^31) behind a base that the wave
+// shares, to where the wave's 1 KB begins.  A buffer load: behind other loads into
+// LDS the compiler waits for everything on its way, loads and LDS reads, wherever it
+// needs a value that came from either.
+__device__ __forceinline__ void words_to_lds(const void* base, int off,
+                                             char* lds) {
+  const auto src = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0x7fffffff,
+                                                     0x00027000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)lds, 16, off, 0, 0, 0);
+}
+
 // The 16-byte slots of a key row are rotated, so that consecutive rows of one
 // column spread over the banks: all 16 of a row of 256 bytes (16 lanes are
 // served at once), else within groups of eight; those of a value row in pieces
