@@ -10,15 +10,15 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef short tr4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr4* lds_tr4;
 
-// 16 bytes a lane from `off` bytes (less than 2^31) behind a base that the wave
-// shares, to where the wave's 1 KB begins.  A buffer load: behind other loads into
+// 16 bytes a lane from `off` + `at` bytes (less than 2^31; the wave shares `at`)
+// behind a base that the wave shares, to where the wave's 1 KB begins.  A buffer load: behind other loads into
 // LDS the compiler waits for everything on its way, loads and LDS reads, wherever it
 // needs a value that came from either.
-__device__ __forceinline__ void words_to_lds(const void* base, int off,
-                                             char* lds) {
+__device__ __forceinline__ void words_to_lds(const void* base, int off, char* lds,
+                                             int at = 0) {
   const auto src = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0x7fffffff,
                                                      0x00027000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)lds, 16, off, 0, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)lds, 16, off, at, 0, 0);
 }
 
 // The 16-byte slots of a key row are rotated, so that consecutive rows of one

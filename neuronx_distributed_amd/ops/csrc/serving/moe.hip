@@ -293,6 +293,7 @@ struct MoeGemmArgs {
                             // 0:   x row = slot,       out row = pair
   int N, K, max_tiles;
   float alpha, limit, shift;  // of the gated activation
+  int rows;                 // of x
 };
 
 // min(g, limit) sigmoid(alpha g) (clamp(u, +-limit) + shift)
@@ -305,7 +306,9 @@ __device__ __forceinline__ float glu(const MoeGemmArgs& a, float g, float u) {
 // -- MFMA tiles ---------------------------------------
 // BM slots x BN weight rows, K in steps of 64 through two LDS buffers; the
 // next step's words travel while this one is multiplied: straight into LDS
-// (DMA, K a multiple of 64) or through registers.  With a gated activation
+// (DMA, K a multiple of 64; with an address a load, and all LDS reads waited for
+// behind them, 36 tiles of 28672 x 4096 and 4096 x 14336 took 2780 us, now 2640) or
+// through registers.  With a gated activation
 // the weight rows of a tile alternate 32 gate, 32 up, so a lane holds both of
 // a column.
 // slot0, rows: the tile's; tn: its columns
@@ -329,13 +332,20 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   // fills places tid, tid + NT, ... of a buffer, NT / 8 rows apart
   const int kc = ((tid ^ (tid >> 4)) & 7) * 8;
 
-  const short* px[LX];
-  const short* pw[LW];
+  // DMA: bytes behind bases that all share (buffer loads, which need no address
+  // a step and are waited for by count), less than 2^31
+  const short* px[DMA ? 1 : LX];
+  const short* pw[DMA ? 1 : LW];
+  int ox[LX], ow[LW];
+  const short* const bx =
+      (const short*)a.x + (a.top ? 0 : (long)slot0 * a.xst);
+  const short* const bw = (const short*)a.w + (long)e * (GLU ? 2 * N : N) * K;
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
-    const int r = (i * NT + tid) / 8;
-    const int s = slot0 + min(r, rows - 1);
-    px[i] = (const short*)a.x + (long)(a.top ? a.order[s] / a.top : s) * a.xst + kc;
+    const int r = min((i * NT + tid) / 8, rows - 1);
+    const int row = a.top ? a.order[slot0 + r] / a.top : r;
+    if (DMA) ox[i] = (row * (int)a.xst + kc) * 2;
+    else px[i] = bx + (long)row * a.xst + kc;
   }
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
@@ -343,7 +353,8 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
     int n = GLU ? tn * NOUT + (r >> 6) * 32 + (r & 31) : tn * NOUT + r;
     n = min(n, N - 1);
     if (GLU && (r & 32)) n += N;
-    pw[i] = (const short*)a.w + ((long)e * (GLU ? 2 * N : N) + n) * K + kc;
+    if (DMA) ow[i] = (n * K + kc) * 2;
+    else pw[i] = bw + (long)n * K + kc;
   }
 
   uint4v rx[LX], rw[LW];
@@ -351,16 +362,12 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   auto issue_x = [&](int k0, short* xs) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < LX; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(px[i] + k0), (lds_ptr)(xs + (i * NT + wid * 64) * 8), 16,
-          0, 0);
+      words_to_lds(bx, ox[i], (char*)(xs + (i * NT + wid * 64) * 8), k0 * 2);
   };
   auto issue_w = [&](int k0, short* ws) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < LW; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (global_ptr)(pw[i] + k0), (lds_ptr)(ws + (i * NT + wid * 64) * 8), 16,
-          0, 0);
+      words_to_lds(bw, ow[i], (char*)(ws + (i * NT + wid * 64) * 8), k0 * 2);
   };
   auto issue = [&](int k0, short* xs, short* ws) __attribute__((always_inline)) {
     if (DMA) {
@@ -371,9 +378,11 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
     const bool in_k = k0 + kc < K;
     const uint4v zero = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < LX; ++i) rx[i] = in_k ? *(const uint4v*)(px[i] + k0) : zero;
+    for (int i = 0; i < LX; ++i)
+      rx[i] = in_k ? *(const uint4v*)(px[DMA ? 0 : i] + k0) : zero;
 #pragma unroll
-    for (int i = 0; i < LW; ++i) rw[i] = in_k ? *(const uint4v*)(pw[i] + k0) : zero;
+    for (int i = 0; i < LW; ++i)
+      rw[i] = in_k ? *(const uint4v*)(pw[DMA ? 0 : i] + k0) : zero;
   };
   auto commit = [&](short* xs, short* ws) {
     if (DMA) return;
@@ -818,7 +827,10 @@ static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
   constexpr int NT = BM / WM * BN / WN * 64;
   constexpr bool TAIL = BM == 256;
   const long grid = (long)a.max_tiles * ((a.N + NOUT - 1) / NOUT);
-  if (a.K % 64 == 0)                     // at most 3 * 64 or 128 pieces more
+  // offsets of a tile's rows, and of an expert's weights, are bytes of 31 bits
+  const bool near = (a.top ? a.rows : 256) * a.xst < 1L << 30 &&
+                    (GLU ? 2L : 1L) * a.N * a.K < 1L << 30;
+  if (a.K % 64 == 0 && near)             // at most 3 * 64 or 128 pieces more
     moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL>
         <<<grid + (TAIL ? 192 : 0), NT, 0, stream>>>(a);
   else

@@ -201,7 +201,8 @@ class _MoeGemmArgs(ctypes.Structure):
     _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
                 + _fields("w out order tiles", ctypes.c_void_p)
                 + _fields("top N K max_tiles", ctypes.c_int)
-                + _fields("alpha limit shift", ctypes.c_float))
+                + _fields("alpha limit shift", ctypes.c_float)
+                + _fields("rows", ctypes.c_int))
 
 
 class _MemoryArgs(ctypes.Structure):
@@ -1618,7 +1619,7 @@ def moe_gemm(x: torch.Tensor, w: torch.Tensor, plan: MoePlan, gated: bool,
                      order=_p(plan.order), tiles=_p(plan.tiles),
                      top=plan.coef.shape[1] if gated else 0, N=N, K=K,
                      max_tiles=plan.tiles.shape[0], alpha=alpha, limit=limit,
-                     shift=shift)
+                     shift=shift, rows=x.shape[0])
     assert plan.how == MOE_PLAIN or (x.dtype == torch.bfloat16
                                      and _aligned((N, K), x))
     _check(library().sv_moe_gemm(ctypes.byref(a), plan.how, int(gated),

@@ -381,6 +381,21 @@ def test_plan_breaks_ties_by_index_and_takes_uneven_loads(sv):
     assert [t[:3] for t in p.tiles.cpu().tolist() if t[2]] == [[7, 0, 70]]
 
 
+@pytest.mark.parametrize("how", [3, 4, 5])
+def test_experts_of_rows_far_apart(sv, how):
+    """Rows over more than 2 GB, which 31 bits of bytes do not reach."""
+    T, E, top, W, ff, pitch = 40, 3, 2, 128, 64, 1 << 25
+    h = _rand(T, W, dtype=torch.bfloat16).cuda()
+    far = torch.empty((T - 1) * pitch + W, dtype=h.dtype,
+                      device="cuda").as_strided((T, W), (pitch, 1))
+    far.copy_(h)
+    gu = _rand(E, 2 * ff, W, dtype=h.dtype, seed=1, scale=W ** -0.5).cuda()
+    p = sv.moe_plan(_rand(T, E, dtype=torch.float32, seed=2).cuda(), None, top,
+                    how)
+    near, apart = (sv.moe_gemm(x, gu, p, True) for x in (h, far))
+    assert near.abs().max() > 0.1 and torch.equal(near, apart)
+
+
 EXPERTS = [
     # T, experts, top, width, ff, limit
     (1, 4, 2, 64, 40, 0.8),
