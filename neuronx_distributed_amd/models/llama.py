@@ -245,7 +245,28 @@ class LlamaAttention(nn.Module):
         many requests) over the paged cache."""
         from ..ops import serving as sv
 
-        q, k, v = self.qkv_proj(h)
+        return self._attend_ragged(self.qkv_proj(h), cos, sin, batch, pool)
+
+    def normed_ragged(self, x, pending, eps, weight, cos, sin, batch, pool):
+        """The new residual and ``forward_ragged`` of its normed row, for a
+        single row that the norm and the projections of are one launch; else
+        None."""
+        from ..ops import serving as sv
+
+        p = self.qkv_proj
+        if pending.delta.shape[0] != 1 or \
+                type(self).forward_ragged is not LlamaAttention.forward_ragged \
+                or type(p) is not GQAQKVColumnParallelLinear or _watched(p):
+            return None
+        w = p.weight_in_one()
+        one = None if w is None else sv.normed_linear(x, pending, eps, weight, w)
+        return one and (one[0], self._attend_ragged(p.split(one[1]), cos, sin,
+                                                    batch, pool))
+
+    def _attend_ragged(self, qkv, cos, sin, batch, pool):
+        from ..ops import serving as sv
+
+        q, k, v = qkv
         sv.rope_rows_(q, k, cos, sin, batch.pos, self.head_dim,
                       batch.max_keys)
         return self.o_proj(sv.ragged_attention(
@@ -326,6 +347,14 @@ class LlamaAttention(nn.Module):
         return self.o_proj(out)
 
 
+def _watched(module) -> bool:
+    """Does anything see, or stand for, this module's calls?"""
+    return bool("forward" in module.__dict__ or module._forward_hooks
+                or module._forward_pre_hooks
+                or nn.modules.module._global_forward_hooks
+                or nn.modules.module._global_forward_pre_hooks)
+
+
 class LlamaMLP(nn.Module):
     def __init__(self, config: LlamaConfig):
         super().__init__()
@@ -348,14 +377,24 @@ class LlamaMLP(nn.Module):
             act = ops.swiglu(self.gate_up_proj(x))
         return self.down_proj(act)
 
+    def normed_ragged(self, x, pending, eps, weight):
+        """The new residual and the feed-forward of its normed row, for a single
+        row that the norm and the gates of are one launch; else None."""
+        from ..ops import serving as sv
+
+        if pending.delta.shape[0] != 1 or _watched(self) or \
+                type(self).forward is not LlamaMLP.forward or \
+                not self._glu_in_one():
+            return None
+        one = sv.normed_linear(x, pending, eps, weight,
+                               self.gate_up_proj.weight, glu=True)
+        return one and (one[0], self.down_proj(one[1]))
+
     def _glu_in_one(self) -> bool:
         """May a few rows skip the call of gate_up_proj: it is the layer made
         here, and nobody watches it?"""
         p = self.gate_up_proj
-        return (type(p) is ColumnParallelLinear and "forward" not in p.__dict__
-                and not (p._forward_hooks or p._forward_pre_hooks)
-                and not (nn.modules.module._global_forward_hooks
-                         or nn.modules.module._global_forward_pre_hooks)
+        return (type(p) is ColumnParallelLinear and not _watched(p)
                 and p.bias is None and not p.skip_bias_add
                 and not (p.gather_output or p.sequence_parallel_enabled))
 
@@ -548,13 +587,21 @@ class LlamaForCausalLM(nn.Module):
         m, eps = self.model, self.config.rms_norm_eps
         x, pending = None, sv.Pending(m.embed_tokens(batch.tokens))
         for layer, pool in zip(m.layers, pools):
-            x, h, _ = sv.residual_norm(x, pending, eps,
-                                       layer.input_layernorm.weight)
-            pending = sv.Pending(layer.self_attn.forward_ragged(
-                h, m.rope_cos, m.rope_sin, batch, pool[0]))
-            x, h, _ = sv.residual_norm(x, pending, eps,
-                                       layer.post_attention_layernorm.weight)
-            pending = sv.Pending(layer.mlp(h))
+            attn, mlp = layer.self_attn, layer.mlp
+            at = m.rope_cos, m.rope_sin, batch, pool[0]
+            w = layer.input_layernorm.weight
+            one = attn.normed_ragged(x, pending, eps, w, *at)
+            if one is None:
+                x, h, _ = sv.residual_norm(x, pending, eps, w)
+                one = x, attn.forward_ragged(h, *at)
+            x, pending = one[0], sv.Pending(one[1])
+            w = layer.post_attention_layernorm.weight
+            one = mlp.normed_ragged(x, pending, eps, w) \
+                if isinstance(mlp, LlamaMLP) else None
+            if one is None:
+                x, h, _ = sv.residual_norm(x, pending, eps, w)
+                one = x, mlp(h)
+            x, pending = one[0], sv.Pending(one[1])
         if not batch.want.shape[0]:
             return None
         _, h, _ = sv.residual_norm(x, pending, eps, m.norm.weight,

@@ -106,7 +106,9 @@ class _StreamArgs(ctypes.Structure):
     _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
                 + _fields("w", ctypes.c_void_p) + _fields("wst", ctypes.c_long)
                 + _fields("out", ctypes.c_void_p)
-                + _fields("T N K", ctypes.c_int))
+                + _fields("T N K", ctypes.c_int)
+                + _fields("res delta res_out weight", ctypes.c_void_p)
+                + _fields("eps", ctypes.c_float))
 
 
 class _ConvArgs(ctypes.Structure):
@@ -1304,6 +1306,43 @@ def _linear_args(x, x_step, w, out, out_step, gate):
         a.gate, a.gst, a.gh = _p(gate), gate.stride(0), N
         mfma = mfma and _aligned((), gate)
     return a, mfma
+
+
+def normed_linear(x: Optional[torch.Tensor], pending: Pending, eps: float,
+                  weight: torch.Tensor, w: torch.Tensor, glu: bool = False):
+    """``residual_norm`` of one row and the product of its result with w (N, K)
+    in one launch: (new x, h w^T, or with ``glu`` silu(gate) * up of w = [gate;
+    up]); None where they are two: other rows, pending things, types and sizes,
+    and where ``stream_how`` leaves the product to the library.  Every workgroup
+    norms the row, 32 KB of a K of 4096, while its weights are on their way; of
+    more than one such round of them (512) the later ones have nothing to hide
+    that behind."""
+    d = pending.delta
+    if d is None or d.shape[0] != 1 or d.dtype != torch.bfloat16 or \
+            not d.is_contiguous() or pending.scale != 1.0 or any(
+                t is not None for t in (pending.delta2, pending.w1, pending.w2,
+                                        pending.vec, pending.coef)):
+        return None
+    K = d.shape[1]
+    if K > 4096 or not (glu or w.shape[0] <= 512 * 16) or \
+            not (_plain(weight) and weight.dtype == d.dtype) or \
+            not _aligned((K,), d) or weight.data_ptr() & 15 or \
+            weight.shape != (K,) or not weight.is_contiguous() or \
+            not (x is None or x.dtype == torch.float32 and x.is_contiguous()
+                 and x.shape == d.shape and not x.data_ptr() & 15):
+        return None
+    how = stream_how(d, w, glu=glu)
+    if how is None:
+        return None
+    N = w.shape[0]
+    x_new = torch.empty(1, K, dtype=torch.float32, device=d.device)
+    out = torch.empty(1, N // 2 if glu else N, dtype=d.dtype, device=d.device)
+    a = _StreamArgs(w=w.data_ptr(), wst=w.stride(0), out=out.data_ptr(), T=1,
+                    N=N, K=K, res=_p(x), delta=d.data_ptr(),
+                    res_out=x_new.data_ptr(), weight=weight.data_ptr(), eps=eps)
+    _check(library().sv_stream_linear(ctypes.byref(a), 2 if glu else 0, how,
+                                      _stream()), "normed_linear")
+    return x_new, out
 
 
 def head_linear(x, x_step: int, w, out, out_step: int,

@@ -307,6 +307,20 @@ class GQAQKVColumnParallelLinear(BaseParallelLinear):
             self._qkv_cat_cache = cached
         return cached[1], cached[2]
 
+    def weight_in_one(self):
+        """[q; k; v] where ``forward`` is one product with it and nothing else,
+        or None."""
+        if torch.is_grad_enabled() or self.training or \
+                self.sequence_parallel_enabled or ps.is_aot_mode() or \
+                self.bias_q is not None or not self.weight_q.is_cuda:
+            return None
+        return self._fused_qkv_weight()[0]
+
+    def split(self, out):
+        nq = self.q_output_size_per_partition
+        nkv = self.kv_output_size_per_partition
+        return out[..., :nq], out[..., nq:nq + nkv], out[..., nq + nkv:]
+
     def forward(self, input_):
         from .. import ops as _ops
 
@@ -320,12 +334,7 @@ class GQAQKVColumnParallelLinear(BaseParallelLinear):
             out = _ops.skinny_or_none(input_, wcat) if bcat is None else None
             if out is None:
                 out = F.linear(input_, wcat, bcat)
-            nq = self.q_output_size_per_partition
-            nkv = self.kv_output_size_per_partition
-            q = out[..., :nq]
-            k = out[..., nq:nq + nkv]
-            v = out[..., nq + nkv:]
-            return q, k, v
+            return self.split(out)
         q, k, v = _QKVLinearWithAsyncCommunication.apply(
             input_, self.weight_q, self.weight_k, self.weight_v,
             self.bias_q, self.bias_k, self.bias_v,

@@ -726,6 +726,43 @@ def test_few_rows_are_streamed_where_nobody_watches(glu):
         assert not any("empty" in str(f) for f in seen)
 
 
+@pytest.mark.parametrize("residual", [True, False])
+@pytest.mark.parametrize("K,N,glu", [
+    (8, 16, False), (520, 1001, False), (2056, 48, False), (4096, 8192, False),
+    (2048, 20480, True), (1032, 20512, True), (4096, 28672, True)])
+def test_product_of_a_normed_row(K, N, glu, residual):
+    """One launch against 64 bits, and where it stays two."""
+    torch.manual_seed(K + N)
+    x = torch.randn(1, K, device="cuda") if residual else None
+    delta = torch.randn(1, K, device="cuda").bfloat16()
+    weight = (1 + 0.1 * torch.randn(K, device="cuda")).bfloat16()
+    w = torch.randn(N, K, device="cuda").div(K ** 0.5).bfloat16()
+    with torch.no_grad():
+        got, out = sv.normed_linear(x, sv.Pending(delta), 1e-5, weight, w, glu)
+        assert torch.equal(got, delta.float() + x if residual else
+                           delta.float())
+        s = got.double()
+        h = s * (s.square().mean(1, keepdim=True) + 1e-5).rsqrt() * \
+            weight.double()
+        ref = h @ w.double().t()
+        if glu:
+            ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
+        # rounded to 8 bits: h, whose K errors of at most 2 ** -9 a part add up
+        # like 2 ** -9 of a result of about 1, gates and projections of up to 4;
+        # and the result
+        torch.testing.assert_close(out.double(), ref, rtol=2.0 ** -8,
+                                   atol=2.0 ** -9 * 6 * (4 if glu else 1))
+        if K < 4096:
+            return
+        two = torch.cat([delta, delta])
+        assert sv.normed_linear(None, sv.Pending(two), 1e-5, weight, w,
+                                glu) is None
+        for other in (sv.Pending(delta.float()), sv.Pending(delta, scale=2.0),
+                      sv.Pending(delta, vec=weight)):
+            assert sv.normed_linear(x, other, 1e-5, weight, w, glu) is None
+    assert sv.normed_linear(x, sv.Pending(delta), 1e-5, weight, w, glu) is None
+
+
 def test_the_switch_keeps_32_bit_products_on_the_library(monkeypatch):
     x = torch.randn(2, 4096, device="cuda").bfloat16()
     w = torch.randn(6144, 4096, device="cuda").bfloat16()
