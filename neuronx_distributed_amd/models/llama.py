@@ -266,12 +266,10 @@ class LlamaAttention(nn.Module):
     def _attend_ragged(self, qkv, cos, sin, batch, pool):
         from ..ops import serving as sv
 
-        q, k, v = qkv
-        sv.rope_rows_(q, k, cos, sin, batch.pos, self.head_dim,
-                      batch.max_keys)
         return self.o_proj(sv.ragged_attention(
-            q, k, v, batch, pool, self.num_heads_local,
-            1.0 / math.sqrt(self.head_dim), self.sliding_window or 0))
+            *qkv, batch, pool, self.num_heads_local,
+            1.0 / math.sqrt(self.head_dim), self.sliding_window or 0,
+            rotary=(cos, sin)))
 
     def _decode_step(self, q, k, v, cos, sin, pos_t, kv_cache, sp):
         """One-token decode with everything derived from the device tensor

@@ -232,6 +232,8 @@ struct RowsArgs {
   int MB, rows, H, G, D, E, splits, append, window, keep;
   float scale;
   ScoreArgs mod;
+  const float *cos, *sin;      // [positions][D / 2]: q and k are still to be
+                               //   turned (form 2, plain scores); or null
 };
 
 // tanh, in the 32-bit mode to the last digits, else to 1e-7
@@ -478,7 +480,10 @@ __device__ __forceinline__ float max_quarters(float x) {
   return max_halves(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
 }
 
-template <bool MOD, int DE>
+// ROT: the row's queries and key are turned here, an element with that half a head
+// on, which the same lane holds.  As a kernel of its own, which every layer waits
+// for, that took 4.6 us (4 layers, 16 steps, one request ROPE1 us, 32 ROPE32).
+template <bool MOD, int DE, bool ROT>
 __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   constexpr int NC = DE / 32;            // chunks of a key
   constexpr int NB = DE / 16;            // 16-row blocks of O^T
@@ -506,17 +511,30 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
     const long page = bt[i_pos / SV_PAGE];
     const long base = (page * a.G + g) * SV_PAGE + i_pos % SV_PAGE;
     for (int i = tid; i < DE; i += 256) {
-      ((short*)a.kc)[base * a.kcs + i] = kn[i];
+      if (!ROT) ((short*)a.kc)[base * a.kcs + i] = kn[i];
       ((short*)a.vc)[base * a.vcs + i] = vn[i];
     }
   }
 
-  frag_u qf[NC];
+  frag_u qf[NC], own[ROT ? NC : 1];      // own: the row's key
   {
     const short* src = (const short*)a.q + row * a.qst + (long)h * DE + grp * 8;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) qf[c].u4 = *(const uint4v*)(src + c * 32);
+    for (int c = 0; c < NC; ++c) {
+      qf[c].u4 = *(const uint4v*)(src + c * 32);
+      if (ROT) own[c].u4 = *(const uint4v*)(kn + c * 32 + grp * 8);
+    }
   }
+  float co[ROT ? NC / 2 : 1][8], si[ROT ? NC / 2 : 1][8];
+  if constexpr (ROT)
+#pragma unroll
+    for (int c = 0; c < NC / 2; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        const long at = (long)i_pos * (DE / 2) + c * 32 + grp * 8 + j;
+        load4(a.cos + at, co[c] + j);
+        load4(a.sin + at, si[c] + j);
+      }
   // scores in units of log 2; of the cap, if there is one
   const float cap = MOD ? a.mod.cap : 0.f;
   float s2 = cap > 0.f ? a.scale / cap : a.scale * SV_LOG2E;
@@ -578,8 +596,15 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   f32x4 o[NB] = {};                      // O^T: rows d, col head
   float m = NEG_BIG, l = 0.f;            // l: of this lane's keys
 
-  auto attend = [&](int n, const frag_u (*kf)[NC], char* vbuf) __attribute__((always_inline)) {
+  auto attend = [&](int n, frag_u (*kf)[NC], char* vbuf) __attribute__((always_inline)) {
     const int t = tile_of(n);
+    if constexpr (ROT)
+      if (t == t_hi)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (i * 16 + c16 >= i_pos - t * 32)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) kf[i][c] = own[c];
     f32x4 s[2] = {};
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -664,6 +689,36 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
     const int first = page_of(n);
     page = page_of(n + 4);
     issue(n, first, ka, v0);
+  }
+  if constexpr (ROT) {                   // while the first tile is on its way
+#pragma unroll
+    for (int c = 0; c < NC / 2; ++c) {
+#pragma unroll
+      for (int z = 0; z < 2; ++z) {
+        frag_u& lo = z ? own[c] : qf[c];
+        frag_u& up = z ? own[c + NC / 2] : qf[c + NC / 2];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float x[2], y[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float p = __uint_as_float(e ? lo.u[u] & 0xffff0000u : lo.u[u] << 16);
+            const float q = __uint_as_float(e ? up.u[u] & 0xffff0000u : up.u[u] << 16);
+            x[e] = p * co[c][2 * u + e] - q * si[c][2 * u + e];
+            y[e] = q * co[c][2 * u + e] + p * si[c][2 * u + e];
+          }
+          lo.u[u] = pack_bf16x2(x[0], x[1]);
+          up.u[u] = pack_bf16x2(y[0], y[1]);
+        }
+      }
+    }
+    if (split == 0 && rc == 0 && wid == 0 && c16 == 0) {
+      const long page = bt[i_pos / SV_PAGE];
+      short* to = (short*)a.kc +
+                  ((page * a.G + g) * SV_PAGE + i_pos % SV_PAGE) * a.kcs + grp * 8;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) *(uint4v*)(to + c * 32) = own[c].u4;
+    }
   }
   for (; n < n1; n += 8) {
     arrived();
@@ -800,10 +855,18 @@ static int launch_rows(const RowsArgs& a, int vec, hipStream_t stream) {
                             : rep >= 8 ? 8 : rep > 2 ? 4 : rep;
   const int nrc = vec == 2 ? (rep + 15) / 16 : (rep + rcn - 1) / rcn;
   const long grid = (long)a.rows * a.G * nrc * a.splits;
+  if (a.cos && vec != 2) return 1;
   if (vec == 2) {
     if (sizeof(T) != 2 || a.D != a.E || (a.D != 64 && a.D != 128)) return 1;
-    if (a.D == 64) attn_rows_mfma_kernel<MOD, 64><<<grid, 256, 0, stream>>>(a);
-    else attn_rows_mfma_kernel<MOD, 128><<<grid, 256, 0, stream>>>(a);
+#define ARM(D, R) attn_rows_mfma_kernel<MOD, D, R><<<grid, 256, 0, stream>>>(a)
+    if (a.cos) {
+      if constexpr (MOD) return 1;
+      else if (!a.append) return 1;
+      else if (a.D == 64) ARM(64, true);
+      else ARM(128, true);
+    } else if (a.D == 64) ARM(64, false);
+    else ARM(128, false);
+#undef ARM
     if (a.splits > 1)
       return sv_attn_merge(a.part, a.out, (long)a.rows * a.H, a.splits, a.E, 0,
                            stream);

@@ -143,7 +143,8 @@ class _RowsArgs(ctypes.Structure):
                 + _fields("pos seq bt part out", ctypes.c_void_p)
                 + _fields("MB rows H G D E splits append window keep",
                           ctypes.c_int)
-                + _fields("scale", ctypes.c_float) + [("mod", _ScoreArgs)])
+                + _fields("scale", ctypes.c_float) + [("mod", _ScoreArgs)]
+                + _fields("cos sin", ctypes.c_void_p))
 
 
 class _TilesArgs(ctypes.Structure):
@@ -862,14 +863,18 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
               scale: float, window: int = 0, keep: int = 0,
               append: bool = True, max_keys: int = 0,
               out: Optional[torch.Tensor] = None,
-              mod: Optional[ScoreMod] = None) -> torch.Tensor:
+              mod: Optional[ScoreMod] = None,
+              rotary=None) -> torch.Tensor:
     """One query row per request row: decoding.  ``append`` also writes the
     row's own k/v into the cache (without it they must be there already).
     ``max_keys`` bounds the visible keys of any row (it only chooses the kernel
-    and how many workgroups share a row)."""
+    and how many workgroups share a row).  ``rotary`` (cos, sin) as in
+    ``rope_rows_``, in the kernel where it has a form for that, else in place."""
     G, D, E = _check_cache(q, k, v, kc, vc, heads)
     rows = q.shape[0]
     assert pos.shape[0] == rows and seq.shape[0] == rows
+    if rotary is not None:
+        _check_rotary(*rotary, q, k, pos, D, max_keys)
     if window > 0:
         max_keys = min(max_keys, window + keep) if max_keys else window + keep
     vec = int(_aligned((D, E), q, k, v))
@@ -878,6 +883,10 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
                                   mod is not None)
     else:
         splits = _row_splits(1024, rows * G, max_keys, 128)
+    if rotary is not None and (vec != 2 or mod is not None or not append or
+                               any(t.data_ptr() & 15 for t in rotary)):
+        rope_rows_(q, k, *rotary, pos, D, 0)
+        rotary = None
     out = _out(out, rows, heads * E, q)
     part = torch.empty(rows * heads * splits * (E + 2), dtype=torch.float32,
                        device=q.device) if splits > 1 else None
@@ -889,6 +898,8 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
                   rows=rows, H=heads, G=G, D=D, E=E, splits=splits,
                   append=int(append), window=window, keep=keep, scale=scale,
                   mod=_score_args(mod, q, heads))
+    if rotary is not None:
+        a.cos, a.sin = map(_p, rotary)
     _check(library().sv_attn_rows(ctypes.byref(a), vec, _f32(q), _stream()),
            "attn_rows")
     return out
@@ -931,12 +942,18 @@ def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
 def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
                      window: int = 0, keep: int = 0,
                      prep: Optional[QkvPrep] = None,
-                     mod: Optional[ScoreMod] = None) -> torch.Tensor:
+                     mod: Optional[ScoreMod] = None,
+                     rotary=None) -> torch.Tensor:
     """Attention of a packed batch over its cache pool: portions first, then
     single tokens, into one (T, heads * E) tensor.  ``prep`` changes q in
-    place."""
+    place, ``rotary`` (cos, sin) turns q and k as ``rope_rows_`` does and may."""
     kc, vc = pool
     T, n = q.shape[0], batch.portion_tokens
+    if rotary is not None:
+        assert prep is None
+        if n:
+            rope_rows_(q, k, *rotary, batch.pos, kc.shape[3], batch.max_keys)
+            rotary = None
     out = torch.empty(T, heads * vc.shape[3], dtype=q.dtype, device=q.device)
     args = dict(heads=heads, scale=scale, window=window, keep=keep,
                 max_keys=batch.max_keys, append=prep is None)
@@ -950,19 +967,24 @@ def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
     if n < T:
         attn_rows(q[n:], k[n:], v[n:], kc, vc, batch.pos[n:], batch.seq[n:],
                   batch.block_table, out=out[n:], mod=mod and mod.rows(n, T),
-                  **args)
+                  rotary=rotary, **args)
     return out
 
 
-def rope_rows_(q, k, cos, sin, pos, dim: int, max_pos: int):
-    """Rotate the heads of q and k (rotate-half) in place, each row at its
-    own position; cos/sin (positions, dim / 2) float32."""
+def _check_rotary(cos, sin, q, k, pos, dim: int, max_pos: int):
     if max_pos > cos.shape[0]:
         raise ValueError(f"position {max_pos - 1} is outside the rotary "
                          f"table of {cos.shape[0]}")
     assert cos.dtype == sin.dtype == torch.float32 and cos.is_contiguous()
     assert sin.is_contiguous() and cos.shape[1] * 2 == dim
+    assert sin.shape == cos.shape
     assert q.stride(1) == k.stride(1) == 1 and pos.shape[0] == q.shape[0]
+
+
+def rope_rows_(q, k, cos, sin, pos, dim: int, max_pos: int):
+    """Rotate the heads of q and k (rotate-half) in place, each row at its
+    own position; cos/sin (positions, dim / 2) float32."""
+    _check_rotary(cos, sin, q, k, pos, dim, max_pos)
     vp, lg = ctypes.c_void_p, ctypes.c_long
     _check(library().sv_rope_rows(
         vp(_p(q)), lg(q.stride(0)), q.shape[1] // dim, vp(_p(k)),

@@ -120,6 +120,50 @@ def test_attention_prompt_portions_and_decoding(sv, case, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,window", [
+    (8, 2, 128, 0), (3, 3, 128, 0), (17, 1, 128, 40), (14, 2, 64, 0),
+    (8, 8, 64, 100), (6, 2, 32, 0)])
+def test_single_rows_turned_in_the_kernel(sv, H, G, D, window, dtype):
+    """Queries and keys turned beside the attention, or before it where it has
+    no form for that: first and last places of tiles, pages and rows."""
+    torch.manual_seed(H + D)
+    at = [0, 31, 32, 63, 64, 95, 127, 300, 701]
+    need = [p // 64 + 1 for p in at]
+    table = torch.zeros(len(at), max(need), dtype=torch.int32)
+    place = torch.randperm(sum(need)).int()
+    for i, n in enumerate(need):
+        table[i, :n] = place[sum(need[:i]):sum(need[:i + 1])]
+    cache = [torch.randn(sum(need), G, 64, D, device="cuda").to(dtype)
+             for _ in "kv"]
+    proj = torch.randn(len(at), (H + 2 * G) * D, device="cuda").to(dtype)
+    angle = torch.rand(702, D // 2, device="cuda") * 6
+    cos, sin = angle.cos(), angle.sin()
+    pos = torch.tensor(at, dtype=torch.int32, device="cuda")
+    seq = torch.arange(len(at), dtype=torch.int32, device="cuda")
+    got = []
+    for turned in (False, True):
+        q, k, v = proj.clone().split([H * D, G * D, G * D], 1)
+        kc, vc = (c.clone() for c in cache)
+        if turned:
+            sv.rope_rows_(q, k, cos, sin, pos, D, 702)
+        out = sv.attn_rows(q, k, v, kc, vc, pos, seq, table.cuda(), H, D ** -0.5,
+                           window, max_keys=702,
+                           rotary=None if turned else (cos, sin))
+        got.append((out.float(), kc.float(), vc.float()))
+    (out, kc, vc), (want, kw, vw) = got
+    # a product may be fused with the other's sum: then an element is rounded
+    # to the other side, and the scores of one key move by 2 ** -9 of a part
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22
+    torch.testing.assert_close(kc, kw, rtol=eps, atol=2 * eps)
+    torch.testing.assert_close(out, want, rtol=eps, atol=2 * eps)
+    assert torch.equal(vc, vw)
+    with pytest.raises(ValueError):
+        sv.attn_rows(q, k, v, kc.to(dtype), vc.to(dtype), pos, seq,
+                     table.cuda(), H, D ** -0.5, window, max_keys=703,
+                     rotary=(cos, sin))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window,keep", [(92, 22), (64, 64), (70, 3),
                                          (33, 0), (128, 65)])
 def test_attention_edges_show(sv, window, keep, dtype):
