@@ -823,11 +823,10 @@ def _row_splits(target: int, units: int, max_keys: int, per: int) -> int:
 # 52.8; 128 rows of 28/4, 1000: 37.5, 28.4), up to 5% over it in 5 of them (45 rows of
 # 32/8, 2000 equal keys: 75.8, 77.7).
 _SHARED_KEYS = (256, 700, 1200, 2500, 5000)
-_SHARED_ROWS = ((64, (0, 256, 256, 256, 512, 512)),
-                (128, (0, 512, 512, 512, 512, 768)),
-                (255, (0, 0, 0, 512, 1024, 1536)),
-                (512, (0, 0, 0, 640, 2048, 2048)),
-                (math.inf, (0, 0, 0, 1024, 2048, 2048)))
+_SHARED_UNITS = (64, 128, 255, 512)
+_SHARED_ROWS = ((0, 256, 256, 256, 512, 512), (0, 512, 512, 512, 512, 768),
+                (0, 0, 0, 512, 1024, 1536), (0, 0, 0, 640, 2048, 2048),
+                (0, 0, 0, 1024, 2048, 2048))
 
 
 def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
@@ -854,8 +853,8 @@ def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
             100 if units > (1024 if modified else 2048) else 64
     if units > 512 and 0 < max_keys <= short:
         return 1, _row_splits(1024, units, max_keys, 128)
-    target = next(t for most, t in _SHARED_ROWS if units <= most)
-    target = target[bisect.bisect_left(_SHARED_KEYS, max_keys)]
+    target = _SHARED_ROWS[bisect.bisect_left(_SHARED_UNITS, units)][
+        bisect.bisect_left(_SHARED_KEYS, max_keys)]
     return 2, _row_splits(target, units, max_keys, 128)
 
 
