@@ -18,6 +18,7 @@
 // 4096 x 4096, 4096 x 14336 and 28672 gated columns now take 7.5, 22 and 43.5.
 
 #include "serving.h"
+#include "words.h"
 
 struct StreamArgs {
   const short* x;           // [T] rows of K
@@ -66,9 +67,6 @@ __device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n,
 // Words past a row are read as its first ones, and become zeros where they are
 // multiplied: a branch a load, or a select behind it, would make every product
 // wait for the loads of the next turn.
-__device__ __forceinline__ uint4v word_at(const short* p, bool in, int k) {
-  return *(const uint4v*)(p + (in ? k : 0));
-}
 __device__ __forceinline__ bf16x8 if_there(bool in, frag_u f) {
   if (!in) f.u4 = uint4v{0, 0, 0, 0};
   return f.bf;
@@ -141,29 +139,31 @@ __global__ void __launch_bounds__(1024) stream_linear_kernel(StreamArgs a) {
   const int K = a.K;
   const int n0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * MT;
 
-  const short* w = a.w + (long)min(n0 + c16, a.N - 1) * a.wst + grp * 8;
+  // words of column k on are at column(k)
+  const int from = FULL ? grp * 8 : 0;
+  auto column = [&](int k) __attribute__((always_inline)) {
+    return FULL ? k : word_column(k, grp, K);
+  };
+  const short* w = a.w + (long)min(n0 + c16, a.N - 1) * a.wst + from;
   const short* x[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
-    x[i] = a.x + (long)min(t0 + i * 16 + c16, a.T - 1) * a.xst + grp * 8;
+    x[i] = NORM ? row + from
+                : a.x + (long)min(t0 + i * 16 + c16, a.T - 1) * a.xst + from;
 
   f32x4 acc[MT] = {};
   auto load_w = [&](int k0, frag_u* fw) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * 32;
-      fw[u].u4 = word_at(w, FULL || k + grp * 8 < K, k);
-    }
+    for (int u = 0; u < U; ++u)
+      fw[u].u4 = *(const uint4v*)(w + column(k0 + u * 32));
   };
   auto load_x = [&](int k0, frag_u (*fx)[MT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * 32;
-      const bool in = FULL || k + grp * 8 < K;
+      const int at = column(k0 + u * 32);
 #pragma unroll
       for (int i = 0; i < MT; ++i)
-        fx[u][i].u4 = NORM ? *(const uint4v*)(row + (in ? k + grp * 8 : 0))
-                           : word_at(x[i], in, k);
+        fx[u][i].u4 = *(const uint4v*)(x[i] + at);
     }
   };
   auto load = [&](int k0, frag_u* fw, frag_u (*fx)[MT])

@@ -1,11 +1,14 @@
 """Decoding: which kernels take products of a few rows, attention of single
 rows and experts of few rows."""
 
+import os
+import shutil
+import subprocess
 import types
 
 import pytest
 
-from neuronx_distributed_amd.ops import serving as sv
+from neuronx_distributed_amd.ops import build, serving as sv
 
 
 def test_a_library_without_the_products_is_not_used(monkeypatch):
@@ -15,6 +18,36 @@ def test_a_library_without_the_products_is_not_used(monkeypatch):
     monkeypatch.setattr(sv, "_LIB",
                         types.SimpleNamespace(sv_stream_linear=None))
     assert sv.available()
+
+
+@pytest.mark.skipif(not shutil.which("g++"), reason="no host compiler")
+def test_every_word_of_a_streamed_row_lies_in_it(tmp_path):
+    """Rows of all K up to 4200 in the turns of 16 waves: words past the end are
+    read from the row too, also of rows shorter than the 32 columns that four
+    groups of lanes read at once."""
+    source = tmp_path / "words.cpp"
+    source.write_text("""
+        #include <cstdio>
+        #include "words.h"
+        int main() {
+          for (int K = 8; K <= 4200; K += 8)
+            for (int turn = 0; turn < K + 1024; turn += 32)
+              for (int grp = 0; grp < 4; ++grp) {
+                const int at = word_column(turn, grp, K), own = turn + grp * 8;
+                if (at < 0 || at + 8 > K || (own < K && at != own)) {
+                  printf("K %d, columns %d, group %d: %d", K, turn, grp, at);
+                  return 1;
+                }
+              }
+          return 0;
+        }
+    """)
+    program = tmp_path / "words"
+    subprocess.run(["g++", "-std=c++17", "-I",
+                    os.path.join(build.CSRC, "serving"), str(source), "-o",
+                    str(program)], check=True)
+    run = subprocess.run([str(program)], stdout=subprocess.PIPE, text=True)
+    assert run.returncode == 0, run.stdout
 
 
 SIZES = (8, 16, 24, 64, 248, 512, 576, 896, 1000, 1408, 2048, 2880, 3072,
