@@ -33,6 +33,8 @@
 #include "mfma.h"
 #include "lds.h"
 
+#include <cfloat>
+
 #define FA_D 128
 #define LOG2E 1.4426950408889634f
 
@@ -132,6 +134,7 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(16))) char d0b[TILE_B], d1b[TILE_B];
   // lse * log2(e) and delta of a step's rows
   __shared__ __attribute__((aligned(16))) float ld0[128], ld1[128];
+  __shared__ int odd;          // is there a row whose lse is no number?
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -168,13 +171,20 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   // (two waves' numbers go into LDS only behind the step: where they are asked for,
   // those two would wait for them, and all others for these two)
   float nl = 0.f;
+  // (a row whose lse is no number has no weights in the steps: masked places would
+  // get them too, and keys that the row does not see)
+  if (tid == 0) odd = 0;
   auto issue = [&](char* qb, char* db) __attribute__((always_inline)) {
     if (wid < 2) nl = (wid ? delta : lse)[min(next + lane, S - 1)];
     fill_rows<64, 512>(qg, a.q_ss, next, S, qb);
     fill_rows<64, 512>(dg, a.do_ss, next, S, db);
   };
   auto leave = [&](float* ld) __attribute__((always_inline)) {
-    if (wid < 2) ld[tid] = wid ? nl : nl * LOG2E;
+    if (wid == 0) {
+      if (!(nl > -INFINITY)) odd = 1;
+      ld[tid] = fabsf(nl) < INFINITY ? nl * LOG2E : FLT_MAX;
+    }
+    if (wid == 1) ld[tid] = nl;
   };
   auto advance = [&]() __attribute__((always_inline)) {
     if ((next += 64) < q_end) return;
@@ -307,8 +317,22 @@ __global__ void __launch_bounds__(512, 2) fa_bwd_dkdv_kernel(BwdArgs a) {
   __syncthreads();
   meet(dk, room);
   if (half || my_k >= S) return;
-  store_turned(dv, 1.f, a.dv + b * a.dv_bs + hd * a.dv_hs + my_k * a.dv_ss, hi);
-  store_turned(dk, a.scale, a.dk + b * a.dk_bs + hd * a.dk_hs + my_k * a.dk_ss, hi);
+  short* to_v = a.dv + b * a.dv_bs + hd * a.dv_hs + my_k * a.dv_ss;
+  short* to_k = a.dk + b * a.dk_bs + hd * a.dk_hs + my_k * a.dk_ss;
+  store_turned(dv, 1.f, to_v, hi);
+  store_turned(dk, a.scale, to_k, hi);
+  if (!odd) return;
+  // keys that an odd row sees
+  lse = a.lse + ((long)b * a.Hq + h) * S;
+  bool seen = false;
+  for (int n = 0; n < heads; ++n, lse += S)
+    for (int q = max(q_start, a.causal ? my_k : 0);
+         q < (window > 0 ? min(S, my_k + window) : S); ++q)
+      seen |= !(lse[q] > -INFINITY);
+  if (!seen) return;
+  for (int nb = 0; nb < 4; ++nb) dv[nb] = f32x16{} + NAN;
+  store_turned(dv, 1.f, to_v, hi);
+  store_turned(dv, 1.f, to_k, hi);
 }
 
 __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {

@@ -200,6 +200,39 @@ def test_flash_attn_bwd_sums_heads_in_a_workgroup(monkeypatch, Hq, Hkv, heads,
         assert err < 3 * 2 ** -8, (name, err)
 
 
+@pytest.mark.parametrize("row", [75, 199])
+@pytest.mark.parametrize("bad", [math.nan, math.inf, -math.inf])
+@pytest.mark.parametrize("causal,window", [(True, None), (True, 70),
+                                           (False, None)])
+def test_flash_attn_bwd_of_a_row_without_weights(causal, window, bad, row):
+    """A row whose lse is no number reaches the keys that it sees, and nothing
+    else: all other gradients are the same bits."""
+    from neuronx_distributed_amd.kernels.ring_attn import _block_bwd, _block_fwd
+
+    torch.manual_seed(7)
+    B, Hq, Hkv, S, D, head = 1, 4, 2, 200, 128, 1
+    q, dout = (torch.randn(B, Hq, S, D, device="cuda").bfloat16()
+               for _ in range(2))
+    k, v = (torch.randn(B, Hkv, S, D, device="cuda").bfloat16()
+            for _ in range(2))
+    out, lse = _block_fwd(q, k, v, causal, 0.09, window)
+    out = out.bfloat16()
+    want = _block_bwd(q, k, v, out, dout, lse, causal, 0.09, window)
+    lse = lse.clone()
+    lse[0, head, row] = bad
+    dq, dk, dv = _block_bwd(q, k, v, out, dout, lse, causal, 0.09, window)
+    alone = torch.ones(B, Hq, S, dtype=torch.bool)
+    alone[0, head, row] = False
+    assert torch.equal(dq[alone.cuda()], want[0][alone.cuda()])
+    unseen = torch.ones(B, Hkv, S, dtype=torch.bool)
+    unseen[0, 0, row - window + 1 if window else 0:
+           row + 1 if causal else S] = False
+    for got, w in ((dk, want[1]), (dv, want[2])):
+        assert torch.equal(got[unseen.cuda()], w[unseen.cuda()])
+        if math.isnan(bad):
+            assert got[~unseen.cuda()].isnan().all()
+
+
 def test_flash_attn_bwd_heads_of_a_workgroup():
     """They divide the group, and no CU is left idle for them."""
     for B, Hq, Hkv, S, causal, window, n in (
