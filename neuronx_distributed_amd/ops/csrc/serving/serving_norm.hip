@@ -317,10 +317,7 @@ __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a)
   float c[P];
   if (DELTA == SUM)
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      c[p] = a.coef[r * a.parts + min(p, a.parts - 1)];
-      c[p] = p < a.parts ? c[p] : 0.f;
-    }
+    for (int p = 0; p < P; ++p) c[p] = a.coef[r * a.parts + min(p, a.parts - 1)];
   f32x4 v[R], t[R];
   s4v u[R], d[R], e[R][DELTA == SUM ? P : 1];
 #pragma unroll
@@ -346,7 +343,8 @@ __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a)
       if (DELTA == SUM) {
         t[k][j] = 0.f;
 #pragma unroll
-        for (int p = 0; p < P; ++p) t[k][j] += c[p] * bits2f(e[k][p][j]);
+        for (int p = 0; p < P; ++p)      // (no weight of zero: of infinities)
+          if (p < a.parts) t[k][j] += c[p] * bits2f(e[k][p][j]);
       }
       if (DELTA != NONE) v[k][j] += a.scale * t[k][j];
       sq += i < W ? v[k][j] * v[k][j] : 0.f;

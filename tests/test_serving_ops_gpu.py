@@ -463,6 +463,21 @@ def test_residual_norm_of_few_rows(sv, W, parts, pending):
                                        rtol=2 ** -8, atol=2e-5)
 
 
+@pytest.mark.parametrize("parts", [1, 3, 8, 9])
+def test_an_infinite_part_of_a_sum_stays_infinite(sv, parts):
+    """Also in the last part, which stands in for those that are not there."""
+    T, W, bf = 3, 4096, torch.bfloat16
+    d = _rand(T * parts, W, dtype=bf)
+    for t in range(T):
+        d[t * parts + parts - 1, 5 + t] = math.inf
+    coef = torch.ones(T, parts, dtype=torch.float32)
+    want = d.double().view(T, parts, W).sum(1)
+    got, _, _ = sv.residual_norm(None, sv.Pending(d.cuda(), coef=coef.cuda()),
+                                 1e-5, _rand(W, dtype=bf).cuda())
+    assert torch.equal(got.isinf().cpu(), want.isinf())
+    assert not got.isnan().any()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("W", [64, 100, 97, 1000, 4096])
 def test_residual_norm(sv, W, dtype):
