@@ -256,6 +256,7 @@ class LlamaAttention(nn.Module):
         p = self.qkv_proj
         if pending.delta.shape[0] != 1 or \
                 type(self).forward_ragged is not LlamaAttention.forward_ragged \
+                or "forward_ragged" in self.__dict__ \
                 or type(p) is not GQAQKVColumnParallelLinear or _watched(p):
             return None
         w = p.weight_in_one()
@@ -588,7 +589,8 @@ class LlamaForCausalLM(nn.Module):
             attn, mlp = layer.self_attn, layer.mlp
             at = m.rope_cos, m.rope_sin, batch, pool[0]
             w = layer.input_layernorm.weight
-            one = attn.normed_ragged(x, pending, eps, w, *at)
+            one = attn.normed_ragged(x, pending, eps, w, *at) \
+                if isinstance(attn, LlamaAttention) else None
             if one is None:
                 x, h, _ = sv.residual_norm(x, pending, eps, w)
                 one = x, attn.forward_ragged(h, *at)

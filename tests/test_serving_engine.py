@@ -3,6 +3,7 @@ configuration — everything of the serving engine that needs no GPU — and
 the oracle's own sensitivity to planted mistakes."""
 
 import json
+import types
 
 import numpy as np
 import pytest
@@ -299,6 +300,59 @@ def test_registry_loads_llama(tmp_path, groups):
     m = load_pretrained(str(tmp_path), torch.float32)
     x = torch.randint(0, c.vocab_size, (2, 7))
     assert torch.equal(generate(m, x, 5), generate(ref, x, 5))
+
+
+@pytest.mark.parametrize("own", ["module", "method"])
+def test_an_attention_of_the_users_own_serves_a_single_row(groups, monkeypatch,
+                                                           own):
+    """One that has ``forward_ragged`` and nothing else in common with the
+    model's, or a method that was put in place of it, is what runs."""
+    from neuronx_distributed_amd.models import build_model, get_config
+    from neuronx_distributed_amd.ops import serving as sv
+    from neuronx_distributed_amd.parallel.qkv_linear import \
+        GQAQKVColumnParallelLinear
+
+    model = build_model("LlamaForCausalLM", get_config("tiny"), torch.float32,
+                        "cpu")
+    ran = []
+
+    def forward_ragged(h, cos, sin, batch, pool):
+        ran.append(pool)
+        return 2 * h
+
+    class Own(torch.nn.Module):
+        def forward_ragged(self, *args):
+            return forward_ragged(*args)
+
+    for layer in model.model.layers:
+        if own == "module":
+            layer.self_attn = Own()
+        else:
+            layer.self_attn.forward_ragged = forward_ragged
+
+    def no_norm(x, pending, *a, **k):
+        x = pending.delta if x is None else x + pending.delta
+        return x, x, None
+
+    def one_launch(*a, **k):
+        raise AssertionError("the attention was passed by")
+
+    monkeypatch.setattr(sv, "residual_norm", no_norm)
+    monkeypatch.setattr(sv, "linear_f32", lambda h, w: h)
+    monkeypatch.setattr(sv, "normed_linear", one_launch)
+    # as on the GPU
+    monkeypatch.setattr(GQAQKVColumnParallelLinear, "weight_in_one",
+                        lambda self: self.weight_q)
+    for layer in model.model.layers:
+        layer.mlp = torch.nn.Identity()
+    batch = types.SimpleNamespace(tokens=torch.tensor([3]),
+                                  want=torch.zeros(1))
+    layers = len(model.model.layers)
+    with torch.no_grad():
+        got = model.forward_ragged(batch, [[i] for i in range(layers)])
+        x = model.model.embed_tokens.weight[3:4] * 6.0 ** layers
+    assert ran == list(range(layers))
+    torch.testing.assert_close(got, x)
 
 
 def test_engine_refuses_the_cpu_and_unfit_models(groups):
