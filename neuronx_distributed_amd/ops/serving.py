@@ -971,12 +971,13 @@ def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
 
 
 def _check_rotary(cos, sin, q, k, pos, dim: int, max_pos: int):
-    if max_pos > cos.shape[0]:
+    rows = min(cos.shape[0], sin.shape[0])
+    if max_pos > rows:
         raise ValueError(f"position {max_pos - 1} is outside the rotary "
-                         f"table of {cos.shape[0]}")
+                         f"table of {rows}")
     assert cos.dtype == sin.dtype == torch.float32 and cos.is_contiguous()
     assert sin.is_contiguous() and cos.shape[1] * 2 == dim
-    assert sin.shape == cos.shape
+    assert sin.shape[1] == cos.shape[1]
     assert q.stride(1) == k.stride(1) == 1 and pos.shape[0] == q.shape[0]
 
 

@@ -7,6 +7,7 @@ import subprocess
 import types
 
 import pytest
+import torch
 
 from neuronx_distributed_amd.ops import build, serving as sv
 
@@ -155,3 +156,16 @@ def test_kernel_of_many_small_experts(rows, experts, width, ff, want):
 def test_a_choice_without_the_sizes_is_refused():
     with pytest.raises(TypeError):
         sv.moe_kernel(64, 8)
+
+
+def test_rotary_tables_hold_every_position():
+    """Of two tables the shorter one counts; the longer one may be so."""
+    cos, sin = torch.zeros(90, 32), torch.zeros(100, 32)
+    q, k = torch.zeros(2, 256), torch.zeros(2, 64)
+    pos = torch.zeros(2, dtype=torch.int32)
+    for pair in ((cos, sin), (sin, cos), (cos, cos)):
+        sv._check_rotary(*pair, q, k, pos, 64, 90)
+        with pytest.raises(ValueError, match="position 90"):
+            sv._check_rotary(*pair, q, k, pos, 64, 91)
+    with pytest.raises(AssertionError):
+        sv._check_rotary(cos, torch.zeros(90, 64), q, k, pos, 64, 90)
