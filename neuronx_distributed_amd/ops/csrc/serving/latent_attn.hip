@@ -384,34 +384,64 @@ __device__ __forceinline__ int2* row_shares(const LatentRowsArgs& a) {
 
 struct Share { int row, i, n; };         // the i-th of n of a row
 
+#define LATENT_SHARES 512                // most of a group of 32 heads
+
 // The share of workgroup `item`; row is -1 if there is none.  Shares are of at
-// most `per` tiles, so there are no more than total / per + rows of them.
+// most `per` tiles, the least for which there are no more of them than
+// workgroups: at least total / items, at most total / (items - rows).  (That bound
+// itself left every second workgroup of two a row without work: 46 rows of 3613
+// keys, 128 heads 253 us, now 162; as many shares of every row, however long: 191.)
 __device__ __forceinline__ Share share_of(const LatentRowsArgs& a, int item) {
+  constexpr int B = LATENT_SHARES / 2 / 64;    // rows of two shares, 64 a time
   const int lane = threadIdx.x & 63;
   const int items = a.rows * a.splits;
-  auto tiles = [&](int b) {
-    if (b + lane >= a.rows) return 0;
-    const int p = a.pos[b + lane];
-    return p / 32 - (a.window > 0 ? max(0, p - a.window + 1) / 32 : 0) + 1;
+  auto sum = [](int x) { return __builtin_amdgcn_readlane(scan64(x), 63); };
+  int n[B], total = 0;
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    n[b] = 0;
+    if (64 * b >= a.rows) continue;
+    if (64 * b + lane < a.rows) {
+      const int p = a.pos[64 * b + lane];
+      n[b] = p / 32 - (a.window > 0 ? max(0, p - a.window + 1) / 32 : 0) + 1;
+    }
+    total += sum(n[b]);
+  }
+  auto shares = [](int tiles, int per, float inv) {
+    const int x = tiles + per - 1;
+    int q = (int)(x * inv);              // off by one at most
+    q -= q * per > x;
+    q += (q + 1) * per <= x;
+    return q;
   };
-  int n = tiles(0), total = __builtin_amdgcn_readlane(scan64(n), 63);
-  for (int b = 64; b < a.rows; b += 64)
-    total += __builtin_amdgcn_readlane(scan64(tiles(b)), 63);
-  const int per = (total + items - a.rows - 1) / (items - a.rows);
-  for (int b = 0;;) {
-    const int mine = (n + per - 1) / per;
+  auto count = [&](int per) {
+    const float inv = __builtin_amdgcn_rcpf(per);
+    int c = 0;
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+      if (64 * b < a.rows) c += shares(n[b], per, inv);
+    return sum(c);
+  };
+  int per = (total + items - 1) / items;
+  for (int most = (total + items - a.rows - 1) / (items - a.rows); per < most;) {
+    const int half = (per + most) / 2;
+    if (count(half) <= items) most = half; else per = half + 1;
+  }
+  const float inv = __builtin_amdgcn_rcpf(per);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    if (64 * b >= a.rows) break;
+    const int mine = shares(n[b], per, inv);
     const int last = scan64(mine);       // of the shares up to this lane's row
-    const int sum = __builtin_amdgcn_readlane(last, 63);
-    if (item < sum) {
+    const int all = __builtin_amdgcn_readlane(last, 63);
+    if (item < all) {
       const int l = __ffsll((unsigned long long)__ballot(last > item)) - 1;
       const int k = __builtin_amdgcn_readlane(mine, l);
-      return {b + l, item - __builtin_amdgcn_readlane(last, l) + k, k};
+      return {64 * b + l, item - __builtin_amdgcn_readlane(last, l) + k, k};
     }
-    item -= sum;
-    b += 64;
-    if (b >= a.rows) return {-1, 0, 0};
-    n = tiles(b);
+    item -= all;
   }
+  return {-1, 0, 0};
 }
 
 // FULL: R = EP and P = 64, no padding
@@ -765,8 +795,6 @@ latent_merge_kernel(LatentRowsArgs a, HeadLinearArgs l) {
     }
   }
 }
-
-#define LATENT_SHARES 512                // most of a group of 32 heads
 
 static int launch_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
   const long grid = (long)a->rows * ((a->H + 31) / 32) * a->splits;

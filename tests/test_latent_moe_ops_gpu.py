@@ -2,6 +2,8 @@
 against the plain implementation in ``nesilorn_oracle`` (float64), one
 mechanism at a time."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -185,6 +187,35 @@ def test_rows_of_all_lengths_share_workgroups(sv, rows, H, R, P, window):
         seen = slice(max(0, p - window + 1) if window else 0, p + 1)
         want[i] = (qd[i] @ kd[seen].T * 0.21).softmax(-1) @ kd[seen, :R]
     _close(got, want, dtype, what=(rows, H, R, P, window))
+
+
+@pytest.mark.parametrize("rows", [1, 2, 46, 64, 65, 130, 256])
+@pytest.mark.parametrize("equal", [True, False])
+@pytest.mark.parametrize("window", [0, 330])
+def test_rows_are_shared_by_all_workgroups(sv, rows, equal, window):
+    """Shares are the smallest of which there are no more than workgroups, so
+    equal rows leave none of them without work."""
+    H, R, P = 3, 64, 64
+    pos = [899 if equal else 899 - 880 * i // rows for i in range(rows)]
+    cache, bt = _cache([900], R + P, torch.bfloat16)
+    q = _rand(rows, H * (R + P), dtype=torch.bfloat16).cuda()
+    out = torch.empty(rows, H * R, dtype=q.dtype, device="cuda")
+    held = _ints(pos), _ints([0] * rows)
+    a, part = sv._latent_rows_args(q, cache, R, *held, bt, H, 0.1, window,
+                                   900, None, out)
+    assert a.splits > 1
+    sv._check(sv.library().sv_latent_rows(ctypes.byref(a), sv._stream()), "")
+    tiles = [p // 32 - max(0, p - window + 1) // 32 * (window > 0) + 1
+             for p in pos]
+    least = next(n for n in range(1, 100)
+                 if sum(-(-t // n) for t in tiles) <= rows * a.splits)
+    got = part[-2 * rows:].view(torch.int32).view(rows, 2).tolist()
+    at = 0
+    for t, (first, n) in zip(tiles, got):
+        assert (first, n) == (at, -(-t // least))
+        at += n
+    if equal and tiles[0] % a.splits == 0:
+        assert at == rows * a.splits
 
 
 @pytest.mark.parametrize("T", [3, 40, 70, 130])
