@@ -513,10 +513,13 @@ latent_rows_kernel(LatentRowsArgs a) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int it = i * 256 + tid;
-      if (FULL)                          // a tile is one piece
+      if (FULL) {                        // a tile is one piece
         reg[i] = *(const uint4v*)(src + it * 8u);
-      else
-        reg[i] = word(src + (uint)(it / CPR * RP), column(it % CPR));
+      } else {                           // (selects spill 18 registers)
+        const int k = column(it % CPR);
+        reg[i] = k < 0 ? uint4v{0, 0, 0, 0}
+                       : *(const uint4v*)(src + it / CPR * RP + k);
+      }
     }
     page = bt[min(t + 1, t1 - 1) / 2];
   };

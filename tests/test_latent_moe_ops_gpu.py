@@ -165,6 +165,7 @@ def test_latent_mixed_batch(sv, dtype):
 
 
 @pytest.mark.parametrize("H,R,P", [(3, 64, 64), (33, 72, 16), (2, 512, 64),
+                                   (2, 320, 64), (3, 384, 24),
                                    (5, 256, 40)])
 @pytest.mark.parametrize("rows", [1, 2, 9, 65, 130, 255, 300])
 @pytest.mark.parametrize("window", [0, 45])
