@@ -857,12 +857,15 @@ extern "C" int sv_latent_step(const LatentStepArgs* a, hipStream_t stream) {
   }
   if (launch_latent_rows(&a->rows, stream)) return 1;
   if (a->rows.splits == 1) return sv_head_linear(&a->values, 1, 0, stream);
+  // as few reads of the weights as leave no CU without a workgroup (88 rows of 8
+  // heads by 16: 48 workgroups)
+  const int H = a->rows.H;
 #define LM(RB)                                                           \
   latent_merge_kernel<RB, true>                                          \
-      <<<dim3(a->rows.H, (T + RB - 1) / RB), 512, 0, stream>>>(a->rows, a->values)
-  if (T <= 32) LM(4);
-  else if (T <= 64) LM(8);
-  else LM(16);
+      <<<dim3(H, (T + RB - 1) / RB), 512, 0, stream>>>(a->rows, a->values)
+  if (H * ((T + 15) / 16) >= 256) LM(16);
+  else if (H * ((T + 7) / 8) >= 256) LM(8);
+  else LM(4);
 #undef LM
   return (int)hipGetLastError();
 }

@@ -1386,11 +1386,13 @@ def _latent_rows_args(q, cache, rank, pos, seq, block_table, heads, scale,
                       window, max_keys, sink, out):
     """Arguments and the workspace that they point to.  Workgroups of 64 keys
     while CUs have none (1 row of 1000 keys: the whole step 28.1 us with 128,
-    24.9 with 64), then of 128 (8 of 4096: 32.5, with 64 35.7), and no merge for
-    up to 128 (43 rows of 82: 23.6, in two 28.7)."""
+    24.9 with 64), then of 128 (8 of 4096: 32.5, with 64 35.7).  A merge is not
+    worth its launch up to 128 keys (43 rows of 82: 23.6, in two 28.7), of more
+    than 32 workgroups up to 256 (94 rows of 192, 64 heads, no values behind
+    them: 17.6, in two 28.1; 58 of 178, 8 heads 25.2, in three 23.1)."""
     rows, D = q.shape[0], cache.shape[2]
     units = rows * -(-heads // 32)
-    splits = 1 if max_keys <= 128 else max(
+    splits = 1 if max_keys <= (256 if units > 32 else 128) else max(
         _row_splits(512, units, max_keys, 128),
         _row_splits(256, units, max_keys, 64))
     # sums, maxima and totals of every share; of every row, its shares

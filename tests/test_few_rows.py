@@ -169,3 +169,23 @@ def test_rotary_tables_hold_every_position():
             sv._check_rotary(*pair, q, k, pos, 64, 91)
     with pytest.raises(AssertionError):
         sv._check_rotary(cos, torch.zeros(90, 64), q, k, pos, 64, 90)
+
+
+@pytest.mark.parametrize("rows,heads,keys,want", [
+    # none merged: short rows, up to 256 keys of more than 32 workgroups
+    (1, 32, 128, 1), (1, 32, 129, 3), (32, 32, 256, 4), (33, 32, 256, 1),
+    (17, 64, 256, 1), (9, 128, 200, 1), (33, 8, 257, 5), (200, 64, 9000, 1),
+    # workgroups of 64 keys, then of 128
+    (1, 32, 1000, 16), (8, 32, 4096, 32), (32, 32, 4096, 16),
+    (256, 32, 9000, 2), (257, 32, 9000, 1)])
+def test_workgroups_of_a_latent_row(rows, heads, keys, want):
+    R, P = 64, 64
+    q = torch.zeros(rows, heads * (R + P), dtype=torch.bfloat16)
+    cache = torch.zeros(1, 64, R + P, dtype=torch.bfloat16)
+    i = torch.zeros(rows, dtype=torch.int32)
+    a, part = sv._latent_rows_args(q, cache, R, i, i, i.view(-1, 1), heads, 1.0,
+                                   0, keys, None, q)
+    assert a.splits == want
+    # the launcher takes no more workgroups of 32 heads, nor the workspace less
+    assert want == 1 or rows * want <= 512 and part.numel() == \
+        rows * want * heads * (R + 2) + 2 * rows
