@@ -482,9 +482,9 @@ latent_rows_kernel(LatentRowsArgs a) {
     if (FULL) return c;
     return c < EP ? (c < R ? c : -1) : (c - EP < P ? R + c - EP : -1);
   };
+  // (read in any case and zeroed behind, words of padding spill 18 registers)
   auto word = [&](const short* src, int k) {
-    const uint4v w = *(const uint4v*)(src + max(k, 0));
-    return k < 0 ? uint4v{0, 0, 0, 0} : w;
+    return k < 0 ? uint4v{0, 0, 0, 0} : *(const uint4v*)(src + k);
   };
   auto swz_slot = [](int r, int slot) {
     return slot ^ (CPR % 16 == 0 ? r & 15 : (r >> 1) & 7);
@@ -513,13 +513,10 @@ latent_rows_kernel(LatentRowsArgs a) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int it = i * 256 + tid;
-      if (FULL) {                        // a tile is one piece
+      if (FULL)                          // a tile is one piece
         reg[i] = *(const uint4v*)(src + it * 8u);
-      } else {                           // (selects spill 18 registers)
-        const int k = column(it % CPR);
-        reg[i] = k < 0 ? uint4v{0, 0, 0, 0}
-                       : *(const uint4v*)(src + it / CPR * RP + k);
-      }
+      else
+        reg[i] = word(src + it / CPR * RP, column(it % CPR));
     }
     page = bt[min(t + 1, t1 - 1) / 2];
   };
@@ -658,18 +655,77 @@ latent_rows_kernel(LatentRowsArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// merge: the shares of RB rows of a head, every row by two waves; LINEAR: then
-// the head's values of them (and their gate), whose weights are asked for first.
-// Two launches with the merged rows in memory took 13.4 us for 32 rows, 32 heads,
-// rank 512, this 11.5.
+// merge: the shares of a row and head, 64 V columns; four waves take every fourth
+// share.
 // ---------------------------------------------------------------------------
-template <int RB, bool LINEAR>
+template <int V>
+__global__ void __launch_bounds__(256) latent_merge_kernel(LatentRowsArgs a) {
+  __shared__ float coef[LATENT_SHARES], sum[4][64][V];
+  const int h = blockIdx.x % a.H, row = blockIdx.x / a.H;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int2 sh = row_shares(a)[row];    // first and number
+  if (wid == 0) {
+    const float2* ml = share_totals(a) + (long)sh.x * a.H + h;
+    auto total = [&](int s) {
+      return s + lane < sh.y ? ml[(long)(s + lane) * a.H] : float2{NEG_BIG, 0.f};
+    };
+    const float2 first = total(0);
+    float mm = first.x, l = 0.f;
+    for (int s = 64; s < sh.y; s += 64) mm = fmaxf(mm, total(s).x);
+    mm = fold64(mm, MaxOp());
+    for (int s = 0; s < sh.y; s += 64) {
+      const float2 v = s ? total(s) : first;
+      const float w = __builtin_amdgcn_exp2f(v.x - mm);
+      l += w * v.y;
+      coef[s + lane] = w;
+    }
+    l = fold64(l, SumOp());
+    for (int s = 0; s < sh.y; s += 64) coef[s + lane] *= 1.f / l;
+  }
+  __syncthreads();
+  const int e = (blockIdx.y * 64 + lane) * V;
+  float acc[V] = {};
+  if (e < a.R) {
+    const long step = (long)a.H * a.R;
+    const float* src = a.part + ((long)sh.x * a.H + h) * a.R + e;
+#pragma unroll 8
+    for (int s = wid; s < sh.y; s += 4) {
+      const float c = coef[s];
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[j] += c * src[s * step + j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < V; ++j) sum[wid][lane][j] = acc[j];
+  __syncthreads();
+  if (wid > 0 || e >= a.R) return;
+  short* out = a.out + ((long)row * a.H + h) * a.R + e;
+#pragma unroll
+  for (int j = 0; j < V; ++j)
+    acc[j] = sum[0][lane][j] + sum[1][lane][j] + sum[2][lane][j] + sum[3][lane][j];
+#pragma unroll
+  for (int j = 0; j < V; j += 2) *(uint*)(out + j) = pack_bf16x2(acc[j], acc[j + 1]);
+}
+
+static void launch_latent_merge(const LatentRowsArgs& a, hipStream_t stream) {
+  // as many columns a lane as fill a wave (128 rows of 4000 keys, 32 heads, rank 512,
+  // a whole step: 115 us in twos, 109 in fours)
+  const dim3 grid(a.rows * a.H, a.R <= 128 ? 1 : (a.R + 255) / 256);
+  if (a.R <= 128) latent_merge_kernel<2><<<grid, 256, 0, stream>>>(a);
+  else latent_merge_kernel<4><<<grid, 256, 0, stream>>>(a);
+}
+
+// ---------------------------------------------------------------------------
+// values: the shares of four rows of a head, every row by two waves, then the
+// head's values of them (and their gate), whose weights are asked for first.
+// ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(512)
-latent_merge_kernel(LatentRowsArgs a, HeadLinearArgs l) {
-  constexpr int XP = 512 + 8;            // pitch of merged rows
+latent_values_kernel(LatentRowsArgs a, HeadLinearArgs l) {
+  constexpr int RB = 4, XP = 512 + 8;    // rows; pitch of merged ones
   __shared__ __attribute__((aligned(16))) float other[4][512];
-  __shared__ __attribute__((aligned(16))) short xs[LINEAR ? 16 * XP : 8];
-  __shared__ __attribute__((aligned(16))) float ys[LINEAR ? 4 : 1][2][256];
+  __shared__ __attribute__((aligned(16))) short xs[16 * XP];
+  __shared__ __attribute__((aligned(16))) float ys[4][2][256];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int part = wid >> 2;             // of the shares, of the columns
@@ -694,17 +750,13 @@ latent_merge_kernel(LatentRowsArgs a, HeadLinearArgs l) {
     }
   };
   int n0 = (wid & 3) * 32;
-  if (LINEAR) {
-    weights(n0);
-    if (RB < 16)                         // rows that are none
-      for (int i = threadIdx.x * 8; i < (16 - RB) * XP; i += 512 * 8)
-        *(uint4v*)(xs + RB * XP + i) = uint4v{0, 0, 0, 0};
-  }
+  weights(n0);
+  for (int i = threadIdx.x * 8; i < (16 - RB) * XP; i += 512 * 8)  // rows that
+    *(uint4v*)(xs + RB * XP + i) = uint4v{0, 0, 0, 0};             //   are none
   const int e = lane * 8;
   const long step = (long)a.H * R;
-#pragma unroll
-  for (int rr = wid & 3; rr < RB; rr += 4) {
-    const int row = r0 + rr;
+  {
+    const int rr = wid & 3, row = r0 + rr;
     f32x4 acc[2] = {};
     float inv = 0.f;
     if (row < a.rows) {
@@ -758,15 +810,10 @@ latent_merge_kernel(LatentRowsArgs a, HeadLinearArgs l) {
                         pack_bf16x2(acc[0][2], acc[0][3]),
                         pack_bf16x2(acc[1][0], acc[1][1]),
                         pack_bf16x2(acc[1][2], acc[1][3])};
-      if (LINEAR) {
-        *(uint4v*)(xs + rr * XP + e) = w;  // zeros past R and past the last row
-      } else if (row < a.rows && e < R) {
-        *(uint4v*)(a.out + ((long)row * a.H + h) * R + e) = w;
-      }
+      *(uint4v*)(xs + rr * XP + e) = w;  // zeros past R and past the last row
     }
-    if (LINEAR || RB > 4) __syncthreads();
+    __syncthreads();
   }
-  if (!LINEAR) return;
   for (int n1 = 0; n1 < l.N; n1 += 128, n0 += 128) {
     if (n1 > 0) {
       __syncthreads();                   // ys has been read
@@ -826,8 +873,7 @@ extern "C" int sv_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
   if (a->rows <= 0) return 0;
   if (launch_latent_rows(a, stream)) return 1;
   if (a->splits > 1)
-    latent_merge_kernel<4, false>
-        <<<dim3(a->H, (a->rows + 3) / 4), 512, 0, stream>>>(*a, HeadLinearArgs{});
+    launch_latent_merge(*a, stream);
   return (int)hipGetLastError();
 }
 
@@ -857,15 +903,18 @@ extern "C" int sv_latent_step(const LatentStepArgs* a, hipStream_t stream) {
   }
   if (launch_latent_rows(&a->rows, stream)) return 1;
   if (a->rows.splits == 1) return sv_head_linear(&a->values, 1, 0, stream);
-  // as few reads of the weights as leave no CU without a workgroup (88 rows of 8
-  // heads by 16: 48 workgroups)
-  const int H = a->rows.H;
-#define LM(RB)                                                           \
-  latent_merge_kernel<RB, true>                                          \
-      <<<dim3(H, (T + RB - 1) / RB), 512, 0, stream>>>(a->rows, a->values)
-  if (H * ((T + 15) / 16) >= 256) LM(16);
-  else if (H * ((T + 7) / 8) >= 256) LM(8);
-  else LM(4);
-#undef LM
+  // The merge and the values in one launch read a head's weights for every four
+  // rows, 16 rows of products of which four are used: only rows of many columns,
+  // and one workgroup a CU or less, earn that (us of a step, in brackets in two
+  // launches: 32 rows of 4096 keys, 32 heads, rank 512 47.4 (48.2); 11 of 363, 64
+  // heads, rank 384 26.1 (27.0); but 5 of 4002, 40 heads, rank 448 33.5 (31.1), 92
+  // of 829, 64 heads, rank 128 63.9 (37.3)).
+  const int H = a->rows.H, groups = H * ((T + 3) / 4);
+  if (a->rows.R > 256 && groups >= 128 && groups <= 256) {
+    latent_values_kernel<<<dim3(H, (T + 3) / 4), 512, 0, stream>>>(a->rows, a->values);
+  } else {
+    launch_latent_merge(a->rows, stream);
+    return sv_head_linear(&a->values, 1, 0, stream);
+  }
   return (int)hipGetLastError();
 }
