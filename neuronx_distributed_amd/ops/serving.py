@@ -813,20 +813,23 @@ def _row_splits(target: int, units: int, max_keys: int, per: int) -> int:
 
 
 # Workgroups of the first form of ``rows_kernel`` to aim at, where up to so many
-# (row, key head) meet keys up to 256, 700, 1200, 2500, 5000 and more; 0 shares no
-# row.  One a CU (256) or less while rows are short: more meet on one CU and read
-# no faster.  Longer rows fill all 512 places, and of many rows there are several
-# rounds, so that unequal ones end together.  Over 740 sizes of 1 to 128 rows of
-# 32/32, 32/8 and 28/4 heads of 128, up to 12000 keys, equal and unequal, 1.8% over
-# the best number, where 1024 to 2048 above 700 keys were 8.6% (us then and now: 8
-# rows of 32/8 heads, 4000 keys 26.4, 21.3; 32, 1000: 26.6, 18.8; 64, 2000: 54.0,
-# 52.8; 128 rows of 28/4, 1000: 37.5, 28.4), up to 5% over it in 5 of them (45 rows of
-# 32/8, 2000 equal keys: 75.8, 77.7).
+# (row, key head) meet keys up to 256, 700, 1200, 2500, 5000 and more; 0 shares
+# no row.  One a CU (256) or less while rows are short: more meet on one CU and
+# read no faster.  Longer rows fill all 512 places, and of many rows there are
+# several rounds, so that unequal ones end together; up to 320 leave few CUs
+# with a second workgroup, which all wait for.  Over 1100 sizes of 1 to 128 rows
+# of 32/32, 32/8 and 28/4 heads of 128 and 64, up to 12000 keys, equal and
+# unequal, 2.4% over the best number, where 1024 to 2048 above 700 keys were
+# 8.6% (us then and now: 8 rows of 32/8 heads, 4000 keys 26.4, 21.3; 32, 1000:
+# 26.6, 18.8; 32 of up to 4096, in eight and in four 62.5, 61.5; 64, 2000: 54.0,
+# 52.8; 128 rows of 28/4, 1000: 37.5, 28.4).  Equal rows of a few more than 256
+# are up to 12% over it between 700 and 1200 keys (34 of 16/8, 1195: 33.0,
+# 37.1), where unequal ones gain as much.
 _SHARED_KEYS = (256, 700, 1200, 2500, 5000)
-_SHARED_UNITS = (64, 128, 255, 512)
+_SHARED_UNITS = (64, 128, 256, 320)
 _SHARED_ROWS = ((0, 256, 256, 256, 512, 512), (0, 512, 512, 512, 512, 768),
-                (0, 0, 0, 512, 1024, 1536), (0, 0, 0, 640, 2048, 2048),
-                (0, 0, 0, 1024, 2048, 2048))
+                (0, 0, 0, 512, 1024, 2048), (0, 0, 0, 1024, 2048, 2048),
+                (0, 0, 0, 0, 2048, 2048))
 
 
 def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
