@@ -687,7 +687,7 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   int page = 0;
   if (n < n1) {
     const int first = page_of(n);
-    page = page_of(n + 4);
+    if (n + 4 < n1) page = page_of(n + 4);
     issue(n, first, ka, v0);
   }
   if constexpr (ROT) {                   // while the first tile is on its way
@@ -722,13 +722,17 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   }
   for (; n < n1; n += 8) {
     arrived();
-    if (n + 4 < n1) issue(n + 4, page, kb, v1);
-    page = page_of(n + 8);
+    if (n + 4 < n1) {
+      issue(n + 4, page, kb, v1);
+      page = page_of(n + 8);
+    }
     attend(n, ka, v0);
     if (n + 4 >= n1) break;
     arrived();
-    if (n + 8 < n1) issue(n + 8, page, ka, v0);
-    page = page_of(n + 12);
+    if (n + 8 < n1) {
+      issue(n + 8, page, ka, v0);
+      page = page_of(n + 12);
+    }
     attend(n + 4, kb, v1);
   }
 

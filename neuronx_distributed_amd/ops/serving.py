@@ -7,10 +7,10 @@ library raises.  Activations and weights are bfloat16, or float32 in the
 gates and recurrent state are 32-bit in both.
 """
 
-import bisect
 import ctypes
 import math
 import os
+from bisect import bisect_left
 from dataclasses import dataclass, replace
 from typing import Optional, Sequence, Union
 
@@ -856,8 +856,8 @@ def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
             100 if units > (1024 if modified else 2048) else 64
     if units > 512 and 0 < max_keys <= short:
         return 1, _row_splits(1024, units, max_keys, 128)
-    target = _SHARED_ROWS[bisect.bisect_left(_SHARED_UNITS, units)][
-        bisect.bisect_left(_SHARED_KEYS, max_keys)]
+    target = _SHARED_ROWS[bisect_left(_SHARED_UNITS, units)][
+        bisect_left(_SHARED_KEYS, max_keys)]
     return 2, _row_splits(target, units, max_keys, 128)
 
 
