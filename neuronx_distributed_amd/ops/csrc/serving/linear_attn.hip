@@ -1376,7 +1376,10 @@ __global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
 // count.  Bound by latency: three workgroups share a CU, vector work fills 40 % of
 // the time, products 25 %.  2 x 2048 tokens, 128 heads of 128 x 64: tiles of 64
 // tokens, one ahead, with all words waited for at every barrier 129 us, now 117
-// (200 MB: 40).
+// (200 MB: 40).  Keys of 64 fitted four times on a CU before and fit three times:
+// calls of all kinds take 0.97 to 0.99 of the time then, at worst 1.04 (3052 tokens
+// and 1188 more, 80 heads of 64 x 64: 107 and 111 us); smaller tiles for four spill
+// 19 registers, 1.06.
 // The weights of an earlier group's keys are products: what is left at the end
 // of their group, and from there to the query.  The skip is part of a token's
 // weight on itself.
