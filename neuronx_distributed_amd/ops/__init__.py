@@ -9,6 +9,7 @@ implementations (the numerics baseline the GPU kernels are tested against).
 """
 
 import ctypes
+import functools
 import math
 import os
 from typing import Optional
@@ -473,6 +474,7 @@ def _fa_alloc_like(t):
     return torch.empty_like(t, memory_format=torch.contiguous_format)
 
 
+@functools.lru_cache(maxsize=256)         # (1.2 to 4.4 us otherwise)
 def _fa_dkv_heads(B: int, Hq: int, Hkv: int, S: int, causal: bool,
                   window: int) -> int:
     """Heads of dK and dV that the kernel writes: a workgroup adds up the q heads
