@@ -200,6 +200,30 @@ def test_flash_attn_bwd_sums_heads_in_a_workgroup(monkeypatch, Hq, Hkv, heads,
         assert err < 3 * 2 ** -8, (name, err)
 
 
+@pytest.mark.parametrize("pitch", [(1 << 25) - 8, 1 << 25])
+def test_flash_attn_of_rows_far_apart(pitch):
+    """Rows as far apart as 31 bits of bytes reach, and one word further, where
+    they are copied: the same bits as of rows that follow each other."""
+    torch.manual_seed(3)
+    S, D = 40, 128
+    near = [torch.randn(1, 1, S, D, device="cuda").bfloat16() for _ in range(4)]
+    # all four in the gaps of one another
+    room = torch.empty((S - 1) * pitch + 4 * D, dtype=torch.bfloat16,
+                       device="cuda")
+    far = []
+    for i, t in enumerate(near):
+        view = room[i * D:].as_strided((1, 1, S, D), (8, 8, pitch, 1))
+        far.append(view.copy_(t))
+
+    def run(q, k, v, dy):
+        q, k, v = (t.detach().requires_grad_() for t in (q, k, v))
+        out = ops.flash_attn(q, k, v, True, 0.09, 0)
+        return (out, *torch.autograd.grad(out, (q, k, v), dy))
+
+    for a, b in zip(run(*far), run(*near)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("row", [75, 199])
 @pytest.mark.parametrize("bad", [math.nan, math.inf, -math.inf])
 @pytest.mark.parametrize("causal,window", [(True, None), (True, 70),

@@ -178,6 +178,12 @@ def test_flash_stride_layout_helpers():
     bshd_view = torch.zeros(B, S, H, D).permute(0, 2, 1, 3)
     assert _fa_ok_layout(bhsd) and _fa_ok_layout(bshd_view)
     assert not _fa_ok_layout(torch.zeros(B, H, S, 2 * D)[..., ::2])
+    # bytes of 31 rows are offsets of 31 bits
+    for pitch, ok in (((1 << 25) - 8, True), (1 << 25, False)):
+        far = torch.empty(1, device="meta").as_strided((1, 2, 40, D),
+                                                       (8, 8, pitch, 1))
+        assert _fa_ok_layout(far) is ok
+        assert not ok or 31 * pitch * 2 + 255 < 1 << 31
 
     # layout preservation: BSHD view in -> BSHD storage out (the model's
     # downstream .transpose(1,2).reshape stays a view)

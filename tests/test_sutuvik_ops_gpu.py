@@ -546,6 +546,32 @@ def test_timed_memory_states_carried_and_scanned(monkeypatch, N, P, carried):
         _near(S[7 - i], S_want, F32, i, 2e-5)
 
 
+@pytest.mark.parametrize("pitch", [(1 << 22) - 8, 1 << 22])
+@pytest.mark.parametrize("carried", [True, False])
+def test_timed_memory_of_rows_far_apart(monkeypatch, pitch, carried):
+    """Chunks of rows as far apart as 31 bits of bytes reach, and one word
+    further, where the general form takes them."""
+    monkeypatch.setattr(sv, "memory_carries", lambda *a: carried)
+    H, G, N, P, T = 2, 1, 128, 64, 300
+    case = _ssm(T, H, G, N, P, 5, BF16)
+    params = _ssm_params(H, BF16)
+    want, S_want = _ssm_want(case, params, H, G, N, P)
+    room = torch.empty((T - 1) * pitch + 1024, dtype=BF16, device="cuda")
+    far, at = [], 0
+    for t in case[:4]:
+        view = room[at:].as_strided(t.shape, (pitch, 1))
+        far.append(view.copy_(t))
+        at += t.shape[1]
+    x, B, C, z = far
+    seg, chunks, first = _segments([(0, T, 0)])
+    S = torch.full((1, H, N, P), 7.0, device="cuda")
+    out = sv.memory_mix(C, B, x, sv.TimeGate(
+        case[4].cuda(), *[t.cuda() for t in params], z), S, None, None, seg, H,
+        chunks, first)
+    _near(out, want, BF16)
+    _near(S[0], S_want, F32, "state", 2e-5)
+
+
 def test_states_are_carried_where_that_is_faster():
     assert sv.memory_carries(17, 2, 128 * 128 * 64)      # 2 x 2048 tokens
     assert sv.memory_carries(4, 1, 64 * 128 * 64)        # 1000 tokens
