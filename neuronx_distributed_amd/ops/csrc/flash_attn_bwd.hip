@@ -97,14 +97,6 @@ __device__ __forceinline__ bf16x8 read_turned(char* lds, int lane_at, int c,
         (lds_tr4)(lds + (lane_at ^ (nb * 64 + u * 32)) + c * 4096 + u * 2048));
   return f.bf;
 }
-// two 16-row fragments of an accumulator, its rows as the contraction
-__device__ __forceinline__ void to_frags(const f32x16& x, frag_u* f) {
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      f[c].u[u] = pack_bf16x2(x[8 * c + 2 * u], x[8 * c + 2 * u + 1]);
-}
 // [d][lane] accumulators to a row of the lane
 __device__ __forceinline__ void store_turned(const f32x16* acc, float scale,
                                              short* dst, int hi) {

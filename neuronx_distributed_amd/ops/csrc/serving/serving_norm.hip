@@ -400,7 +400,9 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
       !a->branches && (!a->coef || (a->parts <= 8 && a->W <= 4096))) {
 #define FRX(R, D, X) \
   few_rows_norm_kernel<R, D, X><<<a->rows_out, 1024, 0, stream>>>(*a)
-#define FRN(R, D) do { if (a->x) FRX(R, D, true); else FRX(R, D, false); } while (0)
+  // (nothing pending: there is a residual)
+#define FRN(R, D) \
+  do { if (D == NONE || a->x) FRX(R, D, true); else FRX(R, D, D == NONE); } while (0)
 #define FR(D)                          \
   do {                                 \
     if (a->W <= 4096) FRN(1, D);       \
