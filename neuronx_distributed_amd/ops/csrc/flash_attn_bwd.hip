@@ -26,8 +26,9 @@
 // same wave, both directions took 1823 us instead of 1874 (2 x 4096, 32 heads: 986
 // for 1021); delta beside the dQ kernel's fragments of dO and the q heads of a kv
 // head in one workgroup 1790 (a kernel for delta 22, the sum over heads 31).
-// Bound by the matrix cores, 45 to 57 % busy at the 1.8 GHz that the
-// card holds under such work.
+// No unit alone bounds them: matrix cores are 57 % busy in dK/dV and 68 % in dQ, LDS 50
+// and 34 %, without bank conflicts.  Of the time of a wave of dK/dV 33 % are waits for
+// words and barriers (dQ 20 %), 27 % waits for a turn (37 %).
 
 #include "common.h"
 #include "mfma.h"

@@ -13,7 +13,7 @@
 //   32000 x 4096, 32 bit 1 row 59 | 42 | 48    4 rows 60 | 45 | 48   16: 60 | 64 | 51
 //   4096 x 14336         1 row 27 | 22 | -     4 rows 27 | 23 | -
 //   4096 x 4096          1 row 14 | 7.5 | 12  16 rows 14 | 10 | 14   32: 13 | 14 | 17
-// One row reads 4.5 to 5.7 TB/s of weights, a copy 5.1.  With a branch a load every
+// One row reads 4.1 (with its norm) to 6.4 TB/s of weights, a copy 5.1.  With a branch a load every
 // product waited for all loads on their way: 8.5, 23 and 45 us where one row of
 // 4096 x 4096, 4096 x 14336 and 28672 gated columns now take 7.5, 22 and 43.5.
 
