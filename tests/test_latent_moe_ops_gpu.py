@@ -241,6 +241,36 @@ def test_decoding_step_of_many_requests(sv, T, H, D, P, E, R):
     _close(got, want, dtype, 4.0, (T, H, D, P, E, R))
 
 
+@pytest.mark.parametrize("T,H,D,P,E,R,ctx", [
+    # merge and values in one: 128 to 256 workgroups of four rows of more than
+    # 256 columns; the last sizes on either side
+    (17, 32, 16, 64, 136, 320, 140), (31, 32, 8, 64, 12, 512, 140),
+    (13, 32, 8, 8, 260, 264, 140), (9, 64, 8, 64, 12, 512, 140),
+    (12, 32, 8, 64, 12, 512, 140), (32, 33, 8, 64, 12, 512, 300),
+    (17, 32, 8, 64, 12, 256, 140),
+    # many rows, merged one by one
+    (40, 3, 40, 8, 12, 40, 300), (70, 2, 16, 64, 136, 512, 300)])
+def test_decoding_step_of_shared_rows(sv, T, H, D, P, E, R, ctx):
+    """Single tokens of T requests, of unequal contexts, whose keys several
+    workgroups share."""
+    dtype = torch.bfloat16
+    at = [ctx - 9 * (i % 7) for i in range(T)]
+    cases = [_latent_case(sv, H, D, P, E, R, 0, ctx + 1, dtype, seed=9 * i)
+             for i in range(2)]
+    w, cfg = cases[0][3:5]
+    cache, bt = _cache([ctx + 1] * T, R + P, dtype)
+    for i in range(T):
+        q, kv, g = (t[:at[i]] for t in cases[i % 2][:3])
+        _run(sv, Batch(sv, [(i, 0, at[i])], bt, 0, False), q, kv, g, cache, w,
+             cfg)
+    b = Batch(sv, [(i, at[i], 1) for i in range(T)], bt, 0, False)
+    q, kv, g = (torch.cat([cases[i % 2][k][at[i]:at[i] + 1] for i in range(T)])
+                for k in range(3))
+    got = _run(sv, b, q, kv, g, cache, w, cfg)
+    want = torch.cat([cases[i % 2][5][at[i]:at[i] + 1] for i in range(T)])
+    _close(got, want, dtype, 4.0, (T, H, D, P, E, R))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [64, 70, 33, 128, 1, 65])
 def test_latent_window_edges_show(sv, window, dtype):
