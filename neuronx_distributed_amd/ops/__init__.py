@@ -722,12 +722,13 @@ def skinny_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def use_skinny_linear(inp: torch.Tensor, weight: torch.Tensor,
                       sequence_parallel_enabled: bool = False) -> bool:
-    """Is ``skinny_linear`` faster than the library for the rows of ``inp``, and
+    """Is ``skinny_linear`` faster than the library for the rows of ``inp`` (other
+    kernels than that may be: ``skinny_or_none``), and
     nobody in its way (autograd, tracing, modes, NXDA_SKINNY_GEMM=0)?"""
     from . import serving as sv
 
     return not sequence_parallel_enabled and \
-        sv.stream_how(inp, weight) is not None
+        sv.stream_how(inp, weight, rings=False) is not None
 
 
 def skinny_or_none(inp: torch.Tensor, weight: torch.Tensor,
@@ -735,7 +736,7 @@ def skinny_or_none(inp: torch.Tensor, weight: torch.Tensor,
                    glu: bool = False):
     """inp (.., K) @ weight (N, K)^T, or with ``glu`` silu(gate) * up of
     weight = [gate; up], by the weight-streaming kernels where they beat the
-    library (a few rows; ``serving.stream_rule``), else None."""
+    library (a few rows; ``serving.stream_how``), else None."""
     if torch.is_grad_enabled() or sequence_parallel_enabled:
         return None
     from . import serving as sv

@@ -6,16 +6,21 @@
 //                      whose first half of rows are gates, the second the
 //                      projections that they multiply
 //
-// Measured cold, us (library product, with the activation behind it | stream |
-// stay), which the rule of ops/serving.py follows:
-//   28672 x 4096 gated   1 row 66 | 46 | 44   16 rows 68 | 71 | 47   32: 60 | - | 51
-//   28672 x 4096         1 row 63 | 40 | 46    4 rows 64 | 43 | 46   16: 65 | 60 | 49
-//   32000 x 4096, 32 bit 1 row 59 | 42 | 48    4 rows 60 | 45 | 48   16: 60 | 64 | 51
-//   4096 x 14336         1 row 27 | 22 | -     4 rows 27 | 23 | -
-//   4096 x 4096          1 row 14 | 7.5 | 12  16 rows 14 | 10 | 14   32: 13 | 14 | 17
-// One row reads 4.1 (with its norm) to 6.4 TB/s of weights, a copy 5.1.  With a branch a load every
-// product waited for all loads on their way: 8.5, 23 and 45 us where one row of
-// 4096 x 4096, 4096 x 14336 and 28672 gated columns now take 7.5, 22 and 43.5.
+// Bound by reading the weights: a read of 235 MB that multiplies nothing takes 36.0 us,
+// of 34 MB 7.1, of which 1.7 are a launch.  Measured cold, us (library product, with
+// the activation behind it | stream | stay | rings, x kept or flowing), which the rules
+// of ops/serving.py follow:
+//   28672 x 4096 gated   1 row 62 | - | 45 | 38.5   16 rows 63 | - | 47 | 39.4   32: 51 | - | 52 | 41.1
+//   32000 x 4096, 32 bit 1 row 59 | 43 | 48 | 42.5  16 rows 59 | 62 | 52 | 43.3  32: 58 | 93 | 55 | 46.4
+//   6144 x 4096          1 row 14 | 12 | 16 | 11.1  16 rows 16 | 17 | 18 | 11.5  32: 16 | 25 | 21 | 13.7
+//   4096 x 4096          1 row 15 | 7.7 | 12 | 7.7  16 rows 15 | 10 | 14 | 8.5   32: 14 | 14 | 18 | 11.1
+//   4096 x 14336         1 row 27 | 23 | - | 21     16 rows 27 | 32 | - | 25     32: 34 | 43 | - | 33
+// A gated product of a normed row: 43.3 us staying, 37.5 through a ring.
+// Rings are the faster ones for three reasons, measured by reads alone: loads of whole
+// lines (64 of 128 bytes a load: 5.6 TB/s of 235 MB, 128: 6.0), lines that no cache
+// keeps (6.5; with halves of a line it reads them twice, 5.5), and as many of them on
+// their way as LDS holds instead of registers.
+// 64 KB a CU are enough: twice as many cost small weights 10 %.
 
 #include "serving.h"
 #include "words.h"
@@ -41,10 +46,10 @@ enum Epilogue { PLAIN = 0, F32 = 1, GLU = 2 };
 // Accumulator rows are weight rows 4 grp + 0..3, columns rows of x: the results
 // of weight rows n ... of row t.  u: what the gates v multiply.
 template <int EPI>
-__device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n,
+__device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n, int n1,
                                            f32x4 v, f32x4 u) {
   const int N = EPI == GLU ? a.N / 2 : a.N;
-  if (t >= a.T || n >= N) return;
+  if (t >= a.T || n >= n1) return;
   if (EPI == GLU)
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = silu_f(v[r]) * u[r];
@@ -70,6 +75,11 @@ __device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n,
 __device__ __forceinline__ bf16x8 if_there(bool in, frag_u f) {
   if (!in) f.u4 = uint4v{0, 0, 0, 0};
   return f.bf;
+}
+
+// A barrier for what is in LDS: it waits for no load.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // The normed row, in LDS, by NT threads.  Every workgroup makes it for itself while
@@ -106,7 +116,7 @@ __device__ __forceinline__ void norm_row(const StreamArgs& a, short* row,
   }
   sq = fold64(sq, SumOp());
   if ((tid & 63) == 0) red[tid >> 6] = sq;
-  __syncthreads();
+  lds_barrier();
   float all = 0.f;
 #pragma unroll
   for (int k = 0; k < NT / 64; ++k) all += red[k];
@@ -119,7 +129,7 @@ __device__ __forceinline__ void norm_row(const StreamArgs& a, short* row,
       y[j] = i < a.K ? v[k][j] * (rstd * bits2f(u[k][j])) : 0.f;
     store4(row + i + 4 * k, y);
   }
-  __syncthreads();
+  lds_barrier();
 }
 
 // One workgroup = 16 weight rows by MT tiles of 16 rows of x; its 16 waves take
@@ -217,18 +227,18 @@ __global__ void __launch_bounds__(1024) stream_linear_kernel(StreamArgs a) {
   for (int s = 0; s < 16; ++s) y[s] = part[s][wid][lane];
 #pragma unroll
   for (int s = 0; s < 16; ++s) v += y[s];
-  store_rows<EPI>(a, t0 + wid * 16 + c16, n0 + 4 * grp, v, v);
+  store_rows<EPI>(a, t0 + wid * 16 + c16, n0 + 4 * grp, a.N, v, v);
 }
 
 // For weights of many rows: a workgroup stays and takes every so many tiles of
 // 16 weight rows (or 16 gates and their projections).  Each of its NW waves
 // keeps its 256 PARTS columns of x in registers and reads the same columns of
 // one tile after the other, 256 at a time, one such part ahead.
-// FULL: K is what they hold.  Otherwise words past it are zeros behind a branch
-// each, and a product waits for all loads on their way (zeros made of words that
-// are read in any case do not fit the registers).
+// Words past K are zeros behind a branch each, and a product waits for all loads on
+// their way (zeros made of words that are read in any case do not fit the registers):
+// whole blocks of 64 columns come through rings instead.
 // NORM: of the normed row.
-template <int NW, int PARTS, int MT, int EPI, bool FULL, bool NORM>
+template <int NW, int PARTS, int MT, int EPI, bool NORM>
 __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   constexpr int RT = EPI == GLU ? 2 : 1;
   constexpr int UNITS = RT * PARTS;      // parts of a tile
@@ -241,8 +251,8 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   const int tiles = a.N / (16 * RT), step = gridDim.x;
   const int k0 = wid * PARTS * 256 + grp * 8;
   auto word = [&](const short* from, int k) __attribute__((always_inline)) {
-    return FULL || k0 + k < a.K ? *(const uint4v*)(from + k0 + k)
-                                : uint4v{0, 0, 0, 0};
+    return k0 + k < a.K ? *(const uint4v*)(from + k0 + k)
+                        : uint4v{0, 0, 0, 0};
   };
 
   frag_u fx[PARTS * 8][MT];
@@ -295,7 +305,7 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
     };
     sum(wid, v);
     if (EPI == GLU) sum(MT + wid, u);
-    store_rows<EPI>(a, wid * 16 + c16, tile * 16 + 4 * grp, v, u);
+    store_rows<EPI>(a, wid * 16 + c16, tile * 16 + 4 * grp, EPI == GLU ? a.N / 2 : a.N, v, u);
   };
 
   frag_u wa[8], wb[8];
@@ -327,6 +337,270 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   }
 }
 
+// Weights through LDS: a workgroup takes an even share of the weight rows (8 at a
+// time, so that no CU has much more than another), 16 rows a tile (8 gates and their
+// projections); each of its 8 waves takes its columns of the tile, 64 at a time, from a
+// ring of its own of R pieces of 8 rows by 64 columns.  Loads that hold no
+// register and wait for nobody fill it: tiles end, sums meet, and the ring goes on.
+template <int R, int EPI>
+struct Ring {
+  static constexpr int NW = 8, TR = EPI == GLU ? 8 : 16, UT = TR / 8;
+  int rows, full, u0, u1, tiles;         // whole tiles, then units of 8 rows of the last
+  int first, nb;                         // the wave's blocks of 64 columns
+  __amdgpu_buffer_rsrc_t ra, rb;
+  int oa, ob, pitch;
+  char* mine;
+  int tile, begin, blk, slot;            // what is asked for next, and its place
+  uint ta, tb;
+  int src0, src1, rd;
+
+  __device__ __forceinline__ Ring(const StreamArgs& a, char* ring, int wid,
+                                  int rotate = 0) {
+    const int lane = threadIdx.x & 63, c16 = lane & 15, grp = lane >> 4;
+    rows = EPI == GLU ? a.N / 2 : a.N;
+    const int units = (rows + 7) / 8, G = gridDim.x, b = blockIdx.x;
+    full = units / (UT * G);
+    const int rest = units - full * UT * G;
+    u0 = rest * b / G + full * UT * G;
+    u1 = rest * (b + 1) / G + full * UT * G;
+    tiles = full + (u1 > u0);
+    const int blocks = a.K / 64;
+    first = blocks * wid / NW;
+    nb = blocks * (wid + 1) / NW - first;
+    // Pieces past the last row are not read: they lie past the end of the buffer.
+    pitch = (int)a.wst * 2;
+    const int end = (rows - 1) * pitch + a.K * 2;
+    ra = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, 0, end, 0x00027000);
+    rb = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(EPI == GLU ? a.w + rows * a.wst : a.w), 0, end, 0x00027000);
+    // A piece has 8 slots of 16 bytes a row; slot s of row r lies at place s ^ r (of
+    // the second piece s ^ r ^ 1), so that 16 rows of one slot touch every bank once.
+    const int pr = lane >> 3, ps = (lane & 7) ^ pr;
+    oa = pr * pitch + ps * 16 + first * 128;
+    ob = (EPI == GLU ? pr : pr + 8) * pitch + (ps ^ 1) * 16 + first * 128;
+    mine = ring + wid * R * 1024;
+    tile = slot = rd = 0;
+    blk = begin = rotate ? blockIdx.x / rotate % nb : 0;
+    locate();
+    const int r8 = c16 & 7, turn = c16 >> 3;
+    src0 = (int)(size_t)(lds_ptr)mine + turn * 1024 + r8 * 128 +
+           ((grp ^ r8 ^ turn) & 7) * 16;
+  }
+  // first row of a tile, and past its last one
+  __device__ __forceinline__ int row0(int t) const {
+    return t < full ? (t * (int)gridDim.x + (int)blockIdx.x) * TR : 8 * u0;
+  }
+  __device__ __forceinline__ int row1(int t) const {
+    return min(rows, t < full ? row0(t) + TR : 8 * u1);
+  }
+  __device__ __forceinline__ void locate() {
+    ta = tile < tiles ? (uint)row0(tile) * pitch : 1u << 31;
+    tb = EPI != GLU && tile == full && u1 - u0 < 2 ? 1u << 31 : ta;
+  }
+  // the next block's two pieces.  Not kept in the caches (each is read once: 235 MB in
+  // 40.0 us, so 36.0).
+  __device__ __forceinline__ void ask() {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(mine + slot), 16,
+                                             oa + ta + blk * 128, 0, 0, 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(mine + slot + 1024), 16,
+                                             ob + tb + blk * 128, 0, 0, 2);
+    slot = (slot + 2048) & (R * 1024 - 1);
+    if (++blk == nb) blk = 0;
+    if (blk == begin) {
+      ++tile;
+      locate();
+    }
+  }
+  // The oldest block, when no more than AFTER loads are on their way behind it.
+  template <int AFTER>
+  __device__ __forceinline__ void take(frag_u& f0, frag_u& f1) {
+    asm volatile("s_waitcnt vmcnt(%4)\n\t"
+                 "ds_read_b128 %0, %2\n\t"
+                 "ds_read_b128 %1, %3\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(f0.u4), "=&v"(f1.u4)
+                 : "v"(src0 + rd), "v"((src0 ^ 64) + rd), "n"(AFTER)
+                 : "memory");
+    rd = (rd + 2048) & (R * 1024 - 1);
+  }
+};
+
+// the sums of a tile's waves meet; the first waves add them up
+template <int MT, int EPI>
+__device__ __forceinline__ void meet(const StreamArgs& a, f32x4 (*part)[MT][64],
+                                     const f32x4* acc, int wid, int n, int n1) {
+  constexpr int NW = 8;
+  const int lane = threadIdx.x & 63, c16 = lane & 15, grp = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) part[wid][j][lane] = acc[j];
+  lds_barrier();
+  if (wid >= MT) return;
+  f32x4 v = {}, p[NW], u;
+#pragma unroll
+  for (int s = 0; s < NW; ++s) p[s] = part[s][wid][lane];
+#pragma unroll
+  for (int s = 0; s < NW; ++s) v += p[s];
+  if (EPI == GLU)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = __shfl_xor(v[r], 32, 64);
+  if (EPI != GLU || grp < 2) store_rows<EPI>(a, wid * 16 + c16, n + 4 * grp, n1, v, u);
+}
+
+// Rows of x as fragments.  A fragment's neighbouring lanes have different rows, and a
+// load of it would look up a cache line a lane; neighbours in fours read 64 bytes of
+// a row instead, and hand them on.
+__device__ __forceinline__ const short* row_words(const StreamArgs& a, int j) {
+  const int lane = threadIdx.x & 63;
+  return a.x + (long)min(j * 16 + (lane >> 2), a.T - 1) * a.xst + (lane & 3) * 8;
+}
+__device__ __forceinline__ frag_u turned(frag_u f) {
+  const int lane = threadIdx.x & 63, from = ((lane & 15) * 4 + (lane >> 4)) * 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f.u[i] = __builtin_amdgcn_ds_bpermute(from, f.u[i]);
+  return f;
+}
+
+// The wave's columns of x stay in registers, at most CB blocks of 64.
+template <int CB, int MT, int EPI>
+__global__ void __launch_bounds__(512) ring_linear_kernel(StreamArgs a) {
+  constexpr int R = 8;
+  __shared__ __attribute__((aligned(1024))) char ring[8 * R * 1024];
+  __shared__ f32x4 part[2][8][MT][64];
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Ring<R, EPI> w(a, ring, wid);
+  const int nb = w.nb;
+  frag_u fx[CB * 2][MT];
+#pragma unroll
+  for (int i = 0; i < R / 2; ++i) w.ask();
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const short* x = row_words(a, j) + w.first * 64;
+#pragma unroll
+    for (int c = 0; c < CB * 2; ++c)     // blocks past the wave's are not used
+      fx[c][j].u4 = *(const uint4v*)(x + (c < 2 * nb ? c * 32 : 0));
+  }
+#pragma unroll
+  for (int c = 0; c < CB * 2; ++c)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) fx[c][j] = turned(fx[c][j]);
+  // x, and the ring is full: from here on only pieces (and results) are on their way
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  for (int t = 0; t < w.tiles; ++t) {
+    f32x4 acc[MT] = {};
+#pragma unroll
+    for (int c = 0; c < CB; ++c) {
+      if (c >= nb) continue;
+      frag_u f0, f1;
+      w.template take<R - 2>(f0, f1);
+      w.ask();
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        acc[j] = mfma16(f0.bf, fx[2 * c][j].bf, acc[j]);
+        acc[j] = mfma16(f1.bf, fx[2 * c + 1][j].bf, acc[j]);
+      }
+    }
+    meet<MT, EPI>(a, part[t & 1], acc, wid, w.row0(t), w.row1(t));
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // LDS is given back
+}
+
+// x flows like the weights, a ring ahead: for few rows, where it is little, and for a
+// workgroup's only tile, where there is nothing to keep.  Workgroups of an XCD begin at
+// different blocks, so that they do not all ask the same channels of its L2 for x
+// (16 rows of 14336: 26.9 us in one order, 23.8).
+// NORM: of the normed row, in LDS.
+template <int MT, int EPI, bool NORM>
+__global__ void __launch_bounds__(512) flow_linear_kernel(StreamArgs a) {
+  constexpr int D = 4, R = 2 * D;        // blocks ahead
+  __shared__ __attribute__((aligned(1024))) char ring[8 * R * 1024];
+  __shared__ f32x4 part[2][8][MT][64];
+  __shared__ __attribute__((aligned(16))) short row[NORM ? 4096 : 8];
+  __shared__ float red[NORM ? 16 : 1];
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Ring<R, EPI> w(a, ring, wid, 8);
+  const int nb = w.nb;
+  frag_u fx[D][2][MT];
+  const short* x[MT];
+  if (!NORM)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) x[j] = row_words(a, j) + w.first * 64;
+  // pieces and words of the wave's next block
+  auto ask = [&](int i) __attribute__((always_inline)) {
+    if (!NORM) {
+      const int k = w.blk * 64;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          fx[i][h][j].u4 = *(const uint4v*)(x[j] + k + h * 32);
+    }
+    w.ask();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int rb = w.begin;                      // block that is multiplied next
+  auto fill = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) ask(i);
+  };
+  if (NORM) norm_row<512>(a, row, red, fill);
+  else fill();
+  f32x4 acc[MT] = {};
+  int c = 0, t = 0;
+  const int total = w.tiles * nb;
+  for (int s = 0; s < total; s += D) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      frag_u f0, f1;
+      w.template take<(D - 1) * (NORM ? 2 : 2 * MT + 2)>(f0, f1);
+      if (NORM) {
+        const short* at = row + (w.first + rb) * 64 + ((threadIdx.x & 63) >> 4) * 8;
+        fx[i][0][0].u4 = *(const uint4v*)at;
+        fx[i][1][0].u4 = *(const uint4v*)(at + 32);
+        if (++rb == nb) rb = 0;
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        acc[j] = mfma16(f0.bf, (NORM ? fx[i][0][j] : turned(fx[i][0][j])).bf, acc[j]);
+        acc[j] = mfma16(f1.bf, (NORM ? fx[i][1][j] : turned(fx[i][1][j])).bf, acc[j]);
+      }
+      ask(i);
+      if (++c == nb && t < w.tiles) {    // past the last tile nothing counts
+        meet<MT, EPI>(a, part[t & 1], acc, wid, w.row0(t), w.row1(t));
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[j] = f32x4{};
+        c = 0;
+        ++t;
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // LDS is given back
+}
+
+template <int EPI, bool NORM = false>
+static int launch_ring(const StreamArgs& a, int how, hipStream_t stream) {
+  // every wave has a block, all offsets are bytes of 31 bits
+  if (a.K % 64 || a.K < 512 || a.wst * 2 * (a.N + 16L) >= 1L << 31 || a.T > 32 ||
+      (EPI == GLU && a.N % 8))
+    return 1;
+  const int units = ((EPI == GLU ? a.N / 2 : a.N) + 7) / 8;
+  const int grid = min(units, 256), blocks = (a.K / 64 + 7) / 8;
+#define RING(C, M) ring_linear_kernel<C, M, EPI><<<grid, 512, 0, stream>>>(a)
+#define FLOW(M) flow_linear_kernel<M, EPI, NORM><<<grid, 512, 0, stream>>>(a)
+  if constexpr (NORM) {
+    FLOW(1);
+  } else if (how == 3) {
+    if (a.T <= 16) FLOW(1); else FLOW(2);
+  } else {                               // at most 128 registers of x
+    if (a.T <= 16 && blocks <= 8) RING(8, 1);
+    else if (a.T <= 16 && blocks <= 16) RING(16, 1);
+    else if (blocks <= 8) RING(8, 2);
+    else return 1;
+  }
+#undef RING
+#undef FLOW
+  return (int)hipGetLastError();
+}
+
 template <int EPI, bool NORM = false>
 static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
   constexpr int rows = EPI == GLU ? 32 : 16;
@@ -336,15 +610,8 @@ static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
     const int grid = min(tiles, 256);
     // at most 128 registers of x beside the weights (plain products of 17 to
     // 32 rows by a direct call alone, here and below: the library is faster)
-#define STAY(P, M)                                                          \
-  do {                                                                      \
-    if (a.K == 2048 * P)                                                    \
-      stay_linear_kernel<8, P, M, EPI, true, NORM>                          \
-          <<<grid, 512, 0, stream>>>(a);                                    \
-    else                                                                    \
-      stay_linear_kernel<8, P, M, EPI, false, NORM>                         \
-          <<<grid, 512, 0, stream>>>(a);                                    \
-  } while (0)
+#define STAY(P, M) \
+  stay_linear_kernel<8, P, M, EPI, NORM><<<grid, 512, 0, stream>>>(a)
     if constexpr (NORM) STAY(2, 1);
     else if (a.T <= 16 && a.K <= 4096) STAY(2, 1);
     else if (a.T <= 16 && a.K <= 8192) STAY(4, 1);
@@ -367,17 +634,20 @@ static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-// K, strides and bases in 8 elements; GLU stays, on whole tiles
-extern "C" int sv_stream_linear(const StreamArgs* a, int epilogue, int stay,
+// how: 0 stream, 1 stay, 2 and 3 rings (K in blocks of 64, at least 512; 2: at most
+// 8192 columns of 16 rows or 4096 of 32).  K, strides and bases in 8 elements; GLU
+// not 0, on whole tiles
+extern "C" int sv_stream_linear(const StreamArgs* a, int epilogue, int how,
                                 hipStream_t stream) {
   if (a->T <= 0 || a->N <= 0) return 0;
   if (a->K % 8) return 1;
-  if (a->weight) {
-    if (a->T != 1 || a->K > 4096 || epilogue == F32) return 1;
-    return epilogue == GLU ? launch<GLU, true>(*a, stay, stream)
-                           : launch<PLAIN, true>(*a, stay, stream);
-  }
-  return epilogue == GLU   ? launch<GLU>(*a, stay, stream)
-         : epilogue == F32 ? launch<F32>(*a, stay, stream)
-                           : launch<PLAIN>(*a, stay, stream);
+  if (a->weight && (a->T != 1 || a->K > 4096 || epilogue == F32)) return 1;
+#define TAKE(E, ...)                                              \
+  (how >= 2 ? launch_ring<E, ##__VA_ARGS__>(*a, how, stream)      \
+            : launch<E, ##__VA_ARGS__>(*a, how, stream))
+  if (a->weight) return epilogue == GLU ? TAKE(GLU, true) : TAKE(PLAIN, true);
+  return epilogue == GLU   ? TAKE(GLU)
+         : epilogue == F32 ? TAKE(F32)
+                           : TAKE(PLAIN);
+#undef TAKE
 }

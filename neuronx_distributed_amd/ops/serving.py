@@ -238,7 +238,7 @@ class _ChunkArgs(ctypes.Structure):
 
 def stream_rule(T: int, N: int, K: int, f32: bool = False,
                 glu: bool = False) -> Optional[int]:
-    """How T rows x (T, K) meet a large weight (N, K): 0 every workgroup
+    """How T rows x (T, K) meet a large weight (N, K) without rings: 0 every workgroup
     streams its weight rows and all of x, 1 workgroups stay with x in registers,
     None the library's product is as fast.  The library reads weights at 2.5 to
     6 TB/s, by their sizes; the lines were drawn where it was not the faster one
@@ -304,6 +304,49 @@ def stream_rule(T: int, N: int, K: int, f32: bool = False,
     return 0 if T <= most else None
 
 
+def ring_rule(T: int, N: int, K: int, f32: bool = False,
+              glu: bool = False) -> Optional[int]:
+    """The same for weights that come through rings in LDS, whole cache lines of a
+    row at a time that no cache keeps: 2 workgroups stay with x in registers, 3 x
+    flows too, None neither is the faster one.  Drawn over 982 sizes (N
+    512..151936, K 512..28672, 1, 4, 16 and 32 rows) against the faster of the
+    library and what ``stream_rule`` takes; us here, that and the rings':
+
+    - x is little up to 8 rows, and read once where a CU has one tile of 16 weight
+      rows: there it flows (16 rows of 4096 x 4096: staying 9.4, flowing 8.8);
+      elsewhere staying saves its way through the L2 (28672 x 4096 gated, 16 rows:
+      flowing 44.0, staying 41.3; 32 rows: 61, 43), but of short rows, whose
+      workgroups have begun when x is there (7168 x 1024, 16 rows: 10.2, 9.0);
+    - short rows of small weights are streamed with 16 waves a workgroup, which
+      begin and end sooner (2048 x 2048, 1 row: 4.7, 5.0; 8192 x 2048: 7.5, 8.7;
+      32000 x 2048: 21.8, 23.7);
+    - 17 rows and more stay in registers up to K = 4096 (not of small weights where
+      only 5 blocks of 64 columns a wave cover the start: 6144 x 2560, 32 rows: 11.4,
+      12.0), and flow for one tile a CU (4096 x 11008, 32 rows: 31.5, 26.5); else
+      the library's are faster (32000 x 5120, 32 rows: 48, 73), as of a K that it
+      takes in even pieces (3072 x 14336: 28.6, 30.6)."""
+    if K % 64 or K < 512 or glu and N % 32:
+        return None
+    tiles = -(-N // 16)                  # 256 a round
+    if T <= 16:
+        if not glu and (T <= 4 and K <= 2048 and (
+                N <= 8192 or T == 1 and K > 1536) or
+                T == 1 and K <= 3584 and N <= 8192 or
+                T <= 4 and K <= 3072 and N <= 4096 or
+                T > 4 and K <= 1536 and N <= 8192):
+            return None
+        if T <= 8 or tiles <= 256 or K <= 1024 and tiles <= 1024 or \
+                K <= 2048 and tiles <= 512:
+            return 3
+        return 2 if K <= 8192 else None if K >= 14336 else 3
+    if tiles <= 512 and K <= 2048:
+        return 3
+    if K <= 4096:
+        return None if N < 1024 or 2048 < K < 3072 and 2048 < N < 8192 else 2
+    return None if glu or tiles > 256 or \
+        K < 16384 and K % 2048 == 0 and N > 2048 else 3
+
+
 def stream_linear(x: torch.Tensor, w: torch.Tensor, stay: int = 0,
                   f32: bool = False, glu: bool = False) -> torch.Tensor:
     """x (T, K) @ w (N, K)^T, bfloat16, with the sums rounded once or not at
@@ -333,9 +376,9 @@ def _plain(t) -> bool:
 
 
 def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
-               glu: bool = False) -> Optional[int]:
+               glu: bool = False, rings: bool = True) -> Optional[int]:
     """How ``stream_linear`` takes the rows of x (..., K) where it is the faster
-    one; None elsewhere, under autograd, and where somebody else watches the
+    one (by ``ring_rule``, if ``rings``, or ``stream_rule``); None elsewhere, under autograd, and where somebody else watches the
     operations (tracing, dispatch modes, autocast).  NXDA_SKINNY_GEMM=0 keeps
     every product on the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
@@ -349,7 +392,10 @@ def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
             w.stride(1) != 1 or w.device != x.device or \
             x.device.index != torch.cuda.current_device():
         return None
-    how = stream_rule(T, w.shape[0], K, f32, glu)
+    how = ring_rule(T, w.shape[0], K, f32, glu) if rings and \
+        w.stride(0) * (w.shape[0] + 16) < 1 << 30 else None
+    if how is None:
+        how = stream_rule(T, w.shape[0], K, f32, glu)
     if how is None or not available() or not _unwatched():
         return None
     rows = x.reshape(T, K)

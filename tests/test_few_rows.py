@@ -193,3 +193,21 @@ def test_workgroups_of_a_latent_row(rows, heads, keys, want):
     # the launcher takes no more workgroups of 32 heads, nor the workspace less
     assert want == 1 or rows * want <= 512 and part.numel() == \
         rows * want * heads * (R + 2) + 2 * rows
+
+
+def test_every_ring_is_one_that_the_launcher_takes():
+    """Blocks of 64 columns, one a wave at least; x in registers up to 8192
+    columns of 16 rows or 4096 of 32; whole words of gated results."""
+    taken = set()
+    for T in range(1, 33):
+        for N in SIZES:
+            for K in SIZES + (512 + 64, 4096 + 64, 11008):
+                for f32, glu in ((False, False), (True, False), (False, True)):
+                    how = sv.ring_rule(T, N, K, f32, glu)
+                    taken.add(how)
+                    if how is None:
+                        continue
+                    assert K % 64 == 0 and K >= 512 and not (glu and N % 8)
+                    if how == 2:
+                        assert K <= (8192 if T <= 16 else 4096)
+    assert taken == {None, 2, 3}

@@ -719,6 +719,34 @@ def test_products_of_few_rows(T, N, K, how):
             atol=tol * 16)
 
 
+@pytest.mark.parametrize("T,N,K,how", [
+    (1, 8, 512, 3), (1, 1001, 576, 3), (4, 4112, 4096, 3), (16, 4100, 14336, 3),
+    (17, 520, 1088, 3), (32, 2056, 11008, 3), (9, 16, 512, 2), (16, 8200, 576, 2),
+    (5, 6144, 4096, 2), (16, 1001, 8192, 2), (17, 24, 960, 2), (32, 8216, 4096, 2)])
+def test_products_of_few_rows_through_rings(T, N, K, how):
+    """The same: waves of unequal numbers of blocks, more blocks than the ring has
+    and fewer, whole tiles, one of 8 rows last, and rows past the last; weights of
+    infinities and no numbers beside them are not read."""
+    torch.manual_seed(T + N + K)
+    x = torch.randn(T, K + 8, device="cuda").bfloat16()[:, :K]
+    wide = torch.full((N + 32, K + 24), float("nan"), device="cuda",
+                      dtype=torch.bfloat16)
+    w = wide[:N, :K]
+    w.copy_(torch.randn(N, K, device="cuda").div(K ** 0.5))
+    ref = x.double() @ w.double().t()
+    tol = 16 * K ** 0.5 * 2.0 ** -24       # as above
+    out = sv.stream_linear(x, w, how, f32=True)
+    torch.testing.assert_close(out.double(), ref, rtol=0, atol=tol)
+    torch.testing.assert_close(sv.stream_linear(x, w, how).double(), ref,
+                               rtol=2.0 ** -8, atol=tol)
+    if N % 8 == 0:
+        gate, up = ref[:, :N // 2], ref[:, N // 2:]
+        torch.testing.assert_close(
+            sv.stream_linear(x, w, how, glu=True).double(),
+            torch.nn.functional.silu(gate) * up, rtol=2.0 ** -8,
+            atol=tol * 16)
+
+
 @pytest.mark.parametrize("glu", [False, True])
 def test_few_rows_are_streamed_where_nobody_watches(glu):
     x = torch.randn(2, 3, 4096, device="cuda").bfloat16()
