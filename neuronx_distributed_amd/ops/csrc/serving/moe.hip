@@ -12,7 +12,7 @@
 // down reads the slot and writes the pair; the weighted sum over a row's
 // pairs is taken by the residual norm.
 
-#include "serving.h"
+#include "ring.h"
 
 #define MOE_MAX_EXPERTS 512
 
@@ -567,16 +567,16 @@ moe_tiles_kernel(MoeGemmArgs a) {
 }
 
 // -- a few rows per expert: stream the weights --------------------------------
-// Weights go from memory straight into registers as fragments, a lane's 16
-// bytes of a row, and meet up to 32 slots of x (16 and less leave the second
-// half out).  A unit is 16 weight rows (16 gates and their 16 up rows) of one
-// slot tile.  Bound by reading the weights.  Plan and two products, us (4 waves
-// that share 32 weight rows, nothing read ahead | now; 32-slot tiles):
-//   64 experts 2048 x 1408, top 6   1 row  46 |  42    8: 156 | 127   32: 279 | 216
-//   64 and 192 rows, on tiles              252 | 236         286 | 236
-//   8 experts 4096 x 14336, top 2   1 row 187 | 140    8: 613 | 464
-//   32 and 64 rows, on tiles               613 | 542         635 | 608
-// 32 rows read 1.07 GB of 64 experts at 5.3 TB/s.
+// Weights meet up to 32 slots of x (16 and less leave the second half out), through
+// rings in LDS where K is whole blocks of 64 columns, else from memory straight into
+// registers as fragments, a lane's 16 bytes of a row.  A unit is 16 weight rows (8 or
+// 16 gates and their up rows) of one slot tile.  Bound by reading the weights, at 6.5
+// to 6.7 TB/s through rings (a read alone: 6.9).  Both products, us (through registers
+// | rings; 32-slot tiles):
+//   64 experts 2048 x 1408, top 6   1 row  30 |  23    8: 108 |  95   32: 199 | 165
+//   128: 219 | 175
+//   8 experts 4096 x 14336, top 2   1 row 124 | 119    8: 488 | 429   32: 533 | 453
+//   16 experts 4096 x 2048, top 2   4 rows 71 |  64    8: 115 | 110   32: 149 | 130
 
 // acc rows 4 grp + 0..3 are the unit's weight rows, columns slots
 template <bool GLU>
@@ -699,6 +699,229 @@ __global__ void __launch_bounds__(NW * 64, 2) moe_stay_kernel(MoeGemmArgs a) {
     if (tl[2] > 16) run(Count<2>());
     else run(Count<1>());
   }
+}
+
+// The same with the weights through rings, for a K in blocks of 64 columns, which the
+// waves share evenly.  A unit is 16 weight rows, or 8 gates and their 8 up rows.
+template <bool GLU>
+struct Units {
+  static constexpr int NW = 8, R = 8, TR = GLU ? 8 : 16;
+  Ring<R> ring;
+  int block, nb;                         // the wave's blocks of 64 columns
+  int ntn, left, tn;                     // units of a tile; the workgroup's, and the
+  const int* tl;                         //   one that is multiplied next, of its tile
+  int asked, blk, to_ask;                // what is asked for next
+  const int* from;
+  __amdgpu_buffer_rsrc_t ra, rb;
+  int oa, ob, pitch;
+
+  __device__ __forceinline__ Units(const MoeGemmArgs& a, char* lds, int wid)
+      : ring(lds + wid * R * 1024) {
+    ntn = (a.N + TR - 1) / TR;
+    const long units = (long)a.tiles[3] * ntn;    // all tiles that have rows
+    const long first = units * blockIdx.x / gridDim.x;
+    left = (int)(units * (blockIdx.x + 1) / gridDim.x - first);
+    block = a.K / 64 * wid / NW;
+    nb = a.K / 64 * (wid + 1) / NW - block;
+    pitch = a.K * 2;
+    oa = Ring<R>::lane_bytes(pitch, 0) + block * 128;
+    ob = Ring<R>::lane_bytes(pitch, 1) + block * 128 + (GLU ? 0 : 8 * pitch);
+    asked = tn = (int)(first % ntn);
+    from = tl = a.tiles + 4 * (first / ntn);
+    blk = 0;
+    to_ask = left;
+  }
+  // of the expert of the tile that is asked for
+  __device__ __forceinline__ void expert(const MoeGemmArgs& a) {
+    const short* w = (const short*)a.w + (long)from[0] * (GLU ? 2 : 1) * a.N * a.K;
+    ra = ring_source(w, a.N * pitch);
+    rb = ring_source(GLU ? w + (long)a.N * a.K : w, a.N * pitch);
+  }
+  // the next block; is the one behind it of another tile?
+  __device__ __forceinline__ bool ask(const MoeGemmArgs& a) {
+    const uint at = to_ask > 0 ? (uint)(asked * TR) * pitch + blk * 128 : RING_NOWHERE;
+    ring.ask(ra, oa + at, rb, ob + at);
+    if (++blk < nb) return false;
+    blk = 0;
+    if (--to_ask <= 0 || ++asked < ntn) return false;
+    asked = 0;
+    from += 4;
+    expert(a);
+    return true;
+  }
+  // on to the next unit
+  __device__ __forceinline__ void advance() {
+    --left;
+    if (++tn < ntn) return;
+    tn = 0;
+    tl += 4;
+  }
+};
+
+// The sums of a unit's waves meet, and the first waves add them up.  `out`: where
+// this lane's row starts, if it is one.
+template <int MT, bool GLU>
+__device__ __forceinline__ void meet(const MoeGemmArgs& a, f32x4 (*part)[2][64],
+                                     const f32x4* acc, int wid, int tn, bool in,
+                                     short* out) {
+  constexpr int NW = 8;
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) part[wid][j][lane] = acc[j];
+  lds_barrier();
+  if (wid >= MT) return;
+  f32x4 v = {}, p[NW];
+#pragma unroll
+  for (int s = 0; s < NW; ++s) p[s] = part[s][wid][lane];
+#pragma unroll
+  for (int s = 0; s < NW; ++s) v += p[s];
+  const int col = tn * Units<GLU>::TR + 4 * grp;
+  if (GLU)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = glu(a, v[i], __shfl_xor(v[i], 32, 64));
+  if (in && col < a.N && (!GLU || grp < 2))
+    *(uint2*)(out + col) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+// K up to 512 CB: a workgroup stays, with the columns of its slots in registers.
+template <int CB, bool GLU>
+__global__ void __launch_bounds__(512) moe_ring_kernel(MoeGemmArgs a) {
+  using U = Units<GLU>;
+  __shared__ __attribute__((aligned(1024))) char lds[U::NW * U::R * 1024];
+  __shared__ f32x4 part[2][U::NW][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  U w(a, lds, wid);
+  if (w.left == 0) return;
+  w.expert(a);
+#pragma unroll
+  for (int i = 0; i < U::R / 2; ++i) w.ask(a);
+  const int nb = w.nb;
+  int buf = 0;
+  // the units of one slot tile, MT times 16 slots
+  auto run = [&](auto tiles_of_16) __attribute__((always_inline)) {
+    constexpr int MT = decltype(tiles_of_16)::value;
+    const int slot0 = w.tl[1], rows = w.tl[2];
+    frag_u fx[CB * 2][MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const short* x = unit_x(a, slot0 + min(j * 16 + (lane >> 2), rows - 1)) +
+                       w.block * 64 + (lane & 3) * 8;
+#pragma unroll
+      for (int c = 0; c < CB * 2; ++c)   // blocks past the wave's are not used
+        fx[c][j].u4 = *(const uint4v*)(x + (c < 2 * nb ? c * 32 : 0));
+    }
+#pragma unroll
+    for (int c = 0; c < CB * 2; ++c)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) fx[c][j] = turned(fx[c][j]);
+    const int r = wid * 16 + (lane & 15);  // the row that this lane stores
+    const int slot = slot0 + min(r, rows - 1);
+    short* const out = (short*)a.out + (long)(a.top ? slot : a.order[slot]) * a.N;
+    // from here on only pieces (and results) are on their way
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    for (int n = min(w.left, w.ntn - w.tn); n > 0; --n, buf ^= 1) {
+      f32x4 acc[MT] = {};
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        if (c >= nb) continue;
+        frag_u f0, f1;
+        w.ring.template take<U::R - 2>(f0, f1);
+        w.ask(a);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          acc[j] = mfma16(f0.bf, fx[2 * c][j].bf, acc[j]);
+          acc[j] = mfma16(f1.bf, fx[2 * c + 1][j].bf, acc[j]);
+        }
+      }
+      meet<MT, GLU>(a, part[buf], acc, wid, w.tn, r < rows, out);
+      w.advance();
+    }
+  };
+  while (w.left > 0) {
+    if (w.tl[2] > 16) run(Count<2>());
+    else run(Count<1>());
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // LDS is given back
+}
+
+// Longer rows: x flows too, a ring ahead.
+template <bool GLU>
+__global__ void __launch_bounds__(512) moe_flow_kernel(MoeGemmArgs a) {
+  using U = Units<GLU>;
+  constexpr int D = U::R / 2;            // blocks ahead
+  __shared__ __attribute__((aligned(1024))) char lds[U::NW * U::R * 1024];
+  __shared__ f32x4 part[2][U::NW][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  U w(a, lds, wid);
+  if (w.left == 0) return;
+  w.expert(a);
+  bool two = false;
+  for (int i = 0; i <= (w.tn + w.left - 1) / w.ntn; ++i) two |= w.tl[4 * i + 2] > 16;
+  const int total = w.left * w.nb;
+  auto run = [&](auto tiles_of_16) __attribute__((always_inline)) {
+    constexpr int MT = decltype(tiles_of_16)::value;
+    const short* x[MT];
+    auto rows_of = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        x[j] = unit_x(a, w.from[1] + min(j * 16 + (lane >> 2), w.from[2] - 1)) +
+               w.block * 64 + (lane & 3) * 8;
+    };
+    frag_u fx[D][2][MT];
+    auto ask = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          fx[i][h][j].u4 = *(const uint4v*)(x[j] + w.blk * 64 + h * 32);
+      if (w.ask(a)) rows_of();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // The row that this lane stores.  Waited for at once: where ways with and
+    // without it join, every product would wait for all loads.
+    const int r = wid * 16 + (lane & 15);
+    short* out;
+    bool in;
+    auto row_of = [&]() __attribute__((always_inline)) {
+      const int rows = w.tl[2], slot = w.tl[1] + min(r, rows - 1);
+      in = r < rows;
+      out = (short*)a.out + (long)(a.top ? slot : a.order[slot]) * a.N;
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+    };
+    row_of();
+    rows_of();
+#pragma unroll
+    for (int i = 0; i < D; ++i) ask(i);
+    f32x4 acc[MT] = {};
+    int c = 0, buf = 0;
+    for (int s = 0; s < total; s += D) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        frag_u f0, f1;
+        w.ring.template take<(D - 1) * (2 * MT + 2)>(f0, f1);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          acc[j] = mfma16(f0.bf, turned(fx[i][0][j]).bf, acc[j]);
+          acc[j] = mfma16(f1.bf, turned(fx[i][1][j]).bf, acc[j]);
+        }
+        ask(i);
+        if (++c == w.nb && w.left > 0) {  // past the last unit nothing counts
+          meet<MT, GLU>(a, part[buf], acc, wid, w.tn, in, out);
+#pragma unroll
+          for (int j = 0; j < MT; ++j) acc[j] = f32x4{};
+          c = 0;
+          buf ^= 1;
+          w.advance();
+          if (w.tn == 0 && w.left > 0) row_of();
+        }
+      }
+    }
+  };
+  if (two) run(Count<2>());
+  else run(Count<1>());
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // LDS is given back
 }
 
 // Longer rows: a workgroup a unit; its 16 waves take turns of 64 columns of
@@ -842,10 +1065,21 @@ template <bool GLU>
 static void launch_stream(const MoeGemmArgs& a, hipStream_t stream) {
   const int units = (a.N + 15) / 16;
   const long all = (long)units * a.max_tiles;
-  // as many workgroups as are resident: with twice as many, 2% to 30% longer.
-  // They share whole units, so they need a few (6 tiles of 2048 x 1408: a
-  // workgroup a unit 42 us, two products and the plan; staying 47).  The host
-  // knows the most tiles there can be: rows that share few experts stay as well.
+  // Rings: a workgroup of 8 waves a CU (of 4 waves, two or three a CU: 168 and 184 us
+  // where one takes 165).  They share whole units, so they need a few (6 tiles of
+  // 2048 x 1408, 528 units: 23 us, a workgroup a unit 30; 16 experts 4096 x 2048, 1
+  // row, 256 and 512 units: 24, 22.5).  The host knows the most tiles there can be:
+  // rows that share few experts stay as well.
+  // every wave has a block, an expert's offsets are bytes of 31 bits
+  if (a.K % 64 == 0 && a.K >= 512 && (GLU ? 2L : 1L) * a.N * a.K < 1L << 30 &&
+      all > 512) {
+    if (a.K <= 2048) moe_ring_kernel<4, GLU><<<256, 512, 0, stream>>>(a);
+    else if (a.K <= 4096) moe_ring_kernel<8, GLU><<<256, 512, 0, stream>>>(a);
+    else moe_flow_kernel<GLU><<<256, 512, 0, stream>>>(a);
+    return;
+  }
+  // through registers, as many workgroups as are resident: with twice as many, 2% to
+  // 30% longer
   const int grid = a.K <= 2048 ? 512 : 256;
   if (a.K > 4096 || all < 2 * grid)
     moe_stream_kernel<GLU><<<dim3(units, a.max_tiles), 1024, 0, stream>>>(a);

@@ -23,6 +23,7 @@
 // 64 KB a CU are enough: twice as many cost small weights 10 %.
 
 #include "serving.h"
+#include "ring.h"
 #include "words.h"
 
 struct StreamArgs {
@@ -75,11 +76,6 @@ __device__ __forceinline__ void store_rows(const StreamArgs& a, int t, int n, in
 __device__ __forceinline__ bf16x8 if_there(bool in, frag_u f) {
   if (!in) f.u4 = uint4v{0, 0, 0, 0};
   return f.bf;
-}
-
-// A barrier for what is in LDS: it waits for no load.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // The normed row, in LDS, by NT threads.  Every workgroup makes it for itself while
@@ -337,26 +333,26 @@ __global__ void __launch_bounds__(NW * 64) stay_linear_kernel(StreamArgs a) {
   }
 }
 
-// Weights through LDS: a workgroup takes an even share of the weight rows (8 at a
-// time, so that no CU has much more than another), 16 rows a tile (8 gates and their
-// projections); each of its 8 waves takes its columns of the tile, 64 at a time, from a
-// ring of its own of R pieces of 8 rows by 64 columns.  Loads that hold no
-// register and wait for nobody fill it: tiles end, sums meet, and the ring goes on.
+// Weights through rings: a workgroup takes tiles of 16 weight rows (8 gates and their
+// projections), and of what is left over an even share in 8 rows, so that no CU has
+// much more than another; each of its 8 waves takes its columns of the tile, 64 at a
+// time.  Neighbours take neighbouring tiles: where each had its rows in one piece, all
+// read at the same distance, and some distances meet few channels (22016 x 3072: 31
+// us, now 24).
 template <int R, int EPI>
-struct Ring {
+struct Tiles {
   static constexpr int NW = 8, TR = EPI == GLU ? 8 : 16, UT = TR / 8;
+  Ring<R> ring;
   int rows, full, u0, u1, tiles;         // whole tiles, then units of 8 rows of the last
   int first, nb;                         // the wave's blocks of 64 columns
   __amdgpu_buffer_rsrc_t ra, rb;
   int oa, ob, pitch;
-  char* mine;
-  int tile, begin, blk, slot;            // what is asked for next, and its place
+  int tile, begin, blk;                  // what is asked for next
   uint ta, tb;
-  int src0, src1, rd;
 
-  __device__ __forceinline__ Ring(const StreamArgs& a, char* ring, int wid,
-                                  int rotate = 0) {
-    const int lane = threadIdx.x & 63, c16 = lane & 15, grp = lane >> 4;
+  __device__ __forceinline__ Tiles(const StreamArgs& a, char* lds, int wid,
+                                   int rotate = 0)
+      : ring(lds + wid * R * 1024) {
     rows = EPI == GLU ? a.N / 2 : a.N;
     const int units = (rows + 7) / 8, G = gridDim.x, b = blockIdx.x;
     full = units / (UT * G);
@@ -367,24 +363,15 @@ struct Ring {
     const int blocks = a.K / 64;
     first = blocks * wid / NW;
     nb = blocks * (wid + 1) / NW - first;
-    // Pieces past the last row are not read: they lie past the end of the buffer.
     pitch = (int)a.wst * 2;
     const int end = (rows - 1) * pitch + a.K * 2;
-    ra = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, 0, end, 0x00027000);
-    rb = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(EPI == GLU ? a.w + rows * a.wst : a.w), 0, end, 0x00027000);
-    // A piece has 8 slots of 16 bytes a row; slot s of row r lies at place s ^ r (of
-    // the second piece s ^ r ^ 1), so that 16 rows of one slot touch every bank once.
-    const int pr = lane >> 3, ps = (lane & 7) ^ pr;
-    oa = pr * pitch + ps * 16 + first * 128;
-    ob = (EPI == GLU ? pr : pr + 8) * pitch + (ps ^ 1) * 16 + first * 128;
-    mine = ring + wid * R * 1024;
-    tile = slot = rd = 0;
+    ra = ring_source(a.w, end);
+    rb = ring_source(EPI == GLU ? a.w + rows * a.wst : a.w, end);
+    oa = Ring<R>::lane_bytes(pitch, 0) + first * 128;
+    ob = Ring<R>::lane_bytes(pitch, 1) + first * 128 + (EPI == GLU ? 0 : 8 * pitch);
+    tile = 0;
     blk = begin = rotate ? blockIdx.x / rotate % nb : 0;
     locate();
-    const int r8 = c16 & 7, turn = c16 >> 3;
-    src0 = (int)(size_t)(lds_ptr)mine + turn * 1024 + r8 * 128 +
-           ((grp ^ r8 ^ turn) & 7) * 16;
   }
   // first row of a tile, and past its last one
   __device__ __forceinline__ int row0(int t) const {
@@ -394,34 +381,16 @@ struct Ring {
     return min(rows, t < full ? row0(t) + TR : 8 * u1);
   }
   __device__ __forceinline__ void locate() {
-    ta = tile < tiles ? (uint)row0(tile) * pitch : 1u << 31;
-    tb = EPI != GLU && tile == full && u1 - u0 < 2 ? 1u << 31 : ta;
+    ta = tile < tiles ? (uint)row0(tile) * pitch : RING_NOWHERE;
+    tb = EPI != GLU && tile == full && u1 - u0 < 2 ? RING_NOWHERE : ta;
   }
-  // the next block's two pieces.  Not kept in the caches (each is read once: 235 MB in
-  // 40.0 us, so 36.0).
   __device__ __forceinline__ void ask() {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(mine + slot), 16,
-                                             oa + ta + blk * 128, 0, 0, 2);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(mine + slot + 1024), 16,
-                                             ob + tb + blk * 128, 0, 0, 2);
-    slot = (slot + 2048) & (R * 1024 - 1);
+    ring.ask(ra, oa + ta + blk * 128, rb, ob + tb + blk * 128);
     if (++blk == nb) blk = 0;
     if (blk == begin) {
       ++tile;
       locate();
     }
-  }
-  // The oldest block, when no more than AFTER loads are on their way behind it.
-  template <int AFTER>
-  __device__ __forceinline__ void take(frag_u& f0, frag_u& f1) {
-    asm volatile("s_waitcnt vmcnt(%4)\n\t"
-                 "ds_read_b128 %0, %2\n\t"
-                 "ds_read_b128 %1, %3\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(f0.u4), "=&v"(f1.u4)
-                 : "v"(src0 + rd), "v"((src0 ^ 64) + rd), "n"(AFTER)
-                 : "memory");
-    rd = (rd + 2048) & (R * 1024 - 1);
   }
 };
 
@@ -446,18 +415,10 @@ __device__ __forceinline__ void meet(const StreamArgs& a, f32x4 (*part)[MT][64],
   if (EPI != GLU || grp < 2) store_rows<EPI>(a, wid * 16 + c16, n + 4 * grp, n1, v, u);
 }
 
-// Rows of x as fragments.  A fragment's neighbouring lanes have different rows, and a
-// load of it would look up a cache line a lane; neighbours in fours read 64 bytes of
-// a row instead, and hand them on.
+// this lane's words of rows 16 j on, to be turned
 __device__ __forceinline__ const short* row_words(const StreamArgs& a, int j) {
   const int lane = threadIdx.x & 63;
   return a.x + (long)min(j * 16 + (lane >> 2), a.T - 1) * a.xst + (lane & 3) * 8;
-}
-__device__ __forceinline__ frag_u turned(frag_u f) {
-  const int lane = threadIdx.x & 63, from = ((lane & 15) * 4 + (lane >> 4)) * 4;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) f.u[i] = __builtin_amdgcn_ds_bpermute(from, f.u[i]);
-  return f;
 }
 
 // The wave's columns of x stay in registers, at most CB blocks of 64.
@@ -467,7 +428,7 @@ __global__ void __launch_bounds__(512) ring_linear_kernel(StreamArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[8 * R * 1024];
   __shared__ f32x4 part[2][8][MT][64];
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Ring<R, EPI> w(a, ring, wid);
+  Tiles<R, EPI> w(a, ring, wid);
   const int nb = w.nb;
   frag_u fx[CB * 2][MT];
 #pragma unroll
@@ -491,7 +452,7 @@ __global__ void __launch_bounds__(512) ring_linear_kernel(StreamArgs a) {
     for (int c = 0; c < CB; ++c) {
       if (c >= nb) continue;
       frag_u f0, f1;
-      w.template take<R - 2>(f0, f1);
+      w.ring.template take<R - 2>(f0, f1);
       w.ask();
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
@@ -517,7 +478,7 @@ __global__ void __launch_bounds__(512) flow_linear_kernel(StreamArgs a) {
   __shared__ __attribute__((aligned(16))) short row[NORM ? 4096 : 8];
   __shared__ float red[NORM ? 16 : 1];
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Ring<R, EPI> w(a, ring, wid, 8);
+  Tiles<R, EPI> w(a, ring, wid, 8);
   const int nb = w.nb;
   frag_u fx[D][2][MT];
   const short* x[MT];
@@ -551,7 +512,7 @@ __global__ void __launch_bounds__(512) flow_linear_kernel(StreamArgs a) {
 #pragma unroll
     for (int i = 0; i < D; ++i) {
       frag_u f0, f1;
-      w.template take<(D - 1) * (NORM ? 2 : 2 * MT + 2)>(f0, f1);
+      w.ring.template take<(D - 1) * (NORM ? 2 : 2 * MT + 2)>(f0, f1);
       if (NORM) {
         const short* at = row + (w.first + rb) * 64 + ((threadIdx.x & 63) >> 4) * 8;
         fx[i][0][0].u4 = *(const uint4v*)at;

@@ -617,6 +617,17 @@ def test_streamed_experts_at_their_edges(sv, E, top, T, W, ff, one):
                torch.bfloat16)
 
 
+@pytest.mark.parametrize("E,top,T,W,ff,one", [
+    (16, 4, 40, 576, 1088, False), (9, 2, 60, 512, 4160, True),
+    (40, 1, 35, 584, 1024, False), (70, 2, 20, 2048, 576, False),
+    (20, 2, 20, 512, 5120, False), (12, 2, 70, 520, 14336, True),
+    (3, 1, 33, 4096, 2048, True)])
+def test_experts_through_rings(sv, E, top, T, W, ff, one):
+    """The same: waves of unequal numbers of blocks, fewer and more than the ring
+    has, x kept and flowing, 8 rows in the last unit, workgroups of several tiles."""
+    test_streamed_experts_at_their_edges(sv, E, top, T, W, ff, one)
+
+
 @pytest.mark.parametrize("kind", ["plain", "sigmoid", "softmax"])
 @pytest.mark.parametrize("T,E,top", [(16, 64, 64), (17, 64, 6), (16, 65, 9),
                                      (17, 256, 40), (3, 257, 7), (64, 512, 64)])
