@@ -513,8 +513,8 @@ latent_rows_kernel(LatentRowsArgs a) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int it = i * 256 + tid;
-      if (FULL)                          // a tile is one piece
-        reg[i] = *(const uint4v*)(src + it * 8u);
+      if (FULL)                          // a tile is one piece, and read once
+        reg[i] = __builtin_nontemporal_load((const uint4v*)(src + it * 8u));
       else
         reg[i] = word(src + it / CPR * RP, column(it % CPR));
     }

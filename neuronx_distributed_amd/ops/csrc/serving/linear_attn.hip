@@ -82,9 +82,14 @@ __device__ __forceinline__ void log_gates(const MemoryArgs& a, long row,
 // token after token: a workgroup owns 32 columns of one head's state
 // ---------------------------------------------------------------------------
 // TAPS: 0 no convolution, 1 any number of taps, else this number
+// once: states that no cache keeps.  Bound by reading and writing them.  One step's are
+// in no cache at the next where there are more of them than the 256 MB behind the L2s,
+// and are then read and written faster past it; fewer may be there still (us, kept and
+// past: 32 heads of 128 x 128, 128 tokens (268 MB) 106, 87; 64: 54, 45; 32 (67 MB)
+// 23, 25; 128 heads of 128 x 64, 32 tokens (134 MB) 55, 46.5).
 template <typename T, int NI, int GATE, bool VEC, int TAPS>
 __global__ void __launch_bounds__(256)
-memory_steps_kernel(MemoryArgs a) {
+memory_steps_kernel(MemoryArgs a, bool once) {
   const int D = a.D, E = a.E;
   const int nt = (E + 31) / 32;
   const int vt = blockIdx.x % nt;
@@ -102,17 +107,32 @@ memory_steps_kernel(MemoryArgs a) {
   float* Sp = a.S + (slot * a.H + h) * D * E;
   float S[NI][4];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int d = dg + 32 * i;
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) S[i][j] = 0.f;
-    if (ctx > 0 && d < D) {
-      if (VEC) {
-        if (e0 < E) load4(Sp + (long)d * E + e0, S[i]);
-      } else {
+  auto each_word = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int d = dg + 32 * i;
+      if (d < D && e0 < E) f((f32x4*)(Sp + (long)d * E + e0), S[i]);
+    }
+  };
+  if (ctx > 0) {
+    if (VEC && once) {
+      each_word([](f32x4* p, float* s) {
+        const f32x4 w = __builtin_nontemporal_load(p);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = w[j];
+      });
+    } else if (VEC) {
+      each_word([](f32x4* p, float* s) { load4((const float*)p, s); });
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int d = dg + 32 * i;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (e0 + j < E) S[i][j] = Sp[(long)d * E + e0 + j];
+          if (d < D && e0 + j < E) S[i][j] = Sp[(long)d * E + e0 + j];
       }
     }
   }
@@ -270,13 +290,17 @@ memory_steps_kernel(MemoryArgs a) {
     }
   }
 
+  if (VEC && once) {
+    each_word([](f32x4* p, float* s) {
+      __builtin_nontemporal_store(f32x4{s[0], s[1], s[2], s[3]}, p);
+    });
+  } else if (VEC) {
+    each_word([](f32x4* p, float* s) { store4((float*)p, s); });
+  } else {
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int d = dg + 32 * i;
-    if (d >= D) continue;
-    if (VEC) {
-      if (e0 < E) store4(Sp + (long)d * E + e0, S[i]);
-    } else {
+    for (int i = 0; i < NI; ++i) {
+      const int d = dg + 32 * i;
+      if (d >= D) continue;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (e0 + j < E) Sp[(long)d * E + e0 + j] = S[i][j];
@@ -296,7 +320,9 @@ template <typename T, int GATE, int TAPS>
 static int launch_steps(const MemoryArgs& a, int n_seg, hipStream_t stream) {
   const long grid = (long)n_seg * a.H * ((a.E + 31) / 32);
   const bool vec = a.E % 4 == 0;
-#define MS(N, V) memory_steps_kernel<T, N, GATE, V, TAPS><<<grid, 256, 0, stream>>>(a)
+  const bool once = (long)n_seg * a.H * a.D * a.E * 4 > 100L << 20;
+#define MS(N, V) \
+  memory_steps_kernel<T, N, GATE, V, TAPS><<<grid, 256, 0, stream>>>(a, once)
 #define MSV(N) do { if (vec) MS(N, true); else MS(N, false); } while (0)
   if (a.D <= 64) MSV(2);
   else if (a.D <= 128) MSV(4);

@@ -466,7 +466,10 @@ attn_rows_kernel(RowsArgs a) {
 // rows, which is the order in which the values come; the weights stay 32-bit, in
 // three planes that add up to them.
 //
-// Bound by memory: 8 waves a CU have 16 KB each on their way.  The kernel above
+// Bound by memory: 8 waves a CU have 16 KB each on their way.  Values are read past the
+// caches, as is right for what is read once a step (32 rows of up to 4096 keys, 309 MB:
+// 61.1 -> 56.4 us; 64 rows of 1000, 16 heads: 33 -> 27.5); keys too are 2 % faster there
+// but 13 % slower here, where their lines come in halves.  The kernel above
 // spends its time on vector work (a key costs 140 cycles of a wave; here 30), but
 // has more workgroups on a CU and less to start with: of many short rows whose
 // heads have keys of their own it is the faster one (rows_kernel in
@@ -585,7 +588,7 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
       const short* src = a.append && r >= newest
                              ? vn : vb + (long)min(r, newest) * a.vcs;
       __builtin_amdgcn_global_load_lds(
-          (global_ptr)(src + c), (lds_ptr)(vd + wid * VB + p * 1024), 16, 0, 0);
+          (global_ptr)(src + c), (lds_ptr)(vd + wid * VB + p * 1024), 16, 0, 2);
     }
   };
   // a transposing read: 16 lanes turn 4 keys by 16 columns
