@@ -6,6 +6,13 @@
 
 #include "serving.h"
 
+// A piece: 16 bytes a lane from `off` on, to where the wave's 1 KB begins.  ONCE: no
+// cache keeps it.
+template <bool ONCE>
+__device__ __forceinline__ void piece(__amdgpu_buffer_rsrc_t src, uint off, char* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)lds, 16, off, 0, 0, ONCE ? 2 : 0);
+}
+
 // One wave's ring of R pieces of 1 KB.
 template <int R>
 struct Ring {
@@ -28,9 +35,8 @@ struct Ring {
   // read.  No cache keeps them (each is read once: 235 MB in 40.0 us, so 36.0).
   __device__ __forceinline__ void ask(__amdgpu_buffer_rsrc_t a, uint oa,
                                       __amdgpu_buffer_rsrc_t b, uint ob) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(a, (lds_ptr)(mine + slot), 16, oa, 0, 0, 2);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (lds_ptr)(mine + slot + 1024), 16, ob, 0,
-                                             0, 2);
+    piece<true>(a, oa, mine + slot);
+    piece<true>(b, ob, mine + slot + 1024);
     slot = (slot + 2048) & (R * 1024 - 1);
   }
   // The oldest block, when no more than AFTER loads are on their way behind it:

@@ -111,6 +111,13 @@ class _StreamArgs(ctypes.Structure):
                 + _fields("eps", ctypes.c_float))
 
 
+class _WideArgs(ctypes.Structure):
+    _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
+                + _fields("w", ctypes.c_void_p) + _fields("wst", ctypes.c_long)
+                + _fields("out", ctypes.c_void_p)
+                + _fields("T N K splits", ctypes.c_int))
+
+
 class _ConvArgs(ctypes.Structure):
     _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
                 + _fields("w bias out", ctypes.c_void_p)
@@ -347,6 +354,69 @@ def ring_rule(T: int, N: int, K: int, f32: bool = False,
         K < 16384 and K % 2048 == 0 and N > 2048 else 3
 
 
+def wide_rule(T: int, N: int, K: int, f32: bool = False,
+              glu: bool = False) -> Optional[int]:
+    """Into how many shares of K ``wide_linear`` cuts the product of T rows with a
+    weight (N, K), or None where the library or ``stream_how`` is the faster one.
+    As many shares as leave no CU without a workgroup of 128 weight rows, of 256
+    columns at least; of many rows no more than 16, whose sums are as much to write
+    as the weights (1024 x 8192, 128 rows: 14.5 us, by 32 19.3).  Drawn over 3312
+    calls of 9 to 128 rows, 1.04 to 1.25 times as fast; us here, there and here:
+
+    - up to 32 rows only a K beyond the registers of ``ring_rule`` (4096 x 14336, 17
+      rows: 29, 24; fewer than 17 of a very long one: 6144 x 18944, 9 rows 110, 42),
+      and weights of many rows;
+    - up to 64 rows are the weights'; more are also bound by their way through LDS,
+      and the library is faster where workgroups leave CUs without work (22016 x
+      5120, 64 rows: 53.4, 54.5, 128 rows: 53, 63; 57344 x 4096, the last of two
+      rounds empty by a quarter);
+    - short K under few weight rows has too little to hide a merge behind (4096 x
+      2048, 40 rows: 9.9, 9.1, 96: 10, 11; 8192 x 3072, 96: 19.2, 21.4)."""
+    if K % 64 or K < 512 or N % 8 or T > 128 or glu and N % 32:
+        return None
+    tiles, many = -(-N // 128), T > 64
+    splits = max(1, min(256 // tiles, K // 256, 16 if many else 64))
+    idle = 1 - tiles * splits / (256 * -(-tiles * splits // 256))
+    if tiles > 256 and idle > (0.1 if many and not glu else 0.15):
+        return None
+    if T <= 32:
+        if K <= 4096:
+            take = T >= 17 and N >= 28000 and K >= 1536
+        else:
+            take = T >= 17 or T >= 9 and N >= 5120 and (
+                K >= 14336 if T < 13 else K >= 11008)
+    elif tiles >= 168:
+        take = K >= 1536 and (not many or glu or idle < 0.3)
+    elif glu or N >= 5000:
+        take = K >= (4096 if many else 3072)
+    elif N < 3072:
+        take = K >= (7168 if many else 4096 if N < 2048 else 3072)
+    else:
+        take = K >= 3072
+    return splits if take else None
+
+
+def wide_linear(x: torch.Tensor, w: torch.Tensor, splits: int = 1,
+                f32: bool = False, glu: bool = False) -> torch.Tensor:
+    """As ``stream_linear``, for up to 128 rows, with K in ``splits`` shares."""
+    T, K = x.shape
+    N = w.shape[0]
+    assert x.dtype == w.dtype == torch.bfloat16 and w.shape[1] == K
+    assert x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
+    assert _words(x) and _words(w) and not (f32 and glu)
+    out = torch.empty(T, N // 2 if glu else N, device=x.device,
+                      dtype=torch.float32 if f32 else torch.bfloat16)
+    part = torch.empty(splits * T * N, dtype=torch.float32,
+                       device=x.device) if splits > 1 else None
+    a = _WideArgs(x=x.data_ptr(), xst=x.stride(0), w=w.data_ptr(),
+                  wst=w.stride(0), out=out.data_ptr(), T=T, N=N, K=K,
+                  splits=splits)
+    _check(library().sv_wide_linear(
+        ctypes.byref(a), ctypes.c_void_p(_p(part)), 2 if glu else int(f32),
+        _stream()), "wide_linear")
+    return out
+
+
 def stream_linear(x: torch.Tensor, w: torch.Tensor, stay: int = 0,
                   f32: bool = False, glu: bool = False) -> torch.Tensor:
     """x (T, K) @ w (N, K)^T, bfloat16, with the sums rounded once or not at
@@ -375,43 +445,74 @@ def _plain(t) -> bool:
     return type(t) in (torch.Tensor, torch.nn.Parameter)
 
 
-def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
-               glu: bool = False, rings: bool = True) -> Optional[int]:
-    """How ``stream_linear`` takes the rows of x (..., K) where it is the faster
-    one (by ``ring_rule``, if ``rings``, or ``stream_rule``); None elsewhere, under autograd, and where somebody else watches the
-    operations (tracing, dispatch modes, autocast).  NXDA_SKINNY_GEMM=0 keeps
-    every product on the library."""
+def _few_rows(x: torch.Tensor, w: torch.Tensor, rule) -> Optional[tuple]:
+    """(rows of x (..., K), what ``rule`` (T, N, K) says of them) for the kernels of
+    few rows; None where it says None, under autograd, and where somebody else
+    watches the operations (tracing, dispatch modes, autocast).
+    NXDA_SKINNY_GEMM=0 keeps every product on the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
             not x.is_cuda or x.dim() < 2 or w.dim() != 2 or \
             os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
         return None
     K = x.shape[-1]
     T = x.numel() // K if K else 0
-    if not 0 < T <= 32 or x.dtype != torch.bfloat16 or \
+    if not 0 < T <= 128 or x.dtype != torch.bfloat16 or \
             w.dtype != torch.bfloat16 or w.shape[1] != K or \
             w.stride(1) != 1 or w.device != x.device or \
             x.device.index != torch.cuda.current_device():
         return None
-    how = ring_rule(T, w.shape[0], K, f32, glu) if rings and \
-        w.stride(0) * (w.shape[0] + 16) < 1 << 30 else None
-    if how is None:
-        how = stream_rule(T, w.shape[0], K, f32, glu)
+    how = rule(T, w.shape[0], K)
     if how is None or not available() or not _unwatched():
         return None
     rows = x.reshape(T, K)
     if rows.stride(1) != 1 or not (_words(rows) and _words(w)):
         return None
-    return how
+    return rows, how
+
+
+def _near(w: torch.Tensor) -> bool:
+    """Are all offsets in w bytes of 31 bits, also a tile past its end?"""
+    return w.stride(0) * (w.shape[0] + 128) < 1 << 30
+
+
+def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
+               glu: bool = False, rings: bool = True) -> Optional[int]:
+    """How ``stream_linear`` takes the rows of x (..., K) where it is the faster
+    one (by ``ring_rule``, if ``rings``, or ``stream_rule``); else None."""
+    def rule(T, N, K):
+        if T > 32:
+            return None
+        how = ring_rule(T, N, K, f32, glu) if rings and _near(w) else None
+        return stream_rule(T, N, K, f32, glu) if how is None else how
+
+    took = _few_rows(x, w, rule)
+    return took and took[1]
 
 
 def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
              glu: bool = False) -> Optional[torch.Tensor]:
-    """``stream_linear`` of the rows of x (..., K) by ``stream_how``, or None."""
-    how = stream_how(x, w, f32, glu)
-    if how is None:
+    """The product of the rows of x (..., K) by ``wide_linear`` where
+    ``wide_rule`` takes it, or ``stream_linear`` by ``stream_how``, or None."""
+    def rule(T, N, K):
+        near = _near(w)
+        splits = wide_rule(T, N, K, f32, glu) if near and \
+            x.stride(-2) < 1 << 22 else None
+        if splits is not None:
+            return True, splits
+        how = None
+        if T <= 32:
+            how = ring_rule(T, N, K, f32, glu) if near else None
+            if how is None:
+                how = stream_rule(T, N, K, f32, glu)
+        return None if how is None else (False, how)
+
+    took = _few_rows(x, w, rule)
+    if took is None:
         return None
-    return stream_linear(x.reshape(-1, x.shape[-1]), w, how, f32,
-                         glu).view(*x.shape[:-1], -1)
+    rows, (wide, how) = took
+    out = wide_linear(rows, w, how, f32, glu) if wide else \
+        stream_linear(rows, w, how, f32, glu)
+    return out.view(*x.shape[:-1], -1)
 
 
 def _unwatched() -> bool:

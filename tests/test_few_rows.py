@@ -211,3 +211,21 @@ def test_every_ring_is_one_that_the_launcher_takes():
                     if how == 2:
                         assert K <= (8192 if T <= 16 else 4096)
     assert taken == {None, 2, 3}
+
+
+def test_every_cut_is_one_that_the_launcher_takes():
+    """Shares of K of 256 columns at least, whole words of gated results, and none
+    of what the kernels of fewer rows are there for."""
+    taken = set()
+    for T in range(1, 130, 3):
+        for N in SIZES:
+            for K in SIZES + (512 + 64, 11008):
+                for f32, glu in ((False, False), (True, False), (False, True)):
+                    splits = sv.wide_rule(T, N, K, f32, glu)
+                    if splits is None:
+                        continue
+                    taken.add(splits)
+                    assert 9 <= T <= 128 and K % 64 == 0 and N % 8 == 0
+                    assert 1 <= splits <= K // 256 and not (glu and N % 32)
+                    assert splits == 1 or splits * -(-N // 128) <= 256
+    assert 1 in taken and len(taken) > 5

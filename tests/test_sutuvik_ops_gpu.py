@@ -747,6 +747,31 @@ def test_products_of_few_rows_through_rings(T, N, K, how):
             atol=tol * 16)
 
 
+@pytest.mark.parametrize("T,N,K,splits", [
+    (9, 8, 512, 1), (17, 136, 576, 2), (32, 264, 14336, 7), (33, 1000, 1088, 3),
+    (64, 4096, 4096, 8), (65, 24, 512, 1), (100, 6144, 2112, 5), (128, 8200, 704, 1)])
+def test_products_of_more_rows(T, N, K, splits):
+    """The same, 32, 64 and 128 rows a workgroup and one more, shares of K of unequal
+    numbers of blocks, fewer than the stages and more, tiles and rows ragged."""
+    torch.manual_seed(T + N + K)
+    x = torch.full((T, K + 8), float("nan"), device="cuda", dtype=torch.bfloat16)[:, :K]
+    x.copy_(torch.randn(T, K, device="cuda"))
+    wide = torch.full((N + 128, K + 24), float("nan"), device="cuda",
+                      dtype=torch.bfloat16)
+    w = wide[:N, :K]
+    w.copy_(torch.randn(N, K, device="cuda").div(K ** 0.5))
+    ref = x.double() @ w.double().t()
+    tol = 16 * K ** 0.5 * 2.0 ** -24       # as above
+    out = sv.wide_linear(x, w, splits, f32=True)
+    torch.testing.assert_close(out.double(), ref, rtol=0, atol=tol)
+    torch.testing.assert_close(sv.wide_linear(x, w, splits).double(), ref,
+                               rtol=2.0 ** -8, atol=tol)
+    gate, up = ref[:, :N // 2], ref[:, N // 2:]
+    torch.testing.assert_close(
+        sv.wide_linear(x, w, splits, glu=True).double(),
+        torch.nn.functional.silu(gate) * up, rtol=2.0 ** -8, atol=tol * 16)
+
+
 @pytest.mark.parametrize("glu", [False, True])
 def test_few_rows_are_streamed_where_nobody_watches(glu):
     x = torch.randn(2, 3, 4096, device="cuda").bfloat16()
