@@ -388,22 +388,26 @@ def apply_rotary_polar_compatible(query, key, freqs):
 # SwiGLU
 # ---------------------------------------------------------------------------
 
+def _swiglu(x: torch.Tensor) -> torch.Tensor:
+    I = x.shape[-1] // 2
+    if x.is_cuda and x.dtype == torch.bfloat16 and I % 8 == 0:
+        lib = _require_lib()
+        x2 = x.contiguous()
+        N = x2.numel() // x2.shape[-1]
+        out = torch.empty(x2.shape[:-1] + (I,), dtype=x2.dtype,
+                          device=x2.device)
+        lib.swiglu_fwd(_ptr(x2), _ptr(out), ctypes.c_long(N),
+                       ctypes.c_int(I), _stream())
+        return out
+    g, u = x[..., :I].float(), x[..., I:].float()
+    return (torch.nn.functional.silu(g) * u).to(x.dtype)
+
+
 class _SwiGLUFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
         ctx.save_for_backward(x)
-        I = x.shape[-1] // 2
-        if x.is_cuda and x.dtype == torch.bfloat16 and I % 8 == 0:
-            lib = _require_lib()
-            x2 = x.contiguous()
-            N = x2.numel() // x2.shape[-1]
-            out = torch.empty(x2.shape[:-1] + (I,), dtype=x2.dtype,
-                              device=x2.device)
-            lib.swiglu_fwd(_ptr(x2), _ptr(out), ctypes.c_long(N),
-                           ctypes.c_int(I), _stream())
-            return out
-        g, u = x[..., :I].float(), x[..., I:].float()
-        return (torch.nn.functional.silu(g) * u).to(x.dtype)
+        return _swiglu(x)
 
     @staticmethod
     def backward(ctx, dy):
@@ -428,7 +432,9 @@ class _SwiGLUFn(torch.autograd.Function):
 
 def swiglu(x: torch.Tensor) -> torch.Tensor:
     """x = [gate; up] on the last dim -> silu(gate)*up."""
-    return _SwiGLUFn.apply(x)
+    from .serving import unseen
+
+    return _swiglu(x) if unseen(x) else _SwiGLUFn.apply(x)
 
 
 # ---------------------------------------------------------------------------

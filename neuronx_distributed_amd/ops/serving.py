@@ -12,6 +12,7 @@ import math
 import os
 from bisect import bisect_left
 from dataclasses import dataclass, replace
+from functools import lru_cache
 from typing import Optional, Sequence, Union
 
 import torch
@@ -43,10 +44,12 @@ def library():
 def available() -> bool:
     """Is the library there, with the products of few rows (one that was built
     before they came has none, and layers then use torch's)?"""
-    from .build import SERVING_LIB
+    if _LIB is None:
+        from .build import SERVING_LIB
 
-    return (_LIB is not None or os.path.exists(SERVING_LIB)) and \
-        hasattr(library(), "sv_stream_linear")
+        if not os.path.exists(SERVING_LIB):
+            return False
+    return hasattr(library(), "sv_stream_linear")
 
 
 def ensure_built():
@@ -451,28 +454,33 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, rule) -> Optional[tuple]:
     watches the operations (tracing, dispatch modes, autocast).
     NXDA_SKINNY_GEMM=0 keeps every product on the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
-            not x.is_cuda or x.dim() < 2 or w.dim() != 2 or \
+            not x.is_cuda:
+        return None
+    shape, size = x.shape, w.shape
+    if len(shape) < 2 or len(size) != 2:
+        return None
+    K = shape[-1]
+    T = shape[0] if len(shape) == 2 else x.numel() // K if K else 0
+    if not 0 < T <= 128 or not K or K != size[1] or x.dtype != torch.bfloat16 or \
+            w.dtype != torch.bfloat16 or w.stride(1) != 1 or \
+            x.get_device() != torch._C._cuda_getDevice() or \
+            w.get_device() != x.get_device() or \
             os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
         return None
-    K = x.shape[-1]
-    T = x.numel() // K if K else 0
-    if not 0 < T <= 128 or x.dtype != torch.bfloat16 or \
-            w.dtype != torch.bfloat16 or w.shape[1] != K or \
-            w.stride(1) != 1 or w.device != x.device or \
-            x.device.index != torch.cuda.current_device():
-        return None
-    how = rule(T, w.shape[0], K)
+    how = rule(T, size[0], K)
     if how is None or not available() or not _unwatched():
         return None
-    rows = x.reshape(T, K)
+    rows = x if len(shape) == 2 else x.reshape(T, K)
     if rows.stride(1) != 1 or not (_words(rows) and _words(w)):
         return None
     return rows, how
 
 
 def _near(w: torch.Tensor) -> bool:
-    """Are all offsets in w bytes of 31 bits, also a tile past its end?"""
-    return w.stride(0) * (w.shape[0] + 128) < 1 << 30
+    """Are all offsets in w bytes of 31 bits, also a tile past its end (and the
+    kernels there that count on it)?"""
+    return w.stride(0) * (w.shape[0] + 128) < 1 << 30 and \
+        hasattr(library(), "sv_wide_linear")
 
 
 def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
@@ -482,7 +490,8 @@ def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
     def rule(T, N, K):
         if T > 32:
             return None
-        how = ring_rule(T, N, K, f32, glu) if rings and _near(w) else None
+        how = ring_rule(T, N, K, f32, glu) if rings and available() and \
+            _near(w) else None
         return stream_rule(T, N, K, f32, glu) if how is None else how
 
     took = _few_rows(x, w, rule)
@@ -494,7 +503,7 @@ def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
     """The product of the rows of x (..., K) by ``wide_linear`` where
     ``wide_rule`` takes it, or ``stream_linear`` by ``stream_how``, or None."""
     def rule(T, N, K):
-        near = _near(w)
+        near = available() and _near(w)
         splits = wide_rule(T, N, K, f32, glu) if near and \
             x.stride(-2) < 1 << 22 else None
         if splits is not None:
@@ -512,7 +521,7 @@ def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
     rows, (wide, how) = took
     out = wide_linear(rows, w, how, f32, glu) if wide else \
         stream_linear(rows, w, how, f32, glu)
-    return out.view(*x.shape[:-1], -1)
+    return out if x.dim() == 2 else out.view(*x.shape[:-1], -1)
 
 
 def _unwatched() -> bool:
@@ -522,6 +531,17 @@ def _unwatched() -> bool:
                 or torch._C._len_torch_function_stack()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0)
+
+
+def unseen(*tensors) -> bool:
+    """May a call on these go past its autograd function: nobody differentiates,
+    traces or transforms it?"""
+    if torch.is_grad_enabled():
+        return False
+    for t in tensors:
+        if t is not None and not _plain(t):
+            return False
+    return _unwatched()
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -636,6 +656,34 @@ def short_conv(x, conv: ShortConv, seg, chunks, silu: bool = False,
     return out
 
 
+def _plain_norm(x, pending, eps, weight, index, centred, scale):
+    """``residual_norm`` of one tensor or sum that is neither normed nor gated, as
+    between a decoder's products: the same with fewer questions."""
+    d, coef = pending.delta, pending.coef
+    rows, W = d.shape
+    parts = 0
+    if coef is not None:
+        assert coef.is_contiguous() and coef.dtype == torch.float32
+        assert coef.numel() == rows and d.dtype == weight.dtype
+        rows, parts = coef.shape
+    dtype = weight.dtype
+    f32 = _f32(d) if dtype == torch.float32 else 0
+    assert d.is_contiguous() and d.dtype in (dtype, torch.float32)
+    out_rows = rows if index is None else index.shape[0]
+    x_new = torch.empty(out_rows, W, dtype=torch.float32, device=d.device)
+    h = torch.empty(out_rows, W, dtype=dtype, device=d.device)
+    a = _ResidualNormArgs(
+        x=_p(x), delta=d.data_ptr(), coef=_p(coef), x_out=x_new.data_ptr(),
+        h=h.data_ptr(), w=weight.data_ptr(), index=_p(index),
+        rows_out=out_rows, W=W, parts=parts, groups=1, p_groups=1, eps=eps,
+        scale=pending.scale, w_base=centred, p_base=pending.centred,
+        h_scale=scale,
+        delta_f32=not f32 and d.dtype == torch.float32)
+    _check(library().sv_residual_norm(ctypes.byref(a), f32, _stream()),
+           "residual_norm")
+    return x_new, h, None
+
+
 def residual_norm(x: Optional[torch.Tensor], pending: Optional[Pending],
                   eps: float, weight: Optional[torch.Tensor] = None,
                   x0: Optional[torch.Tensor] = None, keep_x: bool = True,
@@ -650,6 +698,12 @@ def residual_norm(x: Optional[torch.Tensor], pending: Optional[Pending],
     one of so many equal parts is normed on its own.  ``scale`` multiplies the
     second result.  ``conv``: the second result is h + conv(h) of the rows h of
     ``batch``."""
+    if x0 is None and keep_x and conv is None and not copy and \
+            pending is not None and weight is not None and groups == 1 and \
+            not (dtype or pending.branches or pending.delta2 is not None or
+                 pending.w1 is not None or pending.vec is not None or
+                 pending.groups != 1):
+        return _plain_norm(x, pending, eps, weight, index, centred, scale)
     branches = () if pending is None else pending.branches
     src = x if pending is None else \
         branches[0].delta if branches else pending.delta
@@ -835,8 +889,9 @@ def _low_bits(sizes, tensors) -> int:
 
 
 def _check_cache(q, k, v, kc, vc, H):
-    G, D, E = kc.shape[1], kc.shape[3], vc.shape[3]
-    assert kc.shape[:3] == vc.shape[:3] and kc.shape[2] == PAGE_SIZE
+    n, G, page, D = kc.shape
+    m, g, size, E = vc.shape
+    assert n == m and G == g and page == size == PAGE_SIZE
     assert kc.is_contiguous() and vc.is_contiguous() and H % G == 0
     assert q.shape[1] == H * D and k.shape[1] == G * D and \
         v.shape[1] == G * E
@@ -979,6 +1034,7 @@ _SHARED_ROWS = ((0, 256, 256, 256, 512, 512), (0, 512, 512, 512, 512, 768),
                 (0, 0, 0, 0, 2048, 2048))
 
 
+@lru_cache(maxsize=1024)
 def rows_kernel(rows: int, heads: int, groups: int, D: int, max_keys: int,
                 modified: bool = False):
     """Form (2 on matrix cores, 1 on vectors) and workgroups a row of
@@ -1045,8 +1101,9 @@ def attn_rows(q, k, v, kc, vc, pos, seq, block_table, heads: int,
                   pos=_p(pos), seq=_p(seq), bt=_p(block_table),
                   part=_p(part), out=_p(out), MB=block_table.shape[1],
                   rows=rows, H=heads, G=G, D=D, E=E, splits=splits,
-                  append=int(append), window=window, keep=keep, scale=scale,
-                  mod=_score_args(mod, q, heads))
+                  append=int(append), window=window, keep=keep, scale=scale)
+    if mod is not None:
+        a.mod = _score_args(mod, q, heads)
     if rotary is not None:
         a.cos, a.sin = map(_p, rotary)
     _check(library().sv_attn_rows(ctypes.byref(a), vec, _f32(q), _stream()),
@@ -1081,8 +1138,9 @@ def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
                    vpage=G * PAGE_SIZE * E, vhead=PAGE_SIZE * E, vrow=E,
                    tiles=_p(tiles), bt=_p(block_table), out=_p(out),
                    MB=block_table.shape[1], H=heads, G=G, D=D, E=E, DS=D,
-                   window=window, keep=keep, scale=scale,
-                   mod=_score_args(mod, q, heads))
+                   window=window, keep=keep, scale=scale)
+    if mod is not None:
+        a.mod = _score_args(mod, q, heads)
     _check(library().sv_attn_tiles(ctypes.byref(a), tiles.shape[0],
                                    _stream()), "attn_tiles")
     return out
@@ -1104,19 +1162,25 @@ def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
             rope_rows_(q, k, *rotary, batch.pos, kc.shape[3], batch.max_keys)
             rotary = None
     out = torch.empty(T, heads * vc.shape[3], dtype=q.dtype, device=q.device)
-    args = dict(heads=heads, scale=scale, window=window, keep=keep,
-                max_keys=batch.max_keys, append=prep is None)
+    append = prep is None
     if prep is not None:
         qkv_append(q, k, v, kc, vc, batch.pos, batch.seq, batch.block_table,
                    heads, prep)
-    if n:
-        attn_portions(q[:n], k[:n], v[:n], kc, vc, batch.pos[:n],
-                      batch.seq[:n], batch.block_table, batch.tiles,
-                      out=out[:n], mod=mod and mod.rows(0, n), **args)
-    if n < T:
-        attn_rows(q[n:], k[n:], v[n:], kc, vc, batch.pos[n:], batch.seq[n:],
-                  batch.block_table, out=out[n:], mod=mod and mod.rows(n, T),
-                  rotary=rotary, **args)
+    parts = ((0, T),) if n in (0, T) else ((0, n), (n, T))
+    for a, b in parts:
+        at = (q, k, v, batch.pos, batch.seq, out)
+        if b - a < T:                    # (a slice costs the host 1 us)
+            at = [t[a:b] for t in at]
+        qa, ka, va, pos, seq, oa = at
+        ma = mod and mod.rows(a, b)
+        if a < n:
+            attn_portions(qa, ka, va, kc, vc, pos, seq, batch.block_table,
+                          batch.tiles, heads, scale, window, keep, append,
+                          batch.max_keys, oa, ma)
+        elif a < T:
+            attn_rows(qa, ka, va, kc, vc, pos, seq, batch.block_table, heads,
+                      scale, window, keep, append, batch.max_keys, oa, ma,
+                      rotary)
     return out
 
 
@@ -1426,25 +1490,35 @@ class LatentWeights:
 
 def _append_args(q, rot_at, q_step, qr, qr_at, qr_step, kv, w, cache, pos, seq,
                  block_table, heads, eps):
-    T, R = q.shape[0], w.norm.shape[0]
+    P = cache.shape[2] - w.norm.shape[0]
+    assert qr.stride(1) == 1 and q.dtype == qr.dtype
+    assert (heads - 1) * q_step + rot_at + P <= q.shape[1]
+    assert (heads - 1) * qr_step + qr_at + P <= qr.shape[1]
+    assert q.shape[0] == qr.shape[0]
+    return _append_of(_p(q), q.stride(0), rot_at, q_step, _p(qr), qr.stride(0),
+                      qr_at, qr_step, kv, w, cache, pos, seq, block_table, heads,
+                      eps, q)
+
+
+def _append_of(q, qst, rot_at, q_step, qr, qrst, qr_at, qr_step, kv, w, cache,
+               pos, seq, block_table, heads, eps, like):
+    """Of addresses and pitches; ``like``: the queries."""
+    T, R = like.shape[0], w.norm.shape[0]
     P = cache.shape[2] - R
     half = w.freq.shape[0]
     assert kv.shape == (T, R + P) and cache.shape[1] == PAGE_SIZE
     assert cache.is_contiguous() and 2 * half <= P
     assert w.freq.dtype == torch.float64 and w.freq.is_cuda
-    assert q.stride(1) == qr.stride(1) == kv.stride(1) == 1
-    assert q.dtype == qr.dtype == kv.dtype == cache.dtype == w.norm.dtype
-    assert (heads - 1) * q_step + rot_at + P <= q.shape[1]
-    assert (heads - 1) * qr_step + qr_at + P <= qr.shape[1]
-    assert pos.shape[0] == seq.shape[0] == T == qr.shape[0]
-    size = q.element_size()
+    assert like.stride(1) == kv.stride(1) == 1
+    assert like.dtype == kv.dtype == cache.dtype == w.norm.dtype
+    assert pos.shape[0] == seq.shape[0] == T
+    size = like.element_size()
     return _LatentAppendArgs(
-        q=_p(q) + rot_at * size, qst=q.stride(0), qh=q_step,
-        qr=_p(qr) + qr_at * size, qrst=qr.stride(0), qrh=qr_step, kv=_p(kv),
-        kvst=kv.stride(0), w=_p(w.norm), freq=_p(w.freq), cache=_p(cache),
-        pos=_p(pos), seq=_p(seq), bt=_p(block_table),
-        MB=block_table.shape[1], H=heads, R=R, P=P, rot=2 * half, eps=eps,
-        amp=w.amplitude, pairs=int(w.pairs))
+        q=q + rot_at * size, qst=qst, qh=q_step, qr=qr + qr_at * size,
+        qrst=qrst, qrh=qr_step, kv=_p(kv), kvst=kv.stride(0), w=_p(w.norm),
+        freq=_p(w.freq), cache=_p(cache), pos=_p(pos), seq=_p(seq),
+        bt=_p(block_table), MB=block_table.shape[1], H=heads, R=R, P=P,
+        rot=2 * half, eps=eps, amp=w.amplitude, pairs=int(w.pairs))
 
 
 def latent_append(q, rot_at: int, q_step: int, qr, qr_at: int, qr_step: int,
@@ -1532,23 +1606,28 @@ def latent_rows_supported(dtype, rank: int, shared: int) -> bool:
             and rank <= 512 and shared <= 64)
 
 
-def _latent_rows_args(q, cache, rank, pos, seq, block_table, heads, scale,
-                      window, max_keys, sink, out):
-    """Arguments and the workspace that they point to.  Workgroups of 64 keys
+def _latent_shares(rows, heads, rank, max_keys, device):
+    """Shares of a row and the workspace for them.  Workgroups of 64 keys
     while CUs have none (1 row of 1000 keys: the whole step 28.1 us with 128,
     24.9 with 64), then of 128 (8 of 4096: 32.5, with 64 35.7).  A merge is not
     worth its launch up to 128 keys (43 rows of 82: 23.6, in two 28.7), of more
     than 32 workgroups up to 256 (94 rows of 192, 64 heads, no values behind
     them: 17.6, in two 28.1; 58 of 178, 8 heads 25.2, in three 23.1)."""
-    rows, D = q.shape[0], cache.shape[2]
     units = rows * -(-heads // 32)
     splits = 1 if max_keys <= (256 if units > 32 else 128) else max(
         _row_splits(512, units, max_keys, 128),
         _row_splits(256, units, max_keys, 64))
     # sums, maxima and totals of every share; of every row, its shares
-    part = torch.empty(rows * heads * splits * (rank + 2) + 2 * rows,
-                       dtype=torch.float32, device=q.device) \
-        if splits > 1 else None
+    return splits, torch.empty(
+        rows * heads * splits * (rank + 2) + 2 * rows, dtype=torch.float32,
+        device=device) if splits > 1 else None
+
+
+def _latent_rows_args(q, cache, rank, pos, seq, block_table, heads, scale,
+                      window, max_keys, sink, out):
+    """Arguments and the workspace that they point to."""
+    rows, D = q.shape[0], cache.shape[2]
+    splits, part = _latent_shares(rows, heads, rank, max_keys, q.device)
     return _LatentRowsArgs(
         q=_p(q), cache=_p(cache), pos=_p(pos), seq=_p(seq),
         bt=_p(block_table), part=_p(part), out=_p(out),
@@ -1679,33 +1758,70 @@ def latent_attention(q, kv, gate, batch, cache, w: LatentWeights, heads: int,
             q, kv, gate = (t if t is None else t[n:] for t in (q, kv, gate))
             one = [t[n:] for t in one]
         at = (*one, batch.block_table)
-        ql = torch.empty(T - n, heads * D, dtype=q.dtype, device=q.device)
-        lat = torch.empty(T - n, heads * R, dtype=q.dtype, device=q.device)
-        up, fast = _linear_args(q, dim + P, w.absorb, ql, D, None)
-        down, ok = _linear_args(
-            lat, R, w.expand[heads * dim:].view(heads, vdim, R),
-            out[n:] if n else out, vdim, gate)
-        if fast and ok and latent_rows_supported(q.dtype, R, P):
-            keys = batch.max_keys
-            if window > 0:
-                keys = min(keys, window) if keys else window
-            sink = _score_args(ScoreMod(sink=w.sink), ql, heads).sink
-            rows, part = _latent_rows_args(ql, cache, R, *at, heads, scale,
-                                           window, keys, sink, lat)
-            a = _LatentStepArgs(
-                append=_append_args(q, dim, dim + P, ql, R, D, kv, w, cache,
-                                    *at, heads, eps),
-                absorb=up, rows=rows, values=down)
-            _check(library().sv_latent_step(ctypes.byref(a), _stream()),
-                   "latent_step")
+        to = out[n:] if n else out
+        if _latent_step(q, kv, gate, *at, batch.max_keys, cache, w, heads, dim,
+                        vdim, scale, eps, window, to):
             return out
+        ql = torch.empty(T - n, heads * D, dtype=q.dtype, device=q.device)
         latent_append(q, dim, dim + P, ql, R, D, kv, w, cache, *at, heads, eps)
         head_linear(q, dim + P, w.absorb, ql, D)
         lat = latent_rows(ql, cache, R, *at, heads, scale, window,
                           batch.max_keys, w.sink)
         head_linear(lat, R, w.expand[heads * dim:].view(heads, vdim, R),
-                    out[n:] if n else out, vdim, gate)
+                    to, vdim, gate)
     return out
+
+
+def _latent_step(q, kv, gate, pos, seq, block_table, max_keys, cache,
+                 w: LatentWeights, heads, dim, vdim, scale, eps, window,
+                 out) -> bool:
+    """Single tokens in one call, on matrix cores: rows that are appended, queries
+    taken into the latent space, attention, values into ``out``.  False where one
+    of them has no such form."""
+    rows, R, D = q.shape[0], w.norm.shape[0], cache.shape[2]
+    P = D - R
+    if not (latent_rows_supported(q.dtype, R, P) and dim >= 8 and
+            _aligned((dim, vdim, R, P), q) and
+            (gate is None or _aligned((), gate))):
+        return False
+    assert w.absorb.shape == (heads, R, dim) and w.absorb.is_contiguous()
+    assert w.expand.shape == (heads * (dim + vdim), R)
+    assert w.expand.is_contiguous() and q.stride(1) == out.stride(1) == 1
+    assert q.dtype == w.absorb.dtype == w.expand.dtype == out.dtype
+    assert q.shape[1] >= heads * (dim + P) - P and out.shape[1] == heads * vdim
+    if window > 0:
+        max_keys = min(max_keys, window) if max_keys else window
+    # absorbed queries, then merged rows: a workspace that only kernels see
+    work = torch.empty(rows * heads * (D + R), dtype=q.dtype, device=q.device)
+    ql = work.data_ptr()
+    lat = ql + rows * heads * D * 2
+    values = w.expand.data_ptr() + heads * dim * R * 2
+    sink = w.sink
+    assert sink is None or (sink.shape == (heads,) and sink.is_contiguous()
+                            and sink.dtype == q.dtype and sink.is_cuda)
+    qp, qst = q.data_ptr(), q.stride(0)
+    splits, part = _latent_shares(rows, heads, R, max_keys, q.device)
+    a = _LatentStepArgs(
+        append=_append_of(qp, qst, dim, dim + P, ql, heads * D, R, D, kv, w,
+                          cache, pos, seq, block_table, heads, eps, q),
+        absorb=_HeadLinearArgs(x=qp, xst=qst, xh=dim + P, w=w.absorb.data_ptr(),
+                               out=ql, ost=heads * D, oh=D, T=rows, H=heads,
+                               N=R, K=dim),
+        rows=_LatentRowsArgs(
+            q=ql, cache=cache.data_ptr(), pos=pos.data_ptr(),
+            seq=seq.data_ptr(), bt=block_table.data_ptr(), part=_p(part),
+            out=lat, MB=block_table.shape[1], rows=rows, H=heads, R=R, P=P,
+            splits=splits, window=window, scale=scale, sink=_p(sink)),
+        values=_HeadLinearArgs(x=lat, xst=heads * R, xh=R, w=values,
+                               out=out.data_ptr(), ost=out.stride(0), oh=vdim,
+                               T=rows, H=heads, N=vdim, K=R))
+    if gate is not None:
+        assert gate.shape == (rows, heads * vdim) and gate.stride(1) == 1
+        assert gate.dtype == q.dtype
+        v = a.values
+        v.gate, v.gst, v.gh = gate.data_ptr(), gate.stride(0), vdim
+    _check(library().sv_latent_step(ctypes.byref(a), _stream()), "latent_step")
+    return True
 
 
 # ---------------------------------------------------------------------------
@@ -1823,16 +1939,19 @@ def moe_gemm(x: torch.Tensor, w: torch.Tensor, plan: MoePlan, gated: bool,
     min(g, limit) sigmoid(alpha g) (clamp(u, limit) + shift) of w = [gate;
     up], in slot order.  Else: slots x (T * top, K) -> pairs."""
     pairs = plan.order.shape[0]
-    N, K = w.shape[1] // (2 if gated else 1), w.shape[2]
-    assert x.stride(1) == 1 and x.shape[1] == K and w.is_contiguous()
-    assert x.dtype == w.dtype and w.shape[1] == N * (2 if gated else 1)
-    assert x.shape[0] == (plan.coef.shape[0] if gated else pairs)
+    _, rows, K = w.shape
+    T, cols = x.shape
+    N = rows // 2 if gated else rows
+    assert x.stride(1) == 1 and cols == K and w.is_contiguous()
+    assert x.dtype == w.dtype and rows == (2 * N if gated else N)
+    assert T == (plan.coef.shape[0] if gated else pairs)
     out = torch.empty(pairs, N, dtype=x.dtype, device=x.device)
-    a = _MoeGemmArgs(x=_p(x), xst=x.stride(0), w=_p(w), out=_p(out),
-                     order=_p(plan.order), tiles=_p(plan.tiles),
+    a = _MoeGemmArgs(x=x.data_ptr(), xst=x.stride(0), w=w.data_ptr(),
+                     out=out.data_ptr(), order=plan.order.data_ptr(),
+                     tiles=plan.tiles.data_ptr(),
                      top=plan.coef.shape[1] if gated else 0, N=N, K=K,
                      max_tiles=plan.tiles.shape[0], alpha=alpha, limit=limit,
-                     shift=shift, rows=x.shape[0])
+                     shift=shift, rows=T)
     assert plan.how == MOE_PLAIN or (x.dtype == torch.bfloat16
                                      and _aligned((N, K), x))
     _check(library().sv_moe_gemm(ctypes.byref(a), plan.how, int(gated),

@@ -27,6 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
+from ..ops.serving import unseen
 from . import comm
 from . import parallel_state as ps
 from .mappings import (
@@ -356,6 +357,9 @@ def linear_with_async_allreduce(input_, weight, bias=None,
         out = _ops.skinny_or_none(input_, weight, sequence_parallel_enabled)
         if out is not None:
             return out
+    # a served step spends more of its time here than on the device
+    if not sequence_parallel_enabled and unseen(input_, weight, bias):
+        return _forward_gemm(input_, weight, bias)
     args = cast_if_autocast_enabled(input_, weight, bias)
     with torch.amp.autocast("cuda", enabled=False):
         return LinearWithAsyncCommunication.apply(

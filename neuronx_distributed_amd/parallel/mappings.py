@@ -9,6 +9,7 @@ eager autograd.Functions over RCCL (no XLA graph semantics needed).
 
 import torch
 
+from ..ops.serving import unseen
 from . import comm
 from . import parallel_state as ps
 
@@ -86,10 +87,14 @@ class _GatherFromModelParallelRegion(torch.autograd.Function):
 
 
 def copy_to_tensor_model_parallel_region(input_):
+    if unseen(input_) and not input_.requires_grad:
+        return input_
     return _CopyToModelParallelRegion.apply(input_)
 
 
 def reduce_from_tensor_model_parallel_region(input_):
+    if unseen(input_) and not input_.requires_grad:
+        return _ReduceFromModelParallelRegion.forward(None, input_)
     return _ReduceFromModelParallelRegion.apply(input_)
 
 

@@ -229,3 +229,37 @@ def test_every_cut_is_one_that_the_launcher_takes():
                     assert 1 <= splits <= K // 256 and not (glu and N % 32)
                     assert splits == 1 or splits * -(-N // 128) <= 256
     assert 1 in taken and len(taken) > 5
+
+
+def test_nobody_is_passed_by():
+    """Calls go past an autograd function only where nobody would miss it."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from neuronx_distributed_amd.ops import swiglu
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.randn(3, 16)
+    assert not sv.unseen(x)
+    want = swiglu(x.clone().requires_grad_())
+    assert want.requires_grad
+    with torch.no_grad():
+        assert sv.unseen(x, None, torch.nn.Parameter(x))
+        assert torch.equal(swiglu(x), want)
+        assert not sv.unseen(x, x.as_subclass(Sub))
+        with Mode():
+            assert not sv.unseen(x)
+        with torch.autograd.forward_ad.dual_level():
+            assert not sv.unseen(x)
+        seen = []
+        torch.vmap(lambda t: seen.append(sv.unseen(t)) or t)(x)
+        assert seen == [False]
+        with torch.autocast("cuda"):
+            assert not sv.unseen(x) or not torch.is_autocast_enabled("cuda")
+    with torch.inference_mode():
+        assert sv.unseen(x)
