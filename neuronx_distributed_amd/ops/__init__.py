@@ -385,6 +385,67 @@ def apply_rotary_polar_compatible(query, key, freqs):
 
 
 # ---------------------------------------------------------------------------
+# weight gradients
+# ---------------------------------------------------------------------------
+
+def turn_rule(T: int, N: int, K: int):
+    """Which operands of dy^T x, dy (T, N) and x (T, K), are turned first, so that
+    the library reads them along T: (dy, x).  It reaches 1.05 PFLOP/s with none,
+    1.23 with one and up to 1.55 with both; turning runs at 5.7 TB/s.  Lines, with
+    the time without it and with it in us: the smaller one from 1600 rows and 20
+    million weights (8192 rows, 22016 x 4096: 1430 -> 1222, 32000 x 4096: 2079 ->
+    1552; 2048, 4096 x 11008: 212 -> 159; but 8192, 2048 x 5632: 175 -> 175, and
+    800, 22016 x 4096: 162 -> 205); both below 2600 rows, where the
+    library has no good form for one (1200, 32000 x 4096: 342 -> 278, with one
+    364), unless one is narrow (2048, 3584 x 18944: 275 -> 302, with one 259),
+    and of widths from 8192 (8192, 8192 x 8192: 940 -> 764, with one 797)."""
+    least = min(N, K)
+    if T < 1100 or N * K < 20_000_000:
+        return False, False
+    if least >= 8192 or (T < 2600 and least >= 4096):
+        return True, True
+    return (N <= K, N > K) if T >= 1600 else (False, False)
+
+
+def _turned(x: torch.Tensor) -> torch.Tensor:
+    """x (T, K) as a view of its columns laid out in rows.  64 words beside them
+    keep the rows of a power of two off one memory channel (8192 rows of 4096:
+    23.3 us, without 24.6; the product of it 204, without 225)."""
+    T, K = x.shape
+    pitch = (T + 63) // 64 * 64 + 64
+    out = torch.empty(K, pitch, dtype=x.dtype, device=x.device)
+    if _require_lib().transpose_words(
+            _ptr(x), ctypes.c_long(x.stride(0)), _ptr(out), ctypes.c_long(pitch),
+            T, K, _stream()):
+        raise RuntimeError("transpose_words failed")
+    return out[:, :T].t()
+
+
+def weight_grads(grads, x: torch.Tensor):
+    """[dy^T x for dy in grads] of dy (T, N) and x (T, K)."""
+    T, K = x.shape
+    if T < 1100 or not x.is_cuda:              # as in the rule, for all
+        return [g.t().matmul(x) for g in grads]
+    from .serving import unseen
+
+    def turns(t):
+        return t.is_cuda and t.dtype == torch.bfloat16 and t.stride(1) == 1 and \
+            not (t.shape[1] | t.stride(0)) & 7 and not t.data_ptr() & 15
+
+    ways = [(False, False)] * len(grads)
+    if turns(x) and unseen(x, *grads) and \
+            x.get_device() == torch._C._cuda_getDevice():
+        ways = [turn_rule(T, g.shape[1], K) for g in grads]
+        # x is turned once for all of them
+        if turn_rule(T, sum(g.shape[1] for g in grads), K)[1]:
+            ways = [(dy, True) for dy, _ in ways]
+    if any(way for _, way in ways):
+        xt = _turned(x)
+    return [(_turned(g) if dy and turns(g) else g).t().matmul(xt if way else x)
+            for g, (dy, way) in zip(grads, ways)]
+
+
+# ---------------------------------------------------------------------------
 # SwiGLU
 # ---------------------------------------------------------------------------
 

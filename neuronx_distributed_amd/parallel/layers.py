@@ -27,6 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
+from ..ops import weight_grads
 from ..ops.serving import unseen
 from . import comm
 from . import parallel_state as ps
@@ -192,7 +193,7 @@ class _RPLOverlappedLinearRS(torch.autograd.Function):
         grad_input = g.matmul(weight)
         go2d = g.reshape(-1, g.shape[-1])
         in2d = input_parallel.reshape(-1, input_parallel.shape[-1])
-        grad_weight = go2d.t().matmul(in2d)
+        (grad_weight,) = weight_grads([go2d], in2d)
         return grad_input, grad_weight
 
 
@@ -335,7 +336,7 @@ class LinearWithAsyncCommunication(torch.autograd.Function):
         if ctx.compute_weight_gradient:
             go2d = grad_output.reshape(-1, grad_output.shape[-1])
             in2d = total_input.reshape(-1, total_input.shape[-1])
-            grad_weight = go2d.t().matmul(in2d)
+            (grad_weight,) = weight_grads([go2d], in2d)
             if ctx.use_bias:
                 grad_bias = go2d.sum(dim=0)
         elif ctx.use_bias:

@@ -21,6 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
+from ..ops import weight_grads
 from . import comm
 from . import parallel_state as ps
 from .layers import BaseParallelLinear, default_init_method
@@ -109,8 +110,9 @@ class _QKVLinearWithAsyncCommunication(torch.autograd.Function):
         gk = gk.contiguous()
         gv = gv.contiguous()
         grad_input = gq.matmul(wq)
-        grad_input += gk.matmul(wk)
-        grad_input += gv.matmul(wv)
+        rows = grad_input.view(-1, grad_input.shape[-1])
+        for g, w in ((gk, wk), (gv, wv)):      # sums inside the products
+            rows.addmm_(g.view(-1, g.shape[-1]), w)
 
         handle = None
         if ctx.sequence_parallel:
@@ -136,9 +138,7 @@ class _QKVLinearWithAsyncCommunication(torch.autograd.Function):
         gq2 = gq.reshape(-1, gq.shape[-1])
         gk2 = gk.reshape(-1, gk.shape[-1])
         gv2 = gv.reshape(-1, gv.shape[-1])
-        gwq = gq2.t().matmul(in2d)
-        gwk = gk2.t().matmul(in2d)
-        gwv = gv2.t().matmul(in2d)
+        gwq, gwk, gwv = weight_grads([gq2, gk2, gv2], in2d)
         gbq = gq2.sum(0) if ctx.use_bias else None
         gbk = gk2.sum(0) if ctx.use_bias else None
         gbv = gv2.sum(0) if ctx.use_bias else None

@@ -263,3 +263,14 @@ def test_nobody_is_passed_by():
             assert not sv.unseen(x) or not torch.is_autocast_enabled("cuda")
     with torch.inference_mode():
         assert sv.unseen(x)
+
+
+@pytest.mark.parametrize("T,N,K,want", [
+    (1099, 32000, 4096, (False, False)), (1100, 32000, 4096, (True, True)),
+    (2600, 32000, 4096, (False, True)), (1599, 3584, 18944, (False, False)),
+    (1600, 3584, 18944, (True, False)), (8192, 4096, 4096, (False, False)),
+    (8192, 4096, 11008, (True, False)), (16384, 8192, 8192, (True, True))])
+def test_operands_of_a_weight_gradient(T, N, K, want):
+    from neuronx_distributed_amd.ops import turn_rule
+
+    assert turn_rule(T, N, K) == want

@@ -948,3 +948,40 @@ def test_norms_read_a_32_bit_weight_as_it_is(form):
                                    atol=1e-5)
     assert y.dtype == torch.bfloat16
     torch.testing.assert_close(y.double(), ref, rtol=2.0 ** -8, atol=1e-5)
+
+
+@pytest.mark.parametrize("T,K,pitch", [
+    (1, 8, 8), (7, 72, 80), (8, 64, 64), (65, 136, 136), (257, 520, 1024),
+    (1111, 4096, 4096)])
+def test_turned_rows(T, K, pitch):
+    """Remainders of the 8 x 8 words of a lane and of the tiles of a workgroup."""
+    x = torch.randn(T, pitch, device="cuda", dtype=torch.bfloat16)[:, :K]
+    xt = ops._turned(x)
+    assert torch.equal(xt, x) and xt.t().stride(1) == 1
+
+
+@pytest.mark.parametrize("T,K,widths,aligned", [
+    (1111, 4096, (8200,), True),             # both operands
+    (2601, 2048, (8192, 1024, 1024), True),  # x for all of them
+    (2601, 11008, (2056,), True),            # dy
+    (2600, 8200, (8192,), True),             # both, of wide ones
+    (2601, 2044, (12288,), False),           # rows that are not whole words
+    (300, 64, (32,), True)])                 # as they are
+def test_weight_gradients(T, K, widths, aligned):
+    x = torch.randn(T, K, device="cuda", dtype=torch.bfloat16)
+    grads = [torch.randn(T, n, device="cuda", dtype=torch.bfloat16)
+             for n in widths]
+    got = ops.weight_grads(grads, x)
+    assert not aligned or any(ops.turn_rule(T, sum(widths), K)) == (T > 1000)
+    for g, w in zip(grads, got):
+        want = g.float().t() @ x.float()
+        # rounded to 8 bits; sums of T terms in float32, in any order
+        bound = want.abs() * 2 ** -8 + 2 * T * 2 ** -24 * \
+            (g.float().abs().t() @ x.float().abs())
+        assert w.shape == want.shape and w.is_contiguous()
+        assert ((w.float() - want).abs() <= bound).all()
+    # a backward that is differentiated itself does without
+    with torch.enable_grad():
+        gx = grads[0].clone().requires_grad_()
+        (w,) = ops.weight_grads([gx], x)
+        assert w.requires_grad
