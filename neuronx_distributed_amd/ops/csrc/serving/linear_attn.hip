@@ -395,7 +395,9 @@ struct ChunkArgs {
   float* N;                 // [n_chunks][H][D] (gated): N, then n before
   short* P;                 // [n_chunks][H][3][E][D] state before the chunk; if
                             //   there is no U [n_chunks][H][E / 32][3][D / 16]
-                            //   [64][8]: keys 16 c + 8 hi + 0..7 of column col
+                            //   [64][8]: keys 16 c + 8 hi + 0..7 of column col;
+                            //   or null: nothing is left between chunks (timed, D
+                            //   128, E a multiple of 64, no VT and U)
   float* mst;               // [n_chunks][H] m before the chunk (gated)
   short* VT;                // [n_chunks][H][E][256] V^T, activated; or null
                             //   (timed, D 64 or 128, E a multiple of 64)
@@ -1146,7 +1148,7 @@ memory_outputs_kernel(ChunkArgs x) {
     }
 }
 
-// ---- timed states of D = 64 or 128 by a multiple of 64, chunk after chunk ---
+// ---- timed states of D = 64 by a multiple of 64, chunk after chunk ----------
 // One workgroup carries DP keys x ET columns of a head's state through its
 // segment: the state stays in the accumulators, is scaled by what a chunk
 // forgets, and the chunk's weighted keys and values are added to it, 64 tokens a
@@ -1155,12 +1157,10 @@ memory_outputs_kernel(ChunkArgs x) {
 // transposing reads; values come through registers, two ahead as well, where
 // they are weighted and split.  One barrier a piece, which waits by count.
 //
-// The states of all chunks at once and a scan over them moved 70 MB of 32 bits
-// out and back and took two launches (2 x 2048 tokens, 128 heads of 128 x 64: 49 +
-// 30 us, now 55).  The planes' 107 MB and the values' 67 are what is left.
-template <int DP>
+// The states of all chunks at once and a scan over them move 32 bits out and back and
+// take two launches; the planes and the values are what is left.
 __global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
-  constexpr int MT = DP / 32, ET = 128 / MT;   // tiles of keys; columns
+  constexpr int DP = 64, MT = DP / 32, ET = 128 / MT;   // tiles of keys; columns
   constexpr int NC = DP / 16, SL = DP / 8, VS = ET / 8;
   constexpr int LK = DP / 32, LV = ET / 32;    // words of a thread and piece
   constexpr int PLANE = 64 * ET * 2, VA = 6;   // pieces that values are ahead
@@ -1187,7 +1187,7 @@ __global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
   const int col = lane & 31, hi = lane >> 5;
   const int m = wid % MT, n = wid / MT;
 
-  auto turn = [](int r) { return SL == 16 ? row_turn(r) : value_turn<SL>(r); };
+  auto turn = [](int r) { return value_turn<SL>(r); };
   const short* kp = (const short*)a.k + row0 * a.kst + h / (a.H / a.G) * DP;
   const short* vp = (const short*)a.v + row0 * a.vst + (long)h * E + e0;
   // Pieces past the last are that one again, so that the words on their way keep
@@ -1250,16 +1250,15 @@ __global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
   // this lane's part of the addresses of transposing reads (bytes)
   const int tr_key = 4 * hi + ((lane & 15) >> 2);
   const int tr_col = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
-  const int kx = SL == 16 ? tr_lane(lane)
-                          : tr_key * DP * 2 + tr_col + value_turn<SL>(tr_key) * 16;
-  const int vx = tr_key * ET * 2 + tr_col + (VS == 8 ? value_turn<8>(tr_key) : 0) * 16;
+  const int kx = tr_key * DP * 2 + tr_col + value_turn<SL>(tr_key) * 16;
+  const int vx = tr_key * ET * 2 + tr_col + value_turn<8>(tr_key) * 16;
   // the weighted values of a piece, split
   auto convert = [&](int i, const float* w, char* vb, const uint4v* v)
       __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < LV; ++p) {
       const int r = (p * 256 + tid) / VS;
-      const int s = tid % VS ^ (VS == 8 ? value_turn<8>(r) : 0);
+      const int s = tid % VS ^ value_turn<8>(r);
       float f[8];
       uint4v u[3];
       unpack8(64 * i + r < rows ? v[p] : uint4v{0, 0, 0, 0}, f);
@@ -1305,8 +1304,7 @@ __global__ void __launch_bounds__(256, 2) memory_carry_kernel(ChunkArgs x) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         kf[c].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr4)(
-            kb + (SL == 16 ? (kx ^ (64 * m) ^ (32 * u)) : (kx ^ (64 * m))) +
-            (16 * c + 8 * u) * DP * 2));
+            kb + (kx ^ (64 * m)) + (16 * c + 8 * u) * DP * 2));
 #pragma unroll
         for (int z = 0; z < 3; ++z)
           vf[c][z].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr4)(
@@ -1671,12 +1669,454 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   }
 }
 
+// ---- timed memories of D = 128, states and outputs in one pass -----------------
+// One workgroup takes 64 columns of a head through its segment, 64 tokens a piece:
+// nothing but queries, keys, values, gates and results moves.  Three waves of a SIMD
+// do different things, since one alone issues a vector instruction every eight
+// cycles.  Four hold the state in accumulators, 16 columns each; for every piece they
+// multiply its planes by the queries (the accumulators' row order is the contraction
+// order), scale it and add the weighted keys and values.  Four weight the scores
+// within the piece, 16 tokens each, and add their products a piece later; the one with
+// the fewest scores also makes the next piece's gates.  Four ask for the next piece's
+// tiles, which come straight into LDS, and write the results of two pieces ago.  One
+// barrier a piece.  Bound by what one wave issues: the states' waves alone take 83 of
+// the 105 us below, where a product of 16 x 16 x 32 takes a lone wave 31 cycles, not
+// 16; the tiles alone take 57, a piece's latency each time.  128 heads of 128 x 64 in
+// us, carried states and outputs in chunks of 256 as above | one pass:
+//   2 x 2048 tokens 181 | 105      4 x 500 104 | 62     1 x 4096 177 | 158
+//   64 heads: 1500 tokens 60 | 56, 3 x 500 52 | 38, 50 35 | 19 (its one launch)
+// With two waves a SIMD, states and everything else, 2 x 2048 took 130; with four of
+// 128 registers 133; the gates beside the results' waves 116.
+constexpr int PASS_D = 128;
+template <int N> struct Count { static constexpr int value = N; };
+
+__global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
+  constexpr int DP = PASS_D, L = 64, ET = 64;
+  constexpr int TILE = L * DP * 2, VT = L * ET * 2, PART = ET * L * 4;
+  // apart by name, so that a read of one need not wait for the words on their
+  // way into another
+  __shared__ __attribute__((aligned(16))) char q0[TILE], q1[TILE], k0[TILE], k1[TILE],
+      v0[VT], v1[VT];
+  // the results: four columns of a token in a word, the tokens of 16 words turned by
+  // the columns
+  __shared__ __attribute__((aligned(16))) char s_part[3 * PART];
+  // log forgets and steps; what is left of a token at the end of its 16, and of the
+  // piece; what a piece leaves of the state
+  __shared__ __attribute__((aligned(16))) float s_b[2 * L], s_i[2 * L], s_far[2 * L],
+      s_w[2 * L];
+  __shared__ float s_keep[2];
+  const MemoryArgs& a = x.a;
+  const int E = a.E;
+  // heads that share keys are on one XCD
+  const int units = a.H * (E / ET), per = (units + 7) / 8;
+  const int unit = blockIdx.x % 8 * per + blockIdx.x / 8 % per;
+  const int sg = blockIdx.x / 8 / per;
+  if (unit >= units) return;             // the whole workgroup
+  const int h = unit / (E / ET), e0 = unit % (E / ET) * ET;
+  const int row0 = a.seg[4 * sg + 1], rows = a.seg[4 * sg + 2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, quad = lane >> 4;
+  const int pieces = (rows + L - 1) / L;
+  auto meet = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);              // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // transposing reads: 16 lanes turn 4 tokens by 16 columns; tokens 32 c + 16 u + 4
+  // quad ... of columns 16 n ... are at (kx ^ 32 n) + (32 c + 16 u) rows
+  const int turn_row = 4 * quad + (col >> 2), turn_slot = col >> 1 & 1;
+  const int kx = turn_row * 256 + (row_turn(turn_row) ^ turn_slot) * 16 + (col & 1) * 8;
+  const int vx = turn_row * 128 + (value_turn<8>(turn_row) ^ turn_slot) * 16 +
+                 (col & 1) * 8;
+  union Turned { tr4 t[2]; bf16x8 bf; uint u[4]; };
+  auto turned = [&](const char* at, int pitch) __attribute__((always_inline)) {
+    Turned f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      f.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr4)(at + 16 * u * pitch));
+    return f;
+  };
+  // four columns e4 of token t
+  auto part_at = [](int e4, int t) __attribute__((always_inline)) {
+    return (e4 * 64 + (t ^ (e4 >> 1))) * 16;
+  };
+
+  if (wid < 4) {
+    float* Sp = a.S + ((long)a.seg[4 * sg] * a.H + h) * DP * E +
+                (long)(4 * quad) * E + e0 + 16 * wid + col;
+    f32x4 S[8] = {};                     // keys 16 d + 4 quad ... of column col
+    if (a.seg[4 * sg + 3] > 0)
+#pragma unroll
+      for (int d = 0; d < 8; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[d][j] = Sp[(long)(16 * d + j) * E];
+    // 8 bytes of row col, slot s: at ^ 16 s
+    const int qx = col * 256 + (row_turn(col) ^ (quad >> 1)) * 16 + (quad & 1) * 8;
+    const int wx = vx ^ (32 * wid), ox = part_at(4 * wid + quad, col);
+    // Words are read from LDS a part ahead of the products that need them, and
+    // converted beside the products before.
+    auto piece = [&](int i, const char* qb, const char* kb, const char* vb, char* part)
+        __attribute__((always_inline)) {
+      const int now = i & 1;
+      f32x4 o[4] = {}, w[2][2];
+      frag_u pf[2][3], vf[2][3];
+      Turned qf[2][4], kf[2][8], v[2];
+      auto read_q = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            qf[p & 1][n].t[u] =
+                *(const tr4*)(qb + n * 4096 + (qx ^ (64 * p + 32 * u)));
+      };
+      auto read_k = [&](int c, int d0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = d0; d < d0 + 4; ++d)
+          kf[c][d] = turned(kb + (kx ^ (32 * d)) + c * 32 * 256, 256);
+      };
+      auto split_s = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          uint t[3];
+          split3(S[2 * p + u / 2][u % 2 * 2], S[2 * p + u / 2][u % 2 * 2 + 1], t);
+#pragma unroll
+          for (int z = 0; z < 3; ++z) pf[p & 1][z].u[u] = t[z];
+        }
+      };
+      auto split_v = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          uint t[3];
+          split3(__uint_as_float(v[c].u[u] << 16) * w[c][u / 2][u % 2 * 2],
+                 __uint_as_float(v[c].u[u] & 0xffff0000u) *
+                     w[c][u / 2][u % 2 * 2 + 1], t);
+#pragma unroll
+          for (int z = 0; z < 3; ++z) vf[c][z].u[u] = t[z];
+        }
+      };
+      auto outputs = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+          for (int n = 0; n < 4; ++n)
+            o[n] = mfma16(pf[p & 1][z].bf, qf[p & 1][n].bf, o[n]);
+      };
+      auto updates = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+          for (int d = 0; d < 8; ++d) S[d] = mfma16(kf[c][d].bf, vf[c][z].bf, S[d]);
+      };
+      // reads first, then `each` other instructions behind every product
+      auto order = [](auto reads, auto products, auto each)
+          __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_group_barrier(0x100, decltype(reads)::value, 0);
+#pragma unroll
+        for (int y = 0; y < decltype(products)::value; ++y) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, decltype(each)::value, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+      read_q(0);
+      const float keep = s_keep[now];
+      read_q(1);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        v[c] = turned(vb + wx + c * 32 * 128, 128);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          w[c][u] = *(const f32x4*)(s_w + now * L + 32 * c + 16 * u + 4 * quad);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      split_s(0);
+      __builtin_amdgcn_sched_barrier(0);
+      outputs(0);
+      split_s(1);
+      order(Count<0>{}, Count<12>{}, Count<4>{});
+      read_q(2);
+      outputs(1);
+      split_s(2);
+      order(Count<0>{}, Count<12>{}, Count<4>{});
+      read_q(3);
+      outputs(2);
+      split_s(3);
+      order(Count<8>{}, Count<12>{}, Count<4>{});
+      read_k(0, 0);
+      read_k(0, 4);
+      outputs(3);
+      split_v(0);
+#pragma unroll
+      for (int d = 0; d < 8; ++d) S[d] *= keep;
+      order(Count<16>{}, Count<12>{}, Count<8>{});
+#pragma unroll
+      for (int n = 0; n < 4; ++n) *(f32x4*)(part + ox + 256 * n) = o[n];
+      read_k(1, 0);
+      read_k(1, 4);
+      updates(0);
+      split_v(1);
+      order(Count<16>{}, Count<24>{}, Count<3>{});
+      updates(1);
+    };
+    meet();
+    char *part = s_part, *next = s_part + PART, *after = s_part + 2 * PART;
+    for (int i = 0; i < pieces; ++i) {
+      piece(i, i & 1 ? q1 : q0, i & 1 ? k1 : k0, i & 1 ? v1 : v0, part);
+      meet();
+      char* p = part;
+      part = next, next = after, after = p;
+    }
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) Sp[(long)(16 * d + j) * E] = S[d][j];
+    meet();
+    return;
+  }
+
+  if (wid < 8) {
+    const float skip = bits2f(((const short*)a.skip)[h]);
+    const float ib = bits2f(((const short*)a.ib)[h]);
+    const float rate = -expf(bits2f(((const short*)a.fb)[h]));
+    const float* raw = a.gates + (long)row0 * a.H + h;
+    auto load_gate = [&](int i) __attribute__((always_inline)) {
+      return raw[(long)min(L * i + lane, rows - 1) * a.H];
+    };
+    auto gates = [&](int i, float g) __attribute__((always_inline)) {
+      const float step = L * i + lane < rows ? softplus_f(g + ib) : 0.f;
+      float F = rate * step;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float before = __shfl_up(F, off, 64);
+        if (lane >= off) F += before;
+      }
+      const float end = __shfl(F, 63, 64), near = __shfl(F, lane | 15, 64);
+      const int at = (i & 1) * L + lane;
+      s_b[at] = F;
+      s_i[at] = step;
+      s_far[at] = expf(near - F) * step;
+      s_w[at] = expf(end - F) * step;
+      if (lane == 0) s_keep[i & 1] = expf(end);
+    };
+    const int rx = col * 256 + (row_turn(col) ^ quad) * 16;
+    // tokens 16 n ... of a piece
+    auto run = [&](auto number) __attribute__((always_inline)) {
+      constexpr int n = decltype(number)::value, NP = n / 2 + 1;
+      f32x4 pv[4];                       // columns 16 et + 4 quad ... of token t
+      const int t = 16 * n + col;
+      float inter = 0.f;
+      int at[4];
+#pragma unroll
+      for (int et = 0; et < 4; ++et) at[et] = part_at(4 * et + quad, t);
+      auto add = [&](char* part) __attribute__((always_inline)) {
+        f32x4 o[4];
+#pragma unroll
+        for (int et = 0; et < 4; ++et) o[et] = *(f32x4*)(part + at[et]);
+#pragma unroll
+        for (int et = 0; et < 4; ++et) *(f32x4*)(part + at[et]) = inter * o[et] + pv[et];
+      };
+      auto piece = [&](int i, const char* qb, const char* kb, const char* vb)
+          __attribute__((always_inline)) {
+        frag_u qf[4], kf[4][n + 1];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          qf[c].u4 = *(const uint4v*)(qb + n * 4096 + (rx ^ (64 * c)));
+#pragma unroll
+          for (int J = 0; J <= n; ++J)
+            kf[c][J].u4 = *(const uint4v*)(kb + J * 4096 + (rx ^ (64 * c)));
+        }
+        const float* b = s_b + (i & 1) * L;
+        const float bt = b[t];
+        const f32x4 bs = *(const f32x4*)(b + 16 * n + 4 * quad);
+        const f32x4 step = *(const f32x4*)(s_i + (i & 1) * L + 16 * n + 4 * quad);
+        f32x4 far[n + 1];
+        float from[n + 1];
+#pragma unroll
+        for (int J = 0; J < n; ++J) {
+          far[J] = *(const f32x4*)(s_far + (i & 1) * L + 16 * J + 4 * quad);
+          from[J] = b[16 * J + 15];
+        }
+        f32x4 acc[2 * NP] = {};
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int J = 0; J <= n; ++J) acc[J] = mfma16(kf[c][J].bf, qf[c].bf, acc[J]);
+        inter = __expf(bt);
+#pragma unroll
+        for (int J = 0; J < n; ++J) acc[J] *= far[J] * __expf(bt - from[J]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float w = acc[n][j] * (__expf(bt - bs[j]) * step[j]);
+          const int s = 4 * quad + j;
+          acc[n][j] = (s > col ? 0.f : w) + (s == col ? skip : 0.f);
+        }
+#pragma unroll
+        for (int et = 0; et < 4; ++et) pv[et] = f32x4{};
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          Turned v[4];
+#pragma unroll
+          for (int et = 0; et < 4; ++et)
+            v[et] = turned(vb + (vx ^ (32 * et)) + p * 32 * 128, 128);
+          frag_u pf[3];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            uint w[3];
+            split3(acc[2 * p + u / 2][u % 2 * 2], acc[2 * p + u / 2][u % 2 * 2 + 1], w);
+#pragma unroll
+            for (int z = 0; z < 3; ++z) pf[z].u[u] = w[z];
+          }
+#pragma unroll
+          for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int et = 0; et < 4; ++et)
+              pv[et] = mfma16(v[et].bf, pf[z].bf, pv[et]);
+        }
+      };
+      float g = 0.f;
+      if (n == 0 && pieces) {
+        gates(0, load_gate(0));
+        g = load_gate(1);
+      }
+      meet();
+      char *part = s_part + 2 * PART, *next = s_part, *after = s_part + PART;
+      for (int i = 0; i < pieces; ++i) {
+        if (n == 0) {
+          gates(i + 1, g);
+          g = load_gate(i + 2);
+        }
+        if (i) add(part);                // of the piece before
+        piece(i, i & 1 ? q1 : q0, i & 1 ? k1 : k0, i & 1 ? v1 : v0);
+        meet();
+        char* p = part;
+        part = next, next = after, after = p;
+      }
+      if (pieces) add(part);
+      meet();
+    };
+    if (wid == 4) run(Count<0>{});
+    else if (wid == 5) run(Count<1>{});
+    else if (wid == 6) run(Count<2>{});
+    else run(Count<3>{});
+    return;
+  }
+
+  const int ft = tid - 512, n = wid - 8;
+  const int hk = h / (a.H / a.G);
+  const short* qp = (const short*)a.q + row0 * a.qst + hk * DP;
+  const short* kp = (const short*)a.k + row0 * a.kst + hk * DP;
+  const short* vp = (const short*)a.v + row0 * a.vst + (long)h * E + e0;
+  const int qst = (int)a.qst * 2, kst = (int)a.kst * 2, vst = (int)a.vst * 2;
+  const int rt = ft / 16, rv = ft / 8, turn_t = (ft % 16 ^ row_turn(rt)) * 16;
+  const int qo = rt * qst + turn_t, ko = rt * kst + turn_t;
+  const int vo = rv * vst + (ft % 8 ^ value_turn<8>(rv)) * 16;
+  // rows past the last come as zeros
+  auto issue = [&](int i, char* qb, char* kb, char* vb) __attribute__((always_inline)) {
+    const int end = min(rows - L * i, L) - 1;
+    const auto qs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(qp + (long)L * i * a.qst), 0, end * qst + DP * 2, 0x00027000);
+    const auto ks = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(kp + (long)L * i * a.kst), 0, end * kst + DP * 2, 0x00027000);
+    const auto vs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(vp + (long)L * i * a.vst), 0, end * vst + ET * 2, 0x00027000);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int at = (p * 256 + n * 64) * 16;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(qs, (lds_ptr)(qb + at), 16,
+                                               qo + p * 16 * qst, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ks, (lds_ptr)(kb + at), 16,
+                                               ko + p * 16 * kst, 0, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          vs, (lds_ptr)(vb + (p * 256 + n * 64) * 16), 16, vo + p * 32 * vst, 0, 0, 0);
+  };
+  // two rows of 64 columns, 16 bytes a lane
+  const int r0 = 16 * n + (lane >> 3) * 2, c8 = lane & 7;
+  const long at = (long)h * E + e0 + c8 * 8;
+  uint4v z[2], znext[2];
+  auto load_z = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+      znext[y] = *(const uint4v*)((const short*)a.z + at +
+                                  (long)(row0 + min(L * i + r0 + y, rows - 1)) * a.zst);
+  };
+  uint4v w[2];
+  auto results = [&](const char* part) __attribute__((always_inline)) {
+    float v[2][8];
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        load4((const float*)(part + part_at(2 * c8 + u, r0 + y)), v[y] + 4 * u);
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      float g[8];
+      unpack8(z[y], g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        w[y][j] = pack_bf16x2(v[y][2 * j] * silu_f(g[2 * j]),
+                              v[y][2 * j + 1] * silu_f(g[2 * j + 1]));
+    }
+  };
+  auto store = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+      if (L * i + r0 + y < rows)
+        *(uint4v*)((short*)a.out + (long)(row0 + L * i + r0 + y) * a.H * E + at) = w[y];
+  };
+  // what was asked for is here
+  auto arrive = []() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xf70);               // vmcnt(0)
+    asm volatile("" ::: "memory");
+  };
+  if (pieces) {
+    issue(0, q0, k0, v0);
+    arrive();
+  }
+  meet();
+  const char *part = s_part + PART, *next = s_part + 2 * PART, *after = s_part;
+  for (int i = 0; i < pieces; ++i) {
+    if (i + 1 < pieces) issue(i + 1, i & 1 ? q0 : q1, i & 1 ? k0 : k1, i & 1 ? v0 : v1);
+    if (i) load_z(i - 1);                // for the next turn
+    if (i > 1) results(part);            // of two pieces ago
+    arrive();
+    if (i > 1) store(i - 2);
+    z[0] = znext[0], z[1] = znext[1];
+    meet();
+    const char* p = part;
+    part = next, next = after, after = p;
+  }
+  if (pieces) load_z(pieces - 1);
+  if (pieces > 1) {
+    results(part);
+    store(pieces - 2);
+  }
+  z[0] = znext[0], z[1] = znext[1];
+  meet();
+  if (pieces) {
+    results(next);
+    store(pieces - 1);
+  }
+}
+
 // wider column tiles read the keys less often, as long as the accumulators
 // leave registers for two workgroups per CU
 template <int DP, int GATE>
 static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
   const MemoryArgs& a = x.a;
   const long ch = (long)x.n_chunks * a.H;
+  if constexpr (GATE == TIMED && DP == PASS_D)
+    if (!x.P) {
+      const int units = a.H * (a.E / 64);
+      memory_pass_kernel<<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
+      return;
+    }
   if (!fixed_decay(GATE)) memory_gates_kernel<GATE><<<ch, MC_L, 0, stream>>>(x);
   if (GATE == TURNED) {
     const size_t lds = a.rot * sizeof(float);
@@ -1690,10 +2130,10 @@ static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
         memory_states_kernel<DP, GATE><<<ch * (a.E / 64), 256, 0, stream>>>(x);
         memory_scan_kernel<GATE><<<(long)x.n_seg * a.H * (DP / 64) * (a.E / 16),
                                    256, 0, stream>>>(x);
-      } else {
-        const int units = a.H * (a.E * DP / 4096);
-        memory_carry_kernel<DP>
-            <<<(long)x.n_seg * 8 * ((units + 7) / 8), 256, 0, stream>>>(x);
+      } else if constexpr (DP == 64) {
+        const int units = a.H * (a.E / 64);
+        memory_carry_kernel<<<(long)x.n_seg * 8 * ((units + 7) / 8), 256, 0,
+                              stream>>>(x);
       }
       memory_timed_kernel<DP><<<ch * 2 * (a.E / 64), 256, 0, stream>>>(x);
       return;
@@ -1722,6 +2162,9 @@ extern "C" int sv_memory_chunks(const ChunkArgs* x, int gating,
                  (x->a.D != 64 && x->a.D != 128)))
     return 1;
   if (!x->U && x->VT) return 1;
+  // states are carried for 64 keys; one pass, for 128, leaves none behind
+  if (!x->VT && !x->U && x->a.D != (x->P ? 64 : PASS_D)) return 1;
+  if (!x->P && (x->VT || x->U || x->a.qst >= 1 << 22)) return 1;
   // offsets of a chunk's rows are of 32 bits
   if (!x->VT && (x->a.kst >= 1 << 22 || x->a.vst >= 1 << 22)) return 1;
 #define MC(P)                                                     \

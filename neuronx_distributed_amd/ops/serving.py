@@ -1281,10 +1281,22 @@ def memory_carries(chunks: int, segments: int, state: int) -> bool:
     of the longest segment takes a workgroup 4 us; at once, 4096 elements of a
     chunk's state take 0.018 us of the device, and two launches more.  The
     longest segment is at most as long as all but one chunk a segment.
-    Whole calls, at once and carried: 2 x 2048 tokens, 128 heads of 128 x 64
-    222 and 184 us; 1000 tokens of 64 heads 46 and 46; 16384 tokens of 64 heads
-    419 and 424, of 16 heads of 64 x 64 105 and 286."""
+    Whole calls, at once and carried, of heads of 128 x 64: 2 x 2048 tokens, 128
+    heads 222 and 184 us; 1000 tokens of 64 heads 46 and 46; 16384 tokens of 64
+    heads 419 and 424; of 16 heads of 64 x 64 105 and 286."""
     return chunks - segments + 1 <= chunks * (state // 4096) / 217 + 2
+
+
+def memory_pass(chunks: int, segments: int, columns: int) -> bool:
+    """Does a timed memory of 128 keys go through its segments in one pass, a
+    workgroup for 64 of all heads' ``columns``?  A chunk of the longest segment
+    takes it 8.3 us, 12.4 where all CUs have one; states of all chunks at once and
+    outputs after them take 0.062 us for 64 columns of a chunk and 9 in all.  Whole
+    calls, those and one pass, over 223 sizes (1.37 in the mean): 64 heads of 64,
+    1500 tokens 54.5 and 55.1, 3000 82.7 and 100.8; 128 heads, 2 x 2048 181 and 105,
+    200 tokens 36 and 20; 16 heads, 1500 tokens 34.8 and 52.2.  The longest segment
+    is at most as long as all but one chunk a segment."""
+    return chunks - segments + 1 <= chunks * (columns // 64) / 80 + 2
 
 
 def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
@@ -1370,10 +1382,12 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         f32 = dict(dtype=torch.float32, device=q.device)
         tiled = timed and D in (64, 128) and E % 64 == 0 and \
             max(t.stride(0) for t in strided) < 1 << 22
-        U = None if tiled and memory_carries(nc, seg.shape[0], heads * D * E) \
+        once = tiled and D == 128 and memory_pass(nc, seg.shape[0], heads * E)
+        U = None if once or tiled and D == 64 and memory_carries(
+            nc, seg.shape[0], heads * D * E) \
             else torch.empty(nc, heads, E, D, **f32)
-        P = torch.empty(nc, heads, 3, E, D, dtype=torch.bfloat16,
-                        device=q.device)
+        P = None if once else torch.empty(nc, heads, 3, E, D,
+                                          dtype=torch.bfloat16, device=q.device)
         VT = None if tiled else \
             torch.empty(nc, heads, E, CHUNK, dtype=torch.bfloat16,
                         device=q.device)
@@ -1387,7 +1401,7 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
                        P=_p(P), VT=_p(VT), KA=_p(KA), norm_eps=eps)
         if turned:
             x.QA = _p(QA)
-        if timed:
+        if timed and not once:
             bic = torch.empty(2, heads, T, **f32)
             small = torch.empty(nc, heads, 4, **f32)
             x.b, x.i, x.tot = _p(bic[0]), _p(bic[1]), _p(small)

@@ -572,6 +572,46 @@ def test_timed_memory_of_rows_far_apart(monkeypatch, pitch, carried):
     _near(S[0], S_want, F32, "state", 2e-5)
 
 
+@pytest.mark.parametrize("H,G,P", [(6, 2, 64), (3, 1, 128), (16, 16, 64)])
+def test_timed_memory_in_one_pass(monkeypatch, H, G, P):
+    """Segments that end at, before and behind the 16 tokens of a wave, the 64 of a
+    piece and the turns of its buffers, from empty and from filled slots; against the
+    oracle, and against chunks."""
+    N = 128
+    lens, more = [1, 15, 17, 63, 64, 65, 128, 130, 193, 449], [70, 1, 300, 64, 2, 33,
+                                                              65, 192, 5, 16]
+    cases = [_ssm(a + b, H, G, N, P, 30 * i, BF16)
+             for i, (a, b) in enumerate(zip(lens, more))]
+    params = _ssm_params(H, BF16)
+    pd = [t.cuda() for t in params]
+    got = {}
+    for once in (True, False):
+        monkeypatch.setattr(sv, "memory_pass", lambda *a: once)
+        S = torch.full((10, H, N, P), 7.0, device="cuda")
+        out = []
+        for at, n in (([0] * 10, lens), (lens, more)):
+            x, B, C, z, raw = (torch.cat(t).cuda() for t in zip(*(
+                [t[a:a + k] for t in c] for c, a, k in zip(cases, at, n))))
+            seg, chunks, first = _segments([(9 - i, k, a) for i, (a, k) in
+                                            enumerate(zip(at, n))])
+            out.append(sv.memory_mix(C, B, x, sv.TimeGate(raw, *pd, z), S, None,
+                                     None, seg, H, chunks, first).split(n))
+        got[once] = [torch.cat([o[i] for o in out]) for i in range(10)], S
+    for i, c in enumerate(cases):
+        want, S_want = _ssm_want(c, params, H, G, N, P)
+        _near(got[True][0][i], want, BF16, i)
+        _near(got[True][1][9 - i], S_want, F32, i, 2e-5)
+        off = [(got[way][0][i].cpu().double() - want).norm() for way in got]
+        assert off[0] <= 1.05 * off[1] + 1e-6 * want.norm()
+
+
+def test_memories_of_one_pass():
+    assert sv.memory_pass(16, 2, 128 * 64)               # 2 x 2048 tokens
+    assert sv.memory_pass(6, 1, 64 * 64)                 # 1500 tokens
+    assert not sv.memory_pass(12, 1, 64 * 64)            # 3000 tokens
+    assert not sv.memory_pass(6, 1, 16 * 64)
+
+
 def test_states_are_carried_where_that_is_faster():
     assert sv.memory_carries(17, 2, 128 * 128 * 64)      # 2 x 2048 tokens
     assert sv.memory_carries(4, 1, 64 * 128 * 64)        # 1000 tokens
