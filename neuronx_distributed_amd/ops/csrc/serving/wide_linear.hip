@@ -6,10 +6,10 @@
 //                      first half of rows are gates
 //
 // Bound by reading the weights up to 64 rows, beside that by LDS (28672 x 4096 gated:
-// 36 us to read, 16 us of LDS at 128 rows).  A workgroup has 128 weight rows and a share
-// of K; few weight rows are shared by K among as many workgroups as there are CUs, and the
+// 36 us to read, 16 us of LDS at 128 rows).  A workgroup has up to 128 weight rows and a
+// share of K; few weight rows are shared by K among as many workgroups as there are CUs, and the
 // sums of a product meet in a second launch.  us, library (with the activation) | here:
-//   28672 x 4096 gated     32 rows 55 | 41.0   64: 56 | 42.4   100: 59 | 47.7   128: 60 | 51.6
+//   28672 x 4096 gated     32 rows 55 | 40.4   64: 56 | 40.7   100: 59 | 48.2   128: 60 | 50.1
 //   32000 x 4096, 32 bit   32 rows 57 | 43.7   64: 59 | 44.8   100: 62 | 49.1   128: 62 | 53.2
 //   6144 x 4096, by 5      48 rows 17.5 | 16.6  64: 18.1 | 17.9  100: 23.3 | 21.5
 //   4096 x 14336, by 8     32 rows 34 | 25.3   64: 40 | 27.1   100: 49 | 31.5   128: 75 | 35.1
@@ -23,6 +23,7 @@ struct WideArgs {
   long wst;
   void* out;                // [T][N], or [T][N / 2] with GLU; 32-bit sums [splits][T][N]
   int T, N, K, splits;
+  int g;                    // rows of a block of 32 (set here)
 };
 
 enum Epilogue { PLAIN = 0, F32 = 1, GLU = 2 };
@@ -49,8 +50,8 @@ __device__ __forceinline__ void read_rows(int aw, int ax, frag_u* fw, frag_u* fx
                  : "v"(aw), "v"(ax) : "memory");
 }
 
-// One workgroup: 128 weight rows (32 gates and their projections by turns) by BM rows of
-// x, 64 columns a stage.  Both go straight into LDS, NS - 1 stages ahead, rows of 128 bytes
+// One workgroup: 128 weight rows (32 gates and their projections by turns; or of every 32
+// the first g, for whole rounds of workgroups) by BM rows of x, 64 columns a stage.  Both go straight into LDS, NS - 1 stages ahead, rows of 128 bytes
 // whose 16-byte slots s lie at s ^ row % 8.  Waves have 64 weight rows by BM / WM rows of
 // x and share the columns of a stage; their sums meet at the end.  Workgroups begin at
 // different columns: where all read the same ones, rows of a pitch of 8 KB met few
@@ -75,12 +76,15 @@ __global__ void __launch_bounds__(512) wide_linear_kernel(WideArgs a) {
   const auto rw = ring_source(a.w, (a.N - 1) * wp + a.K * 2);
   const auto rx = ring_source(a.x, (a.T - 1) * xp + a.K * 2);
   int ow[2], ox[LX];
+  bool held[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int r = (wid * 2 + i) * 8 + (lane >> 3);
-    const int n = EPI == GLU ? tile * 64 + (r >> 6) * 32 + (r & 31) + (r & 32 ? a.N / 2 : 0)
-                             : tile * BN + r;
+    const int n = (r & 31) +
+        (EPI == GLU ? (tile * 2 + (r >> 6)) * a.g + (r & 32 ? a.N / 2 : 0)
+                    : (tile * 4 + (r >> 5)) * a.g);
     ow[i] = n * wp + ((lane ^ (lane >> 3)) & 7) * 16 + b0 * 128;
+    held[i] = (r & 31) < a.g;
   }
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
@@ -95,7 +99,7 @@ __global__ void __launch_bounds__(512) wide_linear_kernel(WideArgs a) {
     const uint at = next < steps ? blk * 128 : RING_NOWHERE;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      piece<true>(rw, ow[i] + at, st + (wid * 2 + i) * 1024);
+      piece<true>(rw, held[i] ? ow[i] + at : RING_NOWHERE, st + (wid * 2 + i) * 1024);
 #pragma unroll
     for (int i = 0; i < LX; ++i)
       piece<false>(rx, mine ? ox[i] + at : RING_NOWHERE,
@@ -168,8 +172,8 @@ __global__ void __launch_bounds__(512) wide_linear_kernel(WideArgs a) {
       if (t >= a.T) continue;
       const int r = 8 * rg + 4 * hi;
       if (EPI == GLU && !SPLIT) {
-        const int c = tile * 64 + wn * 32 + r;
-        if (c >= N) continue;
+        const int c = (tile * 2 + wn) * a.g + r;
+        if (r >= a.g || c >= N) continue;
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[0][j] = silu_f(v[0][j]) * v[1][j];
         *(uint2*)((short*)a.out + (long)t * N + c) =
@@ -177,9 +181,9 @@ __global__ void __launch_bounds__(512) wide_linear_kernel(WideArgs a) {
       } else {
 #pragma unroll
         for (int n = 0; n < CN; ++n) {
-          const int c = EPI == GLU ? tile * 64 + wn * 32 + r + n * (N / 2)
-                                   : tile * BN + wn * 64 + n * 32 + r;
-          if (c >= (EPI == GLU && n == 0 ? N / 2 : N)) continue;
+          const int c = r + (EPI == GLU ? (tile * 2 + wn) * a.g + n * (N / 2)
+                                        : (tile * 4 + wn * 2 + n) * a.g);
+          if (r >= a.g || c >= (EPI == GLU && n == 0 ? N / 2 : N)) continue;
           if (SPLIT)
             *(f32x4*)((float*)a.out + ((long)y * a.T + t) * N + c) = v[n];
           else if (EPI == F32)
@@ -225,7 +229,14 @@ extern "C" int sv_wide_linear(const WideArgs* a, float* part, int epilogue,
       a->xst * 2 * 256 >= 1L << 31)
     return 1;
   WideArgs w = *a;
-  const dim3 grid((a->N + 127) / 128, a->splits);
+  // Whole rounds of 256 workgroups, each with as many rows: a CU alone reads 25 GB/s
+  // (28672 x 4096 gated, 32 rows: 43.3 us by 128, 40.4 by 112; 22016 36.8, 33.9 by 96;
+  // 37888 x 3584 64.8, 53.3 by 76; but 57344 x 8192 150.7, 154, an eighth idle).
+  const int tiles = (a->N + 127) / 128, all = (tiles + 255) / 256 * 256;
+  w.g = 32;
+  if (a->splits == 1 && (a->T > 32 || all == 256 || tiles * 5 < all * 4))
+    w.g = min(32, (a->N + 16 * all - 1) / (16 * all) * 4);
+  const dim3 grid((a->N + 4 * w.g - 1) / (4 * w.g), a->splits);
   if (part) w.out = part;
 #define WIDE(M, E, S) wide_linear_kernel<M, E, S><<<grid, 512, 0, stream>>>(w)
 #define WIDE_E(M)                                                             \

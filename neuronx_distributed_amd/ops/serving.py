@@ -118,7 +118,7 @@ class _WideArgs(ctypes.Structure):
     _fields_ = (_fields("x", ctypes.c_void_p) + _fields("xst", ctypes.c_long)
                 + _fields("w", ctypes.c_void_p) + _fields("wst", ctypes.c_long)
                 + _fields("out", ctypes.c_void_p)
-                + _fields("T N K splits", ctypes.c_int))
+                + _fields("T N K splits g", ctypes.c_int))
 
 
 class _ConvArgs(ctypes.Structure):
@@ -370,9 +370,10 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
       rows: 29, 24; fewer than 17 of a very long one: 6144 x 18944, 9 rows 110, 42),
       and weights of many rows;
     - up to 64 rows are the weights'; more are also bound by their way through LDS,
-      and the library is faster where workgroups leave CUs without work (22016 x
-      5120, 64 rows: 53.4, 54.5, 128 rows: 53, 63; 57344 x 4096, the last of two
-      rounds empty by a quarter);
+      and the library is faster where rounds of fewer rows a workgroup leave too
+      little to each (gated 37888 x 3584, 48 rows: 62.5, 55.0, 100 rows: 72.3, 73.3;
+      43008 x 4096, 100 rows: 97.7, 88.2), and rings up to 32 rows there (34816 x
+      4096, 32 rows: 54.0, 56.9; 22016 x 4096, of one round: 36.5, 33.7);
     - short K under few weight rows has too little to hide a merge behind (4096 x
       2048, 40 rows: 9.9, 9.1, 96: 10, 11; 8192 x 3072, 96: 19.2, 21.4)."""
     if K % 64 or K < 512 or N % 8 or T > 128 or glu and N % 32:
@@ -380,11 +381,11 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
     tiles, many = -(-N // 128), T > 64
     splits = max(1, min(256 // tiles, K // 256, 16 if many else 64))
     idle = 1 - tiles * splits / (256 * -(-tiles * splits // 256))
-    if tiles > 256 and idle > (0.1 if many and not glu else 0.15):
+    if tiles > 256 and (idle > 0.15 if T <= 32 else many and idle > 0.38):
         return None
     if T <= 32:
         if K <= 4096:
-            take = T >= 17 and N >= 28000 and K >= 1536
+            take = T >= 17 and N >= 20000 and K >= 1536
         else:
             take = T >= 17 or T >= 9 and N >= 5120 and (
                 K >= 14336 if T < 13 else K >= 11008)

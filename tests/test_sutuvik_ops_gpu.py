@@ -789,10 +789,12 @@ def test_products_of_few_rows_through_rings(T, N, K, how):
 
 @pytest.mark.parametrize("T,N,K,splits", [
     (9, 8, 512, 1), (17, 136, 576, 2), (32, 264, 14336, 7), (33, 1000, 1088, 3),
-    (64, 4096, 4096, 8), (65, 24, 512, 1), (100, 6144, 2112, 5), (128, 8200, 704, 1)])
+    (64, 4096, 4096, 8), (65, 24, 512, 1), (100, 6144, 2112, 5), (128, 8200, 704, 1),
+    (20, 12296, 576, 1), (33, 33000, 512, 1), (32, 57344, 512, 1), (128, 40008, 576, 1)])
 def test_products_of_more_rows(T, N, K, splits):
     """The same, 32, 64 and 128 rows a workgroup and one more, shares of K of unequal
-    numbers of blocks, fewer than the stages and more, tiles and rows ragged."""
+    numbers of blocks, fewer than the stages and more, tiles and rows ragged, tiles of
+    fewer rows in one round and in two."""
     torch.manual_seed(T + N + K)
     x = torch.full((T, K + 8), float("nan"), device="cuda", dtype=torch.bfloat16)[:, :K]
     x.copy_(torch.randn(T, K, device="cuda"))
