@@ -421,6 +421,12 @@ def _turned(x: torch.Tensor) -> torch.Tensor:
     return out[:, :T].t()
 
 
+def _turns(t: torch.Tensor) -> bool:
+    """May these rows be turned: bf16, whole 16-byte words?"""
+    return t.is_cuda and t.dtype == torch.bfloat16 and t.stride(1) == 1 and \
+        not (t.shape[1] | t.stride(0)) & 7 and not t.data_ptr() & 15
+
+
 def weight_grads(grads, x: torch.Tensor):
     """[dy^T x for dy in grads] of dy (T, N) and x (T, K)."""
     T, K = x.shape
@@ -428,12 +434,8 @@ def weight_grads(grads, x: torch.Tensor):
         return [g.t().matmul(x) for g in grads]
     from .serving import unseen
 
-    def turns(t):
-        return t.is_cuda and t.dtype == torch.bfloat16 and t.stride(1) == 1 and \
-            not (t.shape[1] | t.stride(0)) & 7 and not t.data_ptr() & 15
-
     ways = [(False, False)] * len(grads)
-    if turns(x) and unseen(x, *grads) and \
+    if _turns(x) and unseen(x, *grads) and \
             x.get_device() == torch._C._cuda_getDevice():
         ways = [turn_rule(T, g.shape[1], K) for g in grads]
         # x is turned once for all of them
@@ -441,8 +443,31 @@ def weight_grads(grads, x: torch.Tensor):
             ways = [(dy, True) for dy, _ in ways]
     if any(way for _, way in ways):
         xt = _turned(x)
-    return [(_turned(g) if dy and turns(g) else g).t().matmul(xt if way else x)
+    return [(_turned(g) if dy and _turns(g) else g).t().matmul(xt if way else x)
             for g, (dy, way) in zip(grads, ways)]
+
+
+def turn_weight_rule(T: int, N: int, K: int) -> bool:
+    """Is w (N, K) turned for dy w of T rows?  As above, 1.07 to 1.35 times as fast
+    with the turning (8192 rows, 32000 x 4096: 1545 -> 1367 us; 4096 x 4096: 198 ->
+    185; 16384: 391 -> 352).  Not below (6144, 4096 x 11008: 449 -> 493), for other
+    numbers of rows, of which the library has forms that are slower by a third
+    (9000, 4096 x 4096: 338 -> 363), and of the largest weights only for many (8192,
+    27648 x 5120: 2279 -> 2349, 16384: 3429 -> 2982)."""
+    return T >= 8192 and T % 512 == 0 and \
+        16_000_000 < N * K < (140_000_000 if T < 16384 else 1 << 31)
+
+
+def input_weight(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """w (N, K), laid out as dy (..., N) times it is the fastest."""
+    if dy.is_cuda and w.dim() == 2 and dy.shape[-1] and \
+            turn_weight_rule(dy.numel() // dy.shape[-1], *w.shape):
+        from .serving import unseen
+
+        if _turns(w) and dy.dtype == w.dtype and unseen(dy, w) and \
+                dy.get_device() == w.get_device() == torch._C._cuda_getDevice():
+            return _turned(w)
+    return w
 
 
 # ---------------------------------------------------------------------------

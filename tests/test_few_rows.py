@@ -274,3 +274,13 @@ def test_operands_of_a_weight_gradient(T, N, K, want):
     from neuronx_distributed_amd.ops import turn_rule
 
     assert turn_rule(T, N, K) == want
+
+
+@pytest.mark.parametrize("T,N,K,want", [
+    (8192, 32000, 4096, True), (7680, 32000, 4096, False),
+    (9000, 4096, 4096, False), (8192, 2048, 5632, False),
+    (8192, 27648, 5120, False), (16384, 27648, 5120, True)])
+def test_weights_of_an_input_gradient(T, N, K, want):
+    from neuronx_distributed_amd.ops import turn_weight_rule
+
+    assert turn_weight_rule(T, N, K) is want

@@ -985,3 +985,19 @@ def test_weight_gradients(T, K, widths, aligned):
         gx = grads[0].clone().requires_grad_()
         (w,) = ops.weight_grads([gx], x)
         assert w.requires_grad
+
+
+def test_turned_weight_of_an_input_gradient():
+    dy = torch.randn(2, 4096, 4096, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(4096, 4096, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        wt = ops.input_weight(dy, w)
+        assert torch.equal(wt, w) and wt.stride(0) == 1
+        got, want = dy.matmul(wt)[0, :64], dy[0, :64].float() @ w.float()
+    # rounded to 8 bits; sums of 4096 terms in float32, in any order
+    bound = want.abs() * 2 ** -8 + 2 * 4096 * 2 ** -24 * \
+        (dy[0, :64].float().abs() @ w.float().abs())
+    assert ((got.float() - want).abs() <= bound).all()
+    assert ops.input_weight(dy, w) is w                # under autograd
+    with torch.no_grad():
+        assert ops.input_weight(dy[:, :100], w) is w
