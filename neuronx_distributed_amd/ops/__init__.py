@@ -471,6 +471,59 @@ def input_weight(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------------------
+# embedding
+# ---------------------------------------------------------------------------
+
+# a row's tokens are looked for among all between its first and its last
+EMBEDDING_TOKENS = 32768
+
+
+class _EmbeddingFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, ids, weight, padding_idx):
+        ctx.save_for_backward(ids)
+        ctx.rows, ctx.skip = weight.shape[0], padding_idx
+        return torch.nn.functional.embedding(ids, weight, padding_idx)
+
+    @staticmethod
+    def backward(ctx, dy):
+        from .serving import unseen
+
+        (ids,) = ctx.saved_tensors
+        skip = -1 if ctx.skip is None else ctx.skip % ctx.rows
+        T, W = ids.numel(), dy.shape[-1]
+        if not (unseen(dy, ids) and 0 < T <= EMBEDDING_TOKENS and dy.is_cuda
+                and dy.get_device() == torch._C._cuda_getDevice()):
+            return None, torch.ops.aten.embedding_dense_backward(
+                dy, ids, ctx.rows, skip, False), None
+        rows, ids = dy.contiguous(), ids.contiguous()
+        if rows.data_ptr() & 15:
+            rows = rows.clone()
+        out = torch.empty(ctx.rows, W, dtype=dy.dtype, device=dy.device)
+        work = torch.empty(3 * ctx.rows + 1 + T // 9, dtype=torch.int32,
+                           device=dy.device)
+        if _require_lib().embedding_bwd(_ptr(ids), _ptr(rows), _ptr(out), _ptr(work),
+                                        T, ctx.rows, W, skip, _stream()):
+            raise RuntimeError("embedding_bwd failed")
+        return None, out, None
+
+
+def embedding(ids: torch.Tensor, weight: torch.Tensor,
+              padding_idx: Optional[int] = None) -> torch.Tensor:
+    """``torch.nn.functional.embedding``, with its gradient in one pass over the
+    table where that is bf16 and nobody traces or transforms the call."""
+    from .serving import _plain, _unwatched
+
+    if torch.is_grad_enabled() and weight.is_cuda and weight.requires_grad and \
+            weight.dtype == torch.bfloat16 and ids.dtype == torch.int64 and \
+            weight.dim() == 2 and weight.shape[0] and weight.shape[1] and \
+            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 30 and \
+            _plain(weight) and _plain(ids) and _unwatched():
+        return _EmbeddingFn.apply(ids, weight, padding_idx)
+    return torch.nn.functional.embedding(ids, weight, padding_idx)
+
+
+# ---------------------------------------------------------------------------
 # SwiGLU
 # ---------------------------------------------------------------------------
 

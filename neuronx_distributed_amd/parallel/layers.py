@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
-from ..ops import input_weight, weight_grads
+from ..ops import embedding, input_weight, weight_grads
 from ..ops.serving import unseen
 from . import comm
 from . import parallel_state as ps
@@ -614,21 +614,19 @@ class ParallelEmbedding(BaseParallelLinear):
     def forward(self, input_):
         world = ps.get_tensor_model_parallel_size()
         if self.shard_along_embedding:
-            local = F.embedding(input_, self.weight,
-                                padding_idx=self.padding_idx)
+            local = embedding(input_, self.weight, self.padding_idx)
             if world == 1:
                 return local
             return gather_from_tensor_model_parallel_region(local)
         if world > 1:
             input_mask = (input_ >= self.start_index) & (input_ < self.end_index)
             masked_input = (input_ - self.start_index) * input_mask
-            output_parallel = F.embedding(masked_input, self.weight,
-                                          padding_idx=self.padding_idx)
+            output_parallel = embedding(masked_input, self.weight,
+                                        self.padding_idx)
             output_parallel = output_parallel * input_mask.unsqueeze(-1).to(
                 output_parallel.dtype)
         else:
-            output_parallel = F.embedding(input_, self.weight,
-                                          padding_idx=self.padding_idx)
+            output_parallel = embedding(input_, self.weight, self.padding_idx)
         if world == 1:
             return output_parallel
         if self.sequence_parallel_enabled:

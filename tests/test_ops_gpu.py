@@ -1001,3 +1001,38 @@ def test_turned_weight_of_an_input_gradient():
     assert ops.input_weight(dy, w) is w                # under autograd
     with torch.no_grad():
         assert ops.input_weight(dy[:, :100], w) is w
+
+
+@pytest.mark.parametrize("T,V,W,skip,kind", [
+    (1, 5, 8, None, "any"), (8, 3, 24, 1, "any"), (9, 1, 8, None, "one"),
+    (300, 40, 520, -1, "any"), (700, 5000, 2056, 0, "any"),
+    (2000, 32000, 4096, None, "any"), (1500, 900, 1032, 3, "few"),
+    (8192, 100, 512, None, "one")])
+def test_embedding_gradient(T, V, W, skip, kind):
+    """Rows without tokens, of one, two, up to eight and more; of all."""
+    ids = torch.randint(V, (T,), device="cuda")
+    if kind == "one":
+        ids[:] = V // 2
+    elif kind == "few":
+        ids[::3] = 7
+        ids[1::3] %= 40
+    w = torch.randn(V, W, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(T, W, device="cuda", dtype=torch.bfloat16)
+    out = ops.embedding(ids, w, skip)
+    assert torch.equal(out, w[ids])
+    (got,) = torch.autograd.grad(out, w, dy, retain_graph=True)
+    (again,) = torch.autograd.grad(out, w, dy)
+    assert torch.equal(got, again)
+    want = torch.zeros(V, W, device="cuda", dtype=torch.float64)
+    want.index_add_(0, ids, dy.double())
+    size = torch.zeros_like(want).index_add_(0, ids, dy.double().abs())
+    if skip is not None:
+        want[skip % V] = 0
+    # rounded to 8 bits; sums of up to T terms in float32
+    bound = want.abs() * 2 ** -8 + 2 * T * 2 ** -24 * size
+    assert ((got.double() - want).abs() <= bound).all()
+    # a backward that is differentiated itself
+    out = ops.embedding(ids, w, skip)
+    dy.requires_grad_()
+    (g,) = torch.autograd.grad(out, w, dy, create_graph=True)
+    assert g.requires_grad
