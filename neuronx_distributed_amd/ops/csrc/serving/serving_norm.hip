@@ -301,8 +301,8 @@ residual_norm_kernel(ResidualNormArgs a) {
   }
 }
 
-// The same of few rows where one tensor or a weighted sum of up to 8 rows is
-// pending and is neither normed nor gated: a decoder's norms between its products.
+// The same where one tensor or, of few rows, a weighted sum of up to 8 rows is pending
+// and is neither normed nor gated: a decoder's norms between its products.
 // Bound by the way to memory and back: all words (R x 4 of a thread) are asked for
 // first, sums stay in registers but for one turn through LDS (a step of 4 layers,
 // one request: 9 norms, 11 us less than with the kernel above).
@@ -395,7 +395,13 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
   // rows of 2048: 4.5 us, long 6.0; of 4096: 6.8, 7.9; of 8192: 50, 49)
   const bool wide = a->W >= 2048 &&
       a->rows_out <= (a->branches || a->W > 4096 ? 512 : 256);
-  if (wide && vec && !f32 && (a->x || a->delta) && a->h && a->w && a->groups == 1 &&
+  // all words at first is better of many rows, too, of one tensor as wide as most of
+  // the workgroup (4800 rows of 4096: 53 us, here 42.5; of 8192: 121, 87; of 2048, half
+  // of it without words, 600 rows 8.5, 9.5; sums of two rows of 3072 47, 50)
+  const bool few = a->W >= 2048 &&
+      (a->rows_out <= 256 || (a->W > 4096 && a->rows_out <= 512) ||
+       (a->W >= 3072 && !a->coef));
+  if (few && vec && !f32 && (a->x || a->delta) && a->h && a->w && a->groups == 1 &&
       a->W <= 16384 && !a->delta2 && !a->w1 && !a->vec && !a->cat && !a->conv &&
       !a->branches && (!a->coef || (a->parts <= 8 && a->W <= 4096))) {
 #define FRX(R, D, X) \

@@ -587,3 +587,22 @@ def test_rope_rows(sv, T, H, G, D, shift, dtype):
             + (x.abs() + y.abs()).max() * 2.0 ** -23).all()
     assert torch.equal(qkv[:, :shift], before[:, :shift])
     assert torch.equal(qkv[:, shift + n:], before[:, shift + n:])
+
+
+@pytest.mark.parametrize("rows,W", [(257, 3072), (600, 3068), (513, 4100),
+                                    (1100, 8192), (513, 16384)])
+@pytest.mark.parametrize("wide", [False, True])
+def test_residual_norm_of_many_rows(sv, rows, W, wide):
+    """All words of a row at first, and one after the other below 3072 columns; what
+    is pending of 32 bits, or nothing."""
+    eps, bf = 0.03, torch.bfloat16
+    x, w = _rand(rows, W, dtype=torch.float32), _rand(W, dtype=bf, seed=1)
+    for d in (_rand(rows, W, dtype=torch.float32 if wide else bf, seed=2), None):
+        new = x if d is None else x + d.float()
+        want = new.double() * torch.rsqrt(
+            new.double().pow(2).mean(1, keepdim=True) + eps) * w.double()
+        got, h, _ = sv.residual_norm(
+            x.cuda(), None if d is None else sv.Pending(d.cuda()), eps, w.cuda())
+        assert torch.equal(got.cpu(), new)
+        torch.testing.assert_close(h.cpu().double(), want, rtol=2.0 ** -8 + W * 2.0 ** -24,
+                                   atol=1e-30)
