@@ -301,25 +301,26 @@ residual_norm_kernel(ResidualNormArgs a) {
   }
 }
 
-// The same where one tensor or, of few rows, a weighted sum of up to 8 rows is pending
-// and is neither normed nor gated: a decoder's norms between its products.
+// The same where one tensor or a weighted sum of 2 rows, of few up to 8, is pending and
+// is neither normed nor gated: a decoder's norms between its products.
 // Bound by the way to memory and back: all words (R x 4 of a thread) are asked for
 // first, sums stay in registers but for one turn through LDS (a step of 4 layers,
 // one request: 9 norms, 11 us less than with the kernel above).
-enum { NONE, ROW, ROW32, SUM };
+enum { NONE, ROW, ROW32, SUM, PAIR };    // PAIR: a sum of up to two
 // X: there is a residual.
 template <int R, int DELTA, bool X>
 __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a) {
-  constexpr int P = 8;                   // rows of a sum
+  constexpr bool ADD = DELTA == SUM || DELTA == PAIR;
+  constexpr int P = DELTA == PAIR ? 2 : 8;   // rows of a sum
   __shared__ __attribute__((aligned(16))) float red[16];
   const int o = blockIdx.x, tid = threadIdx.x, W = a.W;
   const long r = a.index ? a.index[o] : o;
   float c[P];
-  if (DELTA == SUM)
+  if (ADD)
 #pragma unroll
     for (int p = 0; p < P; ++p) c[p] = a.coef[r * a.parts + min(p, a.parts - 1)];
   f32x4 v[R], t[R];
-  s4v u[R], d[R], e[R][DELTA == SUM ? P : 1];
+  s4v u[R], d[R], e[R][ADD ? P : 1];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int i = min((tid + k * 1024) * 4, W - 4);
@@ -327,7 +328,7 @@ __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a)
     u[k] = *(const s4v*)((const short*)a.w + i);
     if (DELTA == ROW) d[k] = *(const s4v*)((const short*)a.delta + r * W + i);
     if (DELTA == ROW32) t[k] = *(const f32x4*)((const float*)a.delta + r * W + i);
-    if (DELTA == SUM)
+    if (ADD)
 #pragma unroll
       for (int p = 0; p < P; ++p)
         e[k][p] = *(const s4v*)((const short*)a.delta +
@@ -340,7 +341,7 @@ __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (DELTA == ROW) t[k][j] = bits2f(d[k][j]);
-      if (DELTA == SUM) {
+      if (ADD) {
         t[k][j] = 0.f;
 #pragma unroll
         for (int p = 0; p < P; ++p)      // (no weight of zero: of infinities)
@@ -397,10 +398,11 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
       a->rows_out <= (a->branches || a->W > 4096 ? 512 : 256);
   // all words at first is better of many rows, too, of one tensor as wide as most of
   // the workgroup (4800 rows of 4096: 53 us, here 42.5; of 8192: 121, 87; of 2048, half
-  // of it without words, 600 rows 8.5, 9.5; sums of two rows of 3072 47, 50)
+  // of it without words, 600 rows 8.5, 9.5; sums of two rows of 4096 60, 48, of up to
+  // eight of 3072 47, 50)
   const bool few = a->W >= 2048 &&
       (a->rows_out <= 256 || (a->W > 4096 && a->rows_out <= 512) ||
-       (a->W >= 3072 && !a->coef));
+       (a->W >= 3072 && (!a->coef || a->parts <= 2)));
   if (few && vec && !f32 && (a->x || a->delta) && a->h && a->w && a->groups == 1 &&
       a->W <= 16384 && !a->delta2 && !a->w1 && !a->vec && !a->cat && !a->conv &&
       !a->branches && (!a->coef || (a->parts <= 8 && a->W <= 4096))) {
@@ -416,6 +418,7 @@ extern "C" int sv_residual_norm(const ResidualNormArgs* a, int f32,
     else FRN(4, D);                    \
   } while (0)
     if (!a->delta) FR(NONE);
+    else if (a->coef && a->parts <= 2) FRN(1, PAIR);
     else if (a->coef) FRN(1, SUM);
     else if (a->delta_f32) FR(ROW32);
     else FR(ROW);

@@ -606,3 +606,24 @@ def test_residual_norm_of_many_rows(sv, rows, W, wide):
         assert torch.equal(got.cpu(), new)
         torch.testing.assert_close(h.cpu().double(), want, rtol=2.0 ** -8 + W * 2.0 ** -24,
                                    atol=1e-30)
+
+
+@pytest.mark.parametrize("rows,W", [(1, 2048), (257, 3068), (257, 3072), (600, 4096),
+                                    (300, 4100)])
+@pytest.mark.parametrize("parts", [1, 2, 3])
+def test_residual_norm_of_many_sums(sv, rows, W, parts):
+    """Sums of one and two rows by the kernel of many rows, and of more."""
+    eps, bf = 0.03, torch.bfloat16
+    x, w = _rand(rows, W, dtype=torch.float32), _rand(W, dtype=bf, seed=1)
+    d = _rand(rows * parts, W, dtype=bf, seed=2)
+    coef = _rand(rows, parts, dtype=torch.float32, seed=3)
+    terms = d.view(rows, parts, W).double() * coef.double()[..., None]
+    new = x.double() + terms.sum(1)
+    size = x.double().abs() + terms.abs().sum(1)
+    got, h, _ = sv.residual_norm(x.cuda(), sv.Pending(d.cuda(), coef=coef.cuda()), eps,
+                                 w.cuda())
+    assert ((got.cpu().double() - new).abs() <= size * (parts + 1) * 2.0 ** -23).all()
+    mine = got.cpu().double()
+    want = mine * torch.rsqrt(mine.pow(2).mean(1, keepdim=True) + eps) * w.double()
+    torch.testing.assert_close(h.cpu().double(), want, rtol=2.0 ** -8 + W * 2.0 ** -24,
+                               atol=1e-30)
