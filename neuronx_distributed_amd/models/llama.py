@@ -254,7 +254,7 @@ class LlamaAttention(nn.Module):
         from ..ops import serving as sv
 
         p = self.qkv_proj
-        if pending.delta.shape[0] != 1 or \
+        if pending.count() != 1 or \
                 type(self).forward_ragged is not LlamaAttention.forward_ragged \
                 or "forward_ragged" in self.__dict__ \
                 or type(p) is not GQAQKVColumnParallelLinear or _watched(p):
@@ -354,6 +354,20 @@ def _watched(module) -> bool:
                 or nn.modules.module._global_forward_pre_hooks)
 
 
+def _embedded(embed, tokens):
+    """The embeddings of ``tokens`` as a pending result: rows that the first norm
+    takes from the table itself, where nobody sees or stands for the look-up."""
+    from ..ops import serving as sv
+
+    w = embed.weight
+    if type(embed) is ParallelEmbedding and not _watched(embed) and \
+            w.is_cuda and w.is_contiguous() and sv.unseen(w, tokens) and \
+            tokens.dtype == torch.int32 and tokens.is_contiguous() and \
+            w.dtype == torch.bfloat16 and ps.get_tensor_model_parallel_size() == 1:
+        return sv.Pending(w, rows=tokens)
+    return sv.Pending(embed(tokens))
+
+
 class LlamaMLP(nn.Module):
     def __init__(self, config: LlamaConfig):
         super().__init__()
@@ -381,7 +395,7 @@ class LlamaMLP(nn.Module):
         row that the norm and the gates of are one launch; else None."""
         from ..ops import serving as sv
 
-        if pending.delta.shape[0] != 1 or _watched(self) or \
+        if pending.count() != 1 or _watched(self) or \
                 type(self).forward is not LlamaMLP.forward or \
                 not self._glu_in_one():
             return None
@@ -584,7 +598,8 @@ class LlamaForCausalLM(nn.Module):
         from ..ops import serving as sv
 
         m, eps = self.model, self.config.rms_norm_eps
-        x, pending = None, sv.Pending(m.embed_tokens(batch.tokens))
+        x, pending = None, _embedded(m.embed_tokens, batch.tokens) \
+            if len(m.layers) else sv.Pending(m.embed_tokens(batch.tokens))
         for layer, pool in zip(m.layers, pools):
             attn, mlp = layer.self_attn, layer.mlp
             at = m.rope_cos, m.rope_sin, batch, pool[0]

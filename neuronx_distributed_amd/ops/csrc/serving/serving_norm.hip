@@ -46,6 +46,7 @@ struct ResidualNormArgs {
   void* cat;             // [out_rows, 2 W]: new x, then x0; or null
   const void* x0;        // [rows, W]
   const int* index;      // out row -> row, or null
+  long table;            // > 0: rows of delta that index is kept in
   // convolution of the rows from conv_row on, which are single tokens
   const void* conv;      // [taps][W] weights, or null
   void* ring;            // [slots][taps][W]: the input at position p is in
@@ -61,6 +62,12 @@ struct ResidualNormArgs {
   int branches;          // gated results that are pending
   BranchArgs br[2];
 };
+
+__device__ __forceinline__ long row_of(const ResidualNormArgs& a, int o) {
+  if (!a.index) return o;
+  const long r = a.index[o];
+  return a.table ? min(max(r, 0L), a.table - 1) : r;
+}
 
 template <typename T, int VEC>
 __device__ __forceinline__ void ld(const T* p, float* v) {
@@ -78,7 +85,7 @@ residual_norm_kernel(ResidualNormArgs a) {
   float* part_rstd = row + a.W;    // [groups], if a norm has several
   __shared__ float red[16];
   const int o = blockIdx.x;
-  const long r = a.index ? a.index[o] : o;
+  const long r = row_of(a, o);
   const int W = a.W, tid = threadIdx.x;
   const T* d1 = (const T*)a.delta + r * W;
   const float* d1f = (const float*)a.delta + r * W;
@@ -314,7 +321,7 @@ __global__ void __launch_bounds__(1024) few_rows_norm_kernel(ResidualNormArgs a)
   constexpr int P = DELTA == PAIR ? 2 : 8;   // rows of a sum
   __shared__ __attribute__((aligned(16))) float red[16];
   const int o = blockIdx.x, tid = threadIdx.x, W = a.W;
-  const long r = a.index ? a.index[o] : o;
+  const long r = row_of(a, o);
   float c[P];
   if (ADD)
 #pragma unroll

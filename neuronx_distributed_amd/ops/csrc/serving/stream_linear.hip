@@ -34,12 +34,14 @@ struct StreamArgs {
   void* out;                // [T][N], or [T][N / 2] with GLU
   int T, N, K;
   // instead of x, one row: that of the 32-bit residual (or null: zero) plus
-  // `delta`, normed
+  // `delta`, normed; or without residual a row of the table delta
   const float* res;
   const short* delta;
   float* res_out;           // their sum
   const short* weight;
   float eps;
+  const int* row;           // which, or null
+  long rows;
 };
 
 enum Epilogue { PLAIN = 0, F32 = 1, GLU = 2 };
@@ -91,10 +93,12 @@ __device__ __forceinline__ void norm_row(const StreamArgs& a, short* row,
   const int tid = threadIdx.x, i = tid * V, at = min(i, a.K - V);
   f32x4 v[V / 4];
   s4v d[V / 4], u[V / 4];
+  const short* delta = a.delta + at;
+  if (a.row) delta += min(max((long)a.row[0], 0L), a.rows - 1) * a.K;
 #pragma unroll
   for (int k = 0; k < V / 4; ++k) {
     v[k] = a.res ? *(const f32x4*)(a.res + at + 4 * k) : f32x4{};
-    d[k] = *(const s4v*)(a.delta + at + 4 * k);
+    d[k] = *(const s4v*)(delta + 4 * k);
     u[k] = *(const s4v*)(a.weight + at + 4 * k);
   }
   __builtin_amdgcn_sched_barrier(0);

@@ -97,7 +97,9 @@ class _BranchArgs(ctypes.Structure):
 
 class _ResidualNormArgs(ctypes.Structure):
     _fields_ = (_fields("x delta delta2 w1 w2 coef vec x_out h w cat x0 "
-                        "index conv ring singles hc", ctypes.c_void_p)
+                        "index", ctypes.c_void_p)
+                + _fields("table", ctypes.c_long)
+                + _fields("conv ring singles hc", ctypes.c_void_p)
                 + _fields("rows_out W delta_f32 parts groups p_groups taps "
                           "conv_row", ctypes.c_int)
                 + _fields("eps scale w_base p_base h_scale", ctypes.c_float)
@@ -111,7 +113,8 @@ class _StreamArgs(ctypes.Structure):
                 + _fields("out", ctypes.c_void_p)
                 + _fields("T N K", ctypes.c_int)
                 + _fields("res delta res_out weight", ctypes.c_void_p)
-                + _fields("eps", ctypes.c_float))
+                + _fields("eps", ctypes.c_float)
+                + _fields("row", ctypes.c_void_p) + _fields("rows", ctypes.c_long))
 
 
 class _WideArgs(ctypes.Structure):
@@ -566,7 +569,8 @@ class Pending:
     given, over ``groups`` equal parts each.  ``coef`` (rows, parts) makes a row the weighted sum of ``parts``
     rows of ``delta`` (rows * parts, W).  ``centred``: w1 and w2 are stored as
     their distance from one.  ``vec`` is a row added to every token.  Instead
-    of ``delta``, up to two gated ``branches`` may be pending."""
+    of ``delta``, up to two gated ``branches`` may be pending.  ``rows``: delta is
+    a table, of which these rows (int32) are pending, and nothing else is."""
     delta: Optional[torch.Tensor] = None
     delta2: Optional[torch.Tensor] = None
     w1: Optional[torch.Tensor] = None
@@ -577,6 +581,11 @@ class Pending:
     centred: bool = False
     groups: int = 1
     branches: Sequence["Branch"] = ()
+    rows: Optional[torch.Tensor] = None
+
+    def count(self) -> int:
+        """Of rows of one pending tensor."""
+        return (self.delta if self.rows is None else self.rows).shape[0]
 
 
 @dataclass
@@ -662,7 +671,12 @@ def _plain_norm(x, pending, eps, weight, index, centred, scale):
     between a decoder's products: the same with fewer questions."""
     d, coef = pending.delta, pending.coef
     rows, W = d.shape
-    parts = 0
+    parts = table = 0
+    if pending.rows is not None:
+        assert index is None and x is None and coef is None
+        index, table = pending.rows, rows
+        assert index.dtype == torch.int32 and index.is_contiguous() \
+            and index.is_cuda
     if coef is not None:
         assert coef.is_contiguous() and coef.dtype == torch.float32
         assert coef.numel() == rows and d.dtype == weight.dtype
@@ -676,8 +690,8 @@ def _plain_norm(x, pending, eps, weight, index, centred, scale):
     a = _ResidualNormArgs(
         x=_p(x), delta=d.data_ptr(), coef=_p(coef), x_out=x_new.data_ptr(),
         h=h.data_ptr(), w=weight.data_ptr(), index=_p(index),
-        rows_out=out_rows, W=W, parts=parts, groups=1, p_groups=1, eps=eps,
-        scale=pending.scale, w_base=centred, p_base=pending.centred,
+        table=table, rows_out=out_rows, W=W, parts=parts, groups=1, p_groups=1,
+        eps=eps, scale=pending.scale, w_base=centred, p_base=pending.centred,
         h_scale=scale,
         delta_f32=not f32 and d.dtype == torch.float32)
     _check(library().sv_residual_norm(ctypes.byref(a), f32, _stream()),
@@ -705,6 +719,7 @@ def residual_norm(x: Optional[torch.Tensor], pending: Optional[Pending],
                  pending.w1 is not None or pending.vec is not None or
                  pending.groups != 1):
         return _plain_norm(x, pending, eps, weight, index, centred, scale)
+    assert pending is None or pending.rows is None
     branches = () if pending is None else pending.branches
     src = x if pending is None else \
         branches[0].delta if branches else pending.delta
@@ -1578,8 +1593,12 @@ def normed_linear(x: Optional[torch.Tensor], pending: Pending, eps: float,
     norms the row, 32 KB of a K of 4096, while its weights are on their way; of
     more than one such round of them (512) the later ones have nothing to hide
     that behind."""
-    d = pending.delta
-    if d is None or d.shape[0] != 1 or d.dtype != torch.bfloat16 or \
+    d, row = pending.delta, pending.rows
+    table = 0
+    if row is not None and row.shape[0] == 1 and x is None and d.shape[0] and \
+            row.dtype == torch.int32 and row.is_cuda:
+        table, d = d.shape[0], d[:1]
+    if d is None or d.shape[0] != 1 or (row is not None and not table) or d.dtype != torch.bfloat16 or \
             not d.is_contiguous() or pending.scale != 1.0 or any(
                 t is not None for t in (pending.delta2, pending.w1, pending.w2,
                                         pending.vec, pending.coef)):
@@ -1600,7 +1619,8 @@ def normed_linear(x: Optional[torch.Tensor], pending: Pending, eps: float,
     out = torch.empty(1, N // 2 if glu else N, dtype=d.dtype, device=d.device)
     a = _StreamArgs(w=w.data_ptr(), wst=w.stride(0), out=out.data_ptr(), T=1,
                     N=N, K=K, res=_p(x), delta=d.data_ptr(),
-                    res_out=x_new.data_ptr(), weight=weight.data_ptr(), eps=eps)
+                    res_out=x_new.data_ptr(), weight=weight.data_ptr(), eps=eps,
+                    row=_p(row), rows=table)
     _check(library().sv_stream_linear(ctypes.byref(a), 2 if glu else 0, how,
                                       _stream()), "normed_linear")
     return x_new, out

@@ -627,3 +627,25 @@ def test_residual_norm_of_many_sums(sv, rows, W, parts):
     want = mine * torch.rsqrt(mine.pow(2).mean(1, keepdim=True) + eps) * w.double()
     torch.testing.assert_close(h.cpu().double(), want, rtol=2.0 ** -8 + W * 2.0 ** -24,
                                atol=1e-30)
+
+
+@pytest.mark.parametrize("T,V,W", [(1, 5, 4096), (7, 300, 4096), (3, 9, 72),
+                                   (300, 40, 2048), (700, 1000, 3584)])
+def test_norms_of_rows_of_a_table(sv, T, V, W):
+    """The first norm takes its rows from the table, as after a look-up; and a single
+    one in the product behind it."""
+    bf, eps = torch.bfloat16, 1e-3
+    table, w = _rand(V, W, dtype=bf).cuda(), _rand(W, dtype=bf, seed=1).cuda()
+    rows = (torch.arange(T) * 7919 % V).int().cuda()
+    rows[-1], rows[0] = 0, V - 1
+    found = sv.Pending(table[rows.long()])
+    x, h, _ = sv.residual_norm(None, found, eps, w)
+    got, g, _ = sv.residual_norm(None, sv.Pending(table, rows=rows), eps, w)
+    assert torch.equal(got, x) and torch.equal(g, h)
+    with torch.no_grad():
+        p = _rand(6144, W, dtype=bf, seed=2).cuda()
+        one = sv.normed_linear(None, sv.Pending(table, rows=rows), eps, w, p)
+        ref = sv.normed_linear(None, found, eps, w, p)
+    assert (one is None) == (ref is None) and (one is not None) == (T == 1)
+    if one:
+        assert torch.equal(one[0], ref[0]) and torch.equal(one[1], ref[1])
