@@ -453,10 +453,11 @@ def _plain(t) -> bool:
 
 
 def _few_rows(x: torch.Tensor, w: torch.Tensor, rule) -> Optional[tuple]:
-    """(rows of x (..., K), what ``rule`` (T, N, K) says of them) for the kernels of
-    few rows; None where it says None, under autograd, and where somebody else
-    watches the operations (tracing, dispatch modes, autocast).
-    NXDA_SKINNY_GEMM=0 keeps every product on the library."""
+    """(rows of x (..., K), what ``rule`` (T, N, K, far) says of them) for the
+    kernels of few rows; None where it says None, under autograd, and where somebody
+    else watches the operations (tracing, dispatch modes, autocast).  ``far``: the
+    rows are 2^22 elements apart or more.  NXDA_SKINNY_GEMM=0 keeps every product on
+    the library."""
     if torch.is_grad_enabled() or not (_plain(x) and _plain(w)) or \
             not x.is_cuda:
         return None
@@ -471,10 +472,14 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, rule) -> Optional[tuple]:
             w.get_device() != x.get_device() or \
             os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":
         return None
-    how = rule(T, size[0], K)
+    how = rule(T, size[0], K, False)
     if how is None or not available() or not _unwatched():
         return None
     rows = x if len(shape) == 2 else x.reshape(T, K)
+    if rows.stride(0) >= 1 << 22:        # (of the last tokens of long prompts)
+        how = rule(T, size[0], K, True)
+        if how is None:
+            return None
     if rows.stride(1) != 1 or not (_words(rows) and _words(w)):
         return None
     return rows, how
@@ -491,7 +496,7 @@ def stream_how(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
                glu: bool = False, rings: bool = True) -> Optional[int]:
     """How ``stream_linear`` takes the rows of x (..., K) where it is the faster
     one (by ``ring_rule``, if ``rings``, or ``stream_rule``); else None."""
-    def rule(T, N, K):
+    def rule(T, N, K, far):
         if T > 32:
             return None
         how = ring_rule(T, N, K, f32, glu) if rings and available() and \
@@ -506,10 +511,9 @@ def streamed(x: torch.Tensor, w: torch.Tensor, f32: bool = False,
              glu: bool = False) -> Optional[torch.Tensor]:
     """The product of the rows of x (..., K) by ``wide_linear`` where
     ``wide_rule`` takes it, or ``stream_linear`` by ``stream_how``, or None."""
-    def rule(T, N, K):
+    def rule(T, N, K, far):
         near = available() and _near(w)
-        splits = wide_rule(T, N, K, f32, glu) if near and \
-            x.stride(-2) < 1 << 22 else None
+        splits = wide_rule(T, N, K, f32, glu) if near and not far else None
         if splits is not None:
             return True, splits
         how = None

@@ -231,6 +231,63 @@ def test_every_cut_is_one_that_the_launcher_takes():
     assert 1 in taken and len(taken) > 5
 
 
+class _OnDevice(torch.Tensor):
+    """Rows that say they are on device 0."""
+    is_cuda = True
+
+    def get_device(self):
+        return 0
+
+
+@pytest.fixture
+def taken(monkeypatch):
+    """What ``streamed`` hands to the kernels: (kernel, rows, how)."""
+    calls = []
+    monkeypatch.setattr(sv, "_LIB", types.SimpleNamespace(
+        sv_stream_linear=None, sv_wide_linear=None))
+    monkeypatch.setattr(sv, "_plain", lambda t: True)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    for name in ("wide_linear", "stream_linear"):
+        def kernel(x, w, how, f32=False, glu=False, name=name):
+            calls.append((name, x, how))
+            return torch.empty(x.shape[0], w.shape[0] // (2 if glu else 1))
+        monkeypatch.setattr(sv, name, kernel)
+    return calls
+
+
+def _on_device(*shape):
+    return torch.empty(*shape, dtype=torch.bfloat16).as_subclass(_OnDevice)
+
+
+@pytest.mark.parametrize("B,S,K,N,glu,want", [
+    # beyond the 31 bits of 256 rows' offsets: another kernel, or none
+    (20, 1024, 4096, 32000, False, "stream_linear"), (40, 1024, 4096, 32000, False, None),
+    (32, 1024, 4096, 28672, True, "stream_linear"), (40, 400, 11008, 4096, False, None),
+    # below them
+    (20, 1023, 4096, 32000, False, "wide_linear"), (40, 380, 11008, 4096, False, "wide_linear"),
+    (1, 1024, 4096, 32000, False, "stream_linear")])
+def test_rows_far_apart(taken, B, S, K, N, glu, want):
+    """Last tokens of prompts: a view of rows that lie a prompt apart, whatever the
+    stride of its middle dimension of one."""
+    x, w = _on_device(B, S, K)[:, -1:], _on_device(N, K)
+    with torch.no_grad():
+        out = sv.streamed(x, w, glu=glu)
+    assert [c[0] for c in taken] == ([want] if want else [])
+    if want:
+        assert out.shape == (B, 1, N // 2 if glu else N)
+        assert taken[0][1].stride(0) < 1 << 22 or want == "stream_linear"
+    else:
+        assert out is None
+
+
+def test_a_middle_dimension_of_one_counts_for_nothing(taken):
+    """Its stride may be anything."""
+    x = _on_device(40, 4096).as_strided((40, 1, 4096), (4096, 1 << 23, 1))
+    with torch.no_grad():
+        sv.streamed(x, _on_device(32000, 4096))
+    assert [c[0] for c in taken] == ["wide_linear"]
+
+
 def test_nobody_is_passed_by():
     """Calls go past an autograd function only where nobody would miss it."""
     from torch.utils._python_dispatch import TorchDispatchMode

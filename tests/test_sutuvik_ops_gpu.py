@@ -847,6 +847,23 @@ def test_few_rows_are_streamed_where_nobody_watches(glu):
         assert not any("empty" in str(f) for f in seen)
 
 
+@pytest.mark.parametrize("B,S", [(20, 1024), (40, 1024), (40, 1023)])
+def test_products_of_rows_far_apart(B, S):
+    """The last tokens of prompts, 2^22 elements apart and just below."""
+    from neuronx_distributed_amd.parallel.layers import linear_with_async_allreduce
+
+    x = torch.zeros(B, S, 4096, device="cuda", dtype=torch.bfloat16)[:, -1:]
+    x.copy_(torch.randn(B, 1, 4096, device="cuda"))
+    w = torch.randn(32000, 4096, device="cuda").div(64).bfloat16()
+    with torch.no_grad():
+        out = linear_with_async_allreduce(x, w)
+        logits = sv.linear_f32(x[:, 0], w)
+    ref = x.double() @ w.double().t()
+    tol = 16 * 64 * 2.0 ** -24             # of K products, as above
+    torch.testing.assert_close(out.double(), ref, rtol=2.0 ** -8, atol=tol)
+    torch.testing.assert_close(logits.double(), ref[:, 0], rtol=0, atol=tol)
+
+
 @pytest.mark.parametrize("residual", [True, False])
 @pytest.mark.parametrize("K,N,glu", [
     (8, 16, False), (520, 1001, False), (2056, 48, False), (4096, 8192, False),
