@@ -466,8 +466,9 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor, rule) -> Optional[tuple]:
         return None
     K = shape[-1]
     T = shape[0] if len(shape) == 2 else x.numel() // K if K else 0
-    if not 0 < T <= 128 or not K or K != size[1] or x.dtype != torch.bfloat16 or \
-            w.dtype != torch.bfloat16 or w.stride(1) != 1 or \
+    if not 0 < T <= 128 or not K or K != size[1] or not size[0] or \
+            x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or \
+            w.stride(1) != 1 or \
             x.get_device() != torch._C._cuda_getDevice() or \
             w.get_device() != x.get_device() or \
             os.environ.get("NXDA_SKINNY_GEMM", "1") != "1":

@@ -288,6 +288,17 @@ def test_a_middle_dimension_of_one_counts_for_nothing(taken):
     assert [c[0] for c in taken] == ["wide_linear"]
 
 
+@pytest.mark.parametrize("T", [1, 16, 40, 128])
+def test_weights_without_rows_are_the_library_s(taken, T):
+    """There is nothing to share among workgroups."""
+    with torch.no_grad():
+        for glu in (False, True):
+            assert sv.streamed(_on_device(T, 4096), _on_device(0, 4096), glu=glu) is None
+            assert sv.stream_how(_on_device(T, 4096), _on_device(0, 4096),
+                                 glu=glu) is None
+    assert not taken
+
+
 def test_nobody_is_passed_by():
     """Calls go past an autograd function only where nobody would miss it."""
     from torch.utils._python_dispatch import TorchDispatchMode
