@@ -470,6 +470,17 @@ def input_weight(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return w
 
 
+def input_grad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """dy (..., N) w, w (N, K).  With a turned weight it is one product of all rows:
+    torch makes a batch of them where the strides of dy's dimensions of one do not
+    follow from the others (one sequence, tokens first) and nobody differentiates the
+    second operand."""
+    laid = input_weight(dy, w)
+    if laid is w:
+        return dy.matmul(w)
+    return dy.reshape(-1, w.shape[0]).mm(laid).view(*dy.shape[:-1], w.shape[1])
+
+
 # ---------------------------------------------------------------------------
 # embedding
 # ---------------------------------------------------------------------------

@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
-from ..ops import embedding, input_weight, weight_grads
+from ..ops import embedding, input_grad, weight_grads
 from ..ops.serving import unseen
 from . import comm
 from . import parallel_state as ps
@@ -190,7 +190,7 @@ class _RPLOverlappedLinearRS(torch.autograd.Function):
         input_parallel, weight = ctx.saved_tensors
         tp_info = ps.get_group_info("tp")
         g = comm.all_gather(grad_output.contiguous(), dim=0, group=tp_info)
-        grad_input = g.matmul(input_weight(g, weight))
+        grad_input = input_grad(g, weight)
         go2d = g.reshape(-1, g.shape[-1])
         in2d = input_parallel.reshape(-1, input_parallel.shape[-1])
         (grad_weight,) = weight_grads([go2d], in2d)
@@ -304,7 +304,7 @@ class LinearWithAsyncCommunication(torch.autograd.Function):
         handle = None
 
         grad_output = grad_output.contiguous()
-        grad_input = grad_output.matmul(input_weight(grad_output, weight))
+        grad_input = input_grad(grad_output, weight)
 
         if ctx.sequence_parallel_enabled and ctx.compute_weight_gradient:
             # re-gather the saved sharded input for the weight-grad GEMM

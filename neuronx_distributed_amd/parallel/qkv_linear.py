@@ -21,7 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.distributed as dist
 
-from ..ops import input_weight, weight_grads
+from ..ops import input_grad, input_weight, weight_grads
 from . import comm
 from . import parallel_state as ps
 from .layers import BaseParallelLinear, default_init_method
@@ -109,7 +109,7 @@ class _QKVLinearWithAsyncCommunication(torch.autograd.Function):
         gq = gq.contiguous()
         gk = gk.contiguous()
         gv = gv.contiguous()
-        grad_input = gq.matmul(input_weight(gq, wq))
+        grad_input = input_grad(gq, wq)
         rows = grad_input.view(-1, grad_input.shape[-1])
         for g, w in ((gk, wk), (gv, wv)):      # sums inside the products
             rows.addmm_(g.view(-1, g.shape[-1]), input_weight(g, w))

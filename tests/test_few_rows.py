@@ -352,3 +352,49 @@ def test_weights_of_an_input_gradient(T, N, K, want):
     from neuronx_distributed_amd.ops import turn_weight_rule
 
     assert turn_weight_rule(T, N, K) is want
+
+
+@pytest.mark.parametrize("shape,stride", [
+    ((8, 1, 6), (6, 48, 1)), ((1, 8, 6), (6, 6, 1)), ((8, 1, 6), (6, 6, 1)),
+    ((2, 4, 6), (24, 6, 1)), ((8, 6), (6, 1))])
+@pytest.mark.parametrize("overlapped", [False, True])
+def test_input_gradients_are_one_product(monkeypatch, shape, stride, overlapped):
+    """Also of gradients that are contiguous with any stride of a dimension of one:
+    one sequence, tokens first.  Not a batch of products with a turned weight."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from neuronx_distributed_amd import ops
+    from neuronx_distributed_amd.parallel import layers
+
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+            seen.append(str(f))
+            return f(*args, **(kwargs or {}))
+
+    turned = []
+
+    def turn(dy, w):
+        turned.append(w)
+        return w.detach().t().contiguous().t()
+
+    for module in (ops, layers):
+        monkeypatch.setattr(module, "input_weight", turn, raising=False)
+    monkeypatch.setattr(layers.ps, "get_group_info",
+                        lambda name: types.SimpleNamespace(size=1, group=None))
+    monkeypatch.setattr(layers.comm, "all_gather", lambda t, dim, group: t)
+    dy = torch.randn(8, 6).as_strided(shape, stride)
+    assert dy.is_contiguous()
+    x, w = torch.randn(*shape[:-1], 4), torch.randn(6, 4).requires_grad_()
+    ctx = types.SimpleNamespace(
+        saved_tensors=(x, w), compute_weight_gradient=True, use_bias=False,
+        sequence_parallel_enabled=False, async_grad_allreduce=False)
+    function = layers._RPLOverlappedLinearRS if overlapped else \
+        layers.LinearWithAsyncCommunication
+    with torch.no_grad(), Watch():
+        dx, dw = function.backward(ctx, dy)[:2]
+    assert turned and not any("bmm" in f for f in seen)
+    rows = dy.reshape(8, 6)
+    torch.testing.assert_close(dx, (rows @ w).view(x.shape))
+    torch.testing.assert_close(dw, rows.t() @ x.reshape(8, 4))
