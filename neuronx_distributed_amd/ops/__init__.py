@@ -525,11 +525,11 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor,
     table where that is bf16 and nobody traces or transforms the call."""
     from .serving import _plain, _unwatched
 
-    if torch.is_grad_enabled() and weight.is_cuda and weight.requires_grad and \
+    if torch.is_grad_enabled() and _plain(weight) and _plain(ids) and \
+            weight.is_cuda and weight.requires_grad and \
             weight.dtype == torch.bfloat16 and ids.dtype == torch.int64 and \
             weight.dim() == 2 and weight.shape[0] and weight.shape[1] and \
-            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 30 and \
-            _plain(weight) and _plain(ids) and _unwatched():
+            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 30 and _unwatched():
         return _EmbeddingFn.apply(ids, weight, padding_idx)
     return torch.nn.functional.embedding(ids, weight, padding_idx)
 

@@ -398,3 +398,22 @@ def test_input_gradients_are_one_product(monkeypatch, shape, stride, overlapped)
     rows = dy.reshape(8, 6)
     torch.testing.assert_close(dx, (rows @ w).view(x.shape))
     torch.testing.assert_close(dw, rows.t() @ x.reshape(8, 4))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_embeddings_are_traced_symbolically(monkeypatch, grad):
+    """Nothing is asked of a proxy that steers the program."""
+    from neuronx_distributed_amd.parallel import layers
+
+    monkeypatch.setattr(layers.ps, "get_tensor_model_parallel_size", lambda: 1)
+    embed = layers.ParallelEmbedding.__new__(layers.ParallelEmbedding)
+    torch.nn.Module.__init__(embed)
+    embed.weight = torch.nn.Parameter(torch.randn(16, 8))
+    embed.padding_idx, embed.shard_along_embedding = None, False
+    with torch.set_grad_enabled(grad):
+        traced = torch.fx.symbolic_trace(torch.nn.Sequential(embed))
+    ids = torch.randint(16, (3, 5))
+    out = traced(ids)
+    assert torch.equal(out, embed.weight[ids])
+    (g,) = torch.autograd.grad(out.sum(), embed.weight)
+    assert g.shape == embed.weight.shape
