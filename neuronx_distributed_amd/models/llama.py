@@ -359,12 +359,13 @@ def _embedded(embed, tokens):
     takes from the table itself, where nobody sees or stands for the look-up."""
     from ..ops import serving as sv
 
-    w = embed.weight
-    if type(embed) is ParallelEmbedding and not _watched(embed) and \
-            w.is_cuda and w.is_contiguous() and sv.unseen(w, tokens) and \
-            tokens.dtype == torch.int32 and tokens.is_contiguous() and \
-            w.dtype == torch.bfloat16 and ps.get_tensor_model_parallel_size() == 1:
-        return sv.Pending(w, rows=tokens)
+    if type(embed) is ParallelEmbedding and not _watched(embed):
+        w = embed.weight
+        if w.is_cuda and w.is_contiguous() and sv.unseen(w, tokens) and \
+                tokens.dtype == torch.int32 and tokens.is_contiguous() and \
+                w.dtype == torch.bfloat16 and \
+                ps.get_tensor_model_parallel_size() == 1:
+            return sv.Pending(w, rows=tokens)
     return sv.Pending(embed(tokens))
 
 

@@ -417,3 +417,16 @@ def test_embeddings_are_traced_symbolically(monkeypatch, grad):
     assert torch.equal(out, embed.weight[ids])
     (g,) = torch.autograd.grad(out.sum(), embed.weight)
     assert g.shape == embed.weight.shape
+
+
+def test_an_embedding_without_a_weight_is_called():
+    """A served model's look-up may be any module."""
+    from neuronx_distributed_amd.models import llama
+
+    class Twice(torch.nn.Module):
+        def forward(self, tokens):
+            return 2.0 * tokens[:, None]
+
+    pending = llama._embedded(Twice(), torch.tensor([3, 4]))
+    assert pending.rows is None
+    assert torch.equal(pending.delta, torch.tensor([[6.0], [8.0]]))
