@@ -361,7 +361,8 @@ def _embedded(embed, tokens):
 
     if type(embed) is ParallelEmbedding and not _watched(embed):
         w = embed.weight
-        if w.is_cuda and w.is_contiguous() and sv.unseen(w, tokens) and \
+        if w.is_cuda and w.is_contiguous() and not w.data_ptr() & 15 and \
+                sv.unseen(w, tokens) and \
                 tokens.dtype == torch.int32 and tokens.is_contiguous() and \
                 w.dtype == torch.bfloat16 and \
                 ps.get_tensor_model_parallel_size() == 1:

@@ -430,3 +430,22 @@ def test_an_embedding_without_a_weight_is_called():
     pending = llama._embedded(Twice(), torch.tensor([3, 4]))
     assert pending.rows is None
     assert torch.equal(pending.delta, torch.tensor([[6.0], [8.0]]))
+
+
+@pytest.mark.parametrize("shift,rows", [(0, True), (8, True), (4, False), (1, False)])
+def test_rows_of_a_table_start_at_whole_words(taken, monkeypatch, shift, rows):
+    """A table inside a larger buffer may start anywhere; its norm reads words."""
+    from neuronx_distributed_amd.models import llama
+    from neuronx_distributed_amd.parallel import layers
+
+    monkeypatch.setattr(llama.ps, "get_tensor_model_parallel_size", lambda: 1)
+    embed = layers.ParallelEmbedding.__new__(layers.ParallelEmbedding)
+    torch.nn.Module.__init__(embed)
+    embed.__dict__.update(
+        weight=_on_device(5 * 16 + 8)[shift:shift + 80].view(5, 16),
+        padding_idx=None, shard_along_embedding=False)
+    tokens = torch.tensor([1, 4], dtype=torch.int32)
+    with torch.no_grad():
+        pending = llama._embedded(embed, tokens)
+    assert (pending.rows is tokens) == rows
+    assert (pending.delta is embed.weight) == rows
