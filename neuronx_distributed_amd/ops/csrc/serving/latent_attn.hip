@@ -444,8 +444,12 @@ __device__ __forceinline__ Share share_of(const LatentRowsArgs& a, int item) {
   return {-1, 0, 0};
 }
 
-// FULL: R = EP and P = 64, no padding
-template <int EP, bool FULL>
+// FULL: R = EP and P = 64, no padding.  ONCE: up to 32 heads, nobody else reads the
+// tiles, and no cache keeps them (rank 512, caches that no earlier call has read, us,
+// kept | past: 32 heads, 89 rows of 3161 84 | 81, 12 of 402 16.2 | 15.5; 16 heads, 2 of
+// up to 2481 14.5 | 13.3).  Of more heads workgroups of 32 read the same ones (128
+// heads, 128 rows of 1472 146 | 161, 15 of 504 23.5 | 26.8; 40, 10 of 2057 25.0 | 28.3).
+template <int EP, bool FULL, bool ONCE>
 __global__ void __launch_bounds__(256, 2)
 latent_rows_kernel(LatentRowsArgs a) {
   constexpr int KP = EP + 64;            // columns of a tile row
@@ -513,8 +517,10 @@ latent_rows_kernel(LatentRowsArgs a) {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int it = i * 256 + tid;
-      if (FULL)                          // a tile is one piece, and read once
+      if (FULL && ONCE)                  // a tile is one piece
         reg[i] = __builtin_nontemporal_load((const uint4v*)(src + it * 8u));
+      else if (FULL)
+        reg[i] = *(const uint4v*)(src + it * 8u);
       else
         reg[i] = word(src + it / CPR * RP, column(it % CPR));
     }
@@ -850,10 +856,12 @@ static int launch_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
   const long grid = (long)a->rows * ((a->H + 31) / 32) * a->splits;
   const bool full = a->P == 64 && (a->R == 64 || a->R == 128 || a->R == 256 ||
                                    a->R == 512);
-#define LR(E)                                                       \
-  do {                                                              \
-    if (full) latent_rows_kernel<E, true><<<grid, 256, 0, stream>>>(*a); \
-    else latent_rows_kernel<E, false><<<grid, 256, 0, stream>>>(*a);     \
+#define LRK(E, F, O) latent_rows_kernel<E, F, O><<<grid, 256, 0, stream>>>(*a)
+#define LR(E)                                           \
+  do {                                                  \
+    if (full && a->H <= 32) LRK(E, true, true);         \
+    else if (full) LRK(E, true, false);                 \
+    else LRK(E, false, false);                          \
   } while (0)
   if (a->P > 64 ||
       (a->splits > 1 && (long)a->rows * a->splits > LATENT_SHARES))
@@ -864,6 +872,7 @@ static int launch_latent_rows(const LatentRowsArgs* a, hipStream_t stream) {
   else if (a->R <= 512) LR(512);
   else return 1;
 #undef LR
+#undef LRK
   return 0;
 }
 
