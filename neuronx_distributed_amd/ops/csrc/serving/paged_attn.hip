@@ -486,7 +486,9 @@ __device__ __forceinline__ float max_quarters(float x) {
 // ROT: the row's queries and key are turned here, an element with that half a head
 // on, which the same lane holds.  As a kernel of its own, which every layer waits
 // for, that took 4.6 us (4 layers, 16 steps: one request 7840 -> 7740 us).
-template <bool MOD, int DE, bool ROT>
+// ONCE: up to 16 heads a group, nobody else reads a tile, and no cache keeps its values
+// (32 heads of one group, 200 rows of 448, kept 20.1, past 21.0 us; of 180 12.3, 12.9).
+template <bool MOD, int DE, bool ROT, bool ONCE>
 __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
   constexpr int NC = DE / 32;            // chunks of a key
   constexpr int NB = DE / 16;            // 16-row blocks of O^T
@@ -588,7 +590,8 @@ __global__ void __launch_bounds__(256, 2) attn_rows_mfma_kernel(RowsArgs a) {
       const short* src = a.append && r >= newest
                              ? vn : vb + (long)min(r, newest) * a.vcs;
       __builtin_amdgcn_global_load_lds(
-          (global_ptr)(src + c), (lds_ptr)(vd + wid * VB + p * 1024), 16, 0, 2);
+          (global_ptr)(src + c), (lds_ptr)(vd + wid * VB + p * 1024), 16, 0,
+          ONCE ? 2 : 0);
     }
   };
   // a transposing read: 16 lanes turn 4 keys by 16 columns
@@ -865,7 +868,10 @@ static int launch_rows(const RowsArgs& a, int vec, hipStream_t stream) {
   if (a.cos && vec != 2) return 1;
   if (vec == 2) {
     if (sizeof(T) != 2 || a.D != a.E || (a.D != 64 && a.D != 128)) return 1;
-#define ARM(D, R) attn_rows_mfma_kernel<MOD, D, R><<<grid, 256, 0, stream>>>(a)
+#define ARMO(D, R, O) \
+  attn_rows_mfma_kernel<MOD, D, R, O><<<grid, 256, 0, stream>>>(a)
+#define ARM(D, R) \
+  do { if (nrc == 1) ARMO(D, R, true); else ARMO(D, R, false); } while (0)
     if (a.cos) {
       if constexpr (MOD) return 1;
       else if (!a.append) return 1;
@@ -874,6 +880,7 @@ static int launch_rows(const RowsArgs& a, int vec, hipStream_t stream) {
     } else if (a.D == 64) ARM(64, false);
     else ARM(128, false);
 #undef ARM
+#undef ARMO
     if (a.splits > 1)
       return sv_attn_merge(a.part, a.out, (long)a.rows * a.H, a.splits, a.E, 0,
                            stream);
