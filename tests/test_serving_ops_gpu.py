@@ -560,6 +560,13 @@ def test_residual_norm_of_wide_rows(sv, rows, W, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,window", [(17, 0), (40, 70)])
+def test_single_rows_that_several_workgroups_read(sv, H, window, dtype):
+    """The same of heads of 64 whose group several workgroups share."""
+    test_single_rows_turned_in_the_kernel(sv, H, 1, 64, window, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,G,D,shift", [(1, 0, 2, 0), (3, 1, 24, 0),
                                          (5, 2, 36, 0), (32, 8, 128, 0),
                                          (32, 8, 128, 1), (7, 7, 64, 4)])
