@@ -529,7 +529,7 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor,
             weight.is_cuda and weight.requires_grad and \
             weight.dtype == torch.bfloat16 and ids.dtype == torch.int64 and \
             weight.dim() == 2 and weight.shape[0] and weight.shape[1] and \
-            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 30 and _unwatched():
+            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 24 and _unwatched():
         return _EmbeddingFn.apply(ids, weight, padding_idx)
     return torch.nn.functional.embedding(ids, weight, padding_idx)
 

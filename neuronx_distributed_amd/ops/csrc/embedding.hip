@@ -124,7 +124,8 @@ __global__ void __launch_bounds__(1024) embedding_many_kernel(EmbArgs a) {
 // work: 3 V + 1 + T / (EMB_MANY + 1) ints
 extern "C" int embedding_bwd(const void* ids, const void* dy, void* out, int* work,
                              int T, int V, int W, int skip, hipStream_t stream) {
-  if (T <= 0 || V <= 0 || W <= 0 || W % 8) return 1;
+  // (a workgroup of 256 a row: fewer than 2^32 threads)
+  if (T <= 0 || V <= 0 || V >= 1 << 24 || W <= 0 || W % 8) return 1;
   const EmbArgs a = {(const long*)ids, (const short*)dy, (short*)out, work, work + V,
                      work + 2 * V, work + 3 * V, T, V, W, skip};
   embedding_clear_kernel<<<(V + 255) / 256, 256, 0, stream>>>(a);

@@ -449,3 +449,16 @@ def test_rows_of_a_table_start_at_whole_words(taken, monkeypatch, shift, rows):
         pending = llama._embedded(embed, tokens)
     assert (pending.rows is tokens) == rows
     assert (pending.delta is embed.weight) == rows
+
+
+@pytest.mark.parametrize("rows,own", [((1 << 24) - 1, True), (1 << 24, False)])
+def test_embedding_gradients_of_a_grid_s_rows(taken, monkeypatch, rows, own):
+    """A workgroup of 256 a row: a grid has fewer than 2^32 threads."""
+    from neuronx_distributed_amd import ops
+
+    went = []
+    monkeypatch.setattr(ops._EmbeddingFn, "apply",
+                        lambda ids, w, skip: went.append(True) or w[:1])
+    weight = _on_device(rows, 8).requires_grad_()
+    ops.embedding(torch.tensor([3]), weight)
+    assert bool(went) == own
