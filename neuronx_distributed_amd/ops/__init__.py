@@ -35,6 +35,8 @@ def _load():
         _LIB_ERR = str(e)
         return None
     _declare_flash(lib)
+    if hasattr(lib, "embedding_work"):
+        lib.embedding_work.restype = ctypes.c_long
     _LIB = lib
     return _LIB
 
@@ -485,8 +487,16 @@ def input_grad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # embedding
 # ---------------------------------------------------------------------------
 
-# a row's tokens are looked for among all between its first and its last
-EMBEDDING_TOKENS = 32768
+def embedding_rule(T: int, V: int, W: int) -> bool:
+    """Is ``_EmbeddingFn`` the faster one for T tokens and a table (V, W)?  Over 400
+    calls, of tokens evenly and unevenly spread, far apart, of one row and of padding
+    (torch's and this, us): from 2048 tokens on, below which the host takes longer than
+    the device (32000 x 4096: 512 tokens 78, 71, 2048 187, 66; 256 x 512: 512 40, 68,
+    1536 66, 68, 2048 85, 68), up to 32768 (32000 x 4096: 1000, 143; 40 words of 8192 x
+    768: 146, 130, of 65536 tokens 197, 247), of rows from 1 KB and tables up to 2^18
+    (32768 tokens, 262144 x 512: 240, 130; 10^6 x 512, 3073 tokens 222, 240; 10^6 x 64:
+    102, 176)."""
+    return 2048 <= T <= 32768 and W >= 512 and W % 8 == 0 and 0 < V <= 1 << 18
 
 
 class _EmbeddingFn(torch.autograd.Function):
@@ -503,7 +513,7 @@ class _EmbeddingFn(torch.autograd.Function):
         (ids,) = ctx.saved_tensors
         skip = -1 if ctx.skip is None else ctx.skip % ctx.rows
         T, W = ids.numel(), dy.shape[-1]
-        if not (unseen(dy, ids) and 0 < T <= EMBEDDING_TOKENS and dy.is_cuda
+        if not (unseen(dy, ids) and dy.is_cuda
                 and dy.get_device() == torch._C._cuda_getDevice()):
             return None, torch.ops.aten.embedding_dense_backward(
                 dy, ids, ctx.rows, skip, False), None
@@ -511,10 +521,11 @@ class _EmbeddingFn(torch.autograd.Function):
         if rows.data_ptr() & 15:
             rows = rows.clone()
         out = torch.empty(ctx.rows, W, dtype=dy.dtype, device=dy.device)
-        work = torch.empty(3 * ctx.rows + 1 + T // 9, dtype=torch.int32,
+        lib = _require_lib()
+        work = torch.empty(lib.embedding_work(T, ctx.rows, W), dtype=torch.int32,
                            device=dy.device)
-        if _require_lib().embedding_bwd(_ptr(ids), _ptr(rows), _ptr(out), _ptr(work),
-                                        T, ctx.rows, W, skip, _stream()):
+        if lib.embedding_bwd(_ptr(ids), _ptr(rows), _ptr(out), _ptr(work),
+                             T, ctx.rows, W, skip, _stream()):
             raise RuntimeError("embedding_bwd failed")
         return None, out, None
 
@@ -528,8 +539,8 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor,
     if torch.is_grad_enabled() and _plain(weight) and _plain(ids) and \
             weight.is_cuda and weight.requires_grad and \
             weight.dtype == torch.bfloat16 and ids.dtype == torch.int64 and \
-            weight.dim() == 2 and weight.shape[0] and weight.shape[1] and \
-            weight.shape[1] % 8 == 0 and weight.shape[0] < 1 << 24 and _unwatched():
+            weight.dim() == 2 and embedding_rule(ids.numel(), *weight.shape) and \
+            _unwatched():
         return _EmbeddingFn.apply(ids, weight, padding_idx)
     return torch.nn.functional.embedding(ids, weight, padding_idx)
 

@@ -451,14 +451,18 @@ def test_rows_of_a_table_start_at_whole_words(taken, monkeypatch, shift, rows):
     assert (pending.delta is embed.weight) == rows
 
 
-@pytest.mark.parametrize("rows,own", [((1 << 24) - 1, True), (1 << 24, False)])
-def test_embedding_gradients_of_a_grid_s_rows(taken, monkeypatch, rows, own):
-    """A workgroup of 256 a row: a grid has fewer than 2^32 threads."""
+@pytest.mark.parametrize("T,V,W,own", [
+    (2048, 1 << 18, 512, True), (2048, (1 << 18) + 1, 512, False),
+    (2048, 1 << 24, 512, False), (2047, 32000, 4096, False),
+    (32768, 32000, 4096, True), (32769, 32000, 4096, False),
+    (8192, 32000, 504, False), (8192, 32000, 516, False)])
+def test_embedding_gradients_at_their_lines(taken, monkeypatch, T, V, W, own):
     from neuronx_distributed_amd import ops
 
     went = []
     monkeypatch.setattr(ops._EmbeddingFn, "apply",
                         lambda ids, w, skip: went.append(True) or w[:1])
-    weight = _on_device(rows, 8).requires_grad_()
-    ops.embedding(torch.tensor([3]), weight)
+    weight = _on_device(V, W).requires_grad_()
+    assert ops.embedding_rule(T, V, W) is own
+    ops.embedding(torch.zeros(T, dtype=torch.int64), weight)
     assert bool(went) == own

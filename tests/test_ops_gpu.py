@@ -1008,8 +1008,9 @@ def test_turned_weight_of_an_input_gradient():
     (300, 40, 520, -1, "any"), (700, 5000, 2056, 0, "any"),
     (2000, 32000, 4096, None, "any"), (1500, 900, 1032, 3, "few"),
     (8192, 100, 512, None, "one")])
-def test_embedding_gradient(T, V, W, skip, kind):
+def test_embedding_gradient(monkeypatch, T, V, W, skip, kind):
     """Rows without tokens, of one, two, up to eight and more; of all."""
+    monkeypatch.setattr(ops, "embedding_rule", lambda *sizes: True)
     ids = torch.randint(V, (T,), device="cuda")
     if kind == "one":
         ids[:] = V // 2
@@ -1036,3 +1037,29 @@ def test_embedding_gradient(T, V, W, skip, kind):
     dy.requires_grad_()
     (g,) = torch.autograd.grad(out, w, dy, create_graph=True)
     assert g.requires_grad
+
+
+@pytest.mark.parametrize("each,V,W", [
+    (1, 9000, 8), (3, 70, 8), (8, 900, 520), (9, 1900, 2056), (16, 600, 512),
+    (17, 500, 1032), (256, 20, 64), (257, 20, 520), (1000, 9, 64), (6000, 3, 1032)])
+def test_embedding_gradient_of_rows_far_apart(monkeypatch, each, V, W):
+    """Every row's tokens lie over all of them: as many as a wave and a workgroup take
+    and one more, parts of rows; more rows than waves and workgroups at once."""
+    monkeypatch.setattr(ops, "embedding_rule", lambda *sizes: True)
+    T = each * V
+    ids = torch.arange(T, device="cuda") % V
+    if each == 1000:
+        ids[::2] = ids[::2] // 3 * 3       # unequal ones, some without
+        ids[:3000] = 4                     # and parts that have more than others
+    w = torch.randn(V, W, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(T, W, device="cuda", dtype=torch.bfloat16)
+    out = ops.embedding(ids, w)
+    (got,) = torch.autograd.grad(out, w, dy, retain_graph=True)
+    (again,) = torch.autograd.grad(out, w, dy)
+    assert torch.equal(got, again)
+    want = torch.zeros(V, W, device="cuda", dtype=torch.float64)
+    want.index_add_(0, ids, dy.double())
+    size = torch.zeros_like(want).index_add_(0, ids, dy.double().abs())
+    # rounded to 8 bits; sums of up to T terms in float32
+    bound = want.abs() * 2 ** -8 + 2 * T * 2 ** -24 * size
+    assert ((got.double() - want).abs() <= bound).all()
