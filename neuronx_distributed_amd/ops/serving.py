@@ -1828,7 +1828,7 @@ def _latent_step(q, kv, gate, pos, seq, block_table, max_keys, cache,
     assert w.expand.shape == (heads * (dim + vdim), R)
     assert w.expand.is_contiguous() and q.stride(1) == out.stride(1) == 1
     assert q.dtype == w.absorb.dtype == w.expand.dtype == out.dtype
-    assert q.shape[1] >= heads * (dim + P) - P and out.shape[1] == heads * vdim
+    assert q.shape[1] >= heads * (dim + P) and out.shape[1] == heads * vdim
     if window > 0:
         max_keys = min(max_keys, window) if max_keys else window
     # absorbed queries, then merged rows: a workspace that only kernels see

@@ -466,3 +466,29 @@ def test_embedding_gradients_at_their_lines(taken, monkeypatch, T, V, W, own):
     assert ops.embedding_rule(T, V, W) is own
     ops.embedding(torch.zeros(T, dtype=torch.int64), weight)
     assert bool(went) == own
+
+
+@pytest.mark.parametrize("short", [0, 1, 8])
+def test_a_latent_step_reads_whole_queries(monkeypatch, short):
+    """Queries whose last head's turned columns are not all there are refused."""
+    H, dim, P, R, vdim, T = 2, 16, 8, 16, 8, 3
+    calls = []
+    monkeypatch.setattr(sv, "_LIB", types.SimpleNamespace(
+        sv_latent_step=lambda *a: calls.append(a) or 0))
+    monkeypatch.setattr(sv, "_stream", lambda: None)
+    def rand(*shape):
+        return torch.randn(*shape, dtype=torch.bfloat16)
+    w = sv.LatentWeights(rand(R), rand(H, R, dim), rand(H * (dim + vdim), R),
+                         torch.ones(P // 2, dtype=torch.float64).as_subclass(_OnDevice))
+    ints = torch.zeros(T, dtype=torch.int32)
+    batch = types.SimpleNamespace(portion_tokens=0, spans={}, pos=ints, seq=ints,
+                                  block_table=ints.view(-1, 1), max_keys=64)
+    q = rand(T, H * (dim + P) + 8)[:, :H * (dim + P) - short]
+    step = lambda: sv.latent_attention(q, rand(T, R + P), None, batch,  # noqa: E731
+                                       rand(1, 64, R + P), w, H, dim, vdim, 0.1, 1e-5)
+    if short:
+        with pytest.raises(AssertionError):
+            step()
+    else:
+        step()
+    assert len(calls) == (not short)
