@@ -410,12 +410,16 @@ def turn_rule(T: int, N: int, K: int):
 
 
 def _turned(x: torch.Tensor) -> torch.Tensor:
-    """x (T, K) as a view of its columns laid out in rows.  64 words beside them
-    keep the rows of a power of two off one memory channel (8192 rows of 4096:
-    23.3 us, without 24.6; the product of it 204, without 225)."""
+    """x (T, K) as a view of its columns laid out in rows: a copy as large as x, which
+    lives as long as the product that reads it; x itself where there is no room for
+    one.  64 words beside the rows keep those of a power of two off one memory channel
+    (8192 rows of 4096: 23.3 us, without 24.6; the product of it 204, without 225)."""
     T, K = x.shape
     pitch = (T + 63) // 64 * 64 + 64
-    out = torch.empty(K, pitch, dtype=x.dtype, device=x.device)
+    try:
+        out = torch.empty(K, pitch, dtype=x.dtype, device=x.device)
+    except torch.OutOfMemoryError:
+        return x
     if _require_lib().transpose_words(
             _ptr(x), ctypes.c_long(x.stride(0)), _ptr(out), ctypes.c_long(pitch),
             T, K, _stream()):

@@ -492,3 +492,18 @@ def test_a_latent_step_reads_whole_queries(monkeypatch, short):
     else:
         step()
     assert len(calls) == (not short)
+
+
+def test_a_card_without_room_turns_nothing(monkeypatch):
+    """Gradients that fit without a turned copy still do."""
+    from neuronx_distributed_amd import ops
+
+    def full(*a, **k):
+        raise torch.OutOfMemoryError("full")
+
+    x = torch.randn(16, 8)
+    monkeypatch.setattr(torch, "empty", full)
+    assert ops._turned(x) is x
+    monkeypatch.setattr(ops, "input_weight", lambda dy, w: ops._turned(w))
+    w = torch.randn(8, 4)
+    torch.testing.assert_close(ops.input_grad(x, w), x @ w)
