@@ -299,7 +299,7 @@ def test_weights_without_rows_are_the_library_s(taken, T):
     assert not taken
 
 
-def test_nobody_is_passed_by():
+def test_nobody_is_passed_by(monkeypatch):
     """Calls go past an autograd function only where nobody would miss it."""
     from torch.utils._python_dispatch import TorchDispatchMode
 
@@ -328,7 +328,13 @@ def test_nobody_is_passed_by():
         torch.vmap(lambda t: seen.append(sv.unseen(t)) or t)(x)
         assert seen == [False]
         with torch.autocast("cuda"):
-            assert not sv.unseen(x) or not torch.is_autocast_enabled("cuda")
+            # (there is none without a card)
+            assert sv.unseen(x) == (not torch.cuda.is_available())
+        enabled = torch.is_autocast_enabled
+        monkeypatch.setattr(torch, "is_autocast_enabled",
+                            lambda kind=None: kind == "cuda" or enabled(kind))
+        assert not sv.unseen(x)
+        monkeypatch.undo()
     with torch.inference_mode():
         assert sv.unseen(x)
 

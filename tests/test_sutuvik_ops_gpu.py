@@ -521,9 +521,10 @@ def test_timed_memory_in_batches(dtype):
 @pytest.mark.parametrize("N,P", [(64, 64), (128, 64), (64, 192), (128, 128)])
 def test_timed_memory_states_carried_and_scanned(monkeypatch, N, P, carried):
     """Portions that end at, before and behind pieces of 64 and chunks of 256
-    tokens, whose states are carried or made at once, then portions behind
-    them."""
+    tokens, whose states are carried (of 128 keys with their outputs, in one pass) or
+    made at once, then portions behind them."""
     monkeypatch.setattr(sv, "memory_carries", lambda *a: carried)
+    monkeypatch.setattr(sv, "memory_pass", lambda *a: carried)
     H, G = 6, 2
     lens, more = [1, 63, 64, 130, 256, 257, 800, 1025], [70, 1, 300, 64, 2, 511,
                                                          256, 33]
@@ -548,11 +549,14 @@ def test_timed_memory_states_carried_and_scanned(monkeypatch, N, P, carried):
 
 @pytest.mark.parametrize("pitch", [(1 << 22) - 8, 1 << 22])
 @pytest.mark.parametrize("carried", [True, False])
-def test_timed_memory_of_rows_far_apart(monkeypatch, pitch, carried):
+@pytest.mark.parametrize("N", [64, 128])
+def test_timed_memory_of_rows_far_apart(monkeypatch, N, pitch, carried):
     """Chunks of rows as far apart as 31 bits of bytes reach, and one word
-    further, where the general form takes them."""
+    further, where the general form takes them; of 64 keys carried, of 128 in one
+    pass, of both made at once."""
     monkeypatch.setattr(sv, "memory_carries", lambda *a: carried)
-    H, G, N, P, T = 2, 1, 128, 64, 300
+    monkeypatch.setattr(sv, "memory_pass", lambda *a: carried)
+    H, G, P, T = 2, 1, 64, 300
     case = _ssm(T, H, G, N, P, 5, BF16)
     params = _ssm_params(H, BF16)
     want, S_want = _ssm_want(case, params, H, G, N, P)
