@@ -573,8 +573,9 @@ static int launch(const StreamArgs& a, int stay, hipStream_t stream) {
   if (stay) {
     if (a.N % rows) return 1;
     const int grid = min(tiles, 256);
-    // at most 128 registers of x beside the weights (plain products of 17 to
-    // 32 rows by a direct call alone, here and below: the library is faster)
+    // at most 128 registers of x beside the weights; for a K that is not whole blocks
+    // of 64, and sizes that the rings leave (plain products of 17 to 32 rows by a direct
+    // call alone, here and below)
 #define STAY(P, M) \
   stay_linear_kernel<8, P, M, EPI, NORM><<<grid, 512, 0, stream>>>(a)
     if constexpr (NORM) STAY(2, 1);

@@ -617,10 +617,10 @@ def test_memories_of_one_pass():
 
 
 def test_states_are_carried_where_that_is_faster():
-    assert sv.memory_carries(17, 2, 128 * 128 * 64)      # 2 x 2048 tokens
-    assert sv.memory_carries(4, 1, 64 * 128 * 64)        # 1000 tokens
-    assert not sv.memory_carries(64, 1, 64 * 128 * 64)   # 16384 tokens
-    assert not sv.memory_carries(64, 1, 16 * 64 * 64)
+    assert sv.memory_carries(1, 1, 128 * 64 * 64)        # 60 tokens
+    assert not sv.memory_carries(6, 1, 128 * 64 * 64)    # 1472 tokens
+    assert sv.memory_carries(10, 2, 128 * 64 * 128)      # 1445 and 924 tokens
+    assert not sv.memory_carries(14, 1, 16 * 64 * 64)    # 3409 tokens
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
