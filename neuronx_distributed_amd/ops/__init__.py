@@ -393,20 +393,41 @@ def apply_rotary_polar_compatible(query, key, freqs):
 def turn_rule(T: int, N: int, K: int):
     """Which operands of dy^T x, dy (T, N) and x (T, K), are turned first, so that
     the library reads them along T: (dy, x).  It reaches 1.05 PFLOP/s with none,
-    1.23 with one and up to 1.55 with both; turning runs at 5.7 TB/s.  Lines, with
-    the time without it and with it in us: the smaller one from 1600 rows and 20
-    million weights (8192 rows, 22016 x 4096: 1430 -> 1222, 32000 x 4096: 2079 ->
-    1552; 2048, 4096 x 11008: 212 -> 159; but 8192, 2048 x 5632: 175 -> 175, and
-    800, 22016 x 4096: 162 -> 205); both below 2600 rows, where the
-    library has no good form for one (1200, 32000 x 4096: 342 -> 278, with one
-    364), unless one is narrow (2048, 3584 x 18944: 275 -> 302, with one 259),
-    and of widths from 8192 (8192, 8192 x 8192: 940 -> 764, with one 797)."""
-    least = min(N, K)
-    if T < 1100 or N * K < 20_000_000:
+    1.23 with one and up to 1.55 with both; turning runs at 5.7 TB/s.  Its forms, and
+    so the gain, jump with the sizes; lines were drawn over 870 of them where next to
+    none is slower (8 by 2 % to 8 %; gains, with the turning):
+
+    - both of wide ones (from 8192: 1.15 to 1.23), and below 2600 rows, where the
+      library has no good form for one (1200, 32000 x 4096: 342 -> 278 us, with one
+      364), unless a side is below 4096 (2048, 3584 x 18944: 275 -> 302, with one 259)
+      or the weight is small (6144 x 4096: 0.87 to 1.00, 8200 x 4096: 0.86 to 1.05;
+      4096 x 11008: 1100 and 1200 0.97, 1400 to 2600 1.08 to 1.27; 800, 22016 x 4096:
+      162 -> 205);
+    - else the smaller one, from 1600 rows: of weights from 55 million 1.02 to 1.25
+      (8192, 22016 x 4096: 1430 -> 1222; but 1800, 3584 x 18944: 0.96); of smaller
+      ones with a side below 3584 1.00 to 1.41 (8192 x 3072, 22016 x 2048, of which
+      3300 and 5000 rows 0.92; but dy of many rows for weights below 30 million: 2048
+      x 11008: 3300 1.23, from 5000 on 0.97, 2560 x 9728: 0.95 to 1.03); of others up
+      to 9216 rows (5120 x 5120: 1.04 to 1.45, 10752 0.78; 3584 x 8192: 1.03 to 1.6,
+      9728 0.90), with a side from 4096 to 5119 not below 40 million (4096 x 6144:
+      0.87 to 1.02), and not from 3073 to 8191 rows (4096 x 11008: 3072 1.02, 3300
+      0.90, 5000 0.91, 7168 0.98, from 8192 on 0.98 to 1.08; 11008 x 4096: 0.89 to
+      1.16)."""
+    least, size = min(N, K), N * K
+    if T < 1100 or size < 20_000_000:
         return False, False
-    if least >= 8192 or (T < 2600 and least >= 4096):
+    if least >= 8192:
         return True, True
-    return (N <= K, N > K) if T >= 1600 else (False, False)
+    large, square = size >= 55_000_000, 4096 <= least < 5120
+    if T < 2600 and least >= 4096:
+        both = large or not square or size >= 40_000_000 and T >= 1400
+        return both, both
+    if T < 1600 or not large and (
+            square and (size < 40_000_000 or 3072 < T < 8192) or
+            not square and least >= 3584 and T > 9216 or
+            N < K and size < 30_000_000 and T > 3500):
+        return False, False
+    return N <= K, N > K
 
 
 def _turned(x: torch.Tensor) -> torch.Tensor:
@@ -454,13 +475,16 @@ def weight_grads(grads, x: torch.Tensor):
 
 
 def turn_weight_rule(T: int, N: int, K: int) -> bool:
-    """Is w (N, K) turned for dy w of T rows?  As above, 1.07 to 1.35 times as fast
-    with the turning (8192 rows, 32000 x 4096: 1545 -> 1367 us; 4096 x 4096: 198 ->
-    185; 16384: 391 -> 352).  Not below (6144, 4096 x 11008: 449 -> 493), for other
-    numbers of rows, of which the library has forms that are slower by a third
-    (9000, 4096 x 4096: 338 -> 363), and of the largest weights only for many (8192,
-    27648 x 5120: 2279 -> 2349, 16384: 3429 -> 2982)."""
-    return T >= 8192 and T % 512 == 0 and \
+    """Is w (N, K) turned for dy w of T rows?  As above, 1.01 to 1.32 times as fast
+    with the turning where the library's tiles of 256 rows are whole sixteens (8192
+    rows, 32000 x 4096: 1545 -> 1367 us; 4096 x 4096: 198 -> 185, so from 7937 rows
+    on; 12288: 1.03 to 1.10; 16384: 391 -> 352), and of any 24576 rows and more (1.06
+    to 1.18).  Others jump (4096 x 4096: 7872 rows 1.08, 11776 0.87, 12544 0.93, 13568
+    1.10, 20000 0.96; 32000 x 4096: 6656 0.82, 7168 1.30, 7680 0.85, 7872 0.93, 8256
+    0.99, 10240 0.93).  Not below (6144, 4096 x 11008: 449 -> 493), and of the largest
+    weights only for many (8192, 27648 x 5120: 2279 -> 2349, 16384: 3429 -> 2982)."""
+    tiles = -(-T // 256)
+    return tiles >= 32 and (tiles % 16 == 0 or T >= 24576) and \
         16_000_000 < N * K < (140_000_000 if T < 16384 else 1 << 31)
 
 

@@ -360,6 +360,33 @@ def test_weights_of_an_input_gradient(T, N, K, want):
     assert turn_weight_rule(T, N, K) is want
 
 
+@pytest.mark.parametrize("T,N,K,want", [
+    # each line of the rule, and past it
+    (2599, 6144, 4096, (False, False)), (1399, 4096, 11008, (False, False)),
+    (1400, 4096, 11008, (True, True)), (1100, 4096, 14336, (True, True)), (1100, 5120, 5120, (True, True)),
+    (3500, 2560, 9728, (True, False)), (3501, 2560, 9728, (False, False)),
+    (3501, 8192, 3072, (False, True)), (3501, 2560, 12288, (True, False)),
+    (3072, 11008, 4096, (False, True)), (3073, 11008, 4096, (False, False)),
+    (8191, 11008, 4096, (False, False)), (8192, 11008, 4096, (False, True)),
+    (9216, 5120, 5120, (True, False)), (9217, 5120, 5120, (False, False)),
+    (9217, 3584, 8192, (False, False)), (9217, 8192, 3072, (False, True)),
+    (8192, 6144, 4096, (False, False)), (5000, 22016, 4096, (False, True))])
+def test_operands_that_are_not_turned(T, N, K, want):
+    from neuronx_distributed_amd.ops import turn_rule
+
+    assert turn_rule(T, N, K) == want
+
+
+@pytest.mark.parametrize("T,want", [
+    (7936, False), (7937, True), (8192, True), (8193, False), (8704, False),
+    (12032, False), (12288, True), (15872, False), (24575, True), (24577, True),
+    (24320, False), (30000, True)])
+def test_weights_are_turned_for_whole_rounds(T, want):
+    from neuronx_distributed_amd.ops import turn_weight_rule
+
+    assert turn_weight_rule(T, 4096, 4096) is want
+
+
 @pytest.mark.parametrize("shape,stride", [
     ((8, 1, 6), (6, 48, 1)), ((1, 8, 6), (6, 6, 1)), ((8, 1, 6), (6, 6, 1)),
     ((2, 4, 6), (24, 6, 1)), ((8, 6), (6, 1))])

@@ -961,7 +961,7 @@ def test_turned_rows(T, K, pitch):
 
 
 @pytest.mark.parametrize("T,K,widths,aligned", [
-    (1111, 4096, (8200,), True),             # both operands
+    (1111, 4096, (14344,), True),            # both operands
     (2601, 2048, (8192, 1024, 1024), True),  # x for all of them
     (2601, 11008, (2056,), True),            # dy
     (2600, 8200, (8192,), True),             # both, of wide ones
