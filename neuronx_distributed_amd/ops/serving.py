@@ -332,7 +332,8 @@ def ring_rule(T: int, N: int, K: int, f32: bool = False,
       workgroups have begun when x is there (7168 x 1024, 16 rows: 10.2, 9.0);
     - short rows of small weights are streamed with 16 waves a workgroup, which
       begin and end sooner (2048 x 2048, 1 row: 4.7, 5.0; 8192 x 2048: 7.5, 8.7;
-      32000 x 2048: 21.8, 23.7);
+      32000 x 2048: 21.8, 23.7; 4096 x 2560, 6 rows 6.5, 7.1), and of 17 rows and
+      more are the library's (512 x 768: 5.0, 6.0; 1024 x 896: 5.9, 5.4);
     - 17 rows and more stay in registers up to K = 4096 (not of small weights where
       only 5 blocks of 64 columns a wave cover the start: 6144 x 2560, 32 rows: 11.4,
       12.0), and flow for one tile a CU (4096 x 11008, 32 rows: 31.5, 26.5); else
@@ -345,6 +346,8 @@ def ring_rule(T: int, N: int, K: int, f32: bool = False,
         if not glu and (T <= 4 and K <= 2048 and (
                 N <= 8192 or T == 1 and K > 1536) or
                 T == 1 and K <= 3584 and N <= 8192 or
+                T <= 8 and K <= 3072 and 2048 < N <= 4096 and
+                stream_rule(T, N, K, f32) == 0 or
                 T <= 4 and K <= 3072 and N <= 4096 or
                 T > 4 and K <= 1536 and N <= 8192):
             return None
@@ -353,7 +356,7 @@ def ring_rule(T: int, N: int, K: int, f32: bool = False,
             return 3
         return 2 if K <= 8192 else None if K >= 14336 else 3
     if tiles <= 512 and K <= 2048:
-        return 3
+        return 3 if glu or N > 1024 or K >= 1024 else None
     if K <= 4096:
         return None if N < 1024 or 2048 < K < 3072 and 2048 < N < 8192 else 2
     return None if glu or tiles > 256 or \
@@ -375,11 +378,16 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
     - up to 64 rows are the weights'; more are also bound by their way through LDS,
       and the library is faster where rounds of fewer rows a workgroup leave too
       little to each (gated 37888 x 3584, 48 rows: 62.5, 55.0, 100 rows: 72.3, 73.3;
-      43008 x 4096, 100 rows: 97.7, 88.2), and rings up to 32 rows there (34816 x
+      43008 x 4096, 100 rows: 97.7, 88.2; 50304 x 2560, 112 rows: 70.7, 62.5), and rings up to 32 rows there (34816 x
       4096, 32 rows: 54.0, 56.9; 22016 x 4096, of one round: 36.5, 33.7);
     - short K under few weight rows has too little to hide a merge behind (4096 x
-      2048, 40 rows: 9.9, 9.1, 96: 10, 11; 8192 x 3072, 96: 19.2, 21.4)."""
-    if K % 64 or K < 512 or N % 8 or T > 128 or glu and N % 32:
+      2048, 40 rows: 9.9, 9.1; 2560 x 3072, 48: 12.5, 10.4, 3584 x 3584, 56: 14.0,
+      12.5, 4096 x 4096, 100: 19.4, 16.5; 8192 x 3072, 96: 19.2, 21.4), all the more of
+      gates, whose merge has half the threads with twice the sums (1024 x 8192 gated,
+      28 rows: 23.8, 13.7, 3072 x 4096 17.3, 15.8 but 5120 15.3, 16.5), and where the
+      library cuts K evenly (4096 x 8192 gated, 20 rows: 21.8, 20.2; 1024 x 8192, 128
+      rows: 16.4, 14.8)."""
+    if K % 64 or K < 512 or N % 8 or not 0 < T <= 128 or N <= 0 or glu and N % 32:
         return None
     tiles, many = -(-N // 128), T > 64
     splits = max(1, min(256 // tiles, K // 256, 16 if many else 64))
@@ -389,17 +397,22 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
     if T <= 32:
         if K <= 4096:
             take = T >= 17 and N >= 20000 and K >= 1536
+        elif glu and N < 4500:
+            take = T >= 17 and (K > 16384 or N >= 2500 and K >= 5120 and K % 8192 > 0)
         else:
             take = T >= 17 or T >= 9 and N >= 5120 and (
                 K >= 14336 if T < 13 else K >= 11008)
     elif tiles >= 168:
-        take = K >= 1536 and (not many or glu or idle < 0.3)
-    elif glu or N >= 5000:
+        take = K >= 1536 and (not many or glu or
+                              idle < (0.2 if tiles > 256 else 0.3))
+    elif N >= 4500:
         take = K >= (4096 if many else 3072)
-    elif N < 3072:
-        take = K >= (7168 if many else 4096 if N < 2048 else 3072)
+    elif glu:
+        take = K > 16384 or N >= 2500 and K >= (6144 if many and N < 3072 else 5120)
+    elif many:
+        take = K >= (8256 if N < 2500 else 7168 if N < 3072 else 5120)
     else:
-        take = K >= 3072
+        take = K >= (4096 if N < 2048 else 5120)
     return splits if take else None
 
 
