@@ -369,7 +369,10 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
     weight (N, K), or None where the library or ``stream_how`` is the faster one.
     As many shares as leave no CU without a workgroup of 128 weight rows, of 256
     columns at least; of many rows no more than 16, whose sums are as much to write
-    as the weights (1024 x 8192, 128 rows: 14.5 us, by 32 19.3).  Drawn over 3312
+    as the weights (1024 x 8192, 128 rows: 14.5 us, by 32 19.3), and of few columns
+    no more than for 200 CUs (4096 x 4096, 128 rows: by 8 23.6, 6 21.1); of gates of
+    512 columns, and no more than 8 (1024 x 8192, 28 rows: 15.7, by 32 23.8), since
+    their merge has half the threads for as many sums.  Drawn over 7200
     calls of 9 to 128 rows, 1.04 to 1.25 times as fast; us here, there and here:
 
     - up to 32 rows only a K beyond the registers of ``ring_rule`` (4096 x 14336, 17
@@ -382,15 +385,18 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
       4096, 32 rows: 54.0, 56.9; 22016 x 4096, of one round: 36.5, 33.7);
     - short K under few weight rows has too little to hide a merge behind (4096 x
       2048, 40 rows: 9.9, 9.1; 2560 x 3072, 48: 12.5, 10.4, 3584 x 3584, 56: 14.0,
-      12.5, 4096 x 4096, 100: 19.4, 16.5; 8192 x 3072, 96: 19.2, 21.4), all the more of
-      gates, whose merge has half the threads with twice the sums (1024 x 8192 gated,
-      28 rows: 23.8, 13.7, 3072 x 4096 17.3, 15.8 but 5120 15.3, 16.5), and where the
-      library cuts K evenly (4096 x 8192 gated, 20 rows: 21.8, 20.2; 1024 x 8192, 128
-      rows: 16.4, 14.8)."""
+      12.5; 8192 x 3072, 96: 19.2, 21.4), all the more of gates (3072 x 4096 gated, 48
+      rows: 17.3, 15.8, 5120 15.3, 16.5), and where the library cuts K evenly (4096 x
+      8192 gated, 20 rows: 21.8, 20.2; 1024 x 8192, 128 rows: 16.4, 14.8);
+    - 4096 x 4096 is the library's between the batches of captured steps (100 rows:
+      19.3, 17.0; 64: 15.9, 15.6; 128: 21.1, 24.8), where a prompt waits for the host,
+      whose call of it costs 20 us more."""
     if K % 64 or K < 512 or N % 8 or not 0 < T <= 128 or N <= 0 or glu and N % 32:
         return None
     tiles, many = -(-N // 128), T > 64
-    splits = max(1, min(256 // tiles, K // 256, 16 if many else 64))
+    target = 200 if many and not glu and K <= 4096 and tiles <= 64 else 256
+    splits = max(1, min(target // tiles, K // (512 if glu else 256),
+                        8 if glu else 16 if many else 64))
     idle = 1 - tiles * splits / (256 * -(-tiles * splits // 256))
     if tiles > 256 and (idle > 0.15 if T <= 32 else many and idle > 0.38):
         return None
@@ -398,7 +404,8 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
         if K <= 4096:
             take = T >= 17 and N >= 20000 and K >= 1536
         elif glu and N < 4500:
-            take = T >= 17 and (K > 16384 or N >= 2500 and K >= 5120 and K % 8192 > 0)
+            take = T >= 17 and (K >= 5120 and K % 8192 > 0 if N >= 2500 else
+                                K > 8192 and K % 2048 > 0)
         else:
             take = T >= 17 or T >= 9 and N >= 5120 and (
                 K >= 14336 if T < 13 else K >= 11008)
@@ -408,11 +415,12 @@ def wide_rule(T: int, N: int, K: int, f32: bool = False,
     elif N >= 4500:
         take = K >= (4096 if many else 3072)
     elif glu:
-        take = K > 16384 or N >= 2500 and K >= (6144 if many and N < 3072 else 5120)
+        take = K >= (6144 if many and N < 3072 else 5120) if N >= 2500 else \
+            K > 8192 and K % 2048 > 0
     elif many:
-        take = K >= (8256 if N < 2500 else 7168 if N < 3072 else 5120)
+        take = K >= (8256 if N < 2500 else 7168 if N < 3072 else 4096)
     else:
-        take = K >= (4096 if N < 2048 else 5120)
+        take = K >= (4096 if N < 2048 or N >= 3072 else 5120)
     return splits if take else None
 
 

@@ -233,20 +233,24 @@ def test_every_cut_is_one_that_the_launcher_takes():
 
 @pytest.mark.parametrize("T,N,K,glu,want", [
     # each line of a few weight rows, and past it; us by the library, and by shares
-    (28, 1024, 8192, True, None),            # 13.7, 23.8
-    (17, 1024, 18944, True, 32), (20, 4096, 8192, True, None),   # 20.2, 21.8
+    (28, 1024, 8192, True, None),            # 13.7, 15.7
+    (28, 1024, 11008, True, 8), (28, 1024, 14336, True, None),
+    (20, 4096, 8192, True, None),            # 20.2, 21.8
     (20, 4096, 5120, True, 8), (48, 2496, 5120, True, None),
     (48, 3072, 4096, True, None),            # 15.8, 17.3
-    (48, 3072, 5120, True, 10), (72, 2560, 5120, True, None),
-    (72, 2560, 6144, True, 12), (48, 4544, 3072, True, 7),
+    (48, 3072, 5120, True, 8), (72, 2560, 5120, True, None),
+    (72, 2560, 6144, True, 8), (48, 4544, 3072, True, 6),
     (48, 2560, 3072, False, None),           # 10.4, 12.5
-    (48, 3584, 4096, False, None), (48, 3584, 5120, False, 9),
+    (48, 2560, 4096, False, None), (48, 2560, 5120, False, 12),
+    (48, 3584, 3584, False, None), (48, 3584, 4096, False, 9),
     (48, 1536, 4096, False, 16), (48, 1536, 3584, False, None),
-    (100, 4096, 4096, False, None),          # 16.5, 19.4
-    (100, 4096, 5120, False, 8), (128, 1024, 8192, False, None),  # 14.8, 16.4
+    (100, 4096, 3072, False, None), (100, 4096, 4096, False, 6),
+    (64, 4096, 4096, False, 8), (100, 4096, 4160, False, 8),
+    (128, 1024, 8192, False, None),          # 14.8, 16.4
     (128, 1024, 11008, False, 16), (112, 2560, 7168, False, 12),
     (112, 50304, 2560, False, None),         # 62.5, 70.7
-    (112, 24576, 3072, False, 1), (64, 50304, 2560, False, 1)])
+    (112, 24576, 3072, False, 1), (64, 50304, 2560, False, 1),
+    (100, 8192, 4096, False, 3), (100, 8200, 4096, False, 3)])
 def test_lines_of_the_shares(T, N, K, glu, want):
     assert sv.wide_rule(T, N, K, False, glu) == want
 
