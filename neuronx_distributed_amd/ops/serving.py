@@ -1625,8 +1625,8 @@ def normed_linear(x: Optional[torch.Tensor], pending: Pending, eps: float,
     if row is not None and row.shape[0] == 1 and x is None and d.shape[0] and \
             row.dtype == torch.int32 and row.is_cuda:
         table, d = d.shape[0], d[:1]
-    if d is None or d.shape[0] != 1 or (row is not None and not table) or d.dtype != torch.bfloat16 or \
-            not d.is_contiguous() or pending.scale != 1.0 or any(
+    if d is None or d.shape[0] != 1 or (row is not None and not table) or \
+            d.dtype != torch.bfloat16 or not d.is_contiguous() or pending.scale != 1.0 or any(
                 t is not None for t in (pending.delta2, pending.w1, pending.w2,
                                         pending.vec, pending.coef)):
         return None
