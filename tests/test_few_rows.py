@@ -520,7 +520,7 @@ def test_rows_of_a_table_start_at_whole_words(taken, monkeypatch, shift, rows):
 
 @pytest.mark.parametrize("T,V,W,own", [
     (2048, 1 << 18, 512, True), (2048, (1 << 18) + 1, 512, False),
-    (2048, 1 << 24, 512, False), (2047, 32000, 4096, False),
+    (2047, 32000, 4096, False),
     (32768, 32000, 4096, True), (32769, 32000, 4096, False),
     (8192, 32000, 504, False), (8192, 32000, 516, False)])
 def test_embedding_gradients_at_their_lines(taken, monkeypatch, T, V, W, own):
