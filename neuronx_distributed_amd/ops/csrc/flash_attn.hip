@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FwdArgs a) {
   // the largest-causal-work blocks launch first and early finishers absorb
   // the small diagonal blocks.
   const int q0 = (int)(gridDim.y - 1 - blockIdx.y) * FA_QBLK;
-  const int h = blockIdx.x, b = blockIdx.z;
+  const int h = near_head(blockIdx.x, a.Hq), b = blockIdx.z;
   const int hkv = h / (a.Hq / a.Hkv);
   const int qw0 = q0 + wid * 32;         // this wave's first q row
   const int my_q = qw0 + col;            // this lane's q row

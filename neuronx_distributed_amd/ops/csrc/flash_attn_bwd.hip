@@ -340,7 +340,7 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_dq_kernel(BwdArgs a) {
 
   // heads on x, q-blocks on y reversed: biggest-causal-work first
   const int q0 = (int)(gridDim.y - 1 - blockIdx.y) * 128;
-  const int h = blockIdx.x, b = blockIdx.z;
+  const int h = near_head(blockIdx.x, a.Hq), b = blockIdx.z;
   const int hkv = h / (a.Hq / a.Hkv);
   const int qw0 = q0 + wid * 32, my_q = qw0 + col;
   const long q_ld = min(my_q, S - 1);

@@ -986,7 +986,7 @@ attn_tiles_kernel(TilesArgs a) {
   // later tiles of a portion see more keys: they start first
   const int* tl = a.tiles + 4 * (gridDim.y - 1 - blockIdx.y);
   const int seq = tl[0], row0 = tl[1], nrow = tl[2], p0 = tl[3];
-  const int h = blockIdx.x, g = h / (a.H / a.G);
+  const int h = near_head(blockIdx.x, a.H), g = h / (a.H / a.G);
   const int* bt = a.bt + (long)seq * a.MB;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -700,6 +700,26 @@ def test_flash_attn_tile_edges(S, window, causal, Hq, Hkv, scale, offset):
         assert (a.float() - b).norm() <= bound, name
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(8, 2), (16, 16), (24, 6), (40, 8), (20, 4)])
+def test_flash_attn_heads_go_to_their_xcd(Hq, Hkv):
+    """Every head is taken once, with the keys of its group, where heads are a
+    multiple of the XCDs and where they are not."""
+    torch.manual_seed(Hq)
+    B, S, D = 2, 193, 128
+    q, k, v = (torch.randn(B, h, S, D, device="cuda").bfloat16().requires_grad_(True)
+               for h in (Hq, Hkv, Hkv))
+    dy = torch.randn(B, Hq, S, D, device="cuda").bfloat16()
+    out = ops.flash_attn(q, k, v)
+    got = (out, *torch.autograd.grad(out, (q, k, v), dy))
+    qr, kr, vr = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+    ref = _torch_reference(qr, kr, vr)
+    want = (ref, *torch.autograd.grad(ref, (qr, kr, vr), dy.float()))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        # as above, of every head by itself
+        bound = 3 * 2.0 ** -9 * (b.norm(dim=(2, 3)) + 0.05 * (S * D) ** 0.5)
+        assert ((a.float() - b).norm(dim=(2, 3)) <= bound).all(), name
+
+
 def test_add_rmsnorm_train_matches_unfused_autograd():
     """Training fused add+RMSNorm (fwd + the dpass-folding backward) vs
     the unfused bf16 add -> ops.rmsnorm chain: forward outputs equal and
