@@ -196,6 +196,76 @@ def test_attention_edges_show(sv, window, keep, dtype):
                    what=(window, keep, s, cuts[0]))
 
 
+def _halves_values(v, kind):
+    """v (T, G * E) with what decides whether a page becomes halves."""
+    v = v.clone()
+    page = torch.arange(v.shape[0]) // 64
+    if kind == "wide":                     # a page of 2^33 beside usual ones
+        v[70] *= 2.0 ** 20
+        v[71] *= 2.0 ** -13
+    elif kind == "pages":                  # every page is 2^7 of the next one
+        v *= (2.0 ** (-7 * page.double()))[:, None].to(v.dtype)
+    elif kind == "zeros":
+        v[64:128] = 0
+        v[::3, ::5] = 0
+    elif kind == "ends":                   # the least and the largest that fit
+        v[:] = v.sign() * 2.0 ** -29
+        v[::2, 1::3] = 1.9921875
+    elif kind == "tiny":                   # some of them too small for bf16
+        v *= 2.0 ** -120
+    elif kind == "large":
+        v *= 2.0 ** 100
+    return v
+
+
+@pytest.mark.parametrize("kind", ["plain", "wide", "pages", "zeros", "ends",
+                                  "tiny", "large"])
+@pytest.mark.parametrize("H,G,D,E,window,keep", [
+    (4, 2, 128, 128, 0, 0), (3, 1, 64, 64, 90, 21), (2, 2, 96, 40, 64, 64),
+    (4, 1, 24, 72, 0, 0)])
+def test_values_as_halves(sv, monkeypatch, kind, H, G, D, E, window, keep):
+    """Values made halves first, page by page, against 64 bits: the edges of what
+    a half can hold, requests and pages that have no halves, tiles in any order."""
+    dtype, lens, first = torch.bfloat16, [290, 133, 200], [0, 130, 75]
+    mask = {"size": window, "keep_first": keep} if window else None
+    data, bounds = [], []
+    for i, n in enumerate(lens):
+        q, k, v, _ = _attn_case(H, G, D, E, window, keep, n, dtype, seed=40 + n)
+        v = _halves_values(v, kind)
+        qkv = [t.double().view(n, -1, s) for t, s in ((q, D), (k, D), (v, E))]
+        want = vo.windowed_attention(*qkv, 0.11, mask).reshape(n, H * E)
+        size = vo.windowed_attention(*qkv[:2], qkv[2].abs(), 0.11, mask)
+        data.append((q, k, v, want))
+        # the result is rounded to bf16; weights and sums have 32 bits
+        bounds.append(2.0 ** -8 * want.abs() +
+                      2.0 ** -20 * size.reshape(n, H * E))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    c = Paged(lens, G, D, E, dtype)
+    rows = [(r, p) for r, n in enumerate(lens) for p in range(n)]
+    seq, pos = i32([r for r, _ in rows]), i32([p for _, p in rows])
+    _, k, v = (torch.cat([d[i] for d in data]).cuda() for i in range(3))
+    sv.kv_append(k, v, c.kc, c.vc, pos, seq, c.bt)
+    q = torch.cat([d[0][a:] for d, a in zip(data, first)]).cuda()
+    tiles, at = [], 0
+    for r, (n, a) in enumerate(zip(lens, first)):
+        for p in range(a, n, 128):
+            tiles.append((r, at + p - a, min(128, n - p), p))
+        at += n - a
+    monkeypatch.setattr(sv, "value_halves", lambda *a: True)
+    for portions, max_keys, order in ((3, 290, 1), (2, 290, -1), (3, 128, 1)):
+        got = sv.attn_portions(
+            q, k[:q.shape[0]], v[:q.shape[0]], c.kc, c.vc, pos, seq, c.bt,
+            i32(tiles[::order]), H, 0.11, window, keep, append=False,
+            max_keys=max_keys, portions=portions)
+        at = 0
+        for d, a, bound in zip(data, first, bounds):
+            n = d[3].shape[0] - a
+            err = (got[at:at + n].double().cpu() - d[3][a:]).abs()
+            assert (err <= bound[a:] + 2.0 ** -133).all(), (
+                portions, max_keys, (err / bound[a:]).max())
+            at += n
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_batch_of_unequal_requests(sv, dtype):
     H, G, D, E, window, keep = 6, 3, 48, 32, 50, 7
