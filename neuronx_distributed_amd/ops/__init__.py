@@ -762,10 +762,40 @@ class _FlashAttnFn(torch.autograd.Function):
         return dq, dk, dv, None, None, None
 
 
+@functools.lru_cache(maxsize=1)
+def _native_flash():
+    """``_FlashAttnFn`` in csrc/host/flash_autograd.cpp; None where it is not built."""
+    from .build import HOST_LIB
+
+    if not os.path.exists(HOST_LIB):
+        return None
+    _require_lib()                    # its kernels
+    torch.ops.load_library(HOST_LIB)
+    return torch.ops.nxd_host.flash_attention.default
+
+
+def _fa_native(q, k, v) -> bool:
+    """May the native function take these: plain bf16 tensors that nobody traces or
+    transforms?  Python's takes the others, and refuses what neither takes."""
+    from .serving import _plain, _unwatched
+
+    bf16 = torch.bfloat16
+    return q.dtype == k.dtype == v.dtype == bf16 and q.is_cuda and k.is_cuda and \
+        v.is_cuda and q.dim() == k.dim() == v.dim() == 4 and \
+        q.shape[3] == k.shape[3] == v.shape[3] == 128 and \
+        _plain(q) and _plain(k) and _plain(v) and _unwatched()
+
+
 def flash_attn(q, k, v, causal=True, softmax_scale=None, window=0):
     """q (B,Hq,S,D=128), k/v (B,Hkv,S,D) bf16 on GPU.  window > 0:
     sliding-window causal (Mistral), fwd AND bwd on the MFMA kernels."""
     scale = softmax_scale or 1.0 / math.sqrt(q.shape[-1])
+    native = _native_flash()
+    if native is not None and _fa_native(q, k, v):
+        B, Hq, S, _ = q.shape
+        window = int(window or 0)
+        return native(q, k, v, bool(causal), scale, window,
+                      _fa_dkv_heads(B, Hq, k.shape[1], S, bool(causal), window))
     return _FlashAttnFn.apply(q, k, v, causal, scale, window)
 
 

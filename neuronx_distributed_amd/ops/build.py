@@ -5,12 +5,14 @@ device code compiled with ``--offload-arch=gfx950`` and linked into shared
 libraries loaded via ctypes.  Built IN-TREE so the .so files travel with
 the source tree.
 
-Two libraries, so that a serving process compiles only what it runs:
+Libraries, so that a serving process compiles only what it runs:
 
 * ``libnxd_ops.so``      every ``csrc/*.hip`` — training kernels and the
                          batch-synchronous inference kernels,
 * ``libnxd_serving.so``  every ``csrc/serving/*.hip`` — the ragged-batch
-                         kernels of the serving engine.
+                         kernels of the serving engine,
+* ``libnxd_host.so``     ``csrc/host/*.cpp`` — autograd functions in C++, which call
+                         the kernels of ``libnxd_ops.so`` (host code, by g++).
 """
 
 import os
@@ -22,6 +24,7 @@ _THIS = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_THIS, "csrc")
 LIB = os.path.join(_THIS, "libnxd_ops.so")
 SERVING_LIB = os.path.join(_THIS, "libnxd_serving.so")
+HOST_LIB = os.path.join(_THIS, "libnxd_host.so")
 
 GROUPS = {
     "ops": (CSRC, LIB),
@@ -102,9 +105,38 @@ def build_group(group: str, force: bool = False, verbose: bool = True) -> str:
     return lib
 
 
+def build_host(force: bool = False, verbose: bool = True) -> str:
+    """Compile the host library against torch; needs ``libnxd_ops.so``."""
+    sources = _listed(os.path.join(CSRC, "host"), ".cpp")
+    if not force and os.path.exists(HOST_LIB) and \
+            all(os.path.getmtime(s) <= os.path.getmtime(HOST_LIB) for s in sources):
+        return HOST_LIB
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    tmp = f"{HOST_LIB}.{os.getpid()}"
+    include = [os.path.join(root, "include"),
+               os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")]
+    try:
+        _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
+              "-DUSE_ROCM=1",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+              *(f"-I{i}" for i in include), *sources, "-o", tmp,
+              f"-L{_THIS}", "-l:" + os.path.basename(LIB),
+              f"-L{os.path.join(root, 'lib')}", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+              "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], verbose)
+        os.replace(tmp, HOST_LIB)
+    finally:
+        if os.path.exists(tmp):
+            os.unlink(tmp)
+    return HOST_LIB
+
+
 def build(force: bool = False, verbose: bool = True) -> str:
     for group in GROUPS:
         build_group(group, force, verbose)
+    build_host(force, verbose)
     return LIB
 
 

@@ -720,6 +720,71 @@ def test_flash_attn_heads_go_to_their_xcd(Hq, Hkv):
         assert ((a.float() - b).norm(dim=(2, 3)) <= bound).all(), name
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,causal,window,layout", [
+    (1, 4, 4, 1, True, 0, "bshd"), (2, 8, 2, 193, True, 0, "bshd"),
+    (2, 6, 2, 300, True, 70, "bhsd"), (1, 4, 1, 129, False, 0, "bhsd"),
+    (1, 4, 2, 140, True, 0, "odd"), (1, 4, 2, 140, True, 0, "between")])
+def test_native_flash_attn_is_pythons(monkeypatch, B, Hq, Hkv, S, causal, window,
+                                      layout):
+    """The native autograd function and Python's: the same bits and strides, with
+    saved tensors that a hook takes through the host."""
+    torch.manual_seed(S)
+    assert ops._native_flash() is not None
+
+    def make(h):
+        if layout == "bshd":
+            t = torch.randn(B, S, h, 128, device="cuda").bfloat16().transpose(1, 2)
+        elif layout == "odd":              # rows of 129 elements
+            t = torch.randn(B, h, S, 129, device="cuda").bfloat16()[..., :128]
+        elif layout == "between":          # rows that start between two words
+            t = torch.randn(B * h * S * 128 + 3, device="cuda").bfloat16()[3:]
+            t = t.view(B, h, S, 128)
+        else:
+            t = torch.randn(B, h, S, 128, device="cuda").bfloat16()
+        return t.detach().requires_grad_(True)
+
+    q, k, v, dy = make(Hq), make(Hkv), make(Hkv), make(Hq).detach()
+    moved, got = [], []
+
+    def pack(t):
+        moved.append(t.shape)
+        return t.cpu()
+
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(ops, "_native_flash", lambda: None)
+        with torch.no_grad():
+            plain = ops.flash_attn(q, k, v, causal, None, window)
+        out = ops.flash_attn(q, k, v, causal, None, window)
+        grads = torch.autograd.grad(out, (q, k, v), dy)
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+            again = ops.flash_attn(q, k, v, causal, None, window)
+        hooked = torch.autograd.grad(again, (q, k, v), dy)
+        for a, b in zip(grads, hooked):
+            assert torch.equal(a, b)
+        got.append((plain, out.detach(), *grads))
+    assert len(moved) == 10
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and a.stride() == b.stride()
+
+
+def test_native_flash_attn_leaves_others_to_python():
+    q = torch.randn(1, 2, 64, 128, device="cuda").bfloat16()
+
+    class Seen(torch.Tensor):
+        pass
+
+    assert ops._fa_native(q, q, q)
+    for t in (q.float(), q[..., :64], q[0], q.as_subclass(Seen)):
+        assert not ops._fa_native(t, t, t) and not ops._fa_native(q, t, q)
+    with torch.autograd.forward_ad.dual_level():
+        assert not ops._fa_native(q, q, q)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not ops._fa_native(q, q, q)
+    with pytest.raises(AssertionError):
+        ops.flash_attn(q.float(), q.float(), q.float())
+
+
 def test_add_rmsnorm_train_matches_unfused_autograd():
     """Training fused add+RMSNorm (fwd + the dpass-folding backward) vs
     the unfused bf16 add -> ops.rmsnorm chain: forward outputs equal and
