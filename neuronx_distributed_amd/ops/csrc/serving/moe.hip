@@ -312,7 +312,10 @@ __device__ __forceinline__ float glu(const MoeGemmArgs& a, float g, float u) {
 // the weight rows of a tile alternate 32 gate, 32 up, so a lane holds both of
 // a column.
 // slot0, rows: the tile's; tn: its columns
-template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool AHEAD>
+// PAGED (DMA, top 1): slot s is row s % 64 of page order[s / 64], pages of 64 rows may
+// lie anywhere; slot0 and rows are whole pages.
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool AHEAD,
+          bool PAGED = false>
 __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
                                          int rows, int tn, short* xs0,
                                          short* xs1, short* ws0, short* ws1,
@@ -338,10 +341,17 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   const short* pw[DMA ? 1 : LW];
   int ox[LX], ow[LW];
   const short* const bx =
-      (const short*)a.x + (a.top ? 0 : (long)slot0 * a.xst);
+      (const short*)a.x + (PAGED || a.top ? 0 : (long)slot0 * a.xst);
   const short* const bw = (const short*)a.w + (long)e * (GLU ? 2 * N : N) * K;
+  int page[PAGED ? LX : 1];                // a wave's load is 8 rows of one page
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
+    if (PAGED) {
+      const int r = slot0 + min(i * (NT / 8) + wid * 8, rows - 8);
+      page[PAGED ? i : 0] = __builtin_amdgcn_readfirstlane(a.order[r / 64]);
+      ox[i] = ((r % 64 + (lane >> 3)) * (int)a.xst + kc) * 2;
+      continue;
+    }
     const int r = min((i * NT + tid) / 8, rows - 1);
     const int row = a.top ? a.order[slot0 + r] / a.top : r;
     if (DMA) ox[i] = (row * (int)a.xst + kc) * 2;
@@ -362,7 +372,8 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   auto issue_x = [&](int k0, short* xs) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < LX; ++i)
-      words_to_lds(bx, ox[i], (char*)(xs + (i * NT + wid * 64) * 8), k0 * 2);
+      words_to_lds(PAGED ? bx + page[PAGED ? i : 0] * (64 * a.xst) : bx, ox[i],
+                   (char*)(xs + (i * NT + wid * 64) * 8), k0 * 2);
   };
   auto issue_w = [&](int k0, short* ws) __attribute__((always_inline)) {
 #pragma unroll
@@ -485,7 +496,7 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
   for (int m = 0; m < CM; ++m) {
     const int r = wm + 32 * m + col;
     if (r >= rows) continue;
-    const long orow = a.top ? slot0 + r : a.order[slot0 + r];
+    const long orow = PAGED || a.top ? slot0 + r : a.order[slot0 + r];
     short* dst = (short*)a.out + orow * N;
 #pragma unroll
     for (int n = 0; n < CN; n += GLU ? 2 : 1)
@@ -510,9 +521,10 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
 // without one, are computed in halves of the slots, or quarters, by all of them
 // (36 tiles of 4096 x 14336, 576 workgroups on 256 CUs: 966 us, in whole tiles
 // 1128).
-template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL>
-__global__ void __launch_bounds__(BM / WM * BN / WN * 64)
-moe_tiles_kernel(MoeGemmArgs a) {
+// PAGED: all rows are one expert's, `rows` of them.
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL,
+          bool PAGED = false>
+__device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   constexpr int GROUP = 8;
   constexpr int NOUT = GLU ? BN / 2 : BN;
   // apart by name, so that a read of one buffer need not wait for the words
@@ -529,7 +541,7 @@ moe_tiles_kernel(MoeGemmArgs a) {
   // that have rows (all places in the list, the last ones empty: gates of 36
   // tiles of 28672 x 4096 2222 us, now 1789)
   const int ntn = (a.N + NOUT - 1) / NOUT;
-  const int live = a.tiles[3], total = live * ntn;
+  const int live = PAGED ? (a.rows + BM - 1) / BM : a.tiles[3], total = live * ntn;
   const int tail = total % 256;
   const int split = !TAIL || tail == 0 || tail > 128 ? 1 : tail > 64 ? 2 : 4;
   const int whole = split > 1 ? total - tail : total;
@@ -546,24 +558,32 @@ moe_tiles_kernel(MoeGemmArgs a) {
   const int gm = min(GROUP, live - g0);
   const int in = id - g0 * ntn;
   const int tn = in / gm;
-  const int* tl = a.tiles + 4L * (g0 + in % gm);
-  const int e = tl[0], slot0 = tl[1], rows = tl[2];
+  const int tile = g0 + in % gm;
+  const int* tl = PAGED ? nullptr : a.tiles + 4L * tile;
+  const int e = PAGED ? 0 : tl[0], slot0 = PAGED ? tile * BM : tl[1];
+  const int rows = PAGED ? min(BM, a.rows - slot0) : tl[2];
   if (!TAIL || id < whole) {
-    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD>(a, e, slot0, rows, tn, xs0, xs1,
-                                              ws0, ws1, ws2);
+    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD, PAGED>(a, e, slot0, rows, tn, xs0, xs1,
+                                                     ws0, ws1, ws2);
     return;
   }
   if constexpr (TAIL) {
     const int s = piece % 2 * (BM / 2);
     if (s >= rows) return;
     if (split == 2)
-      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD>(
+      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD, PAGED>(
           a, e, slot0 + s, min(rows - s, BM / 2), tn, xs0, xs1, ws0, ws1, ws2);
     else if ((tn * 2 + piece / 2) * (NOUT / 2) < a.N)
-      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD>(
+      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD, PAGED>(
           a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, xs0, xs1,
           ws0, ws1, ws2);
   }
+}
+
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL>
+__global__ void __launch_bounds__(BM / WM * BN / WN * 64)
+moe_tiles_kernel(MoeGemmArgs a) {
+  moe_tiles<BM, BN, WM, WN, GLU, DMA, TAIL>(a);
 }
 
 // -- a few rows per expert: stream the weights --------------------------------
@@ -1116,5 +1136,64 @@ extern "C" int sv_moe_gemm(const MoeGemmArgs* a, int how, int gated, int f32,
     else     { if (gated) PK(short, true); else PK(short, false); }
 #undef PK
   }
+  return (int)hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Keys and values of a latent cache: rows of `pages` (R latents, P shared columns)
+// times w (N, R), page after page, and their shared columns beside them.  The tiles
+// above, with rows that are read where they lie, of 128 x 128 with two workgroups a CU,
+// since R is short: one works while the other's first words come and its results go.
+// As a copy of the pages and a library product it took, us, then and now (R 512, within
+// a call): N 8192: 128 rows 13.2 | 8.6, 704 20.2 | 16.0; N 4096: 1600 rows 25.8 | 17.4,
+// 6656 72.8 | 49.2.  (5120 x 8192 over and over: 70.7 | 63.1, in 256 x 256, one workgroup a
+// CU, 77.5, in 128 x 256 67.5; but within a call 63.1 | 70.4, and so left to the library.)
+// 64 x 128
+// is for what does not fill the chip otherwise.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(BM / WM * BN / WN * 64)
+latent_expand_kernel(MoeGemmArgs a, uint4v* rot, int P, int tiles) {
+  constexpr int NT = BM / WM * BN / WN * 64;
+  if ((int)blockIdx.x < tiles) {
+    moe_tiles<BM, BN, WM, WN, false, true, false, true>(a);
+    return;
+  }
+  const int page = blockIdx.x - tiles, words = P / 8;    // its shared columns
+  const short* src = (const short*)a.x + a.order[page] * (64 * a.xst) + a.K;
+  for (int i = threadIdx.x; i < 64 * words; i += NT)
+    rot[(long)page * 64 * words + i] =
+        *(const uint4v*)(src + i / words * a.xst + i % words * 8);
+}
+
+// R a multiple of 64, P and N of 8; rot [n][64][P]
+extern "C" int sv_latent_expand(const void* cache, const int* pages, int n, const void* w,
+                                void* out, void* rot, int R, int P, int N,
+                                hipStream_t stream) {
+  if (n <= 0) return 0;
+  if (R % 64 || R <= 0 || P % 8 || P < 0 || N % 8 || N <= 0 || (long)N * R >= 1L << 30)
+    return 1;
+  MoeGemmArgs a = {};
+  a.x = cache;
+  a.xst = R + P;
+  a.w = w;
+  a.out = out;
+  a.order = pages;
+  a.top = 1;
+  a.N = N;
+  a.K = R;
+  a.rows = n * 64;
+#define LE(BM, BN, WM, WN)                                                          \
+  do {                                                                              \
+    const long tiles = (a.rows + BM - 1L) / BM * ((N + BN - 1) / BN);               \
+    latent_expand_kernel<BM, BN, WM, WN>                                            \
+        <<<tiles + (P ? n : 0), BM / WM * BN / WN * 64, 0, stream>>>(               \
+            a, (uint4v*)rot, P, (int)tiles);                                        \
+  } while (0)
+  // as many workgroups as are resident (N 8192: 640 rows 13.6 | 14.0 in the larger
+  // tiles, 896 17.8 | 15.1; N 2048: 2688 12.9 | 13.9, 3200 17.1 | 14.1)
+  if (n * ((N + 127L) / 128) <= 768) LE(64, 128, 64, 32);
+  else LE(128, 128, 64, 64);
+#undef LE
   return (int)hipGetLastError();
 }

@@ -1785,6 +1785,29 @@ def latent_tiles_supported(q, gate, dim, vdim, rank, shared) -> bool:
             and (gate is None or _aligned((), gate)))
 
 
+def expand_rule(rows: int, N: int, R: int) -> bool:
+    """Are keys and values (rows, N) of a latent cache made by a kernel that reads its
+    pages where they lie, not by a copy and a library product?  Within a call, R 512, it
+    is 0.97 to 1.9 times as fast (us, copy and product | kernel: 128 x 8192 13.2 | 8.6,
+    1600 x 4096 25.8 | 17.4, 1152 x 8192 22.9 | 22.2, 6656 x 4096 72.8 | 49.2) but where
+    the library's tiles of 256 x 256 fill the CUs, or nearly (4096 x 4096 28.1 | 29.9,
+    1792 x 8192 25.0 | 25.8), and for large products (5184 x 8192 63.1 | 70.4; 10048 x
+    4096 79.8 | 75.2, 12800 76.5 | 82.8)."""
+    tiles = -(-rows // 256) * -(-N // 256)
+    whole = tiles >= 216 and not 0 < tiles % 256 < 216
+    return R % 64 == 0 and N * R < 1 << 30 and rows * N <= 28_000_000 and not whole
+
+
+def _expandable(cache, expand, pages, R: int, P: int) -> bool:
+    return cache.is_contiguous() and expand.is_contiguous() and \
+        pages.is_contiguous() and pages.dtype == torch.int32 and \
+        cache.dtype == expand.dtype == torch.bfloat16 and \
+        cache.shape[1:] == (PAGE_SIZE, R + P) and expand.shape[1] == R and \
+        cache.device == expand.device == pages.device and \
+        not (expand.shape[0] | P) & 7 and \
+        not (cache.data_ptr() | expand.data_ptr()) & 15
+
+
 def latent_portions(q, gate, cache, w: LatentWeights, batch,
                     spans: KeySpans, heads: int, dim: int, vdim: int,
                     scale: float, window: int, out):
@@ -1793,12 +1816,22 @@ def latent_portions(q, gate, cache, w: LatentWeights, batch,
     R = w.norm.shape[0]
     P = cache.shape[2] - R
     n = spans.pages.shape[0]
-    ws = torch.empty(n * PAGE_SIZE, R + P, dtype=q.dtype, device=q.device)
-    _check(library().sv_latent_gather(
-        ctypes.c_void_p(_p(cache)), ctypes.c_void_p(_p(ws)),
-        ctypes.c_void_p(_p(spans.pages)), n,
-        PAGE_SIZE * (R + P) * q.element_size(), _stream()), "latent_gather")
-    kv = torch.mm(ws[:, :R], w.expand.t())
+    N = w.expand.shape[0]
+    if n and P and expand_rule(n * PAGE_SIZE, N, R) and \
+            _expandable(cache, w.expand, spans.pages, R, P):
+        kv = torch.empty(n * PAGE_SIZE, N, dtype=q.dtype, device=q.device)
+        ws = torch.empty(n * PAGE_SIZE, P, dtype=q.dtype, device=q.device)
+        _check(library().sv_latent_expand(
+            ctypes.c_void_p(_p(cache)), ctypes.c_void_p(_p(spans.pages)), n,
+            ctypes.c_void_p(_p(w.expand)), ctypes.c_void_p(_p(kv)),
+            ctypes.c_void_p(_p(ws)), R, P, N, _stream()), "latent_expand")
+    else:
+        ws = torch.empty(n * PAGE_SIZE, R + P, dtype=q.dtype, device=q.device)
+        _check(library().sv_latent_gather(
+            ctypes.c_void_p(_p(cache)), ctypes.c_void_p(_p(ws)),
+            ctypes.c_void_p(_p(spans.pages)), n,
+            PAGE_SIZE * (R + P) * q.element_size(), _stream()), "latent_gather")
+        kv = torch.mm(ws[:, :R], w.expand.t())
     return expanded_attention(q, gate, kv, ws, batch.tiles, spans, heads,
                               dim, vdim, scale, window, out, w.sink)
 

@@ -332,6 +332,55 @@ def test_latent_window_edges_show(sv, window, dtype):
             _close(out, want[a:a + n], dtype, 3.0, (window, spot, a, n))
 
 
+@pytest.mark.parametrize("n,N,R,P,pages", [
+    (1, 8, 64, 8, 1), (2, 200, 128, 16, 5), (3, 128, 512, 64, 9), (13, 8200, 64, 64, 20),
+    (25, 4096, 128, 8, 30), (7, 1032, 512, 64, 29500)])
+def test_pages_are_expanded_where_they_lie(sv, n, N, R, P, pages):
+    """Both sizes of tiles, columns and pages that are no whole ones, and pages more
+    than 2 GB apart."""
+    g = torch.Generator("cuda")
+    g.manual_seed(n + N)
+    cache = torch.empty(pages, 64, R + P, dtype=torch.bfloat16, device="cuda")
+    at = torch.randperm(pages, generator=g, device="cuda")[:n]
+    at[-1] = pages - 1 if n > 1 and pages - 1 not in at[:-1].tolist() else at[-1]
+    rows = torch.randn(n, 64, R + P, generator=g, device="cuda").bfloat16()
+    cache[at] = rows
+    w = torch.randn(N, R, generator=g, device="cuda").bfloat16()
+    assert sv.expand_rule(n * 64, N, R)
+    at = at.int()
+    assert sv._expandable(cache, w, at, R, P)
+    kv = torch.full((n * 64 + 1, N), 7.0, dtype=w.dtype, device="cuda")
+    rot = torch.full((n * 64 + 1, P), 7.0, dtype=w.dtype, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert not sv.library().sv_latent_expand(p(cache), p(at), n, p(w), p(kv), p(rot), R, P,
+                                             N, sv._stream())
+    x = rows.reshape(-1, R + P).double()
+    want, size = x[:, :R] @ w.double().t(), x[:, :R].abs() @ w.double().abs().t()
+    # rounded to bf16 once; R sums of 32 bits
+    assert ((kv[:-1].double() - want).abs() <=
+            2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all()
+    assert torch.equal(rot[:-1], rows.reshape(-1, R + P)[:, R:])
+    assert (kv[-1] == 7).all() and (rot[-1] == 7).all()
+
+
+def test_what_is_not_expanded_in_place(sv):
+    """Other layouts and types take the copy and the library's product."""
+    cache = torch.zeros(3, 64, 72, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(16, 64, dtype=torch.bfloat16, device="cuda")
+    pages = torch.zeros(2, dtype=torch.int32, device="cuda")
+    assert sv._expandable(cache, w, pages, 64, 8)
+    far = torch.zeros(16 * 64 + 4, dtype=w.dtype, device="cuda")[4:].view(16, 64)
+    for c, e, p in ((cache, w.t().contiguous().t(), pages), (cache, far, pages),
+                    (cache.float(), w.float(), pages), (cache, w[:12], pages),
+                    (cache, w, pages.long()), (cache[:, :, ::2], w, pages)):
+        assert not sv._expandable(c, e, p, 64, 8)
+    for rows, N, R in ((4096, 4096, 512), (1792, 8192, 512), (5120, 8192, 512),
+                       (64, 128, 96), (64, 1 << 22, 512)):
+        assert not sv.expand_rule(rows, N, R)
+    for rows, N, R in ((64, 128, 64), (3200, 8192, 512), (1536, 16384, 512)):
+        assert sv.expand_rule(rows, N, R)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_rotation_far_out_and_partial(sv, dtype):
     """Angles stay exact at large positions; columns past the rotated ones
