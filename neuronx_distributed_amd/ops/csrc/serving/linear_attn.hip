@@ -396,11 +396,12 @@ struct ChunkArgs {
   short* P;                 // [n_chunks][H][3][E][D] state before the chunk; if
                             //   there is no U [n_chunks][H][E / 32][3][D / 16]
                             //   [64][8]: keys 16 c + 8 hi + 0..7 of column col;
-                            //   or null: nothing is left between chunks (timed, D
-                            //   128, E a multiple of 64, no VT and U)
+                            //   or null: nothing is left between chunks (timed
+                            //   or decayed, D 128, E a multiple of 64, no VT, U)
   float* mst;               // [n_chunks][H] m before the chunk (gated)
   short* VT;                // [n_chunks][H][E][256] V^T, activated; or null
-                            //   (timed, D 64 or 128, E a multiple of 64)
+                            //   (timed, D 64 or 128, or decayed, in one pass;
+                            //   E a multiple of 64)
   short* KA;                // [T][H][D] activated K (decay); two planes of
                             //   rotated K (turned)
   short* QA;                // two planes of rotated Q (turned)
@@ -1669,7 +1670,7 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   }
 }
 
-// ---- timed memories of D = 128, states and outputs in one pass -----------------
+// ---- timed and decayed memories of D = 128, states and outputs in one pass -----
 // One workgroup takes 64 columns of a head through its segment, 64 tokens a piece:
 // nothing but queries, keys, values, gates and results moves.  Three waves of a SIMD
 // do different things, since one alone issues a vector instruction every eight
@@ -1680,9 +1681,8 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
 // the fewest scores also makes the next piece's gates.  Four ask for the next piece's
 // tiles, which come straight into LDS, and write the results of two pieces ago.  One
 // barrier a piece.  Bound by what one wave issues: the states' waves alone take 83 of
-// the 105 us below, where a product of 16 x 16 x 32 takes a lone wave 31 cycles, not
-// 16; the tiles alone take 57, a piece's latency each time.  128 heads of 128 x 64 in
-// us, carried states and outputs in chunks of 256 as above | one pass:
+// the 105 us below; the tiles alone take 57, a piece's latency each time.  128 heads of
+// 128 x 64 in us, carried states and outputs in chunks of 256 as above | one pass:
 //   2 x 2048 tokens 181 | 105      4 x 500 104 | 62     1 x 4096 177 | 158
 //   64 heads: 1500 tokens 60 | 56, 3 x 500 52 | 38, 50 35 | 19 (its one launch)
 // With two waves a SIMD, states and everything else, 2 x 2048 took 130; with four of
@@ -1690,6 +1690,12 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
 constexpr int PASS_D = 128;
 template <int N> struct Count { static constexpr int value = N; };
 
+// DECAY: queries, keys and values pass through registers and silu on their way into
+// LDS, the weights are the same for every piece, and the results are written as they
+// are.  32 heads of 128 x 128 in us, activated copies, states of all chunks at once, a
+// scan and outputs | one pass:
+//   50 tokens 17.7 | 7.1    500 43.6 | 28.4    4 x 500 40.6 | 18.1    3 x 2000 72 | 56
+template <int GATE>
 __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   constexpr int DP = PASS_D, L = 64, ET = 64;
   constexpr int TILE = L * DP * 2, VT = L * ET * 2, PART = ET * L * 4;
@@ -1878,14 +1884,22 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   }
 
   if (wid < 8) {
-    const float skip = bits2f(((const short*)a.skip)[h]);
-    const float ib = bits2f(((const short*)a.ib)[h]);
-    const float rate = -expf(bits2f(((const short*)a.fb)[h]));
-    const float* raw = a.gates + (long)row0 * a.H + h;
+    const float skip = GATE == TIMED ? bits2f(((const short*)a.skip)[h]) : 0.f;
+    const float ib = GATE == TIMED ? bits2f(((const short*)a.ib)[h]) : 0.f;
+    const float rate = GATE == TIMED ? -expf(bits2f(((const short*)a.fb)[h])) : 0.f;
+    const float l2d = GATE == DECAY ? a.log2_decay[h] : 0.f;
+    const float* raw = GATE == TIMED ? a.gates + (long)row0 * a.H + h : nullptr;
     auto load_gate = [&](int i) __attribute__((always_inline)) {
-      return raw[(long)min(L * i + lane, rows - 1) * a.H];
+      return GATE == TIMED ? raw[(long)min(L * i + lane, rows - 1) * a.H] : 0.f;
     };
     auto gates = [&](int i, float g) __attribute__((always_inline)) {
+      if (GATE == DECAY) {               // only what the state needs
+        const int n = min(rows - L * i, L);
+        s_w[(i & 1) * L + lane] =
+            lane < n ? __builtin_amdgcn_exp2f((n - 1 - lane) * l2d) : 0.f;
+        if (lane == 0) s_keep[i & 1] = __builtin_amdgcn_exp2f(n * l2d);
+        return;
+      }
       const float step = L * i + lane < rows ? softplus_f(g + ib) : 0.f;
       float F = rate * step;
 #pragma unroll
@@ -1907,7 +1921,17 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
       constexpr int n = decltype(number)::value, NP = n / 2 + 1;
       f32x4 pv[4];                       // columns 16 et + 4 quad ... of token t
       const int t = 16 * n + col;
-      float inter = 0.f;
+      float inter = GATE == DECAY ? __builtin_amdgcn_exp2f((t + 1) * l2d) : 0.f;
+      // (of keys 4 quad + j of block J, seen from token t)
+      f32x4 weight[GATE == DECAY ? n + 1 : 1];
+      if (GATE == DECAY)
+#pragma unroll
+        for (int J = 0; J <= n; ++J)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int away = max(t - 16 * J - 4 * quad - j, 0);
+            weight[GATE == DECAY ? J : 0][j] = __builtin_amdgcn_exp2f(away * l2d);
+          }
       int at[4];
 #pragma unroll
       for (int et = 0; et < 4; ++et) at[et] = part_at(4 * et + quad, t);
@@ -1928,6 +1952,18 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
           for (int J = 0; J <= n; ++J)
             kf[c][J].u4 = *(const uint4v*)(kb + J * 4096 + (rx ^ (64 * c)));
         }
+        f32x4 acc[2 * NP] = {};
+        if (GATE == DECAY) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int J = 0; J <= n; ++J) acc[J] = mfma16(kf[c][J].bf, qf[c].bf, acc[J]);
+#pragma unroll
+          for (int J = 0; J <= n; ++J) acc[J] *= weight[GATE == DECAY ? J : 0];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (4 * quad + j > col) acc[n][j] = 0.f;
+        } else {
         const float* b = s_b + (i & 1) * L;
         const float bt = b[t];
         const f32x4 bs = *(const f32x4*)(b + 16 * n + 4 * quad);
@@ -1939,7 +1975,6 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
           far[J] = *(const f32x4*)(s_far + (i & 1) * L + 16 * J + 4 * quad);
           from[J] = b[16 * J + 15];
         }
-        f32x4 acc[2 * NP] = {};
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -1952,6 +1987,7 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
           const float w = acc[n][j] * (__expf(bt - bs[j]) * step[j]);
           const int s = 4 * quad + j;
           acc[n][j] = (s > col ? 0.f : w) + (s == col ? skip : 0.f);
+        }
         }
 #pragma unroll
         for (int et = 0; et < 4; ++et) pv[et] = f32x4{};
@@ -2035,11 +2071,43 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           vs, (lds_ptr)(vb + (p * 256 + n * 64) * 16), 16, vo + p * 32 * vst, 0, 0, 0);
   };
+  // the same through registers, asked for two pieces ahead
+  uint4v words[GATE == DECAY ? 10 : 1];
+  auto fetch = [&](int i) __attribute__((always_inline)) {
+    const int end = min(rows - L * i, L) - 1;
+    const auto qs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(qp + (long)L * i * a.qst), 0, end * qst + DP * 2, 0x00027000);
+    const auto ks = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(kp + (long)L * i * a.kst), 0, end * kst + DP * 2, 0x00027000);
+    const auto vs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(vp + (long)L * i * a.vst), 0, end * vst + ET * 2, 0x00027000);
+    auto load = [](__amdgpu_buffer_rsrc_t src, int off) __attribute__((always_inline)) {
+      return __builtin_bit_cast(uint4v,
+                                __builtin_amdgcn_raw_buffer_load_b128(src, off, 0, 0));
+    };
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      words[GATE == DECAY ? p : 0] = load(qs, qo + p * 16 * qst);
+      words[GATE == DECAY ? 4 + p : 0] = load(ks, ko + p * 16 * kst);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      words[GATE == DECAY ? 8 + p : 0] = load(vs, vo + p * 32 * vst);
+  };
+  auto put = [&](char* qb, char* kb, char* vb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < 10; ++p) {
+      char* to = p < 4 ? qb : p < 8 ? kb : vb;
+      *(uint4v*)(to + ((p < 8 ? p % 4 : p - 8) * 256 + ft) * 16) =
+          silu8<true>(words[GATE == DECAY ? p : 0]);
+    }
+  };
   // two rows of 64 columns, 16 bytes a lane
   const int r0 = 16 * n + (lane >> 3) * 2, c8 = lane & 7;
   const long at = (long)h * E + e0 + c8 * 8;
   uint4v z[2], znext[2];
   auto load_z = [&](int i) __attribute__((always_inline)) {
+    if (GATE != TIMED) return;
 #pragma unroll
     for (int y = 0; y < 2; ++y)
       znext[y] = *(const uint4v*)((const short*)a.z + at +
@@ -2055,12 +2123,14 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
         load4((const float*)(part + part_at(2 * c8 + u, r0 + y)), v[y] + 4 * u);
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
-      float g[8];
-      unpack8(z[y], g);
+      if (GATE == TIMED) {
+        float g[8];
+        unpack8(z[y], g);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        w[y][j] = pack_bf16x2(v[y][2 * j] * silu_f(g[2 * j]),
-                              v[y][2 * j + 1] * silu_f(g[2 * j + 1]));
+        for (int j = 0; j < 8; ++j) v[y][j] *= silu_f(g[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[y][j] = pack_bf16x2(v[y][2 * j], v[y][2 * j + 1]);
     }
   };
   auto store = [&](int i) __attribute__((always_inline)) {
@@ -2076,16 +2146,27 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
     asm volatile("" ::: "memory");
   };
   if (pieces) {
-    issue(0, q0, k0, v0);
-    arrive();
+    if (GATE == DECAY) {
+      fetch(0);
+      put(q0, k0, v0);
+      if (pieces > 1) fetch(1);
+    } else {
+      issue(0, q0, k0, v0);
+      arrive();
+    }
   }
   meet();
   const char *part = s_part + PART, *next = s_part + 2 * PART, *after = s_part;
   for (int i = 0; i < pieces; ++i) {
-    if (i + 1 < pieces) issue(i + 1, i & 1 ? q0 : q1, i & 1 ? k0 : k1, i & 1 ? v0 : v1);
+    if (GATE == DECAY) {
+      if (i + 1 < pieces) put(i & 1 ? q0 : q1, i & 1 ? k0 : k1, i & 1 ? v0 : v1);
+      if (i + 2 < pieces) fetch(i + 2);
+    } else if (i + 1 < pieces) {
+      issue(i + 1, i & 1 ? q0 : q1, i & 1 ? k0 : k1, i & 1 ? v0 : v1);
+    }
     if (i) load_z(i - 1);                // for the next turn
     if (i > 1) results(part);            // of two pieces ago
-    arrive();
+    if (GATE != DECAY) arrive();
     if (i > 1) store(i - 2);
     z[0] = znext[0], z[1] = znext[1];
     meet();
@@ -2111,10 +2192,10 @@ template <int DP, int GATE>
 static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
   const MemoryArgs& a = x.a;
   const long ch = (long)x.n_chunks * a.H;
-  if constexpr (GATE == TIMED && DP == PASS_D)
+  if constexpr ((GATE == TIMED || GATE == DECAY) && DP == PASS_D)
     if (!x.P) {
       const int units = a.H * (a.E / 64);
-      memory_pass_kernel<<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
+      memory_pass_kernel<GATE><<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
       return;
     }
   if (!fixed_decay(GATE)) memory_gates_kernel<GATE><<<ch, MC_L, 0, stream>>>(x);
@@ -2158,7 +2239,7 @@ extern "C" int sv_memory_chunks(const ChunkArgs* x, int gating,
       (x->a.rot % 2 || x->a.rot > x->a.D ||
        (x->a.z && (x->a.E > 128 || (x->a.E > 64 && x->a.D > 128)))))
     return 1;
-  if (!x->VT && (gating != TIMED || x->a.E % 64 ||
+  if (!x->VT && ((gating != TIMED && (gating != DECAY || x->P)) || x->a.E % 64 ||
                  (x->a.D != 64 && x->a.D != 128)))
     return 1;
   if (!x->U && x->VT) return 1;

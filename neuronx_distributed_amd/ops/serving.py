@@ -1381,6 +1381,15 @@ def memory_pass(chunks: int, segments: int, columns: int) -> bool:
     return chunks - segments + 1 <= chunks * (columns // 64) / 80 + 2
 
 
+def decay_pass(chunks: int, segments: int, columns: int) -> bool:
+    """The same for a decayed memory.  A chunk of the longest segment takes one pass
+    11.9 us behind 5 for the call; the launches and passes it stands for take 17 to 44
+    up to a chunk or two and 0.08 us more for every 64 columns of a chunk.  126 random
+    calls of 2 to 128 heads, one pass over those: 0.57 in the mean, none slower; with 1
+    chunk for the 2.5 0.58, with 4 the same and one call 1.45."""
+    return chunks - segments + 1 <= chunks * (columns // 64) / 100 + 2.5
+
+
 def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
                chunks: Optional[torch.Tensor] = None,
                chunk_first: Optional[torch.Tensor] = None,
@@ -1462,19 +1471,22 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         nc = chunks.shape[0]
         assert chunk_first.shape[0] == seg.shape[0] + 1
         f32 = dict(dtype=torch.float32, device=q.device)
-        tiled = timed and D in (64, 128) and E % 64 == 0 and \
+        whole = D in (64, 128) and E % 64 == 0 and \
             max(t.stride(0) for t in strided) < 1 << 22
-        once = tiled and D == 128 and memory_pass(nc, seg.shape[0], heads * E)
+        tiled, decayed = timed and whole, isinstance(gate, DecayGate)
+        once = whole and D == 128 and (
+            timed and memory_pass(nc, seg.shape[0], heads * E) or
+            decayed and decay_pass(nc, seg.shape[0], heads * E))
         U = None if once or tiled and D == 64 and memory_carries(
             nc, seg.shape[0], heads * D * E) \
             else torch.empty(nc, heads, E, D, **f32)
         P = None if once else torch.empty(nc, heads, 3, E, D,
                                           dtype=torch.bfloat16, device=q.device)
-        VT = None if tiled else \
+        VT = None if tiled or once else \
             torch.empty(nc, heads, E, CHUNK, dtype=torch.bfloat16,
                         device=q.device)
         KA = torch.empty(T, heads * D, dtype=q.dtype, device=q.device) \
-            if isinstance(gate, DecayGate) else None
+            if decayed and not once else None
         if turned:
             KA, QA = torch.empty(2, 2, T, heads * D, dtype=q.dtype,
                                  device=q.device)

@@ -453,6 +453,52 @@ def test_gated_memory(sv, H, D, E, i_scale, f_shift, dtype):
             assert err < 2e-4, err
 
 
+@pytest.mark.parametrize("H,E", [(3, 64), (2, 128), (5, 192)])
+@pytest.mark.parametrize("far", [False, True])
+def test_decayed_memory_in_one_pass(sv, monkeypatch, H, E, far):
+    """Segments that end at, before and behind the 16 tokens of a wave and the 64 of
+    a piece, from empty and from filled slots, of adjacent and of distant rows;
+    against the oracle, and against chunks."""
+    D, bf = 128, torch.bfloat16
+    lens, more = [1, 15, 17, 63, 64, 65, 128, 130, 193, 449], [70, 1, 300, 64, 2, 33,
+                                                              65, 192, 5, 16]
+    decay = [0.97, 0.0, 1.0, 0.6, 0.999][:H]
+    gate = sv.decay_gate(decay, "cuda")
+    assert sv.decay_pass(10, 10, H * E)
+    cases = [_mem_inputs(H, D, E, a + b, bf, seed=40 + i)[3]
+             for i, (a, b) in enumerate(zip(lens, more))]
+    sizes = H * D, H * D, H * E
+    got = {}
+    for once in (True, False):
+        monkeypatch.setattr(sv, "decay_pass", lambda *a: once)
+        S = torch.full((10, H, D, E), 7.0).cuda()
+        out = []
+        for at, n in (([0] * 10, lens), (lens, more)):
+            rows = torch.cat([p[a:a + k, :sum(sizes)] for p, a, k in zip(cases, at, n)])
+            # among elements that nothing may see, 748 of the rows 2 MB apart
+            pitch = 1 << 20 if far and at[0] else rows.shape[1] + 8
+            wide = torch.full((len(rows) + 1, pitch), float("nan"), dtype=bf,
+                              device="cuda")
+            x = wide[:len(rows), :rows.shape[1]]
+            x.copy_(rows)
+            seg, *tab = _tables(sv, [(9 - i, sum(n[:i]), k, a) for i, (a, k) in
+                                     enumerate(zip(at, n))], True)
+            out.append(sv.memory_mix(*x.split(sizes, dim=1), gate, S, None, None, seg,
+                                     H, *tab).split(n))
+        got[once] = [torch.cat([o[i] for o in out]) for i in range(10)], S
+    silu = lambda t, s: vo.silu(t.double()).to(bf).double().view(len(t), H, s)
+    for i, p in enumerate(cases):
+        q, k, v = p[:, :sum(sizes)].split(sizes, dim=1)
+        want, S_want = vo.decayed_memory(silu(q, D), silu(k, D), silu(v, E),
+                                         torch.tensor(decay).double())
+        want = want.reshape(len(p), H * E)
+        _close(got[True][0][i], want, bf, 2.0, i)
+        off = [(got[way][0][i].cpu().double() - want).norm() for way in got]
+        assert off[0] <= 1.05 * off[1] + 1e-6 * want.norm()
+        err = [(got[way][1][9 - i].cpu().double() - S_want).norm() for way in got]
+        assert err[0] <= 1.05 * err[1] + 1e-6 * S_want.norm()
+
+
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_memory_batch_and_slots(sv, dtype, gated):
