@@ -417,13 +417,16 @@ __host__ __device__ constexpr int qk_planes(int gate) {
   return gate == TURNED ? 2 : 1;
 }
 
-// split a pair of floats into three planes of packed bf16
+// split a pair of floats into three planes of packed bf16, 8 bits each: cut off, not
+// rounded, since three hold all 24.  (Masks are cheaper than the shift and the packed
+// conversion: one pass of 2731 and 1365 tokens 103.8 -> 102.9 us, of 1293 decayed ones
+// 65.9 -> 65.0.)
 __device__ __forceinline__ void split3(float x, float y, uint* w) {
 #pragma unroll
   for (int z = 0; z < 3; ++z) {
-    w[z] = pack_bf16x2(x, y);
-    x -= __uint_as_float(w[z] << 16);
-    y -= __uint_as_float(w[z] & 0xffff0000u);
+    w[z] = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
+    x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+    y -= __uint_as_float(__float_as_uint(y) & 0xffff0000u);
   }
 }
 
@@ -1680,13 +1683,16 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
 // within the piece, 16 tokens each, and add their products a piece later; the one with
 // the fewest scores also makes the next piece's gates.  Four ask for the next piece's
 // tiles, which come straight into LDS, and write the results of two pieces ago.  One
-// barrier a piece.  Bound by what one wave issues: the states' waves alone take 83 of
-// the 105 us below; the tiles alone take 57, a piece's latency each time.  128 heads of
-// 128 x 64 in us, carried states and outputs in chunks of 256 as above | one pass:
+// barrier a piece.  Bound by what a SIMD issues: up to 136 products of 16 cycles and
+// 720 vector instructions of 2.4 to 5, which products hardly hide, are 4200 of a
+// piece's 4770 cycles; the tiles alone take half of them, a piece's latency each time.
+// 128 heads of 128 x 64 in us, carried states and outputs in chunks of 256 as above |
+// one pass:
 //   2 x 2048 tokens 181 | 105      4 x 500 104 | 62     1 x 4096 177 | 158
 //   64 heads: 1500 tokens 60 | 56, 3 x 500 52 | 38, 50 35 | 19 (its one launch)
 // With two waves a SIMD, states and everything else, 2 x 2048 took 130; with four of
-// 128 registers 133; the gates beside the results' waves 116.
+// 128 registers 133, and with two of them for the halves of the state 120; the gates
+// beside the results' waves 116.
 constexpr int PASS_D = 128;
 template <int N> struct Count { static constexpr int value = N; };
 
