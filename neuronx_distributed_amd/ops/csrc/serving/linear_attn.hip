@@ -70,12 +70,16 @@ __device__ __forceinline__ float softplus_f(float x) {
   return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
 }
 
+__device__ __forceinline__ void log_gates(const MemoryArgs& a, float gi, float gf,
+                                          float ib, float fb, float& i, float& f) {
+  i = a.gate_cap * tanhf((gi + ib) / a.gate_cap);
+  f = log_sigmoid_f(a.gate_cap * tanhf((gf + fb) / a.gate_cap));
+}
 __device__ __forceinline__ void log_gates(const MemoryArgs& a, long row,
                                           int h, float ib, float fb,
                                           float& i, float& f) {
   const float* g = a.gates + row * 2 * a.H;
-  i = a.gate_cap * tanhf((g[h] + ib) / a.gate_cap);
-  f = log_sigmoid_f(a.gate_cap * tanhf((g[a.H + h] + fb) / a.gate_cap));
+  log_gates(a, g[h], g[a.H + h], ib, fb, i, f);
 }
 
 // ---------------------------------------------------------------------------
@@ -396,12 +400,12 @@ struct ChunkArgs {
   short* P;                 // [n_chunks][H][3][E][D] state before the chunk; if
                             //   there is no U [n_chunks][H][E / 32][3][D / 16]
                             //   [64][8]: keys 16 c + 8 hi + 0..7 of column col;
-                            //   or null: nothing is left between chunks (timed
-                            //   or decayed, D 128, E a multiple of 64, no VT, U)
+                            //   or null: nothing is left between chunks (not
+                            //   turned, D 128, E a multiple of 64, no VT and U)
   float* mst;               // [n_chunks][H] m before the chunk (gated)
   short* VT;                // [n_chunks][H][E][256] V^T, activated; or null
-                            //   (timed, D 64 or 128, or decayed, in one pass;
-                            //   E a multiple of 64)
+                            //   (timed, D 64 or 128, or not turned and no P; E a
+                            //   multiple of 64)
   short* KA;                // [T][H][D] activated K (decay); two planes of
                             //   rotated K (turned)
   short* QA;                // two planes of rotated Q (turned)
@@ -1682,7 +1686,7 @@ __global__ void __launch_bounds__(256, 3) memory_timed_kernel(ChunkArgs x) {
   }
 }
 
-// ---- timed and decayed memories of D = 128, states and outputs in one pass -----
+// ---- memories of D = 128, states and outputs in one pass (not turned) -----------
 // One workgroup takes 64 columns of a head through its segment, 64 tokens a piece:
 // nothing but queries, keys, values, gates and results moves.  Three waves of a SIMD
 // do different things, since one alone issues a vector instruction every eight
@@ -1710,6 +1714,11 @@ template <int N> struct Count { static constexpr int value = N; };
 // are.  32 heads of 128 x 128 in us, activated copies, states of all chunks at once, a
 // scan and outputs | one pass:
 //   50 tokens 17.7 | 7.1    500 43.6 | 28.4    4 x 500 40.6 | 18.1    3 x 2000 72 | 56
+// GATED: the waves that hold the state carry 32 keys of the normaliser each, the same
+// in 16 columns, and leave its planes for the scores' waves, which multiply them by the
+// queries.  Exponents are summed from the piece's end and with the running maxima taken
+// from each other first, which halves the state's error.  16 heads of 128 x 256:
+//   50 tokens 21.9 | 7.5    500 49.8 | 25.9    4 x 500 48.0 | 17.4    3 x 2000 75 | 50
 template <int GATE>
 __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   constexpr int DP = PASS_D, L = 64, ET = 64;
@@ -1722,10 +1731,15 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   // the columns
   __shared__ __attribute__((aligned(16))) char s_part[3 * PART];
   // log forgets and steps; what is left of a token at the end of its 16, and of the
-  // piece; what a piece leaves of the state
+  // piece; what a piece leaves of the state.  GATED: the parts of a weight's exponent
+  // that are the query's and the key's, and what is left of the state at a token
   __shared__ __attribute__((aligned(16))) float s_b[2 * L], s_i[2 * L], s_far[2 * L],
       s_w[2 * L];
   __shared__ float s_keep[2];
+  // GATED: e^-m, and in three planes the weights and the normaliser before the piece
+  __shared__ float s_em[GATE == GATED ? 2 * L : 1];
+  __shared__ __attribute__((aligned(16))) short s_wp[GATE == GATED ? 2 * 3 * L : 8],
+      s_np[GATE == GATED ? 2 * 3 * DP : 8];
   const MemoryArgs& a = x.a;
   const int E = a.E;
   // heads that share keys are on one XCD
@@ -1748,7 +1762,7 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   // transposing reads: 16 lanes turn 4 tokens by 16 columns; tokens 32 c + 16 u + 4
   // quad ... of columns 16 n ... are at (kx ^ 32 n) + (32 c + 16 u) rows
   const int turn_row = 4 * quad + (col >> 2), turn_slot = col >> 1 & 1;
-  const int kx = turn_row * 256 + (row_turn(turn_row) ^ turn_slot) * 16 + (col & 1) * 8;
+  const int kx0 = turn_row * 256 + (row_turn(turn_row) ^ turn_slot) * 16 + (col & 1) * 8;
   const int vx = turn_row * 128 + (value_turn<8>(turn_row) ^ turn_slot) * 16 +
                  (col & 1) * 8;
   union Turned { tr4 t[2]; bf16x8 bf; uint u[4]; };
@@ -1765,16 +1779,42 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
   };
 
   if (wid < 4) {
-    float* Sp = a.S + ((long)a.seg[4 * sg] * a.H + h) * DP * E +
-                (long)(4 * quad) * E + e0 + 16 * wid + col;
-    f32x4 S[8] = {};                     // keys 16 d + 4 quad ... of column col
+    const long head = (long)a.seg[4 * sg] * a.H + h;
+    float* Sp = a.S + head * DP * E + (long)(4 * quad) * E + e0 + 16 * wid + col;
+    // GATED: each wave carries two of the normaliser's blocks, and begins with them
+    const int d0 = GATE == GATED ? 2 * wid : 0;
+    f32x4 S[8] = {};                     // keys 16 (d ^ d0) + 4 quad ... of column col
     if (a.seg[4 * sg + 3] > 0)
 #pragma unroll
       for (int d = 0; d < 8; ++d)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) S[d][j] = Sp[(long)(16 * d + j) * E];
+        for (int j = 0; j < 4; ++j) S[d][j] = Sp[(long)(16 * (d ^ d0) + j) * E];
+    f32x4 N[2] = {};                     // the same of the normaliser, in all columns
+    float* Np = GATE == GATED
+                    ? a.n + (head * (E / 32) + e0 / 32) * DP + 16 * d0 + 4 * quad
+                    : nullptr;
+    if (GATE == GATED && a.seg[4 * sg + 3] > 0)
+#pragma unroll
+      for (int d = 0; d < 2; ++d) N[d] = *(const f32x4*)(Np + 16 * d);
+    auto put_n = [&](int now) __attribute__((always_inline)) {
+      if (GATE != GATED) return;
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        uint t0[3], t1[3];
+        cut3(N[d][0], N[d][1], t0);
+        cut3(N[d][2], N[d][3], t1);
+        if (col == 0)
+#pragma unroll
+          for (int z = 0; z < 3; ++z)
+            *(uint2*)(s_np + (now * 3 + z) * DP + 16 * (d + d0) + 4 * quad) =
+                uint2{t0[z], t1[z]};
+      }
+    };
+    put_n(0);
     // 8 bytes of row col, slot s: at ^ 16 s
-    const int qx = col * 256 + (row_turn(col) ^ (quad >> 1)) * 16 + (quad & 1) * 8;
+    const int qx = (col * 256 + (row_turn(col) ^ (quad >> 1)) * 16 + (quad & 1) * 8) ^
+                   32 * d0;
+    const int kx = kx0 ^ 32 * d0;
     const int wx = vx ^ (32 * wid), ox = part_at(4 * wid + quad, col);
     // Words are read from LDS a part ahead of the products that need them, and
     // converted beside the products before.
@@ -1881,6 +1921,27 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
       split_v(1);
       order(Count<16>{}, Count<24>{}, Count<3>{});
       updates(1);
+      if (GATE == GATED) {
+        frag_u wp[2][3];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              *(uint2*)&wp[c][z].u[2 * u] = *(const uint2*)(
+                  s_wp + (now * 3 + z) * L + 32 * c + 16 * u + 4 * quad);
+#pragma unroll
+        for (int d = 0; d < 2; ++d) N[d] *= keep;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+              N[d] = mfma16(kf[c][d].bf, wp[c][z].bf, N[d]);
+        put_n(1 - now);
+      }
     };
     meet();
     char *part = s_part, *next = s_part + PART, *after = s_part + 2 * PART;
@@ -1893,29 +1954,76 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
 #pragma unroll
     for (int d = 0; d < 8; ++d)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) Sp[(long)(16 * d + j) * E] = S[d][j];
+      for (int j = 0; j < 4; ++j) Sp[(long)(16 * (d ^ d0) + j) * E] = S[d][j];
+    if (GATE == GATED && col < 2)        // a copy for every 32 columns
+#pragma unroll
+      for (int d = 0; d < 2; ++d) *(f32x4*)(Np + col * DP + 16 * d) = N[d];
     meet();
     return;
   }
 
   if (wid < 8) {
     const float skip = GATE == TIMED ? bits2f(((const short*)a.skip)[h]) : 0.f;
-    const float ib = GATE == TIMED ? bits2f(((const short*)a.ib)[h]) : 0.f;
-    const float rate = GATE == TIMED ? -expf(bits2f(((const short*)a.fb)[h])) : 0.f;
+    const float ib = GATE == DECAY ? 0.f : bits2f(((const short*)a.ib)[h]);
+    const float fb = GATE == DECAY ? 0.f : bits2f(((const short*)a.fb)[h]);
+    const float rate = GATE == TIMED ? -expf(fb) : 0.f;
     const float l2d = GATE == DECAY ? a.log2_decay[h] : 0.f;
-    const float* raw = GATE == TIMED ? a.gates + (long)row0 * a.H + h : nullptr;
+    float* mp = nullptr;
+    float m = 0.f;                       // before the next piece (GATED)
+    if (GATE == GATED) {
+      mp = a.m + (((long)a.seg[4 * sg] * a.H + h) * E + e0) / 32;
+      if (a.seg[4 * sg + 3] > 0) m = mp[0];
+    }
+    struct Raw { float i, f; };
     auto load_gate = [&](int i) __attribute__((always_inline)) {
-      return GATE == TIMED ? raw[(long)min(L * i + lane, rows - 1) * a.H] : 0.f;
+      const long r = row0 + min(L * i + lane, rows - 1);
+      if (GATE == TIMED) return Raw{a.gates[r * a.H + h], 0.f};
+      if (GATE == GATED)
+        return Raw{a.gates[2 * r * a.H + h], a.gates[(2 * r + 1) * a.H + h]};
+      return Raw{0.f, 0.f};
     };
-    auto gates = [&](int i, float g) __attribute__((always_inline)) {
+    auto gates = [&](int i, Raw g) __attribute__((always_inline)) {
+      const int at = (i & 1) * L + lane;
+      if (GATE == GATED) {
+        float in = -INFINITY, F = 0.f;
+        if (L * i + lane < rows) log_gates(a, g.i, g.f, ib, fb, in, F);
+        float I = in;                    // scan of (F, I) by (+, max)
+        float R = __shfl_down(F, 1, 64); // what comes after, without F's rounding
+        if (lane == 63) R = 0.f;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const float F0 = __shfl_up(F, off, 64), I0 = __shfl_up(I, off, 64);
+          const float R0 = __shfl_down(R, off, 64);
+          if (lane >= off) {
+            I = fmaxf(I0 + F, I);
+            F += F0;
+          }
+          if (lane + off < 64) R += R0;
+        }
+        const float mt = fmaxf(F + m, I);
+        const float end = __shfl(F, 63, 64), mn = __shfl(mt, 63, 64);
+        const float w = expf(R + (in - mn));   // large ones first, exactly
+        s_b[at] = F - mt;
+        s_i[at] = in - F;
+        s_far[at] = __expf(F + (m - mt)) * a.qscale;
+        s_em[at] = expf(-mt);
+        s_w[at] = w;
+        uint t[3];
+        cut3(w, 0.f, t);
+#pragma unroll
+        for (int z = 0; z < 3; ++z) s_wp[((i & 1) * 3 + z) * L + lane] = (short)t[z];
+        if (lane == 0) s_keep[i & 1] = expf(end + (m - mn));
+        m = mn;
+        return;
+      }
       if (GATE == DECAY) {               // only what the state needs
         const int n = min(rows - L * i, L);
-        s_w[(i & 1) * L + lane] =
+        s_w[at] =
             lane < n ? __builtin_amdgcn_exp2f((n - 1 - lane) * l2d) : 0.f;
         if (lane == 0) s_keep[i & 1] = __builtin_amdgcn_exp2f(n * l2d);
         return;
       }
-      const float step = L * i + lane < rows ? softplus_f(g + ib) : 0.f;
+      const float step = L * i + lane < rows ? softplus_f(g.i + ib) : 0.f;
       float F = rate * step;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -1923,7 +2031,6 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
         if (lane >= off) F += before;
       }
       const float end = __shfl(F, 63, 64), near = __shfl(F, lane | 15, 64);
-      const int at = (i & 1) * L + lane;
       s_b[at] = F;
       s_i[at] = step;
       s_far[at] = expf(near - F) * step;
@@ -1937,6 +2044,7 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
       f32x4 pv[4];                       // columns 16 et + 4 quad ... of token t
       const int t = 16 * n + col;
       float inter = GATE == DECAY ? __builtin_amdgcn_exp2f((t + 1) * l2d) : 0.f;
+      float inv = 1.f;                   // GATED: 1 / the normaliser
       // (of keys 4 quad + j of block J, seen from token t)
       f32x4 weight[GATE == DECAY ? n + 1 : 1];
       if (GATE == DECAY)
@@ -1955,7 +2063,8 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
 #pragma unroll
         for (int et = 0; et < 4; ++et) o[et] = *(f32x4*)(part + at[et]);
 #pragma unroll
-        for (int et = 0; et < 4; ++et) *(f32x4*)(part + at[et]) = inter * o[et] + pv[et];
+        for (int et = 0; et < 4; ++et) *(f32x4*)(part + at[et]) = GATE == GATED ? (inter * o[et] + pv[et]) * inv
+                                                    : inter * o[et] + pv[et];
       };
       auto piece = [&](int i, const char* qb, const char* kb, const char* vb)
           __attribute__((always_inline)) {
@@ -1978,6 +2087,37 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             if (4 * quad + j > col) acc[n][j] = 0.f;
+        } else if (GATE == GATED) {
+          f32x4 nq = {};                 // the same in all rows
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+              frag_u nf;
+              nf.u4 = *(const uint4v*)(s_np + ((i & 1) * 3 + z) * DP + 32 * c + 8 * quad);
+              nq = mfma16(nf.bf, qf[c].bf, nq);
+            }
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int J = 0; J <= n; ++J) acc[J] = mfma16(kf[c][J].bf, qf[c].bf, acc[J]);
+          const float bt = s_b[(i & 1) * L + t];
+          inter = s_far[(i & 1) * L + t];
+          float den = 0.f;
+#pragma unroll
+          for (int J = 0; J <= n; ++J) {
+            const f32x4 key = *(const f32x4*)(s_i + (i & 1) * L + 16 * J + 4 * quad);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              acc[J][j] *= __expf(bt + key[j]) * a.qscale;
+              if (J == n && 4 * quad + j > col) acc[J][j] = 0.f;
+              den += acc[J][j];
+            }
+          }
+          den += __shfl_xor(den, 16, 64);
+          den += __shfl_xor(den, 32, 64);
+          den += inter * nq[0];
+          inv = 1.f / (fmaxf(fabsf(den), s_em[(i & 1) * L + t]) + GATED_EPS);
         } else {
         const float* b = s_b + (i & 1) * L;
         const float bt = b[t];
@@ -2027,7 +2167,7 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
               pv[et] = mfma16(v[et].bf, pf[z].bf, pv[et]);
         }
       };
-      float g = 0.f;
+      Raw g{0.f, 0.f};
       if (n == 0 && pieces) {
         gates(0, load_gate(0));
         g = load_gate(1);
@@ -2046,6 +2186,7 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
         part = next, next = after, after = p;
       }
       if (pieces) add(part);
+      if (GATE == GATED && n == 0 && lane < 2) mp[lane] = m;
       meet();
     };
     if (wid == 4) run(Count<0>{});
@@ -2207,7 +2348,7 @@ template <int DP, int GATE>
 static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
   const MemoryArgs& a = x.a;
   const long ch = (long)x.n_chunks * a.H;
-  if constexpr ((GATE == TIMED || GATE == DECAY) && DP == PASS_D)
+  if constexpr (GATE != TURNED && DP == PASS_D)
     if (!x.P) {
       const int units = a.H * (a.E / 64);
       memory_pass_kernel<GATE><<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
@@ -2254,7 +2395,7 @@ extern "C" int sv_memory_chunks(const ChunkArgs* x, int gating,
       (x->a.rot % 2 || x->a.rot > x->a.D ||
        (x->a.z && (x->a.E > 128 || (x->a.E > 64 && x->a.D > 128)))))
     return 1;
-  if (!x->VT && ((gating != TIMED && (gating != DECAY || x->P)) || x->a.E % 64 ||
+  if (!x->VT && ((gating != TIMED && (gating == TURNED || x->P)) || x->a.E % 64 ||
                  (x->a.D != 64 && x->a.D != 128)))
     return 1;
   if (!x->U && x->VT) return 1;

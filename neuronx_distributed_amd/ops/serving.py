@@ -1381,13 +1381,15 @@ def memory_pass(chunks: int, segments: int, columns: int) -> bool:
     return chunks - segments + 1 <= chunks * (columns // 64) / 80 + 2
 
 
-def decay_pass(chunks: int, segments: int, columns: int) -> bool:
-    """The same for a decayed memory.  A chunk of the longest segment takes one pass
-    11.9 us behind 5 for the call; the launches and passes it stands for take 17 to 44
-    up to a chunk or two and 0.08 us more for every 64 columns of a chunk.  126 random
-    calls of 2 to 128 heads, one pass over those: 0.57 in the mean, none slower; with 1
-    chunk for the 2.5 0.58, with 4 the same and one call 1.45."""
-    return chunks - segments + 1 <= chunks * (columns // 64) / 100 + 2.5
+def single_pass(chunks: int, segments: int, columns: int, gated: bool) -> bool:
+    """The same for a decayed or a gated memory.  A chunk of the longest segment takes
+    one pass 11.9 us (gated 11.3) behind 5 for the call; the launches and passes it
+    stands for take 17 to 44 (21 to 50) up to a chunk or two and 0.08 us more for every
+    64 columns of a chunk: 64 x 64 columns, 1000 tokens in one segment 51 and 52 (55 and
+    47), 1300 58 and 65, 1500 66 and 77 (66 and 67).  491 random calls each of 2 to 128
+    heads and up to 12 segments of unequal lengths, this over those: 0.56 (0.52)
+    in the mean, none slower."""
+    return chunks - segments + 1 <= chunks * (columns // 64) / 140 + 2 + gated
 
 
 def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
@@ -1476,7 +1478,8 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         tiled, decayed = timed and whole, isinstance(gate, DecayGate)
         once = whole and D == 128 and (
             timed and memory_pass(nc, seg.shape[0], heads * E) or
-            decayed and decay_pass(nc, seg.shape[0], heads * E))
+            (decayed or gated) and single_pass(nc, seg.shape[0], heads * E,
+                                               gated))
         U = None if once or tiled and D == 64 and memory_carries(
             nc, seg.shape[0], heads * D * E) \
             else torch.empty(nc, heads, E, D, **f32)
@@ -1499,7 +1502,7 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
             bic = torch.empty(2, heads, T, **f32)
             small = torch.empty(nc, heads, 4, **f32)
             x.b, x.i, x.tot = _p(bic[0]), _p(bic[1]), _p(small)
-        elif gated:
+        elif gated and not once:
             bic = torch.empty(3, heads, T, **f32)
             small = torch.empty(nc, heads, 6 + D, **f32)
             x.b, x.i, x.c = (_p(t) for t in bic)

@@ -464,13 +464,13 @@ def test_decayed_memory_in_one_pass(sv, monkeypatch, H, E, far):
                                                               65, 192, 5, 16]
     decay = [0.97, 0.0, 1.0, 0.6, 0.999][:H]
     gate = sv.decay_gate(decay, "cuda")
-    assert sv.decay_pass(10, 10, H * E)
+    assert sv.single_pass(10, 10, H * E, False)
     cases = [_mem_inputs(H, D, E, a + b, bf, seed=40 + i)[3]
              for i, (a, b) in enumerate(zip(lens, more))]
     sizes = H * D, H * D, H * E
     got = {}
     for once in (True, False):
-        monkeypatch.setattr(sv, "decay_pass", lambda *a: once)
+        monkeypatch.setattr(sv, "single_pass", lambda *a: once)
         S = torch.full((10, H, D, E), 7.0).cuda()
         out = []
         for at, n in (([0] * 10, lens), (lens, more)):
@@ -497,6 +497,59 @@ def test_decayed_memory_in_one_pass(sv, monkeypatch, H, E, far):
         assert off[0] <= 1.05 * off[1] + 1e-6 * want.norm()
         err = [(got[way][1][9 - i].cpu().double() - S_want).norm() for way in got]
         assert err[0] <= 1.05 * err[1] + 1e-6 * S_want.norm()
+
+
+@pytest.mark.parametrize("H,E,i_scale,f_shift", [
+    (3, 64, 1.0, 3.0), (2, 128, 6.0, 6.0), (4, 192, 3.0, -8.0), (1, 256, 0.1, 12.0)])
+def test_gated_memory_in_one_pass(sv, monkeypatch, H, E, i_scale, f_shift):
+    """Segments that end at, before and behind the 16 tokens of a wave and the 64 of
+    a piece, from empty and from filled slots; gates that forget at once, that keep
+    all, and inputs that stand out; against the oracle, and against chunks."""
+    D, bf, cap = 128, torch.bfloat16, 15.0
+    lens, more = [1, 15, 17, 63, 64, 65, 128, 130, 193, 449], [70, 1, 300, 64, 2, 33,
+                                                              65, 192, 5, 16]
+    assert sv.single_pass(10, 10, H * E, True)
+    ib, fb = (_rand(H, dtype=bf, seed=s) for s in (1, 2))
+    cases, raws = [], []
+    for i, (a, b) in enumerate(zip(lens, more)):
+        cases.append(_mem_inputs(H, D, E, a + b, bf, seed=60 + i)[3])
+        raws.append(_gates(H, a + b, i_scale, f_shift, seed=80 + i))
+        raws[-1][min(9, a + b - 1)] = 40.0
+    sizes, nt = (H * D, H * D, H * E), E // 32
+    got = {}
+    for once in (True, False):
+        monkeypatch.setattr(sv, "single_pass", lambda *a: once)
+        S = torch.full((10, H, D, E), 7.0).cuda()
+        n, m = torch.full((10, H, nt, D), 9e3).cuda(), torch.full((10, H, nt), 50.0).cuda()
+        out = []
+        for at, ln in (([0] * 10, lens), (lens, more)):
+            rows = torch.cat([p[a:a + k] for p, a, k in zip(cases, at, ln)]).cuda()
+            raw = torch.cat([r[a:a + k] for r, a, k in zip(raws, at, ln)]).cuda()
+            seg, *tab = _tables(sv, [(9 - i, sum(ln[:i]), k, a) for i, (a, k) in
+                                     enumerate(zip(at, ln))], True)
+            gate = sv.ExpGate(raw, ib.cuda(), fb.cuda(), cap, D ** -0.5)
+            out.append(sv.memory_mix(*rows[:, :sum(sizes)].split(sizes, dim=1), gate, S,
+                                     n, m, seg, H, *tab).split(ln))
+        got[once] = [torch.cat([o[i] for o in out]) for i in range(10)], S, n, m
+    for i, (p, raw) in enumerate(zip(cases, raws)):
+        x, T = raw.double(), len(p)
+        gi = cap * torch.tanh((x[:, :H] + ib.double()) / cap)
+        gf = vo.log_sigmoid(cap * torch.tanh((x[:, H:] + fb.double()) / cap))
+        q, k, v = (t.double().view(T, H, -1) for t in
+                   p[:, :sum(sizes)].split(sizes, dim=1))
+        want, (S_w, n_w, m_w) = vo.gated_memory(q * D ** -0.5, k, v, gi, gf)
+        want = want.reshape(T, H * E)
+        _close(got[True][0][i], want, bf, 2.0, i)
+        off = [(got[way][0][i].cpu().double() - want).norm() for way in got]
+        assert off[0] <= 1.05 * off[1] + 1e-6 * want.norm()
+        # as they count, times e^m; gates and maxima of 8 to 15 are rounded by 2^-21,
+        # each way's its own, and so is what they weigh
+        for at, w in ((1, S_w), (2, n_w.unsqueeze(1).expand(H, nt, D))):
+            err = [((got[way][3][9 - i].cpu().double()[:, :1] - m_w.view(H, 1)).exp()
+                    .unsqueeze(2) * got[way][at][9 - i].cpu().double() - w).norm()
+                   for way in got]
+            assert err[0] <= 1.05 * err[1] + 2.0 ** -21 * w.norm(), (i, at)
+        assert (got[True][3][9 - i].cpu().double() - m_w.view(H, 1)).abs().max() < 2e-3
 
 
 @pytest.mark.parametrize("gated", [False, True])
