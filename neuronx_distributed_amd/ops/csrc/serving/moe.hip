@@ -543,7 +543,8 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   const int ntn = (a.N + NOUT - 1) / NOUT;
   const int live = PAGED ? (a.rows + BM - 1) / BM : a.tiles[3], total = live * ntn;
   const int tail = total % 256;
-  const int split = !TAIL || tail == 0 || tail > 128 ? 1 : tail > 64 ? 2 : 4;
+  const int split =
+      !TAIL || tail == 0 || tail > 128 ? 1 : BM < 256 || tail > 64 ? 2 : 4;
   const int whole = split > 1 ? total - tail : total;
   int id = blockIdx.x, piece = 0;
   if (id < whole) {
@@ -567,7 +568,11 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
                                                      ws0, ws1, ws2);
     return;
   }
-  if constexpr (TAIL) {
+  if constexpr (TAIL && BM < 256) {
+    if ((tn * 2 + piece) * (NOUT / 2) < a.N)
+      moe_tile<BM, BN / 2, GLU ? WM / 2 : WM, GLU ? WN : WN / 2, GLU, DMA, AHEAD, PAGED>(
+          a, e, slot0, rows, tn * 2 + piece, xs0, xs1, ws0, ws1, ws2);
+  } else if constexpr (TAIL) {
     const int s = piece % 2 * (BM / 2);
     if (s >= rows) return;
     if (split == 2)
@@ -1068,7 +1073,7 @@ template <int BM, int BN, int WM, int WN, bool GLU>
 static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
   constexpr int NOUT = GLU ? BN / 2 : BN;
   constexpr int NT = BM / WM * BN / WN * 64;
-  constexpr bool TAIL = BM == 256;
+  constexpr bool TAIL = BM >= 128;
   const long grid = (long)a.max_tiles * ((a.N + NOUT - 1) / NOUT);
   // offsets of a tile's rows, and of an expert's weights, are bytes of 31 bits
   const bool near = (a.top ? a.rows : 256) * a.xst < 1L << 30 &&
