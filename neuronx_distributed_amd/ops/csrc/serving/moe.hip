@@ -314,11 +314,12 @@ __device__ __forceinline__ float glu(const MoeGemmArgs& a, float g, float u) {
 // slot0, rows: the tile's; tn: its columns
 // PAGED (DMA, top 1): slot s is row s % 64 of page order[s / 64], pages of 64 rows may
 // lie anywhere; slot0 and rows are whole pages.
-template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool AHEAD,
+// AHEAD: the weights come two steps ahead, XA: the rows as well
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool AHEAD, bool XA,
           bool PAGED = false>
 __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
-                                         int rows, int tn, short* xs0,
-                                         short* xs1, short* ws0, short* ws1,
+                                         int rows, int tn, short* xs0, short* xs1,
+                                         short* xs2, short* ws0, short* ws1,
                                          short* ws2) {
   constexpr int NT = BM / WM * BN / WN * 64;
   constexpr int CM = WM / 32, CN = WN / 32;
@@ -441,37 +442,41 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
     // step i: its words are here, in all waves, and the weights of i + 1 may be
     // on their way; the step before is read.  Past the last step that one
     // again, so that the words on their way keep their number.
-    // The wait counts: it is right only if the LW loads of the weights of i + 1
-    // are the last that were asked for, behind the rows and the weights of i.
-    // Nothing else tells the compiler so (they go to different arrays).
+    // The wait counts: it is right only if the loads of i + 1, LW of weights and with
+    // XA before them LX of rows, are the last that were asked for, behind the rows and
+    // the weights of i.  Nothing else tells the compiler so (they go to different
+    // arrays).
     auto in_order = []() __attribute__((always_inline)) {
       asm volatile("" ::: "memory");
     };
     auto turn = [&](int i, short* xs, short* ws, short* xn, short* wn)
         __attribute__((always_inline)) {
-      static_assert(LW < 16, "");
-      __builtin_amdgcn_s_waitcnt(0x70 | LW);       // vmcnt(LW) lgkmcnt(0)
+      constexpr int AFTER = LW + (XA ? LX : 0);
+      static_assert(AFTER < 16, "");
+      __builtin_amdgcn_s_waitcnt(0x70 | AFTER);    // vmcnt(AFTER) lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       in_order();
-      issue_x(min(i + 1, steps - 1) * 64, xn);
+      issue_x(min(i + (XA ? 2 : 1), steps - 1) * 64, xn);
       in_order();
       issue_w(min(i + 2, steps - 1) * 64, wn);
       step(xs, ws);
     };
-    short *const xr[2] = {xs0, xs1}, *const wr[3] = {ws0, ws1, ws2};
+    constexpr int X = XA ? 3 : 2;
+    short *const xr[3] = {xs0, xs1, xs2}, *const wr[3] = {ws0, ws1, ws2};
     issue_x(0, xs0);
     issue_w(0, ws0);
     in_order();
+    if (XA) issue_x(min(1, steps - 1) * 64, xs1);
     issue_w(min(1, steps - 1) * 64, ws1);
     int i = 0;
     for (; i + 6 <= steps; i += 6)
 #pragma unroll
       for (int j = 0; j < 6; ++j)
-        turn(i + j, xr[j % 2], wr[j % 3], xr[(j + 1) % 2], wr[(j + 2) % 3]);
+        turn(i + j, xr[j % X], wr[j % 3], xr[(j + X - 1) % X], wr[(j + 2) % 3]);
 #pragma unroll
     for (int j = 0; j < 5; ++j)
       if (i + j < steps)
-        turn(i + j, xr[j % 2], wr[j % 3], xr[(j + 1) % 2], wr[(j + 2) % 3]);
+        turn(i + j, xr[j % X], wr[j % 3], xr[(j + X - 1) % X], wr[(j + 2) % 3]);
     __builtin_amdgcn_s_waitcnt(0xf70);             // vmcnt(0): LDS is given back
   } else {
     issue(0, xs0, ws0);
@@ -520,7 +525,8 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
 // One workgroup a tile.  TAIL: the last tiles, if they leave half of the CUs
 // without one, are computed in halves of the slots, or quarters, by all of them
 // (36 tiles of 4096 x 14336, 576 workgroups on 256 CUs: 966 us, in whole tiles
-// 1128).
+// 1128); those of 128 slots, which wait for weights, in halves of the columns (8 tiles
+// of 4096 x 14336, 128 workgroups: 250 us, 222).
 // PAGED: all rows are one expert's, `rows` of them.
 template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL,
           bool PAGED = false>
@@ -531,8 +537,12 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   // on their way into the other
   __shared__ __attribute__((aligned(16))) short xs0[BM * 64], xs1[BM * 64];
   // weights two steps ahead where one workgroup has the CU anyway (128 slots,
-  // 4096 rows of 8 experts 4096 x 14336: 842 -> 741 us, 256 slots 985 -> 965)
+  // 4096 rows of 8 experts 4096 x 14336: 842 -> 741 us, 256 slots 985 -> 965), rows as
+  // well where there is room: a step of few rows is shorter than their way (8 experts
+  // 4096 x 14336, both products: 256 tokens 563 -> 529 us, 384 589 -> 559)
   constexpr bool AHEAD = DMA && BM >= 128;
+  constexpr bool XA = AHEAD && BM == 128 && !PAGED;
+  __shared__ __attribute__((aligned(16))) short xs2[XA ? BM * 64 : 8];
   __shared__ __attribute__((aligned(16))) short ws0[BN * 64], ws1[BN * 64],
       ws2[AHEAD ? BN * 64 : 8];
 
@@ -564,23 +574,23 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   const int e = PAGED ? 0 : tl[0], slot0 = PAGED ? tile * BM : tl[1];
   const int rows = PAGED ? min(BM, a.rows - slot0) : tl[2];
   if (!TAIL || id < whole) {
-    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD, PAGED>(a, e, slot0, rows, tn, xs0, xs1,
-                                                     ws0, ws1, ws2);
+    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD, XA, PAGED>(a, e, slot0, rows, tn, xs0, xs1,
+                                                         xs2, ws0, ws1, ws2);
     return;
   }
   if constexpr (TAIL && BM < 256) {
     if ((tn * 2 + piece) * (NOUT / 2) < a.N)
-      moe_tile<BM, BN / 2, GLU ? WM / 2 : WM, GLU ? WN : WN / 2, GLU, DMA, AHEAD, PAGED>(
-          a, e, slot0, rows, tn * 2 + piece, xs0, xs1, ws0, ws1, ws2);
+      moe_tile<BM, BN / 2, GLU ? WM / 2 : WM, GLU ? WN : WN / 2, GLU, DMA, AHEAD, XA,
+               PAGED>(a, e, slot0, rows, tn * 2 + piece, xs0, xs1, xs2, ws0, ws1, ws2);
   } else if constexpr (TAIL) {
     const int s = piece % 2 * (BM / 2);
     if (s >= rows) return;
     if (split == 2)
-      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD, PAGED>(
-          a, e, slot0 + s, min(rows - s, BM / 2), tn, xs0, xs1, ws0, ws1, ws2);
+      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD, XA, PAGED>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn, xs0, xs1, xs2, ws0, ws1, ws2);
     else if ((tn * 2 + piece / 2) * (NOUT / 2) < a.N)
-      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD, PAGED>(
-          a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, xs0, xs1,
+      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD, XA, PAGED>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, xs0, xs1, xs2,
           ws0, ws1, ws2);
   }
 }

@@ -553,6 +553,35 @@ def test_experts(sv, case, dtype):
     _close(x, want, dtype, 2.0, case)
 
 
+@pytest.mark.parametrize("how", [3, 4, 5])
+@pytest.mark.parametrize("W,ff", [(64, 192), (512, 2880), (2048, 128), (1984, 4288)])
+def test_experts_in_tiles(sv, how, W, ff):
+    """Fewer steps than the buffers of rows and weights, and many more; whole rounds of
+    workgroups, few and many behind them, whose halves of columns end inside; tiles of
+    one row, of all and of one less.  As the product of each slot alone."""
+    bf, counts = torch.bfloat16, [1, 31, 33, 64, 127, 128, 129, 0, 257, 511]
+    E, T = len(counts), sum(counts)
+    z = torch.zeros(T, E)
+    z[torch.arange(T), torch.repeat_interleave(torch.arange(E), torch.tensor(counts))] = 9
+    h = _rand(T, W, dtype=bf).cuda()
+    gu = _rand(E, 2 * ff, W, dtype=bf, seed=1, scale=W ** -0.5).cuda()
+    down = _rand(E, W, ff, dtype=bf, seed=2, scale=ff ** -0.5).cuda()
+    p = sv.moe_plan(z.cuda(), None, 1, how)
+    act = sv.moe_gemm(h, gu, p, True)
+    got = sv.moe_gemm(act, down, p, False)
+    at = 0
+    for e, n in enumerate(counts):
+        if not n:
+            continue
+        y = h[at:at + n].float() @ gu[e].float().T
+        y = y[:, :ff] * torch.sigmoid(y[:, :ff]) * y[:, ff:]
+        slots = p.order[at:at + n].long()          # in an expert, any order
+        _close(act[at:at + n][slots.argsort()], y.cpu(), bf, 2.0, (how, e))
+        want = act[at:at + n].float() @ down[e].float().T
+        _close(got[slots], want.cpu(), bf, 2.0, (how, e))
+        at += n
+
+
 def test_plain_swiglu_is_the_default_activation(sv):
     T, E, W, ff, dtype = 9, 2, 64, 32, torch.float32
     h = _rand(T, W, dtype=dtype)
