@@ -438,6 +438,18 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
     __builtin_amdgcn_sched_barrier(0);
   };
   const int steps = (K + 63) / 64;
+  // Where an XCD's 32 workgroups are on several experts, each expert begins elsewhere in
+  // K and goes round: rows a power of two apart, read at the same place by all, meet in
+  // few channels.  16 experts of 4096 x 2048, 256 tokens 234 -> 163 us, 1024 257 -> 208;
+  // 64 of 2048 x 1408, 256 233 -> 221, 1024 311 -> 280 in 256 slots.  Within an expert
+  // all keep step, since they share rows and weights (8 of 4096 x 14336, each column
+  // tile elsewhere: 512 tokens 573 -> 617; each expert, one an XCD: 587).
+  const int skew =
+      !DMA || PAGED || (K & (K - 1)) || N >= 32 * NOUT ? 0 : e * 5 % steps;
+  auto place = [&](int i) __attribute__((always_inline)) {
+    i = min(i, steps - 1) + skew;
+    return (i < steps ? i : i - steps) * 64;
+  };
   if (AHEAD) {
     // step i: its words are here, in all waves, and the weights of i + 1 may be
     // on their way; the step before is read.  Past the last step that one
@@ -456,18 +468,18 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
       __builtin_amdgcn_s_waitcnt(0x70 | AFTER);    // vmcnt(AFTER) lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       in_order();
-      issue_x(min(i + (XA ? 2 : 1), steps - 1) * 64, xn);
+      issue_x(place(i + (XA ? 2 : 1)), xn);
       in_order();
-      issue_w(min(i + 2, steps - 1) * 64, wn);
+      issue_w(place(i + 2), wn);
       step(xs, ws);
     };
     constexpr int X = XA ? 3 : 2;
     short *const xr[3] = {xs0, xs1, xs2}, *const wr[3] = {ws0, ws1, ws2};
-    issue_x(0, xs0);
-    issue_w(0, ws0);
+    issue_x(place(0), xs0);
+    issue_w(place(0), ws0);
     in_order();
-    if (XA) issue_x(min(1, steps - 1) * 64, xs1);
-    issue_w(min(1, steps - 1) * 64, ws1);
+    if (XA) issue_x(place(1), xs1);
+    issue_w(place(1), ws1);
     int i = 0;
     for (; i + 6 <= steps; i += 6)
 #pragma unroll
@@ -479,15 +491,15 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
         turn(i + j, xr[j % X], wr[j % 3], xr[(j + X - 1) % X], wr[(j + 2) % 3]);
     __builtin_amdgcn_s_waitcnt(0xf70);             // vmcnt(0): LDS is given back
   } else {
-    issue(0, xs0, ws0);
+    issue(place(0), xs0, ws0);
     commit(xs0, ws0);
     __syncthreads();                 // also waits for the words on their way
     for (int i = 0; i + 1 < steps; i += 2) {
-      issue(i * 64 + 64, xs1, ws1);
+      issue(place(i + 1), xs1, ws1);
       step(xs0, ws0);
       commit(xs1, ws1);
       __syncthreads();
-      issue(min(i + 2, steps - 1) * 64, xs0, ws0);   // the last one is not read
+      issue(place(i + 2), xs0, ws0);   // past the last one not read
       step(xs1, ws1);
       commit(xs0, ws0);
       __syncthreads();
