@@ -551,9 +551,10 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   // weights two steps ahead where one workgroup has the CU anyway (128 slots,
   // 4096 rows of 8 experts 4096 x 14336: 842 -> 741 us, 256 slots 985 -> 965), rows as
   // well where there is room: a step of few rows is shorter than their way (8 experts
-  // 4096 x 14336, both products: 256 tokens 563 -> 529 us, 384 589 -> 559)
-  constexpr bool AHEAD = DMA && BM >= 128;
-  constexpr bool XA = AHEAD && BM == 128 && !PAGED;
+  // 4096 x 14336, both products: 256 tokens 563 -> 529 us, 384 589 -> 559; 64 slots by 8
+  // waves instead of two workgroups of 4, 128 tokens 580 -> 504)
+  constexpr bool AHEAD = DMA && (BM >= 128 || (BM == 64 && BM / WM * BN / WN == 8));
+  constexpr bool XA = AHEAD && BM < 256 && !PAGED;
   __shared__ __attribute__((aligned(16))) short xs2[XA ? BM * 64 : 8];
   __shared__ __attribute__((aligned(16))) short ws0[BN * 64], ws1[BN * 64],
       ws2[AHEAD ? BN * 64 : 8];
@@ -1091,21 +1092,23 @@ __global__ void __launch_bounds__(256) moe_plain_kernel(MoeGemmArgs a) {
     }
 }
 
-template <int BM, int BN, int WM, int WN, bool GLU>
+// BN2, WM2, WN2: through registers
+template <int BM, int BN, int WM, int WN, bool GLU, int BN2 = BN, int WM2 = WM,
+          int WN2 = WN>
 static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
-  constexpr int NOUT = GLU ? BN / 2 : BN;
-  constexpr int NT = BM / WM * BN / WN * 64;
-  constexpr bool TAIL = BM >= 128;
-  const long grid = (long)a.max_tiles * ((a.N + NOUT - 1) / NOUT);
+  // halves of 64 slots' gates are too few for 8 waves
+  constexpr bool TAIL = BM >= 128 || (BM == 64 && !GLU && BN / WN == 4);
+  auto grid = [&](int nout) { return (long)a.max_tiles * ((a.N + nout - 1) / nout); };
   // offsets of a tile's rows, and of an expert's weights, are bytes of 31 bits
   const bool near = (a.top ? a.rows : 256) * a.xst < 1L << 30 &&
                     (GLU ? 2L : 1L) * a.N * a.K < 1L << 30;
   if (a.K % 64 == 0 && near)             // at most 3 * 64 or 128 pieces more
     moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL>
-        <<<grid + (TAIL ? 192 : 0), NT, 0, stream>>>(a);
+        <<<grid(GLU ? BN / 2 : BN) + (TAIL ? 192 : 0), BM / WM * BN / WN * 64, 0,
+           stream>>>(a);
   else
-    moe_tiles_kernel<BM, BN, WM, WN, GLU, false, false>
-        <<<grid, NT, 0, stream>>>(a);
+    moe_tiles_kernel<BM, BN2, WM2, WN2, GLU, false, false>
+        <<<grid(GLU ? BN2 / 2 : BN2), BM / WM2 * BN2 / WN2 * 64, 0, stream>>>(a);
 }
 
 template <bool GLU>
@@ -1148,8 +1151,8 @@ extern "C" int sv_moe_gemm(const MoeGemmArgs* a, int how, int gated, int f32,
     if (gated) launch_tiles<128, 256, 64, 64, true>(*a, stream);
     else launch_tiles<128, 256, 64, 64, false>(*a, stream);
   } else if (how == 3) {
-    if (gated) launch_tiles<64, 256, 64, 64, true>(*a, stream);
-    else launch_tiles<64, 128, 64, 32, false>(*a, stream);
+    if (gated) launch_tiles<64, 256, 32, 64, true, 256, 64, 64>(*a, stream);
+    else launch_tiles<64, 256, 32, 64, false, 128, 64, 32>(*a, stream);
   } else if (how == 2) {
     if (gated) launch_tiles<32, 256, 32, 64, true>(*a, stream);
     else launch_tiles<32, 128, 32, 32, false>(*a, stream);
