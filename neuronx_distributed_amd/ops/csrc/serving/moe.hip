@@ -315,12 +315,19 @@ __device__ __forceinline__ float glu(const MoeGemmArgs& a, float g, float u) {
 // PAGED (DMA, top 1): slot s is row s % 64 of page order[s / 64], pages of 64 rows may
 // lie anywhere; slot0 and rows are whole pages.
 // AHEAD: the weights come two steps ahead, XA: the rows as well
+// APART: Where an XCD's 32 workgroups are on several experts, each expert begins
+// elsewhere in K and goes round: rows a power of two apart, read at the same place by
+// all, meet in few channels.  16 experts of 4096 x 2048, 256 tokens 234 -> 163 us, 1024
+// 257 -> 208; 64 of 2048 x 1408, 256 233 -> 221, 1024 311 -> 280 in 256 slots; but where
+// matrix cores are the bound, from 224 rows an expert on, not (4096 593 -> 600).  Within
+// an expert all keep step, since they share rows and weights (8 of 4096 x 14336, each
+// column tile elsewhere: 512 tokens 573 -> 617; each expert, one an XCD: 587).
 template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool AHEAD, bool XA,
-          bool PAGED = false>
+          bool APART, bool PAGED = false>
 __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
-                                         int rows, int tn, bool apart, short* xs0,
-                                         short* xs1, short* xs2, short* ws0,
-                                         short* ws1, short* ws2) {
+                                         int rows, int tn, short* xs0, short* xs1,
+                                         short* xs2, short* ws0, short* ws1,
+                                         short* ws2) {
   constexpr int NT = BM / WM * BN / WN * 64;
   constexpr int CM = WM / 32, CN = WN / 32;
   constexpr int LX = BM * 8 / NT, LW = BN * 8 / NT;
@@ -438,20 +445,11 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
     __builtin_amdgcn_sched_barrier(0);
   };
   const int steps = (K + 63) / 64;
-  // Where an XCD's 32 workgroups are on several experts, each expert begins elsewhere in
-  // K and goes round: rows a power of two apart, read at the same place by all, meet in
-  // few channels.  16 experts of 4096 x 2048, 256 tokens 234 -> 163 us, 1024 257 -> 208;
-  // 64 of 2048 x 1408, 256 233 -> 221, 1024 311 -> 280 in 256 slots; but where matrix
-  // cores are the bound, from 224 rows an expert on, not (`apart`; 4096 593 -> 600).
-  // Within an expert all keep step, since they share rows and weights (8 of 4096 x
-  // 14336, each column tile elsewhere: 512 tokens 573 -> 617; each expert, one an XCD:
-  // 587).
-  const int skew = !DMA || PAGED || !apart || (K & (K - 1)) || N >= 32 * NOUT
-                       ? 0
-                       : e * 5 % steps;
+  const int skew = APART ? e * 5 % steps : 0;
+  // past the last step that one again
   auto place = [&](int i) __attribute__((always_inline)) {
     i = min(i, steps - 1) + skew;
-    return (i < steps ? i : i - steps) * 64;
+    return (!APART || i < steps ? i : i - steps) * 64;
   };
   if (AHEAD) {
     // step i: its words are here, in all waves, and the weights of i + 1 may be
@@ -543,9 +541,9 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, int e, int slot0,
 // 1128); those of 128 slots, which wait for weights, in halves of the columns (8 tiles
 // of 4096 x 14336, 128 workgroups: 250 us, 222).
 // PAGED: all rows are one expert's, `rows` of them.
-template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL,
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL, bool APART,
           bool PAGED = false>
-__device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a, bool apart = false) {
+__device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a) {
   constexpr int GROUP = 8;
   constexpr int NOUT = GLU ? BN / 2 : BN;
   // apart by name, so that a read of one buffer need not wait for the words
@@ -590,32 +588,32 @@ __device__ __forceinline__ void moe_tiles(const MoeGemmArgs& a, bool apart = fal
   const int e = PAGED ? 0 : tl[0], slot0 = PAGED ? tile * BM : tl[1];
   const int rows = PAGED ? min(BM, a.rows - slot0) : tl[2];
   if (!TAIL || id < whole) {
-    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD, XA, PAGED>(
-        a, e, slot0, rows, tn, apart, xs0, xs1, xs2, ws0, ws1, ws2);
+    moe_tile<BM, BN, WM, WN, GLU, DMA, AHEAD, XA, APART, PAGED>(
+        a, e, slot0, rows, tn, xs0, xs1, xs2, ws0, ws1, ws2);
     return;
   }
   if constexpr (TAIL && BM < 256) {
     if ((tn * 2 + piece) * (NOUT / 2) < a.N)
       moe_tile<BM, BN / 2, GLU ? WM / 2 : WM, GLU ? WN : WN / 2, GLU, DMA, AHEAD, XA,
-               PAGED>(a, e, slot0, rows, tn * 2 + piece, apart, xs0, xs1, xs2, ws0,
-                      ws1, ws2);
+               APART, PAGED>(a, e, slot0, rows, tn * 2 + piece, xs0, xs1, xs2, ws0, ws1,
+                             ws2);
   } else if constexpr (TAIL) {
     const int s = piece % 2 * (BM / 2);
     if (s >= rows) return;
     if (split == 2)
-      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD, XA, PAGED>(
-          a, e, slot0 + s, min(rows - s, BM / 2), tn, apart, xs0, xs1, xs2, ws0, ws1, ws2);
+      moe_tile<BM / 2, BN, WM / 2, WN, GLU, DMA, AHEAD, XA, APART, PAGED>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn, xs0, xs1, xs2, ws0, ws1, ws2);
     else if ((tn * 2 + piece / 2) * (NOUT / 2) < a.N)
-      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD, XA, PAGED>(
-          a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, apart, xs0, xs1,
-          xs2, ws0, ws1, ws2);
+      moe_tile<BM / 2, BN / 2, WM / 4, WN, GLU, DMA, AHEAD, XA, APART, PAGED>(
+          a, e, slot0 + s, min(rows - s, BM / 2), tn * 2 + piece / 2, xs0, xs1, xs2,
+          ws0, ws1, ws2);
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL>
+template <int BM, int BN, int WM, int WN, bool GLU, bool DMA, bool TAIL, bool APART>
 __global__ void __launch_bounds__(BM / WM * BN / WN * 64)
-moe_tiles_kernel(MoeGemmArgs a, bool apart) {
-  moe_tiles<BM, BN, WM, WN, GLU, DMA, TAIL>(a, apart);
+moe_tiles_kernel(MoeGemmArgs a) {
+  moe_tiles<BM, BN, WM, WN, GLU, DMA, TAIL, APART>(a);
 }
 
 // -- a few rows per expert: stream the weights --------------------------------
@@ -1102,21 +1100,27 @@ template <int BM, int BN, int WM, int WN, bool GLU, int BN2 = BN, int WM2 = WM,
 static void launch_tiles(const MoeGemmArgs& a, hipStream_t stream) {
   // halves of 64 slots' gates are too few for 8 waves
   constexpr bool TAIL = BM >= 128 || (BM == 64 && !GLU && BN / WN == 4);
-  auto grid = [&](int nout) { return (long)a.max_tiles * ((a.N + nout - 1) / nout); };
+  auto launch = [&](auto kernel, int nout, int nt, int more) {
+    const long grid = (long)a.max_tiles * ((a.N + nout - 1) / nout) + more;
+    kernel<<<grid, nt, 0, stream>>>(a);
+  };
+  constexpr int NOUT = GLU ? BN / 2 : BN, NT = BM / WM * BN / WN * 64;
   // a plan has a tile for every BM pairs and one for every expert
   const long pairs = (long)a.rows * (a.top ? a.top : 1);
-  const bool apart = pairs < 224 * (a.max_tiles - pairs / BM);
+  const bool apart = !(a.K & (a.K - 1)) && a.N < 32 * NOUT &&
+                     pairs < 224 * (a.max_tiles - pairs / BM);
   // offsets of a tile's rows, and of an expert's weights, are bytes of 31 bits
   const bool near = (a.top ? a.rows : 256) * a.xst < 1L << 30 &&
                     (GLU ? 2L : 1L) * a.N * a.K < 1L << 30;
-  if (a.K % 64 == 0 && near)             // at most 3 * 64 or 128 pieces more
-    moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL>
-        <<<grid(GLU ? BN / 2 : BN) + (TAIL ? 192 : 0), BM / WM * BN / WN * 64, 0,
-           stream>>>(a, apart);
+  if (a.K % 64 || !near)
+    launch(moe_tiles_kernel<BM, BN2, WM2, WN2, GLU, false, false, false>,
+           GLU ? BN2 / 2 : BN2, BM / WM2 * BN2 / WN2 * 64, 0);
+  else if (apart)                        // at most 3 * 64 or 128 pieces more
+    launch(moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL, true>, NOUT, NT,
+           TAIL ? 192 : 0);
   else
-    moe_tiles_kernel<BM, BN2, WM2, WN2, GLU, false, false>
-        <<<grid(GLU ? BN2 / 2 : BN2), BM / WM2 * BN2 / WN2 * 64, 0, stream>>>(a,
-                                                                              false);
+    launch(moe_tiles_kernel<BM, BN, WM, WN, GLU, true, TAIL, false>, NOUT, NT,
+           TAIL ? 192 : 0);
 }
 
 template <bool GLU>
@@ -1194,7 +1198,7 @@ __global__ void __launch_bounds__(BM / WM * BN / WN * 64)
 latent_expand_kernel(MoeGemmArgs a, uint4v* rot, int P, int tiles) {
   constexpr int NT = BM / WM * BN / WN * 64;
   if ((int)blockIdx.x < tiles) {
-    moe_tiles<BM, BN, WM, WN, false, true, false, true>(a);
+    moe_tiles<BM, BN, WM, WN, false, true, false, false, true>(a);
     return;
   }
   const int page = blockIdx.x - tiles, words = P / 8;    // its shared columns

@@ -1985,27 +1985,33 @@ MOE_TILE_ROWS = (32, 32, 32, 64, 128, 256)
 
 def moe_kernel(pairs: int, experts: int, width: int, ff: int) -> int:
     """The fastest kernel for ``pairs`` spread over ``experts`` of ff x width
-    (measured).  Multiples of 64, us, both products: streaming up to 24 rows an expert,
-    16 where rows of the second product are longer than 4096, 4 where the first one's
-    are, since they are read again and again (64 experts 2048 x 1408, 20 rows: streamed
-    203, tiles of 64 slots 210, 24: 224 and 212; 8 of 4096 x 14336, 12: 489, 515, 16:
-    516, 516, 20: 605, 521; 256 of 7168 x 2048, 3: 3493, 3533, 6: 3865, 3649); then
-    tiles, whose weights and rows come two steps ahead: of 64 slots up to 38 rows, 128 up
-    to 112 (64 experts 2048 x 1408, 32 rows: 217 and 221, 48: 234, 227; 8 of 4096 x
-    14336, 48: 595, 520, and of 128 and 256 slots 96: 582, 664, 112: 774, 679).
-
-    Other sizes: streaming, where workgroups can stay with their rows (width and ff up to
-    4096; 16 rows where only the gates' can), and less than half of the columns that a
-    staying workgroup covers are not there alone, else up to 4 rows; tiles of 32, 64, 128
-    and 256 slots.  The mean rows are all that the host knows."""
+    (measured): streaming up to 24 rows an expert where workgroups can stay with
+    their rows (width and ff up to 4096), 16 where only the gates' can; else the
+    rows are read again and again, and tiles are faster from 4 on (256 experts
+    7168 x 2048, 4 rows: 3.64 ms, streamed 4.21), as where less than half of the
+    columns that a staying workgroup covers are there and the tiles of 256 gates
+    and projections fill the CUs (8 rows of 128 experts 2048 x 768: 238 us,
+    streamed 254; of 64 of 2048 x 512: 104, 96).  Tiles of 64 slots and more
+    read weights two steps ahead where width and ff are multiples of 64, and are
+    the faster ones from 16 rows on (8 experts 4096 x 14336, 16 rows: 32 slots 549
+    us, 64 516; 256 of 7168 x 2048: 3930, 3774), those of 128 from 24 (64 experts
+    2048 x 1408, 24 rows: 64 slots 212, 128 215, 64 rows: 260, 235), with long rows
+    from 48 (8 experts 4096 x 14336, 32 rows: 504, 526, 48: 595, 520), those of 256
+    from 112 (96 rows: 128 slots 582, 256 664, 112: 774, 679).  The mean rows are all
+    that the host knows: 32 rows that go to the same 6 of 64 experts stay as well,
+    528 units on 512 workgroups (58 us; 71 before staying came).  One size is
+    slower than it was: 64 experts 4096 x 2048 of 24 to 32 rows, 777 to 796 us
+    where tiles of 64 took 732 to 760 before the XCDs shared the tiles that have
+    rows."""
     rows = pairs / experts
-    even = not (width | ff) & 63
-    stay = width <= 4096 and (even or min(width, ff) > 960 or
+    stay = width <= 4096 and (min(width, ff) > 960 or
                               experts * ff <= 256 * 128)
     if rows < ((24 if ff <= 4096 else 16) if stay else 4):
         return MOE_STREAM
-    if even:
-        return MOE_TILES[1 + (rows >= 38) + (rows >= 112)]
+    if rows >= 16 and not (width | ff) & 63:
+        if rows < 24 or rows < 48 and max(width, ff) > 4096:
+            return MOE_TILES[1]
+        return MOE_TILES[2 if rows < 112 else 3]
     return MOE_TILES[sum(rows >= r for r in (24, 112, 160))]
 
 
