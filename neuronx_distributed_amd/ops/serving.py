@@ -1476,7 +1476,9 @@ def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,
         whole = D in (64, 128) and E % 64 == 0 and \
             max(t.stride(0) for t in strided) < 1 << 22
         tiled, decayed = timed and whole, isinstance(gate, DecayGate)
-        once = whole and D == 128 and (
+        # one pass writes 16 bytes of the results at once, and of the normaliser
+        once = whole and D == 128 and _aligned((), out) and \
+            (not gated or n.data_ptr() % 16 == 0) and (
             timed and memory_pass(nc, seg.shape[0], heads * E) or
             (decayed or gated) and single_pass(nc, seg.shape[0], heads * E,
                                                gated))

@@ -499,6 +499,33 @@ def test_decayed_memory_in_one_pass(sv, monkeypatch, H, E, far):
         assert err[0] <= 1.05 * err[1] + 1e-6 * S_want.norm()
 
 
+@pytest.mark.parametrize("gated", [False, True])
+def test_results_where_one_pass_cannot_write(sv, gated):
+    """Results and normalisers that begin 8 bytes behind the 16 that are written at
+    once: the same as elsewhere, by chunks."""
+    H, D, E, T, bf = 2, 128, 64, 70, torch.bfloat16
+    q, k, v, p = _mem_inputs(H, D, E, T, bf, seed=5)
+    q, k, v = (t.cuda() for t in (q.contiguous(), k.contiguous(), v.contiguous()))
+    raw, b = _gates(H, T, 1.0, 2.0).cuda(), torch.zeros(H, dtype=bf).cuda()
+    gate = sv.ExpGate(raw, b, b, 15.0, 0.2) if gated else \
+        sv.decay_gate([0.9, 0.99], "cuda")
+    seg, *tab = _tables(sv, [(0, 0, T, 0)], True)
+    outs, normalisers = [], []
+    for out_at, n_at in ((0, 0), (4, 0), (0, 2)):
+        S = torch.zeros(1, H, D, E).cuda()
+        n = torch.zeros(H * 2 * D + 2).cuda()[n_at:n_at + H * 2 * D].view(1, H, 2, D)
+        m = torch.zeros(1, H, 2).cuda()
+        out = torch.full((T * H * E + 8,), 3.0, dtype=bf).cuda()
+        sv.memory_mix(q, k, v, gate, S, n, m, seg, H, *tab,
+                      out=out[out_at:out_at + T * H * E].view(T, H * E))
+        assert (out[:out_at] == 3.0).all() and (out[out_at + T * H * E:] == 3.0).all()
+        outs.append(out[out_at:out_at + T * H * E].float().cpu().view(T, -1))
+        normalisers.append(n.cpu())
+    for got, n in zip(outs[1:], normalisers[1:]):
+        _close(got, outs[0], bf, 2.0)
+        assert (n - normalisers[0]).abs().max() <= 1e-5 * normalisers[0].abs().max()
+
+
 @pytest.mark.parametrize("H,E,i_scale,f_shift", [
     (3, 64, 1.0, 3.0), (2, 128, 6.0, 6.0), (4, 192, 3.0, -8.0), (1, 256, 0.1, 12.0)])
 def test_gated_memory_in_one_pass(sv, monkeypatch, H, E, i_scale, f_shift):
