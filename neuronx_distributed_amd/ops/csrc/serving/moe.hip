@@ -1192,8 +1192,7 @@ extern "C" int sv_moe_gemm(const MoeGemmArgs* a, int how, int gated, int f32,
 // a call): N 8192: 128 rows 13.2 | 8.6, 704 20.2 | 16.0; N 4096: 1600 rows 25.8 | 17.4,
 // 6656 72.8 | 49.2.  (5120 x 8192 over and over: 70.7 | 63.1, in 256 x 256, one workgroup a
 // CU, 77.5, in 128 x 256 67.5; but within a call 63.1 | 70.4, and so left to the library.)
-// 64 x 128
-// is for what does not fill the chip otherwise.
+// 64 x 128 is for what does not fill the chip otherwise.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int WM, int WN>
 __global__ void __launch_bounds__(BM / WM * BN / WN * 64)
