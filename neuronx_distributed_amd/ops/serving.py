@@ -1165,7 +1165,7 @@ def attn_tiles_supported(q, kc, vc) -> bool:
 _HALF_PAGES, _HALF_BYTES = 1024, 1 << 28
 
 
-def value_halves(n_tiles: int, heads: int, groups: int, portions: int,
+def value_halves(n_tiles: int, heads: int, groups: int, portions: Sequence,
                  max_keys: int) -> bool:
     """Do the values of ``portions`` become halves before the query tiles read them?
     That is a kernel and a pass over the pages more, and the tiles' products are a
@@ -1175,9 +1175,9 @@ def value_halves(n_tiles: int, heads: int, groups: int, portions: int,
     128.9, 20 (640 workgroups) 49.0 and 50.1; 16/8, 45 tiles (720) 162 and 151, 24 (384)
     109 and 113; 32/16, 24 tiles in 4 portions, 12 a page, 94.3 and 93.2, 20 51.9 and
     55.0.  Heads of 64: 32/8, 48 tiles 336 and 283, 16/8, 42 tiles (672) 80.3 and 81.7."""
-    return portions > 0 and max_keys > 0 and n_tiles * heads >= 768 and \
-        n_tiles * (heads // groups) >= 16 * portions and \
-        max_keys <= _HALF_PAGES * PAGE_SIZE
+    return n_tiles * heads >= 768 and \
+        n_tiles * (heads // groups) >= 16 * len(portions) and \
+        0 < max_keys <= _HALF_PAGES * PAGE_SIZE
 
 
 def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
@@ -1185,12 +1185,12 @@ def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
                   append: bool = True, max_keys: int = 0,
                   out: Optional[torch.Tensor] = None,
                   mod: Optional[ScoreMod] = None,
-                  portions: int = 0) -> torch.Tensor:
+                  portions: Sequence = ()) -> torch.Tensor:
     """Prompt portions: append k/v (unless they are there), then causal
     attention of every row over its request's cache.  ``tiles`` (n, 4) int32
     lists (request, first row, rows <= 128, position of the first row);
-    ``portions`` requests, the first ones, may have their values made halves first
-    (``value_halves``)."""
+    the first requests, one for each of ``portions``, may have their values made halves
+    before (``value_halves``)."""
     G, D, E = _check_cache(q, k, v, kc, vc, heads)
     if append:
         kv_append(k, v, kc, vc, pos, seq, block_table)
@@ -1205,25 +1205,25 @@ def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
                    tiles=_p(tiles), bt=_p(block_table), out=_p(out),
                    MB=block_table.shape[1], H=heads, G=G, D=D, E=E, DS=D,
                    window=window, keep=keep, scale=scale)
+    n_tiles = tiles.shape[0]
     if mod is not None:
         a.mod = _score_args(mod, q, heads)
-    elif max(D, E) <= 128 and value_halves(tiles.shape[0], heads, G, portions,
-                                           max_keys):
-        cols = -(-max_keys // PAGE_SIZE)
-        size = portions * cols * G * PAGE_SIZE * E
+    elif value_halves(n_tiles, heads, G, portions, max_keys) and \
+            len(portions) and max(D, E) <= 128:
+        seqs, cols = len(portions), -(-max_keys // PAGE_SIZE)
+        size = seqs * cols * G * PAGE_SIZE * E
         half = None
         if 2 * size <= _HALF_BYTES:
             try:
-                half = torch.empty(size + 2 * portions * cols * G,
+                half = torch.empty(size + 2 * seqs * cols * G,
                                    dtype=torch.float16, device=q.device)
             except torch.OutOfMemoryError:
                 pass                  # values stay as they are
         if half is not None:
             a.half, a.half_low = _p(half), _p(half) + 2 * size
-            a.half_seqs, a.half_cols = portions, cols
-            a.n_tiles = tiles.shape[0]
-    _check(library().sv_attn_tiles(ctypes.byref(a), tiles.shape[0],
-                                   _stream()), "attn_tiles")
+            a.half_seqs, a.half_cols, a.n_tiles = seqs, cols, n_tiles
+    _check(library().sv_attn_tiles(ctypes.byref(a), n_tiles, _stream()),
+           "attn_tiles")
     return out
 
 
@@ -1257,7 +1257,7 @@ def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
         if a < n:
             attn_portions(qa, ka, va, kc, vc, pos, seq, batch.block_table,
                           batch.tiles, heads, scale, window, keep, append,
-                          batch.max_keys, oa, ma, batch.portions.shape[0])
+                          batch.max_keys, oa, ma, batch.portions)
         elif a < T:
             attn_rows(qa, ka, va, kc, vc, pos, seq, batch.block_table, heads,
                       scale, window, keep, append, batch.max_keys, oa, ma,

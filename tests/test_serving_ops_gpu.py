@@ -256,7 +256,7 @@ def test_values_as_halves(sv, monkeypatch, kind, H, G, D, E, window, keep):
         got = sv.attn_portions(
             q, k[:q.shape[0]], v[:q.shape[0]], c.kc, c.vc, pos, seq, c.bt,
             i32(tiles[::order]), H, 0.11, window, keep, append=False,
-            max_keys=max_keys, portions=portions)
+            max_keys=max_keys, portions=range(portions))
         at = 0
         for d, a, bound in zip(data, first, bounds):
             n = d[3].shape[0] - a
