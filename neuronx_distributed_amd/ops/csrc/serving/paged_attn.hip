@@ -18,15 +18,10 @@
 
 #include "serving.h"
 
-#include <climits>
-
 #define NEG_BIG (-1e30f)
 // The running maximum may lag behind by this much (in log 2): O is rescaled only
 // when a row outgrows it.  The weights are 32-bit either way.
 #define TILES_LAG 8.f
-// Weights that are split into halves are that much larger (in log 2), so that the
-// halves have room below: up to 2^15.
-#define HALF_UP 7.f
 
 // ---------------------------------------------------------------------------
 // append
@@ -934,8 +929,8 @@ extern "C" int sv_attn_rows(const RowsArgs* a, int vec, int f32,
 // One workgroup = 4 waves x 32 query rows of one head; a key tile is one
 // cache page.  S^T = K Q^T keeps every softmax statistic lane-local (a lane
 // owns one query row).  The weights stay 32-bit: P is split exactly into
-// three bf16 planes (they carry the full 24-bit significand), or into two halves
-// where the values are halves, too, and V enters once per plane.  P never leaves registers: the accumulator's row order
+// NP bf16 planes (3 planes carry the full 24-bit significand) and V enters
+// once per plane.  P never leaves registers: the accumulator's row order
 // {4 hi + 0..3, 8 + 4 hi + 0..3} of a 16-key chunk is used as the
 // contraction order of P V, and V^T is read from LDS in the same order
 // (transposing loads).
@@ -972,144 +967,11 @@ struct TilesArgs {
   int window, keep;
   float scale;
   ScoreArgs mod;            // its gate is one number a head
-  // Values as halves, of the requests before `half_seqs` and `half_cols` pages of each
-  // (value_halves_kernel); or null
-  short* half;              // [request][page][G][64][E]
-  int* half_low;            // [request][G][page]
-  int half_seqs, half_cols, n_tiles;
 };
-
-// The key tiles that `nrow` queries from position p0 on see: the kept first ones, then
-// from t_lo on.
-struct KeyTiles {
-  int nk, t_lo, n;
-  __device__ __forceinline__ KeyTiles(int p0, int nrow, int window, int keep) {
-    const int t_hi = (p0 + nrow - 1) / SV_PAGE;
-    const int lo = window > 0 ? max(0, p0 - window + 1) : 0;
-    nk = window > 0 ? min((keep + SV_PAGE - 1) / SV_PAGE, t_hi + 1) : 0;
-    t_lo = max(nk, lo / SV_PAGE);
-    n = nk + max(0, t_hi - t_lo + 1);
-  }
-};
-
-// ---------------------------------------------------------------------------
-// Values as halves.  A weight of 32 bits is the sum of three bf16, but to its last
-// place that of two halves, and those cost less to make, 4 instructions a pair for 11,
-// where the tiles are bound by the matrix cores and vector work together.  So where
-// many query tiles read a page, its values become halves first, times a power of two
-// that is the page's own.  A bf16 has 8 bits, a half 11: nothing is rounded where every
-// value but zero is within 2^29 of the largest.  A page where one is not, or is no
-// number, is read as it is (HALF_KEPT), with three planes.  The result is as far from
-// 64 bits as with three planes: 6000 tokens of three portions behind up to 4096, 32/8
-// heads, 1.614e-3 either way, and 0.042 % of the bf16 results are not the nearest
-// (0.046 %).  That takes 497 us for 557, 15 of them this kernel's, which moves the
-// pages at the rate of a copy; turning values inside the tiles' kernel, 16 keys a wave,
-// took 548, since that is vector work again.
-//
-// One workgroup a page and key head.  half_low: what the exponent of a bf16 has more
-// than that of its half.
-// ---------------------------------------------------------------------------
-#define HALF_KEPT 256
-#define HALF_ANY 511                 // kept, and its largest value is not known
-#define HALF_COLS 1024               // pages of a request at most
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-
-__global__ void __launch_bounds__(256) value_halves_kernel(TilesArgs a) {
-  const int page = blockIdx.x, g = blockIdx.y, seq = blockIdx.z, E = a.E;
-  // the request's new rows, of all its tiles
-  int p0 = INT_MAX, end = 0;
-  for (int i = threadIdx.x & 63; i < a.n_tiles; i += 64) {
-    const int* t = a.tiles + 4 * i;
-    if (t[0] != seq) continue;
-    p0 = min(p0, t[3]);
-    end = max(end, t[3] + t[2]);
-  }
-#pragma unroll
-  for (int off = 32; off; off >>= 1) {
-    p0 = min(p0, __shfl_xor(p0, off, 64));
-    end = max(end, __shfl_xor(end, off, 64));
-  }
-  if (p0 >= end) return;
-  const KeyTiles seen(p0, end - p0, a.window, a.keep);
-  if (page * SV_PAGE >= end || (page >= seen.nk && page < seen.t_lo)) return;
-
-  const long from = a.bt[(long)seq * a.MB + page];
-  const uint4v* src = (const uint4v*)(a.vc + from * a.vpage + g * a.vhead);
-  const int words = SV_PAGE * E / 8, live = min(end - page * SV_PAGE, SV_PAGE) * E / 8;
-  constexpr int N = 4;                 // words a thread at most, of 128 columns
-  uint4v w[N];
-  ushort2v least = {0xffff, 0xffff}, most = {0, 0};
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int at = i * 256 + threadIdx.x;
-    // rows past the request's last one are zero
-    w[i] = at < live ? src[at] : uint4v{0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const ushort2v m = __builtin_bit_cast(ushort2v, w[i][j] & 0x7fff7fffu);
-      least = __builtin_elementwise_min(least, m - (unsigned short)1);  // 0 is largest
-      most = __builtin_elementwise_max(most, m);
-    }
-  }
-  int lo = min(least.x, least.y), hi = max(most.x, most.y);
-#pragma unroll
-  for (int off = 32; off; off >>= 1) {
-    lo = min(lo, __shfl_xor(lo, off, 64));
-    hi = max(hi, __shfl_xor(hi, off, 64));
-  }
-  __shared__ int s_lo[4], s_hi[4];
-  if ((threadIdx.x & 63) == 0) {
-    s_lo[threadIdx.x >> 6] = lo;
-    s_hi[threadIdx.x >> 6] = hi;
-  }
-  __syncthreads();
-  lo = min(min(s_lo[0], s_lo[1]), min(s_lo[2], s_lo[3]));
-  hi = max(max(s_hi[0], s_hi[1]), max(s_hi[2], s_hi[3]));
-  // the largest exponent of a half that is a number is 30, the least 1
-  const bool number = hi < 0x7f80;
-  const int low = max((hi >> 7) - 30, 0);
-  const bool kept = !number || lo < (low + 1) * 128 - 1;
-  if (threadIdx.x == 0)
-    a.half_low[((long)seq * a.G + g) * a.half_cols + page] =
-        !number ? HALF_ANY : kept ? low | HALF_KEPT : low;
-  if (kept) return;
-  const ushort2v less = {(unsigned short)(low << 7), (unsigned short)(low << 7)};
-  uint4v* dst = (uint4v*)(a.half + (((long)seq * a.half_cols + page) * a.G + g) *
-                                       SV_PAGE * E);
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int at = i * 256 + threadIdx.x;
-    if (at >= words) break;
-    uint4v o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const ushort2v m = __builtin_bit_cast(ushort2v, w[i][j] & 0x7fff7fffu);
-      o[j] = (w[i][j] & 0x80008000u) |
-             __builtin_bit_cast(uint, __builtin_elementwise_sub_sat(m, less)
-                                          << (unsigned short)3);
-    }
-    dst[at] = o;
-  }
-}
-
-// x and y as sums of two halves each, rounded to nearest
-__device__ __forceinline__ void split_halves(float x, float y, uint& near, uint& rest) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  near = __builtin_bit_cast(uint, __builtin_convertvector((f32x2{x, y}), f16x2));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]"
-      : "=v"(x) : "v"(near), "v"(x));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-      : "=v"(y) : "v"(near), "v"(y));
-  rest = __builtin_bit_cast(uint, __builtin_convertvector((f32x2{x, y}), f16x2));
-}
 
 // MOD: 0 plain scores, 1 with a distance bias, 2 with a soft cap (and the bias,
 // if there is one); a sink and the gates are handled in all.
-// HALF: values come as halves where they can.
-template <int DK, int DE, bool SHARED, int MOD, bool HALF>
+template <int DK, int DE, int NP, bool SHARED, int MOD>
 __global__ void __launch_bounds__(256, DE <= 128 ? 2 : 1)
 attn_tiles_kernel(TilesArgs a) {
   constexpr int NC = DK / 16;        // 16-wide chunks of the key size
@@ -1120,8 +982,6 @@ attn_tiles_kernel(TilesArgs a) {
   // need not wait for the words on their way into the other
   __shared__ __attribute__((aligned(16))) char k0[64 * KP], k1[64 * KP];
   __shared__ __attribute__((aligned(16))) char v0[128 * DE], v1[128 * DE];
-  __shared__ int s_low[HALF ? HALF_COLS : 1];  // of the key tiles' pages
-  static_assert(!HALF || (MOD == 0 && !SHARED));
 
   // later tiles of a portion see more keys: they start first
   const int* tl = a.tiles + 4 * (gridDim.y - 1 - blockIdx.y);
@@ -1164,8 +1024,12 @@ attn_tiles_kernel(TilesArgs a) {
   float l_run = 0.f;                 // over this half wave's keys
 
   const int q_hi = p0 + nrow - 1;
-  const KeyTiles seen(p0, nrow, a.window, a.keep);
-  const int nk = seen.nk, t_lo = seen.t_lo, ntiles = seen.n;
+  const int t_hi = q_hi / SV_PAGE;
+  const int lo = a.window > 0 ? max(0, p0 - a.window + 1) : 0;
+  const int nk = a.window > 0
+                     ? min((a.keep + SV_PAGE - 1) / SV_PAGE, t_hi + 1) : 0;
+  const int t_lo = max(nk, lo / SV_PAGE);
+  const int ntiles = nk + max(0, t_hi - t_lo + 1);
   const int w_lo = p0 + wid * 32, w_hi = min(w_lo + 31, q_hi);
 
   // 32-bit within a page
@@ -1202,19 +1066,8 @@ attn_tiles_kernel(TilesArgs a) {
       for (int p = 0; p < CK / 4; ++p) word(p, false);
     }
   };
-  // Halves are counted from the largest exponent of all pages (low_run): weights of a
-  // page of smaller ones are so much smaller, and kept pages are multiplied.  Pages of
-  // less than 2^-10 of that are taken as kept ones.
-  int low_run = 0;
-  auto low_of = [&](int n) {
-    return !HALF ? 0 : n >= HALF_COLS ? HALF_ANY
-                                      : __builtin_amdgcn_readfirstlane(s_low[n]);
-  };
-  auto is_half = [&](int low) { return HALF && low >= low_run - 10 && low <= low_run; };
-  auto issue_v = [&](long page, int n, char* vd) {
+  auto issue_v = [&](long page, char* vd) {
     const short* vb = a.vc + page * a.vpage + g * a.vhead;
-    if (HALF && is_half(low_of(n)))
-      vb = a.half + (((long)seq * a.half_cols + tile_of(n)) * a.G + g) * SV_PAGE * E;
     auto word = [&](int p, bool all) __attribute__((always_inline)) {
       const int it = p * 256 + tid, r = it / CV;
       const int c = (it % CV ^ value_turn<CV>(r)) * 8;
@@ -1317,75 +1170,51 @@ attn_tiles_kernel(TilesArgs a) {
       for (int nb = 0; nb < NB; ++nb) ot[nb] *= alpha;
     }
   };
-  auto weigh = [&](f32x16* s, int low) __attribute__((always_inline)) {
+  auto weigh = [&](f32x16* s) __attribute__((always_inline)) {
     float ps = 0.f;
-    const int less = is_half(low) ? low_run - low : 0;
-    const float m = HALF ? m_run - (HALF_UP - less) : m_run;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s[kb][r] = __builtin_amdgcn_exp2f(MOD == 0 ? s[kb][r] * s2 - m
-                                                   : s[kb][r] - m);
+        s[kb][r] = __builtin_amdgcn_exp2f(MOD == 0 ? s[kb][r] * s2 - m_run
+                                                   : s[kb][r] - m_run);
         ps += s[kb][r];
       }
-    l_run += HALF ? ps * __uint_as_float((uint)(127 + less) << 23) : ps;
+    l_run += ps;
   };
   // O^T += V^T P, 16 keys after 16; the next ones' planes are made beside the
-  // products.  A plane of all columns after the other: a product that adds to the one
-  // before it waits for it (6000 prompt tokens: 590 -> 582 us, latent 395 -> 381)
-  union Values { tr4 t[2]; bf16x8 bf; f16x8 h; };
-  auto read_v = [&](Values* vf, char* vbuf, int c) __attribute__((always_inline)) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        vf[nb].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_tr4)(vbuf + (vx ^ (nb * 64)) + (16 * c + 8 * u) * DE * 2));
-  };
+  // products
   auto gather = [&](const f32x16* s, char* vbuf) __attribute__((always_inline)) {
-    const float up = HALF ? __uint_as_float((uint)(239 - low_run) << 23) : 1.f;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      frag_u pf[3];
+      frag_u pf[NP];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         float x = s[c >> 1][8 * (c & 1) + 2 * u];
         float y = s[c >> 1][8 * (c & 1) + 2 * u + 1];
-        if (HALF) x *= up, y *= up;
 #pragma unroll
-        for (int z = 0; z < 3; ++z) {
+        for (int z = 0; z < NP; ++z) {
           const uint w = pack_bf16x2(x, y);
           pf[z].u[u] = w;
           x -= __uint_as_float(w << 16);
           y -= __uint_as_float(w & 0xffff0000u);
         }
       }
-      Values vf[NB];
-      read_v(vf, vbuf, c);
+      // a plane of all columns after the other: a product that adds to the one
+      // before it waits for it (6000 prompt tokens: 590 -> 582 us, latent 395 ->
+      // 381)
+      union { tr4 t[2]; bf16x8 bf; } vf[NB];
 #pragma unroll
-      for (int z = 0; z < 3; ++z)
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          vf[nb].t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_tr4)(vbuf + (vx ^ (nb * 64)) + (16 * c + 8 * u) * DE * 2));
+#pragma unroll
+      for (int z = 0; z < NP; ++z)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
           ot[nb] = mfma_bf16(vf[nb].bf, pf[z].bf, ot[nb]);
-    }
-  };
-  auto gather_halves = [&](const f32x16* s, char* vbuf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      union { uint u[4]; f16x8 h; } pf[2];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        split_halves(s[c >> 1][8 * (c & 1) + 2 * u],
-                     s[c >> 1][8 * (c & 1) + 2 * u + 1], pf[0].u[u], pf[1].u[u]);
-      Values vf[NB];
-      read_v(vf, vbuf, c);
-#pragma unroll
-      for (int z = 0; z < 2; ++z)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          ot[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[nb].h, pf[z].h, ot[nb], 0,
-                                                          0, 0);
     }
   };
   auto active = [&](int n) {
@@ -1401,13 +1230,8 @@ attn_tiles_kernel(TilesArgs a) {
     if (now) level(n, s);
     if (now || active(n + 1)) scores(next, kbuf);
     if (now) {
-      const int low = low_of(n);
-      weigh(s, low);
-      // (two branches, which the compiler must not join: joined, 37 registers spill)
-      int again = low;
-      if (HALF && is_half(low)) gather_halves(s, vbuf);
-      if (HALF) asm volatile("" : "+s"(again));
-      if (!is_half(again)) gather(s, vbuf);
+      weigh(s);
+      gather(s, vbuf);
     }
   };
 
@@ -1421,38 +1245,23 @@ attn_tiles_kernel(TilesArgs a) {
   f32x16 sa[2], sb[2];
   int pa = page_of(0), pb = page_of(1), pc = page_of(2);
   issue_k(pa, k0);
-  if (!HALF) issue_v(pa, 0, v0);
+  issue_v(pa, v0);
   if (ntiles > 1) issue_k(pb, k1);
-  if (HALF)
-    for (int n = tid; n < min(ntiles, HALF_COLS); n += 256) {
-      const int c = tile_of(n);
-      s_low[n] = seq < a.half_seqs && c < a.half_cols
-          ? a.half_low[((long)seq * a.G + g) * a.half_cols + c] : HALF_ANY;
-    }
   __syncthreads();             // also waits for the words on their way
-  if (HALF) {
-    float most = 0.f;
-    for (int n = lane; n < min(ntiles, HALF_COLS); n += 64)
-      most = fmaxf(most, (float)(s_low[n] & (HALF_KEPT - 1)));
-    low_run = __builtin_amdgcn_readfirstlane((int)fold64(most, MaxOp()));
-    // values that are not known are multiplied by the weights as they are
-    if (low_run == 255 || ntiles > HALF_COLS) low_run = 112 + (int)HALF_UP;
-    issue_v(pa, 0, v0);
-  }
   if (active(0)) scores(sa, k0);
   __syncthreads();
   for (int n = 0; n < ntiles; n += 2) {
     // keys of n + 1 and values of n are there; pb, pc: pages of n + 1, n + 2
     const int vd = page_of(n + 3);
     if (n + 2 < ntiles) issue_k(pc, k0);
-    if (n + 1 < ntiles) issue_v(pb, n + 1, v1);
+    if (n + 1 < ntiles) issue_v(pb, v1);
     step(n, sa, sb, k1, v0);
     __syncthreads();
     if (n + 1 >= ntiles) break;
     pb = settle(vd);
     const int ve = page_of(n + 4);
     if (n + 3 < ntiles) issue_k(pb, k1);
-    if (n + 2 < ntiles) issue_v(pc, n + 2, v0);
+    if (n + 2 < ntiles) issue_v(pc, v0);
     step(n + 1, sb, sa, k0, v1);
     __syncthreads();
     pc = settle(ve);
@@ -1470,7 +1279,6 @@ attn_tiles_kernel(TilesArgs a) {
   if (a.mod.gate)
     inv *= sigmoid_f(bits2f(
         ((const short*)a.mod.gate)[(long)(row0 + my) * a.mod.gst + h]));
-  if (HALF) inv *= __uint_as_float((uint)(low_run + 15) << 23);
   short* dst = a.out + ((long)(row0 + my) * a.H + h) * E;
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
@@ -1500,20 +1308,8 @@ extern "C" int sv_attn_tiles(const TilesArgs* a, int n_tiles,
   const dim3 grid(a->H, n_tiles);
   const int mod = a->mod.cap > 0.f ? 2 : a->mod.slope ? 1 : 0;
   if (a->kr && mod) return 1;
-  if (a->half) {               // values as halves, then the tiles
-    if (mod || a->mod.temp || a->mod.sink || a->mod.gate || a->kr || a->gate ||
-        a->n_tiles != n_tiles || a->vrow != a->E || a->D > 128 || a->E > 128 ||
-        a->half_seqs <= 0 || a->half_cols <= 0 || a->half_cols > HALF_COLS)
-      return 1;
-    value_halves_kernel<<<dim3(a->half_cols, a->G, a->half_seqs), 256, 0, stream>>>(*a);
-    if (a->D <= 64 && a->E <= 64)
-      attn_tiles_kernel<64, 64, false, 0, true><<<grid, 256, 0, stream>>>(*a);
-    else
-      attn_tiles_kernel<128, 128, false, 0, true><<<grid, 256, 0, stream>>>(*a);
-    return (int)hipGetLastError();
-  }
 #define ATK(K, V, S, M) \
-  attn_tiles_kernel<K, V, S, M, false><<<grid, 256, 0, stream>>>(*a)
+  attn_tiles_kernel<K, V, 3, S, M><<<grid, 256, 0, stream>>>(*a)
 #define AT(K, V)                          \
   do {                                    \
     if (a->kr) ATK(K, V, true, 0);        \

@@ -169,9 +169,7 @@ class _TilesArgs(ctypes.Structure):
                 + _fields("gst", ctypes.c_long)
                 + _fields("tiles bt out", ctypes.c_void_p)
                 + _fields("MB H G D E DS window keep", ctypes.c_int)
-                + _fields("scale", ctypes.c_float) + [("mod", _ScoreArgs)]
-                + _fields("half half_low", ctypes.c_void_p)
-                + _fields("half_seqs half_cols n_tiles", ctypes.c_int))
+                + _fields("scale", ctypes.c_float) + [("mod", _ScoreArgs)])
 
 
 class _LatentAppendArgs(ctypes.Structure):
@@ -1161,36 +1159,14 @@ def attn_tiles_supported(q, kc, vc) -> bool:
             and _aligned((D, E), q))
 
 
-# pages of a request whose values may become halves, and bytes of all
-_HALF_PAGES, _HALF_BYTES = 1024, 1 << 28
-
-
-def value_halves(n_tiles: int, heads: int, groups: int, portions: Sequence,
-                 max_keys: int) -> bool:
-    """Do the values of ``portions`` become halves before the query tiles read them?
-    That is a kernel and a pass over the pages more, and the tiles' products are a
-    quarter less: it pays where workgroups fill the chip, from 768 on, and 16 of them
-    read a page.  Over 125 sizes, heads of 128, without halves and with them, us: 32/8
-    heads, 48 tiles 537 and 470, 28 104 and 98.6, 34 with a window of 1024 127.3 and
-    128.9, 20 (640 workgroups) 49.0 and 50.1; 16/8, 45 tiles (720) 162 and 151, 24 (384)
-    109 and 113; 32/16, 24 tiles in 4 portions, 12 a page, 94.3 and 93.2, 20 51.9 and
-    55.0.  Heads of 64: 32/8, 48 tiles 336 and 283, 16/8, 42 tiles (672) 80.3 and 81.7."""
-    return n_tiles * heads >= 768 and \
-        n_tiles * (heads // groups) >= 16 * len(portions) and \
-        0 < max_keys <= _HALF_PAGES * PAGE_SIZE
-
-
 def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
                   scale: float, window: int = 0, keep: int = 0,
                   append: bool = True, max_keys: int = 0,
                   out: Optional[torch.Tensor] = None,
-                  mod: Optional[ScoreMod] = None,
-                  portions: Sequence = ()) -> torch.Tensor:
+                  mod: Optional[ScoreMod] = None) -> torch.Tensor:
     """Prompt portions: append k/v (unless they are there), then causal
     attention of every row over its request's cache.  ``tiles`` (n, 4) int32
-    lists (request, first row, rows <= 128, position of the first row);
-    the first requests, one for each of ``portions``, may have their values made halves
-    before (``value_halves``)."""
+    lists (request, first row, rows <= 128, position of the first row)."""
     G, D, E = _check_cache(q, k, v, kc, vc, heads)
     if append:
         kv_append(k, v, kc, vc, pos, seq, block_table)
@@ -1205,25 +1181,10 @@ def attn_portions(q, k, v, kc, vc, pos, seq, block_table, tiles, heads: int,
                    tiles=_p(tiles), bt=_p(block_table), out=_p(out),
                    MB=block_table.shape[1], H=heads, G=G, D=D, E=E, DS=D,
                    window=window, keep=keep, scale=scale)
-    n_tiles = tiles.shape[0]
     if mod is not None:
         a.mod = _score_args(mod, q, heads)
-    elif value_halves(n_tiles, heads, G, portions, max_keys) and \
-            len(portions) and max(D, E) <= 128:
-        seqs, cols = len(portions), -(-max_keys // PAGE_SIZE)
-        size = seqs * cols * G * PAGE_SIZE * E
-        half = None
-        if 2 * size <= _HALF_BYTES:
-            try:
-                half = torch.empty(size + 2 * seqs * cols * G,
-                                   dtype=torch.float16, device=q.device)
-            except torch.OutOfMemoryError:
-                pass                  # values stay as they are
-        if half is not None:
-            a.half, a.half_low = _p(half), _p(half) + 2 * size
-            a.half_seqs, a.half_cols, a.n_tiles = seqs, cols, n_tiles
-    _check(library().sv_attn_tiles(ctypes.byref(a), n_tiles, _stream()),
-           "attn_tiles")
+    _check(library().sv_attn_tiles(ctypes.byref(a), tiles.shape[0],
+                                   _stream()), "attn_tiles")
     return out
 
 
@@ -1257,7 +1218,7 @@ def ragged_attention(q, k, v, batch, pool, heads: int, scale: float,
         if a < n:
             attn_portions(qa, ka, va, kc, vc, pos, seq, batch.block_table,
                           batch.tiles, heads, scale, window, keep, append,
-                          batch.max_keys, oa, ma, batch.portions)
+                          batch.max_keys, oa, ma)
         elif a < T:
             attn_rows(qa, ka, va, kc, vc, pos, seq, batch.block_table, heads,
                       scale, window, keep, append, batch.max_keys, oa, ma,

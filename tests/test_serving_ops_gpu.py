@@ -2,6 +2,7 @@
 ``voletar_oracle`` (float64), one mechanism at a time."""
 
 import math
+import types
 
 import pytest
 import torch
@@ -196,8 +197,8 @@ def test_attention_edges_show(sv, window, keep, dtype):
                    what=(window, keep, s, cuts[0]))
 
 
-def _halves_values(v, kind):
-    """v (T, G * E) with what decides whether a page becomes halves."""
+def _sized_values(v, kind):
+    """v (T, G * E) of one page beside the next, and within a page."""
     v = v.clone()
     page = torch.arange(v.shape[0]) // 64
     if kind == "wide":                     # a page of 2^33 beside usual ones
@@ -208,7 +209,7 @@ def _halves_values(v, kind):
     elif kind == "zeros":
         v[64:128] = 0
         v[::3, ::5] = 0
-    elif kind == "ends":                   # the least and the largest that fit
+    elif kind == "ends":                   # 2^29 apart everywhere
         v[:] = v.sign() * 2.0 ** -29
         v[::2, 1::3] = 1.9921875
     elif kind == "tiny":                   # some of them too small for bf16
@@ -223,15 +224,15 @@ def _halves_values(v, kind):
 @pytest.mark.parametrize("H,G,D,E,window,keep", [
     (4, 2, 128, 128, 0, 0), (3, 1, 64, 64, 90, 21), (2, 2, 96, 40, 64, 64),
     (4, 1, 24, 72, 0, 0)])
-def test_values_as_halves(sv, monkeypatch, kind, H, G, D, E, window, keep):
-    """Values made halves first, page by page, against 64 bits: the edges of what
-    a half can hold, requests and pages that have no halves, tiles in any order."""
+def test_values_of_all_sizes(sv, kind, H, G, D, E, window, keep):
+    """Values that differ by page, that nearly leave the range of the type or are
+    zero, against 64 bits; tiles in any order."""
     dtype, lens, first = torch.bfloat16, [290, 133, 200], [0, 130, 75]
     mask = {"size": window, "keep_first": keep} if window else None
     data, bounds = [], []
     for i, n in enumerate(lens):
         q, k, v, _ = _attn_case(H, G, D, E, window, keep, n, dtype, seed=40 + n)
-        v = _halves_values(v, kind)
+        v = _sized_values(v, kind)
         qkv = [t.double().view(n, -1, s) for t, s in ((q, D), (k, D), (v, E))]
         want = vo.windowed_attention(*qkv, 0.11, mask).reshape(n, H * E)
         size = vo.windowed_attention(*qkv[:2], qkv[2].abs(), 0.11, mask)
@@ -251,18 +252,17 @@ def test_values_as_halves(sv, monkeypatch, kind, H, G, D, E, window, keep):
         for p in range(a, n, 128):
             tiles.append((r, at + p - a, min(128, n - p), p))
         at += n - a
-    monkeypatch.setattr(sv, "value_halves", lambda *a: True)
-    for portions, max_keys, order in ((3, 290, 1), (2, 290, -1), (3, 128, 1)):
+    for order in (1, -1):
         got = sv.attn_portions(
             q, k[:q.shape[0]], v[:q.shape[0]], c.kc, c.vc, pos, seq, c.bt,
             i32(tiles[::order]), H, 0.11, window, keep, append=False,
-            max_keys=max_keys, portions=range(portions))
+            max_keys=290)
         at = 0
         for d, a, bound in zip(data, first, bounds):
             n = d[3].shape[0] - a
             err = (got[at:at + n].double().cpu() - d[3][a:]).abs()
             assert (err <= bound[a:] + 2.0 ** -133).all(), (
-                portions, max_keys, (err / bound[a:]).max())
+                order, (err / bound[a:]).max())
             at += n
 
 
@@ -334,6 +334,37 @@ def test_attention_weights_keep_32_bits(sv):
     assert small.sum() > 20
     assert ((got - want).abs()[small] <
             2e-5 + 4e-3 * want.abs()[small]).all()
+
+
+def test_small_weights_keep_32_bits(sv):
+    """A key without a value takes nearly all the weight, by 2^8 to 2^22 in the eight
+    groups of heads, and one that nobody looks at has a value of 2^9 times the others':
+    what is left, equal weights of the many, keeps its bits.  (Weights of 16 bits, also
+    two of them, end at a fixed distance from the largest.)"""
+    H, G, D, T, bf = 32, 8, 128, 3200, torch.bfloat16
+    q = torch.zeros(T, H, D, dtype=bf, device="cuda")
+    q[:, :, 0] = 8.0
+    k = torch.zeros(T, G, D, dtype=bf, device="cuda")
+    k[0, :, 0] = torch.arange(8.0, 24.0, 2.0) * (math.log(2.0) / 0.88)
+    k[1, :, 0] = -k[0, :, 0]
+    v = 1 + torch.rand(T, G, D, device="cuda").to(bf)
+    v[0], v[1] = 0.0, 2.0 ** 9
+    c = Paged([T], G, D, D, bf)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    batch = types.SimpleNamespace(
+        portion_tokens=T, pos=i32(range(T)), seq=i32([0] * T), block_table=c.bt,
+        tiles=i32([(0, s, min(128, T - s), s) for s in range(0, T, 128)]),
+        portions=i32([(0, 0, T, 0)]), max_keys=T)
+    got = sv.ragged_attention(q.view(T, -1), k.view(T, -1), v.view(T, -1), batch,
+                              (c.kc, c.vc), H, 0.11).view(T, H, D)
+    for g in range(G):
+        # the same query everywhere: running sums of weights and of weighted values
+        w = (0.11 * 8.0 * (k[:, g, 0] - k[0, g, 0]).double()).exp()
+        want = (w[:, None] * v[:, g].double()).cumsum(0) / w.cumsum(0)[:, None]
+        err = (got[:, 4 * g:4 * g + 4].double() - want[:, None]).abs()
+        # rounded to bf16 once; sums of 32 bits
+        assert (err <= (2.0 ** -8 + 2.0 ** -15) * want[:, None]).all(), (
+            g, (err / want[:, None])[1:].max().item())
 
 
 # ---------------------------------------------------------------------------
