@@ -12,6 +12,7 @@ import ctypes
 import functools
 import math
 import os
+import warnings
 from typing import Optional
 
 import torch
@@ -764,14 +765,20 @@ class _FlashAttnFn(torch.autograd.Function):
 
 @functools.lru_cache(maxsize=1)
 def _native_flash():
-    """``_FlashAttnFn`` in csrc/host/flash_autograd.cpp; None where it is not built."""
+    """``_FlashAttnFn`` in csrc/host/flash_autograd.cpp; None where it is not built, or
+    does not load: calls are Python's then, on the same kernels."""
     from .build import HOST_LIB
 
     if not os.path.exists(HOST_LIB):
         return None
     _require_lib()                    # its kernels
-    torch.ops.load_library(HOST_LIB)
-    return torch.ops.nxd_host.flash_attention.default
+    try:
+        torch.ops.load_library(HOST_LIB)
+        return torch.ops.nxd_host.flash_attention.default
+    except (OSError, RuntimeError, AttributeError) as e:
+        warnings.warn(f"{HOST_LIB} does not load ({e}): short attention takes its "
+                      "host up to 1.5 times as long")
+        return None
 
 
 def _fa_native(q, k, v) -> bool:
