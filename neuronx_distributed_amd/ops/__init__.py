@@ -765,20 +765,25 @@ class _FlashAttnFn(torch.autograd.Function):
 
 @functools.lru_cache(maxsize=1)
 def _native_flash():
-    """``_FlashAttnFn`` in csrc/host/flash_autograd.cpp; None where it is not built, or
-    does not load: calls are Python's then, on the same kernels."""
-    from .build import HOST_LIB
+    """``_FlashAttnFn`` in csrc/host/flash_autograd.cpp; None where it is not built for
+    this torch and these kernels, or does not load: calls are Python's then, on the same
+    kernels."""
+    from .build import host_lib, host_libs
 
-    if not os.path.exists(HOST_LIB):
-        return None
-    _require_lib()                    # its kernels
+    why = None
     try:
-        torch.ops.load_library(HOST_LIB)
-        return torch.ops.nxd_host.flash_attention.default
-    except (OSError, RuntimeError, AttributeError) as e:
-        warnings.warn(f"{HOST_LIB} does not load ({e}): short attention takes its "
-                      "host up to 1.5 times as long")
-        return None
+        lib = host_lib()
+        if os.path.exists(lib):
+            _require_lib()            # its kernels
+            torch.ops.load_library(lib)
+            return torch.ops.nxd_host.flash_attention.default
+        if host_libs():
+            why = f"{host_libs()} built for another torch or from other sources"
+    except (OSError, AttributeError) as e:
+        why = f"the native autograd library does not load ({e})"
+    if why:
+        warnings.warn(f"{why}: short attention takes its host up to 1.5 times as long")
+    return None
 
 
 def _fa_native(q, k, v) -> bool:

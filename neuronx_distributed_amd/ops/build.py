@@ -11,10 +11,11 @@ Libraries, so that a serving process compiles only what it runs:
                          batch-synchronous inference kernels,
 * ``libnxd_serving.so``  every ``csrc/serving/*.hip`` — the ragged-batch
                          kernels of the serving engine,
-* ``libnxd_host.so``     ``csrc/host/*.cpp`` — autograd functions in C++, which call
+* ``libnxd_host.<key>.so``  ``csrc/host/*.cpp`` — autograd functions in C++, which call
                          the kernels of ``libnxd_ops.so`` (host code, by g++).
 """
 
+import hashlib
 import os
 import subprocess
 import sys
@@ -24,7 +25,6 @@ _THIS = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_THIS, "csrc")
 LIB = os.path.join(_THIS, "libnxd_ops.so")
 SERVING_LIB = os.path.join(_THIS, "libnxd_serving.so")
-HOST_LIB = os.path.join(_THIS, "libnxd_host.so")
 
 GROUPS = {
     "ops": (CSRC, LIB),
@@ -105,16 +105,40 @@ def build_group(group: str, force: bool = False, verbose: bool = True) -> str:
     return lib
 
 
+def _host_sources():
+    return _listed(os.path.join(CSRC, "host"), ".cpp")
+
+
+def host_lib() -> str:
+    """The host library of these sources and of this torch, built or not.  What it
+    depends on is in its name: torch's C++ interface changes with every version, and
+    the kernels' prototypes (``csrc/flash_attn.h``) are compiled into it, so another
+    one is never loaded in its place."""
+    import torch
+
+    key = hashlib.sha256(repr((torch.__version__, torch.version.git_version,
+                               torch._C._GLIBCXX_USE_CXX11_ABI)).encode())
+    for path in _host_sources() + [os.path.join(CSRC, "flash_attn.h")]:
+        with open(path, "rb") as f:
+            key.update(f.read())
+    return os.path.join(_THIS, f"libnxd_host.{key.hexdigest()[:12]}.so")
+
+
+def host_libs():
+    """All that are built."""
+    return [p for p in _listed(_THIS, ".so")
+            if os.path.basename(p).startswith("libnxd_host.")]
+
+
 def build_host(force: bool = False, verbose: bool = True) -> str:
     """Compile the host library against torch; needs ``libnxd_ops.so``."""
-    sources = _listed(os.path.join(CSRC, "host"), ".cpp")
-    if not force and os.path.exists(HOST_LIB) and \
-            all(os.path.getmtime(s) <= os.path.getmtime(HOST_LIB) for s in sources):
-        return HOST_LIB
+    lib, sources = host_lib(), _host_sources()
+    if not force and os.path.exists(lib):
+        return lib
     import torch
 
     root = os.path.dirname(torch.__file__)
-    tmp = f"{HOST_LIB}.{os.getpid()}"
+    tmp = f"{lib}.{os.getpid()}"
     include = [os.path.join(root, "include"),
                os.path.join(root, "include", "torch", "csrc", "api", "include"),
                os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")]
@@ -126,11 +150,14 @@ def build_host(force: bool = False, verbose: bool = True) -> str:
               f"-L{_THIS}", "-l:" + os.path.basename(LIB),
               f"-L{os.path.join(root, 'lib')}", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
               "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], verbose)
-        os.replace(tmp, HOST_LIB)
+        os.replace(tmp, lib)
     finally:
         if os.path.exists(tmp):
             os.unlink(tmp)
-    return HOST_LIB
+    for old in host_libs():
+        if old != lib:
+            os.unlink(old)
+    return lib
 
 
 def build(force: bool = False, verbose: bool = True) -> str:

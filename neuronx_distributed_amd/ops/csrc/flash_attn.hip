@@ -29,6 +29,7 @@
 // f32 (natural-log row logsumexp, saved for backward).
 
 #include "common.h"
+#include "flash_attn.h"
 #include "mfma.h"
 #include "lds.h"
 

@@ -31,6 +31,7 @@
 // words and barriers (dQ 20 %), 27 % waits for a turn (37 %).
 
 #include "common.h"
+#include "flash_attn.h"
 #include "mfma.h"
 #include "lds.h"
 

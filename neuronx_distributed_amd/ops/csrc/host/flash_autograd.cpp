@@ -14,18 +14,7 @@
 #include <ATen/ops/empty_like.h>
 #include <c10/hip/HIPStream.h>
 
-extern "C" {
-void flash_attn_fwd_strided(const void* q, const void* k, const void* v, void* out,
-                            void* lse, int B, int Hq, int Hkv, int S, float scale,
-                            int causal, int window, const long* st, hipStream_t stream);
-void flash_attn_bwd_strided(const void* q, const void* k, const void* v, const void* out,
-                            const void* dout, const void* lse, void* delta, void* dq,
-                            void* dk, void* dv, int B, int Hq, int Hkv, int Hdk, int S,
-                            float scale, int causal, int window, const long* st,
-                            hipStream_t stream);
-void flash_attn_bwd_reduce(const void* kq, const void* vq, void* dk, void* dv, int B,
-                           int Hq, int Hkv, int S, const long* st, hipStream_t stream);
-}
+#include "../flash_attn.h"
 
 namespace {
 
