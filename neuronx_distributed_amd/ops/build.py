@@ -75,7 +75,8 @@ def _run(cmd, verbose):
     if out.strip() and (verbose or r.returncode):
         print(out, file=sys.stderr, flush=True)
     if r.returncode:
-        raise RuntimeError(f"hipcc failed ({r.returncode}): {' '.join(cmd)}")
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({r.returncode}): "
+                           f"{' '.join(cmd)}")
 
 
 def build_group(group: str, force: bool = False, verbose: bool = True) -> str:
@@ -163,7 +164,11 @@ def build_host(force: bool = False, verbose: bool = True) -> str:
 def build(force: bool = False, verbose: bool = True) -> str:
     for group in GROUPS:
         build_group(group, force, verbose)
-    build_host(force, verbose)
+    try:
+        build_host(force, verbose)
+    except (OSError, RuntimeError) as e:    # no g++, or none of torch's headers
+        print(f"[nxd_ops] no native autograd library, Python's functions serve: {e}",
+              file=sys.stderr, flush=True)
     return LIB
 
 

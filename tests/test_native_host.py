@@ -60,6 +60,21 @@ def test_a_library_of_other_sources_or_another_torch_is_not_loaded(
     assert build.host_libs() == [build.host_lib()]
 
 
+def test_a_build_without_a_host_compiler_ends_well(monkeypatch, tmp_path, capsys):
+    """Kernels are what a build has to make; Python's functions serve beside them."""
+    monkeypatch.setattr(build, "build_group", lambda *a: None)
+    monkeypatch.setattr(build, "_THIS", str(tmp_path))
+    monkeypatch.setenv("PATH", str(tmp_path))          # no g++
+    assert build.build(force=True, verbose=False) == build.LIB
+    assert "Python's functions serve" in capsys.readouterr().err
+    assert not build.host_libs()
+    gxx = tmp_path / "g++"                             # one without torch's headers
+    gxx.write_text("#!/bin/sh\nexit 1\n")
+    gxx.chmod(0o755)
+    build.build(force=True, verbose=False)
+    assert "g++ failed (1)" in capsys.readouterr().err
+
+
 def test_prototypes_are_in_one_place():
     """Callers and kernels include them, so a signature cannot change on one side."""
     for name in ("host/flash_autograd.cpp", "flash_attn.hip", "flash_attn_bwd.hip"):
