@@ -1765,15 +1765,26 @@ def latent_tiles_supported(q, gate, dim, vdim, rank, shared) -> bool:
 
 def expand_rule(rows: int, N: int, R: int) -> bool:
     """Are keys and values (rows, N) of a latent cache made by a kernel that reads its
-    pages where they lie, not by a copy and a library product?  Within a call, R 512, it
-    is 0.97 to 1.9 times as fast (us, copy and product | kernel: 128 x 8192 13.2 | 8.6,
-    1600 x 4096 25.8 | 17.4, 1152 x 8192 22.9 | 22.2, 6656 x 4096 72.8 | 49.2) but where
-    the library's tiles of 256 x 256 fill the CUs, or nearly (4096 x 4096 28.1 | 29.9,
-    1792 x 8192 25.0 | 25.8), and for large products (5184 x 8192 63.1 | 70.4; 10048 x
-    4096 79.8 | 75.2, 12800 76.5 | 82.8)."""
+    pages where they lie, not by a copy and a library product?  Both within a call, over
+    7161 sizes of rank 64 to 1536, us, copy and product | kernel.  Yes where its tiles of
+    128 x 128 are one round of workgroups and the rank is not so long that the library's
+    larger ones gain (128 x 8192, R 64 7.9 | 5.0, R 512 13.9 | 9.2; 128 x 2048 of R 1536
+    11.0 | 15.2); past that where the library's tiles of 256 x 256 leave CUs idle and the
+    rank is neither so short that the results alone decide nor so long (R 512: 1344 x 8192
+    39 | 23, 2048 x 10240 49 | 36, 2048 x 12288 45.5 | 41.7), but not where they fill them
+    or nearly (4096 x 4096 28.1 | 29.9, 3136 x 4096 25.5 | 29.6; R 64, 2240 x 12288 22.3 |
+    29.0), nor for large products (5184 x 8192 63.1 | 70.4).  Of the 4283 that it takes 3
+    lose more than 3 % and 0.5 us, 6 % at most: 128 tokens of two long ranks, and 768 x
+    32768 of 512, 45.1 | 47.4; the mean is 1.37 of the speed."""
+    own = -(-rows // 128) * -(-N // 128)
     tiles = -(-rows // 256) * -(-N // 256)
     whole = tiles >= 216 and not 0 < tiles % 256 < 216
-    return R % 64 == 0 and N * R < 1 << 30 and rows * N <= 28_000_000 and not whole
+    if R % 64 or N * R >= 1 << 30 or rows * N > 28_000_000 or whole:
+        return False
+    if own <= 512:
+        return R <= 640 or R <= 1024 and own <= 256
+    return 256 <= R <= 512 and (172 <= tiles <= 192 or 256 < tiles < 384 or
+                                R >= 384 and own >= 1440)
 
 
 def _expandable(cache, expand, pages, R: int, P: int) -> bool:

@@ -21,6 +21,19 @@ def test_a_library_without_the_products_is_not_used(monkeypatch):
     assert sv.available()
 
 
+@pytest.mark.parametrize("rows,N,R,kernel", [
+    # one round of workgroups, up to ranks of 640 and 1024
+    (64, 8, 64, True), (2048, 4096, 640, True), (2048, 4096, 704, False),
+    (2048, 2048, 1024, True), (2112, 2048, 1024, False), (64, 8, 1088, False),
+    # two and more: 172 to 192 of the library's tiles, 257 to 383, and full ones of our own
+    (2112, 4096, 512, False), (1344, 8192, 512, True), (1344, 8192, 192, False),
+    (1344, 8192, 576, False), (3136, 4096, 512, False), (2048, 10240, 256, True),
+    (2048, 10240, 192, False), (2048, 12288, 512, True), (2048, 12288, 320, False),
+    (1408, 16384, 512, False), (6592, 4096, 576, False), (2240, 12288, 64, False)])
+def test_latents_are_expanded_in_place_where_that_was_faster(rows, N, R, kernel):
+    assert sv.expand_rule(rows, N, R) == kernel
+
+
 @pytest.mark.skipif(not shutil.which("g++"), reason="no host compiler")
 def test_every_word_of_a_streamed_row_lies_in_it(tmp_path):
     """Rows of all K up to 4200 in the turns of 16 waves: words past the end are
