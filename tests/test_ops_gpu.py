@@ -785,6 +785,84 @@ def test_native_flash_attn_leaves_others_to_python():
         ops.flash_attn(q.float(), q.float(), q.float())
 
 
+def test_native_flash_attn_leaves_watched_calls_to_python():
+    """Transforms, and dispatch and function modes: what they see is Python's function,
+    which functorch refuses as it did."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    q = torch.randn(1, 2, 64, 128, device="cuda").bfloat16()
+    seen = []
+
+    def look(x):
+        seen.append(ops._fa_native(x, x, x))
+        return x.float().sum()
+
+    torch.func.grad(look)(q)
+    torch.func.vmap(look)(q[None])
+    torch.func.jvp(look, (q,), (q,))
+    assert seen == [False] * 3
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: ops.flash_attn(x, x, x).float().sum())(q)
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    want = ops.flash_attn(q, q, q)
+    for mode in (Dispatch, Function):
+        with mode():
+            assert not ops._fa_native(q, q, q)
+            got = ops.flash_attn(q, q, q)
+        assert torch.equal(got, want)
+    with torch.inference_mode():
+        assert ops._fa_native(q, q, q)
+        assert torch.equal(ops.flash_attn(q, q, q), want)
+
+
+@pytest.mark.parametrize("how", ["stream", "checkpoint", "twice", "create_graph"])
+def test_native_flash_attn_in_a_program(monkeypatch, how):
+    """On a stream of its own, recomputed, differentiated twice from one graph, and by a
+    graph of the gradients, which ends there: as Python's."""
+    from torch.utils.checkpoint import checkpoint
+
+    torch.manual_seed(3)
+    q, k, v = (torch.randn(1, 200, h, 128, device="cuda").bfloat16().transpose(1, 2)
+               .requires_grad_(True) for h in (4, 2, 2))
+    dy = torch.randn(1, 4, 200, 128, device="cuda").bfloat16()
+    side, got = torch.cuda.Stream(), []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(ops, "_native_flash", lambda: None)
+        torch.cuda.synchronize()
+        if how == "stream":
+            with torch.cuda.stream(side):
+                x = [t * 2 for t in (q, k, v)]       # (what the call has to wait for)
+                out = ops.flash_attn(*x) * 2
+                grads = torch.autograd.grad(out, (q, k, v), dy)
+            side.synchronize()
+        elif how == "checkpoint":
+            out = checkpoint(lambda *x: ops.flash_attn(*x) * 2, q, k, v,
+                             use_reentrant=False)
+            grads = torch.autograd.grad(out, (q, k, v), dy)
+        else:
+            out = ops.flash_attn(q, k, v)
+            grads = torch.autograd.grad(out, (q, k, v), dy, retain_graph=True,
+                                        create_graph=how == "create_graph")
+            if how == "twice":
+                again = torch.autograd.grad(out, (q, k, v), dy)
+                assert all(torch.equal(a, b) for a, b in zip(grads, again))
+                with pytest.raises(RuntimeError):    # the graph is freed
+                    torch.autograd.grad(out, (q, k, v), dy)
+        got.append((out.detach(), *grads))
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and a.requires_grad == b.requires_grad
+
+
 def test_add_rmsnorm_train_matches_unfused_autograd():
     """Training fused add+RMSNorm (fwd + the dpass-folding backward) vs
     the unfused bf16 add -> ops.rmsnorm chain: forward outputs equal and
