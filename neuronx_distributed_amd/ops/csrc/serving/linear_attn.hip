@@ -2063,8 +2063,9 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
 #pragma unroll
         for (int et = 0; et < 4; ++et) o[et] = *(f32x4*)(part + at[et]);
 #pragma unroll
-        for (int et = 0; et < 4; ++et) *(f32x4*)(part + at[et]) = GATE == GATED ? (inter * o[et] + pv[et]) * inv
-                                                    : inter * o[et] + pv[et];
+        for (int et = 0; et < 4; ++et)
+          *(f32x4*)(part + at[et]) = GATE == GATED ? (inter * o[et] + pv[et]) * inv
+                                                   : inter * o[et] + pv[et];
       };
       auto piece = [&](int i, const char* qb, const char* kb, const char* vb)
           __attribute__((always_inline)) {
@@ -2119,30 +2120,30 @@ __global__ void __launch_bounds__(768) memory_pass_kernel(ChunkArgs x) {
           den += inter * nq[0];
           inv = 1.f / (fmaxf(fabsf(den), s_em[(i & 1) * L + t]) + GATED_EPS);
         } else {
-        const float* b = s_b + (i & 1) * L;
-        const float bt = b[t];
-        const f32x4 bs = *(const f32x4*)(b + 16 * n + 4 * quad);
-        const f32x4 step = *(const f32x4*)(s_i + (i & 1) * L + 16 * n + 4 * quad);
-        f32x4 far[n + 1];
-        float from[n + 1];
+          const float* b = s_b + (i & 1) * L;
+          const float bt = b[t];
+          const f32x4 bs = *(const f32x4*)(b + 16 * n + 4 * quad);
+          const f32x4 step = *(const f32x4*)(s_i + (i & 1) * L + 16 * n + 4 * quad);
+          f32x4 far[n + 1];
+          float from[n + 1];
 #pragma unroll
-        for (int J = 0; J < n; ++J) {
-          far[J] = *(const f32x4*)(s_far + (i & 1) * L + 16 * J + 4 * quad);
-          from[J] = b[16 * J + 15];
-        }
+          for (int J = 0; J < n; ++J) {
+            far[J] = *(const f32x4*)(s_far + (i & 1) * L + 16 * J + 4 * quad);
+            from[J] = b[16 * J + 15];
+          }
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+          for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int J = 0; J <= n; ++J) acc[J] = mfma16(kf[c][J].bf, qf[c].bf, acc[J]);
-        inter = __expf(bt);
+            for (int J = 0; J <= n; ++J) acc[J] = mfma16(kf[c][J].bf, qf[c].bf, acc[J]);
+          inter = __expf(bt);
 #pragma unroll
-        for (int J = 0; J < n; ++J) acc[J] *= far[J] * __expf(bt - from[J]);
+          for (int J = 0; J < n; ++J) acc[J] *= far[J] * __expf(bt - from[J]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float w = acc[n][j] * (__expf(bt - bs[j]) * step[j]);
-          const int s = 4 * quad + j;
-          acc[n][j] = (s > col ? 0.f : w) + (s == col ? skip : 0.f);
-        }
+          for (int j = 0; j < 4; ++j) {
+            const float w = acc[n][j] * (__expf(bt - bs[j]) * step[j]);
+            const int s = 4 * quad + j;
+            acc[n][j] = (s > col ? 0.f : w) + (s == col ? skip : 0.f);
+          }
         }
 #pragma unroll
         for (int et = 0; et < 4; ++et) pv[et] = f32x4{};
@@ -2351,7 +2352,8 @@ static void launch_chunks(const ChunkArgs& x, hipStream_t stream) {
   if constexpr (GATE != TURNED && DP == PASS_D)
     if (!x.P) {
       const int units = a.H * (a.E / 64);
-      memory_pass_kernel<GATE><<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
+      memory_pass_kernel<GATE>
+          <<<(long)x.n_seg * 8 * ((units + 7) / 8), 768, 0, stream>>>(x);
       return;
     }
   if (!fixed_decay(GATE)) memory_gates_kernel<GATE><<<ch, MC_L, 0, stream>>>(x);
