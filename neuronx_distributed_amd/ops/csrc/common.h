@@ -73,9 +73,9 @@ __device__ __forceinline__ float block_reduce_sum(float v, float* lds_scratch) {
 
 // The head of workgroup x of a row of `heads`.  Workgroups go to the eight XCDs in
 // turn: heads that follow each other, which may share keys, meet in one L2.  Keys of
-// four heads each: forward and dQ of 8192 tokens, 32/8 heads 2271 -> 2251 us (all of the
-// backward in it), 2 x 3001 with a window of 1024 480 -> 472; 6000 tokens against pages
-// 563 -> 557.  Heads that are no multiple of 8 go to all XCDs either way.
+// four heads each: forward and dQ of 8192 tokens, 32/8 heads 2291 -> 2264 us (all of the
+// backward in it), 2 x 3001 with a window of 1024 483 -> 472; 6000 tokens against pages
+// 565 -> 553, with all else the same, where two runs differ by 0.2 %.  Heads that are no multiple of 8 go to all XCDs either way.
 __device__ __forceinline__ int near_head(int x, int heads) {
   return heads % 8 ? x : (x % 8) * (heads / 8) + x / 8;
 }

@@ -432,7 +432,7 @@ __device__ __forceinline__ void split3(float x, float y, uint* w) {
 }
 // The same, cut off instead of rounded, since three of 8 bits hold all 24 either way.
 // Masks take fewer cycles than shifts and packed conversions: one pass over 2731 and
-// 1365 tokens 103.8 -> 102.9 us, 1293 decayed ones 65.9 -> 65.0; but chunks' states and
+// 1365 tokens 104.4 -> 103.1 us (two runs differ by 0.1), 1293 decayed ones 65.9 -> 65.0; but chunks' states and
 // outputs of decayed memories took 2.5 % longer with it, of others 0.5 % less.
 __device__ __forceinline__ void cut3(float x, float y, uint* w) {
 #pragma unroll
