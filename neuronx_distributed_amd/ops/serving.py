@@ -1347,10 +1347,13 @@ def single_pass(chunks: int, segments: int, columns: int, gated: bool) -> bool:
     one pass 11.9 us (gated 11.3) behind 5 for the call; the launches and passes it
     stands for take 17 to 44 (21 to 50) up to a chunk or two and 0.08 us more for every
     64 columns of a chunk: 64 x 64 columns, 1000 tokens in one segment 51 and 52 (55 and
-    47), 1300 58 and 65, 1500 66 and 77 (66 and 67).  491 random calls each of 2 to 128
-    heads and up to 12 segments of unequal lengths, this over those: 0.56 (0.52)
-    in the mean, none slower."""
-    return chunks - segments + 1 <= chunks * (columns // 64) / 140 + 2 + gated
+    47), 1300 58 and 65, 1500 66 and 77 (66 and 67).  A segment's last chunk is half full
+    in the mean, and of many segments half of a chunk each is not there (16 x 256 columns,
+    2192 tokens beside 9 short segments 96 and 105, counted as whole ones).  4664 random
+    calls of 1 to 128 heads and up to 40 segments, this over those in the 3090 where it is
+    chosen: 0.41 in the mean, none slower by more than 2 %."""
+    full = chunks - (segments - 1) / 2
+    return chunks - segments + 1 <= full * (columns // 64) / 140 + 2 + gated
 
 
 def memory_mix(q, k, v, gate, S, n, m, seg, heads: int,

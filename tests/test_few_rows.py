@@ -34,6 +34,18 @@ def test_latents_are_expanded_in_place_where_that_was_faster(rows, N, R, kernel)
     assert sv.expand_rule(rows, N, R) == kernel
 
 
+@pytest.mark.parametrize("chunks,segments,columns,gated,once", [
+    (1, 1, 128, False, True), (10, 10, 128, True, True), (4, 1, 8192, False, True),
+    (6, 1, 4096, False, False), (4, 1, 4096, True, True),
+    # segments of less than a chunk beside a long one
+    (18, 10, 4096, False, False), (36, 26, 2048, True, False),
+    (47, 38, 1536, True, False), (12, 5, 4096, True, False),
+    (15, 7, 6144, False, True), (33, 22, 4096, False, True)])
+def test_memories_go_through_their_segments_at_once_where_that_was_faster(
+        chunks, segments, columns, gated, once):
+    assert sv.single_pass(chunks, segments, columns, gated) == once
+
+
 @pytest.mark.skipif(not shutil.which("g++"), reason="no host compiler")
 def test_every_word_of_a_streamed_row_lies_in_it(tmp_path):
     """Rows of all K up to 4200 in the turns of 16 waves: words past the end are
